@@ -28,27 +28,27 @@ QWEN = {1024: (28, 16, 3072, True), 2048: (28, 16, 6144, True), 2560: (36, 32, 9
 def listed():
     return [
         # one user chatting with a small model: every kernel is short, launches and round trips decide
-        dict(name="qwen 0.6b, 1 decoding", family="qwen", width=1024, layers=28, dtype="bfloat16", kind="decode", requests=1, shortest=500, longest=500),
+        dict(name="qwen-0.6b/1-decoding", family="qwen", width=1024, layers=28, dtype="bfloat16", kind="decode", requests=1, shortest=500, longest=500),
         # the benchmark's headline: eight requests in the middle of their answers
-        dict(name="qwen 8b, 8 decoding", family="qwen", width=4096, layers=36, dtype="bfloat16", kind="decode", requests=8, shortest=1152, longest=1152),
+        dict(name="qwen-8b/8-decoding", family="qwen", width=4096, layers=36, dtype="bfloat16", kind="decode", requests=8, shortest=1152, longest=1152),
         # a busy server: many requests of uneven lengths
-        dict(name="qwen 4b, 64 decoding", family="qwen", width=2560, layers=36, dtype="bfloat16", kind="decode", requests=64, shortest=100, longest=1300),
+        dict(name="qwen-4b/64-decoding", family="qwen", width=2560, layers=36, dtype="bfloat16", kind="decode", requests=64, shortest=100, longest=1300),
         # a long prompt, one portion of the engine's default size
-        dict(name="qwen 8b, prompt", family="qwen", width=4096, layers=36, dtype="bfloat16", kind="prompt", requests=1, shortest=2048, longest=2048),
+        dict(name="qwen-8b/prompt", family="qwen", width=4096, layers=36, dtype="bfloat16", kind="prompt", requests=1, shortest=2048, longest=2048),
         # several short questions that arrive together, sizes multiples of nothing
-        dict(name="qwen 1.7b, 6 prompts", family="qwen", width=2048, layers=28, dtype="bfloat16", kind="prompt", requests=6, shortest=19, longest=433),
+        dict(name="qwen-1.7b/6-prompts", family="qwen", width=2048, layers=28, dtype="bfloat16", kind="prompt", requests=6, shortest=19, longest=433),
         # continuous batching: a portion of a new prompt in one step with requests that decode
-        dict(name="qwen 4b, portion and 20", family="qwen", width=2560, layers=36, dtype="bfloat16", kind="mixed", requests=20, shortest=60, longest=700, portion=389),
+        dict(name="qwen-4b/portion-and-20", family="qwen", width=2560, layers=36, dtype="bfloat16", kind="mixed", requests=20, shortest=60, longest=700, portion=389),
         # the 32-bit mode, which checks and offline scoring run in: a prompt, and decoding
-        dict(name="qwen 0.6b f32, prompt", family="qwen", width=1024, layers=28, dtype="float32", kind="prompt", requests=1, shortest=611, longest=611),
-        dict(name="qwen 1.7b f32, 4 decoding", family="qwen", width=2048, layers=28, dtype="float32", kind="decode", requests=4, shortest=300, longest=420),
+        dict(name="qwen-0.6b-f32/prompt", family="qwen", width=1024, layers=28, dtype="float32", kind="prompt", requests=1, shortest=611, longest=611),
+        dict(name="qwen-1.7b-f32/4-decoding", family="qwen", width=2048, layers=28, dtype="float32", kind="decode", requests=4, shortest=300, longest=420),
         # mixtures of experts: a prompt, whose tokens use every expert, and decoding, where most experts have one or two
-        dict(name="balelorn 2048, prompt", family="balelorn", width=2048, layers=8, dtype="bfloat16", kind="prompt", requests=1, shortest=2011, longest=2011),
-        dict(name="balelorn 4096, 12 decoding", family="balelorn", width=4096, layers=8, dtype="bfloat16", kind="decode", requests=12, shortest=40, longest=800),
+        dict(name="balelorn-2048/prompt", family="balelorn", width=2048, layers=8, dtype="bfloat16", kind="prompt", requests=1, shortest=2011, longest=2011),
+        dict(name="balelorn-4096/12-decoding", family="balelorn", width=4096, layers=8, dtype="bfloat16", kind="decode", requests=12, shortest=40, longest=800),
         # recurrences: a prompt through matrix memories and the delta rule
-        dict(name="sodedra 2048, prompt", family="sodedra", width=2048, layers=8, dtype="bfloat16", kind="prompt", requests=1, shortest=1500, longest=1500),
+        dict(name="sodedra-2048/prompt", family="sodedra", width=2048, layers=8, dtype="bfloat16", kind="prompt", requests=1, shortest=1500, longest=1500),
         # whole requests, prompts and answers, through latent attention and minimal recurrences
-        dict(name="sefevik 2048, 5 whole", family="sefevik", width=2048, layers=8, dtype="bfloat16", kind="whole", requests=5, shortest=60, longest=500, steps=24),
+        dict(name="sefevik-2048/5-whole", family="sefevik", width=2048, layers=8, dtype="bfloat16", kind="whole", requests=5, shortest=60, longest=500, steps=24),
     ]
 
 
