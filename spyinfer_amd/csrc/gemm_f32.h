@@ -1,0 +1,7 @@
+// The float32 products (gemm_f32.hip): C[M, N] = A[M, K] . W[N, K]^T, all three float32, rows dense, K a multiple of 4 and both
+// operands 16-byte aligned.  gemm_f32_takes: whether they stand for these operands.
+#pragma once
+#include "common.h"
+
+bool gemm_f32_takes(const void* A, const void* W, const void* C, int M, int N, int K);
+int gemm_f32(const float* A, const float* W, float* C, int M, int N, int K, hipStream_t st);

@@ -1,0 +1,360 @@
+// C[M, N] = A[M, K] . W[N, K]^T in float32: products and sums of 32-bit numbers, no reduced-precision mode (the matrix cores'
+// float32 instructions multiply and add as fmaf does).  Three kernels by the number of rows:
+//
+//   few    (up to 4 or 8 rows)   bound by streaming W from memory.  A wave owns NR rows of W and walks K with 64 lanes side by side, so
+//                           that every load of W is 1 KiB in one piece; A comes from the caches; the lanes' sums meet at the end.
+//   narrow (tens of rows)   bound by W from memory as well, but A's rows would be read once per row of W by the kernel above.
+//                           A block owns 16 rows of W and MT tiles of 16 rows of A; its eight waves take the chunks of 64 of K in
+//                           turn, operands straight from memory into v_mfma_f32_16x16x4_f32 registers, and add through LDS.
+//   tile   (many rows)      bound by the matrix cores (256 flops a cycle and compute unit).  Tiles of A and W through LDS.
+//
+// The operands' order of K inside an MFMA step is free as long as both agree: a lane (r = lane % 16, g = lane / 16) loads the four
+// values k + 4 g .. + 3 of its row in one piece, and instruction j of four multiplies the j-th of them.
+#include "gemm_f32.h"
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float gf_f32x4_t;
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float gf_f32x16_t;
+
+__device__ __forceinline__ gf_f32x4_t gf_load(const float* p) { return *reinterpret_cast<const gf_f32x4_t*>(p); }
+__device__ __forceinline__ gf_f32x4_t gf_stream(const float* p) { return __builtin_nontemporal_load(reinterpret_cast<const gf_f32x4_t*>(p)); }
+
+// ---- few rows ------------------------------------------------------------------------------------------------------------
+template <int MR, int NR, int U>
+__global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
+                                                           int M, int N, int K) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int n0 = (blockIdx.x * 4 + wave) * NR;
+    if (n0 >= N) return;
+    const float* wrow[NR];
+    const float* arow[MR];
+#pragma unroll
+    for (int n = 0; n < NR; ++n) wrow[n] = W + (size_t)min(n0 + n, N - 1) * K + 4 * lane;      // rows beyond N or M: the last row's, not stored
+#pragma unroll
+    for (int m = 0; m < MR; ++m) arow[m] = A + (size_t)min(m, M - 1) * K + 4 * lane;
+    float acc[NR][MR] = {};
+    auto fetch = [&](gf_f32x4_t (&w)[U][NR], int c) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int n = 0; n < NR; ++n) w[u][n] = gf_stream(wrow[n] + (c + u) * 256);
+    };
+    auto products = [&](const gf_f32x4_t (&w)[U][NR], int c) {
+        gf_f32x4_t a[U][MR];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int m = 0; m < MR; ++m) a[u][m] = gf_load(arow[m] + (c + u) * 256);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int m = 0; m < MR; ++m)
+#pragma unroll
+                for (int n = 0; n < NR; ++n)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[n][m] = fmaf(a[u][m][j], w[u][n][j], acc[n][m]);
+    };
+    auto single = [&](int k) {
+        gf_f32x4_t w[NR];
+#pragma unroll
+        for (int n = 0; n < NR; ++n) w[n] = gf_stream(wrow[n] + k);
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+            const gf_f32x4_t a = gf_load(arow[m] + k);
+#pragma unroll
+            for (int n = 0; n < NR; ++n)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[n][m] = fmaf(a[j], w[n][j], acc[n][m]);
+        }
+    };
+    // groups of U chunks of 256 of K; the next group's rows of W are asked for before this one's products (no load under a
+    // condition: the compiler would wait for all of them)
+    const int groups = (K >> 8) / U;
+    gf_f32x4_t w0[U][NR], w1[U][NR];
+    if (groups > 0) {
+        fetch(w0, 0);
+        int i = 0;
+        for (; i + 2 < groups; i += 2) {
+            fetch(w1, (i + 1) * U);
+            products(w0, i * U);
+            fetch(w0, (i + 2) * U);
+            products(w1, (i + 1) * U);
+        }
+        if (i + 1 < groups) {
+            fetch(w1, (i + 1) * U);
+            products(w0, i * U);
+            products(w1, (i + 1) * U);
+        } else {
+            products(w0, i * U);
+        }
+    }
+    int k = groups * U * 256;
+    for (; k + 256 <= K; k += 256) single(k);
+    if (k + 4 * lane < K) single(k);                              // the rest of K, a multiple of 4
+#pragma unroll
+    for (int n = 0; n < NR; ++n)
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+            const float s = wave_sum(acc[n][m]);
+            if (lane == 0 && m < M && n0 + n < N) C[(size_t)m * N + n0 + n] = s;
+        }
+}
+
+// ---- a few tiles of rows ----------------------------------------------------------------------------------------------------
+#define GF_WAVES 8
+template <int MT>
+__global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_narrow_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                                        float* __restrict__ C, int M, int N, int K) {
+    __shared__ float red[GF_WAVES][MT][64][4];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int r = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * 16;
+    A += (size_t)blockIdx.y * (16 * MT) * K;
+    C += (size_t)blockIdx.y * (16 * MT) * N;
+    M -= blockIdx.y * (16 * MT);
+    const float* wrow = W + (size_t)min(n0 + r, N - 1) * K + 4 * g;
+    const float* arow[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) arow[mt] = A + (size_t)min(mt * 16 + r, M - 1) * K + 4 * g;
+    gf_f32x4_t acc[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt] = gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto fetch = [&](gf_f32x4_t (&w)[4], gf_f32x4_t (&a)[MT][4], int k) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            w[s] = gf_stream(wrow + k + 16 * s);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) a[mt][s] = gf_load(arow[mt] + k + 16 * s);
+        }
+    };
+    auto products = [&](const gf_f32x4_t (&w)[4], const gf_f32x4_t (&a)[MT][4]) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) acc[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[s][j], a[mt][s][j], acc[mt], 0, 0, 0);
+    };
+    // two sets of operands taken in turn: the next chunk's are asked for before this chunk's products
+    const int chunks = K >> 6, mine = (chunks - wave + GF_WAVES - 1) / GF_WAVES;
+    gf_f32x4_t w0[4], a0[MT][4], w1[4], a1[MT][4];
+    if (mine > 0) {
+        auto at = [&](int i) { return (wave + i * GF_WAVES) * 64; };
+        fetch(w0, a0, at(0));
+        int i = 0;
+        for (; i + 2 < mine; i += 2) {
+            fetch(w1, a1, at(i + 1));
+            products(w0, a0);
+            fetch(w0, a0, at(i + 2));
+            products(w1, a1);
+        }
+        if (i + 1 < mine) {
+            fetch(w1, a1, at(i + 1));
+            products(w0, a0);
+            products(w1, a1);
+        } else {
+            products(w0, a0);
+        }
+    }
+    if (wave == (chunks & (GF_WAVES - 1))) {              // the rest of K: the wave whose turn it would be
+        for (int k = chunks * 64; k < K; k += 16) {
+            const bool ok = k + 4 * g < K;
+            const gf_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+            const gf_f32x4_t w = ok ? gf_stream(wrow + k) : zero;
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const gf_f32x4_t a = ok ? gf_load(arow[mt] + k) : zero;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], a[j], acc[mt], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) *reinterpret_cast<gf_f32x4_t*>(red[wave][mt][lane]) = acc[mt];
+    __syncthreads();
+    if (wave >= MT) return;
+    // row tile mt is summed, in the order of the waves, and stored by wave mt: lane (r, g) has C[row r][columns 4 g ..]
+    gf_f32x4_t sum = *reinterpret_cast<const gf_f32x4_t*>(red[0][wave][lane]);
+#pragma unroll
+    for (int w = 1; w < GF_WAVES; ++w) sum += *reinterpret_cast<const gf_f32x4_t*>(red[w][wave][lane]);
+    const int m = wave * 16 + r;
+    if (m >= M) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (n0 + 4 * g + i < N) C[(size_t)m * N + n0 + 4 * g + i] = sum[i];
+}
+
+// ---- many rows ----------------------------------------------------------------------------------------------------------------
+// A tile of 64 x 64 of C per 256 threads, a wave a quarter of it (v_mfma_f32_32x32x2_f32, 64 cycles each).  Steps of 32 of K: two
+// steps' pieces of A and W are on their way to registers while this one's products run from LDS, two LDS stages, one barrier a
+// step.  Rows are padded to 36 floats: eight neighbouring rows start in different groups of four banks.  A wave's operands are 2 KB
+// of LDS per 256 cycles of products, a quarter of what LDS gives.  KS > 1: so many groups of 256 threads share a tile, each a part
+// of K.  Tiles of 128 x 128 were no faster (611 rows, 12288 x 2048: 308 against 304 us) and leave small products fewer blocks.
+// Measured: 102 TFLOP/s at 611 rows of 12288 x 2048, 110 at 1200 (the library's own float32 product gets 134 at 4096^3, the chip's
+// nominal rate is 157); the plain FMA kernel it stands for 10.
+#define GF_BK 32
+#define GF_LD 36
+template <int KS>
+__global__ __launch_bounds__(256 * KS) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
+                                                                 int M, int N, int K, int tiles_m, int tiles_n) {
+    __shared__ float lds[KS][2][128 * GF_LD];         // per part of K two stages: 64 rows of A, then 64 of W
+    // blocks go to the eight dies in turn: die x takes a run of neighbouring tiles, rows fastest, so that a piece of W is read into one L2
+    const int total = tiles_m * tiles_n, per = (total + 7) >> 3;
+    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (tile >= total) return;
+    const int m0 = (tile % tiles_m) * 64, n0 = (tile / tiles_m) * 64;
+    const int part = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, tid = threadIdx.x & 255;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = threadIdx.x & 63;
+    const int i = lane & 31, h = lane >> 5;
+    const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+    // staging: thread t has rows t / 8 and t / 8 + 32, values 4 (t % 8) .. of the step: eight lanes read 128 bytes of one row
+    const int sr = tid >> 3, sk = (tid & 7) * 4;
+    const float* ap[2];
+    const float* wp[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        ap[p] = A + (size_t)min(m0 + sr + 32 * p, M - 1) * K;       // rows beyond M or N: the last row's, not stored
+        wp[p] = W + (size_t)min(n0 + sr + 32 * p, N - 1) * K;
+    }
+    // this part's steps of K: `steps` for every part (the barriers are the block's), those from its end on staged as zeros
+    const int all = (K + GF_BK - 1) / GF_BK, steps = (all + KS - 1) / KS;
+    const int k_first = part * steps * GF_BK, k_end = min(K, k_first + steps * GF_BK);
+    const gf_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    auto fetch = [&](gf_f32x4_t (&va)[2], gf_f32x4_t (&vw)[2], int s) {
+        const int k = min(k_first + s * GF_BK + sk, K - 4);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            va[p] = gf_load(ap[p] + k);
+            vw[p] = gf_load(wp[p] + k);
+        }
+    };
+    auto stage = [&](const gf_f32x4_t (&va)[2], const gf_f32x4_t (&vw)[2], int s) {
+        const bool in = k_first + s * GF_BK + sk < k_end;
+        float* to = lds[part][s & 1] + sr * GF_LD + sk;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            *reinterpret_cast<gf_f32x4_t*>(to + 32 * p * GF_LD) = in ? va[p] : zero;
+            *reinterpret_cast<gf_f32x4_t*>(to + (64 + 32 * p) * GF_LD) = in ? vw[p] : zero;
+        }
+    };
+    // A sum over all of K in one chain would round K times: every 256 of K the chain's value goes to a second sum (611 x 1024 x 3072:
+    // relative error 2.9e-7 against 1.0e-6 for one chain)
+    gf_f32x16_t acc, sum;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = sum[e] = 0.f;
+    auto products = [&](int s) {
+        const float* fa_at = lds[part][s & 1] + (wm + i) * GF_LD + 4 * h;
+        const float* fw_at = lds[part][s & 1] + (64 + wn + i) * GF_LD + 4 * h;
+#pragma unroll
+        for (int kk = 0; kk < GF_BK; kk += 8) {
+            const gf_f32x4_t fa = gf_load(fa_at + kk), fw = gf_load(fw_at + kk);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fw[j], fa[j], acc, 0, 0, 0);
+        }
+        if ((s & 7) == 7 || s + 1 == steps) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                sum[e] += acc[e];
+                acc[e] = 0.f;
+            }
+        }
+    };
+    // step s runs from LDS stage s & 1 while the pieces of steps s + 1 and s + 2 are on their way (steps beyond the last read the
+    // last values of K again); a stage written behind step s was read last in step s - 1, which every wave left at a barrier
+    gf_f32x4_t a0[2], v0[2], a1[2], v1[2];
+    fetch(a0, v0, 0);
+    fetch(a1, v1, 1);
+    stage(a0, v0, 0);
+    __syncthreads();
+    int s = 0;
+    for (; s + 2 < steps; s += 2) {
+        fetch(a0, v0, s + 2);
+        products(s);
+        stage(a1, v1, s + 1);
+        __syncthreads();
+        fetch(a1, v1, s + 3);
+        products(s + 1);
+        stage(a0, v0, s + 2);
+        __syncthreads();
+    }
+    products(s);
+    if (s + 1 < steps) {
+        stage(a1, v1, s + 1);
+        __syncthreads();
+        products(s + 1);
+    }
+    if (KS > 1) {
+        // the other parts' sums through LDS (their own stages) to the first part's waves, added in the order of the parts
+        __syncthreads();
+        float* at = lds[part][0] + wave * 1024 + 4 * lane;
+        if (part > 0) {
+#pragma unroll
+            for (int e = 0; e < 16; e += 4) *reinterpret_cast<float4*>(at + e * 64) = make_float4(sum[e], sum[e + 1], sum[e + 2], sum[e + 3]);
+        }
+        __syncthreads();
+        if (part > 0) return;
+#pragma unroll
+        for (int p = 1; p < KS; ++p)
+#pragma unroll
+            for (int e = 0; e < 16; e += 4) {
+                const float4 v = *reinterpret_cast<const float4*>(lds[p][0] + wave * 1024 + 4 * lane + e * 64);
+                sum[e] += v.x; sum[e + 1] += v.y; sum[e + 2] += v.z; sum[e + 3] += v.w;
+            }
+    }
+    // lane (i, h) has C[row i][columns 8 q + 4 h .. + 3], q < 4
+    const int m = m0 + wm + i;
+    if (m >= M) return;
+    const bool whole = (N & 3) == 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int n = n0 + wn + 8 * q + 4 * h;
+        float* to = C + (size_t)m * N + n;
+        if (whole) {
+            if (n < N) *reinterpret_cast<float4*>(to) = make_float4(sum[4 * q], sum[4 * q + 1], sum[4 * q + 2], sum[4 * q + 3]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (n + e < N) to[e] = sum[4 * q + e];
+        }
+    }
+}
+
+// ---- dispatch --------------------------------------------------------------------------------------------------------------
+bool gemm_f32_takes(const void* A, const void* W, const void* C, int M, int N, int K) {
+    const uintptr_t at = (uintptr_t)A | (uintptr_t)W | (uintptr_t)C;
+    return K % 4 == 0 && at % 16 == 0 && (int64_t)((N + 63) / 64) * ((M + 63) / 64) < (1 << 28);
+}
+
+int gemm_f32(const float* A, const float* W, float* C, int M, int N, int K, hipStream_t st) {
+#define GF_FEW(MR, NR, U) gemm_f32_few_kernel<MR, NR, U><<<(N + 4 * NR - 1) / (4 * NR), 256, 0, st>>>(A, W, C, M, N, K)
+#define GF_NARROW(MT) gemm_f32_narrow_kernel<MT><<<dim3(tiles16, (M + 16 * MT - 1) / (16 * MT)), GF_WAVES * 64, 0, st>>>(A, W, C, M, N, K)
+#define GF_TILE(KS) gemm_f32_tile_kernel<KS><<<((tm * tn + 7) / 8) * 8, 256 * KS, 0, st>>>(A, W, C, M, N, K, tm, tn)
+    const int tiles16 = (N + 15) / 16, tm = (M + 63) / 64, tn = (N + 63) / 64;
+    if (M <= 4 || (M <= 8 && N <= 1024)) {
+        // Rows of W per wave: each more reads A once less, but takes waves away.  One up to 2048 rows of W (four rows of A, 2048 x
+        // 2048: 7.3 us against 7.4 with two, 9.8 with four), four from 12288 on (29.9 / 25.1 / 23.8 us for 12288 x 2048); with one
+        // or two rows of A, where A costs little, one up to 12288 (20.4 / 21.8 / 21.1) and for the output heads (1 row of A, 151936 x
+        // 1024: 100 / 106 / 115) or two (116 / 108 / 125).  5 to 8 rows take this kernel only where the next has blocks for a
+        // quarter of the compute units (1024 x 3072: 8.9 against 12.7 us; 2048 x 2048 10.3 against 9.3).
+        if (M == 1) GF_FEW(1, 1, 4);
+        else if (M == 2) { if (N > 12288) GF_FEW(2, 2, 2); else GF_FEW(2, 1, 4); }
+        else if (M <= 4) { if (N >= 12288) GF_FEW(4, 4, 2); else if (N > 2048) GF_FEW(4, 2, 2); else GF_FEW(4, 1, 4); }
+        else GF_FEW(8, 1, 2);
+    } else if (tm * tn < 160) {
+        // Row tiles per block: as many as leave a block for every compute unit, W being read once per group of them (24 rows, 2048 x
+        // 2048: 10.4 us with one, 13.1 with two; 4096 x 2048: 19.4 with one, 14.5 with two; 64 rows, 4096 x 1024: 20 / 15.3 / 13.9
+        // with one / two / four).  Up to 64-row tiles for 160 blocks this kernel is ahead of the next (64 rows, 6144 x 1024: 22.6
+        // against 24.6 us; 200 rows, 1024 x 2048: 21.5 / 40.7; behind it at 64 rows, 12288 x 2048: 68 / 49 and at 300, 2048 x 2048: 58 / 42).
+        if (M > 32 && tiles16 * ((M + 63) / 64) >= 256) GF_NARROW(4);
+        else if (M > 16 && tiles16 * ((M + 31) / 32) >= 256) GF_NARROW(2);
+        else GF_NARROW(1);
+    } else {
+        // Parts of K in a block: where a compute unit has one or two blocks, more waves hide the loads, LDS and barriers of each
+        // other (611 rows, 1024 x 2048, 160 blocks: 51.6 / 43.8 / 41.1 us with one / two / four; 300 rows, 4096 x 2048, 320 blocks:
+        // 80.9 / 76.8 / 80.2; 1200 rows, 12288 x 2048: 550 / 556 / 596).
+        if (tm * tn <= 256) GF_TILE(4);
+        else if (tm * tn <= 512) GF_TILE(2);
+        else GF_TILE(1);
+    }
+    SPY_CHECK_LAUNCH("spy_gemm (float32)");
+    return 0;
+}

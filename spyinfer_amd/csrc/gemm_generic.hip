@@ -1,9 +1,10 @@
 // C[M, N] = A[M, K] . W[N, K]^T with float32 products and sums (no reduced-precision matrix
-// mode), operands float32 or bfloat16 in any combination.  This is the true 32-bit product of
-// the engine and the fallback for shapes the MFMA kernels refuse.  A 64x64 tile of C per block,
+// mode), operands float32 or bfloat16 in any combination.  All-float32 operands in whole 16-byte pieces go to
+// gemm_f32.hip; this kernel is for mixed types and for shapes that neither those nor the bfloat16 MFMA kernels take.  A 64x64 tile of C per block,
 // 16x16 threads with 4x4 outputs each, K walked in steps of 16 through LDS.  Each output sums its
 // products in ascending k, so a row's result does not depend on the other rows of the batch.
 #include "common.h"
+#include "gemm_f32.h"
 
 #define GT 64
 #define GK 16
@@ -54,6 +55,8 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(const TA* __restrict_
 extern "C" int spy_gemm(const void* A, int a_dtype, const void* W, int w_dtype, void* C, int c_dtype, int M, int N, int K,
                         hipStream_t st) {
     SPY_REQUIRE(M > 0 && N > 0 && K > 0, "spy_gemm: empty operand");
+    if (a_dtype == SPY_F32 && w_dtype == SPY_F32 && c_dtype == SPY_F32 && gemm_f32_takes(A, W, C, M, N, K))
+        return gemm_f32((const float*)A, (const float*)W, (float*)C, M, N, K, st);
     const dim3 grid((N + GT - 1) / GT, (M + GT - 1) / GT);
     SPY_REQUIRE(grid.y <= 65535, "spy_gemm: M = %d is too large for this kernel", M);
     SPY_DISPATCH(a_dtype, TA, SPY_DISPATCH(w_dtype, TW, SPY_DISPATCH(c_dtype, TC, (gemm_generic_kernel<TA, TW, TC><<<grid, 256, 0, st>>>(
