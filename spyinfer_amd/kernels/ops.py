@@ -71,7 +71,7 @@ class _Hip:
         self.lib = _build.load()
         self.lib.spy_last_error.restype = ctypes.c_char_p
         for name in ("spy_embedding", "spy_add_rmsnorm", "spy_rmsnorm", "spy_gemm", "spy_qknorm_rope_store",
-                     "spy_attention_generic", "spy_attention_mfma", "spy_attention_mfma_workspace", "spy_attention_mfma_part_workspace", "spy_attention_prefill",
+                     "spy_attention_generic", "spy_attention_f32", "spy_attention_f32_workspace", "spy_attention_mfma", "spy_attention_mfma_workspace", "spy_attention_mfma_part_workspace", "spy_attention_prefill",
                      "spy_attention_prefill_workspace", "spy_swiglu", "spy_untile_weight",
                      "spy_sample", "spy_sample_workspace", "spy_gemm_skinny", "spy_gemm_skinny_swiglu",
                      "spy_gemm_decode", "spy_gemm_decode_workspace", "spy_embedding_sumsq", "spy_sample_static", "spy_measure_read",
@@ -886,6 +886,11 @@ def prefill_tile_rows(d: int, rows_of_entries, n_kv: int) -> int:
     return 256 if (tiles + 1) // 2 * n_kv >= PREFILL_WIDE_TILES_MIN_BLOCKS else 128
 
 
+def f32_attention_ok(dtype, d: int, page_size: int) -> bool:
+    """Whether the float32 kernel on the matrix cores takes these heads and pages (in 16-row tiles only)."""
+    return dtype == torch.float32 and d in (64, 128) and page_size % 16 == 0
+
+
 def mfma_attention_ok(dtype, d: int, page_size: int) -> bool:
     return MFMA_ATTENTION and dtype == torch.bfloat16 and d % 16 == 0 and 16 <= d <= 256 and page_size % 8 == 0
 
@@ -1052,6 +1057,20 @@ def paged_attention(q: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: t
                        ctypes.c_int(0 if counters is None else ATTENTION_COUNTERS), _ptr(pieces),
                        ctypes.c_int(0 if pieces is None else pieces.shape[0]), *extras, _Hip.stream())
         return operand if operand is not None else out
+    if f32_attention_ok(q.dtype, d, page_size) and meta.tiles is not None and meta.tiles_group == group and meta.tiles["big"][2] == 0 \
+            and meta.tiles["small"][2] <= 65535 and (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0:
+        tile_entry, tile_row0, n_tiles = meta.tiles["small"]
+        for name, t in (("small tile entries", tile_entry), ("small tile rows", tile_row0)):
+            _check(t.dtype == torch.int32 and tuple(t.shape) == (n_tiles,), "paged_attention: %s must be int32 [%d]", name, n_tiles)
+        # few tiles cannot fill the chip: their keys go in parts of 128 at least (a number that follows the captured step's key_parts_for)
+        splits = max(1, min(DECODE_SPLIT_TARGET // max(1, n_tiles * n_kv), 2 * key_parts_for(max_keys)))
+        ws = torch.empty((max(1, hip().lib.spy_attention_f32_workspace(ctypes.c_int(n_tiles), ctypes.c_int(n_kv), ctypes.c_int(d), ctypes.c_int(splits))),),
+                         dtype=torch.float32, device=q.device)
+        hip().call("spy_attention_f32", _ptr(out), _ptr(q), _ptr(k_cache), _ptr(v_cache), ctypes.c_int(page_size), ctypes.c_int(num_pages),
+                   _ptr(meta.cu_q), _ptr(meta.pos0), _ptr(meta.kv_len), _ptr(meta.block_table), ctypes.c_int(meta.max_blocks), _ptr(tile_entry),
+                   _ptr(tile_row0), ctypes.c_int(n_tiles), ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(n_q), ctypes.c_int(n_kv), ctypes.c_int(d),
+                   ctypes.c_float(scale), ctypes.c_int(win), ctypes.c_float(softcap), ctypes.c_int(splits), _ptr(ws), *extras, _Hip.stream())
+        return out
     hip().call("spy_attention_generic", _ptr(out), _ptr(q), _code(q, "q"), _ptr(k_cache), _ptr(v_cache),
                ctypes.c_int(page_size), ctypes.c_int(num_pages), _ptr(meta.kv_len), _ptr(meta.block_table),
                ctypes.c_int(meta.max_blocks), _ptr(meta.token_entry), _ptr(meta.positions), ctypes.c_int(S), ctypes.c_int(T),

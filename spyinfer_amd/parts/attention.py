@@ -296,8 +296,8 @@ class PagedAttention(Mixer):
 
     def _big_rows(self, batch, page_size: int) -> int:
         """Rows of the tiles for this step's entries with many rows; 0 if the prefill kernel does not take this head
-        size or page."""
-        if not ops.prefill_attention_ok(self.head_dim, page_size):
+        size or page, and in float32 steps (the float32 kernel has 16-row tiles only)."""
+        if batch.act_dtype == torch.float32 or not ops.prefill_attention_ok(self.head_dim, page_size):
             return 0
         note = ("attention_big_rows", self.num_heads, self.num_kv_heads, self.head_dim)
         if note not in batch.shared:
