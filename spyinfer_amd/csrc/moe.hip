@@ -133,12 +133,19 @@ extern "C" int spy_moe_route(int* ids, float* weights, const float* z, const flo
     return 0;
 }
 
+// Groups of neighbouring row tiles of one expert, which the products of many rows per expert go by: [0] how many there are, then two
+// ints for each: first tile * 16 + tiles (MOE_GROUP of them but for an expert's last group), and its band, first group * 8 + groups:
+// up to MOE_BAND groups of one expert whose blocks run beside each other.
+#define MOE_GROUP 8
+#define MOE_BAND 4
+__device__ __host__ __forceinline__ int moe_max_groups(int max_tiles, int E, int P) { return max_tiles / MOE_GROUP + (E < P ? E : P); }
+
 // One block.  Pair p's expert is expert_of(p) (outside 0 .. E - 1: the pair has no row) -> sorted_pair [max_tiles MOE_TM]
-// (pair or -1), pair_row [P], tile_expert [max_tiles] (expert or -1).
+// (pair or -1), pair_row [P], tile_expert [max_tiles] (expert or -1), group [1 + 2 moe_max_groups].
 template <typename F>
 __device__ __forceinline__ void moe_align_block(int* __restrict__ sorted_pair, int* __restrict__ pair_row, int* __restrict__ tile_expert,
-                                                F expert_of, int P, int E, int max_tiles) {
-    __shared__ int count[MOE_MAX_EXPERTS], first[MOE_MAX_EXPERTS], cursor[MOE_MAX_EXPERTS];
+                                                int* __restrict__ group, F expert_of, int P, int E, int max_tiles) {
+    __shared__ int count[MOE_MAX_EXPERTS], first[MOE_MAX_EXPERTS], cursor[MOE_MAX_EXPERTS], first_group[MOE_MAX_EXPERTS];
     __shared__ int total_tiles;
     const int tid = threadIdx.x;
     for (int e = tid; e < E; e += blockDim.x) { count[e] = 0; cursor[e] = 0; }
@@ -149,17 +156,27 @@ __device__ __forceinline__ void moe_align_block(int* __restrict__ sorted_pair, i
     }
     __syncthreads();
     if (tid == 0) {
-        int tiles = 0;
+        int tiles = 0, groups = 0;
         for (int e = 0; e < E; ++e) {
+            const int nt = (count[e] + MOE_TM - 1) / MOE_TM;
             first[e] = tiles;
-            tiles += (count[e] + MOE_TM - 1) / MOE_TM;
+            first_group[e] = groups;
+            tiles += nt;
+            groups += (nt + MOE_GROUP - 1) / MOE_GROUP;
         }
         total_tiles = tiles;
+        group[0] = min(groups, moe_max_groups(max_tiles, E, P));
     }
     __syncthreads();
     for (int e = tid; e < E; e += blockDim.x) {
         const int nt = (count[e] + MOE_TM - 1) / MOE_TM;
         for (int i = 0; i < nt && first[e] + i < max_tiles; ++i) tile_expert[first[e] + i] = e;
+        for (int i = 0; i * MOE_GROUP < nt && first_group[e] + i < moe_max_groups(max_tiles, E, P); ++i)
+        {
+            const int ng = (nt + MOE_GROUP - 1) / MOE_GROUP, band = i / MOE_BAND * MOE_BAND, at = 1 + 2 * (first_group[e] + i);
+            group[at] = (first[e] + i * MOE_GROUP) * 16 + min(MOE_GROUP, nt - i * MOE_GROUP);
+            group[at + 1] = (first_group[e] + band) * 8 + min(MOE_BAND, ng - band);
+        }
         for (int r = count[e]; r < nt * MOE_TM; ++r)
             if (first[e] * MOE_TM + r < max_tiles * MOE_TM) sorted_pair[first[e] * MOE_TM + r] = -1;
     }
@@ -175,32 +192,35 @@ __device__ __forceinline__ void moe_align_block(int* __restrict__ sorted_pair, i
 }
 
 __global__ __launch_bounds__(1024) void moe_align_kernel(int* __restrict__ sorted_pair, int* __restrict__ pair_row,
-                                                         int* __restrict__ tile_expert, const int* __restrict__ ids, int P, int E,
-                                                         int max_tiles) {
-    moe_align_block(sorted_pair, pair_row, tile_expert, [=](int p) { return ids[p]; }, P, E, max_tiles);
+                                                         int* __restrict__ tile_expert, int* __restrict__ group,
+                                                         const int* __restrict__ ids, int P, int E, int max_tiles) {
+    moe_align_block(sorted_pair, pair_row, tile_expert, group, [=](int p) { return ids[p]; }, P, E, max_tiles);
 }
 
 // Experts named by tables of the token ids: all of a step's mixtures at once, one block per mixture.  Mixture l: the table
 // [V, top] (int32), E experts; pair p = (token p / top, choice p % top).  out: the mixtures' arrays one after the other, each
-// sorted_pair [max_tiles MOE_TM], pair_row [T top], tile_expert [max_tiles], every array rounded up to four ints.
+// sorted_pair [max_tiles MOE_TM], pair_row [T top], tile_expert [max_tiles], group [1 + 2 moe_max_groups], every array rounded up to
+// four ints.
 struct MoeTable { const int* table; int E, top; };
 __device__ __forceinline__ int moe_up4(int n) { return (n + 3) & ~3; }
 __global__ __launch_bounds__(1024) void moe_align_tables_kernel(int* __restrict__ out, const MoeTable* __restrict__ tables,
                                                                 const int* __restrict__ ids, int T, int V) {
     size_t off = 0;
-    int P = 0, max_tiles = 0;
+    int P = 0, max_tiles = 0, groups = 0;
     for (int l = 0; l <= (int)blockIdx.x; ++l) {
-        if (l) off += moe_up4(max_tiles * MOE_TM) + moe_up4(P) + moe_up4(max_tiles);
+        if (l) off += moe_up4(max_tiles * MOE_TM) + moe_up4(P) + moe_up4(max_tiles) + moe_up4(1 + 2 * groups);
         P = T * tables[l].top;
         max_tiles = P / MOE_TM + min(tables[l].E, P);
+        groups = moe_max_groups(max_tiles, tables[l].E, P);
     }
     const MoeTable tb = tables[blockIdx.x];
     int* sorted_pair = out + off;
     int* pair_row = sorted_pair + moe_up4(max_tiles * MOE_TM);
     int* tile_expert = pair_row + moe_up4(P);
+    int* group = tile_expert + moe_up4(max_tiles);
     const int top = tb.top;
     const int* table = tb.table;
-    moe_align_block(sorted_pair, pair_row, tile_expert, [=](int p) {
+    moe_align_block(sorted_pair, pair_row, tile_expert, group, [=](int p) {
         const int t = p / top, id = ids[t];
         return id >= 0 && id < V ? table[(size_t)id * top + (p - t * top)] : -1;
     }, P, tb.E, max_tiles);
@@ -219,16 +239,17 @@ extern "C" int spy_moe_align_tables(int* out, int64_t out_ints, const void* tabl
     return 0;
 }
 
-extern "C" int spy_moe_align(int* sorted_pair, int* pair_row, int* tile_expert, const int* ids, int P, int E, int max_tiles,
+extern "C" int spy_moe_align(int* sorted_pair, int* pair_row, int* tile_expert, int* group, const int* ids, int P, int E, int max_tiles,
                              hipStream_t st) {
     SPY_REQUIRE(P > 0 && E > 0 && E <= MOE_MAX_EXPERTS, "spy_moe_align: %d experts (1..%d)", E, MOE_MAX_EXPERTS);
     SPY_REQUIRE(max_tiles >= P / MOE_TM + (E < P ? E : P), "spy_moe_align: %d tiles are too few for %d pairs of %d experts", max_tiles, P, E);
-    moe_align_kernel<<<1, 1024, 0, st>>>(sorted_pair, pair_row, tile_expert, ids, P, E, max_tiles);
+    moe_align_kernel<<<1, 1024, 0, st>>>(sorted_pair, pair_row, tile_expert, group, ids, P, E, max_tiles);
     SPY_CHECK_LAUNCH("spy_moe_align");
     return 0;
 }
 
 extern "C" int spy_moe_tile_rows() { return MOE_TM; }
+extern "C" int spy_moe_group_ints(int max_tiles, int E, int P) { return 1 + 2 * moe_max_groups(max_tiles, E, P); }
 
 // A tile of MOE_TM sorted rows x 64 columns per block; 256 threads, thread (ty, tx) has row ty and columns 4 tx .. + 3.
 // gather > 0: row r reads A[sorted_pair[r] / gather] (the token of the pair); 0: A[r].
@@ -571,6 +592,147 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_mfma_lds_kernel(TC* __restric
     }
 }
 
+// Many rows per expert, K in whole steps of 64: a block has one group of up to 8 row tiles (128 sorted rows of one expert) and 128
+// rows of W (gated: the gate and up rows of 64 columns); both operands go through LDS and are shared by its four waves (2 x 2, each 64
+// x 64 of the products), two LDS stages of a step of 64 of K, two steps' pieces on their way in registers, one barrier a step.  A row
+// of a stage is 128 bytes, piece p of row r lies at place p ^ (r % 8), so that neither the writes nor the operands' reads meet in a bank.
+// What bounds it: LDS (a wave reads 16 KB for its 32 products of 16 cycles a step, 128 bytes a cycle and compute unit with four waves,
+// beside 32 KB of writes), which two blocks per compute unit keep busy in turn.  Measured, both products of 32 experts of 2 x 1536 x 2048,
+// four a token: 183 + 108 us at 2011 tokens (550 and 470 TFLOP/s; 132 us with one expert's matrices in the caches) against 286 + 175
+// for the kernel above, which is left for other sizes of K; 93 + 35 at 300 tokens against 184 + 85, where the matrices' way from memory
+// bounds it (4.4 TB/s).
+template <bool GATED, typename TC>
+__global__ __launch_bounds__(256, 2) void moe_gemm_group_kernel(TC* __restrict__ C, const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                                                const int* __restrict__ tile_expert, const int* __restrict__ sorted_pair,
+                                                                const int* __restrict__ group, int gather, int N, int K, int gy,
+                                                                long long w_stride, MoeAct act) {
+    __shared__ __align__(16) bf16_t stage_[2][256 * 64];       // 128 rows of A, then 128 of W
+    __shared__ int src_row[128];
+    // Blocks go to the dies in turn: a die takes a run of the blocks there are in (band, columns, group of the band) order, so that
+    // the blocks that read the same rows of W run beside each other, and an expert's matrix comes into one L2 once (in (group,
+    // columns) order half of the L2's requests missed, 955 MB a call for 403 MB of matrices: 184 us at 2011 tokens, 32 experts of
+    // 2 x 1536 x 2048, four a token)
+    const int total = group[0] * gy, per = (total + MOE_DIES - 1) / MOE_DIES, idx = blockIdx.x / MOE_DIES;
+    const int v = (blockIdx.x % MOE_DIES) * per + idx;
+    if (idx >= per || v >= total) return;
+    const int band = group[2 + 2 * (v / gy)], first = band >> 3, n_band = band & 7, in_band = v - first * gy;
+    const int by = in_band / n_band, gr = group[1 + 2 * (first + in_band % n_band)];
+    const int t = gr >> 4, rows = (gr & 15) * MOE_TM;
+    const int e = tile_expert[t];
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave & 1, wn = wave >> 1;
+    if (tid < 128) {
+        int src = -1;
+        if (tid < rows) {
+            const int p = sorted_pair[t * MOE_TM + tid];
+            src = p < 0 ? -1 : (gather > 0 ? p / gather : t * MOE_TM + tid);
+        }
+        src_row[tid] = src;
+    }
+    __syncthreads();
+    // staging: thread t has rows t / 8 + 32 i of A and of W, 16-byte piece t % 8.  Rows that do not exist are read as row 0 or the
+    // last one: what they give is not stored
+    const int sr = tid >> 3, piece = tid & 7;
+    const bf16_t* ap[4];
+    const bf16_t* wp[4];
+    const bf16_t* We = W + (size_t)e * w_stride;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = sr + 32 * i;
+        ap[i] = A + (size_t)max(src_row[row], 0) * K + 8 * piece;
+        const int wrow = GATED ? (row < 64 ? min(by * 64 + row, N - 1) : N + min(by * 64 + row - 64, N - 1)) : min(by * 128 + row, N - 1);
+        wp[i] = We + (size_t)wrow * K + 8 * piece;
+    }
+    const int to = sr * 64 + ((piece ^ (sr & 7)) * 8);
+    moe_f32x4_t acc[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[a][b] = moe_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int steps = K / 64;
+    auto fetch = [&](moe_bf16x8_t (&va)[4], moe_bf16x8_t (&vw)[4], int s) {
+        const int k = min(s, steps - 1) * 64;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vw[i] = *reinterpret_cast<const moe_bf16x8_t*>(wp[i] + k);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) va[i] = *reinterpret_cast<const moe_bf16x8_t*>(ap[i] + k);
+    };
+    auto stage = [&](const moe_bf16x8_t (&va)[4], const moe_bf16x8_t (&vw)[4], int s) {
+        bf16_t* base = stage_[s & 1] + to;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            *reinterpret_cast<moe_bf16x8_t*>(base + 32 * i * 64) = va[i];
+            *reinterpret_cast<moe_bf16x8_t*>(base + (128 + 32 * i) * 64) = vw[i];
+        }
+    };
+    const bool busy = wm * 64 < rows;                // a wave whose rows do not exist stages only
+    auto products = [&](int s) {
+        if (!busy) return;
+        const bf16_t* base = stage_[s & 1];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const int at = ((4 * ks + g) ^ (r & 7)) * 8;
+            moe_bf16x8_t fa[4], fw[4];
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) {
+                const int row = GATED ? (nt < 2 ? wn * 32 + nt * 16 : 64 + wn * 32 + (nt - 2) * 16) : wn * 64 + nt * 16;
+                fw[nt] = *reinterpret_cast<const moe_bf16x8_t*>(base + (128 + row + r) * 64 + at);
+            }
+#pragma unroll
+            for (int mt = 0; mt < 4; ++mt) fa[mt] = *reinterpret_cast<const moe_bf16x8_t*>(base + (wm * 64 + mt * 16 + r) * 64 + at);
+#pragma unroll
+            for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+                for (int nt = 0; nt < 4; ++nt) acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[nt], fa[mt], acc[nt][mt], 0, 0, 0);
+        }
+    };
+    moe_bf16x8_t a0[4], w0[4], a1[4], w1[4];
+    fetch(a0, w0, 0);
+    fetch(a1, w1, 1);
+    stage(a0, w0, 0);
+    __syncthreads();
+    int s = 0;
+    for (; s + 2 < steps; s += 2) {
+        fetch(a0, w0, s + 2);
+        products(s);
+        stage(a1, w1, s + 1);                        // (read last in step s - 1, which every wave has left)
+        __syncthreads();
+        fetch(a1, w1, s + 3);
+        products(s + 1);
+        stage(a0, w0, s + 2);
+        __syncthreads();
+    }
+    products(s);
+    if (s + 1 < steps) {
+        stage(a1, w1, s + 1);
+        __syncthreads();
+        products(s + 1);
+    }
+    const bool whole = N % 4 == 0;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+        const int lrow = wm * 64 + mt * 16 + r;
+        if (src_row[lrow] < 0) continue;
+        const size_t row = (size_t)t * MOE_TM + lrow;
+        const float rw = (GATED && act.pair_w) ? act.pair_w[sorted_pair[row]] : 1.f;
+#pragma unroll
+        for (int nt = 0; nt < (GATED ? 2 : 4); ++nt) {
+            const int col = GATED ? by * 64 + wn * 32 + nt * 16 + 4 * g : by * 128 + wn * 64 + nt * 16 + 4 * g;
+            float y[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[i] = GATED ? moe_gated(acc[nt][mt][i], acc[GATED ? nt + 2 : nt][mt][i], act, rw) : moe_ungated(acc[nt][mt][i], act);
+            TC* c = C + row * N + col;
+            if (whole) {
+                if (col < N) Vec4<TC>::store(c, y);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (col + i < N) c[i] = from_f32<TC>(y[i]);
+            }
+        }
+    }
+}
+
 template <int MT>
 static int moe_gemm_mfma_launch(void* C, int c_dtype, const void* A, const void* W, const int* tile_expert, const int* sorted_pair,
                                 int gather, int gated, int max_tiles, int N, int K, MoeAct act, hipStream_t st) {
@@ -597,12 +759,28 @@ static int moe_gemm_mfma_launch(void* C, int c_dtype, const void* A, const void*
 }
 
 extern "C" int spy_moe_gemm(void* C, int c_dtype, const void* A, int a_dtype, const void* W, int w_dtype, const int* tile_expert,
-                            const int* sorted_pair, int gather, int gated, int max_tiles, int E, int N, int K, int tiles_per_block,
-                            int act_kind, float limit, const float* pair_w, hipStream_t st) {
+                            const int* sorted_pair, const int* group, int P, int gather, int gated, int max_tiles, int E, int N, int K,
+                            int tiles_per_block, int act_kind, float limit, const float* pair_w, hipStream_t st) {
     SPY_REQUIRE(max_tiles > 0 && E > 0 && N > 0 && K > 0 && gather >= 0, "spy_moe_gemm: bad sizes (%d tiles)", max_tiles);
     SPY_REQUIRE((act_kind == 0 && !pair_w) || (act_kind == 1 && gated && limit > 0.f) || (act_kind == 2 && !gated && !pair_w), "spy_moe_gemm: activation %d with limit %g", act_kind, (double)limit);
     const MoeAct act = {act_kind, limit, pair_w};
     // bfloat16 operands in 16-byte pieces: the matrix cores; tiles_per_block: 0 = the plain float32 kernel
+    if (tiles_per_block >= 8 && group && a_dtype == SPY_BF16 && w_dtype == SPY_BF16 && K % 64 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16) == 0) {
+        const int cols = gated ? 64 : 128, gy = (N + cols - 1) / cols;
+        const int64_t blocks = (int64_t)moe_max_groups(max_tiles, E, P) * gy;
+        SPY_REQUIRE(blocks < (1 << 30), "spy_moe_gemm: too many blocks");
+        const unsigned grid = (unsigned)((blocks + MOE_DIES - 1) / MOE_DIES * MOE_DIES);
+        const long long ws = (long long)(gated ? 2 : 1) * N * K;
+        if (gated) {
+            SPY_DISPATCH(c_dtype, TC, (moe_gemm_group_kernel<true, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (const bf16_t*)W, tile_expert, sorted_pair,
+                                                                                            group, gather, N, K, gy, ws, act)));
+        } else {
+            SPY_DISPATCH(c_dtype, TC, (moe_gemm_group_kernel<false, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (const bf16_t*)W, tile_expert, sorted_pair,
+                                                                                             group, gather, N, K, gy, ws, act)));
+        }
+        SPY_CHECK_LAUNCH("spy_moe_gemm (groups)");
+        return 0;
+    }
     if (tiles_per_block > 0 && a_dtype == SPY_BF16 && w_dtype == SPY_BF16 && K % 8 == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0) {
         const int rc = tiles_per_block >= 8 ? moe_gemm_mfma_launch<8>(C, c_dtype, A, W, tile_expert, sorted_pair, gather, gated, max_tiles, N, K, act, st)
                                             : moe_gemm_mfma_launch<1>(C, c_dtype, A, W, tile_expert, sorted_pair, gather, gated, max_tiles, N, K, act, st);

@@ -78,7 +78,7 @@ class _Hip:
                      "spy_pair_embedding", "spy_norm_residual", "spy_depth_mix", "spy_xielu", "spy_mingru", "spy_latent_prepare",
                      "spy_gemm_strided", "spy_latent_attention", "spy_latent_attention_mfma", "spy_latent_attention_mfma_workspace", "spy_head_products",
                      "spy_bias_rope_store", "spy_sigmoid_gate", "spy_mlstm", "spy_causal_conv_silu", "spy_delta_rule", "spy_moe_route",
-                     "spy_moe_align", "spy_moe_gemm", "spy_moe_combine", "spy_moe_tile_rows", "spy_token_shift", "spy_tanh", "spy_time_mix",
+                     "spy_moe_align", "spy_moe_gemm", "spy_moe_combine", "spy_moe_tile_rows", "spy_moe_group_ints", "spy_token_shift", "spy_tanh", "spy_time_mix",
                      "spy_norm_pair_mean", "spy_scale_cap", "spy_result_norm", "spy_moe_align_tables", "spy_layer_norm", "spy_layer_norm_residual",
                      "spy_gelu", "spy_norm_rope_store", "spy_map_difference", "spy_rotation_angles", "spy_decay_memory", "spy_group_norm"):
             if not hasattr(self.lib, name):
@@ -1854,20 +1854,21 @@ MOE_MFMA = True            # False forces the plain float32 kernel for bfloat16 
 
 class MoEAlignment:
     """A step's (token, choice) pairs of one mixture sorted by expert, on the device: ``sorted_pair`` [tiles * rows of a tile]
-    (the pair of a sorted row, -1: none), ``pair_row`` [T * top] (the row of a pair), ``tile_expert`` [tiles] (-1: no rows)."""
-    __slots__ = ("sorted_pair", "pair_row", "tile_expert", "T", "top", "experts")
+    (the pair of a sorted row, -1: none), ``pair_row`` [T * top] (the row of a pair), ``tile_expert`` [tiles] (-1: no rows), ``groups``
+    (how many groups of neighbouring tiles of one expert there are, then each group)."""
+    __slots__ = ("sorted_pair", "pair_row", "tile_expert", "groups", "T", "top", "experts")
 
-    def __init__(self, sorted_pair, pair_row, tile_expert, T, top, experts):
-        self.sorted_pair, self.pair_row, self.tile_expert = sorted_pair, pair_row, tile_expert
+    def __init__(self, sorted_pair, pair_row, tile_expert, groups, T, top, experts):
+        self.sorted_pair, self.pair_row, self.tile_expert, self.groups = sorted_pair, pair_row, tile_expert, groups
         self.T, self.top, self.experts = T, top, experts
 
 
 def _align_sizes(T: int, top: int, experts: int):
-    """(sorted rows, pairs, tiles) of a mixture's alignment: they follow the numbers of tokens and choices alone."""
+    """(sorted rows, pairs, tiles, ints for the groups) of a mixture's alignment: they follow the numbers of tokens and choices alone."""
     tm = hip().lib.spy_moe_tile_rows()
     P = T * top
     tiles = P // tm + min(experts, P)
-    return tiles * tm, P, tiles
+    return tiles * tm, P, tiles, hip().lib.spy_moe_group_ints(ctypes.c_int(tiles), ctypes.c_int(experts), ctypes.c_int(P))
 
 
 class ExpertTables:
@@ -1909,9 +1910,9 @@ class ExpertTables:
                    ctypes.c_int(max(self.experts)), ctypes.c_int(max(t.shape[1] for t in self.tables)), _ptr(token_ids), ctypes.c_int(T),
                    ctypes.c_int(self.tables[0].shape[0]), _Hip.stream())
         out, at = [], 0
-        for (rows, pairs, tiles), t, e in zip(sizes, self.tables, self.experts):
+        for lengths, t, e in zip(sizes, self.tables, self.experts):
             parts = []
-            for n in (rows, pairs, tiles):
+            for n in lengths:
                 parts.append(buf[at:at + n])
                 at += up4(n)
             out.append(MoEAlignment(*parts, T, t.shape[1], e))
@@ -1970,28 +1971,30 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
     if not T:
         return torch.empty((T, K), dtype=x.dtype, device=x.device)
     dev = x.device
-    rows, P, max_tiles = _align_sizes(T, top, E)
+    rows, P, max_tiles, group_ints = _align_sizes(T, top, E)
     tm = rows // max_tiles
     if align is None:
         sorted_pair = torch.empty((rows,), dtype=torch.int32, device=dev)
         pair_row = torch.empty((P,), dtype=torch.int32, device=dev)
         tile_expert = torch.empty((max_tiles,), dtype=torch.int32, device=dev)
-        hip().call("spy_moe_align", _ptr(sorted_pair), _ptr(pair_row), _ptr(tile_expert), _ptr(ids), ctypes.c_int(P), ctypes.c_int(E),
+        groups = torch.empty((group_ints,), dtype=torch.int32, device=dev)
+        hip().call("spy_moe_align", _ptr(sorted_pair), _ptr(pair_row), _ptr(tile_expert), _ptr(groups), _ptr(ids), ctypes.c_int(P), ctypes.c_int(E),
                    ctypes.c_int(max_tiles), _Hip.stream())
     else:
-        sorted_pair, pair_row, tile_expert = align.sorted_pair, align.pair_row, align.tile_expert
-        _dev(sorted_pair, pair_row, tile_expert)
-        _check(sorted_pair.shape == (rows,) and pair_row.shape == (P,) and tile_expert.shape == (max_tiles,), "moe_experts: the alignment does not fit")
+        sorted_pair, pair_row, tile_expert, groups = align.sorted_pair, align.pair_row, align.tile_expert, align.groups
+        _dev(sorted_pair, pair_row, tile_expert, groups)
+        _check(sorted_pair.shape == (rows,) and pair_row.shape == (P,) and tile_expert.shape == (max_tiles,) and groups.shape == (group_ints,),
+               "moe_experts: the alignment does not fit")
     # bfloat16: the matrix cores, a block taking one row tile of an expert when the experts have few rows (decoding:
     # blocks for the whole device), up to eight when they have many (an expert's matrices are read once per 128 rows)
     per_block = 0 if not MOE_MFMA or x.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16 else (8 if P >= 16 * E else 1)
     act = torch.empty((max_tiles * tm, F), dtype=x.dtype, device=dev)
     hip().call("spy_moe_gemm", _ptr(act), _code(act, "act"), _ptr(x), _code(x, "x"), _ptr(w_gate_up), _code(w_gate_up, "expert matrices"),
-               _ptr(tile_expert), _ptr(sorted_pair), ctypes.c_int(top), ctypes.c_int(1 if gated else 0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(F),
+               _ptr(tile_expert), _ptr(sorted_pair), _ptr(groups), ctypes.c_int(P), ctypes.c_int(top), ctypes.c_int(1 if gated else 0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(F),
                ctypes.c_int(K), ctypes.c_int(per_block), ctypes.c_int(act_kind), ctypes.c_float(limit), _ptr(weights if weight_input else None), _Hip.stream())
     y = torch.empty((max_tiles * tm, K), dtype=torch.float32, device=dev)
     hip().call("spy_moe_gemm", _ptr(y), F32, _ptr(act), _code(act, "act"), _ptr(w_down), _code(w_down, "expert matrices"), _ptr(tile_expert),
-               _ptr(sorted_pair), ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(K), ctypes.c_int(F),
+               _ptr(sorted_pair), _ptr(groups), ctypes.c_int(P), ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(K), ctypes.c_int(F),
                ctypes.c_int(per_block), ctypes.c_int(0), ctypes.c_float(0.0), _ptr(None), _Hip.stream())
     result = ExpertRows(y, pair_row, None if weight_input else weights, add, top, scale, T, x.dtype)
     return result if unsummed else result.combine()

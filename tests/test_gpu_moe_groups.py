@@ -1,0 +1,75 @@
+"""The experts' products over groups of row tiles (csrc/moe.hip, many rows per expert and K in whole steps of 64): one step of K, two,
+an odd number of them, columns that are no multiple of a tile or of four, groups with one row and with 128, experts with more groups
+than a band, experts without rows, every form of the product; against float64."""
+import pytest
+import torch
+
+from tests.gpu_util import close, require_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+def rows_for(kind, E, top, g):
+    """ids [T, top]: how many rows the experts get."""
+    if kind == "even":
+        return torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(40 * E // top)]).int()
+    # the first expert gets every token (more groups than a band), the last none, the others a few
+    T = {"one": 700, "edges": 128}[kind]
+    ids = torch.zeros((T, top), dtype=torch.int32)
+    for t in range(T):
+        ids[t, 1:] = torch.randperm(E - 2, generator=g)[:top - 1].int() + 1
+    return ids
+
+
+@pytest.mark.parametrize("form", ["silu", "clamped", "weighted", "gelu"])
+@pytest.mark.parametrize("kind,E,top,K,F", [("even", 6, 2, 64, 64), ("one", 5, 2, 128, 192), ("edges", 9, 3, 192, 320), ("one", 4, 2, 320, 130), ("even", 7, 3, 256, 67 * 4)])
+def test_products_over_groups(kind, E, top, K, F, form):
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(E + K)
+    ids = rows_for(kind, E, top, g)
+    T, gated = ids.shape[0], form != "gelu"
+    bf = lambda *s, std=1.0: (torch.randn(s, generator=g) * std).bfloat16()
+    x, wgu, wd = bf(T, K), bf(E, (2 if gated else 1) * F, K, std=K ** -0.5), bf(E, K, F, std=F ** -0.5)
+    w = torch.rand((T, top), generator=g)
+    assert T * top >= 16 * E
+    kw = dict(silu={}, clamped=dict(activation="clamped", limit=0.8), weighted=dict(activation="clamped", limit=0.8, weight_input=True), gelu=dict(activation="gelu"))[form]
+    out = ops.moe_experts(x.to(dev), ids.to(dev), w.to(dev), wgu.to(dev), wd.to(dev), **kw)
+    ref = torch.zeros((T, K), dtype=torch.float64)
+    xd, wgud, wdd = x.double(), wgu.double(), wd.double()
+    for e in range(E):
+        for j in range(top):
+            at = (ids[:, j] == e).nonzero()[:, 0]
+            scale = w[at, j].double()[:, None]
+            h = xd[at] @ wgud[e].T * (scale if form == "weighted" else 1.0)
+            if form == "gelu":
+                a = torch.nn.functional.gelu(h)
+            elif form == "silu":
+                a = torch.nn.functional.silu(h[:, :F]) * h[:, F:]
+            else:
+                gate, up = h[:, :F].clamp(max=0.8), h[:, F:].clamp(-0.8, 0.8)
+                a = gate * torch.sigmoid(1.702 * gate) * (up + 1.0)
+            ref[at] += (a @ wdd[e].T) * (1.0 if form == "weighted" else scale)
+    close(out, ref, torch.bfloat16, scale=2.0, what="experts over groups")
+
+
+def test_groups_of_an_alignment():
+    """Every sorted row of an expert lies in one group, groups begin every eight tiles of an expert, bands hold up to four of them."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(5)
+    for T, E, top in ((1, 1, 1), (3, 7, 2), (900, 3, 1), (700, 40, 3)):
+        routes = ops.ExpertTables()
+        table = torch.rand((11, E), generator=g).argsort(dim=1)[:, :top].to(torch.int32).contiguous()
+        routes.add(table.to(dev), E)
+        al = routes.align(torch.randint(0, 11, (T,), generator=g, dtype=torch.int32).to(dev))[0]
+        te, gr = al.tile_expert.cpu().tolist(), al.groups.cpu().tolist()
+        seen, n = [], gr[0]
+        assert 1 + 2 * n <= len(gr)
+        for i in range(n):
+            tile, tiles, first, in_band = gr[1 + 2 * i] >> 4, gr[1 + 2 * i] & 15, gr[2 + 2 * i] >> 3, gr[2 + 2 * i] & 7
+            assert 1 <= tiles <= 8 and len({te[t] for t in range(tile, tile + tiles)}) == 1 and te[tile] >= 0
+            assert first <= i < first + in_band and 1 <= in_band <= 4
+            assert all(te[gr[1 + 2 * j] >> 4] == te[tile] for j in range(first, first + in_band))
+            seen += list(range(tile, tile + tiles))
+        assert seen == [t for t, e in enumerate(te) if e >= 0]
