@@ -1,0 +1,278 @@
+// The gated delta rule, S = diag(g) S; u = beta (v - S^T k); S = S + k u^T; o = S^T q, over chunks of 16 tokens.
+//
+// Token by token (matrix_memory.hip) its time is tokens times the length of one token's chain, 1.1 us.  Within a chunk that starts
+// from S0, with G_t the product of the decays up to t (per key channel, from the chunk's start):
+//   S_t = diag(G_t) S0 + sum_{s <= t} diag(G_t / G_s) k_s u_s^T
+//   u_t = beta_t (v_t - S0^T (G_t k_t) - sum_{s < t} A_ts u_s),   A_ts = sum_c k_t[c] k_s[c] G_t[c] / G_s[c]
+//   o_t = S0^T (G_t q_t) + sum_{s <= t} B_ts u_s,                 B_ts = sum_c q_t[c] k_s[c] G_t[c] / G_s[c]
+// so with M = (I + diag(beta) A)^-1 diag(beta), lower triangular, u = M V - (M W) S0 with W_t = G_t k_t.  Everything but the products
+// with S0 is known for all chunks at once:
+//   delta_chunk_prepare   a block per (chunk, head): A, B, M and from them MV = M V, MW = M W, Q_t = G_t q_t, K_s = G_15 / G_s k_s (stored
+//                         [channel][token]), G_15, into a workspace.  The quotients of decays are never formed as quotients, which
+//                         underflow: they are powers of two of differences of sums of logarithms, sums in 64 bits.
+//   delta_chunk_walk      a block of four waves per (entry, head, 16 value channels); a wave has a quarter of the key channels' rows of
+//                         S in registers.  Per chunk, on v_mfma_f32_16x16x4_f32: its part of MW S0 and of Q S0, the parts of u met in
+//                         LDS, S = G_15 S + K^T u, and B u for the read-out, whose parts meet one chunk later.
+// The result's layout (lane (column r, g): rows 4 g + i) is the second operand's layout of the next product, so S and u go from product to
+// product without a move.  All of it is float32 (the sums of logarithms float64), as the token walk is.
+// What bounds it: the walk's chain of about 1000 cycles a chunk (8 products, LDS, 8 products), 94 times for 1500 tokens; the preparation's
+// 136 x d powers of two a chunk.  Chunks of 16 because a chunk's tokens are then one matrix tile; the preparation grows with the square.
+// Measured: 1500 tokens, 16 heads of 128 x 128: 51 us of preparation and 104 us of walk a layer against 1712 us token by token.
+#include "delta_chunks.h"
+#include <math.h>
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float dc_f32x4_t;
+
+#define DC_TOKENS 16
+#define DC_SEGMENT 128           // chunks that are prepared and walked at a time: bounds the workspace
+
+// An entry's chunks have neighbouring numbers from cu_q[e] / 16 + e on (entries' ranges cannot meet: they have at most
+// cu_q[e + 1] / 16 - cu_q[e] / 16 + 1 chunks); some numbers belong to nobody.
+__device__ __forceinline__ int dc_first(const int* cu_q, int e) { return cu_q[e] / DC_TOKENS + e; }
+static int64_t dc_numbers(int S, int T) { return (int64_t)T / DC_TOKENS + S; }
+
+// floats of one (chunk, head) in the workspace: MW [16][d], Q [16][d], K [d][16], MV [16][dv], B [16][16], G [d]
+__device__ __host__ __forceinline__ int dc_record(int d, int dv) { return 48 * d + 16 * dv + 256 + d; }
+
+__device__ __forceinline__ float dc_pow2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+template <typename TA, int D>
+__global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunks a, int number0) {
+    __shared__ __align__(16) float kk[16][D + 4], qq[16][D + 4];
+    __shared__ __align__(16) double ll[16][D + 2];
+    __shared__ __align__(16) float A[16][20], M[16][20];
+    __shared__ float beta[16];
+    __shared__ int entry;
+    const int number = number0 + blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+    if (tid == 0) entry = -1;
+    __syncthreads();
+    for (int e = tid; e < a.S; e += 256) {
+        const int f = dc_first(a.cu_q, e), n = a.cu_q[e + 1] - a.cu_q[e];
+        if (number >= f && number < f + (n + DC_TOKENS - 1) / DC_TOKENS) entry = e;
+    }
+    __syncthreads();
+    if (entry < 0) return;
+    const int t0 = a.cu_q[entry] + (number - dc_first(a.cu_q, entry)) * DC_TOKENS, n = min(DC_TOKENS, a.cu_q[entry + 1] - t0);
+    const int g = h / (a.H / a.G);
+    // tokens beyond the entry's end: k, q, v and beta zero, no decay
+    for (int i = tid; i < 16 * D; i += 256) {
+        const int t = i / D, c = i % D;
+        const float* row = a.qk + (size_t)(t0 + t) * 2 * a.G * D + c;
+        qq[t][c] = t < n ? row[(size_t)g * D] : 0.f;
+        kk[t][c] = t < n ? row[(size_t)(a.G + g) * D] : 0.f;
+        const float z = t < n ? a.dec[(size_t)(t0 + t) * a.zs + (size_t)h * a.dd + (a.dd == 1 ? 0 : c)] : 1.f;
+        const float l = log2f(z);
+        ll[t][c] = (double)(l < -1e5f ? -1e5f : l);         // (a decay of zero is 2^-100000: zero in every product, and differences stay numbers)
+    }
+    if (tid < 16) beta[tid] = tid < n ? a.beta[(size_t)(t0 + tid) * a.bs + h] : 0.f;
+    __syncthreads();
+    if (tid < D) {
+        double sum = 0.0;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            sum += ll[t][tid];
+            ll[t][tid] = sum;
+        }
+    }
+    __syncthreads();
+    float* out = a.ws + ((size_t)blockIdx.x * a.H + h) * dc_record(D, a.dv);
+    float* o_mw = out;
+    float* o_q = o_mw + 16 * D;
+    float* o_k = o_q + 16 * D;
+    float* o_mv = o_k + 16 * D;
+    float* o_b = o_mv + 16 * a.dv;
+    float* o_g = o_b + 256;
+    {   // thread (t, s): A and B of the pair
+        const int t = tid >> 4, s = tid & 15;
+        float x = 0.f, y = 0.f;
+        if (s <= t) {
+            for (int c = 0; c < D; c += 4) {
+                const dc_f32x4_t kt = *reinterpret_cast<const dc_f32x4_t*>(&kk[t][c]), ks = *reinterpret_cast<const dc_f32x4_t*>(&kk[s][c]);
+                const dc_f32x4_t qt = *reinterpret_cast<const dc_f32x4_t*>(&qq[t][c]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float w = ks[e] * dc_pow2((float)(ll[t][c + e] - ll[s][c + e]));
+                    x = fmaf(kt[e], w, x);
+                    y = fmaf(qt[e], w, y);
+                }
+            }
+        }
+        A[t][s] = s < t ? x : 0.f;
+        o_b[t * 16 + s] = y;                                // (zero above the diagonal)
+    }
+    __syncthreads();
+    if (tid < 16) {                                         // column tid of M, forwards
+        float m[16];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            float x = t == tid ? 1.f : 0.f;
+#pragma unroll
+            for (int s = 0; s < t; ++s) x = fmaf(-A[t][s], m[s], x);
+            m[t] = beta[t] * x;
+            M[t][tid] = m[t];
+        }
+    }
+    __syncthreads();
+    // a thread per column of W or V: the column of M W or M V
+    for (int i = tid; i < D + a.dv; i += 256) {
+        float x[16];
+        if (i < D) {
+#pragma unroll
+            for (int s = 0; s < 16; ++s) x[s] = kk[s][i] * dc_pow2((float)ll[s][i]);
+        } else {
+            const TA* v = (const TA*)a.qkv + (size_t)t0 * (2 * a.G * D + a.H * a.dv) + 2 * a.G * D + (size_t)h * a.dv + (i - D);
+#pragma unroll
+            for (int s = 0; s < 16; ++s) x[s] = s < n ? to_f32<TA>(v[(size_t)s * (2 * a.G * D + a.H * a.dv)]) : 0.f;
+        }
+        float* to = i < D ? o_mw + i : o_mv + (i - D);
+        const int ld = i < D ? D : a.dv;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            float y = 0.f;
+#pragma unroll
+            for (int s = 0; s <= t; ++s) y = fmaf(M[t][s], x[s], y);
+            to[(size_t)t * ld] = y;
+        }
+    }
+    for (int i = tid; i < 16 * D; i += 256) {
+        o_q[i] = qq[i / D][i % D] * dc_pow2((float)ll[i / D][i % D]);
+        const int c = i / 16, s = i % 16;
+        o_k[i] = kk[s][c] * dc_pow2((float)(ll[15][c] - ll[s][c]));
+    }
+    if (tid < D) o_g[tid] = dc_pow2((float)ll[15][tid]);
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void delta_chunk_walk_kernel(DeltaChunks a, int number0, int number1) {
+    constexpr int TI = D / 64;                              // tiles of 16 key channels that a wave has
+    __shared__ __align__(16) float pu[2][4][64][4], po[2][4][64][4];
+    const int e = blockIdx.x, h = blockIdx.y, col0 = blockIdx.z * 16;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int slot = a.slot_ids[e];
+    if (slot < 0 || slot >= a.num_slots) return;
+    const int q0 = a.cu_q[e], q1 = a.cu_q[e + 1], first = dc_first(a.cu_q, e), chunks = (q1 - q0 + DC_TOKENS - 1) / DC_TOKENS;
+    const int c0 = max(0, number0 - first), c1 = min(chunks, number1 - first);
+    if (c0 >= c1) return;
+    const int row0 = wave * (D / 4) + 4 * g;                // lane (column r, g) has rows row0 + 16 i + e
+    float* st = a.state + (size_t)slot * a.state_stride + (size_t)h * D * a.dv + col0 + r;
+    dc_f32x4_t S[TI];
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) S[i][x] = st[(size_t)(row0 + 16 * i + x) * a.dv];
+    const int rec = dc_record(D, a.dv);
+    // this lane's operands of a chunk
+    struct Ops { dc_f32x4_t mw[TI], q[TI], k[TI], gl[TI], b, mv; };
+    auto load = [&](Ops& x, int c) {
+        const float* p = a.ws + ((size_t)(first + min(c, c1 - 1) - number0) * a.H + h) * rec;
+        const float* mv = p + 48 * D + 4 * g * a.dv + col0 + r;
+#pragma unroll
+        for (int i = 0; i < TI; ++i) {
+            x.mw[i] = *reinterpret_cast<const dc_f32x4_t*>(p + r * D + row0 + 16 * i);
+            x.q[i] = *reinterpret_cast<const dc_f32x4_t*>(p + 16 * D + r * D + row0 + 16 * i);
+            x.k[i] = *reinterpret_cast<const dc_f32x4_t*>(p + 32 * D + (row0 - 4 * g + 16 * i + r) * 16 + 4 * g);
+            x.gl[i] = *reinterpret_cast<const dc_f32x4_t*>(p + 48 * D + 16 * a.dv + 256 + row0 + 16 * i);
+        }
+        x.b = *reinterpret_cast<const dc_f32x4_t*>(p + 48 * D + 16 * a.dv + r * 16 + 4 * g);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x.mv[i] = mv[(size_t)i * a.dv];
+    };
+    // read-out of chunk c: the waves' parts, row 4 g + wave of lane (column r, g)
+    auto read_out = [&](int c) {
+        const int t = q0 + c * DC_TOKENS + 4 * g + wave;
+        float y = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) y += po[c & 1][w][lane][wave];
+        if (t < q1) a.o[((size_t)t * a.H + h) * a.dv + col0 + r] = y;
+    };
+    auto chunk = [&](const Ops& x, int c) {
+        dc_f32x4_t u0 = {0.f, 0.f, 0.f, 0.f}, u1 = {0.f, 0.f, 0.f, 0.f}, o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < TI; ++i) {
+#pragma unroll
+            for (int j = 0; j < 4; j += 2) {
+                u0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[i][j], S[i][j], u0, 0, 0, 0);
+                u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[i][j + 1], S[i][j + 1], u1, 0, 0, 0);
+            }
+        }
+        *reinterpret_cast<dc_f32x4_t*>(pu[c & 1][wave][lane]) = u0 + u1;
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; j += 2) {
+                o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][j], S[i][j], o0, 0, 0, 0);
+                o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][j + 1], S[i][j + 1], o1, 0, 0, 0);
+            }
+        __syncthreads();                                    // parts of u of this chunk, and of the read-out of the chunk before
+        dc_f32x4_t u = x.mv;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) u -= *reinterpret_cast<const dc_f32x4_t*>(pu[c & 1][w][lane]);
+#pragma unroll
+        for (int i = 0; i < TI; ++i) S[i] *= x.gl[i];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < TI; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i][j], u[j], S[i], 0, 0, 0);
+        // of B u, this wave's share: tokens s = 4 g + wave
+        float bw = x.b[0], uw = u[0];
+#pragma unroll
+        for (int j = 1; j < 4; ++j)
+            if (wave == j) { bw = x.b[j]; uw = u[j]; }
+        // (B is zero where a token does not read: infinities and NaN, which zero does not take away, go to the rows that do read them)
+        const bool odd = !(fabsf(uw) < INFINITY);
+        if (__any(odd)) {
+            const dc_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+            const dc_f32x4_t f = __builtin_amdgcn_mfma_f32_16x16x4f32(4 * g + wave <= r ? 1.f : 0.f, odd ? 1.f : 0.f, zero, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (f[i] > 0.f) o0[i] = __builtin_nanf("");
+            if (odd) uw = 0.f;
+        }
+        o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(bw, uw, o0, 0, 0, 0);
+        if (c > c0) read_out(c - 1);
+        // (the place was read for chunk c - 2 behind the barrier of chunk c - 1, which every wave has passed)
+        *reinterpret_cast<dc_f32x4_t*>(po[c & 1][wave][lane]) = o0 + o1;
+    };
+    Ops x0, x1;
+    load(x0, c0);
+    int c = c0;
+    for (; c + 2 <= c1; c += 2) {
+        load(x1, c + 1);
+        chunk(x0, c);
+        load(x0, c + 2);
+        chunk(x1, c + 1);
+    }
+    if (c < c1) chunk(x0, c);
+    __syncthreads();
+    read_out(c1 - 1);
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) st[(size_t)(row0 + 16 * i + y) * a.dv] = S[i][y];
+}
+
+bool delta_chunks_takes(int S, int T, int d, int dv) { return T > S && (d == 64 || d == 128) && dv % 16 == 0; }
+
+int64_t delta_chunks_workspace(int S, int T, int H, int d, int dv) {
+    const int64_t n = dc_numbers(S, T);
+    return (n < DC_SEGMENT ? n : DC_SEGMENT) * H * dc_record(d, dv);
+}
+
+int delta_chunks(const DeltaChunks& a, int dtype, hipStream_t st) {
+    SPY_REQUIRE(a.ws && a.ws_floats >= delta_chunks_workspace(a.S, a.T, a.H, a.d, a.dv), "delta rule: the chunks' workspace is too small");
+    SPY_REQUIRE(((uintptr_t)a.ws % 16) == 0 && a.H <= 65535 && a.dv / 16 <= 65535, "delta rule: workspace alignment or heads");
+    const int64_t numbers = dc_numbers(a.S, a.T);
+    for (int64_t n0 = 0; n0 < numbers; n0 += DC_SEGMENT) {
+        const int n1 = (int)(n0 + DC_SEGMENT < numbers ? n0 + DC_SEGMENT : numbers);
+        const dim3 pgrid((unsigned)(n1 - n0), a.H), wgrid(a.S, a.H, a.dv / 16);
+        if (a.d == 64) {
+            SPY_DISPATCH(dtype, TA, (delta_chunk_prepare_kernel<TA, 64><<<pgrid, 256, 0, st>>>(a, (int)n0)));
+            delta_chunk_walk_kernel<64><<<wgrid, 256, 0, st>>>(a, (int)n0, n1);
+        } else {
+            SPY_DISPATCH(dtype, TA, (delta_chunk_prepare_kernel<TA, 128><<<pgrid, 256, 0, st>>>(a, (int)n0)));
+            delta_chunk_walk_kernel<128><<<wgrid, 256, 0, st>>>(a, (int)n0, n1);
+        }
+        SPY_CHECK_LAUNCH("spy_delta_rule (chunks)");
+    }
+    return 0;
+}

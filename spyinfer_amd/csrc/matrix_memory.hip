@@ -12,6 +12,7 @@
 //                vectors; then o / rms(o) * w * sigmoid(gate).
 //   causal_conv_silu: the short convolution over time that feeds the delta rule, with its last inputs kept per request.
 #include "common.h"
+#include "delta_chunks.h"
 #include <math.h>
 
 __device__ __forceinline__ float mm_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
@@ -694,10 +695,16 @@ __global__ __launch_bounds__(MM_SLICE) void delta_rule_kernel(
         if (col && row0 + i < d) st[(size_t)(row0 + i) * dv + j] = S[i];
 }
 
+// floats of workspace that a step of S entries and T tokens needs (0: it walks token by token)
+extern "C" int64_t spy_delta_rule_workspace(int S, int T, int H, int d, int dv) {
+    return delta_chunks_takes(S, T, d, dv) ? delta_chunks_workspace(S, T, H, d, dv) : 0;
+}
+
 extern "C" int spy_delta_rule(void* out, float* o_tmp, float* qk_tmp, float* state, long long state_stride, const void* qkv, int dtype,
                               float* beta_pre, float* dec_pre, const void* a_log, const void* dt_bias, int w_dtype, const void* gate, long long gs,
                               const void* norm_w, float eps, const int* cu_q, const int* slot_ids, int num_slots, int S, int T, int H,
-                              int G, int d, int dv, int dd, int silu_gate, long long bs, long long zs, hipStream_t st) {
+                              int G, int d, int dv, int dd, int silu_gate, long long bs, long long zs, float* ws, int64_t ws_floats,
+                              hipStream_t st) {
     SPY_REQUIRE(S > 0 && T > 0 && H > 0 && G > 0 && H % G == 0 && d > 0 && dv > 0 && num_slots > 0 && o_tmp, "spy_delta_rule: empty operand");
     SPY_REQUIRE(dd == d || dd == 1, "spy_delta_rule: %d decays for a head of %d key channels (one, or one per channel)", dd, d);
     SPY_REQUIRE(bs >= H && zs >= (long long)H * dd, "spy_delta_rule: rows of beta or of the decays are too short");
@@ -708,10 +715,18 @@ extern "C" int spy_delta_rule(void* out, float* o_tmp, float* qk_tmp, float* sta
     SPY_DISPATCH(dtype, TA, SPY_DISPATCH(w_dtype, TW, (delta_prepare_kernel<TA, TW><<<pgrid, 64, 0, st>>>(
         qk_tmp, (const TA*)qkv, beta_pre, dec_pre, (const TW*)a_log, (const TW*)dt_bias, H, G, d, dv, dd, bs, zs))));
     SPY_CHECK_LAUNCH("spy_delta_rule (unit vectors and decays)");
-    const dim3 grid(S, H, (dv + MM_COLS - 1) / MM_COLS);
-    SPY_DISPATCH(dtype, TA, SPY_DISPATCH(w_dtype, TW, MM_LAUNCH(delta_rule_kernel, o_tmp, state, state_stride, (const TA*)qkv, qk_tmp, beta_pre,
-        dec_pre, cu_q, slot_ids, num_slots, H, G, d, dv, dd, bs, zs)));
-    SPY_CHECK_LAUNCH("spy_delta_rule");
+    // Steps of single tokens, and head sizes that are no whole matrix tiles, walk token by token; in the others every entry, also one of a
+    // single token, goes by chunks (a chunk's chain costs about what one token's does).
+    if (delta_chunks_takes(S, T, d, dv)) {
+        const DeltaChunks a = {o_tmp, state, state_stride, qkv, qk_tmp, beta_pre, dec_pre, cu_q, slot_ids, num_slots, S, T, H, G, d, dv, dd, bs, zs, ws, ws_floats};
+        const int rc = delta_chunks(a, dtype, st);
+        if (rc) return rc;
+    } else {
+        const dim3 grid(S, H, (dv + MM_COLS - 1) / MM_COLS);
+        SPY_DISPATCH(dtype, TA, SPY_DISPATCH(w_dtype, TW, MM_LAUNCH(delta_rule_kernel, o_tmp, state, state_stride, (const TA*)qkv, qk_tmp, beta_pre,
+            dec_pre, cu_q, slot_ids, num_slots, H, G, d, dv, dd, bs, zs)));
+        SPY_CHECK_LAUNCH("spy_delta_rule");
+    }
     const dim3 ngrid(T, H);
     const int nthreads = dv >= 256 ? 256 : 64;
     SPY_DISPATCH(dtype, TA, SPY_DISPATCH(w_dtype, TW, (head_norm_gate_kernel<TA, TW><<<ngrid, nthreads, 0, st>>>(

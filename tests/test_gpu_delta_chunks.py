@@ -1,0 +1,87 @@
+"""The gated delta rule over chunks of 16 tokens (csrc/delta_chunks.hip): entries of every length around a chunk and a few chunks, one
+long enough for several segments, single tokens beside them, states carried from step to step, decays from none to all, one decay per
+head and one per channel; against the recurrence in float64, token by token."""
+import pytest
+import torch
+
+from tests.gpu_util import require_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+def walk(q, k, v, beta, decay, S):
+    """One head: q, k, decay [T, d], v [T, dv], beta [T], S [d, dv] -> (o [T, dv], S)."""
+    out = []
+    for t in range(q.shape[0]):
+        S = decay[t][:, None] * S
+        u = beta[t] * (v[t] - S.T @ k[t])
+        S = S + torch.outer(k[t], u)
+        out.append(S.T @ q[t])
+    return torch.stack(out), S
+
+
+def unit(x):
+    return x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6)
+
+
+# heads, kv heads, key size, value size, decays per head (0: one per channel), lengths of the steps' entries
+CASES = [(2, 1, 128, 128, 0, [(1, 17), (16, 31)]), (4, 2, 64, 48, 0, [(15, 1, 40), (2, 33, 1)]), (3, 3, 128, 16, 1, [(50, 5), (1, 1), (64, 2)]),
+         (1, 1, 64, 32, 0, [(2300,), (7,)]), (2, 2, 128, 32, 1, [(1, 1, 1, 1, 2)])]
+
+
+@pytest.mark.parametrize("how", ["slow", "fast", "mixed"])
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_chunks_against_the_recurrence(case, how):
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    H, G, d, dv, per_head, steps = CASES[case]
+    if case == 3 and how != "slow":
+        pytest.skip("the long entry once")
+    dd = 1 if per_head else d
+    g = torch.Generator().manual_seed(10 * case + len(how))
+    slots, slot_ids = len(steps[0]) + 1, torch.randperm(len(steps[0]) + 1, generator=g)[:len(steps[0])].int()
+    state = torch.randn(slots, H * d * dv + 8, generator=g) * 0.1
+    S = [[state[int(s), h * d * dv:(h + 1) * d * dv].double().view(d, dv) for h in range(H)] for s in slot_ids]
+    untouched = state[[i for i in range(slots) if i not in slot_ids.tolist()]].clone()
+    state_dev = state.to(dev)
+    a_log, dtb, nw = torch.rand(H, generator=g), torch.randn(H * dd, generator=g) * 0.1, 1.0 + 0.1 * torch.randn(dv, generator=g)
+    for lens in steps:
+        T = sum(lens)
+        qkv = torch.randn(T, 2 * G * d + H * dv, generator=g)
+        beta_pre = torch.randn(T, H, generator=g)
+        # slow: decays near one; fast: most of the state is gone after a token; mixed: some channels of some tokens lose everything
+        dec_pre = torch.randn(T, H * dd, generator=g) + {"slow": -6.0, "fast": 2.0, "mixed": -4.0}[how]
+        if how == "mixed":
+            dec_pre = torch.where(torch.rand(dec_pre.shape, generator=g) < 0.1, torch.full_like(dec_pre, 300.0), dec_pre)
+        gate = torch.randn(T, H * dv, generator=g)
+        cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+        y = ops.delta_rule(qkv.to(dev), beta_pre.clone().to(dev), dec_pre.clone().to(dev), a_log.to(dev), dtb.to(dev), gate.to(dev), nw.to(dev), 1e-6,
+                           state_dev, cu.to(dev), slot_ids.to(dev), H, G, d, dv).cpu().double().view(T, H, dv)
+        x = qkv.double()
+        q, k = unit(x[:, :G * d].view(T, G, d)) * d ** -0.5, unit(x[:, G * d:2 * G * d].view(T, G, d))
+        v, beta = x[:, 2 * G * d:].view(T, H, dv), torch.sigmoid(beta_pre.double())
+        dt = torch.nn.functional.softplus(dec_pre.double() + dtb.double()).view(T, H, dd).expand(T, H, d)
+        decay = torch.exp(-torch.exp(a_log.double())[None, :, None] * dt)
+        for e, n in enumerate(lens):
+            at = slice(int(cu[e]), int(cu[e + 1]))
+            for h in range(H):
+                o, S[e][h] = walk(q[at, h // (H // G)], k[at, h // (H // G)], v[at, h], beta[at, h], decay[at, h], S[e][h])
+                ref = o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-6) * nw.double() * torch.sigmoid(gate[at].double().view(n, H, dv)[:, h])
+                # float32 sums of up to 2 d terms of size one, over a root mean square: a few hundred roundings of 2^-24 of the largest
+                assert float((y[at, h] - ref).abs().max()) < 2e-5 * max(1.0, float(ref.abs().max())), (e, h, n)
+                got = state_dev[int(slot_ids[e]), h * d * dv:(h + 1) * d * dv].cpu().double().view(d, dv)
+                assert float((got - S[e][h]).abs().max()) < 1e-5 * max(1.0, float(S[e][h].abs().max())), (e, h, n)
+    assert torch.equal(state_dev.cpu()[[i for i in range(slots) if i not in slot_ids.tolist()]], untouched)
+
+
+def test_an_infinite_value_stays_with_the_tokens_that_read_it():
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(1)
+    T, d, dv = 40, 64, 16
+    qkv = torch.randn(T, 2 * d + dv, generator=g)
+    qkv[21, 2 * d + 3] = float("inf")
+    cu, slot = torch.tensor([0, T], dtype=torch.int32).to(dev), torch.zeros(1, dtype=torch.int32).to(dev)
+    ones = lambda *s: torch.ones(*s, device=dev)
+    y = ops.delta_rule(qkv.to(dev), ones(T, 1) * 0.3, ones(T, d) * -3, ones(1), ones(d), ones(T, dv), ones(dv), 1e-6, torch.zeros(1, d * dv, device=dev), cu, slot, 1, 1, d, dv)
+    assert bool(y[:21].isfinite().all()) and not bool(y[21:].isfinite().all(dim=1).any())
