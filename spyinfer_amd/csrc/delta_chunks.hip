@@ -18,6 +18,10 @@
 // What bounds it: the walk's chain of about 1000 cycles a chunk (8 products, LDS, 8 products), 94 times for 1500 tokens; the preparation's
 // 136 x d powers of two a chunk.  Chunks of 16 because a chunk's tokens are then one matrix tile; the preparation grows with the square.
 // Measured: 1500 tokens, 16 heads of 128 x 128: 51 us of preparation and 104 us of walk a layer against 1712 us token by token.
+// The mLSTM, S = a S + b k v^T with numbers a and b a token, is the same with nothing taken back: u = v, B_ts = b_s G_t / G_s (q_t . k_s), K_s =
+// b_s G_15 / G_s k_s, and its vector n = a n + b k goes along in the lanes' registers (a lane has the rows of n that it has of Q as an
+// operand, so n . q costs eight products a lane).  8 heads of 128 x 256, 1500 tokens: 190 us
+// a layer, scalars and preparation among it, against 765 for pieces of 64 tokens walked twice and folded.
 #include "delta_chunks.h"
 #include <math.h>
 
@@ -36,21 +40,27 @@ __device__ __host__ __forceinline__ int dc_record(int d, int dv) { return 48 * d
 
 __device__ __forceinline__ float dc_pow2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// The entry that chunk `number` is of, by all threads of a block together; -1: nobody's
+__device__ __forceinline__ int dc_entry(const int* cu_q, int S, int number, int* shared) {
+    if (threadIdx.x == 0) *shared = -1;
+    __syncthreads();
+    for (int e = threadIdx.x; e < S; e += 256) {
+        const int f = dc_first(cu_q, e), n = cu_q[e + 1] - cu_q[e];
+        if (number >= f && number < f + (n + DC_TOKENS - 1) / DC_TOKENS) *shared = e;
+    }
+    __syncthreads();
+    return *shared;
+}
+
 template <typename TA, int D>
 __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunks a, int number0) {
     __shared__ __align__(16) float kk[16][D + 4], qq[16][D + 4];
     __shared__ __align__(16) double ll[16][D + 2];
     __shared__ __align__(16) float A[16][20], M[16][20];
     __shared__ float beta[16];
-    __shared__ int entry;
+    __shared__ int shared;
     const int number = number0 + blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
-    if (tid == 0) entry = -1;
-    __syncthreads();
-    for (int e = tid; e < a.S; e += 256) {
-        const int f = dc_first(a.cu_q, e), n = a.cu_q[e + 1] - a.cu_q[e];
-        if (number >= f && number < f + (n + DC_TOKENS - 1) / DC_TOKENS) entry = e;
-    }
-    __syncthreads();
+    const int entry = dc_entry(a.cu_q, a.S, number, &shared);
     if (entry < 0) return;
     const int t0 = a.cu_q[entry] + (number - dc_first(a.cu_q, entry)) * DC_TOKENS, n = min(DC_TOKENS, a.cu_q[entry + 1] - t0);
     const int g = h / (a.H / a.G);
@@ -142,10 +152,100 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(DeltaChunks a,
     if (tid < D) o_g[tid] = dc_pow2((float)ll[15][tid]);
 }
 
-template <int D>
-__global__ __launch_bounds__(256) void delta_chunk_walk_kernel(DeltaChunks a, int number0, int number1) {
+// The mLSTM's chunks: the same records, with the sum of K over the chunk's tokens [d], the sums of B's rows [16] and e^-m [16] in MW's place.
+template <typename TA, int D>
+__global__ __launch_bounds__(256) void memory_chunk_prepare_kernel(MemoryChunks a, int number0) {
+    __shared__ __align__(16) float kk[16][D + 4], qq[16][D + 4];
+    __shared__ __align__(16) float B[16][20];
+    __shared__ double ll[16];
+    __shared__ float b[16];
+    __shared__ int shared;
+    const int number = number0 + blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+    const int entry = dc_entry(a.cu_q, a.S, number, &shared);
+    if (entry < 0) return;
+    const int t0 = a.cu_q[entry] + (number - dc_first(a.cu_q, entry)) * DC_TOKENS, n = min(DC_TOKENS, a.cu_q[entry + 1] - t0);
+    const float qscale = 1.0f / sqrtf((float)D);
+    for (int i = tid; i < 16 * D; i += 256) {
+        const int t = i / D, c = i % D;
+        const TA* row = (const TA*)a.x + (size_t)(t0 + t) * a.xs + (size_t)h * D + c;
+        qq[t][c] = t < n ? to_f32<TA>(row[a.q_off]) * qscale : 0.f;
+        kk[t][c] = t < n ? to_f32<TA>(row[a.k_off]) : 0.f;
+    }
+    float* out = a.ws + ((size_t)blockIdx.x * a.H + h) * dc_record(D, a.dv);
+    float* o_q = out + 16 * D;
+    float* o_k = o_q + 16 * D;
+    float* o_v = o_k + 16 * D;
+    float* o_b = o_v + 16 * a.dv;
+    float* o_g = o_b + 256;
+    if (tid < 16) {
+        const float* g = a.abe + (size_t)(t0 + tid) * 3 * a.H + h;
+        const float l = tid < n ? log2f(g[0]) : 0.f;
+        double sum = (double)(l < -1e5f ? -1e5f : l);
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) {
+            const double x = __shfl_up(sum, o, 16);
+            if (tid >= o) sum += x;
+        }
+        ll[tid] = sum;
+        b[tid] = tid < n ? g[a.H] : 0.f;
+        out[D + 16 + tid] = tid < n ? g[2 * a.H] : 1.f;
+    }
+    __syncthreads();
+    {
+        const int t = tid >> 4, s = tid & 15;
+        float y = 0.f, y2 = 0.f;
+        if (s <= t) {
+            for (int c = 0; c < D; c += 4) {
+                const dc_f32x4_t qt = *reinterpret_cast<const dc_f32x4_t*>(&qq[t][c]), ks = *reinterpret_cast<const dc_f32x4_t*>(&kk[s][c]);
+                y = fmaf(qt[0], ks[0], y); y2 = fmaf(qt[1], ks[1], y2);
+                y = fmaf(qt[2], ks[2], y); y2 = fmaf(qt[3], ks[3], y2);
+            }
+            y = (y + y2) * (b[s] * dc_pow2((float)(ll[t] - ll[s])));
+        }
+        o_b[t * 16 + s] = y;
+        B[t][s] = y;
+    }
+    for (int i = tid; i < 16 * D; i += 256) {
+        o_q[i] = qq[i / D][i % D] * dc_pow2((float)ll[i / D]);
+        const int c = i / 16, s = i % 16;
+        o_k[i] = kk[s][c] * (b[s] * dc_pow2((float)(ll[15] - ll[s])));
+    }
+    for (int i = tid; i < 16 * a.dv; i += 256) {
+        const int t = i / a.dv, c = i % a.dv;
+        o_v[i] = t < n ? to_f32<TA>(((const TA*)a.x)[(size_t)(t0 + t) * a.xs + a.v_off + (size_t)h * a.dv + c]) : 0.f;
+    }
+    if (tid < D) {
+        o_g[tid] = dc_pow2((float)ll[15]);
+        float sum = 0.f;
+#pragma unroll
+        for (int s = 0; s < 16; ++s) sum = fmaf(kk[s][tid], b[s] * dc_pow2((float)(ll[15] - ll[s])), sum);
+        out[tid] = sum;
+    }
+    __syncthreads();
+    if (tid < 16) {
+        float sum = 0.f;
+        for (int s = 0; s <= tid; ++s) sum += B[tid][s];
+        out[D + tid] = sum;
+    }
+}
+
+// What the walk needs of either recurrence
+struct ChunkWalk {
+    float* o;
+    float* state;
+    long long slot_stride, head_stride;
+    const float* mfin;
+    const int* cu_q;
+    const int* slot_ids;
+    int num_slots, H, dv;
+    const float* ws;
+};
+
+template <int D, bool DELTA>
+__global__ __launch_bounds__(256) void chunk_walk_kernel(ChunkWalk a, int number0, int number1) {
     constexpr int TI = D / 64;                              // tiles of 16 key channels that a wave has
-    __shared__ __align__(16) float pu[2][4][64][4], po[2][4][64][4];
+    __shared__ __align__(16) float pu[DELTA ? 2 : 1][4][64][4], po[2][4][64][4];
+    __shared__ float pn[2][4][16];
     const int e = blockIdx.x, h = blockIdx.y, col0 = blockIdx.z * 16;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int slot = a.slot_ids[e];
@@ -154,21 +254,27 @@ __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(DeltaChunks a, in
     const int c0 = max(0, number0 - first), c1 = min(chunks, number1 - first);
     if (c0 >= c1) return;
     const int row0 = wave * (D / 4) + 4 * g;                // lane (column r, g) has rows row0 + 16 i + e
-    float* st = a.state + (size_t)slot * a.state_stride + (size_t)h * D * a.dv + col0 + r;
-    dc_f32x4_t S[TI];
+    float* head = a.state + (size_t)slot * a.slot_stride + (size_t)h * a.head_stride;
+    float* st = head + col0 + r;
+    float* nm = head + (size_t)D * a.dv + (size_t)blockIdx.z * (D + 1);          // (mLSTM)
+    dc_f32x4_t S[TI], N[TI];
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int x = 0; x < 4; ++x) S[i][x] = st[(size_t)(row0 + 16 * i + x) * a.dv];
+        for (int x = 0; x < 4; ++x) {
+            S[i][x] = st[(size_t)(row0 + 16 * i + x) * a.dv];
+            N[i][x] = DELTA ? 0.f : nm[row0 + 16 * i + x];
+        }
     const int rec = dc_record(D, a.dv);
-    // this lane's operands of a chunk
+    auto record = [&](int c) { return a.ws + ((size_t)(first + min(c, c1 - 1) - number0) * a.H + h) * rec; };
+    // this lane's operands of a chunk (mw: the mLSTM's sums of K)
     struct Ops { dc_f32x4_t mw[TI], q[TI], k[TI], gl[TI], b, mv; };
     auto load = [&](Ops& x, int c) {
-        const float* p = a.ws + ((size_t)(first + min(c, c1 - 1) - number0) * a.H + h) * rec;
+        const float* p = record(c);
         const float* mv = p + 48 * D + 4 * g * a.dv + col0 + r;
 #pragma unroll
         for (int i = 0; i < TI; ++i) {
-            x.mw[i] = *reinterpret_cast<const dc_f32x4_t*>(p + r * D + row0 + 16 * i);
+            x.mw[i] = *reinterpret_cast<const dc_f32x4_t*>(p + (DELTA ? r * D : 0) + row0 + 16 * i);
             x.q[i] = *reinterpret_cast<const dc_f32x4_t*>(p + 16 * D + r * D + row0 + 16 * i);
             x.k[i] = *reinterpret_cast<const dc_f32x4_t*>(p + 32 * D + (row0 - 4 * g + 16 * i + r) * 16 + 4 * g);
             x.gl[i] = *reinterpret_cast<const dc_f32x4_t*>(p + 48 * D + 16 * a.dv + 256 + row0 + 16 * i);
@@ -179,23 +285,32 @@ __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(DeltaChunks a, in
     };
     // read-out of chunk c: the waves' parts, row 4 g + wave of lane (column r, g)
     auto read_out = [&](int c) {
-        const int t = q0 + c * DC_TOKENS + 4 * g + wave;
+        const int row = 4 * g + wave, t = q0 + c * DC_TOKENS + row;
         float y = 0.f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) y += po[c & 1][w][lane][wave];
+        if (!DELTA) {
+            const float* p = record(c) + D;
+            float nq = p[row];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) nq += pn[c & 1][w][row];
+            y /= fmaxf(fabsf(nq), p[16 + row]) + 1e-6f;
+        }
         if (t < q1) a.o[((size_t)t * a.H + h) * a.dv + col0 + r] = y;
     };
     auto chunk = [&](const Ops& x, int c) {
-        dc_f32x4_t u0 = {0.f, 0.f, 0.f, 0.f}, u1 = {0.f, 0.f, 0.f, 0.f}, o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
+        dc_f32x4_t o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
+        if (DELTA) {
+            dc_f32x4_t u0 = {0.f, 0.f, 0.f, 0.f}, u1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < TI; ++i) {
+            for (int i = 0; i < TI; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; j += 2) {
-                u0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[i][j], S[i][j], u0, 0, 0, 0);
-                u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[i][j + 1], S[i][j + 1], u1, 0, 0, 0);
-            }
+                for (int j = 0; j < 4; j += 2) {
+                    u0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[i][j], S[i][j], u0, 0, 0, 0);
+                    u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[i][j + 1], S[i][j + 1], u1, 0, 0, 0);
+                }
+            *reinterpret_cast<dc_f32x4_t*>(pu[DELTA ? c & 1 : 0][wave][lane]) = u0 + u1;
         }
-        *reinterpret_cast<dc_f32x4_t*>(pu[c & 1][wave][lane]) = u0 + u1;
 #pragma unroll
         for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -203,10 +318,25 @@ __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(DeltaChunks a, in
                 o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][j], S[i][j], o0, 0, 0, 0);
                 o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][j + 1], S[i][j + 1], o1, 0, 0, 0);
             }
+        float nq = 0.f;
+        if (!DELTA) {
+#pragma unroll
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) nq = fmaf(x.q[i][j], N[i][j], nq);        // lane (token r, g): its rows' share of n . q
+            nq += __shfl_xor(nq, 16, 64);
+            nq += __shfl_xor(nq, 32, 64);
+#pragma unroll
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) N[i][j] = fmaf(x.gl[i][j], N[i][j], x.mw[i][j]);
+        }
         __syncthreads();                                    // parts of u of this chunk, and of the read-out of the chunk before
         dc_f32x4_t u = x.mv;
+        if (DELTA) {
 #pragma unroll
-        for (int w = 0; w < 4; ++w) u -= *reinterpret_cast<const dc_f32x4_t*>(pu[c & 1][w][lane]);
+            for (int w = 0; w < 4; ++w) u -= *reinterpret_cast<const dc_f32x4_t*>(pu[DELTA ? c & 1 : 0][w][lane]);
+        }
 #pragma unroll
         for (int i = 0; i < TI; ++i) S[i] *= x.gl[i];
 #pragma unroll
@@ -232,8 +362,9 @@ __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(DeltaChunks a, in
         if (c > c0) read_out(c - 1);
         // (the place was read for chunk c - 2 behind the barrier of chunk c - 1, which every wave has passed)
         *reinterpret_cast<dc_f32x4_t*>(po[c & 1][wave][lane]) = o0 + o1;
+        if (!DELTA && g == 0) pn[c & 1][wave][r] = nq;
     };
-    Ops x0, x1;
+    Ops x0, x1;                                             // (three chunks' operands under way instead of one: no faster)
     load(x0, c0);
     int c = c0;
     for (; c + 2 <= c1; c += 2) {
@@ -248,7 +379,11 @@ __global__ __launch_bounds__(256) void delta_chunk_walk_kernel(DeltaChunks a, in
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int y = 0; y < 4; ++y) st[(size_t)(row0 + 16 * i + y) * a.dv] = S[i][y];
+        for (int y = 0; y < 4; ++y) {
+            st[(size_t)(row0 + 16 * i + y) * a.dv] = S[i][y];
+            if (!DELTA && r == 0) nm[row0 + 16 * i + y] = N[i][y];
+        }
+    if (!DELTA && threadIdx.x == 0) nm[D] = a.mfin[(size_t)e * a.H + h];
 }
 
 bool delta_chunks_takes(int S, int T, int d, int dv) { return T > S && (d == 64 || d == 128) && dv % 16 == 0; }
@@ -261,18 +396,40 @@ int64_t delta_chunks_workspace(int S, int T, int H, int d, int dv) {
 int delta_chunks(const DeltaChunks& a, int dtype, hipStream_t st) {
     SPY_REQUIRE(a.ws && a.ws_floats >= delta_chunks_workspace(a.S, a.T, a.H, a.d, a.dv), "delta rule: the chunks' workspace is too small");
     SPY_REQUIRE(((uintptr_t)a.ws % 16) == 0 && a.H <= 65535 && a.dv / 16 <= 65535, "delta rule: workspace alignment or heads");
+    const ChunkWalk w = {a.o, a.state, a.state_stride, (long long)a.d * a.dv, nullptr, a.cu_q, a.slot_ids, a.num_slots, a.H, a.dv, a.ws};
     const int64_t numbers = dc_numbers(a.S, a.T);
     for (int64_t n0 = 0; n0 < numbers; n0 += DC_SEGMENT) {
         const int n1 = (int)(n0 + DC_SEGMENT < numbers ? n0 + DC_SEGMENT : numbers);
         const dim3 pgrid((unsigned)(n1 - n0), a.H), wgrid(a.S, a.H, a.dv / 16);
         if (a.d == 64) {
             SPY_DISPATCH(dtype, TA, (delta_chunk_prepare_kernel<TA, 64><<<pgrid, 256, 0, st>>>(a, (int)n0)));
-            delta_chunk_walk_kernel<64><<<wgrid, 256, 0, st>>>(a, (int)n0, n1);
+            chunk_walk_kernel<64, true><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
         } else {
             SPY_DISPATCH(dtype, TA, (delta_chunk_prepare_kernel<TA, 128><<<pgrid, 256, 0, st>>>(a, (int)n0)));
-            delta_chunk_walk_kernel<128><<<wgrid, 256, 0, st>>>(a, (int)n0, n1);
+            chunk_walk_kernel<128, true><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
         }
         SPY_CHECK_LAUNCH("spy_delta_rule (chunks)");
+    }
+    return 0;
+}
+
+int memory_chunks(const MemoryChunks& a, int dtype, hipStream_t st) {
+    SPY_REQUIRE(a.ws && a.ws_floats >= delta_chunks_workspace(a.S, a.T, a.H, a.d, a.dv), "mLSTM: the chunks' workspace is too small");
+    SPY_REQUIRE(((uintptr_t)a.ws % 16) == 0 && a.H <= 65535 && a.dv / 16 <= 65535, "mLSTM: workspace alignment or heads");
+    const long long head = (long long)a.d * a.dv + (long long)(a.dv / 16) * (a.d + 1);
+    const ChunkWalk w = {a.o, a.state, head * a.H, head, a.mfin, a.cu_q, a.slot_ids, a.num_slots, a.H, a.dv, a.ws};
+    const int64_t numbers = dc_numbers(a.S, a.T);
+    for (int64_t n0 = 0; n0 < numbers; n0 += DC_SEGMENT) {
+        const int n1 = (int)(n0 + DC_SEGMENT < numbers ? n0 + DC_SEGMENT : numbers);
+        const dim3 pgrid((unsigned)(n1 - n0), a.H), wgrid(a.S, a.H, a.dv / 16);
+        if (a.d == 64) {
+            SPY_DISPATCH(dtype, TA, (memory_chunk_prepare_kernel<TA, 64><<<pgrid, 256, 0, st>>>(a, (int)n0)));
+            chunk_walk_kernel<64, false><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
+        } else {
+            SPY_DISPATCH(dtype, TA, (memory_chunk_prepare_kernel<TA, 128><<<pgrid, 256, 0, st>>>(a, (int)n0)));
+            chunk_walk_kernel<128, false><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
+        }
+        SPY_CHECK_LAUNCH("spy_mlstm (chunks)");
     }
     return 0;
 }

@@ -76,8 +76,8 @@ __global__ void mlstm_gates_kernel(float* __restrict__ gates, const TW* __restri
 // not wait for each other, so none may read what another has already moved on).
 #define MM_AHEAD 4          // tokens whose operands are in flight ahead of the one being worked on
 // MODE 0: block x is an entry, walked whole from the request's state, which is left at the end.
-// Entries of many tokens are cut into pieces (block x is a piece then): with the running maximum known for every token
-// (mlstm_scalars_kernel: a, b and exp(-m) per token in `gates` [T, 3 H]) the state is linear in itself with scalar
+// Entries of many tokens (whose heads do not go by chunks, delta_chunks.hip) are cut into pieces (block x is a piece then): with the
+// running maximum known for every token (mlstm_scalars_kernel: a, b and exp(-m) per token in `gates` [T, 3 H]) the state is linear in itself with scalar
 // coefficients, S_end = A S_start + B with A the product of the piece's a.  MODE 1 walks a piece from zero and leaves
 // (B, A) in the piece's record of `work` (laid out as a request's state, A where m lies); MODE 2 folds the records of
 // the entry's pieces before its own into the request's state, walks its piece from there and writes the read-outs;
@@ -220,54 +220,49 @@ __global__ __launch_bounds__(MM_SLICE) void mlstm_kernel(
     if (lane == 0) nm[d] = m;
 }
 
-// One thread per (entry, head): the running maximum over the entry's tokens, from the request's state, before and after
-// every token in abe [T, 3 H]; the last maximum goes to mfin [S, H].
-__global__ void mlstm_scalars_kernel(float* __restrict__ abe, float* __restrict__ mfin, const float* __restrict__ lg,
-                                     const float* __restrict__ state, const int* __restrict__ cu_q, const int* __restrict__ slot_ids,
-                                     int num_slots, int S, int H, int d, int dv, int NS) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= S * H) return;
-    const int s = i / H, h = i - s * H;
+// One wave per (entry, head), 64 tokens at a time: the running maximum m = max(f + m', i) is F + max(m0, max_s (i_s - F_s)) with F the
+// sums of f, so a prefix sum and a prefix maximum over the lanes give it for all of them (in 64 bits: the sums' difference cancels).
+// abe [T, 3 H] gets a = exp(f + m' - m), b = exp(i - m) and exp(-m) of every token, mfin [S, H] the last maximum.  (A thread a chain
+// of one token after another took 146 us for 1500 tokens, and a second pass for the exponentials.)
+__global__ __launch_bounds__(64) void mlstm_scalars_kernel(float* __restrict__ abe, float* __restrict__ mfin, const float* __restrict__ lg,
+                                                           const float* __restrict__ state, const int* __restrict__ cu_q,
+                                                           const int* __restrict__ slot_ids, int num_slots, int H, int d, int dv, int NS) {
+    const int s = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
     const int slot = slot_ids[s];
     if (slot < 0 || slot >= num_slots) return;
     const size_t head_state = (size_t)d * dv + (size_t)NS * (d + 1);
-    float m = state[((size_t)slot * H + h) * head_state + (size_t)d * dv + d];
-    const int t1 = cu_q[s + 1];
-    // (the gates of 16 tokens are asked for together: the loads do not depend on the maximum, only the arithmetic does)
-    for (int tb = cu_q[s]; tb < t1; tb += 16) {
-        float ig[16], fg[16];
+    double m = (double)state[((size_t)slot * H + h) * head_state + (size_t)d * dv + d];
+    const int t0 = cu_q[s], t1 = cu_q[s + 1];
+    auto gate = [&](int t, int which) { return lg[(size_t)min(t, t1 - 1) * 2 * H + which * H + h]; };
+    float ig = gate(t0 + lane, 0), fg = gate(t0 + lane, 1);
+    for (int tb = t0; tb < t1; tb += 64) {
+        const int t = tb + lane;
+        const float i = ig, f = fg;
+        ig = gate(t + 64, 0);
+        fg = gate(t + 64, 1);
+        double F = (double)f;
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int t = tb + u < t1 ? tb + u : t1 - 1;
-            ig[u] = lg[(size_t)t * 2 * H + h];
-            fg[u] = lg[(size_t)t * 2 * H + H + h];
+        for (int o = 1; o < 64; o <<= 1) {
+            const double x = __shfl_up(F, o, 64);
+            if (lane >= o) F += x;
         }
+        double P = (double)i - F;
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int t = tb + u;
-            if (t < t1) {
-                const float m_new = fmaxf(fg[u] + m, ig[u]);
-                abe[(size_t)t * 3 * H + h] = m;                      // (the exponentials follow for all tokens at once)
-                abe[(size_t)t * 3 * H + H + h] = m_new;
-                m = m_new;
-            }
+        for (int o = 1; o < 64; o <<= 1) {
+            const double x = __shfl_up(P, o, 64);
+            if (lane >= o) P = fmax(P, x);
         }
+        const double now = F + fmax(m, P);
+        const double up = __shfl_up(now, 1, 64), before = lane == 0 ? m : up;
+        if (t < t1) {
+            float* to = abe + (size_t)t * 3 * H + h;
+            to[0] = expf((float)((double)f + before - now));
+            to[H] = expf((float)((double)i - now));
+            to[2 * H] = expf((float)-now);
+        }
+        m = __shfl(now, min(63, t1 - 1 - tb), 64);
     }
-    mfin[i] = m;
-}
-
-// abe [T, 3 H] holds the maximum before and after every token (mlstm_scalars_kernel); with the log gates lg [T, 2 H] it
-// becomes a = exp(f + m' - m), b = exp(i - m) and exp(-m).
-__global__ void mlstm_abe_kernel(float* __restrict__ abe, const float* __restrict__ lg, int T, int H) {
-    const size_t total = (size_t)T * H;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-        const size_t t = i / H, h = i - t * H;
-        const float mp = abe[t * 3 * H + h], mn = abe[t * 3 * H + H + h];
-        const float ig = lg[t * 2 * H + h], fg = lg[t * 2 * H + H + h];
-        abe[t * 3 * H + h] = expf(fg + mp - mn);
-        abe[t * 3 * H + H + h] = expf(ig - mn);
-        abe[t * 3 * H + 2 * H + h] = expf(-mn);
-    }
+    if (lane == 0) mfin[(size_t)s * H + h] = (float)m;
 }
 
 // Block x is a piece; the last piece of an entry folds all of the entry's records into the request's state.
@@ -336,11 +331,13 @@ __global__ __launch_bounds__(MM_SLICE) void mlstm_keep_kernel(float* __restrict_
     } while (0)
 
 // pieces: int32 [4][n_pieces] (entry, first row, end row, index of the entry's first piece), used when `multi` says that an
-// entry has several; then work [n_pieces][state of a request], abe [T][3 H] and mfin [S][H] are scratch.
+// entry has several; then work [n_pieces][state of a request], abe [T][3 H] and mfin [S][H] are scratch (the latter two, and ws instead
+// of work, where spy_mlstm_workspace says that the step goes by chunks).
 extern "C" int spy_mlstm(void* out, float* o_tmp, float* state, const void* x, long long xs, int dtype, int q_off, int k_off, int v_off,
                          int g_off, float* gates, const void* bi, const void* bf, int w_dtype, float cap, const void* norm_w,
                          float eps, const int* cu_q, const int* slot_ids, int num_slots, int S, int T, int H, int d, int dv,
-                         const int* pieces, int n_pieces, int multi, float* work, float* abe, float* mfin, hipStream_t st) {
+                         const int* pieces, int n_pieces, int multi, float* work, float* abe, float* mfin, float* ws, int64_t ws_floats,
+                         hipStream_t st) {
     SPY_REQUIRE(S > 0 && T > 0 && H > 0 && d > 0 && dv > 0 && num_slots > 0 && o_tmp, "spy_mlstm: empty operand");
     SPY_REQUIRE(d <= 256 && dv <= 1024 && H <= 65535, "spy_mlstm: heads of %d x %d (key size up to 256, value size up to 1024)", d, dv);
     SPY_REQUIRE(cap > 0.f, "spy_mlstm: the gates' cap must be positive");
@@ -352,24 +349,27 @@ extern "C" int spy_mlstm(void* out, float* o_tmp, float* state, const void* x, l
         SPY_DISPATCH(w_dtype, TW, (mlstm_gates_kernel<TW><<<blocks, 256, 0, st>>>(gates, (const TW*)bi, (const TW*)bf, cap, T, H)));
         SPY_CHECK_LAUNCH("spy_mlstm (gates)");
     }
-    if (!multi) {
+    // Steps of single tokens walk token by token; the others go by chunks where the head sizes are whole matrix tiles, else by pieces
+    const bool chunks = delta_chunks_takes(S, T, d, dv);
+    if (chunks || multi) {
+        SPY_REQUIRE(abe && mfin, "spy_mlstm: no room for the tokens' scalars");
+        mlstm_scalars_kernel<<<dim3(S, H), 64, 0, st>>>(abe, mfin, gates, state, cu_q, slot_ids, num_slots, H, d, dv, NS);
+        SPY_CHECK_LAUNCH("spy_mlstm (running maximum)");
+    }
+    if (chunks) {
+        const MemoryChunks a = {o_tmp, state, x, xs, q_off, k_off, v_off, abe, mfin, cu_q, slot_ids, num_slots, S, T, H, d, dv, ws, ws_floats};
+        const int rc = memory_chunks(a, dtype, st);
+        if (rc) return rc;
+    } else if (!multi) {
         SPY_DISPATCH(dtype, TA, SPY_DISPATCH(w_dtype, TW, MM_LAUNCH_MODE(mlstm_kernel, 0, o_tmp, state, (const TA*)x, xs, q_off, k_off, v_off,
             gates, cu_q, slot_ids, num_slots, H, d, dv, NS, nullptr, nullptr, nullptr, nullptr, nullptr)));
         SPY_CHECK_LAUNCH("spy_mlstm");
     } else {
-        SPY_REQUIRE(pieces && n_pieces > 0 && work && abe && mfin, "spy_mlstm: entries in several pieces need their scratch memory");
+        SPY_REQUIRE(pieces && n_pieces > 0 && work, "spy_mlstm: entries in several pieces need their scratch memory");
         const int* pe = pieces;
         const int* p0 = pieces + n_pieces;
         const int* p1 = pieces + 2 * (size_t)n_pieces;
         const int* pf = pieces + 3 * (size_t)n_pieces;
-        mlstm_scalars_kernel<<<(S * H + 63) / 64, 64, 0, st>>>(abe, mfin, gates, state, cu_q, slot_ids, num_slots, S, H, d, dv, NS);
-        SPY_CHECK_LAUNCH("spy_mlstm (running maximum)");
-        {
-            const size_t total = (size_t)T * H;
-            const unsigned blocks = (unsigned)((total + 255) / 256 > 4096 ? 4096 : (total + 255) / 256);
-            mlstm_abe_kernel<<<blocks, 256, 0, st>>>(abe, gates, T, H);
-            SPY_CHECK_LAUNCH("spy_mlstm (decays)");
-        }
         const dim3 grid(n_pieces, H, NS);
         SPY_DISPATCH(dtype, TA, SPY_DISPATCH(w_dtype, TW, MM_LAUNCH_MODE(mlstm_kernel, 1, o_tmp, state, (const TA*)x, xs, q_off, k_off, v_off,
             abe, cu_q, slot_ids, num_slots, H, d, dv, NS, work, pe, p0, p1, pf)));
@@ -695,7 +695,10 @@ __global__ __launch_bounds__(MM_SLICE) void delta_rule_kernel(
         if (col && row0 + i < d) st[(size_t)(row0 + i) * dv + j] = S[i];
 }
 
-// floats of workspace that a step of S entries and T tokens needs (0: it walks token by token)
+// floats of workspace that a step of S entries and T tokens needs (0: it does not go by chunks)
+extern "C" int64_t spy_mlstm_workspace(int S, int T, int H, int d, int dv) {
+    return delta_chunks_takes(S, T, d, dv) ? delta_chunks_workspace(S, T, H, d, dv) : 0;
+}
 extern "C" int64_t spy_delta_rule_workspace(int S, int T, int H, int d, int dv) {
     return delta_chunks_takes(S, T, d, dv) ? delta_chunks_workspace(S, T, H, d, dv) : 0;
 }

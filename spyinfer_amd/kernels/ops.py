@@ -77,7 +77,7 @@ class _Hip:
                      "spy_gemm_decode", "spy_gemm_decode_workspace", "spy_embedding_sumsq", "spy_sample_static", "spy_measure_read",
                      "spy_pair_embedding", "spy_norm_residual", "spy_depth_mix", "spy_xielu", "spy_mingru", "spy_latent_prepare",
                      "spy_gemm_strided", "spy_latent_attention", "spy_latent_attention_mfma", "spy_latent_attention_mfma_workspace", "spy_head_products",
-                     "spy_bias_rope_store", "spy_sigmoid_gate", "spy_mlstm", "spy_causal_conv_silu", "spy_delta_rule", "spy_delta_rule_workspace", "spy_moe_route",
+                     "spy_bias_rope_store", "spy_sigmoid_gate", "spy_mlstm", "spy_mlstm_workspace", "spy_causal_conv_silu", "spy_delta_rule", "spy_delta_rule_workspace", "spy_moe_route",
                      "spy_moe_align", "spy_moe_gemm", "spy_moe_combine", "spy_moe_tile_rows", "spy_moe_group_ints", "spy_token_shift", "spy_tanh", "spy_time_mix",
                      "spy_norm_pair_mean", "spy_scale_cap", "spy_result_norm", "spy_moe_align_tables", "spy_layer_norm", "spy_layer_norm_residual",
                      "spy_gelu", "spy_norm_rope_store", "spy_map_difference", "spy_rotation_angles", "spy_decay_memory", "spy_group_norm"):
@@ -1574,18 +1574,22 @@ def mlstm(x: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: int, gates
     if T:
         tmp = torch.empty((T, H * dv), dtype=torch.float32, device=x.device)        # the read-outs before the heads' norm
         parr, n_pieces, multi, work, abe, mfin = None, 0, False, None, None, None
+        ws_floats = hip().lib.spy_mlstm_workspace(ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(H), ctypes.c_int(d), ctypes.c_int(dv))
+        ws = torch.empty((ws_floats,), dtype=torch.float32, device=x.device) if ws_floats else None
         if pieces is not None and pieces[2]:
             parr, n_pieces, multi = pieces
             _dev(parr)
             _check(parr.dtype == torch.int32 and parr.shape == (4 * n_pieces,) and n_pieces > 0, "mlstm: pieces must be int32 [4 n]")
-            work = torch.empty((n_pieces, state.shape[1]), dtype=torch.float32, device=x.device)
+            if ws is None:
+                work = torch.empty((n_pieces, state.shape[1]), dtype=torch.float32, device=x.device)
+        if multi or ws is not None:
             abe = torch.empty((T, 3 * H), dtype=torch.float32, device=x.device)
             mfin = torch.empty((S, H), dtype=torch.float32, device=x.device)
         hip().call("spy_mlstm", _ptr(out), _ptr(tmp), _ptr(state), ctypes.c_void_p(x.data_ptr()), ctypes.c_longlong(xs), _code(x, "x"), ctypes.c_int(q_off),
                    ctypes.c_int(k_off), ctypes.c_int(v_off), ctypes.c_int(g_off), _ptr(gates), _ptr(bi), _ptr(bf), _code(bi, "gate biases"),
                    ctypes.c_float(cap), _ptr(norm_w), ctypes.c_float(eps), _ptr(cu_q), _ptr(slot_ids), ctypes.c_int(state.shape[0]),
                    ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(H), ctypes.c_int(d), ctypes.c_int(dv), _ptr(parr), ctypes.c_int(n_pieces),
-                   ctypes.c_int(1 if multi else 0), _ptr(work), _ptr(abe), _ptr(mfin), _Hip.stream())
+                   ctypes.c_int(1 if multi else 0), _ptr(work), _ptr(abe), _ptr(mfin), _ptr(ws), ctypes.c_int64(ws_floats), _Hip.stream())
     return out
 
 

@@ -1,6 +1,8 @@
 """The gated delta rule over chunks of 16 tokens (csrc/delta_chunks.hip): entries of every length around a chunk and a few chunks, one
 long enough for several segments, single tokens beside them, states carried from step to step, decays from none to all, one decay per
 head and one per channel; against the recurrence in float64, token by token."""
+import math
+
 import pytest
 import torch
 
@@ -85,3 +87,63 @@ def test_an_infinite_value_stays_with_the_tokens_that_read_it():
     ones = lambda *s: torch.ones(*s, device=dev)
     y = ops.delta_rule(qkv.to(dev), ones(T, 1) * 0.3, ones(T, d) * -3, ones(1), ones(d), ones(T, dv), ones(dv), 1e-6, torch.zeros(1, d * dv, device=dev), cu, slot, 1, 1, d, dv)
     assert bool(y[:21].isfinite().all()) and not bool(y[21:].isfinite().all(dim=1).any())
+
+
+# heads, key size, value size, lengths of the steps' entries
+MEMORIES = [(2, 128, 128, [(1, 17), (16, 31)]), (3, 64, 48, [(15, 1, 40), (2, 33, 1)]), (1, 128, 16, [(150, 65), (1, 1), (64, 2)]), (1, 64, 32, [(2200,), (7,)])]
+
+
+@pytest.mark.parametrize("how", ["keep", "lose", "wild"])
+@pytest.mark.parametrize("case", range(len(MEMORIES)))
+def test_matrix_memory_chunks_against_the_recurrence(case, how):
+    """The mLSTM likewise; its gates: little forgotten, much forgotten, both with inputs that move the running maximum about."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    H, d, dv, steps = MEMORIES[case]
+    if case == 3 and how != "keep":
+        pytest.skip("the long entry once")
+    g = torch.Generator().manual_seed(20 * case + len(how))
+    n = len(steps[0])
+    slot_ids = torch.randperm(n + 1, generator=g)[:n].int()
+    state = torch.zeros(n + 1, ops.mlstm_state_size(H, d, dv))
+    spare = [i for i in range(n + 1) if i not in slot_ids.tolist()]
+    state[spare] = 7.0
+    state_dev, cap = state.to(dev), 15.0
+    S, N, M = ([[torch.zeros(z, dtype=torch.float64) for _ in range(H)] for _ in range(n)] for z in ((d, dv), (d,), ()))
+    bi, bf, nw = torch.randn(H, generator=g), torch.randn(H, generator=g), 1.0 + 0.1 * torch.randn(H * dv, generator=g)
+    for lens in steps:
+        T = sum(lens)
+        x = torch.randn(T, 2 * H * d + 2 * H * dv, generator=g)
+        gates = torch.randn(T, 2 * H, generator=g) * {"keep": 0.5, "lose": 0.5, "wild": 9.0}[how]
+        gates[:, H:] += {"keep": 4.0, "lose": -3.0, "wild": 0.0}[how]
+        cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+        y = ops.mlstm(x.to(dev), 0, H * d, 2 * H * d, 2 * H * d + H * dv, gates.clone().to(dev), bi.to(dev), bf.to(dev), cap, nw.to(dev), 1e-6, state_dev,
+                      cu.to(dev), slot_ids.to(dev), H, d, dv).cpu().double().view(T, H, dv)
+        xd = x.double()
+        q, k = xd[:, :H * d].view(T, H, d) * d ** -0.5, xd[:, H * d:2 * H * d].view(T, H, d)
+        v, og = xd[:, 2 * H * d:2 * H * d + H * dv].view(T, H, dv), torch.sigmoid(xd[:, 2 * H * d + H * dv:]).view(T, H, dv)
+        ig = cap * torch.tanh((gates[:, :H].double() + bi.double()) / cap)
+        fg = torch.nn.functional.logsigmoid(cap * torch.tanh((gates[:, H:].double() + bf.double()) / cap))
+        for e, L in enumerate(lens):
+            for h in range(H):
+                for t in range(int(cu[e]), int(cu[e]) + L):
+                    new = torch.maximum(fg[t, h] + M[e][h], ig[t, h])
+                    a, b = torch.exp(fg[t, h] + M[e][h] - new), torch.exp(ig[t, h] - new)
+                    S[e][h] = a * S[e][h] + b * torch.outer(k[t, h], v[t, h])
+                    N[e][h] = a * N[e][h] + b * k[t, h]
+                    M[e][h] = new
+                    nq = float(N[e][h] @ q[t, h])
+                    den = max(abs(nq), math.exp(-new)) + 1e-6
+                    o = S[e][h].T @ q[t, h] / den
+                    ref = o / torch.sqrt((o * o).mean() + 1e-6) * nw.double().view(H, dv)[h] * og[t, h]
+                    # float32: a value of S^T q is rounded by at most 100 times 2^-24 of the sum of its terms' sizes (chains of 36 products,
+                    # the parts' sums, the state's own roundings of the last chunks), and the head's norm divides by its root mean square
+                    terms = float((S[e][h].abs().T @ q[t, h].abs()).max()) / den
+                    bound = 100 * 2.0 ** -24 * terms / float(torch.sqrt((o * o).mean() + 1e-6)) * float((nw.double().view(H, dv)[h] * og[t, h]).abs().max())
+                    assert float((y[t, h] - ref).abs().max()) < max(2e-5, bound), (e, h, t)
+                st = state_dev[int(slot_ids[e])].cpu().double()
+                head = st[h * (len(st) // H):(h + 1) * (len(st) // H)]
+                assert float((head[:d * dv].view(d, dv) - S[e][h]).abs().max()) < 1e-5 * max(1.0, float(S[e][h].abs().max()))
+                own = head[d * dv:].view(-1, d + 1)                          # n and m once for every slice of value channels
+                assert float((own[:, :d] - N[e][h]).abs().max()) < 1e-5 * max(1.0, float(N[e][h].abs().max())) and float((own[:, d] - M[e][h]).abs().max()) < 1e-4
+    assert bool((state_dev[spare] == 7.0).all())
