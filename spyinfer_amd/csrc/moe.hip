@@ -318,137 +318,110 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(TC* __restrict__ C, const
 }
 
 
-// The same product on the matrix cores, bfloat16 operands and float32 sums (v_mfma_f32_16x16x32_bf16).  A block of four
-// waves takes up to MT neighbouring row tiles (16 sorted rows each) that belong to one expert, and a group of columns:
-// every wave owns its columns' rows of W (gated: 16 gate rows and the 16 up rows of the same columns; else 32 rows) and
-// walks K, loading its W fragments once per step and using them for all the row tiles, whose rows of A are gathered
-// through the pairs' tokens.  Operands go from memory straight into MFMA operand registers: lane (r = lane % 16,
-// g = lane / 16) holds row r, values k + 8 g .. + 7; the result tile is C^T: lane (r, g) holds C[row r][column 4 g + i].
-// A block whose MT tiles belong to several experts takes their runs in turn.
+// The same product on the matrix cores, bfloat16 operands and float32 sums (v_mfma_f32_16x16x32_bf16), for few rows per expert (decoding):
+// a block has one row tile (16 sorted rows) and 32 rows of W (gated: 16 gate rows and the 16 up rows of the same columns), whose K
+// its four waves take in chunks of 128 in turn and add through LDS.  Operands go from memory straight into MFMA operand registers: lane
+// (r = lane % 16, g = lane / 16) holds row r, values k + 8 g .. + 7; the result tile is C^T: lane (r, g) holds C[row r][column 4 g + i].
+// What bounds it: the experts' matrices from memory.  A wave that walks all of K for 32 rows of W has four times the work of one that
+// takes a quarter, and the last round of such blocks, a sixth of the chip, costs what a whole one does.  Measured, both products of 32
+// experts of 2 x 3072 x 4096, 12 tokens with four each: 199 + 105 us (6.4 TB/s over the experts touched) against 236 + 141 for such
+// blocks; 8 tokens, 2 x 1536 x 2048: 43 + 20 against 60 + 42.  Blocks of one expert's columns are neighbours in the grid (229 + 123 us
+// with an expert's tiles outermost); loads with the hint that they are not read again cost a fifth (245 + 134): a row's 64 bytes of
+// one load are half a line, the other half is the next load's.
 typedef __attribute__((__vector_size__(8 * sizeof(short)))) short moe_bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float moe_f32x4_t;
 
-template <int MT, bool GATED, typename TC>
-__global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(TC* __restrict__ C, const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+template <bool GATED, typename TC>
+__global__ __launch_bounds__(256) void moe_gemm_tile_kernel(TC* __restrict__ C, const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                                             const int* __restrict__ tile_expert, const int* __restrict__ sorted_pair,
-                                                            int gather, int max_tiles, int N, int K, long long w_stride, MoeAct act) {
+                                                            int gather, int N, int K, long long w_stride, MoeAct act) {
+    __shared__ __align__(16) float red[4][2][64][4];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r = lane & 15, g = lane >> 4;
-    constexpr int NT = 2;
-    const int n0 = (blockIdx.y * 4 + wave) * (GATED ? 16 : 32);
-    if (n0 >= N) return;
-    int t = blockIdx.x * MT;
-    const int t_end = min(t + MT, max_tiles);
-    const moe_bf16x8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-    while (t < t_end) {
-        const int e = __builtin_amdgcn_readfirstlane(tile_expert[t]);
-        if (e < 0) break;
-        int run = 1;
-        while (t + run < t_end && __builtin_amdgcn_readfirstlane(tile_expert[t + run]) == e) ++run;
-        const bf16_t* xrow[MT];
-        bool xok[MT];
+    const int t = blockIdx.y, n0 = blockIdx.x * (GATED ? 16 : 32);
+    const int e = __builtin_amdgcn_readfirstlane(tile_expert[t]);
+    if (e < 0) return;
+    const int row = t * MOE_TM + r, p = sorted_pair[row], p0 = sorted_pair[t * MOE_TM];
+    // a tile with an expert has a first row; rows that do not exist read that one's values, and what they give is not stored
+    const int src = gather > 0 ? max(p >= 0 ? p : p0, 0) / gather : (p >= 0 ? row : t * MOE_TM);
+    const bf16_t* xrow = A + (size_t)src * K + 8 * g;
+    const bf16_t* We = W + (size_t)e * w_stride;
+    const bf16_t* wrow[2];
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            xok[mt] = false;
-            xrow[mt] = A;
-            if (mt < run) {
-                const int row = (t + mt) * MOE_TM + r;
-                const int p = sorted_pair[row];
-                xok[mt] = p >= 0;
-                const int src = gather > 0 ? p / gather : row;
-                xrow[mt] = A + (size_t)(p >= 0 ? src : 0) * K + 8 * g;
-            }
+    for (int nt = 0; nt < 2; ++nt) wrow[nt] = We + (size_t)(GATED ? nt * N + min(n0 + r, N - 1) : min(n0 + nt * 16 + r, N - 1)) * K + 8 * g;
+    moe_f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    auto load = [&](const bf16_t* q) { return *reinterpret_cast<const moe_bf16x8_t*>(q); };
+    auto fetch = [&](moe_bf16x8_t (&a)[2][4], moe_bf16x8_t (&b)[4], int k) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt) a[nt][j] = load(wrow[nt] + k + 32 * j);
+            b[j] = *reinterpret_cast<const moe_bf16x8_t*>(xrow + k + 32 * j);
         }
-        const bf16_t* We = W + (size_t)e * w_stride;
-        const bf16_t* wrow[NT];
+    };
+    auto products = [&](const moe_bf16x8_t (&a)[2][4], const moe_bf16x8_t (&b)[4]) {
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int row = GATED ? nt * N + min(n0 + r, N - 1) : min(n0 + nt * 16 + r, N - 1);
-            wrow[nt] = We + (size_t)row * K + 8 * g;
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[nt][j], b[j], acc[nt], 0, 0, 0);
+    };
+    // two sets of operands taken in turn, the next chunk's asked for ahead of this one's products (no load under a condition)
+    const int chunks = K >> 7, mine = (chunks - wave + 3) >> 2;
+    moe_bf16x8_t a0[2][4], b0[4], a1[2][4], b1[4];
+    if (mine > 0) {
+        auto at = [&](int i) { return (wave + 4 * i) << 7; };
+        fetch(a0, b0, at(0));
+        int i = 0;
+        for (; i + 2 < mine; i += 2) {
+            fetch(a1, b1, at(i + 1));
+            products(a0, b0);
+            fetch(a0, b0, at(i + 2));
+            products(a1, b1);
         }
-        moe_f32x4_t acc[NT][MT];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = moe_f32x4_t{0.f, 0.f, 0.f, 0.f};
-        int k = 0;
-        auto fetch = [&](moe_bf16x8_t (&a)[NT][4], moe_bf16x8_t (&b)[MT][4], int k0) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) a[nt][j] = *reinterpret_cast<const moe_bf16x8_t*>(wrow[nt] + k0 + 32 * j);
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) b[mt][j] = xok[mt] ? *reinterpret_cast<const moe_bf16x8_t*>(xrow[mt] + k0 + 32 * j) : zero8;
-            }
-        };
-        auto products = [&](const moe_bf16x8_t (&a)[NT][4], const moe_bf16x8_t (&b)[MT][4]) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    if (mt < run) {
-#pragma unroll
-                        for (int nt = 0; nt < NT; ++nt) acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[nt][j], b[mt][j], acc[nt][mt], 0, 0, 0);
-                    }
-        };
-        if constexpr (MT == 1) {
-            // a block with one row tile is bound by the memory's round trips: the operands of the step after this one
-            // are asked for before this step's products (two sets of operand registers, taken in turn)
-            const int steps = K / 128;
-            moe_bf16x8_t a0[NT][4], b0[MT][4], a1[NT][4], b1[MT][4];
-            if (steps > 0) fetch(a0, b0, 0);
-            for (int s = 0; s < steps; s += 2) {
-                if (s + 1 < steps) fetch(a1, b1, (s + 1) * 128);
-                products(a0, b0);
-                if (s + 1 < steps) {
-                    if (s + 2 < steps) fetch(a0, b0, (s + 2) * 128);
-                    products(a1, b1);
-                }
-            }
-            k = steps * 128;
+        if (i + 1 < mine) {
+            fetch(a1, b1, at(i + 1));
+            products(a0, b0);
+            products(a1, b1);
         } else {
-            for (; k + 128 <= K; k += 128) {
-                moe_bf16x8_t a[NT][4], b[MT][4];
-                fetch(a, b, k);
-                products(a, b);
-            }
+            products(a0, b0);
         }
-        for (; k < K; k += 32) {                  // the rest of K (a multiple of 8)
+    }
+    if (wave == (chunks & 3)) {                              // the rest of K (a multiple of 8): the wave whose turn it would be
+        const moe_bf16x8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+        for (int k = chunks << 7; k < K; k += 32) {
             const bool kok = k + 8 * g < K;
-            moe_bf16x8_t a[NT], b[MT];
+            const moe_bf16x8_t b = kok ? *reinterpret_cast<const moe_bf16x8_t*>(xrow + k) : zero8;
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) a[nt] = kok ? *reinterpret_cast<const moe_bf16x8_t*>(wrow[nt] + k) : zero8;
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) b[mt] = (kok && xok[mt]) ? *reinterpret_cast<const moe_bf16x8_t*>(xrow[mt] + k) : zero8;
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-                if (mt < run) {
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt) acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[nt], b[mt], acc[nt][mt], 0, 0, 0);
-                }
-        }
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            if (mt >= run || !xok[mt]) continue;
-            const size_t row = (size_t)(t + mt) * MOE_TM + r;
-            if (GATED) {
-                const float rw = act.pair_w ? act.pair_w[sorted_pair[row]] : 1.f;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int col = n0 + 4 * g + i;
-                    if (col < N) C[row * N + col] = from_f32<TC>(moe_gated(acc[0][mt][i], acc[1][mt][i], act, rw));
-                }
-            } else {
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int col = n0 + nt * 16 + 4 * g + i;
-                        if (col < N) C[row * N + col] = from_f32<TC>(moe_ungated(acc[nt][mt][i], act));
-                    }
+            for (int nt = 0; nt < 2; ++nt) {
+                const moe_bf16x8_t a = kok ? load(wrow[nt] + k) : zero8;
+                acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[nt], 0, 0, 0);
             }
         }
-        t += run;
+    }
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) *reinterpret_cast<moe_f32x4_t*>(red[wave][nt][lane]) = acc[nt];
+    __syncthreads();
+    if (wave > (GATED ? 0 : 1) || p < 0) return;
+    moe_f32x4_t sum[2];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+        sum[nt] = *reinterpret_cast<const moe_f32x4_t*>(red[0][nt][lane]);
+#pragma unroll
+        for (int w = 1; w < 4; ++w) sum[nt] += *reinterpret_cast<const moe_f32x4_t*>(red[w][nt][lane]);
+    }
+    if (GATED) {
+        const float rw = act.pair_w ? act.pair_w[p] : 1.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int col = n0 + 4 * g + i;
+            if (col < N) C[(size_t)row * N + col] = from_f32<TC>(moe_gated(sum[0][i], sum[1][i], act, rw));
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int col = n0 + wave * 16 + 4 * g + i;
+            if (col < N) C[(size_t)row * N + col] = from_f32<TC>(moe_ungated(wave ? sum[1][i] : sum[0][i], act));
+        }
     }
 }
 
@@ -733,14 +706,12 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_group_kernel(TC* __restrict__
     }
 }
 
-template <int MT>
 static int moe_gemm_mfma_launch(void* C, int c_dtype, const void* A, const void* W, const int* tile_expert, const int* sorted_pair,
-                                int gather, int gated, int max_tiles, int N, int K, MoeAct act, hipStream_t st) {
+                                int gather, int gated, bool many, int max_tiles, int N, int K, MoeAct act, hipStream_t st) {
     const long long ws = (long long)(gated ? 2 : 1) * N * K;
-    const int cols = gated ? 64 : 128;
-    const dim3 grid((max_tiles + MT - 1) / MT, (N + cols - 1) / cols);
-    SPY_REQUIRE(grid.y <= 65535, "spy_moe_gemm: too many columns");
-    if (MT == 8) {
+    if (many) {
+        const dim3 grid((max_tiles + 7) / 8, (N + (gated ? 63 : 127)) / (gated ? 64 : 128));
+        SPY_REQUIRE(grid.y <= 65535, "spy_moe_gemm: too many columns");
         if (gated) {
             SPY_DISPATCH(c_dtype, TC, (moe_gemm_mfma_lds_kernel<true, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (const bf16_t*)W, tile_expert,
                                                                                                sorted_pair, gather, max_tiles, N, K, ws, act)));
@@ -748,12 +719,16 @@ static int moe_gemm_mfma_launch(void* C, int c_dtype, const void* A, const void*
             SPY_DISPATCH(c_dtype, TC, (moe_gemm_mfma_lds_kernel<false, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (const bf16_t*)W, tile_expert,
                                                                                                 sorted_pair, gather, max_tiles, N, K, ws, act)));
         }
-    } else if (gated) {
-        SPY_DISPATCH(c_dtype, TC, (moe_gemm_mfma_kernel<MT, true, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (const bf16_t*)W, tile_expert,
-                                                                                           sorted_pair, gather, max_tiles, N, K, ws, act)));
+        return 0;
+    }
+    const dim3 grid((N + (gated ? 15 : 31)) / (gated ? 16 : 32), max_tiles);
+    SPY_REQUIRE(grid.y <= 65535, "spy_moe_gemm: too many row tiles");
+    if (gated) {
+        SPY_DISPATCH(c_dtype, TC, (moe_gemm_tile_kernel<true, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (const bf16_t*)W, tile_expert,
+                                                                                       sorted_pair, gather, N, K, ws, act)));
     } else {
-        SPY_DISPATCH(c_dtype, TC, (moe_gemm_mfma_kernel<MT, false, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (const bf16_t*)W, tile_expert,
-                                                                                            sorted_pair, gather, max_tiles, N, K, ws, act)));
+        SPY_DISPATCH(c_dtype, TC, (moe_gemm_tile_kernel<false, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (const bf16_t*)W, tile_expert,
+                                                                                        sorted_pair, gather, N, K, ws, act)));
     }
     return 0;
 }
@@ -782,8 +757,7 @@ extern "C" int spy_moe_gemm(void* C, int c_dtype, const void* A, int a_dtype, co
         return 0;
     }
     if (tiles_per_block > 0 && a_dtype == SPY_BF16 && w_dtype == SPY_BF16 && K % 8 == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0) {
-        const int rc = tiles_per_block >= 8 ? moe_gemm_mfma_launch<8>(C, c_dtype, A, W, tile_expert, sorted_pair, gather, gated, max_tiles, N, K, act, st)
-                                            : moe_gemm_mfma_launch<1>(C, c_dtype, A, W, tile_expert, sorted_pair, gather, gated, max_tiles, N, K, act, st);
+        const int rc = moe_gemm_mfma_launch(C, c_dtype, A, W, tile_expert, sorted_pair, gather, gated, tiles_per_block >= 8, max_tiles, N, K, act, st);
         if (rc) return rc;
         SPY_CHECK_LAUNCH("spy_moe_gemm (mfma)");
         return 0;

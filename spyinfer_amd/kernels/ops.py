@@ -1992,8 +1992,11 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
         _check(sorted_pair.shape == (rows,) and pair_row.shape == (P,) and tile_expert.shape == (max_tiles,) and groups.shape == (group_ints,),
                "moe_experts: the alignment does not fit")
     # bfloat16: the matrix cores, a block taking one row tile of an expert when the experts have few rows (decoding:
-    # blocks for the whole device), up to eight when they have many (an expert's matrices are read once per 128 rows)
-    per_block = 0 if not MOE_MFMA or x.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16 else (8 if P >= 16 * E else 1)
+    # blocks for the whole device), up to eight when they have many (an expert's matrices are read once per 128 rows).  Few: under 8 rows
+    # an expert on average (64 tokens of four choices, 32 experts of 2 x 3072 x 4096: 468 us a tile at a time, 422 by groups; 2 x 1536 x
+    # 2048: 123 / 124; 100 tokens 135 / 123), or 16 where K is no multiple of 64 and the kernel with groups does not stand
+    many = P >= (8 if K % 64 == 0 and F % 64 == 0 else 16) * E
+    per_block = 0 if not MOE_MFMA or x.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16 else (8 if many else 1)
     act = torch.empty((max_tiles * tm, F), dtype=x.dtype, device=dev)
     hip().call("spy_moe_gemm", _ptr(act), _code(act, "act"), _ptr(x), _code(x, "x"), _ptr(w_gate_up), _code(w_gate_up, "expert matrices"),
                _ptr(tile_expert), _ptr(sorted_pair), _ptr(groups), ctypes.c_int(P), ctypes.c_int(top), ctypes.c_int(1 if gated else 0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(F),
