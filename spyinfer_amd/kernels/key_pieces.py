@@ -15,17 +15,22 @@ import numpy as np
 MAX_PARTS = 32              # most parts of an (entry, kv head): what the kernel's merging block takes (8 kv heads of one long
                             # request give every compute unit a block only in 32 parts: 38 000 keys 39.5 us against 53.7 in 16)
 PIECE_UNITS = 256           # compute units that the pieces are dealt to; each runs two blocks at a time
-PIECE_MIN_BLOCKS = 8        # a part wants this many blocks of 32 keys at least (measured at 1100 keys, 1 to 4 requests: 4-8 parts best)
+PIECE_MIN_BLOCKS = 4        # a part wants this many blocks of 32 keys at least: one for each wave of its block
+PIECE_WAVES = 4             # waves of a block, which take its blocks of keys in turn
 PIECE_RECORD = 8            # ints per record
 # What the estimate of a cut's time is made of, in microseconds (measured with 8 kv heads of 128, 8 to 96 requests of
 # even and uneven lengths; the estimates are within 8 % rms of the kernel's times, and the cut they choose was the
 # fastest of those measured, to within the timings' noise, in every case):
 PIECE_START_US = 7.0        # from the kernel's start to a block's first keys, and its end
 PIECE_MERGE_US = 3.0        # the way of the parts through memory, once per step that cuts any entry
+PIECE_MERGE_PART = 1 / 80   # of it more for each part, of heads of 128, of the entry with the most
 PIECE_MERGE_MORE_US = 2.5   # each eight parts beyond sixteen of the entry with the most (the merging block asks for eight at a time)
 PIECE_ROUND_US = 4.0        # each further round of blocks on the units beyond the two that are there from the start
 PIECE_BLOCK_US = 0.45       # a unit's time for a block of 32 keys (16 KB) while it reads alone
 PIECE_SHARED_US = 0.56      # what all units reading at once add to it (the two add as squares)
+# Where the units are not what bounds a step, a block's time goes by its waves' turns: four blocks of keys cost what one does, and the
+# last part of an entry, which prepares the new key and stores it, takes a turn more (one request of 501 keys, 28 layers of 8 kv heads:
+# 1058 us a step whole, 1035 in two parts of 8 blocks, 987 in parts of 6, 6, 4 or of 4 blocks; of 250 keys 1075 whole, 1106 in parts of 4).
 
 
 def decode_pieces_capacity(entries: int, n_kv: int) -> int:
@@ -74,13 +79,17 @@ def _estimated_time(sizes_per_entry, n_kv, d=128) -> float:
     load = np.sort(load)
     steps = np.diff(load, prepend=0.0)
     reading = U - np.arange(U)                              # units still reading while the i-th fullest finishes
-    t = float((steps * np.sqrt(PIECE_BLOCK_US ** 2 + (reading * (PIECE_SHARED_US / U)) ** 2)).sum()) * (d / 128.0)
+    t = float((steps * np.sqrt(PIECE_BLOCK_US ** 2 + (reading * (PIECE_SHARED_US / U)) ** 2)).sum())
+    turns = -(-sizes_per_entry // PIECE_WAVES)
+    last = np.maximum(0, (sizes_per_entry > 0).sum(axis=1) - 1)
+    turns = turns + (np.arange(sizes_per_entry.shape[1])[None, :] == last[:, None])
+    t = max(t, PIECE_BLOCK_US * PIECE_WAVES * float(turns.max(initial=1))) * (d / 128.0)
     return t + PIECE_START_US + PIECE_ROUND_US * max(0, -(-int(s.shape[0]) // (2 * U)) - 1)
 
 
-def _merge_time(parts) -> float:
+def _merge_time(parts, d=128) -> float:
     """Microseconds that a step's merges add: the last block of the entry with the most parts asks for eight at a time."""
-    return PIECE_MERGE_US + PIECE_MERGE_MORE_US * max(0, -(-int(parts.max(initial=1)) // 8) - 2)
+    return PIECE_MERGE_US * (1 + PIECE_MERGE_PART * (d / 128.0) * int(parts.max(initial=1))) + PIECE_MERGE_MORE_US * max(0, -(-int(parts.max(initial=1)) // 8) - 2)
 
 
 def _fill_widths(nblk, n_kv):
@@ -119,13 +128,16 @@ def _piece_choice(nblk, n_kv, d=128):
     blocks, W being the whole step's blocks over the compute units or over twice as many (and no less than gives the
     longest entry 16 parts, or 32), an entry's parts of one size or W and a rest, or ("fill", True) (``_fill_widths``):
     whichever has the shortest estimated time.
-    Decided from the lengths rounded up to 8 blocks, so that a step is always cut the same way and the choice is looked
-    up in most steps (a request's rounded length changes once in 256 steps); the last choices are kept."""
-    coarse = nblk >> 3
-    key = (coarse.tobytes(), n_kv, d, MAX_PARTS, PIECE_UNITS, PIECE_MIN_BLOCKS, PIECE_START_US, PIECE_MERGE_US, PIECE_ROUND_US)
+    Decided from the lengths, of more than four requests rounded up to 8 blocks, so that a step is always cut the same way
+    and the choice (0.2 to 0.6 ms) is looked up in most steps: a request's rounded length changes once in 256 steps.  Of
+    few requests the lengths as they are (a choice in 8 to 32 steps): 8 blocks taken for 15 would be cut, and are faster
+    whole; 16 taken for 19 would get parts of 8, and are 4 % of a step faster in parts of 4.  The last choices are kept."""
+    shift = 0 if nblk.shape[0] <= 4 else 3
+    coarse = nblk >> shift
+    key = (coarse.tobytes(), n_kv, d, MAX_PARTS, PIECE_UNITS, PIECE_MIN_BLOCKS, PIECE_START_US, PIECE_MERGE_US, PIECE_MERGE_MORE_US, PIECE_ROUND_US)
     if key in _piece_choices:
         return _piece_choices[key]
-    rounded = (coarse << 3) + 7
+    rounded = (coarse << shift) + (1 << shift) - 1
     total = int(rounded.sum()) * n_kv
     if 4 * PIECE_UNITS * int(rounded.max(initial=1)) <= total:
         # the longest entry is no more than a quarter of a unit's even share: whole entries, dealt out as blocks end,
@@ -138,18 +150,21 @@ def _piece_choice(nblk, n_kv, d=128):
     best = (_estimated_time(whole, n_kv, d), None)
     # (the longest entry in at most 16 parts as well as in at most MAX_PARTS: more than 16 cost the merge further round trips)
     widths = {max(PIECE_MIN_BLOCKS, -(-longest // most), -(-total // (PIECE_UNITS * k))) for k in (1, 2) for most in (16, MAX_PARTS)}
+    seen = set()
     for width in sorted(widths):
         for even in (True, False):
             sizes, parts = _piece_sizes(rounded, width, even)
-            if int(parts.max(initial=1)) > 1:
-                t = _estimated_time(sizes, n_kv, d) + _merge_time(parts)
+            cut = sizes.tobytes()
+            if int(parts.max(initial=1)) > 1 and cut not in seen:
+                seen.add(cut)
+                t = _estimated_time(sizes, n_kv, d) + _merge_time(parts, d)
                 if t < best[0]:
                     best = (t, (width, even))
     per_entry = _fill_widths(rounded, n_kv)
     if per_entry is not None:
         sizes, parts = _piece_sizes(rounded, per_entry, True)
         if int(parts.max(initial=1)) > 1:
-            t = _estimated_time(sizes, n_kv, d) + _merge_time(parts)
+            t = _estimated_time(sizes, n_kv, d) + _merge_time(parts, d)
             if t < best[0]:
                 best = (t, ("fill", True))
     if len(_piece_choices) >= 64:
