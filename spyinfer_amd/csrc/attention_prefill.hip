@@ -38,7 +38,7 @@ __global__ __launch_bounds__(PF_ROWS / RT * 4, MINW) void attention_prefill_kern
     int P, int num_pages, const int* __restrict__ cu_q, const int* __restrict__ pos0, const int* __restrict__ kv_len,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ tile_entry, const int* __restrict__ tile_row0,
     int n_q, int n_kv, int d, float scale, int window, float softcap, int log2p, int num_tiles, int splits, float* __restrict__ ws, int out_tiles,
-    const float* __restrict__ dist, const float* __restrict__ sink, int chunk, OutGate og) {
+    const float* __restrict__ dist, const float* __restrict__ sink, int chunk, OutGate og, int paired) {
     // dist != null: [2, n_q] float32, a penalty on the distance taken off every (capped) score: dist[h] ln(1 + dist[n_q + h] (pos - key)).
     // sink != null: [n_q] float32, the softmax's denominator holds one more term, e^sink[h], that has no value: in the keys'
     // first part a row's running maximum starts at sink[h] with a sum of 1 (in one of the row's four lanes, whose sums are
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(PF_ROWS / RT * 4, MINW) void attention_prefill_kern
     __shared__ __attribute__((aligned(16))) bf16_t ks[PF_KEYS * KLD];
     __shared__ __attribute__((aligned(16))) bf16_t vs[DMAX * VLD];
 
-    // A block works on two tiles, one after the other: tile b and tile n - 1 - b of a list that the host
+    // A block works on two tiles (paired != 0), one after the other: tile b and tile n - 1 - b of a list that the host
     // has sorted by the number of keys a tile reads.  So every block has about the same work, which a
     // causal prompt's tiles alone (few keys early, many late) do not give.
     // Blocks go to the chip's 8 dies in turn, by their number in the grid, and each die has an L2 of its own.  So the
@@ -76,10 +76,11 @@ __global__ __launch_bounds__(PF_ROWS / RT * 4, MINW) void attention_prefill_kern
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63, r16 = lane & 15, g = lane >> 4;
     // With key parts (splits > 1: few tiles, many keys, e.g. a late portion of a long prompt) a block has one
-    // tile and the rounds of one part; the parts are merged by attention_merge_kernel.
+    // tile and the rounds of one part; the parts are merged by attention_merge_kernel.  So few tiles that every one
+    // has a compute unit for itself are not paired either.
     for (int which = 0; which < 2; ++which) {
     const int tile = which == 0 ? bx : num_tiles - 1 - bx;
-    if (which == 1 && (splits > 1 || tile <= bx)) break;
+    if (which == 1 && (!paired || tile <= bx)) break;
     __syncthreads();                                   // the first tile's last readers of LDS are done
     const int s = tile_entry[tile];
     const int row0 = tile_row0[tile];
@@ -391,7 +392,9 @@ extern "C" int64_t spy_attention_prefill_workspace(int num_tiles, int tile_rows,
 // Tiles of 256 rows against tiles of 128, same measurement: 92 against 73 us at 2048 tokens (128 blocks: half the CUs
 // idle), 125 against 133 at 3072, 170 against 195 at 4096, 607 against 675 at 8192, 2331 against 2565 at 16384 (0.94
 // PFLOP/s); the caller picks the tile size by the number of blocks.  One tile per block instead of two, so that a grid
-// of one block per CU becomes two per CU, was slower at every length (88 against 73 us at 2048 tokens).
+// of one block per CU becomes two per CU, was slower at every length (88 against 73 us at 2048 tokens); where one tile per
+// block leaves every block a CU of its own it is the faster way: 12.0 against 19.0 us at 100 tokens (32 tiles), 19.6 against
+// 26.6 at 389 (104), 30.7 against 36.9 at 800 (200), 35.9 against 41.8 at 1000 (256), 17.8 against 24.5 for two prompts of 300.
 // Measured on MI355X (256 CUs), 32 query heads of 128, microseconds per call for 2048 / 2304 / 3072 / 4096 / 8192
 // tokens of one prompt (256 / 288 / 384 / 512 / 1024 blocks): 4 waves of two row tiles 85 / 115 / 148 / 193 / 717;
 // 8 waves of one row tile with registers for one block per CU 65 / 130 / 165 / 217 / 807, with 128 registers (two
@@ -431,12 +434,13 @@ extern "C" int spy_attention_prefill(void* out, const void* q, const void* kc, c
     SPY_REQUIRE(!gate || (gate_ld >= (long long)n_q * d && gate_ld % 4 == 0 && ((uintptr_t)gate % 8) == 0),
                 "spy_attention_prefill: the gate's rows are too short or not aligned");
     const OutGate og = {(const bf16_t*)gate, gate_ld};
-    const dim3 grid(splits > 1 ? num_tiles : (num_tiles + 1) / 2, n_kv, splits);
+    const bool paired = splits == 1 && (long long)num_tiles * n_kv > cu_count();
+    const dim3 grid(paired ? (num_tiles + 1) / 2 : num_tiles, n_kv, splits);
     const dim3 mgrid(num_tiles * (tile_rows / 16), n_kv);
     const bool one_per_cu = (long long)grid.x * grid.y * grid.z <= cu_count();
 #define PF_ARGS (bf16_t*)out, (const bf16_t*)q, (const bf16_t*)kc, (const bf16_t*)vc, P, num_pages, cu_q, pos0, kv_len, block_table,   \
                 max_blocks, tile_entry, tile_row0, n_q, n_kv, d, scale, window, softcap, log2p, num_tiles, splits, ws, out_tiles, dist, sink, \
-                chunk, og
+                chunk, og, paired
     // (head sizes other than 64 and 128 keep the 4-wave shape: with conditions in the head-dim loops the other needs too many registers)
 #define PF_CASE(DM)                                                                                                              \
     if (tile_rows == 256) attention_prefill_kernel<DM, true, 2, 2, 256><<<grid, 512, 0, st>>>(PF_ARGS);                          \

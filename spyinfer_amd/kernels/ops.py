@@ -821,11 +821,11 @@ class AttentionMeta:
     head-in-group) rows for entries with few rows and 128-row tiles for entries with many, built
     for one group size ``tiles_group``; None if not built.
     ``big_rows``: rows of a "big" tile (128 or 256, see ``prefill_tile_rows``).
-    Host-side: S, T, max_blocks, max_kv_len, max_q_len.
+    Host-side: S, T, max_blocks, max_kv_len, max_q_len, max_big_keys.
     What the arrays say must be true: the kernels read entries, pages and pieces as they are given."""
 
     def __init__(self, cu_q, pos0, kv_len, block_table, token_entry, positions, S, T, max_blocks, max_kv_len, max_q_len,
-                 tiles=None, tiles_group=0, fixed_shape=False, big_rows=128, pieces=None):
+                 tiles=None, tiles_group=0, fixed_shape=False, big_rows=128, pieces=None, max_big_keys=None):
         self.cu_q, self.pos0, self.kv_len, self.block_table = cu_q, pos0, kv_len, block_table
         self.token_entry, self.positions = token_entry, positions
         self.S, self.T, self.max_blocks, self.max_kv_len, self.max_q_len = S, T, max_blocks, max_kv_len, max_q_len
@@ -836,6 +836,8 @@ class AttentionMeta:
         #: {(n_kv, window, head_dim): int32 [records, 8] on the device}: the keys of a step of single tokens cut into pieces by
         #: ``decode_pieces``, for the attention that takes the raw product; empty if not built
         self.pieces = pieces or {}
+        #: keys of the longest entry that has "big" tiles (not given: of the longest entry)
+        self.max_big_keys = max_kv_len if max_big_keys is None else max_big_keys
 
 
 MFMA_ATTENTION = True      # False forces the plain kernel for bfloat16 too (the kernel tests flip it; nothing else does)
@@ -863,6 +865,20 @@ def decode_pieces_ok(entries: int, tokens: int, act_dtype, n_kv: int, d: int) ->
 
 PREFILL_ATTENTION_MAX_HEAD_DIM = 128
 PREFILL_SPLIT_BELOW = 256   # fewer (128-row tile, kv head) pairs than this: split the keys to fill the chip
+
+
+def prefill_key_parts(blocks: int, keys: int) -> int:
+    """Into how many parts the keys of ``blocks`` (128-row tile, kv head) pairs are split when the tile with the most reads
+    ``keys``: the number with the least of what was measured, a round of 64 keys 1.6 us, the merge kernel 5 us and 0.045 us
+    for each part of a pair (its way through memory).  32 query heads of 128 in 8 groups, microseconds in 1 / 2 / 3 / 4 / 8
+    parts: 512 tokens of a new prompt 22.4 / 29.7 / 34.7 / 33.2 / 50.2, 1000 tokens 35.9 / 50.2 / 53.1 / 56.0 / 81.6; 300
+    tokens behind 1000: 41.5 / 36.6 / 35.8 / 39.5 / 50.5, 100 behind 2000: 60.1 / 41.9 / 36.4 / 34.1 / 36.0, 200 behind
+    4000: 111.3 / 70.3 / 56.8 / 49.8 / 55.4."""
+    if blocks >= PREFILL_SPLIT_BELOW:
+        return 1
+    rounds = -(-keys // 64)
+    return min(range(1, max(1, min(PREFILL_SPLIT_BELOW * 2 // blocks, keys // 256, 16)) + 1),
+               key=lambda parts: 1.6 * -(-rounds // parts) + (5 + 0.045 * parts * blocks if parts > 1 else 0))
 
 
 def prefill_attention_ok(d: int, page_size: int) -> bool:
@@ -1012,9 +1028,10 @@ def paged_attention(q: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: t
                               "kernel refuses; build 16-row tiles only (ops.prefill_attention_ok)" % (d, page_size))
         if n_big:
             # few tiles with many keys (a late portion of a long prompt): their keys are split into parts as well
-            bsplits = 1
-            if n_big * n_kv < PREFILL_SPLIT_BELOW:
-                bsplits = max(1, min(PREFILL_SPLIT_BELOW * 2 // (n_big * n_kv), max_keys // 256, 16))
+            big_keys = min(meta.max_big_keys, max_keys)
+            if win:
+                big_keys = min(big_keys, win + meta.big_rows // group + 1)
+            bsplits = prefill_key_parts(n_big * n_kv, big_keys)
             _check(meta.big_rows in (128, 256), "paged_attention: tiles of 128 or 256 rows expected")
             bws_floats = hip().lib.spy_attention_prefill_workspace(ctypes.c_int(n_big), ctypes.c_int(meta.big_rows), ctypes.c_int(n_kv),
                                                                    ctypes.c_int(d), ctypes.c_int(bsplits))

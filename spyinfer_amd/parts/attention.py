@@ -81,6 +81,7 @@ def plan_attention_tiles(batch, group_size: int, big_rows: int = 0, key_parts: b
         batch.add_array("tile_entry_%s_%s" % (kind, name), tile_entry)
         batch.add_array("tile_row0_%s_%s" % (kind, name), tile_row0)
     batch.shared[note] = counts
+    batch.shared[("attention_big_keys",) + note[1:]] = int(batch.host_array("kv_len")[big].max(initial=1))
 
 
 def plan_decode_pieces(batch, n_kv: int, window: int, head_dim: int) -> None:
@@ -109,7 +110,8 @@ def attention_meta(batch, group: int, group_size: int, big_rows: int = 0, chunk:
         meta = ops.AttentionMeta(batch.array("cu_q"), batch.array("pos0"), batch.array("kv_len"), batch.block_table(group),
                                  batch.array("token_entry"), batch.array("positions"), batch.S, batch.T, batch.max_blocks[group],
                                  batch.max_kv_len, batch.max_q_len, tiles, group_size, fixed_shape=batch.fixed_shape,
-                                 big_rows=big_rows or 128, pieces=pieces)
+                                 big_rows=big_rows or 128, pieces=pieces,
+                                 max_big_keys=batch.shared.get(("attention_big_keys", group_size, big_rows, chunk)))
         batch.shared[note] = meta
     return meta
 
