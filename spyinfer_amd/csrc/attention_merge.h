@@ -5,6 +5,17 @@
 #include "common.h"
 #include <math.h>
 
+// Compute units of the device (asked for once).
+inline long long attention_compute_units() {
+    static long long cus = 0;
+    if (cus == 0) {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        cus = n;
+    }
+    return cus;
+}
+
 // tanh for capped scores, float32: 1 - 2 / (1 + e^2x); absolute error of a few 1e-7 (the exponential overflows to the
 // right limit on both sides)
 __device__ __forceinline__ float capped_tanh(float x) { return 1.0f - 2.0f / (1.0f + __expf(2.0f * x)); }

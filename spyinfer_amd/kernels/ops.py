@@ -71,7 +71,7 @@ class _Hip:
         self.lib = _build.load()
         self.lib.spy_last_error.restype = ctypes.c_char_p
         for name in ("spy_embedding", "spy_add_rmsnorm", "spy_rmsnorm", "spy_gemm", "spy_qknorm_rope_store",
-                     "spy_attention_generic", "spy_attention_f32", "spy_attention_f32_workspace", "spy_attention_mfma", "spy_attention_mfma_workspace", "spy_attention_mfma_part_workspace", "spy_attention_prefill",
+                     "spy_attention_generic", "spy_attention_f32", "spy_attention_f32_workspace", "spy_attention_mfma", "spy_attention_mfma_workspace", "spy_attention_mfma_part_workspace", "spy_attention_prefill", "spy_attention_mixed",
                      "spy_attention_prefill_workspace", "spy_swiglu", "spy_untile_weight",
                      "spy_sample", "spy_sample_workspace", "spy_gemm_skinny", "spy_gemm_skinny_swiglu",
                      "spy_gemm_decode", "spy_gemm_decode_workspace", "spy_embedding_sumsq", "spy_sample_static", "spy_measure_read",
@@ -821,11 +821,11 @@ class AttentionMeta:
     head-in-group) rows for entries with few rows and 128-row tiles for entries with many, built
     for one group size ``tiles_group``; None if not built.
     ``big_rows``: rows of a "big" tile (128 or 256, see ``prefill_tile_rows``).
-    Host-side: S, T, max_blocks, max_kv_len, max_q_len, max_big_keys.
+    Host-side: S, T, max_blocks, max_kv_len, max_q_len, max_big_keys, max_small_keys.
     What the arrays say must be true: the kernels read entries, pages and pieces as they are given."""
 
     def __init__(self, cu_q, pos0, kv_len, block_table, token_entry, positions, S, T, max_blocks, max_kv_len, max_q_len,
-                 tiles=None, tiles_group=0, fixed_shape=False, big_rows=128, pieces=None, max_big_keys=None):
+                 tiles=None, tiles_group=0, fixed_shape=False, big_rows=128, pieces=None, max_big_keys=None, max_small_keys=None):
         self.cu_q, self.pos0, self.kv_len, self.block_table = cu_q, pos0, kv_len, block_table
         self.token_entry, self.positions = token_entry, positions
         self.S, self.T, self.max_blocks, self.max_kv_len, self.max_q_len = S, T, max_blocks, max_kv_len, max_q_len
@@ -836,8 +836,9 @@ class AttentionMeta:
         #: {(n_kv, window, head_dim): int32 [records, 8] on the device}: the keys of a step of single tokens cut into pieces by
         #: ``decode_pieces``, for the attention that takes the raw product; empty if not built
         self.pieces = pieces or {}
-        #: keys of the longest entry that has "big" tiles (not given: of the longest entry)
+        #: keys of the longest entry that has "big" tiles, and of the longest with "small" ones (not given: of the longest entry)
         self.max_big_keys = max_kv_len if max_big_keys is None else max_big_keys
+        self.max_small_keys = max_kv_len if max_small_keys is None else max_small_keys
 
 
 MFMA_ATTENTION = True      # False forces the plain kernel for bfloat16 too (the kernel tests flip it; nothing else does)
@@ -876,9 +877,26 @@ def prefill_key_parts(blocks: int, keys: int) -> int:
     4000: 111.3 / 70.3 / 56.8 / 49.8 / 55.4."""
     if blocks >= PREFILL_SPLIT_BELOW:
         return 1
-    rounds = -(-keys // 64)
-    return min(range(1, max(1, min(PREFILL_SPLIT_BELOW * 2 // blocks, keys // 256, 16)) + 1),
-               key=lambda parts: 1.6 * -(-rounds // parts) + (5 + 0.045 * parts * blocks if parts > 1 else 0))
+    return min(range(1, max(1, min(PREFILL_SPLIT_BELOW * 2 // blocks, keys // 256, 16)) + 1), key=lambda parts: _prefill_us(blocks, keys, parts))
+
+
+def _prefill_us(blocks: int, keys: int, parts: int) -> float:
+    return 8 + 1.6 * -(-(-(-keys // 64)) // parts) + (5 + 0.045 * parts * blocks if parts > 1 else 0)
+
+
+def mixed_attention_pays(blocks: int, keys: int, small_keys: int) -> bool:
+    """Whether entries with many rows (``blocks`` pairs of a 128-row tile and a kv head, the most keys ``keys``) and entries
+    with few (the most ``small_keys``) go in one launch, all keys in one part: where its longest block, a turn of eight
+    waves over 256 keys taking 3.1 us, ends before two launches would, the second of which takes 12 us at least, and the
+    large tiles have a compute unit each or share one by twos (more of them run faster with half the registers, 129 against
+    148 us at 3072 tokens).  32 query heads of 128 in 8 groups, microseconds apart / together: 389 tokens beside 20 single
+    tokens of 60 to 700 keys 35.9 / 18.9, of 1300 keys 48.5 / 34.0, beside 100 of 100 to 200 keys 42.8 / 33.5; 1000 tokens
+    beside the first 20 54.2 / 36.3; 2000 tokens beside 10 82 / 73; 800 beside three of 3000 keys 48 / 45; 100 beside one of
+    8000, whose keys go in parts otherwise, 30.4 / 98.7; prompts of 7 and 60 to 600 tokens, 16 heads, 32.8 / 23.7."""
+    if blocks > 2 * PREFILL_SPLIT_BELOW:
+        return False
+    together = max(_prefill_us(blocks, keys, 1), 8 + 3.1 * -(-small_keys // 256))
+    return together <= _prefill_us(blocks, keys, prefill_key_parts(blocks, keys)) + 12
 
 
 def prefill_attention_ok(d: int, page_size: int) -> bool:
@@ -1032,6 +1050,12 @@ def paged_attention(q: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: t
             if win:
                 big_keys = min(big_keys, win + meta.big_rows // group + 1)
             bsplits = prefill_key_parts(n_big * n_kv, big_keys)
+            if n_small and raw is None and not meta.fixed_shape and d in (64, 128) and meta.big_rows == 128 \
+                    and mixed_attention_pays(n_big * n_kv, big_keys, min(meta.max_small_keys, max_keys, win + 16 if win else max_keys)):
+                hip().call("spy_attention_mixed", _ptr(out), _ptr(q), _ptr(k_cache), _ptr(v_cache), *common, _ptr(big_entry), _ptr(big_row0),
+                           ctypes.c_int(n_big), _ptr(small_entry), _ptr(small_row0), ctypes.c_int(n_small), *sizes,
+                           ctypes.c_int(operand.tiles if operand is not None else 0), *extras, _Hip.stream())
+                return operand if operand is not None else out
             _check(meta.big_rows in (128, 256), "paged_attention: tiles of 128 or 256 rows expected")
             bws_floats = hip().lib.spy_attention_prefill_workspace(ctypes.c_int(n_big), ctypes.c_int(meta.big_rows), ctypes.c_int(n_kv),
                                                                    ctypes.c_int(d), ctypes.c_int(bsplits))

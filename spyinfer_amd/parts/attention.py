@@ -81,7 +81,8 @@ def plan_attention_tiles(batch, group_size: int, big_rows: int = 0, key_parts: b
         batch.add_array("tile_entry_%s_%s" % (kind, name), tile_entry)
         batch.add_array("tile_row0_%s_%s" % (kind, name), tile_row0)
     batch.shared[note] = counts
-    batch.shared[("attention_big_keys",) + note[1:]] = int(batch.host_array("kv_len")[big].max(initial=1))
+    kv_len = batch.host_array("kv_len")
+    batch.shared[("attention_longest",) + note[1:]] = tuple(int(kv_len[m].max(initial=1)) for m in (big, ~big))
 
 
 def plan_decode_pieces(batch, n_kv: int, window: int, head_dim: int) -> None:
@@ -107,11 +108,12 @@ def attention_meta(batch, group: int, group_size: int, big_rows: int = 0, chunk:
             tiles = {kind: (batch.array("tile_entry_%s_%s" % (kind, name)), batch.array("tile_row0_%s_%s" % (kind, name)), n) for kind, n in counts.items()}
         pieces = {key[1:]: batch.array("decode_pieces_%d_%d_%d" % key[1:]).view(-1, key_pieces.PIECE_RECORD)
                   for key in batch.shared if isinstance(key, tuple) and key[0] == "decode_pieces"}
+        big_keys, small_keys = batch.shared.get(("attention_longest",) + note[2:], (None, None))
         meta = ops.AttentionMeta(batch.array("cu_q"), batch.array("pos0"), batch.array("kv_len"), batch.block_table(group),
                                  batch.array("token_entry"), batch.array("positions"), batch.S, batch.T, batch.max_blocks[group],
                                  batch.max_kv_len, batch.max_q_len, tiles, group_size, fixed_shape=batch.fixed_shape,
                                  big_rows=big_rows or 128, pieces=pieces,
-                                 max_big_keys=batch.shared.get(("attention_big_keys", group_size, big_rows, chunk)))
+                                 max_big_keys=big_keys, max_small_keys=small_keys)
         batch.shared[note] = meta
     return meta
 
