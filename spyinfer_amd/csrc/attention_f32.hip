@@ -58,8 +58,9 @@ __device__ __forceinline__ void af_store(const AfArgs& a, int t, int col, int wi
     *reinterpret_cast<float4*>(a.out + (size_t)t * width + col) = y;
 }
 
+// (two blocks a compute unit: left to itself the compiler takes 260 registers for heads of 128 and leaves room for one)
 template <int D>
-__global__ __launch_bounds__(AF * 64) void attention_f32_kernel(AfArgs a, int tiles) {
+__global__ __launch_bounds__(AF * 64, 2) void attention_f32_kernel(AfArgs a, int tiles) {
     constexpr int DT = D / 16;
     __shared__ float lo_[AF][DT][64][4];
     __shared__ float lm_[AF][16], ll_[AF][16];
@@ -128,13 +129,16 @@ __global__ __launch_bounds__(AF * 64) void attention_f32_kernel(AfArgs a, int ti
             page = page_n;
             page_n = page_of(b + 2 * AF);
             load_k(b + AF, page);                                                          // (behind the part's last block: that block again)
+            const int n_ok = page_ok ? hi - c0 + 1 : 0;                                    // of this lane's keys, those that exist
             float sc[4], bm = -INFINITY;
+            bool hidden = false;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 float x = (s0[j] + s1[j]) * a.scale;
                 if (a.softcap > 0.f) x = a.softcap * tanhf(x / a.softcap);
                 if (a.dist) x -= d1 * log1pf(d2 * (float)(p0 + tq - (c0 + j)));
                 const bool seen = c0 + j <= pos && c0 + j >= first && page_ok;
+                hidden |= row_ok && !seen && j < n_ok;
                 sc[j] = seen ? x : -INFINITY;
                 bm = fmaxf(bm, sc[j]);
             }
@@ -153,14 +157,43 @@ __global__ __launch_bounds__(AF * 64) void attention_f32_kernel(AfArgs a, int ti
                 l += sc[j];
             }
             // values of keys that do not exist (behind the request's end, in a page that is gone) may be anything
-            const int n_ok = page_ok ? hi - c0 + 1 : 0;
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int i = 0; i < DT; ++i)
 #pragma unroll
-                for (int i = 0; i < DT; ++i) {
-                    const float x = j < n_ok ? v[i][j] : 0.f;
-                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, sc[j], acc[i], 0, 0, 0);
-                }
+                for (int j = 0; j < 4; ++j) v[i][j] = j < n_ok ? v[i][j] : 0.f;
+            // A key that some rows read and others do not has weight zero for these, which takes no infinity and no NaN away:
+            // a block with both goes key by key, each row by its own keys
+            bool odd = false;
+            if (__any(hidden)) {
+                af_f32x4_t z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < DT; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) z[j] = fmaf(v[i][j], 0.f, z[j]);
+                odd = __any(!(z[0] + z[1] + z[2] + z[3] == 0.f));
+            }
+            if (!odd) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int i = 0; i < DT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i][j], sc[j], acc[i], 0, 0, 0);
+            } else {
+#pragma unroll 1
+                for (int kg = 0; kg < 4; ++kg)                                             // (lane kg of a group of four has its keys)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int key = lo + 16 * b + 4 * kg + j;
+                        const bool reads = key <= pos && key >= first && page_ok;
+                        const float w = __shfl(sc[j], 16 * kg + r, 64);
+#pragma unroll
+                        for (int i = 0; i < DT; ++i)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const float x = __shfl(v[i][j], 16 * kg + 4 * g + e, 64);
+                                if (reads) acc[i][e] = fmaf(w, x, acc[i][e]);
+                            }
+                    }
+            }
         }
     }
     l += __shfl_xor(l, 16, 64);

@@ -88,3 +88,36 @@ def test_float32_attention(case, monkeypatch):
     assert called == ["spy_attention_f32"]
     # scores up to 100 here: each is rounded by d / 2 products or so, which moves a weight by that much relatively: 2e-5 of the largest value
     assert float((out - ref).abs().max()) < 2e-5 * max(1.0, float(vc[~vc.isnan()].abs().max()))
+
+
+# n_q, n_kv, d, page, entries (cached, new), options, (entry, position, kv head, dim, value) of what is not finite
+HIDDEN = [
+    (4, 2, 64, 16, [(0, 21)], {}, [(0, 9, 0, 3, "inf"), (0, 17, 1, 63, "nan")]),                    # a later token of the portion
+    (8, 8, 128, 16, [(300, 20), (5, 2)], {}, [(0, 311, 2, 100, "-inf"), (1, 6, 7, 0, "nan")]),       # the same behind keys in parts
+    (8, 2, 128, 32, [(70, 3)], dict(window=40), [(0, 31, 1, 5, "nan"), (0, 32, 0, 77, "inf")]),      # just before a window, in its first block
+    (8, 2, 64, 16, [(88, 1), (86, 12)], dict(chunk=41), [(0, 81, 0, 1, "inf"), (1, 80, 1, 2, "nan")]),
+    (8, 1, 128, 16, [(0, 18)], dict(window=5), [(0, 15, 0, 9, "inf"), (0, 15, 0, 10, "-inf"), (0, 16, 0, 9, "inf")]),
+]
+
+
+@pytest.mark.parametrize("case", range(len(HIDDEN)))
+def test_a_value_that_is_not_finite_stays_with_the_rows_that_read_it(case):
+    """Rows of one 16-row tile read different keys; a weight of zero would not take an infinity or a NaN away."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    n_q, n_kv, d, P, entries, opt, odd = HIDDEN[case]
+    q, kc, vc, bt, te, ps, meta = make_attention_case(torch.float32, dev, n_q, n_kv, d, P, entries, seed=130 + case)
+    for s, c, hk, j, x in odd:
+        vc[bt[s][c // P], hk, j, c % P] = float(x)
+    G = n_q // n_kv
+    rows = [(s, r0) for s, (_, n) in enumerate(entries) for r0 in range(0, n * G, 16)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
+    meta.tiles = {"small": (i32([s for s, _ in rows]), i32([r for _, r in rows]), len(rows)), "big": (i32([]), i32([]), 0)}
+    ref = plain(q, kc, vc, P, bt, te, ps, n_q, n_kv, d, d ** -0.5, **opt)
+    on = dict(opt)
+    out = ops.paged_attention(q.to(dev), kc.to(dev), vc.to(dev), P, meta, n_q, n_kv, d, d ** -0.5, on.pop("window", None), **on).cpu().double()
+    fine = ref.isfinite()
+    assert bool(fine.any()) and (case == 3 or not bool(fine.all()))
+    assert bool(out[fine].isfinite().all())
+    assert float((out - ref)[fine].abs().max()) < 2e-5 * float(vc[vc.isfinite()].abs().max())      # (as above)
+    assert torch.equal(torch.nan_to_num(out[~fine], nan=7.0), torch.nan_to_num(ref[~fine], nan=7.0))
