@@ -15,22 +15,24 @@ import numpy as np
 MAX_PARTS = 32              # most parts of an (entry, kv head): what the kernel's merging block takes (8 kv heads of one long
                             # request give every compute unit a block only in 32 parts: 38 000 keys 39.5 us against 53.7 in 16)
 PIECE_UNITS = 256           # compute units that the pieces are dealt to; each runs two blocks at a time
-PIECE_MIN_BLOCKS = 4        # a part wants this many blocks of 32 keys at least: one for each wave of its block
-PIECE_WAVES = 4             # waves of a block, which take its blocks of keys in turn
+PIECE_MIN_BLOCKS = 8        # a part wants this many blocks of 32 keys at least (measured at 1100 keys, 1 to 4 requests: 4-8 parts best)
 PIECE_RECORD = 8            # ints per record
 # What the estimate of a cut's time is made of, in microseconds (measured with 8 kv heads of 128, 8 to 96 requests of
 # even and uneven lengths; the estimates are within 8 % rms of the kernel's times, and the cut they choose was the
 # fastest of those measured, to within the timings' noise, in every case):
 PIECE_START_US = 7.0        # from the kernel's start to a block's first keys, and its end
 PIECE_MERGE_US = 3.0        # the way of the parts through memory, once per step that cuts any entry
-PIECE_MERGE_PART = 1 / 80   # of it more for each part, of heads of 128, of the entry with the most
 PIECE_MERGE_MORE_US = 2.5   # each eight parts beyond sixteen of the entry with the most (the merging block asks for eight at a time)
 PIECE_ROUND_US = 4.0        # each further round of blocks on the units beyond the two that are there from the start
 PIECE_BLOCK_US = 0.45       # a unit's time for a block of 32 keys (16 KB) while it reads alone
 PIECE_SHARED_US = 0.56      # what all units reading at once add to it (the two add as squares)
-# Where the units are not what bounds a step, a block's time goes by its waves' turns: four blocks of keys cost what one does, and the
-# last part of an entry, which prepares the new key and stores it, takes a turn more (one request of 501 keys, 28 layers of 8 kv heads:
-# 1058 us a step whole, 1035 in two parts of 8 blocks, 987 in parts of 6, 6, 4 or of 4 blocks; of 250 keys 1075 whole, 1106 in parts of 4).
+# Few requests, whose pieces all have a unit of their own: there a piece's time goes by the turns of its block's waves, four blocks
+# of keys costing what one does, and the last part of an entry, which prepares the new key and stores it, takes a turn more.
+PIECE_FEW = 4               # most requests whose lengths are taken as they are (a choice in 8 to 32 steps)
+PIECE_WAVES = 4             # waves of a block, which take its blocks of keys in turn
+PIECE_TURN_US = 1.75        # a turn (heads of 128: 1 to 4 requests of 130 to 1300 keys)
+PIECE_PARTS_US = 2.35       # the merge of an entry's parts, and
+PIECE_PART_US = 0.17        # each part of it, up to the eight that the merging block asks for at a time
 
 
 def decode_pieces_capacity(entries: int, n_kv: int) -> int:
@@ -39,12 +41,13 @@ def decode_pieces_capacity(entries: int, n_kv: int) -> int:
     return 2 * PIECE_UNITS + entries * n_kv
 
 
-def _piece_sizes(nblk, width, even):
+def _piece_sizes(nblk, width, even, least=None):
     """How entries of ``nblk`` blocks of 32 keys are cut into parts of at most ``width`` blocks: [entries, MAX_PARTS]
     sizes (0: no such part) and the numbers of parts.  Parts of one size and the rest (the last part, which also prepares
     and stores the new key, is the shortest); a rest shorter than half of what a part may be joins the part before it.
     ``even``: the size is the least that gives the entry no more parts than ``width`` does (37 blocks at width 12: 10,
-    10, 10, 7 instead of 12, 12, 13).  ``width``: one for all entries, or one per entry."""
+    10, 10, 7 instead of 12, 12, 13).  ``width``: one for all entries, or one per entry.  ``least``: blocks that a part wants
+    (None: PIECE_MIN_BLOCKS)."""
     n = nblk.astype(np.int64)
     idx = np.arange(MAX_PARTS, dtype=np.int64)[None, :]
     w = np.broadcast_to(np.asarray(width, dtype=np.int64), n.shape).copy()      # (one width, or one per entry)
@@ -52,7 +55,7 @@ def _piece_sizes(nblk, width, even):
         w = np.maximum(1, -(-n // np.maximum(1, -(-n // width))))
     full = n // w
     rest = n - full * w
-    joined = (rest > 0) & (2 * rest < np.minimum(PIECE_MIN_BLOCKS, w)) & (full > 0)
+    joined = (rest > 0) & (2 * rest < np.minimum(PIECE_MIN_BLOCKS if least is None else least, w)) & (full > 0)
     parts = np.maximum(1, full + ((rest > 0) & ~joined))
     sizes = np.where(idx < full[:, None], w[:, None], 0)
     last = (parts - 1)[:, None]
@@ -79,17 +82,13 @@ def _estimated_time(sizes_per_entry, n_kv, d=128) -> float:
     load = np.sort(load)
     steps = np.diff(load, prepend=0.0)
     reading = U - np.arange(U)                              # units still reading while the i-th fullest finishes
-    t = float((steps * np.sqrt(PIECE_BLOCK_US ** 2 + (reading * (PIECE_SHARED_US / U)) ** 2)).sum())
-    turns = -(-sizes_per_entry // PIECE_WAVES)
-    last = np.maximum(0, (sizes_per_entry > 0).sum(axis=1) - 1)
-    turns = turns + (np.arange(sizes_per_entry.shape[1])[None, :] == last[:, None])
-    t = max(t, PIECE_BLOCK_US * PIECE_WAVES * float(turns.max(initial=1))) * (d / 128.0)
+    t = float((steps * np.sqrt(PIECE_BLOCK_US ** 2 + (reading * (PIECE_SHARED_US / U)) ** 2)).sum()) * (d / 128.0)
     return t + PIECE_START_US + PIECE_ROUND_US * max(0, -(-int(s.shape[0]) // (2 * U)) - 1)
 
 
-def _merge_time(parts, d=128) -> float:
+def _merge_time(parts) -> float:
     """Microseconds that a step's merges add: the last block of the entry with the most parts asks for eight at a time."""
-    return PIECE_MERGE_US * (1 + PIECE_MERGE_PART * (d / 128.0) * int(parts.max(initial=1))) + PIECE_MERGE_MORE_US * max(0, -(-int(parts.max(initial=1)) // 8) - 2)
+    return PIECE_MERGE_US + PIECE_MERGE_MORE_US * max(0, -(-int(parts.max(initial=1)) // 8) - 2)
 
 
 def _fill_widths(nblk, n_kv):
@@ -120,6 +119,43 @@ def _fill_widths(nblk, n_kv):
     return np.where(first, np.maximum(share, floor), np.maximum(fine, floor))
 
 
+def _few_width(nblk, n_kv):
+    """The width for up to PIECE_FEW requests of heads of 128 whose pieces all find a unit of their own: None (whole), parts of at
+    most W blocks (W, even, of PIECE_WAVES blocks at least), or False where the entries are too long for that (more than eight parts or
+    256 pieces at 8 blocks a part).  Parts of four blocks where every part is one turn then; else the width of 5 to 8 with the fewest
+    turns, and of these the fewest parts.  One request of 8 kv heads, microseconds whole / in parts of 4 / of 8, and of what is
+    taken: 8 blocks 10.8 / 11.7 / -, whole; 13 blocks 13.8 / 13.7 / 13.6, 5: 12.3; 16 blocks 13.9 / 12.2 / 13.5, 4; 22 blocks 18.3 / 12.6 /
+    14.2, 5: 12.5; 25 blocks 19.9 / 14.3 / 12.7, 7 (parts of 4, 5 or 6 leave a block over, so that the last part has three turns); 37
+    blocks 25.4 / 15.8 (nine parts) / 14.4, 7: 12.9; four requests of 37 blocks 26.4 / 16.8 / 15.0, 7: 13.8.  (A rule that took parts of
+    four blocks for any number of requests was up to an eighth slower than parts of eight: 8 requests of 700 keys 16.2 / 15.5.)"""
+    lens = nblk.tolist()
+    longest = max(lens)
+    if longest > 64:
+        return False
+    best = None
+    for width in range(PIECE_MIN_BLOCKS, PIECE_WAVES - 1, -1):
+        pieces = most = turns = 0
+        time = 0.0
+        for n in lens:                                      # (as _piece_sizes cuts; a choice in numpy takes 0.1 ms)
+            w = -(-n // max(1, -(-n // width)))
+            parts, rest = divmod(n, w) if w else (1, 0)
+            if rest and not (parts and 2 * rest < min(PIECE_WAVES, w)):
+                parts, last = parts + 1, rest
+            else:
+                last = w + rest
+            t = max(-(-w // PIECE_WAVES) if parts > 1 else 0, -(-last // PIECE_WAVES) + 1)
+            pieces, most, turns = pieces + parts * n_kv, max(most, parts), max(turns, t)
+            time = max(time, PIECE_TURN_US * t + (PIECE_PARTS_US + PIECE_PART_US * parts if parts > 1 else 0.0))
+        if most > 8 or pieces > PIECE_UNITS:
+            break
+        if best is None or turns < best[0] or (width == PIECE_WAVES and turns == 2):
+            best = (turns, width, time)
+    if best is None:
+        return False
+    whole = PIECE_TURN_US * (1 + -(-longest // PIECE_WAVES))
+    return None if whole <= best[2] else (best[1], True, PIECE_WAVES)
+
+
 _piece_choices = {}
 
 
@@ -128,16 +164,24 @@ def _piece_choice(nblk, n_kv, d=128):
     blocks, W being the whole step's blocks over the compute units or over twice as many (and no less than gives the
     longest entry 16 parts, or 32), an entry's parts of one size or W and a rest, or ("fill", True) (``_fill_widths``):
     whichever has the shortest estimated time.
-    Decided from the lengths, of more than four requests rounded up to 8 blocks, so that a step is always cut the same way
-    and the choice (0.2 to 0.6 ms) is looked up in most steps: a request's rounded length changes once in 256 steps.  Of
-    few requests the lengths as they are (a choice in 8 to 32 steps): 8 blocks taken for 15 would be cut, and are faster
-    whole; 16 taken for 19 would get parts of 8, and are 4 % of a step faster in parts of 4.  The last choices are kept."""
-    shift = 0 if nblk.shape[0] <= 4 else 3
-    coarse = nblk >> shift
-    key = (coarse.tobytes(), n_kv, d, MAX_PARTS, PIECE_UNITS, PIECE_MIN_BLOCKS, PIECE_START_US, PIECE_MERGE_US, PIECE_MERGE_MORE_US, PIECE_ROUND_US)
+    Decided from the lengths rounded up to 8 blocks, so that a step is always cut the same way and the choice is looked
+    up in most steps (a request's rounded length changes once in 256 steps); the last choices are kept.  Few requests: by their
+    lengths as they are where ``_few_width`` stands."""
+    if nblk.shape[0] <= PIECE_FEW and d == 128:
+        key = (nblk.tobytes(), n_kv, PIECE_UNITS, PIECE_MIN_BLOCKS)
+        few = _piece_choices.get(key, 0)
+        if few == 0:
+            few = _few_width(nblk, n_kv)
+            if len(_piece_choices) >= 64:
+                _piece_choices.pop(next(iter(_piece_choices)))
+            _piece_choices[key] = few
+        if few is not False:
+            return few
+    coarse = nblk >> 3
+    key = (coarse.tobytes(), n_kv, d, MAX_PARTS, PIECE_UNITS, PIECE_MIN_BLOCKS, PIECE_START_US, PIECE_MERGE_US, PIECE_ROUND_US)
     if key in _piece_choices:
         return _piece_choices[key]
-    rounded = (coarse << shift) + (1 << shift) - 1
+    rounded = (coarse << 3) + 7
     total = int(rounded.sum()) * n_kv
     if 4 * PIECE_UNITS * int(rounded.max(initial=1)) <= total:
         # the longest entry is no more than a quarter of a unit's even share: whole entries, dealt out as blocks end,
@@ -150,21 +194,18 @@ def _piece_choice(nblk, n_kv, d=128):
     best = (_estimated_time(whole, n_kv, d), None)
     # (the longest entry in at most 16 parts as well as in at most MAX_PARTS: more than 16 cost the merge further round trips)
     widths = {max(PIECE_MIN_BLOCKS, -(-longest // most), -(-total // (PIECE_UNITS * k))) for k in (1, 2) for most in (16, MAX_PARTS)}
-    seen = set()
     for width in sorted(widths):
         for even in (True, False):
             sizes, parts = _piece_sizes(rounded, width, even)
-            cut = sizes.tobytes()
-            if int(parts.max(initial=1)) > 1 and cut not in seen:
-                seen.add(cut)
-                t = _estimated_time(sizes, n_kv, d) + _merge_time(parts, d)
+            if int(parts.max(initial=1)) > 1:
+                t = _estimated_time(sizes, n_kv, d) + _merge_time(parts)
                 if t < best[0]:
                     best = (t, (width, even))
     per_entry = _fill_widths(rounded, n_kv)
     if per_entry is not None:
         sizes, parts = _piece_sizes(rounded, per_entry, True)
         if int(parts.max(initial=1)) > 1:
-            t = _estimated_time(sizes, n_kv, d) + _merge_time(parts, d)
+            t = _estimated_time(sizes, n_kv, d) + _merge_time(parts)
             if t < best[0]:
                 best = (t, ("fill", True))
     if len(_piece_choices) >= 64:
@@ -181,7 +222,7 @@ def _piece_plan(nblk, n_kv, d=128):
         choice = None if widths is None else (widths, True)
     if choice is None:
         return nblk[:, None] * (np.arange(MAX_PARTS)[None, :] == 0), np.ones(nblk.shape[0], dtype=np.int64)
-    return _piece_sizes(nblk, choice[0], choice[1])
+    return _piece_sizes(nblk, *choice)
 
 
 def decode_pieces(kv_len, n_kv: int, window: int = 0, capacity: Optional[int] = None, head_dim: int = 128):
