@@ -36,6 +36,9 @@
 
 typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
+// f32x4_t read from LDS as two pairs of 32-bit values (the alignment decides which instruction the compiler takes): the merge of a
+// block's waves is faster this way than with 16-byte reads (8 requests of 1153 keys 15.9 against 16.6 us, one of 501 12.6 / 13.3)
+typedef f32x4_t __attribute__((aligned(4))) f32x4_loose_t;
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
 
 __device__ __forceinline__ bf16x8_t zero8() { return bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0}; }
@@ -140,9 +143,9 @@ __device__ __forceinline__ void attention_mfma_body(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, bf16_t* kc, bf16_t* vc,
     int P, int num_pages, const int* __restrict__ cu_q, const int* __restrict__ pos0, const int* __restrict__ kv_len,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ tile_entry, const int* __restrict__ tile_row0,
-    int n_q, int n_kv, int d, float scale, int window, float softcap, int splits, float* __restrict__ ws, const FusedQKV& fz, int out_tiles,
+    int n_q, int n_kv, int d, float scale, int window, float softcap, int splits, float* __restrict__ ws, FusedQKV fz, int out_tiles,
     unsigned* counters, int log2p, const int* __restrict__ pieces, const float* __restrict__ dist,
-    const float* __restrict__ sink, int chunk, const OutGate& og, int tile, int hk, int sp, float* lds) {
+    const float* __restrict__ sink, int chunk, OutGate og, int tile, int hk, int sp, float* lds) {
     // dist != null: [2, n_q] float32, a penalty on the distance taken off every (capped) score: dist[h] ln(1 + dist[n_q + h] (pos - key)).
     // sink != null: [n_q] float32, the softmax's denominator holds one more term, e^sink[h], that has no value: the first wave
     // of the keys' first part starts its running maximum at sink[h] with a sum of 1 (in one of a row's four lanes, whose sums
@@ -504,7 +507,7 @@ __device__ __forceinline__ void attention_mfma_body(
             l += lw[w] * a;
 #pragma unroll
             for (int i = 0; i < MINE; ++i) {
-                const f32x4_t o = *reinterpret_cast<const f32x4_t*>(lds + (((size_t)w * PER * 64) + ((dt0 + i) * 64 + lane) * 4));
+                const f32x4_t o = *reinterpret_cast<const f32x4_loose_t*>(lds + (((size_t)w * PER * 64) + ((dt0 + i) * 64 + lane) * 4));
                 mo[i] += o * a;
             }
         }
