@@ -233,6 +233,10 @@ __global__ __launch_bounds__(64) void mlstm_scalars_kernel(float* __restrict__ a
     const size_t head_state = (size_t)d * dv + (size_t)NS * (d + 1);
     double m = (double)state[((size_t)slot * H + h) * head_state + (size_t)d * dv + d];
     const int t0 = cu_q[s], t1 = cu_q[s + 1];
+    if (t0 >= t1) {                                       // no token whose gates could be asked for
+        if (lane == 0) mfin[(size_t)s * H + h] = (float)m;
+        return;
+    }
     auto gate = [&](int t, int which) { return lg[(size_t)min(t, t1 - 1) * 2 * H + which * H + h]; };
     float ig = gate(t0 + lane, 0), fg = gate(t0 + lane, 1);
     for (int tb = t0; tb < t1; tb += 64) {

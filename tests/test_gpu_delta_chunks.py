@@ -147,3 +147,27 @@ def test_matrix_memory_chunks_against_the_recurrence(case, how):
                 own = head[d * dv:].view(-1, d + 1)                          # n and m once for every slice of value channels
                 assert float((own[:, :d] - N[e][h]).abs().max()) < 1e-5 * max(1.0, float(N[e][h].abs().max())) and float((own[:, d] - M[e][h]).abs().max()) < 1e-4
     assert bool((state_dev[spare] == 7.0).all())
+
+
+@pytest.mark.parametrize("lengths", [[0, 20], [0, 0, 70, 0, 1]])
+def test_entries_without_tokens_read_and_write_nothing(lengths):
+    """The first entry's gates would lie before the rows; the other entries' results and states are those of a step without the empty ones."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    H, d, dv = 2, 64, 16
+    g = torch.Generator().manual_seed(3)
+    S, T = len(lengths), sum(lengths)
+    state = torch.randn(S, ops.mlstm_state_size(H, d, dv), generator=g) * 0.1
+    x, gates = torch.randn(T, 2 * H * d + 2 * H * dv, generator=g).to(dev), torch.randn(T, 2 * H, generator=g)
+    bi, bf, nw = torch.randn(H, generator=g).to(dev), torch.randn(H, generator=g).to(dev), torch.ones(H * dv, device=dev)
+
+    def run(entries):
+        st = state.to(dev)
+        cu = torch.tensor([0] + list(torch.tensor([lengths[e] for e in entries]).cumsum(0)), dtype=torch.int32).to(dev)
+        y = ops.mlstm(x, 0, H * d, 2 * H * d, 2 * H * d + H * dv, gates.clone().to(dev), bi, bf, 15.0, nw, 1e-6, st, cu,
+                      torch.tensor(entries, dtype=torch.int32).to(dev), H, d, dv)
+        return y, st
+    y, st = run(list(range(S)))
+    y2, st2 = run([e for e in range(S) if lengths[e]])
+    assert torch.equal(y, y2) and torch.equal(st, st2) and bool(y.isfinite().all())
+    assert all(torch.equal(st[e].cpu(), state[e]) for e in range(S) if not lengths[e])
