@@ -1581,6 +1581,12 @@ def mlstm_state_size(H: int, d: int, dv: int) -> int:
     return H * (d * dv + -(-dv // MATRIX_MEMORY_SLICE) * (d + 1))
 
 
+def recurrence_by_chunks(d: int, dv: int) -> bool:
+    """Whether the mLSTM and the delta rule take steps with more tokens than entries by chunks of 16 tokens for heads of d x dv
+    (csrc/delta_chunks.hip): such steps need no pieces."""
+    return d in (64, 128) and dv % 16 == 0
+
+
 def _entries(cu_q: torch.Tensor, slot_ids: torch.Tensor, what: str) -> int:
     S = slot_ids.shape[0]
     _check(cu_q.dtype == torch.int32 and cu_q.shape == (S + 1,) and slot_ids.dtype == torch.int32, "%s: cu_q int32 [S + 1] and slot_ids int32 [S] expected", what)
@@ -1596,8 +1602,8 @@ def mlstm(x: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: int, gates
     cap tanh(. / cap)); ``state [slots, mlstm_state_size(H, d, dv)]`` float32 holds S, n and the running maximum of every
     head, read at an entry's start and left at its end.  ``pieces`` = (int32 [4 n]: entry, first row, end row and the
     entry's first piece for every piece of tokens; n; whether an entry has several): entries in several pieces are walked
-    by several waves, whose effects on the state are composed.  Returns [T, H dv]: each head's read-out over its root
-    mean square, times ``norm_w``, times sigmoid(gate)."""
+    by several waves, whose effects on the state are composed (not read where ``recurrence_by_chunks``).  Returns [T, H dv]:
+    each head's read-out over its root mean square, times ``norm_w``, times sigmoid(gate)."""
     xs = _row_view(x, "mlstm")
     T = x.shape[0]
     _dev(gates, bi, bf, norm_w, state, cu_q, slot_ids)

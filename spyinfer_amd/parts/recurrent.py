@@ -155,15 +155,16 @@ class MLSTM(Mixer):
     def cache_spec(self):
         return FixedState((ops.mlstm_state_size(self.heads, self.dim, self.vdim),), "float32")
 
-    #: tokens of an entry that one wave walks in a row; longer entries are cut (their pieces' effects on the state are
-    #: composed: with the running maximum known, the state is linear in itself)
+    #: tokens of an entry that one wave walks in a row, for heads that do not go by chunks (``ops.recurrence_by_chunks``): longer
+    #: entries are cut (their pieces' effects on the state are composed: with the running maximum known, the state is linear in itself)
     PIECE = 64
 
     def plan(self, batch) -> None:
-        plan_scan_pieces(batch, self.PIECE)
+        if not ops.recurrence_by_chunks(self.dim, self.vdim):
+            plan_scan_pieces(batch, self.PIECE)
 
     def plan_arrays(self, entries):
-        return {scan_pieces_name(self.PIECE): 4 * entries}
+        return {} if ops.recurrence_by_chunks(self.dim, self.vdim) else {scan_pieces_name(self.PIECE): 4 * entries}
 
     def capturable(self, batch):
         return True
@@ -174,10 +175,12 @@ class MLSTM(Mixer):
         H, d, dv = self.heads, self.dim, self.vdim
         proj = ops.linear_few(x, self.w_in, self.w_in_tiled)
         gates = ops.linear(x, self.w_gates, torch.float32)
-        name = scan_pieces_name(self.PIECE)
-        n, multi = batch.shared[name]
+        pieces = None
+        if not ops.recurrence_by_chunks(d, dv):
+            name = scan_pieces_name(self.PIECE)
+            pieces = (batch.array(name), *batch.shared[name])
         y = ops.mlstm(proj, 0, H * d, 2 * H * d, 2 * H * d + H * dv, gates, self.b_i, self.b_f, self.gate_cap, self.norm, self.norm_eps,
-                      cache.state, batch.array("cu_q"), batch.array("slot_ids"), H, d, dv, pieces=(batch.array(name), n, multi))
+                      cache.state, batch.array("cu_q"), batch.array("slot_ids"), H, d, dv, pieces=pieces)
         return ops.linear_few(y, self.w_o, self.w_o_tiled)
 
 

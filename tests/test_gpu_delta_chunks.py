@@ -171,3 +171,14 @@ def test_entries_without_tokens_read_and_write_nothing(lengths):
     y2, st2 = run([e for e in range(S) if lengths[e]])
     assert torch.equal(y, y2) and torch.equal(st, st2) and bool(y.isfinite().all())
     assert all(torch.equal(st[e].cpu(), state[e]) for e in range(S) if not lengths[e])
+
+
+@pytest.mark.parametrize("d, dv", [(64, 16), (128, 256), (64, 24), (128, 8), (96, 64), (256, 64)])
+def test_who_goes_by_chunks_is_known_to_the_plans(d, dv):
+    import ctypes
+
+    from spyinfer_amd.kernels import ops
+    require_gpu()
+    I = ctypes.c_int
+    for f in (ops.hip().lib.spy_mlstm_workspace, ops.hip().lib.spy_delta_rule_workspace):
+        assert (f(I(2), I(40), I(3), I(d), I(dv)) > 0) == ops.recurrence_by_chunks(d, dv) and f(I(5), I(5), I(3), I(d), I(dv)) == 0

@@ -152,3 +152,26 @@ def test_greedy_generation_through_the_entry_point(folders, emu_ops):
     assert eng.generate(prompts, SamplingParams(max_new_tokens=10, ignore_eos=True)) == want
     assert eng.scheduler.num_preemptions > 0
     eng.runner.manager.check()
+
+
+@pytest.mark.parametrize("dim, vdim, pieces", [(128, 256, False), (64, 48, False), (128, 24, True), (40, 64, True)])
+def test_pieces_of_the_matrix_memory_are_planned_where_the_kernel_reads_them(dim, vdim, pieces):
+    """Heads that go by chunks read no pieces: none are cut, sent to the device or counted for a captured step."""
+    import numpy as np
+
+    from spyinfer_amd.parts.recurrent import MLSTM, scan_pieces_name
+
+    class Batch:
+        S, lens, shared = 2, np.array([200, 1], dtype=np.int32), {}
+        arrays = {}
+
+        def host_array(self, name):
+            return np.array([0, 200, 201], dtype=np.int32)
+
+        def add_array(self, name, values):
+            self.arrays[name] = values
+    batch, part = Batch(), MLSTM(64, 2, dim, vdim, 10.0, 1e-6)
+    batch.shared, batch.arrays = {}, {}
+    part.plan(batch)
+    name = scan_pieces_name(part.PIECE)
+    assert list(batch.arrays) == ([name] if pieces else []) and list(part.plan_arrays(5)) == ([name] if pieces else [])
