@@ -821,11 +821,12 @@ class AttentionMeta:
     head-in-group) rows for entries with few rows and 128-row tiles for entries with many, built
     for one group size ``tiles_group``; None if not built.
     ``big_rows``: rows of a "big" tile (128 or 256, see ``prefill_tile_rows``).
-    Host-side: S, T, max_blocks, max_kv_len, max_q_len, max_big_keys, max_small_keys.
+    Host-side: S, T, max_blocks, max_kv_len, max_q_len, max_big_keys, max_small_keys, big_keys, small_keys.
     What the arrays say must be true: the kernels read entries, pages and pieces as they are given."""
 
     def __init__(self, cu_q, pos0, kv_len, block_table, token_entry, positions, S, T, max_blocks, max_kv_len, max_q_len,
-                 tiles=None, tiles_group=0, fixed_shape=False, big_rows=128, pieces=None, max_big_keys=None, max_small_keys=None):
+                 tiles=None, tiles_group=0, fixed_shape=False, big_rows=128, pieces=None, max_big_keys=None, max_small_keys=None,
+                 big_keys=None, small_keys=None):
         self.cu_q, self.pos0, self.kv_len, self.block_table = cu_q, pos0, kv_len, block_table
         self.token_entry, self.positions = token_entry, positions
         self.S, self.T, self.max_blocks, self.max_kv_len, self.max_q_len = S, T, max_blocks, max_kv_len, max_q_len
@@ -839,6 +840,8 @@ class AttentionMeta:
         #: keys of the longest entry that has "big" tiles, and of the longest with "small" ones (not given: of the longest entry)
         self.max_big_keys = max_kv_len if max_big_keys is None else max_big_keys
         self.max_small_keys = max_kv_len if max_small_keys is None else max_small_keys
+        #: keys that all "big" and all "small" tiles read (not given: as if every tile read the most)
+        self.big_keys, self.small_keys = big_keys, small_keys
 
 
 MFMA_ATTENTION = True      # False forces the plain kernel for bfloat16 too (the kernel tests flip it; nothing else does)
@@ -884,19 +887,37 @@ def _prefill_us(blocks: int, keys: int, parts: int) -> float:
     return 8 + 1.6 * -(-(-(-keys // 64)) // parts) + (5 + 0.045 * parts * blocks if parts > 1 else 0)
 
 
-def mixed_attention_pays(blocks: int, keys: int, small_keys: int) -> bool:
-    """Whether entries with many rows (``blocks`` pairs of a 128-row tile and a kv head, the most keys ``keys``) and entries
-    with few (the most ``small_keys``) go in one launch, all keys in one part: where its longest block, a turn of eight
-    waves over 256 keys taking 3.1 us, ends before two launches would, the second of which takes 12 us at least, and the
-    large tiles have a compute unit each or share one by twos (more of them run faster with half the registers, 129 against
-    148 us at 3072 tokens).  32 query heads of 128 in 8 groups, microseconds apart / together: 389 tokens beside 20 single
-    tokens of 60 to 700 keys 35.9 / 18.9, of 1300 keys 48.5 / 34.0, beside 100 of 100 to 200 keys 42.8 / 33.5; 1000 tokens
-    beside the first 20 54.2 / 36.3; 2000 tokens beside 10 82 / 73; 800 beside three of 3000 keys 48 / 45; 100 beside one of
-    8000, whose keys go in parts otherwise, 30.4 / 98.7; prompts of 7 and 60 to 600 tokens, 16 heads, 32.8 / 23.7."""
+def mixed_attention_pays(blocks: int, keys: int, small_keys: int, d: int = 128, small_blocks: int = 1, big_total: Optional[int] = None,
+                         small_total: Optional[int] = None) -> bool:
+    """Whether entries with many rows (``blocks`` pairs of a 128-row tile and a kv head, the most keys ``keys``, ``big_total`` keys
+    over all pairs) and entries with few (``small_blocks`` pairs of a 16-row tile and a kv head, the most keys ``small_keys``,
+    ``small_total`` over all) go in one launch, all keys in one part.  Not given: every pair has the most keys.
+
+    Heads of 128 leave a compute unit room for one of the launch's blocks of eight waves: it ends with its longest block (a round of 64
+    keys 1.6 us, a turn of eight waves over 256 keys 3.1 us) or when the units have done all blocks' work, of which a small block's
+    is its start and round trips, 3.4 us, and 0.021 us a key.  Apart, the blocks of four waves hide each other's round trips (1.75 us and
+    0.019 us a key, 3.8 us a turn over 128 keys), but wait for the large tiles, and where lengths are uneven for the longest.  Microseconds
+    apart / together, 32 query heads in 8 groups, 389 new tokens beside 20 requests of 60 to 700 keys 38 / 24, 96 of 300 to 500 60 / 46, 96
+    of 60 to 1000 79 / 59, 256 of 200 68 / 75, 400 of 300 111 / 129; 100 tokens beside 32 of 1400 47 / 40, beside one of 8000, whose keys go
+    in parts otherwise, 30 / 99; 2000 tokens beside 96 of 100 to 500 108 / 103, of 1000 139 / 153.  Of 195 steps measured the choice loses
+    0.3 % to the better way on average, and in none more than 1 % to two launches as they were before prompts' keys went in parts by an estimate.
+
+    Heads of 64 leave room for two, and together was the faster way in all of 68 steps with up to 400 requests (128 of 1000 keys beside 389
+    tokens 69 / 54); only a longest block that outlasts both launches is left apart."""
     if blocks > 2 * PREFILL_SPLIT_BELOW:
-        return False
-    together = max(_prefill_us(blocks, keys, 1), 8 + 3.1 * -(-small_keys // 256))
-    return together <= _prefill_us(blocks, keys, prefill_key_parts(blocks, keys)) + 12
+        return False                                         # (large tiles beyond two rounds run faster with half the registers)
+    rounds, turns = -(-keys // 64), -(-small_keys // 256)
+    apart = _prefill_us(blocks, keys, prefill_key_parts(blocks, keys))
+    if d == 64:
+        return max(_prefill_us(blocks, keys, 1), 8 + 3.1 * turns) <= apart + 12
+    big_total = blocks * keys if big_total is None else big_total
+    small_total = small_blocks * small_keys if small_total is None else small_total
+    parts = max(1, min(DECODE_SPLIT_TARGET // small_blocks, key_parts_for(small_keys)))
+    work = (8.6 * blocks + 0.025 * big_total + 3.4 * small_blocks + 0.021 * small_total) / 256
+    together = 7 + max(work, 1.6 * rounds, 3.1 * turns)
+    small = (1.75 * small_blocks + 0.019 * small_total) / 256 + 0.03 * (small_keys - small_total / small_blocks)
+    apart += 13 * max(0.0, blocks / 256 - 1) + 6.4 + max(small, 3.8 * -(-small_keys // (128 * parts)))
+    return together < 0.98 * apart
 
 
 def prefill_attention_ok(d: int, page_size: int) -> bool:
@@ -1050,8 +1071,11 @@ def paged_attention(q: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: t
             if win:
                 big_keys = min(big_keys, win + meta.big_rows // group + 1)
             bsplits = prefill_key_parts(n_big * n_kv, big_keys)
+            small_keys = min(meta.max_small_keys, max_keys, win + 16 if win else max_keys)
+            total = lambda n, most, keys: n_kv * (n * most if keys is None else min(n * most, keys))
             if n_small and raw is None and not meta.fixed_shape and d in (64, 128) and meta.big_rows == 128 \
-                    and mixed_attention_pays(n_big * n_kv, big_keys, min(meta.max_small_keys, max_keys, win + 16 if win else max_keys)):
+                    and mixed_attention_pays(n_big * n_kv, big_keys, small_keys, d, n_small * n_kv, total(n_big, big_keys, meta.big_keys),
+                                             total(n_small, small_keys, meta.small_keys)):
                 hip().call("spy_attention_mixed", _ptr(out), _ptr(q), _ptr(k_cache), _ptr(v_cache), *common, _ptr(big_entry), _ptr(big_row0),
                            ctypes.c_int(n_big), _ptr(small_entry), _ptr(small_row0), ctypes.c_int(n_small), *sizes,
                            ctypes.c_int(operand.tiles if operand is not None else 0), *extras, _Hip.stream())

@@ -61,28 +61,34 @@ def plan_attention_tiles(batch, group_size: int, big_rows: int = 0, key_parts: b
     S, lens = batch.S, batch.lens
     rows = lens.astype(np.int64) * group_size
     big = (rows >= BIG_MIN_ROWS) & bool(big_rows)
-    counts = {}
+    counts, read = {}, {"big": 0, "small": 0}
     for kind, size, mask in (("small", ROWS_PER_TILE, ~big), ("big", max(big_rows, 1), big)):
         ntiles = np.where(mask, (rows + size - 1) // size, 0)
         tile_entry = np.repeat(np.arange(S, dtype=np.int32), ntiles)
         first = np.zeros(S + 1, dtype=np.int64)
         np.cumsum(ntiles, out=first[1:])
         tile_row0 = ((np.arange(int(first[-1]), dtype=np.int64) - first[:-1][tile_entry]) * size).astype(np.int32)
-        if kind == "big" and tile_entry.shape[0] > 2:
+        if kind == "big" and tile_entry.shape[0]:
             # the prefill kernel gives a block the tiles b and n - 1 - b: sorted by the keys they read, blocks are even
             pos0 = batch.host_array("pos0")[tile_entry].astype(np.int64)
             last_tok = np.minimum(lens[tile_entry].astype(np.int64), (tile_row0.astype(np.int64) + size + group_size - 1) // group_size)
             keys = pos0 + last_tok
             if chunk:
                 keys -= (pos0 + tile_row0 // group_size) // chunk * chunk        # the tile's first row has its first key
-            order = np.argsort(-keys, kind="stable")
-            tile_entry, tile_row0 = tile_entry[order], tile_row0[order]
+            read[kind] = int(keys.sum())
+            if tile_entry.shape[0] > 2:
+                order = np.argsort(-keys, kind="stable")
+                tile_entry, tile_row0 = tile_entry[order], tile_row0[order]
         counts[kind] = int(first[-1])
         batch.add_array("tile_entry_%s_%s" % (kind, name), tile_entry)
         batch.add_array("tile_row0_%s_%s" % (kind, name), tile_row0)
     batch.shared[note] = counts
-    kv_len = batch.host_array("kv_len")
-    batch.shared[("attention_longest",) + note[1:]] = tuple(int(kv_len[m].max(initial=1)) for m in (big, ~big))
+    if counts["big"]:
+        # what the launches of a step with large tiles go by: the most keys of an entry of each kind, and the keys that all tiles read
+        kv_len = batch.host_array("kv_len").astype(np.int64)
+        read["small"] = int((np.where(big, 0, (rows + ROWS_PER_TILE - 1) // ROWS_PER_TILE) * kv_len).sum())
+        most = [int(kv_len[m].max(initial=1)) for m in (big, ~big)]
+        batch.shared[("attention_keys",) + note[1:]] = dict(max_big_keys=most[0], max_small_keys=most[1], big_keys=read["big"], small_keys=read["small"])
 
 
 def plan_decode_pieces(batch, n_kv: int, window: int, head_dim: int) -> None:
@@ -108,12 +114,11 @@ def attention_meta(batch, group: int, group_size: int, big_rows: int = 0, chunk:
             tiles = {kind: (batch.array("tile_entry_%s_%s" % (kind, name)), batch.array("tile_row0_%s_%s" % (kind, name)), n) for kind, n in counts.items()}
         pieces = {key[1:]: batch.array("decode_pieces_%d_%d_%d" % key[1:]).view(-1, key_pieces.PIECE_RECORD)
                   for key in batch.shared if isinstance(key, tuple) and key[0] == "decode_pieces"}
-        big_keys, small_keys = batch.shared.get(("attention_longest",) + note[2:], (None, None))
+        keys = batch.shared.get(("attention_keys",) + note[2:], {})
         meta = ops.AttentionMeta(batch.array("cu_q"), batch.array("pos0"), batch.array("kv_len"), batch.block_table(group),
                                  batch.array("token_entry"), batch.array("positions"), batch.S, batch.T, batch.max_blocks[group],
                                  batch.max_kv_len, batch.max_q_len, tiles, group_size, fixed_shape=batch.fixed_shape,
-                                 big_rows=big_rows or 128, pieces=pieces,
-                                 max_big_keys=big_keys, max_small_keys=small_keys)
+                                 big_rows=big_rows or 128, pieces=pieces, **keys)
         batch.shared[note] = meta
     return meta
 
