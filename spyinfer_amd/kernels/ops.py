@@ -13,6 +13,7 @@ the activations (a tensor stored in 32-bit stays so).
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Optional
 
 import torch
@@ -871,20 +872,27 @@ PREFILL_ATTENTION_MAX_HEAD_DIM = 128
 PREFILL_SPLIT_BELOW = 256   # fewer (128-row tile, kv head) pairs than this: split the keys to fill the chip
 
 
-def prefill_key_parts(blocks: int, keys: int) -> int:
+@functools.lru_cache(maxsize=256)          # (asked by every layer of a step: 1 to 6 us)
+def prefill_key_parts(blocks: int, keys: int, d: int = 128) -> int:
     """Into how many parts the keys of ``blocks`` (128-row tile, kv head) pairs are split when the tile with the most reads
-    ``keys``: the number with the least of what was measured, a round of 64 keys 1.6 us, the merge kernel 5 us and 0.045 us
-    for each part of a pair (its way through memory).  32 query heads of 128 in 8 groups, microseconds in 1 / 2 / 3 / 4 / 8
-    parts: 512 tokens of a new prompt 22.4 / 29.7 / 34.7 / 33.2 / 50.2, 1000 tokens 35.9 / 50.2 / 53.1 / 56.0 / 81.6; 300
-    tokens behind 1000: 41.5 / 36.6 / 35.8 / 39.5 / 50.5, 100 behind 2000: 60.1 / 41.9 / 36.4 / 34.1 / 36.0, 200 behind
-    4000: 111.3 / 70.3 / 56.8 / 49.8 / 55.4."""
+    ``keys``: the number with the least of what was measured (``_prefill_us``), or the most that there may be where these come within
+    a microsecond of it.  32 query heads of 128 in 8 groups, microseconds in 1 / 2 / 3 / 4 / 8 parts: 512 tokens of a new prompt 22.8 /
+    28.3 / 33.0 / 32.1 / -, 1000 tokens 36.4 / 50.2 / 56.5 / 58.0 / -; 300 tokens behind 1000: 42.8 / 35.9 / 34.5 / 38.2 / 49.2, 100 behind
+    2000: 61.4 / 42.9 / 37.2 / 34.7 / 35.5, 200 behind 4000: 114.0 / 71.3 / 57.4 / 49.2 / 54.7; with 16 query heads of 64, whose parts merge for
+    less, 300 behind 1000: 39.3 / 29.2 / 24.7 / 23.4 / 24.9.  In 77 cases of 7 shapes of heads none is more than 2 % slower than in the most parts."""
     if blocks >= PREFILL_SPLIT_BELOW:
         return 1
-    return min(range(1, max(1, min(PREFILL_SPLIT_BELOW * 2 // blocks, keys // 256, 16)) + 1), key=lambda parts: _prefill_us(blocks, keys, parts))
+    most = max(1, min(PREFILL_SPLIT_BELOW * 2 // blocks, keys // 256, 16))
+    able = [parts for parts in range(1, most + 1) if parts <= 4 or parts % 2 == 0 or parts == most]     # (seven parts: 36.2 us where six and eight take 35.2)
+    best = min(able, key=lambda parts: _prefill_us(blocks, keys, parts, d))
+    return most if best > 1 and _prefill_us(blocks, keys, most, d) <= _prefill_us(blocks, keys, best, d) + 1 else best
 
 
-def _prefill_us(blocks: int, keys: int, parts: int) -> float:
-    return 8 + 1.6 * -(-(-(-keys // 64)) // parts) + (5 + 0.045 * parts * blocks if parts > 1 else 0)
+def _prefill_us(blocks: int, keys: int, parts: int, d: int = 128) -> float:
+    """Microseconds: a round of 64 keys 1.6, a quarter more where parts share the compute units, the merge kernel 5 and 0.045
+    for each part of a pair (its way through memory; 0.034 for heads of 64)."""
+    shared = 1.25 if parts * blocks > 256 and parts > 1 else 1.0
+    return 8 + 1.6 * shared * -(-(-(-keys // 64)) // parts) + (5 + (0.045 if d > 64 else 0.034) * parts * blocks if parts > 1 else 0)
 
 
 def mixed_attention_pays(blocks: int, keys: int, small_keys: int, d: int = 128, small_blocks: int = 1, big_total: Optional[int] = None,
@@ -1070,7 +1078,7 @@ def paged_attention(q: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: t
             big_keys = min(meta.max_big_keys, max_keys)
             if win:
                 big_keys = min(big_keys, win + meta.big_rows // group + 1)
-            bsplits = prefill_key_parts(n_big * n_kv, big_keys)
+            bsplits = prefill_key_parts(n_big * n_kv, big_keys, d)
             small_keys = min(meta.max_small_keys, max_keys, win + 16 if win else max_keys)
             total = lambda n, most, keys: n_kv * (n * most if keys is None else min(n * most, keys))
             if n_small and raw is None and not meta.fixed_shape and d in (64, 128) and meta.big_rows == 128 \
