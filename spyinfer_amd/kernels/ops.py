@@ -1135,8 +1135,16 @@ def paged_attention(q: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: t
         tile_entry, tile_row0, n_tiles = meta.tiles["small"]
         for name, t in (("small tile entries", tile_entry), ("small tile rows", tile_row0)):
             _check(t.dtype == torch.int32 and tuple(t.shape) == (n_tiles,), "paged_attention: %s must be int32 [%d]", name, n_tiles)
-        # few tiles cannot fill the chip: their keys go in parts of 128 at least (a number that follows the captured step's key_parts_for)
-        splits = max(1, min(DECODE_SPLIT_TARGET // max(1, n_tiles * n_kv), 2 * key_parts_for(max_keys)))
+        # Few tiles cannot fill the chip: their keys go in two parts for each that key_parts_for counts, and a second kernel merges them
+        # (the number follows key_parts_for, which a captured step keeps).  What a window or chunk hides is not there to split, and 128
+        # keys are read before a merge would be done: one part where there are never more, and in steps with several tokens of a
+        # request, which are not captured, where there are no more now (8 kv heads of 128, two parts / one: a prompt of 17 tokens 10.1 /
+        # 7.8 us, 15 keys 9.1 / 7.7, 127 keys 9.8 / 10.0, 255 keys 11.4 / 13.2)
+        most = min(x for x in (chunk or 1 << 30, win + 16 if win else 1 << 30))
+        reach = min(meta.max_kv_len, most)
+        splits = 1
+        if reach > 128 or (most > 128 and meta.max_q_len == 1):
+            splits = max(1, min(DECODE_SPLIT_TARGET // max(1, n_tiles * n_kv), 2 * key_parts_for(reach)))
         ws = torch.empty((max(1, hip().lib.spy_attention_f32_workspace(ctypes.c_int(n_tiles), ctypes.c_int(n_kv), ctypes.c_int(d), ctypes.c_int(splits))),),
                          dtype=torch.float32, device=q.device)
         hip().call("spy_attention_f32", _ptr(out), _ptr(q), _ptr(k_cache), _ptr(v_cache), ctypes.c_int(page_size), ctypes.c_int(num_pages),

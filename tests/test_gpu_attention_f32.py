@@ -121,3 +121,29 @@ def test_a_value_that_is_not_finite_stays_with_the_rows_that_read_it(case):
     assert bool(out[fine].isfinite().all())
     assert float((out - ref)[fine].abs().max()) < 2e-5 * float(vc[vc.isfinite()].abs().max())      # (as above)
     assert torch.equal(torch.nan_to_num(out[~fine], nan=7.0), torch.nan_to_num(ref[~fine], nan=7.0))
+
+
+# entries (cached, new), window, chunk, parts of the keys
+PARTS = [([(0, 5)], None, None, 1), ([(100, 28)], None, None, 1), ([(100, 29)], None, None, 2), ([(15, 1)], None, None, 2), ([(600, 1)], None, None, 6),
+         ([(600, 1)], 16, None, 1), ([(600, 1)], 112, None, 1), ([(600, 1)], 113, None, 2), ([(600, 1)], 300, None, 4), ([(600, 3)], None, 128, 1),
+         ([(600, 3)], None, 129, 2), ([(700, 1)] * 40, None, None, 3)]
+
+
+@pytest.mark.parametrize("case", range(len(PARTS)))
+def test_parts_follow_the_keys_that_can_be_read(case, monkeypatch):
+    """A window or chunk of a long context leaves little to split, and a short prompt nothing."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    entries, window, chunk, parts = PARTS[case]
+    n_q, n_kv, d, P = 2, 2, 64, 16
+    q, kc, vc, bt, te, ps, meta = make_attention_case(torch.float32, dev, n_q, n_kv, d, P, entries, seed=160 + case)
+    rows = [(s, r0) for s, (_, n) in enumerate(entries) for r0 in range(0, n, 16)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
+    meta.tiles = {"small": (i32([s for s, _ in rows]), i32([r for _, r in rows]), len(rows)), "big": (i32([]), i32([]), 0)}
+    seen = []
+    real = ops.hip().call
+    monkeypatch.setattr(ops.hip(), "call", lambda name, *a: (seen.append((name, a[22].value)), real(name, *a))[1])
+    out = ops.paged_attention(q.to(dev), kc.to(dev), vc.to(dev), P, meta, n_q, n_kv, d, d ** -0.5, window, chunk=chunk).cpu().double()
+    assert seen == [("spy_attention_f32", parts)]
+    ref = plain(q, kc, vc, P, bt, te, ps, n_q, n_kv, d, d ** -0.5, window, chunk)
+    assert float((out - ref).abs().max()) < 2e-5 * float(vc[vc.isfinite()].abs().max())
