@@ -28,7 +28,10 @@
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float dc_f32x4_t;
 
 #define DC_TOKENS 16
-#define DC_SEGMENT 128           // chunks that are prepared and walked at a time: bounds the workspace
+// Chunks that are prepared and walked at a time, which bounds the workspace: 128, or as many as 64 MB hold (150 chunks of 70 KB, 60
+// entries of 24 tokens with 4 heads of 64 x 64: 51 us for the delta rule in two segments, 40 in one)
+#define DC_SEGMENT 128
+#define DC_SEGMENT_BYTES (64 << 20)
 
 // An entry's chunks have neighbouring numbers from cu_q[e] / 16 + e on (entries' ranges cannot meet: they have at most
 // cu_q[e + 1] / 16 - cu_q[e] / 16 + 1 chunks); some numbers belong to nobody.
@@ -37,6 +40,11 @@ static int64_t dc_numbers(int S, int T) { return (int64_t)T / DC_TOKENS + S; }
 
 // floats of one (chunk, head) in the workspace: MW [16][d], Q [16][d], K [d][16], MV [16][dv], B [16][16], G [d]
 __device__ __host__ __forceinline__ int dc_record(int d, int dv) { return 48 * d + 16 * dv + 256 + d; }
+
+static int64_t dc_segment(int H, int d, int dv) {
+    const int64_t n = DC_SEGMENT_BYTES / ((int64_t)H * dc_record(d, dv) * 4);
+    return n > DC_SEGMENT ? n : DC_SEGMENT;
+}
 
 __device__ __forceinline__ float dc_pow2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -389,17 +397,17 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(ChunkWalk a, int number
 bool delta_chunks_takes(int S, int T, int d, int dv) { return T > S && (d == 64 || d == 128) && dv % 16 == 0; }
 
 int64_t delta_chunks_workspace(int S, int T, int H, int d, int dv) {
-    const int64_t n = dc_numbers(S, T);
-    return (n < DC_SEGMENT ? n : DC_SEGMENT) * H * dc_record(d, dv);
+    const int64_t n = dc_numbers(S, T), most = dc_segment(H, d, dv);
+    return (n < most ? n : most) * H * dc_record(d, dv);
 }
 
 int delta_chunks(const DeltaChunks& a, int dtype, hipStream_t st) {
     SPY_REQUIRE(a.ws && a.ws_floats >= delta_chunks_workspace(a.S, a.T, a.H, a.d, a.dv), "delta rule: the chunks' workspace is too small");
     SPY_REQUIRE(((uintptr_t)a.ws % 16) == 0 && a.H <= 65535 && a.dv / 16 <= 65535, "delta rule: workspace alignment or heads");
     const ChunkWalk w = {a.o, a.state, a.state_stride, (long long)a.d * a.dv, nullptr, a.cu_q, a.slot_ids, a.num_slots, a.H, a.dv, a.ws};
-    const int64_t numbers = dc_numbers(a.S, a.T);
-    for (int64_t n0 = 0; n0 < numbers; n0 += DC_SEGMENT) {
-        const int n1 = (int)(n0 + DC_SEGMENT < numbers ? n0 + DC_SEGMENT : numbers);
+    const int64_t numbers = dc_numbers(a.S, a.T), segment = dc_segment(a.H, a.d, a.dv);
+    for (int64_t n0 = 0; n0 < numbers; n0 += segment) {
+        const int n1 = (int)(n0 + segment < numbers ? n0 + segment : numbers);
         const dim3 pgrid((unsigned)(n1 - n0), a.H), wgrid(a.S, a.H, a.dv / 16);
         if (a.d == 64) {
             SPY_DISPATCH(dtype, TA, (delta_chunk_prepare_kernel<TA, 64><<<pgrid, 256, 0, st>>>(a, (int)n0)));
@@ -418,9 +426,9 @@ int memory_chunks(const MemoryChunks& a, int dtype, hipStream_t st) {
     SPY_REQUIRE(((uintptr_t)a.ws % 16) == 0 && a.H <= 65535 && a.dv / 16 <= 65535, "mLSTM: workspace alignment or heads");
     const long long head = (long long)a.d * a.dv + (long long)(a.dv / 16) * (a.d + 1);
     const ChunkWalk w = {a.o, a.state, head * a.H, head, a.mfin, a.cu_q, a.slot_ids, a.num_slots, a.H, a.dv, a.ws};
-    const int64_t numbers = dc_numbers(a.S, a.T);
-    for (int64_t n0 = 0; n0 < numbers; n0 += DC_SEGMENT) {
-        const int n1 = (int)(n0 + DC_SEGMENT < numbers ? n0 + DC_SEGMENT : numbers);
+    const int64_t numbers = dc_numbers(a.S, a.T), segment = dc_segment(a.H, a.d, a.dv);
+    for (int64_t n0 = 0; n0 < numbers; n0 += segment) {
+        const int n1 = (int)(n0 + segment < numbers ? n0 + segment : numbers);
         const dim3 pgrid((unsigned)(n1 - n0), a.H), wgrid(a.S, a.H, a.dv / 16);
         if (a.d == 64) {
             SPY_DISPATCH(dtype, TA, (memory_chunk_prepare_kernel<TA, 64><<<pgrid, 256, 0, st>>>(a, (int)n0)));

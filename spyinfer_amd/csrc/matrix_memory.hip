@@ -335,13 +335,13 @@ __global__ __launch_bounds__(MM_SLICE) void mlstm_keep_kernel(float* __restrict_
     } while (0)
 
 // pieces: int32 [4][n_pieces] (entry, first row, end row, index of the entry's first piece), used when `multi` says that an
-// entry has several; then work [n_pieces][state of a request], abe [T][3 H] and mfin [S][H] are scratch (the latter two, and ws instead
-// of work, where spy_mlstm_workspace says that the step goes by chunks).
+// entry has several; then work [n_pieces][state of a request], abe [T][3 H] and mfin [S][H] are scratch.  by_chunks: every entry goes by
+// chunks (the head sizes must be for it, and abe, mfin and ws of spy_mlstm_workspace are scratch; pieces are not read).
 extern "C" int spy_mlstm(void* out, float* o_tmp, float* state, const void* x, long long xs, int dtype, int q_off, int k_off, int v_off,
                          int g_off, float* gates, const void* bi, const void* bf, int w_dtype, float cap, const void* norm_w,
                          float eps, const int* cu_q, const int* slot_ids, int num_slots, int S, int T, int H, int d, int dv,
                          const int* pieces, int n_pieces, int multi, float* work, float* abe, float* mfin, float* ws, int64_t ws_floats,
-                         hipStream_t st) {
+                         int by_chunks, hipStream_t st) {
     SPY_REQUIRE(S > 0 && T > 0 && H > 0 && d > 0 && dv > 0 && num_slots > 0 && o_tmp, "spy_mlstm: empty operand");
     SPY_REQUIRE(d <= 256 && dv <= 1024 && H <= 65535, "spy_mlstm: heads of %d x %d (key size up to 256, value size up to 1024)", d, dv);
     SPY_REQUIRE(cap > 0.f, "spy_mlstm: the gates' cap must be positive");
@@ -353,8 +353,8 @@ extern "C" int spy_mlstm(void* out, float* o_tmp, float* state, const void* x, l
         SPY_DISPATCH(w_dtype, TW, (mlstm_gates_kernel<TW><<<blocks, 256, 0, st>>>(gates, (const TW*)bi, (const TW*)bf, cap, T, H)));
         SPY_CHECK_LAUNCH("spy_mlstm (gates)");
     }
-    // Steps of single tokens walk token by token; the others go by chunks where the head sizes are whole matrix tiles, else by pieces
-    const bool chunks = delta_chunks_takes(S, T, d, dv);
+    const bool chunks = by_chunks != 0;
+    SPY_REQUIRE(!chunks || delta_chunks_takes(S, T, d, dv), "spy_mlstm: heads of %d x %d and %d tokens of %d entries do not go by chunks", d, dv, T, S);
     if (chunks || multi) {
         SPY_REQUIRE(abe && mfin, "spy_mlstm: no room for the tokens' scalars");
         mlstm_scalars_kernel<<<dim3(S, H), 64, 0, st>>>(abe, mfin, gates, state, cu_q, slot_ids, num_slots, H, d, dv, NS);
@@ -699,7 +699,7 @@ __global__ __launch_bounds__(MM_SLICE) void delta_rule_kernel(
         if (col && row0 + i < d) st[(size_t)(row0 + i) * dv + j] = S[i];
 }
 
-// floats of workspace that a step of S entries and T tokens needs (0: it does not go by chunks)
+// floats of workspace that a step of S entries and T tokens needs to go by chunks (0: it cannot)
 extern "C" int64_t spy_mlstm_workspace(int S, int T, int H, int d, int dv) {
     return delta_chunks_takes(S, T, d, dv) ? delta_chunks_workspace(S, T, H, d, dv) : 0;
 }
@@ -711,7 +711,7 @@ extern "C" int spy_delta_rule(void* out, float* o_tmp, float* qk_tmp, float* sta
                               float* beta_pre, float* dec_pre, const void* a_log, const void* dt_bias, int w_dtype, const void* gate, long long gs,
                               const void* norm_w, float eps, const int* cu_q, const int* slot_ids, int num_slots, int S, int T, int H,
                               int G, int d, int dv, int dd, int silu_gate, long long bs, long long zs, float* ws, int64_t ws_floats,
-                              hipStream_t st) {
+                              int by_chunks, hipStream_t st) {
     SPY_REQUIRE(S > 0 && T > 0 && H > 0 && G > 0 && H % G == 0 && d > 0 && dv > 0 && num_slots > 0 && o_tmp, "spy_delta_rule: empty operand");
     SPY_REQUIRE(dd == d || dd == 1, "spy_delta_rule: %d decays for a head of %d key channels (one, or one per channel)", dd, d);
     SPY_REQUIRE(bs >= H && zs >= (long long)H * dd, "spy_delta_rule: rows of beta or of the decays are too short");
@@ -722,9 +722,9 @@ extern "C" int spy_delta_rule(void* out, float* o_tmp, float* qk_tmp, float* sta
     SPY_DISPATCH(dtype, TA, SPY_DISPATCH(w_dtype, TW, (delta_prepare_kernel<TA, TW><<<pgrid, 64, 0, st>>>(
         qk_tmp, (const TA*)qkv, beta_pre, dec_pre, (const TW*)a_log, (const TW*)dt_bias, H, G, d, dv, dd, bs, zs))));
     SPY_CHECK_LAUNCH("spy_delta_rule (unit vectors and decays)");
-    // Steps of single tokens, and head sizes that are no whole matrix tiles, walk token by token; in the others every entry, also one of a
-    // single token, goes by chunks (a chunk's chain costs about what one token's does).
-    if (delta_chunks_takes(S, T, d, dv)) {
+    // (by_chunks: every entry, also one of a single token, goes by chunks of 16; else token by token.  The caller knows the lengths.)
+    SPY_REQUIRE(!by_chunks || delta_chunks_takes(S, T, d, dv), "spy_delta_rule: heads of %d x %d and %d tokens of %d entries do not go by chunks", d, dv, T, S);
+    if (by_chunks) {
         const DeltaChunks a = {o_tmp, state, state_stride, qkv, qk_tmp, beta_pre, dec_pre, cu_q, slot_ids, num_slots, S, T, H, G, d, dv, dd, bs, zs, ws, ws_floats};
         const int rc = delta_chunks(a, dtype, st);
         if (rc) return rc;

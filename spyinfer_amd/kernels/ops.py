@@ -1627,6 +1627,27 @@ def recurrence_by_chunks(d: int, dv: int) -> bool:
     return d in (64, 128) and dv % 16 == 0
 
 
+def recurrence_goes_by_chunks(S: int, T: int, H: int, d: int, dv: int, longest: Optional[int], delta: bool) -> bool:
+    """Whether a step of the mLSTM or (``delta``) the delta rule goes by chunks, or token by token.  ``longest``: the longest entry's
+    tokens (None: not known, by chunks wherever it can).
+
+    A token's turn of the walk is 1.1 us however many tokens go beside it, and a chunk's turn about the same; but a chunk costs its
+    preparation and the products of 16 rows whether it holds one token or 16, 0.08 us for each head of 128 x 128 of the delta rule.  So entries
+    beside the longest, of single tokens mostly, decide how long that has to be.  Delta rule, 16 heads of 128 x 128, microseconds token by
+    token / by chunks: 1 entry of 8 tokens 26 / 24, of 16 35 / 27, of 100 133 / 37; 15 single tokens beside 8 30 / 40, beside 24 52 / 52, beside 48 83 / 59; 63
+    beside 32 112 / 120, beside 48 150 / 129; 95 beside 2 68 / 146, beside 32 124 / 156, beside 64 197 / 180.  Many long entries keep the walk's
+    waves busy, and its work is less than the chunks': 60 entries of 24 tokens 152 / 222, of 64 342 / 457, 20 of 64 125 / 134, 5 of 64 100 / 53.
+    The mLSTM has little to prepare: 8 heads of 128 x 256, 95 beside 2 104 / 114, beside 8 125 / 115, 60 of 24 219 / 149."""
+    if not recurrence_by_chunks(d, dv) or T <= S:
+        return False
+    if longest is None:
+        return True
+    if not delta:
+        return longest > 4
+    heads = H * d * dv / (128 * 128)
+    return longest > max(8.0, 2 + 1.15 * (S * heads) ** 0.5) and heads * (T - S - longest) <= 250 * longest
+
+
 def _entries(cu_q: torch.Tensor, slot_ids: torch.Tensor, what: str) -> int:
     S = slot_ids.shape[0]
     _check(cu_q.dtype == torch.int32 and cu_q.shape == (S + 1,) and slot_ids.dtype == torch.int32, "%s: cu_q int32 [S + 1] and slot_ids int32 [S] expected", what)
@@ -1635,15 +1656,16 @@ def _entries(cu_q: torch.Tensor, slot_ids: torch.Tensor, what: str) -> int:
 
 def mlstm(x: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: int, gates: torch.Tensor, bi: torch.Tensor, bf: torch.Tensor,
           cap: float, norm_w: torch.Tensor, eps: float, state: torch.Tensor, cu_q: torch.Tensor, slot_ids: torch.Tensor, H: int, d: int,
-          dv: int, pieces=None) -> torch.Tensor:
+          dv: int, pieces=None, longest: Optional[int] = None) -> torch.Tensor:
     """The mLSTM recurrence over the step's tokens.  ``x``: rows of the fused projection with q (H heads of d) at column
     ``q_off``, k at ``k_off``, v (H heads of dv) at ``v_off`` and the output gate's rows at ``g_off``; ``gates [T, 2 H]``
     float32: the raw products of the input and forget gates, overwritten with the log gates (their biases ``bi``, ``bf [H]``; both capped by
     cap tanh(. / cap)); ``state [slots, mlstm_state_size(H, d, dv)]`` float32 holds S, n and the running maximum of every
     head, read at an entry's start and left at its end.  ``pieces`` = (int32 [4 n]: entry, first row, end row and the
     entry's first piece for every piece of tokens; n; whether an entry has several): entries in several pieces are walked
-    by several waves, whose effects on the state are composed (not read where ``recurrence_by_chunks``).  Returns [T, H dv]:
-    each head's read-out over its root mean square, times ``norm_w``, times sigmoid(gate)."""
+    by several waves, whose effects on the state are composed (not read where ``recurrence_by_chunks``).  ``longest``: the
+    longest entry's tokens, where the caller knows it (``recurrence_goes_by_chunks``).  Returns [T, H dv]: each head's
+    read-out over its root mean square, times ``norm_w``, times sigmoid(gate)."""
     xs = _row_view(x, "mlstm")
     T = x.shape[0]
     _dev(gates, bi, bf, norm_w, state, cu_q, slot_ids)
@@ -1661,7 +1683,8 @@ def mlstm(x: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: int, gates
     if T:
         tmp = torch.empty((T, H * dv), dtype=torch.float32, device=x.device)        # the read-outs before the heads' norm
         parr, n_pieces, multi, work, abe, mfin = None, 0, False, None, None, None
-        ws_floats = hip().lib.spy_mlstm_workspace(ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(H), ctypes.c_int(d), ctypes.c_int(dv))
+        chunks = recurrence_goes_by_chunks(S, T, H, d, dv, longest, False)
+        ws_floats = hip().lib.spy_mlstm_workspace(ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(H), ctypes.c_int(d), ctypes.c_int(dv)) if chunks else 0
         ws = torch.empty((ws_floats,), dtype=torch.float32, device=x.device) if ws_floats else None
         if pieces is not None and pieces[2]:
             parr, n_pieces, multi = pieces
@@ -1676,7 +1699,8 @@ def mlstm(x: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: int, gates
                    ctypes.c_int(k_off), ctypes.c_int(v_off), ctypes.c_int(g_off), _ptr(gates), _ptr(bi), _ptr(bf), _code(bi, "gate biases"),
                    ctypes.c_float(cap), _ptr(norm_w), ctypes.c_float(eps), _ptr(cu_q), _ptr(slot_ids), ctypes.c_int(state.shape[0]),
                    ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(H), ctypes.c_int(d), ctypes.c_int(dv), _ptr(parr), ctypes.c_int(n_pieces),
-                   ctypes.c_int(1 if multi else 0), _ptr(work), _ptr(abe), _ptr(mfin), _ptr(ws), ctypes.c_int64(ws_floats), _Hip.stream())
+                   ctypes.c_int(1 if multi else 0), _ptr(work), _ptr(abe), _ptr(mfin), _ptr(ws), ctypes.c_int64(ws_floats),
+                   ctypes.c_int(1 if chunks else 0), _Hip.stream())
     return out
 
 
@@ -1706,13 +1730,13 @@ def causal_conv_silu(x: torch.Tensor, taps: torch.Tensor, state: torch.Tensor, k
 
 def delta_rule(qkv: torch.Tensor, beta_pre: torch.Tensor, dec_pre: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
                gate: torch.Tensor, norm_w: torch.Tensor, eps: float, state: torch.Tensor, cu_q: torch.Tensor, slot_ids: torch.Tensor,
-               H: int, G: int, d: int, dv: int, gate_act: str = "sigmoid") -> torch.Tensor:
+               H: int, G: int, d: int, dv: int, gate_act: str = "sigmoid", longest: Optional[int] = None) -> torch.Tensor:
     """The gated delta rule over the step's tokens.  ``qkv [T, 2 G d + H dv]``: q and k (G heads of d; made unit vectors
     here, q also times d^-1/2) and v (H heads of dv); ``beta_pre [T, H]`` and ``dec_pre [T, H d]`` float32: the raw products
     (overwritten with what they turn into) behind beta = sigmoid(.) and the decay exp(-exp(a_log[h]) softplus(. + dt_bias)) per head and key channel; per head
     S = diag(decay) S, u = beta (v - S^T k), S += k u^T, o = S^T q with ``state[slot, h d dv ..]`` float32.  Returns
     [T, H dv]: o over its root mean square, times ``norm_w [dv]``, times sigmoid(``gate``) (rows of H dv values, a view
-    into a wider product allowed; ``gate_act`` "silu": times silu(gate)).  One decay per head instead of one per key
+    into a wider product allowed; ``gate_act`` "silu": times silu(gate)).  ``longest``: as for ``mlstm``.  One decay per head instead of one per key
     channel: ``dec_pre [T, H]`` and ``dt_bias [H]``."""
     _dev(qkv, a_log, dt_bias, norm_w, state, cu_q, slot_ids)
     gs = _row_view(gate, "delta_rule")
@@ -1734,13 +1758,14 @@ def delta_rule(qkv: torch.Tensor, beta_pre: torch.Tensor, dec_pre: torch.Tensor,
     if T:
         tmp = torch.empty((T, H * dv), dtype=torch.float32, device=qkv.device)      # the read-outs before the heads' norm
         unit = torch.empty((T, 2 * G * d), dtype=torch.float32, device=qkv.device)  # q and k as unit vectors
-        ws_floats = hip().lib.spy_delta_rule_workspace(ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(H), ctypes.c_int(d), ctypes.c_int(dv))
+        chunks = recurrence_goes_by_chunks(S, T, H, d, dv, longest, True)
+        ws_floats = hip().lib.spy_delta_rule_workspace(ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(H), ctypes.c_int(d), ctypes.c_int(dv)) if chunks else 0
         ws = torch.empty((max(1, ws_floats),), dtype=torch.float32, device=qkv.device)
         hip().call("spy_delta_rule", _ptr(out), _ptr(tmp), _ptr(unit), _ptr(state), ctypes.c_longlong(state.shape[1]), _ptr(qkv), _code(qkv, "qkv"),
                    ctypes.c_void_p(beta_pre.data_ptr()), ctypes.c_void_p(dec_pre.data_ptr()), _ptr(a_log), _ptr(dt_bias), _code(a_log, "decay numbers"), ctypes.c_void_p(gate.data_ptr()), ctypes.c_longlong(gs),
                    _ptr(norm_w), ctypes.c_float(eps), _ptr(cu_q), _ptr(slot_ids), ctypes.c_int(state.shape[0]), ctypes.c_int(S), ctypes.c_int(T),
                    ctypes.c_int(H), ctypes.c_int(G), ctypes.c_int(d), ctypes.c_int(dv), ctypes.c_int(dd), ctypes.c_int(1 if gate_act == "silu" else 0),
-                   ctypes.c_longlong(bs), ctypes.c_longlong(zs), _ptr(ws), ctypes.c_int64(ws_floats), _Hip.stream())
+                   ctypes.c_longlong(bs), ctypes.c_longlong(zs), _ptr(ws), ctypes.c_int64(ws_floats), ctypes.c_int(1 if chunks else 0), _Hip.stream())
     return out
 
 

@@ -180,7 +180,8 @@ class MLSTM(Mixer):
             name = scan_pieces_name(self.PIECE)
             pieces = (batch.array(name), *batch.shared[name])
         y = ops.mlstm(proj, 0, H * d, 2 * H * d, 2 * H * d + H * dv, gates, self.b_i, self.b_f, self.gate_cap, self.norm, self.norm_eps,
-                      cache.state, batch.array("cu_q"), batch.array("slot_ids"), H, d, dv, pieces=pieces)
+                      cache.state, batch.array("cu_q"), batch.array("slot_ids"), H, d, dv, pieces=pieces,
+                      longest=batch.max_q_len)
         return ops.linear_few(y, self.w_o, self.w_o_tiled)
 
 
@@ -258,7 +259,7 @@ class ChannelDelta(Mixer):
         cu_q, slots = batch.array("cu_q"), batch.array("slot_ids")
         qkv = ops.causal_conv_silu(proj[:, :C], self.taps, cache.state, H * d * dv, batch.array("token_entry"), cu_q, slots)
         y = ops.delta_rule(qkv, beta_pre, dec_pre, self.a_log, self.dt_bias, gate, self.norm, self.norm_eps, cache.state, cu_q, slots,
-                           H, G, d, dv)
+                           H, G, d, dv, longest=batch.max_q_len)
         return ops.linear_few(y, self.w_o, self.w_o_tiled)
 
 
@@ -325,7 +326,7 @@ class HeadDelta(Mixer):
         cu_q, slots = batch.array("cu_q"), batch.array("slot_ids")
         qkv = ops.causal_conv_silu(proj[:, :C], self.taps, cache.state, H * d * dv, batch.array("token_entry"), cu_q, slots)
         y = ops.delta_rule(qkv, beta_pre, dec_pre, self.a_log, self.dt_bias, proj[:, C:], self.norm, self.norm_eps, cache.state, cu_q, slots,
-                           H, G, d, dv, gate_act="silu")
+                           H, G, d, dv, gate_act="silu", longest=batch.max_q_len)
         return ops.linear_few(y, self.w_o, self.w_o_tiled)
 
 

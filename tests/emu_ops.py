@@ -301,7 +301,7 @@ class EmuOps:
         return y
 
     # ---- matrix memories ----
-    def mlstm(self, x, q_off, k_off, v_off, g_off, gates, bi, bf, cap, norm_w, eps, state, cu_q, slot_ids, H, d, dv, pieces=None):
+    def mlstm(self, x, q_off, k_off, v_off, g_off, gates, bi, bf, cap, norm_w, eps, state, cu_q, slot_ids, H, d, dv, pieces=None, longest=None):
         T = x.shape[0]
         f = x.float()
         out = torch.zeros((T, H, dv), dtype=torch.float32)
@@ -348,7 +348,7 @@ class EmuOps:
                 keep.copy_(rows[rows.shape[0] - (n - 1):])
         return y.to(x.dtype)
 
-    def delta_rule(self, qkv, beta_pre, dec_pre, a_log, dt_bias, gate, norm_w, eps, state, cu_q, slot_ids, H, G, d, dv, gate_act="sigmoid"):
+    def delta_rule(self, qkv, beta_pre, dec_pre, a_log, dt_bias, gate, norm_w, eps, state, cu_q, slot_ids, H, G, d, dv, gate_act="sigmoid", longest=None):
         T = qkv.shape[0]
         f = qkv.float()
         q = f[:, :G * d].reshape(T, G, d)

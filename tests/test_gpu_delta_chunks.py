@@ -182,3 +182,34 @@ def test_who_goes_by_chunks_is_known_to_the_plans(d, dv):
     I = ctypes.c_int
     for f in (ops.hip().lib.spy_mlstm_workspace, ops.hip().lib.spy_delta_rule_workspace):
         assert (f(I(2), I(40), I(3), I(d), I(dv)) > 0) == ops.recurrence_by_chunks(d, dv) and f(I(5), I(5), I(3), I(d), I(dv)) == 0
+
+
+@pytest.mark.parametrize("lengths", [[3, 1], [9, 1, 1], [40, 1], [17, 30, 2]])
+def test_both_ways_give_the_same_results(lengths, monkeypatch):
+    """Entries token by token where the longest is known to be short, by chunks where it is not known: the same read-outs and states
+    to rounding, and the way that the caller's rule names."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    H, G, d, dv = 4, 2, 64, 32
+    g = torch.Generator().manual_seed(8)
+    S, T = len(lengths), sum(lengths)
+    cu = torch.tensor([0] + list(torch.tensor(lengths).cumsum(0)), dtype=torch.int32).to(dev)
+    sl = torch.arange(S, dtype=torch.int32).to(dev)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    qkv, beta, dec, gate, x, gates = rnd(T, 2 * G * d + H * dv), rnd(T, H), rnd(T, H * d) - 3, rnd(T, H * dv), rnd(T, 2 * H * d + 2 * H * dv), rnd(T, 2 * H)
+    start = [rnd(S, H * d * dv) * 0.1, torch.zeros(S, ops.mlstm_state_size(H, d, dv))]
+    ones = lambda n: torch.ones(n, device=dev)
+    ways = []
+    real = ops.hip().call
+    monkeypatch.setattr(ops.hip(), "call", lambda name, *a: (ways.append(a[-2].value) if name in ("spy_delta_rule", "spy_mlstm") else None, real(name, *a))[1])
+    out = []
+    for longest in (None, max(lengths)):
+        states = [s.to(dev) for s in start]
+        y = [ops.delta_rule(qkv.to(dev), beta.to(dev), dec.to(dev), ones(H), ones(H * d), gate.to(dev), ones(dv), 1e-6, states[0], cu, sl, H, G, d, dv, longest=longest),
+             ops.mlstm(x.to(dev), 0, H * d, 2 * H * d, 2 * H * d + H * dv, gates.clone().to(dev), ones(H), ones(H), 15.0, ones(H * dv), 1e-6, states[1], cu, sl, H, d, dv,
+                       longest=longest)]
+        out.append(y + states)
+    assert ways == [1, 1] + [int(ops.recurrence_goes_by_chunks(S, T, H, d, dv, max(lengths), delta)) for delta in (True, False)]
+    for a, b in zip(*out):
+        # float32 sums of 64 products in other orders, over a root mean square: some dozens of roundings of 2^-24 of the largest
+        assert float((a - b).abs().max()) < 1e-5 * max(1.0, float(b.abs().max()))

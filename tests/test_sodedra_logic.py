@@ -175,3 +175,37 @@ def test_pieces_of_the_matrix_memory_are_planned_where_the_kernel_reads_them(dim
     part.plan(batch)
     name = scan_pieces_name(part.PIECE)
     assert list(batch.arrays) == ([name] if pieces else []) and list(part.plan_arrays(5)) == ([name] if pieces else [])
+
+
+# the delta rule?, heads, key size, value size, single tokens, further entries and their tokens, by chunks? (where the two ways differ by more than 4 %)
+RECURRENCE = [
+    (True, 16, 128, 128, 0, 1, 16, True),         # 35 us token by token, 27 by chunks
+    (True, 16, 128, 128, 0, 1, 2, False),         # 19 / 23
+    (True, 16, 128, 128, 15, 1, 2, False),        # 23 / 40
+    (True, 16, 128, 128, 15, 1, 48, True),        # 83 / 59
+    (True, 16, 128, 128, 95, 1, 32, False),       # 124 / 156
+    (True, 16, 128, 128, 95, 1, 100, True),       # 280 / 215
+    (True, 32, 128, 128, 95, 1, 64, False),       # 334 / 367
+    (True, 32, 128, 128, 3, 1, 100, True),        # 143 / 63
+    (True, 16, 128, 128, 0, 60, 24, False),       # 152 / 222
+    (True, 32, 128, 128, 0, 60, 64, False),       # 691 / 887
+    (True, 16, 128, 128, 0, 5, 64, True),         # 100 / 53
+    (True, 4, 64, 64, 95, 1, 8, False),           # 20 / 28
+    (True, 4, 64, 64, 95, 1, 24, True),           # 32 / 30
+    (True, 4, 64, 64, 0, 60, 64, True),           # 80 / 62
+    (False, 8, 128, 256, 95, 1, 2, False),        # 104 / 114
+    (False, 8, 128, 256, 95, 1, 16, True),        # 150 / 118
+    (False, 8, 128, 256, 0, 60, 64, True),        # 510 / 253
+    (False, 4, 64, 64, 0, 1, 8, True),            # 21 / 18
+    (False, 4, 64, 40, 0, 1, 800, False),         # heads that do not go by chunks
+    (True, 64, 128, 512, 0, 1, 2000, True),       # heads so large that one entry is many waves' work: nothing beside it
+]
+
+
+@pytest.mark.parametrize("delta, H, d, dv, singles, more, tokens, chunks", RECURRENCE)
+def test_recurrences_go_the_way_that_was_faster(delta, H, d, dv, singles, more, tokens, chunks):
+    from spyinfer_amd.kernels import ops
+    S, T = singles + more, singles + more * tokens
+    assert ops.recurrence_goes_by_chunks(S, T, H, d, dv, tokens, delta) == chunks
+    assert not ops.recurrence_goes_by_chunks(S, S, H, d, dv, 1, delta)
+    assert ops.recurrence_goes_by_chunks(S, T, H, d, dv, None, delta) == ops.recurrence_by_chunks(d, dv)
