@@ -11,6 +11,7 @@ CASES = [
     (8, 2, 128, 16, [(0, 33)], None, 1),                              # two tiles, the second with four rows
     (8, 8, 64, 16, [(0, 129), (5, 64)], None, 1),
     (4, 1, 128, 16, [(700, 40), (3, 1), (0, 200)], None, 2),           # parts: few tiles behind many keys
+    (4, 1, 64, 16, [(900, 33), (2500, 1)], None, 3),                   # the same beside a single token with more keys
     (4, 1, 128, 16, [(0, 100), (1500, 1)], None, 1),                   # the single token's keys split nothing
     (4, 1, 64, 64, [(1500, 40)], 90, 1),                               # a window leaves nothing to split
     (256, 256, 64, 16, [(0, 130)], None, 1),                           # 512 pairs: two tiles a block
@@ -20,7 +21,7 @@ CASES = [
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", range(len(CASES)))
-def test_few_tiles(case):
+def test_few_tiles(case, monkeypatch):
     from spyinfer_amd.kernels import ops
     dev = require_gpu()
     n_q, n_kv, d, P, entries, window, parts = CASES[case]
@@ -30,9 +31,15 @@ def test_few_tiles(case):
     blocks = meta.tiles["big"][2] * n_kv
     assert blocks > 0
     keys = meta.max_big_keys if window is None else min(meta.max_big_keys, window + 128 // group + 1)
-    assert ops.prefill_key_parts(blocks, keys) == parts
+    assert ops.prefill_key_parts(blocks, keys, d) == parts
     ref = plain_paged_attention(q, kc, vc, P, bt, te, ps, n_q, n_kv, d, 0.11, window)
+    # entries of both kinds: two launches, so that the large tiles' own launch is what is tested
+    monkeypatch.setattr(ops, "mixed_attention_pays", lambda *a: False)
+    launches = []
+    real = ops.hip().call
+    monkeypatch.setattr(ops.hip(), "call", lambda name, *a: (launches.append((name, a[23].value if name == "spy_attention_prefill" else None)), real(name, *a))[1])
     got = ops.paged_attention(q.to(dev), kc.to(dev), vc.to(dev), P, meta, n_q, n_kv, d, 0.11, window)
+    assert launches[0] == ("spy_attention_prefill", parts) and [n for n, _ in launches[1:]] == ["spy_attention_mfma"] * (meta.tiles["small"][2] > 0)
     close(got, ref, torch.bfloat16, scale=3.0, what="few tiles, case %d" % case)
 
 
