@@ -1981,6 +1981,7 @@ class MoEAlignment:
         self.T, self.top, self.experts = T, top, experts
 
 
+@functools.lru_cache(maxsize=256)          # (asked by every mixture of a step)
 def _align_sizes(T: int, top: int, experts: int):
     """(sorted rows, pairs, tiles, ints for the groups) of a mixture's alignment: they follow the numbers of tokens and choices alone."""
     tm = hip().lib.spy_moe_tile_rows()
@@ -2092,17 +2093,18 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
     rows, P, max_tiles, group_ints = _align_sizes(T, top, E)
     tm = rows // max_tiles
     if align is None:
-        sorted_pair = torch.empty((rows,), dtype=torch.int32, device=dev)
-        pair_row = torch.empty((P,), dtype=torch.int32, device=dev)
-        tile_expert = torch.empty((max_tiles,), dtype=torch.int32, device=dev)
-        groups = torch.empty((group_ints,), dtype=torch.int32, device=dev)
-        hip().call("spy_moe_align", _ptr(sorted_pair), _ptr(pair_row), _ptr(tile_expert), _ptr(groups), _ptr(ids), ctypes.c_int(P), ctypes.c_int(E),
+        # one allocation for the four arrays (four take a mixture of few rows, whose launches are a few microseconds each, a fifth longer)
+        buf = torch.empty((P + rows + max_tiles + group_ints,), dtype=torch.int32, device=dev)
+        pair_row, at = buf[:P], buf.data_ptr()
+        pairs, sorted_pairs, tile_experts, group_list = (ctypes.c_void_p(at + 4 * n) for n in (0, P, P + rows, P + rows + max_tiles))
+        hip().call("spy_moe_align", sorted_pairs, pairs, tile_experts, group_list, _ptr(ids), ctypes.c_int(P), ctypes.c_int(E),
                    ctypes.c_int(max_tiles), _Hip.stream())
     else:
         sorted_pair, pair_row, tile_expert, groups = align.sorted_pair, align.pair_row, align.tile_expert, align.groups
         _dev(sorted_pair, pair_row, tile_expert, groups)
         _check(sorted_pair.shape == (rows,) and pair_row.shape == (P,) and tile_expert.shape == (max_tiles,) and groups.shape == (group_ints,),
                "moe_experts: the alignment does not fit")
+        sorted_pairs, tile_experts, group_list = _ptr(sorted_pair), _ptr(tile_expert), _ptr(groups)
     # bfloat16: the matrix cores, a block taking one row tile of an expert when the experts have few rows (decoding:
     # blocks for the whole device), up to eight when they have many (an expert's matrices are read once per 128 rows).  Few: under 8 rows
     # an expert on average (64 tokens of four choices, 32 experts of 2 x 3072 x 4096: 468 us a tile at a time, 422 by groups; 2 x 1536 x
@@ -2111,11 +2113,11 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
     per_block = 0 if not MOE_MFMA or x.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16 else (8 if many else 1)
     act = torch.empty((max_tiles * tm, F), dtype=x.dtype, device=dev)
     hip().call("spy_moe_gemm", _ptr(act), _code(act, "act"), _ptr(x), _code(x, "x"), _ptr(w_gate_up), _code(w_gate_up, "expert matrices"),
-               _ptr(tile_expert), _ptr(sorted_pair), _ptr(groups), ctypes.c_int(P), ctypes.c_int(top), ctypes.c_int(1 if gated else 0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(F),
+               tile_experts, sorted_pairs, group_list, ctypes.c_int(P), ctypes.c_int(top), ctypes.c_int(1 if gated else 0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(F),
                ctypes.c_int(K), ctypes.c_int(per_block), ctypes.c_int(act_kind), ctypes.c_float(limit), _ptr(weights if weight_input else None), _Hip.stream())
     y = torch.empty((max_tiles * tm, K), dtype=torch.float32, device=dev)
-    hip().call("spy_moe_gemm", _ptr(y), F32, _ptr(act), _code(act, "act"), _ptr(w_down), _code(w_down, "expert matrices"), _ptr(tile_expert),
-               _ptr(sorted_pair), _ptr(groups), ctypes.c_int(P), ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(K), ctypes.c_int(F),
+    hip().call("spy_moe_gemm", _ptr(y), F32, _ptr(act), _code(act, "act"), _ptr(w_down), _code(w_down, "expert matrices"), tile_experts,
+               sorted_pairs, group_list, ctypes.c_int(P), ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(K), ctypes.c_int(F),
                ctypes.c_int(per_block), ctypes.c_int(0), ctypes.c_float(0.0), _ptr(None), _Hip.stream())
     result = ExpertRows(y, pair_row, None if weight_input else weights, add, top, scale, T, x.dtype)
     return result if unsummed else result.combine()
