@@ -2056,6 +2056,27 @@ class ExpertRows:
         return out
 
 
+@functools.lru_cache(maxsize=256)          # (asked by every mixture of a step)
+def experts_by_groups(pairs: int, experts: int, K: int, F: int, gated: bool) -> bool:
+    """Whether ``pairs`` rows of ``experts`` experts (matrices of K and F) go by groups of up to 128 rows of one expert, or a tile of 16
+    rows at a time: whichever should take less time.  A tile at a time, every tile reads its expert's matrices out of the caches; by
+    groups they are read once, but a block takes all of K for 128 of their rows, 0.7 us for each 64 of K and F, which few experts leave
+    most of the chip waiting for.  Microseconds a tile at a time / by groups: one expert of 2 x 1024 x 1024 with 8 rows 15 / 33, with 96
+    rows 19 / 38; 8 such with 8 rows each 21 / 36, with 48 44 / 41; 64 with 4 rows each 87 / 86, with 8 92 / 87; 32 experts of 2 x 1536 x 2048
+    with 4 127 / 137, with 8 138 / 137, with 16 181 / 139; of 2 x 3072 x 4096 with 4 451 / 426, with 8 479 / 429.  The estimates' numbers are
+    those that make the fewest wrong choices: of 823 cases measured (1 to 128 experts of 2 to 96 rows each, nine sizes of matrices) the
+    choice is 0.13 % behind the better one on average, at most 15 % in a case.  K or F no multiple of 64, where the kernel with groups does
+    not stand: from 16 rows an expert on."""
+    if K % 64 or F % 64:
+        return pairs >= 16 * experts
+    used = min(experts, pairs)
+    megabytes = (3 if gated else 2) * K * F * 2e-6                   # of an expert's matrices
+    tiles = max(used, pairs / 16 + used / 2)
+    one = 8 + (0.04 * used + tiles / 5.1 + pairs / 180) * megabytes
+    groups = max(9 + 1.3 * (K + F) / 64, 15 + used * megabytes / 3.9) + pairs * megabytes / 3000
+    return groups < one
+
+
 def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[torch.Tensor], w_gate_up: torch.Tensor, w_down: torch.Tensor,
                 activation: str = "silu", limit: float = 0.0, weight_input: bool = False, add: Optional[torch.Tensor] = None,
                 align: Optional[MoEAlignment] = None, scale: float = 1.0, unsummed: bool = False):
@@ -2105,11 +2126,8 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
         _check(sorted_pair.shape == (rows,) and pair_row.shape == (P,) and tile_expert.shape == (max_tiles,) and groups.shape == (group_ints,),
                "moe_experts: the alignment does not fit")
         sorted_pairs, tile_experts, group_list = _ptr(sorted_pair), _ptr(tile_expert), _ptr(groups)
-    # bfloat16: the matrix cores, a block taking one row tile of an expert when the experts have few rows (decoding:
-    # blocks for the whole device), up to eight when they have many (an expert's matrices are read once per 128 rows).  Few: under 8 rows
-    # an expert on average (64 tokens of four choices, 32 experts of 2 x 3072 x 4096: 468 us a tile at a time, 422 by groups; 2 x 1536 x
-    # 2048: 123 / 124; 100 tokens 135 / 123), or 16 where K is no multiple of 64 and the kernel with groups does not stand
-    many = P >= (8 if K % 64 == 0 and F % 64 == 0 else 16) * E
+    # bfloat16: the matrix cores, a block taking one row tile of an expert (decoding: blocks for the whole device) or up to eight
+    many = experts_by_groups(P, E, K, F, gated)
     per_block = 0 if not MOE_MFMA or x.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16 else (8 if many else 1)
     act = torch.empty((max_tiles * tm, F), dtype=x.dtype, device=dev)
     hip().call("spy_moe_gemm", _ptr(act), _code(act, "act"), _ptr(x), _code(x, "x"), _ptr(w_gate_up), _code(w_gate_up, "expert matrices"),

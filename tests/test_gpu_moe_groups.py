@@ -1,6 +1,6 @@
 """The experts' products over groups of row tiles (csrc/moe.hip, many rows per expert and K in whole steps of 64): one step of K, two,
 an odd number of them, columns that are no multiple of a tile or of four, groups with one row and with 128, experts with more groups
-than a band, experts without rows, every form of the product; against float64."""
+than a band, experts without rows, every form of the product; and the same rows a tile of 16 at a time; against float64."""
 import pytest
 import torch
 
@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 def rows_for(kind, E, top, g):
     """ids [T, top]: how many rows the experts get."""
-    if kind in ("even", "few"):                  # few: eight to fifteen rows an expert on average, from where the groups take over
+    if kind in ("even", "few"):                  # few: eight to fifteen rows an expert on average
         return torch.stack([torch.randperm(E, generator=g)[:top] for _ in range((40 if kind == "even" else 9) * E // top)]).int()
     # the first expert gets every token (more groups than a band), the last none, the others a few
     T = {"one": 700, "edges": 128}[kind]
@@ -21,11 +21,13 @@ def rows_for(kind, E, top, g):
     return ids
 
 
+@pytest.mark.parametrize("by_groups", [True, False])
 @pytest.mark.parametrize("form", ["silu", "clamped", "weighted", "gelu"])
 @pytest.mark.parametrize("kind,E,top,K,F", [("even", 6, 2, 64, 64), ("one", 5, 2, 128, 192), ("edges", 9, 3, 192, 320), ("one", 4, 2, 320, 130), ("even", 7, 3, 256, 67 * 4),
                                              ("few", 8, 2, 128, 192), ("few", 16, 4, 64, 320)])
-def test_products_over_groups(kind, E, top, K, F, form):
+def test_products_over_groups(kind, E, top, K, F, form, by_groups, monkeypatch):
     from spyinfer_amd.kernels import ops
+    monkeypatch.setattr(ops, "experts_by_groups", lambda *sizes: by_groups)         # (few and small experts would not go by groups)
     dev = require_gpu()
     g = torch.Generator().manual_seed(E + K)
     ids = rows_for(kind, E, top, g)
@@ -33,7 +35,6 @@ def test_products_over_groups(kind, E, top, K, F, form):
     bf = lambda *s, std=1.0: (torch.randn(s, generator=g) * std).bfloat16()
     x, wgu, wd = bf(T, K), bf(E, (2 if gated else 1) * F, K, std=K ** -0.5), bf(E, K, F, std=F ** -0.5)
     w = torch.rand((T, top), generator=g)
-    assert T * top >= (8 if K % 64 == 0 and F % 64 == 0 else 16) * E and (kind != "few" or T * top < 16 * E)
     kw = dict(silu={}, clamped=dict(activation="clamped", limit=0.8), weighted=dict(activation="clamped", limit=0.8, weight_input=True), gelu=dict(activation="gelu"))[form]
     out = ops.moe_experts(x.to(dev), ids.to(dev), w.to(dev), wgu.to(dev), wd.to(dev), **kw)
     ref = torch.zeros((T, K), dtype=torch.float64)
