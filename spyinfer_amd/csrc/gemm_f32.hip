@@ -8,6 +8,9 @@
 //                           turn, operands straight from memory into v_mfma_f32_16x16x4_f32 registers, and add through LDS.
 //   tile   (many rows)      bound by the matrix cores (256 flops a cycle and compute unit).  Tiles of A and W through LDS.
 //
+// Which kernel, how many row tiles a block and how many parts of K follow the number of rows, and with them the order of a row's sums: a
+// row in a step of other sizes is the same within rounding, not bit for bit (as it is from gemm_generic.hip).
+//
 // The operands' order of K inside an MFMA step is free as long as both agree: a lane (r = lane % 16, g = lane / 16) loads the four
 // values k + 4 g .. + 3 of its row in one piece, and instruction j of four multiplies the j-th of them.
 #include "gemm_f32.h"

@@ -318,7 +318,8 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(TC* __restrict__ C, const
 }
 
 
-// The same product on the matrix cores, bfloat16 operands and float32 sums (v_mfma_f32_16x16x32_bf16), for few rows per expert (decoding):
+// The same product on the matrix cores, bfloat16 operands and float32 sums (v_mfma_f32_16x16x32_bf16), for few rows per expert (decoding)
+// and for experts so few or small that blocks of 128 rows would leave the chip idle (ops.experts_by_groups has the line):
 // a block has one row tile (16 sorted rows) and 32 rows of W (gated: 16 gate rows and the 16 up rows of the same columns), whose K
 // its four waves take in chunks of 128 in turn and add through LDS.  Operands go from memory straight into MFMA operand registers: lane
 // (r = lane % 16, g = lane / 16) holds row r, values k + 8 g .. + 7; the result tile is C^T: lane (r, g) holds C[row r][column 4 g + i].

@@ -427,8 +427,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
     ``tiled``: the same matrix from ``tile_weight``, used when few bfloat16 rows stream it.
     ``out``: the result is written there (a tensor of the result's shape and dtype) instead of into a new tensor.
 
-    float32 anywhere among x and w -> the hand-written true-fp32 kernel.  All bfloat16: the streaming
-    MFMA kernel for few rows, the library product for many."""
+    float32 anywhere among x and w -> the hand-written true-fp32 kernels.  All of it float32: the kernel, and with it the
+    order of a row's sums, goes by the number of rows (csrc/gemm_f32.hip), so that a row of another batch is the same within
+    rounding and not bit for bit.  All bfloat16: the streaming MFMA kernel for few rows, the library product for many."""
     _dev(x, w)
     _check(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1], "linear: x [M, K] and w [N, K] expected, got %s and %s"
            % (tuple(x.shape), tuple(w.shape)))
