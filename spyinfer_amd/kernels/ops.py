@@ -1080,11 +1080,13 @@ def paged_attention(q: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: t
             if win:
                 big_keys = min(big_keys, win + meta.big_rows // group + 1)
             bsplits = prefill_key_parts(n_big * n_kv, big_keys, d)
-            small_keys = min(meta.max_small_keys, max_keys, win + 16 if win else max_keys)
-            total = lambda n, most, keys: n_kv * (n * most if keys is None else min(n * most, keys))
-            if n_small and raw is None and not meta.fixed_shape and d in (64, 128) and meta.big_rows == 128 \
-                    and mixed_attention_pays(n_big * n_kv, big_keys, small_keys, d, n_small * n_kv, total(n_big, big_keys, meta.big_keys),
-                                             total(n_small, small_keys, meta.small_keys)):
+            together = False
+            if n_small and raw is None and not meta.fixed_shape and d in (64, 128) and meta.big_rows == 128:
+                small_keys = min(meta.max_small_keys, max_keys, win + 16 if win else max_keys)
+                total = lambda n, most, keys: n_kv * (n * most if keys is None else min(n * most, keys))
+                together = mixed_attention_pays(n_big * n_kv, big_keys, small_keys, d, n_small * n_kv, total(n_big, big_keys, meta.big_keys),
+                                                total(n_small, small_keys, meta.small_keys))
+            if together:
                 hip().call("spy_attention_mixed", _ptr(out), _ptr(q), _ptr(k_cache), _ptr(v_cache), *common, _ptr(big_entry), _ptr(big_row0),
                            ctypes.c_int(n_big), _ptr(small_entry), _ptr(small_row0), ctypes.c_int(n_small), *sizes,
                            ctypes.c_int(operand.tiles if operand is not None else 0), *extras, _Hip.stream())

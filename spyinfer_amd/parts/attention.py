@@ -68,14 +68,15 @@ def plan_attention_tiles(batch, group_size: int, big_rows: int = 0, key_parts: b
         first = np.zeros(S + 1, dtype=np.int64)
         np.cumsum(ntiles, out=first[1:])
         tile_row0 = ((np.arange(int(first[-1]), dtype=np.int64) - first[:-1][tile_entry]) * size).astype(np.int32)
-        if kind == "big" and tile_entry.shape[0]:
+        if kind == "big" and (tile_entry.shape[0] > 2 or (counts["small"] and tile_entry.shape[0])):
             # the prefill kernel gives a block the tiles b and n - 1 - b: sorted by the keys they read, blocks are even
             pos0 = batch.host_array("pos0")[tile_entry].astype(np.int64)
             last_tok = np.minimum(lens[tile_entry].astype(np.int64), (tile_row0.astype(np.int64) + size + group_size - 1) // group_size)
             keys = pos0 + last_tok
             if chunk:
                 keys -= (pos0 + tile_row0 // group_size) // chunk * chunk        # the tile's first row has its first key
-            read[kind] = int(keys.sum())
+            if counts["small"]:
+                read[kind] = int(keys.sum())
             if tile_entry.shape[0] > 2:
                 order = np.argsort(-keys, kind="stable")
                 tile_entry, tile_row0 = tile_entry[order], tile_row0[order]
@@ -83,8 +84,9 @@ def plan_attention_tiles(batch, group_size: int, big_rows: int = 0, key_parts: b
         batch.add_array("tile_entry_%s_%s" % (kind, name), tile_entry)
         batch.add_array("tile_row0_%s_%s" % (kind, name), tile_row0)
     batch.shared[note] = counts
-    if counts["big"]:
-        # what the launches of a step with large tiles go by: the most keys of an entry of each kind, and the keys that all tiles read
+    if counts["big"] and counts["small"]:
+        # what the launches of a step with both kinds of tiles go by: the most keys of an entry of each kind, and the keys that all
+        # tiles read (with one kind that is the longest entry, and nothing asks for the sums: 20 us a step of a prompt's host time)
         kv_len = batch.host_array("kv_len").astype(np.int64)
         read["small"] = int((np.where(big, 0, (rows + ROWS_PER_TILE - 1) // ROWS_PER_TILE) * kv_len).sum())
         most = [int(kv_len[m].max(initial=1)) for m in (big, ~big)]
