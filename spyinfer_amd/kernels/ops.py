@@ -1630,6 +1630,7 @@ def recurrence_by_chunks(d: int, dv: int) -> bool:
     return d in (64, 128) and dv % 16 == 0
 
 
+@functools.lru_cache(maxsize=256)          # (asked by every layer of a step)
 def recurrence_goes_by_chunks(S: int, T: int, H: int, d: int, dv: int, longest: Optional[int], delta: bool) -> bool:
     """Whether a step of the mLSTM or (``delta``) the delta rule goes by chunks, or token by token.  ``longest``: the longest entry's
     tokens (None: not known, by chunks wherever it can).
@@ -1649,6 +1650,23 @@ def recurrence_goes_by_chunks(S: int, T: int, H: int, d: int, dv: int, longest: 
         return longest > 4
     heads = H * d * dv / (128 * 128)
     return longest > max(8.0, 2 + 1.15 * (S * heads) ** 0.5) and heads * (T - S - longest) <= 250 * longest
+
+
+@functools.lru_cache(maxsize=256)
+def _chunks_workspace(S: int, T: int, H: int, d: int, dv: int) -> int:
+    """Floats of workspace for a step of the mLSTM or the delta rule by chunks (the same for both)."""
+    return hip().lib.spy_mlstm_workspace(ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(H), ctypes.c_int(d), ctypes.c_int(dv))
+
+
+def _scratch(device, *floats):
+    """One float32 allocation and the addresses of its parts, each 16-byte aligned (a part without floats: null)."""
+    at, starts = 0, []
+    for n in floats:
+        starts.append(at)
+        at += (n + 3) // 4 * 4
+    buf = torch.empty((at,), dtype=torch.float32, device=device)
+    base = buf.data_ptr()
+    return buf, [ctypes.c_void_p(base + 4 * start if n else 0) for start, n in zip(starts, floats)]
 
 
 def _entries(cu_q: torch.Tensor, slot_ids: torch.Tensor, what: str) -> int:
@@ -1684,25 +1702,23 @@ def mlstm(x: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: int, gates
            "mlstm: state must be float32 [slots, mlstm_state_size(H, d, dv)]")
     out = torch.empty((T, H * dv), dtype=x.dtype, device=x.device)
     if T:
-        tmp = torch.empty((T, H * dv), dtype=torch.float32, device=x.device)        # the read-outs before the heads' norm
-        parr, n_pieces, multi, work, abe, mfin = None, 0, False, None, None, None
+        parr, n_pieces, multi, work = None, 0, False, None
         chunks = recurrence_goes_by_chunks(S, T, H, d, dv, longest, False)
-        ws_floats = hip().lib.spy_mlstm_workspace(ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(H), ctypes.c_int(d), ctypes.c_int(dv)) if chunks else 0
-        ws = torch.empty((ws_floats,), dtype=torch.float32, device=x.device) if ws_floats else None
+        ws_floats = _chunks_workspace(S, T, H, d, dv) if chunks else 0
         if pieces is not None and pieces[2]:
             parr, n_pieces, multi = pieces
             _dev(parr)
             _check(parr.dtype == torch.int32 and parr.shape == (4 * n_pieces,) and n_pieces > 0, "mlstm: pieces must be int32 [4 n]")
-            if ws is None:
+            if not chunks:
                 work = torch.empty((n_pieces, state.shape[1]), dtype=torch.float32, device=x.device)
-        if multi or ws is not None:
-            abe = torch.empty((T, 3 * H), dtype=torch.float32, device=x.device)
-            mfin = torch.empty((S, H), dtype=torch.float32, device=x.device)
-        hip().call("spy_mlstm", _ptr(out), _ptr(tmp), _ptr(state), ctypes.c_void_p(x.data_ptr()), ctypes.c_longlong(xs), _code(x, "x"), ctypes.c_int(q_off),
+        scalars = multi or chunks
+        # the read-outs before the heads' norm, the tokens' scalars, the entries' last maxima, the chunks
+        _buf, (tmp, abe, mfin, ws) = _scratch(x.device, T * H * dv, 3 * T * H if scalars else 0, S * H if scalars else 0, ws_floats)
+        hip().call("spy_mlstm", _ptr(out), tmp, _ptr(state), ctypes.c_void_p(x.data_ptr()), ctypes.c_longlong(xs), _code(x, "x"), ctypes.c_int(q_off),
                    ctypes.c_int(k_off), ctypes.c_int(v_off), ctypes.c_int(g_off), _ptr(gates), _ptr(bi), _ptr(bf), _code(bi, "gate biases"),
                    ctypes.c_float(cap), _ptr(norm_w), ctypes.c_float(eps), _ptr(cu_q), _ptr(slot_ids), ctypes.c_int(state.shape[0]),
                    ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(H), ctypes.c_int(d), ctypes.c_int(dv), _ptr(parr), ctypes.c_int(n_pieces),
-                   ctypes.c_int(1 if multi else 0), _ptr(work), _ptr(abe), _ptr(mfin), _ptr(ws), ctypes.c_int64(ws_floats),
+                   ctypes.c_int(1 if multi else 0), _ptr(work), abe, mfin, ws, ctypes.c_int64(ws_floats),
                    ctypes.c_int(1 if chunks else 0), _Hip.stream())
     return out
 
@@ -1759,16 +1775,15 @@ def delta_rule(qkv: torch.Tensor, beta_pre: torch.Tensor, dec_pre: torch.Tensor,
     _check(state.dtype == torch.float32 and state.dim() == 2 and state.shape[1] >= H * d * dv, "delta_rule: state must be float32 [slots, >= H d dv]")
     out = torch.empty((T, H * dv), dtype=qkv.dtype, device=qkv.device)
     if T:
-        tmp = torch.empty((T, H * dv), dtype=torch.float32, device=qkv.device)      # the read-outs before the heads' norm
-        unit = torch.empty((T, 2 * G * d), dtype=torch.float32, device=qkv.device)  # q and k as unit vectors
         chunks = recurrence_goes_by_chunks(S, T, H, d, dv, longest, True)
-        ws_floats = hip().lib.spy_delta_rule_workspace(ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(H), ctypes.c_int(d), ctypes.c_int(dv)) if chunks else 0
-        ws = torch.empty((max(1, ws_floats),), dtype=torch.float32, device=qkv.device)
-        hip().call("spy_delta_rule", _ptr(out), _ptr(tmp), _ptr(unit), _ptr(state), ctypes.c_longlong(state.shape[1]), _ptr(qkv), _code(qkv, "qkv"),
+        ws_floats = _chunks_workspace(S, T, H, d, dv) if chunks else 0
+        # the read-outs before the heads' norm, q and k as unit vectors, the chunks
+        _buf, (tmp, unit, ws) = _scratch(qkv.device, T * H * dv, 2 * T * G * d, ws_floats)
+        hip().call("spy_delta_rule", _ptr(out), tmp, unit, _ptr(state), ctypes.c_longlong(state.shape[1]), _ptr(qkv), _code(qkv, "qkv"),
                    ctypes.c_void_p(beta_pre.data_ptr()), ctypes.c_void_p(dec_pre.data_ptr()), _ptr(a_log), _ptr(dt_bias), _code(a_log, "decay numbers"), ctypes.c_void_p(gate.data_ptr()), ctypes.c_longlong(gs),
                    _ptr(norm_w), ctypes.c_float(eps), _ptr(cu_q), _ptr(slot_ids), ctypes.c_int(state.shape[0]), ctypes.c_int(S), ctypes.c_int(T),
                    ctypes.c_int(H), ctypes.c_int(G), ctypes.c_int(d), ctypes.c_int(dv), ctypes.c_int(dd), ctypes.c_int(1 if gate_act == "silu" else 0),
-                   ctypes.c_longlong(bs), ctypes.c_longlong(zs), _ptr(ws), ctypes.c_int64(ws_floats), ctypes.c_int(1 if chunks else 0), _Hip.stream())
+                   ctypes.c_longlong(bs), ctypes.c_longlong(zs), ws, ctypes.c_int64(ws_floats), ctypes.c_int(1 if chunks else 0), _Hip.stream())
     return out
 
 
