@@ -330,6 +330,87 @@ extern "C" int spy_add_rmsnorm(float* resid, const void* delta, const void* delt
     return 0;
 }
 
+// The same norm where the addend is still a product's parts [n_parts, T, H] (float32, gemm_rows.hip): resid += their sum, which is
+// not rounded before it meets the stream.  Bound by the parts' way through the caches; a thread asks for all pieces of two parts at once.
+template <typename TA, typename TW>
+__global__ void add_parts_rmsnorm_kernel(float* __restrict__ resid, const float* __restrict__ parts, int n_parts, const TW* __restrict__ w,
+                                         float eps, TA* __restrict__ out, const int* __restrict__ rows, int T, int H) {
+    __shared__ float red[16];
+    const int r = blockIdx.x;
+    int t = r;
+    if (rows) {
+        t = rows[r];
+        if (t < 0 || t >= T) {
+            for (int i = threadIdx.x; i < H; i += blockDim.x) out[(size_t)r * H + i] = from_f32<TA>(0.f);
+            return;
+        }
+    }
+    float* x = resid + (size_t)t * H;
+    const float* pr = parts + (size_t)t * H;
+    const size_t step = (size_t)T * H;
+    float v[NORM_PASSES][4], s[NORM_PASSES][4];
+#pragma unroll
+    for (int p = 0; p < NORM_PASSES; ++p) {
+        const int i = (p * blockDim.x + threadIdx.x) * 4;
+        if (i < H) {
+            Vec4<float>::load(x + i, v[p]);
+            Vec4<float>::load(pr + i, s[p]);
+        }
+    }
+#pragma unroll 2
+    for (int k = 1; k < n_parts; ++k) {
+#pragma unroll
+        for (int p = 0; p < NORM_PASSES; ++p) {
+            const int i = (p * blockDim.x + threadIdx.x) * 4;
+            if (i < H) {
+                float a[4];
+                Vec4<float>::load(pr + k * step + i, a);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[p][e] += a[e];
+            }
+        }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int p = 0; p < NORM_PASSES; ++p) {
+        const int i = (p * blockDim.x + threadIdx.x) * 4;
+        if (i < H) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[p][e] += s[p][e];
+                ss += v[p][e] * v[p][e];
+            }
+            if (!rows) Vec4<float>::store(x + i, v[p]);
+        }
+    }
+    ss = block_sum(ss, red);
+    const float scale = 1.0f / sqrtf(ss / (float)H + eps);
+#pragma unroll
+    for (int p = 0; p < NORM_PASSES; ++p) {
+        const int i = (p * blockDim.x + threadIdx.x) * 4;
+        if (i < H) {
+            float w4[4], y[4];
+            Vec4<TW>::load(w + i, w4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = (scale * v[p][e]) * w4[e];
+            Vec4<TA>::store(out + (size_t)r * H + i, y);
+        }
+    }
+}
+
+// rows as in spy_add_rmsnorm.  H % 4 == 0, H <= 1024 NORM_PASSES, 16-byte aligned operands.
+extern "C" int spy_add_parts_rmsnorm(float* resid, const float* parts, int n_parts, const void* w, int w_dtype, float eps, void* out, int out_dtype,
+                                     const int* rows, int n_out, int T, int H, hipStream_t st) {
+    SPY_REQUIRE(n_out > 0 && T > 0 && H > 0 && n_parts > 0, "spy_add_parts_rmsnorm: empty operand");
+    const int threads = H >= 2048 ? 256 : (H >= 512 ? 128 : 64);
+    SPY_REQUIRE(H % 4 == 0 && H <= threads * 4 * NORM_PASSES, "spy_add_parts_rmsnorm: rows of %d", H);
+    SPY_REQUIRE((((uintptr_t)resid | (uintptr_t)parts | (uintptr_t)w | (uintptr_t)out) % 16) == 0, "spy_add_parts_rmsnorm: operands must be 16-byte aligned");
+    SPY_DISPATCH(out_dtype, TA, SPY_DISPATCH(w_dtype, TW, (add_parts_rmsnorm_kernel<TA, TW><<<n_out, threads, 0, st>>>(
+        resid, parts, n_parts, (const TW*)w, eps, (TA*)out, rows, T, H))));
+    SPY_CHECK_LAUNCH("spy_add_parts_rmsnorm");
+    return 0;
+}
+
 template <typename TA, typename TW>
 __global__ void rmsnorm_kernel(const TA* __restrict__ x, long long ldx, const TW* __restrict__ w, float eps, TA* __restrict__ out, int n) {
     // (ldx: values from one input row to the next: the rows may lie inside a wider product; the output is dense)

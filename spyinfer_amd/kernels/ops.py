@@ -81,7 +81,8 @@ class _Hip:
                      "spy_bias_rope_store", "spy_sigmoid_gate", "spy_mlstm", "spy_mlstm_workspace", "spy_causal_conv_silu", "spy_delta_rule", "spy_delta_rule_workspace", "spy_moe_route",
                      "spy_moe_align", "spy_moe_gemm", "spy_moe_combine", "spy_moe_tile_rows", "spy_moe_group_ints", "spy_token_shift", "spy_tanh", "spy_time_mix",
                      "spy_norm_pair_mean", "spy_scale_cap", "spy_result_norm", "spy_moe_align_tables", "spy_layer_norm", "spy_layer_norm_residual",
-                     "spy_gelu", "spy_norm_rope_store", "spy_map_difference", "spy_rotation_angles", "spy_decay_memory", "spy_group_norm"):
+                     "spy_gelu", "spy_norm_rope_store", "spy_map_difference", "spy_rotation_angles", "spy_decay_memory", "spy_group_norm", "spy_gemm_rows",
+                     "spy_add_parts_rmsnorm"):
             if not hasattr(self.lib, name):
                 raise KernelError("the kernel library %s lacks %s: it is older than its sources; build it again "
                                   "(spyinfer_amd.kernels.build.build())" % (self.lib._name, name))
@@ -480,6 +481,90 @@ def linear_few(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor] =
     return linear(x, w, out_dtype, tiled=tiled, out=out)
 
 
+#: most bytes of a product's parts
+PARTS_MAX_BYTES = 64 << 20
+
+
+def _rows_product_us(M: int, N: int, K: int, tiles: int, parts: int) -> float:
+    """Estimated time of ``spy_gemm_rows`` with ``tiles`` row tiles a block: turns of 128 of K one after the other on the
+    compute unit that has most blocks, and the parts' way to memory.  The four numbers are fitted to 700 launches of 130 to 2011
+    rows, 1024 to 6144 columns and K of 1024 to 12288; the choice it makes costs 0.8 % more than the best one on average,
+    9 % at most, the sum of the parts counted on both sides."""
+    blocks = -(-M // (16 * tiles)) * -(-N // 256) * parts
+    return 5.0 + -(-blocks // 256) * -(-K // 128 // parts) * (0.7 + 0.05 * tiles) + parts * M * N * 4 / 2.25e6
+
+
+@functools.lru_cache(maxsize=1024)
+def rows_product_parts(M: int, N: int, K: int):
+    """(row tiles, parts of K) for a product of M rows whose result the next norm sums from its parts (``linear_parts``), or None
+    where the library's product is the better one: it has tiles for the whole chip, or K is too short for the parts to pay.
+    Measured, us with the parts' sum against the library's: 409 rows, 2560 x 9728: 33 / 54; 1100 rows: 64 / 70, 2011 rows (beyond
+    the line): 106 / 104; 1356 rows, 4096 x 12288: 137 / 138; 800 rows, 2560 x 4096: 29 / 35, 1100 rows (beyond): 33 / 31; 1356 rows,
+    2048 x 6144: 46 / 45; 560 rows, 1024 x 3072: 12.0 / 13.8; K = 2048: 409 rows, 2048 columns: 14 / 11."""
+    if M <= DECODE_ROWS_PLAIN or N % 16 or K % 128 or K < 3072 or M * N * 4096 > 2.3e6 * K or N * K >= 1 << 30 or M * K >= 1 << 30:
+        return None
+    fits = [(t, p) for t in range(4, 9) if 16 * t <= M for p in range(1, min(12, K // 256) + 1)
+            if p * M * N * 4 <= PARTS_MAX_BYTES and -(-M // (16 * t)) * -(-N // 256) * p <= 512]
+    return min(fits, key=lambda f: _rows_product_us(M, N, K, *f), default=None)
+
+
+@functools.lru_cache(maxsize=1024)
+def rows_product_gated(M: int, N: int, K: int, library: bool) -> int:
+    """Row tiles a block of the gated product of many rows (N = 2 I rows of the matrix), or 0 where the library's product and a pass
+    for the activation are the better ones (``library`` false: that way is not at hand at its own price).  It loses where its blocks
+    leave half of the chip idle, but for a short K (us, with the library's activation pass: 409 rows, 6144 x 4096: 44 against 38, 560
+    rows: 44 / 46, 409 rows, 6144 x 1024: 14 / 21), and to the library's larger tiles for the largest products (1700 rows, 24576 x
+    4096: 291 / 284, 1356 rows: 237 / 259; 2011 rows, 19456 x 2560: 171 / 221)."""
+    if M <= DECODE_ROWS_PLAIN or N % 32 or K % 128 or N * K >= 1 << 30 or M * K >= 1 << 30:
+        return 0
+    if library and ((-(-M // 64) * -(-N // 256) < 128 and K > 1024) or (M > 1500 and N * K > 90e6)):
+        return 0
+    return min((t for t in range(4, 9) if 16 * t <= M), key=lambda t: _rows_product_us(M, N, K, t, 1))
+
+
+class ProductParts:
+    """A product's result while it still lies in parts [parts, T, N] float32 (K cut over blocks); the norm that reads the result
+    sums them in its pass (``add_parts_rms_norm``)."""
+    __slots__ = ("parts",)
+
+    def __init__(self, parts):
+        self.parts = parts
+
+    def resolve(self):
+        return self.parts.sum(dim=0)
+
+
+def linear_parts(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor] = None):
+    """``linear_few``, or, where a product of many rows is better cut along K, its ``ProductParts``."""
+    M, K = x.shape
+    plan = rows_product_parts(M, w.shape[0], K) if tiled is not None and x.dtype == torch.bfloat16 and x.is_contiguous() else None
+    if plan is None:
+        return linear_few(x, w, tiled)
+    _dev(x, tiled)
+    N = w.shape[0]
+    _check(tuple(tiled.shape) == (N, K) and w.shape[1] == K, "linear_parts: the matrix or its tiled copy does not fit rows of %d", K)
+    parts = torch.empty((plan[1], M, N), dtype=torch.float32, device=x.device)
+    hip().call("spy_gemm_rows", _ptr(parts), _ptr(x), _ptr(tiled), M, N, K, plan[0], plan[1], 0, 0, _Hip.stream())
+    return ProductParts(parts)
+
+
+def add_parts_rms_norm(resid: torch.Tensor, addend: ProductParts, weight: torch.Tensor, eps: float, out_dtype: torch.dtype,
+                       rows: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``add_rms_norm`` of an addend in parts, which are summed in float32 in the order of K and not rounded."""
+    T, H = resid.shape
+    parts = addend.parts
+    _dev(resid, parts, weight, rows)
+    _check(resid.dtype == torch.float32 and parts.dtype == torch.float32 and tuple(parts.shape[1:]) == (T, H) and weight.shape == (H,),
+           "add_parts_rms_norm: stream [T, H], parts [parts, T, H] in float32 and a weight [H] expected")
+    _check(rows is None or (rows.dtype == torch.int32 and rows.dim() == 1), "add_parts_rms_norm: rows must be int32 [R]")
+    n_out = T if rows is None else rows.shape[0]
+    out = torch.empty((n_out, H), dtype=out_dtype, device=resid.device)
+    if n_out:
+        hip().call("spy_add_parts_rmsnorm", _ptr(resid), _ptr(parts), parts.shape[0], _ptr(weight), _code(weight, "norm weight"),
+                   ctypes.c_float(eps), _ptr(out), _code(out, "norm output"), _ptr(rows), n_out, T, H, _Hip.stream())
+    return out
+
+
 #: activations of a gated feed-forward: "silu", or the tanh form of gelu, z/2 (1 + tanh(sqrt(2/pi) (z + 0.044715 z^3)))
 GATED_ACTIVATIONS = {"silu": 0, "gelu_tanh": 1}
 #: code of the exact gelu, the activation of products without a gate
@@ -489,7 +574,7 @@ ACT_GELU = 2
 def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, tiled: Optional[torch.Tensor] = None, few_rows: int = 0,
                   activation: str = "silu") -> torch.Tensor:
     """act(x . Wgate^T) * (x . Wup^T) with ``w_gate_up [2 I, K]`` = [Wgate | Wup] -> [M, I].  For few bfloat16 rows
-    (decode) one kernel does both products and the activation; otherwise it is linear() followed by swiglu().  ``few_rows``:
+    (decode), and for most sizes of many, one kernel does both products and the activation; otherwise it is linear() followed by swiglu().  ``few_rows``:
     most rows that the tiled kernel takes here (0: SKINNY_MAX_ROWS).  ``activation``: one of GATED_ACTIVATIONS."""
     _dev(x, w_gate_up)
     _check(x.dim() == 2 and w_gate_up.dim() == 2 and x.shape[1] == w_gate_up.shape[1] and w_gate_up.shape[0] % 2 == 0,
@@ -505,6 +590,13 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, tiled: Optional[torc
         hip().call("spy_gemm_skinny_swiglu", _ptr(x), _ptr(w_gate_up), _ptr(out), _code(out, "out"), ctypes.c_int(M),
                    ctypes.c_int(I), ctypes.c_int(K), ctypes.c_int(GATED_ACTIVATIONS[activation]), _Hip.stream())
         return out
+    if x.dtype == torch.bfloat16 and tiled is not None and x.is_contiguous():
+        tiles = rows_product_gated(M, 2 * I, K, not isinstance(w_gate_up, TiledOnly))
+        if tiles:
+            _check(tiled.shape == w_gate_up.shape, "linear_swiglu: the tiled copy does not fit")
+            out = torch.empty((M, I), dtype=x.dtype, device=x.device)
+            hip().call("spy_gemm_rows", _ptr(out), _ptr(x), _ptr(tiled), M, 2 * I, K, tiles, 1, 1, GATED_ACTIVATIONS[activation], _Hip.stream())
+            return out
     return swiglu(linear(x, w_gate_up), activation)
 
 
@@ -584,7 +676,7 @@ class EntryAddends:
         pend = None if isinstance(self.pending, ScaledInput) else self.pending
         for addend in (pend if isinstance(pend, (tuple, list)) else (pend,)):
             if addend is not None:
-                resid.add_((addend.resolve() if isinstance(addend, (GatedAddend, NormedAddend)) else addend).float())
+                resid.add_((addend.resolve() if isinstance(addend, (GatedAddend, NormedAddend, ProductParts)) else addend).float())
         if self.base is not None:
             resid.add_(self.base)
         if self.vec is not None:

@@ -394,6 +394,12 @@ class PagedAttention(Mixer):
             return ops.linear_few(self._attend(x, batch, cache, store), self.w_o, self.w_o_tiled)
         return ops.linear(self._attend(x, batch, cache, store), self.w_o, tiled=self.w_o_tiled)
 
+    def forward_parts(self, x, batch, cache, store=True):
+        """``forward`` for a block whose next norm takes the result in parts (``ops.ProductParts``)."""
+        if type(self).forward is not PagedAttention.forward or batch.T <= ops.DECODE_ROWS_PLAIN:
+            return self.forward(x, batch, cache, store)
+        return ops.linear_parts(self._attend(x, batch, cache, store), self.w_o, self.w_o_tiled)
+
     def forward_into(self, x, batch, cache, store, resid, next_norm):
         weight, eps = next_norm.foldable(batch.act_dtype)
         return ops.decode_linear_residual(self._attend(x, batch, cache, store, for_product=True), self.w_o_tiled, resid, weight, eps,

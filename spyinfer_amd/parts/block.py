@@ -117,12 +117,17 @@ class PreNormBlock(Block):
                 return resid, self.ffn.forward_into(n2, batch, resid, next_norm)
             return resid, self.ffn.forward(n2, batch)
         n1 = self.norm1.add_norm(resid, None if ready else pending, act)
-        a = self.mixer.forward(n1, batch, cache, store)
+        # (a result in parts goes to the norm that sums them: to the next block's only if that one is known)
+        in_parts = self.gate1 is None and hasattr(self.mixer, "forward_parts") \
+            and getattr(next_norm if self.ffn is None else self.norm2, "takes_product_parts", False)
+        a = (self.mixer.forward_parts if in_parts else self.mixer.forward)(n1, batch, cache, store)
         if self.gate1 is not None:
             a = self.gate1.apply(a, n1)
         if self.ffn is None:
             return resid, a
         n2 = self.norm2.add_norm(resid, a, act)
+        if self.gate2 is None and hasattr(self.ffn, "forward_parts") and getattr(next_norm, "takes_product_parts", False):
+            return resid, self.ffn.forward_parts(n2, batch)
         if getattr(self.gate2, "takes_expert_rows", False) and hasattr(self.ffn, "forward_unsummed"):
             f = self.ffn.forward_unsummed(n2, batch)
         else:

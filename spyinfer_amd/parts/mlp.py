@@ -59,6 +59,13 @@ class GatedMLP(FeedForward):
         return ops.linear_few(ops.linear_swiglu(x, self.w_gate_up, self.w_gate_up_tiled, few_rows=ops.DECODE_ROWS_PLAIN, activation=self.activation),
                               self.w_down, self.w_down_tiled)
 
+    def forward_parts(self, x, batch):
+        """``forward`` for a block whose next norm takes the result in parts (``ops.ProductParts``)."""
+        if type(self).forward is not GatedMLP.forward or isinstance(x, ops.ScaledInput):
+            return self.forward(x, batch)
+        return ops.linear_parts(ops.linear_swiglu(x, self.w_gate_up, self.w_gate_up_tiled, few_rows=ops.DECODE_ROWS_PLAIN, activation=self.activation),
+                                self.w_down, self.w_down_tiled)
+
     def forward_into(self, x, batch, resid, next_norm):
         weight, eps = next_norm.foldable(batch.act_dtype)
         act = ops.decode_linear_swiglu(x, self.w_gate_up_tiled, for_product=True, activation=self.activation)

@@ -11,6 +11,8 @@ from .base import Norm
 
 
 class RMSNorm(Norm):
+    takes_product_parts = True     # ``add_norm`` sums a product's parts (``ops.ProductParts``) in its own pass
+
     def __init__(self, size: int, eps: float, suffix: str = ".weight", offset: float = 0.0, groups: int = 1, scalar: bool = False):
         """``groups``: the vector is cut into that many equal consecutive parts, each over its own root mean square (the
         weight still spans the whole vector).  ``suffix``: what the weight's name has behind the part's prefix (some checkpoints name the vector by the
@@ -47,6 +49,10 @@ class RMSNorm(Norm):
         ``ops.GatedAddend`` or ``ops.NormedAddend`` (a result behind a gate or a norm of its own), or an
         ``ops.EntryAddends`` (any of these plus an earlier state of the stream and a vector for every row).  ``second``:
         another norm of this kind that reads the same sum: the result is the pair of both outputs, from one pass."""
+        if isinstance(delta, ops.ProductParts):
+            if second is None and self.groups == 1 and self.size % 4 == 0 and self.size <= 8192:
+                return ops.add_parts_rms_norm(resid, delta, self.weight, self.eps, out_dtype, rows)
+            delta = delta.resolve().to(out_dtype)
         if isinstance(delta, ops.NormedAddend):
             # a sublayer's result behind a norm of its own: both norms and the sum in one pass
             if second is None and self.groups == 1:
@@ -58,7 +64,7 @@ class RMSNorm(Norm):
             delta = None if isinstance(delta.pending, ops.ScaledInput) else delta.pending
             if isinstance(delta, ops.GatedAddend):
                 delta = delta.resolve()
-            elif isinstance(delta, ops.NormedAddend):
+            elif isinstance(delta, (ops.NormedAddend, ops.ProductParts)):
                 delta = delta.resolve().to(out_dtype)
         if second is not None:
             if (second.size, second.eps, second.groups) != (self.size, self.eps, self.groups) or second.weight.dtype != self.weight.dtype:

@@ -1,0 +1,61 @@
+"""Products of many rows from the tiled copy (csrc/gemm_rows.hip): one turn of K, two, an odd number of them, parts of uneven length,
+every number of row tiles, a last tile of rows that reaches back, columns that are no multiple of a block's; and the norm that sums a
+product's parts; against float64."""
+import pytest
+import torch
+
+from tests.gpu_util import close, require_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,N,K,tiles,parts", [(65, 272, 128, 4, 1), (128, 256, 256, 8, 2), (200, 1040, 384, 7, 3), (131, 512, 640, 5, 2), (193, 48, 1280, 6, 4),
+                                               (112, 768, 896, 7, 7), (500, 256, 512, 8, 1)])
+def test_parts(M, N, K, tiles, parts, monkeypatch):
+    from spyinfer_amd.kernels import ops
+    monkeypatch.setattr(ops, "rows_product_parts", lambda *size: (tiles, parts))
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn((M, K), generator=g).bfloat16(), (torch.randn((N, K), generator=g) * K ** -0.5).bfloat16()
+    wd = w.to(dev)
+    out = ops.linear_parts(x.to(dev), wd, ops.tile_weight(wd))
+    assert isinstance(out, ops.ProductParts) and tuple(out.parts.shape) == (parts, M, N)
+    # exact products of bfloat16 values, K float32 sums of terms of size K^-1/2: an error of some 2^-24 sqrt(K) terms' sizes
+    bounds = [K // 128 * p // parts * 128 for p in range(parts + 1)]
+    for p, (a, b) in enumerate(zip(bounds, bounds[1:])):
+        ref = x[:, a:b].double() @ w[:, a:b].double().T
+        assert float((out.parts[p].cpu().double() - ref).abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("M,I,K,tiles", [(65, 128, 128, 4), (200, 144, 256, 7), (131, 16, 384, 5), (193, 1040, 640, 6), (300, 384, 1152, 8)])
+def test_gated(M, I, K, tiles, activation, monkeypatch):
+    from spyinfer_amd.kernels import ops
+    monkeypatch.setattr(ops, "rows_product_gated", lambda *size: tiles)
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(M + I)
+    x, w = torch.randn((M, K), generator=g).bfloat16(), (torch.randn((2 * I, K), generator=g) * K ** -0.5).bfloat16()
+    wd = w.to(dev)
+    out = ops.linear_swiglu(x.to(dev), wd, ops.tile_weight(wd), activation=activation)
+    h = x.double() @ w.double().T
+    act = torch.nn.functional.silu if activation == "silu" else lambda z: torch.nn.functional.gelu(z, approximate="tanh")
+    close(out, act(h[:, :I]) * h[:, I:], torch.bfloat16, what="gated product of many rows")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,H,parts", [(65, 64, 1), (70, 516, 3), (130, 2560, 6), (66, 8192, 2)])
+def test_norm_of_a_sum_of_parts(T, H, parts, dtype):
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(T + H)
+    resid, y = torch.randn((T, H), generator=g), torch.randn((parts, T, H), generator=g)
+    w = torch.randn((H,), generator=g).to(dtype)
+    rows = torch.tensor([T - 1, 0, 7], dtype=torch.int32)
+    total = resid.double() + y.double().sum(0)
+    ref = total / torch.sqrt((total * total).mean(-1, keepdim=True) + 1e-6) * w.double()
+    stream = resid.to(dev)
+    some = ops.add_parts_rms_norm(stream, ops.ProductParts(y.to(dev)), w.to(dev), 1e-6, dtype, rows.to(dev))
+    assert torch.equal(stream.cpu(), resid)                       # (picked rows: the stream stays as it is)
+    close(some, ref[rows.long()], dtype, what="picked rows")
+    close(ops.add_parts_rms_norm(stream, ops.ProductParts(y.to(dev)), w.to(dev), 1e-6, dtype), ref, dtype, what="normed sum")
+    close(stream, total, torch.float32, what="the stream")

@@ -1,0 +1,26 @@
+"""The sizes that go to the products of many rows, and what they are launched with: within what the kernel takes, for every size."""
+import random
+
+from spyinfer_amd.kernels import ops
+
+
+def test_launches_fit_the_kernel():
+    rng = random.Random(3)
+    for _ in range(3000):
+        M, N, K = int(2 ** rng.uniform(0, 14)), 16 * rng.randint(1, 2000), 128 * rng.randint(1, 120)
+        plan = ops.rows_product_parts.__wrapped__(M, N, K)
+        if plan is not None:
+            tiles, parts = plan
+            assert M > 64 and 4 <= tiles <= 8 and 16 * tiles <= M and 1 <= parts <= K // 256 and parts * M * N * 4 <= ops.PARTS_MAX_BYTES
+            assert N * K < 1 << 30 and M * K < 1 << 30
+        tiles = ops.rows_product_gated.__wrapped__(M, 2 * N, K, True)
+        assert tiles == 0 or (M > 64 and 4 <= tiles <= 8 and 16 * tiles <= M and 2 * N * K < 1 << 30 and M * K < 1 << 30)
+
+
+def test_sizes_on_both_sides_of_the_line():
+    assert ops.rows_product_parts(409, 2560, 9728) == (7, 6)
+    assert ops.rows_product_parts(2011, 2560, 9728) is not None and ops.rows_product_parts(2011, 4096, 12288) is None
+    assert ops.rows_product_parts(64, 2560, 9728) is None and ops.rows_product_parts(409, 2048, 2048) is None
+    assert ops.rows_product_gated(1356, 12288, 2048, True) == 6 and ops.rows_product_gated(64, 12288, 2048, True) == 0
+    assert ops.rows_product_gated(2011, 24576, 4096, True) == 0 and ops.rows_product_gated(2011, 24576, 4096, False) > 0
+    assert ops.rows_product_gated(200, 6144, 4096, True) == 0
