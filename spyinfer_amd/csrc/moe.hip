@@ -332,7 +332,8 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(TC* __restrict__ C, const
 typedef __attribute__((__vector_size__(8 * sizeof(short)))) short moe_bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float moe_f32x4_t;
 
-template <bool GATED, typename TC>
+// TILED: the experts' matrices lie in operand order (gemm_decode.h), so that a load is 1 KB in one piece.
+template <bool GATED, bool TILED, typename TC>
 __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(TC* __restrict__ C, const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                                             const int* __restrict__ tile_expert, const int* __restrict__ sorted_pair,
                                                             int gather, int N, int K, long long w_stride, MoeAct act) {
@@ -349,14 +350,18 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(TC* __restrict__ C, 
     const bf16_t* We = W + (size_t)e * w_stride;
     const bf16_t* wrow[2];
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) wrow[nt] = We + (size_t)(GATED ? nt * N + min(n0 + r, N - 1) : min(n0 + nt * 16 + r, N - 1)) * K + 8 * g;
+    for (int nt = 0; nt < 2; ++nt) {
+        if (TILED) wrow[nt] = We + (size_t)(GATED ? (nt * N + n0) / 16 : min(n0 / 16 + nt, N / 16 - 1)) * 2048 + lane * 8;
+        else wrow[nt] = We + (size_t)(GATED ? nt * N + min(n0 + r, N - 1) : min(n0 + nt * 16 + r, N - 1)) * K + 8 * g;
+    }
+    const size_t w_step = TILED ? 512 : 32, w_wide = TILED ? (size_t)(GATED ? 2 : 1) * N : 1;          // (a chunk's values are K's 128 of all rows)
     moe_f32x4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
     auto load = [&](const bf16_t* q) { return *reinterpret_cast<const moe_bf16x8_t*>(q); };
     auto fetch = [&](moe_bf16x8_t (&a)[2][4], moe_bf16x8_t (&b)[4], int k) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
 #pragma unroll
-            for (int nt = 0; nt < 2; ++nt) a[nt][j] = load(wrow[nt] + k + 32 * j);
+            for (int nt = 0; nt < 2; ++nt) a[nt][j] = load(wrow[nt] + k * w_wide + w_step * j);
             b[j] = *reinterpret_cast<const moe_bf16x8_t*>(xrow + k + 32 * j);
         }
     };
@@ -387,7 +392,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tile_kernel(TC* __restrict__ C, 
             products(a0, b0);
         }
     }
-    if (wave == (chunks & 3)) {                              // the rest of K (a multiple of 8): the wave whose turn it would be
+    if (!TILED && wave == (chunks & 3)) {                    // the rest of K (a multiple of 8): the wave whose turn it would be
         const moe_bf16x8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
         for (int k = chunks << 7; k < K; k += 32) {
             const bool kok = k + 8 * g < K;
@@ -707,10 +712,141 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_group_kernel(TC* __restrict__
     }
 }
 
+// Many rows per expert, the experts' matrices in operand order: as in gemm_rows.hip (the comments on the data flow and the waits are
+// there), a block has a group's rows and 256 rows of W (gated: the gate and up rows of 128 columns), a wave all of the group's rows and 64
+// of W's; W goes from memory straight into operand registers, the gathered rows of A through two LDS stages, which carry half of what the
+// kernel above needs, whose bound they are.  Groups of fewer rows take fewer products: a block goes by two, four, six or eight row tiles.
+// Measured, both products, us, the kernel above / this one: 32 experts of 2 x 1536 x 2048 with 16 rows each 136 / 118, 64 rows 151 / 136,
+// 251 rows 268 / 235, 500 rows 470 / 371; 32 of 2 x 3072 x 4096 with 251 rows 980 / 745 (840 TFLOP/s), with 16 435 / 397 (6.1 TB/s); with
+// the same rows of W loaded from row order, 64 bytes of 16 rows a load, 322 for 268 of the first ones' 251 rows.
+#define MOE_HALVES 128
+template <int MT, bool GATED, typename TC>
+__device__ __forceinline__ void moe_rows_block(TC* C, const bf16_t* A, unsigned a_bytes, const bf16_t* We, const int* src_row, bf16_t* stage0,
+                                               bf16_t* stage1, int N, int K, int by, int t, const int* sorted_pair, const MoeAct& act) {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int NT = N / 16;
+    const auto wres = __builtin_amdgcn_make_buffer_rsrc((void*)We, 0, (GATED ? 2 : 1) * N * K * 2, 0x00020000);
+    const auto ares = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, a_bytes, 0x00020000);
+    const int w_lane = lane * 16, w_turn = (GATED ? 2 : 1) * N * 256;
+    int w_at[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int tile = GATED ? (j >> 1) * NT + min(by * 8 + wave * 2 + (j & 1), NT - 1) : min(by * 16 + wave * 4 + j, NT - 1);
+        w_at[j] = __builtin_amdgcn_readfirstlane(tile * 4096);
+    }
+    const int s_row = wave * 4 + (lane >> 4), s_piece = ((lane & 15) ^ s_row) * 16;
+    int a_lane[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) a_lane[i] = max(src_row[i * 16 + s_row], 0) * K * 2 + s_piece;
+    moe_f32x4_t acc[4][MT];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[j][i] = moe_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    moe_bf16x8_t w[4][4];
+    auto load_a = [&](bf16_t* stage, int c) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, (__attribute__((address_space(3))) void*)(stage + (i * 4 + wave) * 512), 16, a_lane[i], c * 256, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto load_w = [&](int s, int c) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            w[s][j] = __builtin_bit_cast(moe_bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(wres, w_lane, w_at[j] + c * w_turn + s * 1024, 0));
+    };
+    auto products = [&](const bf16_t* stage, int next, bool more) {
+        const bf16_t* ab = stage + r * 128;
+        moe_bf16x8_t a[4];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) a[q] = *reinterpret_cast<const moe_bf16x8_t*>(ab + (q % MT) * 2048 + ((4 * (q / MT) + g) ^ r) * 8);
+#pragma unroll
+        for (int q = 0; q < 4 * MT; ++q) {
+            const int s = q / MT, i = q % MT, ahead = q + 3;
+            if (ahead < 4 * MT) a[ahead % 4] = *reinterpret_cast<const moe_bf16x8_t*>(ab + (ahead % MT) * 2048 + ((4 * (ahead / MT) + g) ^ r) * 8);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[s][j], a[q % 4], acc[j][i], 0, 0, 0);
+            if (i == MT - 1 && more) load_w(s, next);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto turn = [&]() {                               // (the 16 loads of W are a turn's last)
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const int n = K / 128;
+    load_a(stage0, 0);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) load_w(s, 0);
+    turn();
+    int c = 0;
+    for (; c + 1 < n; c += 2) {
+        load_a(stage1, c + 1);
+        products(stage0, c + 1, true);
+        turn();
+        const int after = min(c + 2, n - 1);
+        load_a(stage0, after);
+        products(stage1, after, true);
+        turn();
+    }
+    if (c < n) products(stage0, 0, false);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        if (src_row[i * 16 + r] < 0) continue;
+        const size_t row = (size_t)t * MOE_TM + i * 16 + r;
+        const float rw = (GATED && act.pair_w) ? act.pair_w[sorted_pair[row]] : 1.f;
+#pragma unroll
+        for (int j = 0; j < (GATED ? 2 : 4); ++j) {
+            const int tile = GATED ? by * 8 + wave * 2 + j : by * 16 + wave * 4 + j;
+            if (tile >= NT) continue;
+            float y[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = GATED ? moe_gated(acc[j][i][e], acc[GATED ? j + 2 : j][i][e], act, rw) : moe_ungated(acc[j][i][e], act);
+            Vec4<TC>::store(C + row * N + tile * 16 + 4 * g, y);
+        }
+    }
+}
+
+template <bool GATED, typename TC>
+__global__ __launch_bounds__(256, 2) void moe_gemm_rows_kernel(TC* C, const bf16_t* A, unsigned a_bytes, const bf16_t* W, const int* tile_expert,
+                                                               const int* sorted_pair, const int* group, int gather, int N, int K, int gy,
+                                                               long long w_stride, MoeAct act) {
+    __shared__ __align__(1024) bf16_t stage0[128 * 128];
+    __shared__ __align__(1024) bf16_t stage1[128 * 128];
+    __shared__ int src_row[128];
+    // (blocks to the dies in runs of the (band, columns, group of the band) order, as above)
+    // Up to MOE_HALVES blocks, which leave half of the compute units idle, become two with half of their group's rows (2 experts of 2 x
+    // 1536 x 2048 with 128 rows each: 38 us for both products, 64 without; 8 of 2 x 4096 x 2048: 138, 151; with a line at 256 blocks 8
+    // experts with 64 rows take 122, 107 without)
+    const int total = group[0] * gy, halves = total <= MOE_HALVES ? 2 : 1, per = (total + MOE_DIES - 1) / MOE_DIES, idx = blockIdx.x / MOE_DIES;
+    const int half = idx >= per, v = (blockIdx.x % MOE_DIES) * per + (half ? idx - per : idx);
+    if (idx >= per * halves || v >= total) return;
+    const int band = group[2 + 2 * (v / gy)], first = band >> 3, n_band = band & 7, in_band = v - first * gy;
+    const int by = in_band / n_band, gr = group[1 + 2 * (first + in_band % n_band)], skip = half * (MOE_GROUP / 2);
+    const int t = (gr >> 4) + skip, tiles = halves == 1 ? gr & 15 : min((gr & 15) - skip, MOE_GROUP / 2);
+    if (tiles <= 0) return;
+    const bf16_t* We = W + (size_t)tile_expert[t] * w_stride;
+    if (threadIdx.x < 128) {
+        int src = -1;
+        if ((int)threadIdx.x < tiles * MOE_TM) {
+            const int p = sorted_pair[t * MOE_TM + threadIdx.x];
+            src = p < 0 ? -1 : (gather > 0 ? p / gather : t * MOE_TM + (int)threadIdx.x);
+        }
+        src_row[threadIdx.x] = src;
+    }
+    __syncthreads();
+    if (tiles > 6) moe_rows_block<8, GATED>(C, A, a_bytes, We, src_row, stage0, stage1, N, K, by, t, sorted_pair, act);
+    else if (tiles > 4) moe_rows_block<6, GATED>(C, A, a_bytes, We, src_row, stage0, stage1, N, K, by, t, sorted_pair, act);
+    else if (tiles > 2) moe_rows_block<4, GATED>(C, A, a_bytes, We, src_row, stage0, stage1, N, K, by, t, sorted_pair, act);
+    else moe_rows_block<2, GATED>(C, A, a_bytes, We, src_row, stage0, stage1, N, K, by, t, sorted_pair, act);
+}
+
 static int moe_gemm_mfma_launch(void* C, int c_dtype, const void* A, const void* W, const int* tile_expert, const int* sorted_pair,
-                                int gather, int gated, bool many, int max_tiles, int N, int K, MoeAct act, hipStream_t st) {
+                                int gather, int gated, int tiled, bool many, int max_tiles, int N, int K, MoeAct act, hipStream_t st) {
     const long long ws = (long long)(gated ? 2 : 1) * N * K;
-    if (many) {
+    if (many && !tiled) {
         const dim3 grid((max_tiles + 7) / 8, (N + (gated ? 63 : 127)) / (gated ? 64 : 128));
         SPY_REQUIRE(grid.y <= 65535, "spy_moe_gemm: too many columns");
         if (gated) {
@@ -724,30 +860,48 @@ static int moe_gemm_mfma_launch(void* C, int c_dtype, const void* A, const void*
     }
     const dim3 grid((N + (gated ? 15 : 31)) / (gated ? 16 : 32), max_tiles);
     SPY_REQUIRE(grid.y <= 65535, "spy_moe_gemm: too many row tiles");
-    if (gated) {
-        SPY_DISPATCH(c_dtype, TC, (moe_gemm_tile_kernel<true, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (const bf16_t*)W, tile_expert,
-                                                                                       sorted_pair, gather, N, K, ws, act)));
-    } else {
-        SPY_DISPATCH(c_dtype, TC, (moe_gemm_tile_kernel<false, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (const bf16_t*)W, tile_expert,
-                                                                                        sorted_pair, gather, N, K, ws, act)));
-    }
+#define MOE_TILE_LAUNCH(G, TILED)                                                                                                     \
+    SPY_DISPATCH(c_dtype, TC, (moe_gemm_tile_kernel<G, TILED, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (const bf16_t*)W, tile_expert, \
+                                                                                        sorted_pair, gather, N, K, ws, act)))
+    if (gated && tiled) { MOE_TILE_LAUNCH(true, true); }
+    else if (gated) { MOE_TILE_LAUNCH(true, false); }
+    else if (tiled) { MOE_TILE_LAUNCH(false, true); }
+    else { MOE_TILE_LAUNCH(false, false); }
+#undef MOE_TILE_LAUNCH
     return 0;
 }
 
-extern "C" int spy_moe_gemm(void* C, int c_dtype, const void* A, int a_dtype, const void* W, int w_dtype, const int* tile_expert,
+// byte offsets within an operand are 31 bits wide in the kernel for groups of rows and matrices in operand order (beyond: a tile at a time)
+static int64_t moe_a_bytes(int gather, int P, int max_tiles, int K) { return 2LL * K * (gather > 0 ? P / gather : (int64_t)max_tiles * MOE_TM); }
+static bool moe_rows_fit(int gather, int P, int max_tiles, int gated, int N, int K) {
+    return moe_a_bytes(gather, P, max_tiles, K) < (1LL << 31) && (int64_t)(gated ? 2 : 1) * N * K * 2 < (1LL << 31);
+}
+
+// w_tiled: every expert's matrix lies in operand order (bfloat16, whole tiles of 16 rows and whole steps of 128 of K)
+extern "C" int spy_moe_gemm(void* C, int c_dtype, const void* A, int a_dtype, const void* W, int w_dtype, int w_tiled, const int* tile_expert,
                             const int* sorted_pair, const int* group, int P, int gather, int gated, int max_tiles, int E, int N, int K,
                             int tiles_per_block, int act_kind, float limit, const float* pair_w, hipStream_t st) {
     SPY_REQUIRE(max_tiles > 0 && E > 0 && N > 0 && K > 0 && gather >= 0, "spy_moe_gemm: bad sizes (%d tiles)", max_tiles);
     SPY_REQUIRE((act_kind == 0 && !pair_w) || (act_kind == 1 && gated && limit > 0.f) || (act_kind == 2 && !gated && !pair_w), "spy_moe_gemm: activation %d with limit %g", act_kind, (double)limit);
     const MoeAct act = {act_kind, limit, pair_w};
     // bfloat16 operands in 16-byte pieces: the matrix cores; tiles_per_block: 0 = the plain float32 kernel
-    if (tiles_per_block >= 8 && group && a_dtype == SPY_BF16 && w_dtype == SPY_BF16 && K % 64 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16) == 0) {
-        const int cols = gated ? 64 : 128, gy = (N + cols - 1) / cols;
+    SPY_REQUIRE(!w_tiled || (tiles_per_block > 0 && a_dtype == SPY_BF16 && w_dtype == SPY_BF16 && K % 128 == 0 && N % 16 == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0),
+                "spy_moe_gemm: matrices in operand order are for bfloat16 rows, %d x %d", N, K);
+    if (tiles_per_block >= 8 && group && a_dtype == SPY_BF16 && w_dtype == SPY_BF16 && K % 64 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16) == 0 && (!w_tiled || moe_rows_fit(gather, P, max_tiles, gated, N, K))) {
+        const bool wide = w_tiled != 0;
+        const int cols = wide ? (gated ? 128 : 256) : (gated ? 64 : 128), gy = (N + cols - 1) / cols;
         const int64_t blocks = (int64_t)moe_max_groups(max_tiles, E, P) * gy;
         SPY_REQUIRE(blocks < (1 << 30), "spy_moe_gemm: too many blocks");
-        const unsigned grid = (unsigned)((blocks + MOE_DIES - 1) / MOE_DIES * MOE_DIES);
+        const int64_t most = wide ? max(blocks, min(2 * blocks, (int64_t)2 * MOE_HALVES + MOE_DIES)) : blocks;
+        const unsigned grid = (unsigned)((most + MOE_DIES - 1) / MOE_DIES * MOE_DIES);
         const long long ws = (long long)(gated ? 2 : 1) * N * K;
-        if (gated) {
+        if (wide && gated) {
+            SPY_DISPATCH(c_dtype, TC, (moe_gemm_rows_kernel<true, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (unsigned)moe_a_bytes(gather, P, max_tiles, K), (const bf16_t*)W, tile_expert,
+                                                                                           sorted_pair, group, gather, N, K, gy, ws, act)));
+        } else if (wide) {
+            SPY_DISPATCH(c_dtype, TC, (moe_gemm_rows_kernel<false, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (unsigned)moe_a_bytes(gather, P, max_tiles, K), (const bf16_t*)W, tile_expert,
+                                                                                            sorted_pair, group, gather, N, K, gy, ws, act)));
+        } else if (gated) {
             SPY_DISPATCH(c_dtype, TC, (moe_gemm_group_kernel<true, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (const bf16_t*)W, tile_expert, sorted_pair,
                                                                                             group, gather, N, K, gy, ws, act)));
         } else {
@@ -758,7 +912,7 @@ extern "C" int spy_moe_gemm(void* C, int c_dtype, const void* A, int a_dtype, co
         return 0;
     }
     if (tiles_per_block > 0 && a_dtype == SPY_BF16 && w_dtype == SPY_BF16 && K % 8 == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0) {
-        const int rc = moe_gemm_mfma_launch(C, c_dtype, A, W, tile_expert, sorted_pair, gather, gated, tiles_per_block >= 8, max_tiles, N, K, act, st);
+        const int rc = moe_gemm_mfma_launch(C, c_dtype, A, W, tile_expert, sorted_pair, gather, gated, w_tiled, tiles_per_block >= 8, max_tiles, N, K, act, st);
         if (rc) return rc;
         SPY_CHECK_LAUNCH("spy_moe_gemm (mfma)");
         return 0;

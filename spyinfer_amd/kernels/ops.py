@@ -2167,7 +2167,7 @@ class ExpertRows:
 
 
 @functools.lru_cache(maxsize=256)          # (asked by every mixture of a step)
-def experts_by_groups(pairs: int, experts: int, K: int, F: int, gated: bool) -> bool:
+def experts_by_groups(pairs: int, experts: int, K: int, F: int, gated: bool, tiled: bool = False) -> bool:
     """Whether ``pairs`` rows of ``experts`` experts (matrices of K and F) go by groups of up to 128 rows of one expert, or a tile of 16
     rows at a time: whichever should take less time.  A tile at a time, every tile reads its expert's matrices out of the caches; by
     groups they are read once, but a block takes all of K for 128 of their rows, 0.7 us for each 64 of K and F, which few experts leave
@@ -2176,15 +2176,57 @@ def experts_by_groups(pairs: int, experts: int, K: int, F: int, gated: bool) -> 
     with 4 127 / 137, with 8 138 / 137, with 16 181 / 139; of 2 x 3072 x 4096 with 4 451 / 426, with 8 479 / 429.  The estimates' numbers are
     those that make the fewest wrong choices: of 823 cases measured (1 to 128 experts of 2 to 96 rows each, nine sizes of matrices) the
     choice is 0.13 % behind the better one on average, at most 15 % in a case.  K or F no multiple of 64, where the kernel with groups does
-    not stand: from 16 rows an expert on."""
+    not stand: from 16 rows an expert on.  ``tiled``: the matrices lie in operand order, whose kernels are faster by different shares
+    (32 experts of 2 x 1536 x 2048 with 8 rows 112 / 114, with 16 132 / 118; two with 96 31 / 36, with 256 63 / 39): numbers of their own,
+    from 912 cases, 0.11 % behind on average and 9 % at most."""
     if K % 64 or F % 64:
         return pairs >= 16 * experts
     used = min(experts, pairs)
     megabytes = (3 if gated else 2) * K * F * 2e-6                   # of an expert's matrices
     tiles = max(used, pairs / 16 + used / 2)
+    if tiled:
+        one = 8 + (0.05 * used + 0.194 * tiles + 0.005 * pairs) * megabytes
+        return max(12.45 + 1.436 * (K + F) / 64, 22.4 + used * 0.2527 * megabytes) + pairs * megabytes * 0.00104 < one
     one = 8 + (0.04 * used + tiles / 5.1 + pairs / 180) * megabytes
     groups = max(9 + 1.3 * (K + F) / 64, 15 + used * megabytes / 3.9) + pairs * megabytes / 3000
     return groups < one
+
+
+class TiledExperts:
+    """Experts' matrices [E, N, K], each in the order of ``tile_weight``: every load of the products is then 1 KB in one piece."""
+    __slots__ = ("data", "shape")
+    dtype = property(lambda self: self.data.dtype)
+
+    def __init__(self, mats):
+        """``mats``: per expert the matrices whose rows make it up, one after the other (whole tiles of 16 rows of each)."""
+        E, N, K = len(mats), sum(m.shape[0] for m in mats[0]), mats[0][0].shape[1]
+        self.shape = torch.Size((E, N, K))
+        self.data = torch.empty((E, K // 128, N // 16, 4, 4, 16, 8), dtype=torch.bfloat16, device=mats[0][0].device)
+        for e, parts in enumerate(mats):
+            at = 0
+            for m in parts:
+                n = m.shape[0] // 16
+                self.data[e, :, at:at + n].copy_(m.view(n, 16, K // 128, 4, 4, 8).permute(2, 0, 3, 4, 1, 5))
+                at += n
+
+    @staticmethod
+    def takes(mats) -> bool:
+        return all(m.is_cuda and m.dtype == torch.bfloat16 and m.shape[0] % 16 == 0 and m.shape[1] % 128 == 0 and m.is_contiguous() for parts in mats for m in parts)
+
+    def dim(self) -> int:
+        return 3
+
+    def rows(self) -> torch.Tensor:
+        E, N, K = self.shape
+        return self.data.permute(0, 2, 5, 1, 3, 4, 6).reshape(E, N, K)
+
+
+def expert_forms(mats):
+    """Experts' matrices (per expert a list, one below the other) as a mixture keeps them for ``moe_experts``: in operand order where
+    shapes and dtype allow it, else [E, N, K]."""
+    if TiledExperts.takes(mats):
+        return TiledExperts(mats)
+    return torch.stack([torch.cat(parts, dim=0) if len(parts) > 1 else parts[0] for parts in mats]).contiguous()
 
 
 def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[torch.Tensor], w_gate_up: torch.Tensor, w_down: torch.Tensor,
@@ -2199,14 +2241,18 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
     in the pass that sums the choices (the result of a layer that every token uses).  ``align``: the pairs already sorted
     (``ids`` is not read then, and ``weights`` may be None: all one).  ``scale``: a factor on the sum over the choices.
     ``unsummed``: the result is ``ExpertRows`` instead of [T, K].  ``activation`` "gelu": experts without a gate, ``w_gate_up
-    [E, F, K]`` = every expert's up rows, down_e(gelu(up_e x)), the exact gelu."""
+    [E, F, K]`` = every expert's up rows, down_e(gelu(up_e x)), the exact gelu.  The matrices may be ``TiledExperts``."""
     _dev(add)
     _check(add is None or (add.shape == x.shape and add.dtype == x.dtype and add.is_contiguous()), "moe_experts: the addend must be like x")
     _check(activation in ("silu", "clamped", "gelu") and (activation != "clamped" or limit > 0.0), "moe_experts: activation silu, gelu, or clamped with a positive limit")
     act_kind = {"silu": 0, "clamped": 1, "gelu": ACT_GELU}[activation]
     gated = activation != "gelu"
     _check(gated or not weight_input, "moe_experts: experts without a gate take their weights at the output")
-    _dev(x, ids, weights, w_gate_up, w_down)
+    if x.dtype != torch.bfloat16:              # (the kernels for float32 rows read the matrices' rows)
+        w_gate_up, w_down = (w.rows() if isinstance(w, TiledExperts) else w for w in (w_gate_up, w_down))
+    up_tiled, down_tiled = isinstance(w_gate_up, TiledExperts), isinstance(w_down, TiledExperts)
+    up, down = w_gate_up.data if up_tiled else w_gate_up, w_down.data if down_tiled else w_down
+    _dev(x, ids, weights, up, down)
     T, K = x.shape
     top = ids.shape[1] if align is None else align.top
     E, F2, _ = w_gate_up.shape
@@ -2237,14 +2283,14 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
                "moe_experts: the alignment does not fit")
         sorted_pairs, tile_experts, group_list = _ptr(sorted_pair), _ptr(tile_expert), _ptr(groups)
     # bfloat16: the matrix cores, a block taking one row tile of an expert (decoding: blocks for the whole device) or up to eight
-    many = experts_by_groups(P, E, K, F, gated)
-    per_block = 0 if not MOE_MFMA or x.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16 else (8 if many else 1)
+    many = experts_by_groups(P, E, K, F, gated, up_tiled and down_tiled)
+    per_block = 0 if not (MOE_MFMA or up_tiled or down_tiled) or x.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16 else (8 if many else 1)
     act = torch.empty((max_tiles * tm, F), dtype=x.dtype, device=dev)
-    hip().call("spy_moe_gemm", _ptr(act), _code(act, "act"), _ptr(x), _code(x, "x"), _ptr(w_gate_up), _code(w_gate_up, "expert matrices"),
+    hip().call("spy_moe_gemm", _ptr(act), _code(act, "act"), _ptr(x), _code(x, "x"), _ptr(up), _code(up, "expert matrices"), ctypes.c_int(up_tiled),
                tile_experts, sorted_pairs, group_list, ctypes.c_int(P), ctypes.c_int(top), ctypes.c_int(1 if gated else 0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(F),
                ctypes.c_int(K), ctypes.c_int(per_block), ctypes.c_int(act_kind), ctypes.c_float(limit), _ptr(weights if weight_input else None), _Hip.stream())
     y = torch.empty((max_tiles * tm, K), dtype=torch.float32, device=dev)
-    hip().call("spy_moe_gemm", _ptr(y), F32, _ptr(act), _code(act, "act"), _ptr(w_down), _code(w_down, "expert matrices"), tile_experts,
+    hip().call("spy_moe_gemm", _ptr(y), F32, _ptr(act), _code(act, "act"), _ptr(down), _code(down, "expert matrices"), ctypes.c_int(down_tiled), tile_experts,
                sorted_pairs, group_list, ctypes.c_int(P), ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(K), ctypes.c_int(F),
                ctypes.c_int(per_block), ctypes.c_int(0), ctypes.c_float(0.0), _ptr(None), _Hip.stream())
     result = ExpertRows(y, pair_row, None if weight_input else weights, add, top, scale, T, x.dtype)

@@ -106,17 +106,17 @@ class DenseMLP(FeedForward):
 
 def stacked_experts(weights, experts: int, gate: str, up: str, down: str):
     """Takes the experts' matrices out of ``weights`` (names with a place for the expert's number): every expert's [gate rows |
-    up rows] (``gate`` None: up rows alone) and its down matrix, the experts one after the other."""
+    up rows] (``gate`` None: up rows alone) and its down matrix, the experts one after the other, in the form the kernels read
+    (``ops.expert_forms``)."""
     if gate is None:
         mats = [weights.pop(n % e) for e in range(experts) for n in (up, down)]
         if len({m.dtype for m in mats}) > 1:
             mats = [m.float() for m in mats]
-        return torch.stack(mats[0::2]).contiguous(), torch.stack(mats[1::2]).contiguous()
+        return ops.expert_forms([[m] for m in mats[0::2]]), ops.expert_forms([[m] for m in mats[1::2]])
     mats = [weights.pop(n % e) for e in range(experts) for n in (gate, up, down)]
     if len({m.dtype for m in mats}) > 1:
         mats = [m.float() for m in mats]
-    return (torch.stack([torch.cat([mats[3 * e], mats[3 * e + 1]], dim=0) for e in range(experts)]).contiguous(),
-            torch.stack([mats[3 * e + 2] for e in range(experts)]).contiguous())
+    return (ops.expert_forms([mats[3 * e:3 * e + 2] for e in range(experts)]), ops.expert_forms([[m] for m in mats[2::3]]))
 
 
 class MoEMLP(FeedForward):

@@ -75,3 +75,26 @@ def test_groups_of_an_alignment():
             assert all(te[gr[1 + 2 * j] >> 4] == te[tile] for j in range(first, first + in_band))
             seen += list(range(tile, tile + tiles))
         assert seen == [t for t, e in enumerate(te) if e >= 0]
+
+
+@pytest.mark.parametrize("by_groups", [True, False])
+@pytest.mark.parametrize("form", ["silu", "weighted", "gelu"])
+@pytest.mark.parametrize("kind,E,top,K,F", [("even", 6, 2, 128, 128), ("one", 5, 2, 384, 128), ("edges", 9, 3, 256, 640), ("few", 16, 4, 128, 384), ("one", 40, 3, 640, 1024)])
+def test_experts_in_operand_order(kind, E, top, K, F, form, by_groups, monkeypatch):
+    """Matrices in operand order: one turn of 128 of K, an odd number of them, groups in halves and whole, against the rows' kernels."""
+    from spyinfer_amd.kernels import ops
+    monkeypatch.setattr(ops, "experts_by_groups", lambda *sizes: by_groups)
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(E + K)
+    ids = rows_for(kind, E, top, g)
+    T, gated = ids.shape[0], form != "gelu"
+    bf = lambda *s, std=1.0: (torch.randn(s, generator=g) * std).bfloat16().to(dev)
+    x, wgu, wd, w = bf(T, K), bf(E, (2 if gated else 1) * F, K, std=K ** -0.5), bf(E, K, F, std=F ** -0.5), torch.rand((T, top), generator=g).to(dev)
+    kw = dict(silu={}, weighted=dict(activation="clamped", limit=0.8, weight_input=True), gelu=dict(activation="gelu"))[form]
+    tiled = [ops.expert_forms([m.tensor_split(2) if gated and mats is wgu else [m] for m in mats]) for mats in (wgu, wd)]
+    assert all(isinstance(m, ops.TiledExperts) for m in tiled) and torch.equal(tiled[0].rows(), wgu)
+    out = ops.moe_experts(x, ids.to(dev), w, *tiled, **kw)
+    ref = ops.moe_experts(x.float(), ids.to(dev), w, wgu.float(), wd.float(), **kw)          # (float32 kernels, no rounding in between)
+    close(out, ref, torch.bfloat16, scale=2.0, what="experts in operand order")
+    if kind == "even":
+        close(ops.moe_experts(x.float(), ids.to(dev), w, *tiled, **kw), ref, torch.float32, what="float32 rows of the same matrices")
