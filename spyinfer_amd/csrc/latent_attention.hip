@@ -427,29 +427,188 @@ __global__ __launch_bounds__(NW * 64) void latent_attention_mfma_kernel(
         }
         return;
     }
-    // parts: ws[(global row * splits + part)] = { O[R] unnormalised, m, l }
-    float* w = ws + (((size_t)q0 * H + row) * splits + sp) * (R + 2);
+    // parts: ws[(global row * splits + part)] = { O[R] unnormalised, m, l, two unused }
+    float* w = ws + (((size_t)q0 * H + row) * splits + sp) * (R + 4);
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
         const int v0 = 16 * i + 4 * g;
-        if (i < r_tiles && v0 < R) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) w[v0 + j] = acc[i][j];
-        }
+        if (i < r_tiles && v0 < R) *reinterpret_cast<lf32x4_t*>(w + v0) = acc[i];
     }
     if (g == 0) { w[R] = m; w[R + 1] = l; }
 }
 
+// The same for steps of single tokens, by tiles of 16 rows (heads of one token): the four waves of a block share its one tile, where
+// the kernel above has a wave for each 16 rows and three of four had no products to do.  A wave takes every fourth step of D of the
+// scores, which meet in LDS, and a quarter of the values' tiles; every wave forms the same softmax.  No list of tiles is read: entry e is
+// token e.  What bounds it is the chain of round trips (position, page, row, the scores' sum, the part's way out), which a part walks
+// once for every 32 keys, so parts are one chunk long where the chip has room (ops.latent_few_key_parts).
+// Measured, 16 heads of 512 + 64 values, tiles of 64 rows / this kernel, both with the merge of the parts: 5 tokens of 100 keys 19.3 / 11.2
+// us, of 500 19.4 / 11.8, of 1500 25.1 / 15.7; 64 tokens of 500 40.4 / 21.7; one of 4000 47.5 / 19.0.
+template <int QS, int RT, typename TW>
+__global__ __launch_bounds__(256) void latent_attention_few_kernel(
+    bf16_t* __restrict__ out, float* __restrict__ ws, const bf16_t* __restrict__ qa, const bf16_t* __restrict__ cache, int P, int num_pages,
+    const int* __restrict__ pos0, const int* __restrict__ kv_len, const int* __restrict__ block_table, int max_blocks,
+    const TW* __restrict__ sink, int H, int R, int D, float scale, int window) {
+    constexpr int QW = (QS + 3) / 4, RW = (RT + 3) / 4;             // a wave's steps of D and tiles of R
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r16 = lane & 15, g = lane >> 4;
+    const int tiles_per_token = (H + 15) / 16, sp = blockIdx.y, splits = gridDim.y;
+    const int e = blockIdx.x / tiles_per_token, head = (blockIdx.x % tiles_per_token) * 16 + r16;
+    const int p = pos0[e], kvl = kv_len[e];
+    const bool row_ok = head < H;
+    const int lo = window > 0 ? max(0, p - window + 1) : 0, hi = min(p, kvl - 1);
+    const int c_start = lo & ~31, n_chunks = (hi - c_start) / 32 + 1;
+    const int c_begin = (int)((long long)n_chunks * sp / splits), c_end = (int)((long long)n_chunks * (sp + 1) / splits);
+    const int q_steps = (D + 31) / 32, r_tiles = (R + 15) / 16;
+    const int Dp = q_steps * 32, krow = Dp + LKPAD;
+    bf16_t* Ks = reinterpret_cast<bf16_t*>(lds_raw);                 // keys [32][krow], values [r_tiles 16][LVROW], scores [4][64][8]
+    bf16_t* Vs = Ks + 32 * krow;
+    float* part_scores = reinterpret_cast<float*>(Vs + r_tiles * 16 * LVROW);
+    // staging as above: one key of the chunk and every eighth 16-byte piece of its row
+    constexpr int NP = (QS * 4 + 7) / 8;
+    const int* bt = block_table + (size_t)e * max_blocks;
+    const int sk = tid & 31, sd0 = (tid >> 5) * 8;
+    lu32x4_t pf[NP];
+    // the page of a thread's key is looked up a chunk before its row is asked for
+    auto page_of = [&](int c) {
+        const int key = c_start + 32 * c + sk;
+        return c < c_end && key >= lo && key <= hi ? bt[key / P] : -1;
+    };
+    auto fetch = [&](int c, int page) {
+        const bf16_t* src = page >= 0 && page < num_pages ? cache + ((size_t)page * P + (c_start + 32 * c + sk) % P) * D : nullptr;
+#pragma unroll
+        for (int it = 0; it < NP; ++it) {
+            const int d8 = sd0 + 64 * it;
+            pf[it] = lu32x4_t{0u, 0u, 0u, 0u};
+            if (src && d8 < D) pf[it] = *reinterpret_cast<const lu32x4_t*>(src + d8);
+        }
+    };
+    const int first_page = page_of(c_begin);
+    int next_page = page_of(c_begin + 1);
+    fetch(c_begin, first_page);
+    lbf16x8_t bq[QW];
+#pragma unroll
+    for (int i = 0; i < QW; ++i) {
+        const int d0 = 32 * (wave + 4 * i) + 8 * g;
+        lu32x4_t packed = {0u, 0u, 0u, 0u};
+        if (row_ok && d0 < D) packed = *reinterpret_cast<const lu32x4_t*>(qa + ((size_t)e * H + head) * D + d0);
+        bq[i] = __builtin_bit_cast(lbf16x8_t, packed);
+    }
+    const bool with_sink = sink != nullptr && sp == 0;
+    float m = with_sink && row_ok ? to_f32<TW>(sink[head]) : -INFINITY;
+    float l = with_sink && row_ok && g == 0 ? 1.f : 0.f;          // a row's sum is spread over its four lanes
+    lf32x4_t acc[RW];
+#pragma unroll
+    for (int i = 0; i < RW; ++i) acc[i] = lf32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int ka_row = 8 * (r16 >> 2) + (r16 & 3);                  // tile a's key of this lane's operand row; tile b: + 4
+    for (int c = c_begin; c < c_end; ++c) {
+        if (c > c_begin) __syncthreads();                           // the chunk before is read by all
+#pragma unroll
+        for (int it = 0; it < NP; ++it) {
+            const int d8 = sd0 + 64 * it;
+            if (d8 < Dp) {
+                *reinterpret_cast<lu32x4_t*>(Ks + sk * krow + d8) = pf[it];
+                if (d8 < r_tiles * 16) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        Vs[(d8 + 2 * j) * LVROW + sk] = (bf16_t)(pf[it][j] & 0xffffu);
+                        Vs[(d8 + 2 * j + 1) * LVROW + sk] = (bf16_t)(pf[it][j] >> 16);
+                    }
+                }
+            }
+        }
+        fetch(c + 1, next_page);
+        next_page = page_of(c + 2);
+        __syncthreads();
+        lf32x4_t sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < QW; ++i) {
+            const int s = wave + 4 * i;
+            if (s < q_steps) {
+                const lbf16x8_t ka = *reinterpret_cast<const lbf16x8_t*>(Ks + ka_row * krow + 32 * s + 8 * g);
+                const lbf16x8_t kb = *reinterpret_cast<const lbf16x8_t*>(Ks + (ka_row + 4) * krow + 32 * s + 8 * g);
+                sa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, bq[i], sa, 0, 0, 0);
+                sb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb, bq[i], sb, 0, 0, 0);
+            }
+        }
+        *reinterpret_cast<lf32x4_t*>(part_scores + (wave * 64 + lane) * 8) = sa;
+        *reinterpret_cast<lf32x4_t*>(part_scores + (wave * 64 + lane) * 8 + 4) = sb;
+        __syncthreads();
+        sa = *reinterpret_cast<const lf32x4_t*>(part_scores + lane * 8);
+        sb = *reinterpret_cast<const lf32x4_t*>(part_scores + lane * 8 + 4);
+#pragma unroll
+        for (int i = 1; i < 4; ++i) {
+            sa += *reinterpret_cast<const lf32x4_t*>(part_scores + (i * 64 + lane) * 8);
+            sb += *reinterpret_cast<const lf32x4_t*>(part_scores + (i * 64 + lane) * 8 + 4);
+        }
+        // ---- softmax over this lane's 8 keys of its row ----
+        float sc[8];
+        float bmax = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int key = c_start + 32 * c + 8 * g + j;
+            const float v = (j < 4 ? sa[j] : sb[j - 4]) * scale;
+            const bool ok = row_ok && key <= p && key >= lo && key < kvl;
+            sc[j] = ok ? v : -INFINITY;
+            bmax = fmaxf(bmax, sc[j]);
+        }
+        bmax = fmaxf(bmax, __shfl_xor(bmax, 16, 64));
+        bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
+        const float m_new = fmaxf(m, bmax);
+        float alpha = 1.f;
+        lbf16x8_t pb = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (m_new != -INFINITY) {
+            alpha = (m == -INFINITY) ? 0.f : __expf(m - m_new);
+            float psum = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float pj = (sc[j] == -INFINITY) ? 0.f : __expf(sc[j] - m_new);
+                psum += pj;
+                pb[j] = (short)f32_to_bf16(pj);
+            }
+            l = l * alpha + psum;
+            m = m_new;
+        }
+#pragma unroll
+        for (int i = 0; i < RW; ++i) {
+            const int tile = wave * RW + i;
+            if (tile < r_tiles) {
+                const lbf16x8_t vt = *reinterpret_cast<const lbf16x8_t*>(Vs + (16 * tile + r16) * LVROW + 8 * g);
+                acc[i] *= alpha;
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt, pb, acc[i], 0, 0, 0);
+            }
+        }
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (!row_ok) return;
+    const size_t row = (size_t)e * H + head;
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    float* w = ws + (row * splits + sp) * (R + 4);
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+        const int v0 = 16 * (wave * RW + i) + 4 * g;
+        if (v0 >= R) continue;
+        if (splits == 1) {
+            const uint2 o = {pack_bf16x2(acc[i][0] * inv, acc[i][1] * inv), pack_bf16x2(acc[i][2] * inv, acc[i][3] * inv)};
+            *reinterpret_cast<uint2*>(out + row * R + v0) = o;
+        } else {
+            *reinterpret_cast<lf32x4_t*>(w + v0) = acc[i];
+        }
+    }
+    if (splits > 1 && wave == 0 && g == 0) { w[R] = m; w[R + 1] = l; }
+}
+
 // out[row] = sum_i O_i e^(m_i - M) / sum_i l_i e^(m_i - M) over the parts i of a row, added in ascending i
-__global__ __launch_bounds__(256) void latent_attention_merge_kernel(bf16_t* __restrict__ out, const float* __restrict__ ws, int R, int splits) {
+__global__ __launch_bounds__(128) void latent_attention_merge_kernel(bf16_t* __restrict__ out, const float* __restrict__ ws, int R, int splits) {
     __shared__ float wgt[64];
     __shared__ float inv_l;
     const size_t row = blockIdx.x;
-    const float* base = ws + row * splits * (R + 2);
+    const float* base = ws + row * splits * (R + 4);
     if (threadIdx.x < 64) {                        // the parts' maxima and sums, one lane each (at most 64 parts)
         const int i = threadIdx.x;
-        const float mi = i < splits ? base[(size_t)i * (R + 2) + R] : -INFINITY;
-        const float li = i < splits ? base[(size_t)i * (R + 2) + R + 1] : 0.f;
+        const float mi = i < splits ? base[(size_t)i * (R + 4) + R] : -INFINITY;
+        const float li = i < splits ? base[(size_t)i * (R + 4) + R + 1] : 0.f;
         const float M = wave_max(mi);
         const float e = (mi == -INFINITY) ? 0.f : __expf(mi - M);
         wgt[i] = e;
@@ -457,19 +616,25 @@ __global__ __launch_bounds__(256) void latent_attention_merge_kernel(bf16_t* __r
         if (i == 0) inv_l = L > 0.f ? 1.0f / L : 0.f;
     }
     __syncthreads();
-    for (int j = threadIdx.x; j < R; j += blockDim.x) {
-        float o = 0.f;
+    const int j = threadIdx.x * 4;                 // (R is a multiple of 8, and a thread has one piece of it)
+    if (j >= R) return;
+    float o[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
-        for (int i = 0; i < splits; ++i) o = fmaf(base[(size_t)i * (R + 2) + j], wgt[i], o);      // (unrolled: the parts' loads go out together)
-        out[row * R + j] = f32_to_bf16(o * inv_l);
+    for (int i = 0; i < splits; ++i) {             // (unrolled: the parts' loads go out together)
+        const float4 v = *reinterpret_cast<const float4*>(base + (size_t)i * (R + 4) + j);
+        const float e = wgt[i];
+        o[0] = fmaf(v.x, e, o[0]); o[1] = fmaf(v.y, e, o[1]); o[2] = fmaf(v.z, e, o[2]); o[3] = fmaf(v.w, e, o[3]);
     }
+    const uint2 y = {pack_bf16x2(o[0] * inv_l, o[1] * inv_l), pack_bf16x2(o[2] * inv_l, o[3] * inv_l)};
+    *reinterpret_cast<uint2*>(out + row * R + j) = y;
 }
 
 extern "C" long long spy_latent_attention_mfma_workspace(int T, int H, int R, int splits) {
-    return splits > 1 ? (long long)T * H * splits * (R + 2) : 0;
+    return splits > 1 ? (long long)T * H * splits * (R + 4) : 0;
 }
 
-// tiles: num_tiles records (entry, first row) of tile_rows (64 or 128) rows each: a block of 4 or 8 waves.  ws: float32, spy_latent_attention_mfma_workspace values.
+// tiles: num_tiles records (entry, first row) of tile_rows (64 or 128) rows each: a block of 4 or 8 waves; tile_rows 16: a step of single
+// tokens (entry e is token e), no records.  ws: float32, spy_latent_attention_mfma_workspace values.
 extern "C" int spy_latent_attention_mfma(void* out, float* ws, const void* qa, const void* cache, int P, int num_pages,
                                          const int* cu_q, const int* pos0, const int* kv_len, const int* block_table,
                                          int max_blocks, const int* tile_entry, const int* tile_row0, int num_tiles,
@@ -479,32 +644,45 @@ extern "C" int spy_latent_attention_mfma(void* out, float* ws, const void* qa, c
     SPY_REQUIRE(T > 0 && H > 0 && R > 0 && DR >= 0 && P > 0 && num_pages > 0 && max_blocks > 0 && num_tiles > 0,
                 "spy_latent_attention_mfma: empty operand");
     SPY_REQUIRE(D % 8 == 0 && R % 8 == 0 && D <= 576 && R <= 512, "spy_latent_attention_mfma: rows of %d + %d values are not taken", R, DR);
-    SPY_REQUIRE(tile_rows == 64 || tile_rows == 128, "spy_latent_attention_mfma: tiles of %d rows (64 or 128)", tile_rows);
+    SPY_REQUIRE(tile_rows == 64 || tile_rows == 128 || tile_rows == 16, "spy_latent_attention_mfma: tiles of %d rows (16, 64 or 128)", tile_rows);
+    SPY_REQUIRE(tile_rows != 16 || num_tiles == (long long)T * ((H + 15) / 16), "spy_latent_attention_mfma: %d tiles of 16 rows for %d tokens", num_tiles, T);
+    SPY_REQUIRE(((uintptr_t)ws % 16) == 0, "spy_latent_attention_mfma: the workspace is not aligned");
     SPY_REQUIRE(splits >= 1 && splits <= 64 && (splits == 1 || ws), "spy_latent_attention_mfma: %d parts (1..64, with a workspace)", splits);
     SPY_REQUIRE(((uintptr_t)qa % 16) == 0 && ((uintptr_t)cache % 16) == 0 && ((uintptr_t)out % 8) == 0, "spy_latent_attention_mfma: operands are not aligned");
     const int q_steps = (D + 31) / 32, r_tiles = (R + 15) / 16;
-    const size_t lds = 2 * ((size_t)32 * (q_steps * 32 + LKPAD) + (size_t)r_tiles * 16 * LVROW) * sizeof(bf16_t);
+    const size_t chunk = ((size_t)32 * (q_steps * 32 + LKPAD) + (size_t)r_tiles * 16 * LVROW) * sizeof(bf16_t);
+    const size_t lds = tile_rows == 16 ? chunk + 4 * 64 * 8 * sizeof(float) : 2 * chunk;
     SPY_REQUIRE(lds <= 160 * 1024, "spy_latent_attention_mfma: two staged chunks of %d + %d values take %zu bytes of LDS", R, DR, lds);
     const dim3 grid(num_tiles, splits);
-#define SPY_LA_LAUNCH_W(QS, RT, NW)                                                                                             \
-    SPY_DISPATCH(sink_dtype, TW, {                                                                                              \
-        auto kernel = latent_attention_mfma_kernel<QS, RT, NW, TW>;                                                             \
+#define SPY_LA_KERNEL(...)                                                                                                      \
+        auto kernel = __VA_ARGS__;                                                                                              \
         if (lds > 48 * 1024) {                                                                                                  \
             hipError_t e_ = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);      \
             if (e_ != hipSuccess) return spy_fail("spy_latent_attention_mfma: %zu bytes of LDS refused: %s", lds, hipGetErrorString(e_)); \
-        }                                                                                                                       \
+        }
+#define SPY_LA_LAUNCH_F(QS, RT)                                                                                                 \
+    SPY_DISPATCH(sink_dtype, TW, {                                                                                              \
+        SPY_LA_KERNEL(latent_attention_few_kernel<QS, RT, TW>)                                                                  \
+        kernel<<<grid, 256, lds, st>>>((bf16_t*)out, ws, (const bf16_t*)qa, (const bf16_t*)cache, P, num_pages, pos0, kv_len,  \
+                                       block_table, max_blocks, (const TW*)sink, H, R, D, scale, window);                      \
+    })
+#define SPY_LA_LAUNCH_W(QS, RT, NW)                                                                                             \
+    SPY_DISPATCH(sink_dtype, TW, {                                                                                              \
+        SPY_LA_KERNEL(latent_attention_mfma_kernel<QS, RT, NW, TW>)                                                             \
         kernel<<<grid, NW * 64, lds, st>>>((bf16_t*)out, ws, (const bf16_t*)qa, (const bf16_t*)cache, P, num_pages, cu_q, pos0, kv_len, \
                                            block_table, max_blocks, tile_entry, tile_row0, (const TW*)sink, H, R, D, scale, window); \
     })
-#define SPY_LA_LAUNCH(QS, RT) if (tile_rows == 128) { SPY_LA_LAUNCH_W(QS, RT, 8); } else { SPY_LA_LAUNCH_W(QS, RT, 4); }
+#define SPY_LA_LAUNCH(QS, RT) if (tile_rows == 16) { SPY_LA_LAUNCH_F(QS, RT); } else if (tile_rows == 128) { SPY_LA_LAUNCH_W(QS, RT, 8); } else { SPY_LA_LAUNCH_W(QS, RT, 4); }
     if (q_steps <= 8 && r_tiles <= 8) { SPY_LA_LAUNCH(8, 8); }
     else if (q_steps <= 12 && r_tiles <= 16) { SPY_LA_LAUNCH(12, 16); }
     else { SPY_LA_LAUNCH(18, 32); }
 #undef SPY_LA_LAUNCH_W
+#undef SPY_LA_LAUNCH_F
+#undef SPY_LA_KERNEL
 #undef SPY_LA_LAUNCH
     SPY_CHECK_LAUNCH("spy_latent_attention_mfma");
     if (splits > 1) {
-        latent_attention_merge_kernel<<<(unsigned)((size_t)T * H), R > 128 ? 256 : 64, 0, st>>>((bf16_t*)out, ws, R, splits);
+        latent_attention_merge_kernel<<<(unsigned)((size_t)T * H), R > 256 ? 128 : 64, 0, st>>>((bf16_t*)out, ws, R, splits);
         SPY_CHECK_LAUNCH("spy_latent_attention_mfma (merge)");
     }
     return 0;

@@ -1525,10 +1525,25 @@ def latent_attention_mfma_ok(dtype, R: int, D: int) -> bool:
     return LATENT_MFMA and dtype == torch.bfloat16 and D % 8 == 0 and R % 8 == 0 and D <= 576 and R <= 512
 
 
+def latent_few_tiles(tokens: int, heads: int, max_keys: int) -> int:
+    """Tiles of 16 (token, head) rows of a step of single tokens whose blocks share them among their waves
+    (latent_attention_few_kernel), or 0 where tiles of 64 rows are the better ones: many heads, whose tiles read the same keys each for
+    itself, with many keys (128 heads, tiles of 64 rows / 16 rows: 12 tokens of 100 keys 25 / 16, of 500 33 / 35 us, of 1500 63 / 70; 5
+    tokens of 500 28 / 25), and steps that fill the chip either way (32 heads: 128 tokens of 1500 keys 144 / 140)."""
+    tiles = tokens * -(-heads // 16)
+    return tiles if (tiles <= 256 if heads <= 32 else tiles * -(-max_keys // 32) <= 640) else 0
+
+
 def latent_key_parts(num_tiles: int, max_keys: int) -> int:
     """Parts into which the MFMA latent attention cuts every tile's keys so that a step of few tiles (single tokens)
     still has blocks for the whole device; a part wants 64 keys at least."""
     return max(1, min(512 // max(1, num_tiles), 16, -(-max_keys // 64)))
+
+
+def latent_few_key_parts(num_tiles: int, max_keys: int) -> int:
+    """The same for ``latent_few_tiles``: chunks of 32 keys one after the other cost 2.6 us each, a second block on a compute unit as much
+    (32 tiles, 500 keys: 17.7 us in 8 parts, 22.4 in 16; one tile: 19.1 / 13.2 / 11.0 in 4 / 8 / 16)."""
+    return max(1, min(256 // max(1, num_tiles), 32, -(-max_keys // 32)))
 
 
 def latent_attention(qa: torch.Tensor, cache: torch.Tensor, page_size: int, meta: "AttentionMeta", sink: Optional[torch.Tensor],
@@ -1548,11 +1563,14 @@ def latent_attention(qa: torch.Tensor, cache: torch.Tensor, page_size: int, meta
     _check(meta.block_table.shape == (meta.S, meta.max_blocks), "latent_attention: block table must be [S, max_blocks]")
     out = torch.empty((T, H, R), dtype=out_dtype, device=qa.device)
     if T and mfma:
-        # tiles: (entry [n], first row [n], n, rows of a tile) planned on the host
+        # tiles: (entry [n], first row [n], n, rows of a tile) planned on the host; of 16 rows: (None, None, n, 16)
         tile_entry, tile_row0, n = tiles[:3]
         tile_rows = tiles[3] if len(tiles) > 3 else LATENT_TILE_ROWS
         _dev(tile_entry, tile_row0, meta.cu_q, meta.pos0)
-        _check(n > 0 and tile_entry.shape == (n,) and tile_row0.shape == (n,), "latent_attention: the tiles' arrays do not fit their number")
+        if tile_rows == 16:
+            _check(meta.S == T and meta.max_q_len == 1 and n == T * -(-H // 16), "latent_attention: tiles of 16 rows are for steps of single tokens")
+        else:
+            _check(n > 0 and tile_entry.shape == (n,) and tile_row0.shape == (n,), "latent_attention: the tiles' arrays do not fit their number")
         ws = None
         if key_parts > 1:
             ws = torch.empty((hip().lib.spy_latent_attention_mfma_workspace(ctypes.c_int(T), ctypes.c_int(H), ctypes.c_int(R),

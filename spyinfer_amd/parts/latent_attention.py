@@ -120,6 +120,15 @@ class LatentAttention(Mixer):
         if not ops.latent_attention_mfma_ok(batch.act_dtype, self.kv_rank, self.kv_rank + self.rot_dim):
             return
         note = ("latent_tiles", self.heads)
+        keys = batch.max_kv_len if self.window is None else min(batch.max_kv_len, self.window + batch.max_q_len - 1)
+        few = ops.latent_few_tiles(batch.T, self.heads, keys) if batch.max_q_len == 1 and batch.S == batch.T else 0
+        parts_note = ("latent_parts", self.heads, self.window)
+        if few:
+            # (tile and token follow from the block's number: no arrays)
+            parts = ops.latent_few_key_parts(few, keys)
+            batch.shared[parts_note] = (parts, few)
+            batch.add_graph_key("latent_parts_%d_%s" % (self.heads, self.window), -parts)
+            return
         if note not in batch.shared:
             rows = batch.lens.astype(np.int64) * self.heads
             size = ops.latent_tile_rows(int(rows.sum()))
@@ -132,9 +141,8 @@ class LatentAttention(Mixer):
             batch.add_array("latent_tile_row0_%d" % self.heads, row0)
             batch.shared[note] = int(first[-1])
             batch.shared[("latent_tile_rows", self.heads)] = size
-        keys = batch.max_kv_len if self.window is None else min(batch.max_kv_len, self.window + batch.max_q_len - 1)
         parts = ops.latent_key_parts(batch.shared[note], keys)
-        batch.shared[("latent_parts", self.heads, self.window)] = parts
+        batch.shared[parts_note] = (parts, 0)
         batch.add_graph_key("latent_parts_%d_%s" % (self.heads, self.window), parts)
 
     def plan_arrays(self, entries):
@@ -187,9 +195,10 @@ class LatentAttention(Mixer):
         meta = attention_meta(batch, cache.group, nh)
         tiles, parts = None, 1
         if mfma:
-            tiles = (batch.array("latent_tile_entry_%d" % nh), batch.array("latent_tile_row0_%d" % nh), batch.shared[("latent_tiles", nh)],
-                     batch.shared[("latent_tile_rows", nh)])
-            parts = batch.shared[("latent_parts", nh, self.window)]
+            parts, few = batch.shared[("latent_parts", nh, self.window)]
+            tiles = (None, None, few, 16) if few else \
+                (batch.array("latent_tile_entry_%d" % nh), batch.array("latent_tile_row0_%d" % nh), batch.shared[("latent_tiles", nh)],
+                 batch.shared[("latent_tile_rows", nh)])
         lat = ops.latent_attention(qa, cache.rows, cache.page_size, meta, self.sink, r, self.scale, self.window, x.dtype, tiles, parts)
         # the summed latents through the values' expansion: v[t, h, e] = sum_j lat[t, h, j] Wuv[h dv + e, j]
         if library and self.w_uv.dtype == torch.bfloat16:

@@ -178,6 +178,39 @@ def test_latent_attention_on_mfma_equals_the_plain_kernel(case):
     close(got, ref, torch.bfloat16, what="latent attention on MFMA")
 
 
+@pytest.mark.parametrize("H,R,DR,P,window,parts,kv", [(16, 512, 64, 16, None, 16, [500, 33, 1, 32, 64]), (8, 128, 64, 4, 40, 3, [200, 41, 7]), (20, 80, 16, 16, None, 1, [65, 31]),
+                                                      (3, 256, 32, 16, 100, 5, [333]), (40, 512, 64, 64, 1000, 7, [1500, 900, 17])])
+def test_latent_attention_of_single_tokens_by_shared_tiles(H, R, DR, P, window, parts, kv):
+    """Tiles of 16 rows whose four waves share them: last chunks of one key and of 32, more parts than chunks, windows, heads that are no
+    multiple of 16, one and several steps of D a wave; against the plain kernel."""
+    import numpy as np
+
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(H + R)
+    S, D, width = len(kv), R + DR, max(-(-k // P) for k in kv)
+    pages = sum(-(-k // P) for k in kv) + 3
+    perm = torch.randperm(pages, generator=g).tolist()
+    table = np.full((S, width), -1, dtype=np.int32)
+    for s, k in enumerate(kv):
+        for b in range(0 if window is None else max(0, k - window) // P, -(-k // P)):
+            table[s, b] = perm.pop()
+    cache = torch.full((pages, P, D), float("nan"))
+    for s, k in enumerate(kv):
+        for b in table[s]:
+            if b >= 0:
+                cache[b] = torch.randn((P, D), generator=g)
+    cache = cache.to(torch.bfloat16).to(dev)
+    qa = (3.0 * torch.randn((S, H, D), generator=g) / D ** 0.5).to(dev)
+    sink = torch.randn((H,), generator=g).to(torch.bfloat16).to(dev)
+    pos = [k - 1 for k in kv]
+    meta = ops.AttentionMeta(i32(np.arange(S + 1), dev), i32(pos, dev), i32(kv, dev), torch.tensor(table, device=dev), i32(np.arange(S), dev), i32(pos, dev),
+                             S, S, width, max(kv), 1)
+    ref = ops.latent_attention(qa, cache, P, meta, sink, R, 0.7, window, torch.float32)
+    got = ops.latent_attention(qa.to(torch.bfloat16), cache, P, meta, sink, R, 0.7, window, torch.bfloat16, (None, None, S * -(-H // 16), 16), parts)
+    close(got, ref, torch.bfloat16, what="latent attention by shared tiles")
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("dims,scaling", [(8, None), (6, dict(factor=8.0, original=64, fast=16.0, slow=2.0)), (0, None)])
 def test_latent_prepare_norms_rotates_and_stores(dtype, dims, scaling):
