@@ -198,12 +198,14 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_narrow_kernel(const fl
 #define GF_LD 36
 template <int KS>
 __global__ __launch_bounds__(256 * KS) void gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
-                                                                 int M, int N, int K, int tiles_m, int tiles_n) {
+                                                                 int M, int N, int K, int tiles_m, int tiles_n, int parts) {
     __shared__ float lds[KS][2][128 * GF_LD];         // per part of K two stages: 64 rows of A, then 64 of W
     // blocks go to the eight dies in turn: die x takes a run of neighbouring tiles, rows fastest, so that a piece of W is read into one L2
-    const int total = tiles_m * tiles_n, per = (total + 7) >> 3;
-    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if (tile >= total) return;
+    const int tiles = tiles_m * tiles_n, total = tiles * parts, per = (total + 7) >> 3;
+    const int at = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || at >= total) return;
+    const int tile = at % tiles, k_part = at / tiles;
+    C += (size_t)k_part * M * N;
     const int m0 = (tile % tiles_m) * 64, n0 = (tile / tiles_m) * 64;
     const int part = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, tid = threadIdx.x & 255;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = threadIdx.x & 63;
@@ -219,8 +221,10 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_tile_kernel(const float* __
         wp[p] = W + (size_t)min(n0 + sr + 32 * p, N - 1) * K;
     }
     // this part's steps of K: `steps` for every part (the barriers are the block's), those from its end on staged as zeros
-    const int all = (K + GF_BK - 1) / GF_BK, steps = (all + KS - 1) / KS;
-    const int k_first = part * steps * GF_BK, k_end = min(K, k_first + steps * GF_BK);
+    const int all_steps = (K + GF_BK - 1) / GF_BK, step0 = (int)((long long)all_steps * k_part / parts);
+    const int all = (int)((long long)all_steps * (k_part + 1) / parts) - step0, steps = (all + KS - 1) / KS;
+    const int k_last = min(K, (step0 + all) * GF_BK);
+    const int k_first = (step0 + part * steps) * GF_BK, k_end = min(k_last, k_first + steps * GF_BK);
     const gf_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
     auto fetch = [&](gf_f32x4_t (&va)[2], gf_f32x4_t (&vw)[2], int s) {
         const int k = min(k_first + s * GF_BK + sk, K - 4);
@@ -288,10 +292,10 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_tile_kernel(const float* __
     if (KS > 1) {
         // the other parts' sums through LDS (their own stages) to the first part's waves, added in the order of the parts
         __syncthreads();
-        float* at = lds[part][0] + wave * 1024 + 4 * lane;
+        float* mine = lds[part][0] + wave * 1024 + 4 * lane;
         if (part > 0) {
 #pragma unroll
-            for (int e = 0; e < 16; e += 4) *reinterpret_cast<float4*>(at + e * 64) = make_float4(sum[e], sum[e + 1], sum[e + 2], sum[e + 3]);
+            for (int e = 0; e < 16; e += 4) *reinterpret_cast<float4*>(mine + e * 64) = make_float4(sum[e], sum[e + 1], sum[e + 2], sum[e + 3]);
         }
         __syncthreads();
         if (part > 0) return;
@@ -330,7 +334,7 @@ bool gemm_f32_takes(const void* A, const void* W, const void* C, int M, int N, i
 int gemm_f32(const float* A, const float* W, float* C, int M, int N, int K, hipStream_t st) {
 #define GF_FEW(MR, NR, U) gemm_f32_few_kernel<MR, NR, U><<<(N + 4 * NR - 1) / (4 * NR), 256, 0, st>>>(A, W, C, M, N, K)
 #define GF_NARROW(MT) gemm_f32_narrow_kernel<MT><<<dim3(tiles16, (M + 16 * MT - 1) / (16 * MT)), GF_WAVES * 64, 0, st>>>(A, W, C, M, N, K)
-#define GF_TILE(KS) gemm_f32_tile_kernel<KS><<<((tm * tn + 7) / 8) * 8, 256 * KS, 0, st>>>(A, W, C, M, N, K, tm, tn)
+#define GF_TILE(KS) gemm_f32_tile_kernel<KS><<<((tm * tn + 7) / 8) * 8, 256 * KS, 0, st>>>(A, W, C, M, N, K, tm, tn, 1)
     const int tiles16 = (N + 15) / 16, tm = (M + 63) / 64, tn = (N + 63) / 64;
     if (M <= 4 || (M <= 8 && N <= 1024)) {
         // Rows of W per wave: each more reads A once less, but takes waves away.  One up to 2048 rows of W (four rows of A, 2048 x
@@ -359,5 +363,21 @@ int gemm_f32(const float* A, const float* W, float* C, int M, int N, int K, hipS
         else GF_TILE(1);
     }
     SPY_CHECK_LAUNCH("spy_gemm (float32)");
+    return 0;
+}
+
+// A [M, K] . W [N, K]^T in parts of K: C [parts][M][N], a block a tile of one part, which the reader sums (spy_add_parts_rmsnorm).  For
+// results whose tiles fill no whole number of rounds of the chip (or of which there are too few even for that: the narrow kernel above
+// reads half lines of W).  Parts beat groups of a block's waves, which leave the other compute units idle.  Measured, us, the
+// kernels above / this one and what the sum adds to the norm's pass: 611 rows, 1024 x 2048 43.4 / 33.8 + 2; 1024 x 3072 62.6 / 44.6 + 5; 2048
+// x 6144 223 / 145 + 5; 65 rows, 2048 x 6144 62 / 35 + 2; 17 rows, 2560 x 4096 29 / 18.5 + 1.
+extern "C" int spy_gemm_f32_parts(float* C, const float* A, const float* W, int M, int N, int K, int parts, hipStream_t st) {
+    SPY_REQUIRE(M > 0 && N > 0 && K > 0 && parts >= 1 && parts <= (K + GF_BK - 1) / GF_BK, "spy_gemm_f32_parts: %d parts of %d x %d x %d", parts, M, N, K);
+    SPY_REQUIRE(gemm_f32_takes(A, W, C, M, N, K), "spy_gemm_f32_parts: operands of %d x %d x %d are not taken", M, N, K);
+    const int tm = (M + 63) / 64, tn = (N + 63) / 64;
+    const int64_t blocks = (int64_t)tm * tn * parts;
+    SPY_REQUIRE(blocks < (1 << 28), "spy_gemm_f32_parts: too many blocks");
+    gemm_f32_tile_kernel<1><<<(unsigned)((blocks + 7) / 8 * 8), 256, 0, st>>>(A, W, C, M, N, K, tm, tn, parts);
+    SPY_CHECK_LAUNCH("spy_gemm_f32_parts");
     return 0;
 }

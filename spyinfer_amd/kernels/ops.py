@@ -82,7 +82,7 @@ class _Hip:
                      "spy_moe_align", "spy_moe_gemm", "spy_moe_combine", "spy_moe_tile_rows", "spy_moe_group_ints", "spy_token_shift", "spy_tanh", "spy_time_mix",
                      "spy_norm_pair_mean", "spy_scale_cap", "spy_result_norm", "spy_moe_align_tables", "spy_layer_norm", "spy_layer_norm_residual",
                      "spy_gelu", "spy_norm_rope_store", "spy_map_difference", "spy_rotation_angles", "spy_decay_memory", "spy_group_norm", "spy_gemm_rows",
-                     "spy_add_parts_rmsnorm"):
+                     "spy_add_parts_rmsnorm", "spy_gemm_f32_parts"):
             if not hasattr(self.lib, name):
                 raise KernelError("the kernel library %s lacks %s: it is older than its sources; build it again "
                                   "(spyinfer_amd.kernels.build.build())" % (self.lib._name, name))
@@ -509,6 +509,23 @@ def rows_product_parts(M: int, N: int, K: int):
 
 
 @functools.lru_cache(maxsize=1024)
+def f32_product_parts(M: int, N: int, K: int):
+    """Parts of K for a float32 product whose result the next norm sums from them, or None where one pass is the better one.  A part of a
+    tile of 64 x 64 is a block; the numbers are fitted to 380 launches of 17 to 2048 rows (the choice is 0.13 % behind the best on average,
+    6 % at most, the parts' sum counted), and up to 16 rows the streaming kernel stands."""
+    if M <= 16 or K % 4 or -(-M // 64) * -(-N // 64) >= 1 << 20:
+        return None
+    tiles = -(-M // 64) * -(-N // 64)
+
+    def us(p):
+        total = p * M * N * 4
+        return -(-tiles * p // 256) * (K / p) * 0.0178 + (K / p) * 0.0066 + total / 8e6 + (total / 4.5e6 + 0.3 if p > 1 else 0.0)
+
+    best = min((p for p in (1, 2, 3, 4, 5, 6, 8, 12) if p == 1 or (K // 32 // p >= 4 and tiles * p <= 1400 and p * M * N * 4 <= PARTS_MAX_BYTES)), key=us)
+    return best if best > 1 else None
+
+
+@functools.lru_cache(maxsize=1024)
 def rows_product_gated(M: int, N: int, K: int, library: bool) -> int:
     """Row tiles a block of the gated product of many rows (N = 2 I rows of the matrix), or 0 where the library's product and a pass
     for the activation are the better ones (``library`` false: that way is not at hand at its own price).  It loses where its blocks
@@ -537,6 +554,14 @@ class ProductParts:
 def linear_parts(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor] = None):
     """``linear_few``, or, where a product of many rows is better cut along K, its ``ProductParts``."""
     M, K = x.shape
+    if x.dtype == torch.float32 and x.is_cuda and isinstance(w, torch.Tensor) and w.dtype == torch.float32 and x.is_contiguous() and w.is_contiguous() \
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0 and w.shape[1] == K:
+        parts = f32_product_parts(M, w.shape[0], K)
+        if parts is not None:
+            _dev(x, w)
+            out = torch.empty((parts, M, w.shape[0]), dtype=torch.float32, device=x.device)
+            hip().call("spy_gemm_f32_parts", _ptr(out), _ptr(x), _ptr(w), M, w.shape[0], K, parts, _Hip.stream())
+            return ProductParts(out)
     plan = rows_product_parts(M, w.shape[0], K) if tiled is not None and x.dtype == torch.bfloat16 and x.is_contiguous() else None
     if plan is None:
         return linear_few(x, w, tiled)

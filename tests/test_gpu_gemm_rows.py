@@ -27,6 +27,22 @@ def test_parts(M, N, K, tiles, parts, monkeypatch):
         assert float((out.parts[p].cpu().double() - ref).abs().max()) < 1e-5
 
 
+@pytest.mark.parametrize("M,N,K,parts", [(17, 64, 32, 1), (65, 100, 132, 2), (64, 1000, 2048, 12), (130, 66, 1000, 5), (200, 384, 612, 3)])
+def test_float32_parts(M, N, K, parts, monkeypatch):
+    from spyinfer_amd.kernels import ops
+    monkeypatch.setattr(ops, "f32_product_parts", lambda *size: parts)
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn((M, K), generator=g), torch.randn((N, K), generator=g) * K ** -0.5
+    out = ops.linear_parts(x.to(dev), w.to(dev))
+    assert isinstance(out, ops.ProductParts) and tuple(out.parts.shape) == (parts, M, N)
+    steps = -(-K // 32)
+    bounds = [min(K, steps * p // parts * 32) for p in range(parts + 1)]
+    for p, (a, b) in enumerate(zip(bounds, bounds[1:])):
+        ref = x[:, a:b].double() @ w[:, a:b].double().T
+        assert float((out.parts[p].cpu().double() - ref).abs().max()) < 1e-5           # (as above)
+
+
 @pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
 @pytest.mark.parametrize("M,I,K,tiles", [(65, 128, 128, 4), (200, 144, 256, 7), (131, 16, 384, 5), (193, 1040, 640, 6), (300, 384, 1152, 8)])
 def test_gated(M, I, K, tiles, activation, monkeypatch):
