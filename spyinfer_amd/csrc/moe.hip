@@ -892,8 +892,9 @@ extern "C" int spy_moe_gemm(void* C, int c_dtype, const void* A, int a_dtype, co
         const int cols = wide ? (gated ? 128 : 256) : (gated ? 64 : 128), gy = (N + cols - 1) / cols;
         const int64_t blocks = (int64_t)moe_max_groups(max_tiles, E, P) * gy;
         SPY_REQUIRE(blocks < (1 << 30), "spy_moe_gemm: too many blocks");
-        const int64_t most = wide ? max(blocks, min(2 * blocks, (int64_t)2 * MOE_HALVES + MOE_DIES)) : blocks;
-        const unsigned grid = (unsigned)((most + MOE_DIES - 1) / MOE_DIES * MOE_DIES);
+        // (up to MOE_HALVES blocks become two each, every die with its whole run twice)
+        const int64_t runs = (blocks + MOE_DIES - 1) / MOE_DIES, halved = 2 * ((min(blocks, (int64_t)MOE_HALVES) + MOE_DIES - 1) / MOE_DIES);
+        const unsigned grid = (unsigned)((wide ? max(runs, halved) : runs) * MOE_DIES);
         const long long ws = (long long)(gated ? 2 : 1) * N * K;
         if (wide && gated) {
             SPY_DISPATCH(c_dtype, TC, (moe_gemm_rows_kernel<true, TC><<<grid, 256, 0, st>>>((TC*)C, (const bf16_t*)A, (unsigned)moe_a_bytes(gather, P, max_tiles, K), (const bf16_t*)W, tile_expert,

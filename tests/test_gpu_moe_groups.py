@@ -79,9 +79,9 @@ def test_groups_of_an_alignment():
 
 @pytest.mark.parametrize("by_groups", [True, False])
 @pytest.mark.parametrize("form", ["silu", "weighted", "gelu"])
-@pytest.mark.parametrize("kind,E,top,K,F", [("even", 6, 2, 128, 128), ("one", 5, 2, 384, 128), ("edges", 9, 3, 256, 640), ("few", 16, 4, 128, 384), ("one", 40, 3, 640, 1024)])
+@pytest.mark.parametrize("kind,E,top,K,F", [("even", 6, 2, 128, 128), ("one", 5, 2, 384, 128), ("edges", 9, 3, 256, 640), ("few", 16, 4, 128, 384), ("one", 40, 3, 640, 1024), ("few", 3, 1, 128, 384)])
 def test_experts_in_operand_order(kind, E, top, K, F, form, by_groups, monkeypatch):
-    """Matrices in operand order: one turn of 128 of K, an odd number of them, groups in halves and whole, against the rows' kernels."""
+    """Matrices in operand order: one turn of 128 of K, an odd number of them, groups in halves and whole, as many blocks as the grid can have at most, against the rows' kernels."""
     from spyinfer_amd.kernels import ops
     monkeypatch.setattr(ops, "experts_by_groups", lambda *sizes: by_groups)
     dev = require_gpu()
