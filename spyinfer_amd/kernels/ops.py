@@ -82,7 +82,7 @@ class _Hip:
                      "spy_moe_align", "spy_moe_gemm", "spy_moe_combine", "spy_moe_tile_rows", "spy_moe_group_ints", "spy_token_shift", "spy_tanh", "spy_time_mix",
                      "spy_norm_pair_mean", "spy_scale_cap", "spy_result_norm", "spy_moe_align_tables", "spy_layer_norm", "spy_layer_norm_residual",
                      "spy_gelu", "spy_norm_rope_store", "spy_map_difference", "spy_rotation_angles", "spy_decay_memory", "spy_group_norm", "spy_gemm_rows",
-                     "spy_add_parts_rmsnorm", "spy_gemm_f32_parts"):
+                     "spy_add_parts_rmsnorm", "spy_gemm_f32_parts", "spy_gemm_f32_gated"):
             if not hasattr(self.lib, name):
                 raise KernelError("the kernel library %s lacks %s: it is older than its sources; build it again "
                                   "(spyinfer_amd.kernels.build.build())" % (self.lib._name, name))
@@ -614,6 +614,11 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, tiled: Optional[torc
         out = torch.empty((M, I), dtype=x.dtype, device=x.device)
         hip().call("spy_gemm_skinny_swiglu", _ptr(x), _ptr(w_gate_up), _ptr(out), _code(out, "out"), ctypes.c_int(M),
                    ctypes.c_int(I), ctypes.c_int(K), ctypes.c_int(GATED_ACTIVATIONS[activation]), _Hip.stream())
+        return out
+    if x.dtype == torch.float32 and x.is_cuda and isinstance(w_gate_up, torch.Tensor) and w_gate_up.dtype == torch.float32 and 0 < M <= 4 and K % 4 == 0 \
+            and x.is_contiguous() and w_gate_up.is_contiguous() and (x.data_ptr() | w_gate_up.data_ptr()) % 16 == 0:
+        out = torch.empty((M, I), dtype=x.dtype, device=x.device)
+        hip().call("spy_gemm_f32_gated", _ptr(out), _ptr(x), _ptr(w_gate_up), M, I, K, GATED_ACTIVATIONS[activation], _Hip.stream())
         return out
     if x.dtype == torch.bfloat16 and tiled is not None and x.is_contiguous():
         tiles = rows_product_gated(M, 2 * I, K, not isinstance(w_gate_up, TiledOnly))

@@ -3,7 +3,7 @@ multiples of nothing (K: of four), each choice of the dispatch."""
 import pytest
 import torch
 
-from tests.gpu_util import require_gpu
+from tests.gpu_util import close, require_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +50,15 @@ def test_infinities_and_nan_stay_in_their_rows(M, N):
     x[M - 1, 3], w[N - 1, 7], w[0, 99] = float("inf"), float("nan"), float("-inf")
     assert torch.equal(ops.linear(x, w).isnan(), (x @ w.t()).isnan())
     assert torch.equal(ops.linear(x, w).isinf(), (x @ w.t()).isinf())
+
+
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("M,I,K", [(1, 5, 4), (1, 1023, 1028), (2, 130, 516), (3, 64, 2048), (4, 1001, 260), (4, 6144, 512)])
+def test_gated_float32_product_of_few_rows(M, I, K, activation):
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(M + I + K)
+    x, w = torch.randn((M, K), generator=g), torch.randn((2 * I, K), generator=g) * K ** -0.5
+    h = x.double() @ w.double().T
+    act = torch.nn.functional.silu if activation == "silu" else lambda z: torch.nn.functional.gelu(z, approximate="tanh")
+    close(ops.linear_swiglu(x.to(dev), w.to(dev), activation=activation), act(h[:, :I]) * h[:, I:], torch.float32, what="gated float32 product")
