@@ -500,8 +500,10 @@ def rows_product_parts(M: int, N: int, K: int):
     where the library's product is the better one: it has tiles for the whole chip, or K is too short for the parts to pay.
     Measured, us with the parts' sum against the library's: 409 rows, 2560 x 9728: 33 / 54; 1100 rows: 64 / 70, 2011 rows (beyond
     the line): 106 / 104; 1356 rows, 4096 x 12288: 137 / 138; 800 rows, 2560 x 4096: 29 / 35, 1100 rows (beyond): 33 / 31; 1356 rows,
-    2048 x 6144: 46 / 45; 560 rows, 1024 x 3072: 12.0 / 13.8; K = 2048: 409 rows, 2048 columns: 14 / 11."""
-    if M <= DECODE_ROWS_PLAIN or N % 16 or K % 128 or K < 3072 or M * N * 4096 > 2.3e6 * K or N * K >= 1 << 30 or M * K >= 1 << 30:
+    2048 x 6144: 46 / 45; 560 rows, 1024 x 3072: 12.0 / 13.8; K = 2048: 288 rows, 2048 columns: 10.4 / 10.6, 409 rows
+    (beyond): 13 / 11; 200 rows, 1024 columns: 7.9 / 8.3 (and a launch costs the host 8 us, the library's product 20: a step of 200
+    tokens, 1024 wide, whose launches bound it: 4.19 -> 3.43 ms)."""
+    if M <= DECODE_ROWS_PLAIN or N % 16 or K % 128 or K < 2048 or M * N * 4096 > 2.3e6 * K or (K < 3072 and M * N > 6e5) or N * K >= 1 << 30 or M * K >= 1 << 30:
         return None
     fits = [(t, p) for t in range(4, 9) if 16 * t <= M for p in range(1, min(12, K // 256) + 1)
             if p * M * N * 4 <= PARTS_MAX_BYTES and -(-M // (16 * t)) * -(-N // 256) * p <= 512]
@@ -2249,13 +2251,9 @@ class TiledExperts:
         """``mats``: per expert the matrices whose rows make it up, one after the other (whole tiles of 16 rows of each)."""
         E, N, K = len(mats), sum(m.shape[0] for m in mats[0]), mats[0][0].shape[1]
         self.shape = torch.Size((E, N, K))
-        self.data = torch.empty((E, K // 128, N // 16, 4, 4, 16, 8), dtype=torch.bfloat16, device=mats[0][0].device)
-        for e, parts in enumerate(mats):
-            at = 0
-            for m in parts:
-                n = m.shape[0] // 16
-                self.data[e, :, at:at + n].copy_(m.view(n, 16, K // 128, 4, 4, 8).permute(2, 0, 3, 4, 1, 5))
-                at += n
+        rows = torch.stack([m for parts in mats for m in parts]) if len({m.shape for parts in mats for m in parts}) == 1 \
+            else torch.stack([torch.cat(parts, dim=0) for parts in mats])
+        self.data = rows.view(E, N // 16, 16, K // 128, 4, 4, 8).permute(0, 3, 1, 4, 5, 2, 6).contiguous()
 
     @staticmethod
     def takes(mats) -> bool:

@@ -23,6 +23,7 @@ def test_sizes_on_both_sides_of_the_line():
     assert ops.rows_product_parts(409, 2560, 9728) == (7, 6)
     assert ops.rows_product_parts(2011, 2560, 9728) is not None and ops.rows_product_parts(2011, 4096, 12288) is None
     assert ops.rows_product_parts(64, 2560, 9728) is None and ops.rows_product_parts(409, 2048, 2048) is None
+    assert ops.rows_product_parts(200, 1024, 2048) is not None and ops.rows_product_parts(200, 1024, 1920) is None
     assert ops.rows_product_gated(1356, 12288, 2048, True) == 6 and ops.rows_product_gated(64, 12288, 2048, True) == 0
     assert ops.rows_product_gated(2011, 24576, 4096, True) == 0 and ops.rows_product_gated(2011, 24576, 4096, False) > 0
     assert ops.rows_product_gated(200, 6144, 4096, True) == 0
