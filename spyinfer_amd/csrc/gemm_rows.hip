@@ -2,6 +2,7 @@
 // sums on v_mfma_f32_16x16x32_bf16:
 //   ROWS_PARTS:  K cut into parts, one block each: parts[p][M][N] float32, added in the pass of the norm that reads the result
 //                (spy_add_parts_rmsnorm), which reads the stream there anyway;
+//   ROWS_STORE:  C[M][N] in bfloat16;
 //   ROWS_GATED:  W = [gate rows | up rows], C[M][N / 2] = act(gate) * up in bfloat16, without the [M][N] tensor in between.
 //
 // A block has 16 MT rows of X and 256 rows of W (gated: 128 gate rows and the 128 up rows of the same columns); each of its four
@@ -21,6 +22,7 @@
 // is the loads' way, from memory where few tiles share W, and the turn's barrier.
 #include "common.h"
 
+#define ROWS_STORE 0
 #define ROWS_PARTS 1
 #define ROWS_GATED 2
 #define ROWS_DIES 8
@@ -130,6 +132,14 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(void* C, const bf16_t
                 const int tile = col_t * 16 + wave * 4 + j;
                 if (tile < NT) *reinterpret_cast<gr_f32x4_t*>(c_row + tile * 16) = acc[j][i];
             }
+        } else if (EPI == ROWS_STORE) {
+            bf16_t* c_row = (bf16_t*)C + (size_t)row * N + 4 * g;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int tile = col_t * 16 + wave * 4 + j;
+                const uint2 o = {pack_bf16x2(acc[j][i][0], acc[j][i][1]), pack_bf16x2(acc[j][i][2], acc[j][i][3])};
+                if (tile < NT) *reinterpret_cast<uint2*>(c_row + tile * 16) = o;
+            }
         } else {
             bf16_t* c_row = (bf16_t*)C + (size_t)row * (N / 2) + 4 * g;
 #pragma unroll
@@ -146,32 +156,33 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(void* C, const bf16_t
 }
 
 template <int MT>
-static int rows_launch(void* C, const void* X, const void* W, int M, int N, int K, int parts, bool gated, GateAct act, hipStream_t st) {
+static int rows_launch(void* C, const void* X, const void* W, int M, int N, int K, int parts, int epi, GateAct act, hipStream_t st) {
     const int n_rows = (M + MT * 16 - 1) / (MT * 16), n_cols = (N + 255) / 256;
     const int64_t blocks = (int64_t)n_rows * n_cols * parts;
     SPY_REQUIRE(M >= MT * 16 && blocks < (1 << 30), "spy_gemm_rows: %d rows in tiles of %d, %lld blocks", M, MT * 16, (long long)blocks);
     const unsigned grid = (unsigned)((blocks + ROWS_DIES - 1) / ROWS_DIES * ROWS_DIES);
-    if (gated) gemm_rows_kernel<MT, ROWS_GATED><<<grid, 256, 0, st>>>(C, (const bf16_t*)X, (const bf16_t*)W, M, N, K, n_rows, n_cols, 1, (int)blocks, act);
+    if (epi == ROWS_STORE) gemm_rows_kernel<MT, ROWS_STORE><<<grid, 256, 0, st>>>(C, (const bf16_t*)X, (const bf16_t*)W, M, N, K, n_rows, n_cols, 1, (int)blocks, act);
+    else if (epi == ROWS_GATED) gemm_rows_kernel<MT, ROWS_GATED><<<grid, 256, 0, st>>>(C, (const bf16_t*)X, (const bf16_t*)W, M, N, K, n_rows, n_cols, 1, (int)blocks, act);
     else gemm_rows_kernel<MT, ROWS_PARTS><<<grid, 256, 0, st>>>(C, (const bf16_t*)X, (const bf16_t*)W, M, N, K, n_rows, n_cols, parts, (int)blocks, act);
     SPY_CHECK_LAUNCH("spy_gemm_rows");
     return 0;
 }
 
-// C: gated: bfloat16 [M, N / 2]; else float32 [parts, M, N].  X: bfloat16 rows [M, K]; W: the tiled copy of [N, K].  row_tiles: MT.
-extern "C" int spy_gemm_rows(void* C, const void* X, const void* W, int M, int N, int K, int row_tiles, int parts, int gated, int act_code,
+// epi: what is formed (see the top): C bfloat16 [M, N], float32 [parts, M, N] or bfloat16 [M, N / 2].  X: bfloat16 rows [M, K]; W: the tiled copy of [N, K].  row_tiles: MT.
+extern "C" int spy_gemm_rows(void* C, const void* X, const void* W, int M, int N, int K, int row_tiles, int parts, int epi, int act_code,
                              hipStream_t st) {
     GateAct act = {1.f, 0.f};
-    SPY_REQUIRE(M > 0 && N > 0 && K > 0 && N % (gated ? 32 : 16) == 0 && K % 128 == 0, "spy_gemm_rows: bad sizes %d x %d x %d", M, N, K);
+    SPY_REQUIRE(M > 0 && N > 0 && K > 0 && N % (epi == ROWS_GATED ? 32 : 16) == 0 && K % 128 == 0, "spy_gemm_rows: bad sizes %d x %d x %d", M, N, K);
     SPY_REQUIRE((int64_t)N * K < (1 << 30) && (int64_t)M * K < (1 << 30), "spy_gemm_rows: operands of %d x %d x %d are too large", M, N, K);
-    SPY_REQUIRE(parts >= 1 && parts <= K / 128 && (parts == 1 || !gated), "spy_gemm_rows: %d parts of K = %d", parts, K);
+    SPY_REQUIRE(parts >= 1 && parts <= K / 128 && (parts == 1 || epi == ROWS_PARTS) && epi >= ROWS_STORE && epi <= ROWS_GATED, "spy_gemm_rows: %d parts of K = %d", parts, K);
     SPY_REQUIRE((((uintptr_t)C | (uintptr_t)X | (uintptr_t)W) % 16) == 0, "spy_gemm_rows: operands must be 16-byte aligned");
-    SPY_REQUIRE(!gated || gate_act_of(act_code, &act), "spy_gemm_rows: unknown activation %d", act_code);
+    SPY_REQUIRE(epi != ROWS_GATED || gate_act_of(act_code, &act), "spy_gemm_rows: unknown activation %d", act_code);
     switch (row_tiles) {
-        case 4: return rows_launch<4>(C, X, W, M, N, K, parts, gated, act, st);
-        case 5: return rows_launch<5>(C, X, W, M, N, K, parts, gated, act, st);
-        case 6: return rows_launch<6>(C, X, W, M, N, K, parts, gated, act, st);
-        case 7: return rows_launch<7>(C, X, W, M, N, K, parts, gated, act, st);
-        case 8: return rows_launch<8>(C, X, W, M, N, K, parts, gated, act, st);
+        case 4: return rows_launch<4>(C, X, W, M, N, K, parts, epi, act, st);
+        case 5: return rows_launch<5>(C, X, W, M, N, K, parts, epi, act, st);
+        case 6: return rows_launch<6>(C, X, W, M, N, K, parts, epi, act, st);
+        case 7: return rows_launch<7>(C, X, W, M, N, K, parts, epi, act, st);
+        case 8: return rows_launch<8>(C, X, W, M, N, K, parts, epi, act, st);
     }
     return spy_fail("spy_gemm_rows: %d row tiles", row_tiles);
 }

@@ -448,6 +448,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
     if all_bf16 and tiled is not None and M <= (TILED_ONLY_DIRECT_ROWS if isinstance(w, TiledOnly) else SKINNY_MAX_ROWS):
         _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
         return decode_linear(x, tiled, out_dtype, out)
+    if all_bf16 and tiled is not None and out_dtype == torch.bfloat16 and x.is_contiguous():
+        tiles = rows_product_stored(M, N, K)
+        if tiles:
+            _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
+            hip().call("spy_gemm_rows", _ptr(out), _ptr(x), _ptr(tiled), M, N, K, tiles, 1, ROWS_STORE, 0, _Hip.stream())
+            return out
     if isinstance(w, TiledOnly):
         w = w.rows()
     global _LIBRARY_F32_OUT
@@ -481,6 +487,8 @@ def linear_few(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor] =
     return linear(x, w, out_dtype, tiled=tiled, out=out)
 
 
+#: what ``spy_gemm_rows`` forms: bfloat16 rows, float32 parts, or a gated feed-forward's activation
+ROWS_STORE, ROWS_PARTS, ROWS_GATED = 0, 1, 2
 #: most bytes of a product's parts
 PARTS_MAX_BYTES = 64 << 20
 
@@ -508,6 +516,18 @@ def rows_product_parts(M: int, N: int, K: int):
     fits = [(t, p) for t in range(4, 9) if 16 * t <= M for p in range(1, min(12, K // 256) + 1)
             if p * M * N * 4 <= PARTS_MAX_BYTES and -(-M // (16 * t)) * -(-N // 256) * p <= 512]
     return min(fits, key=lambda f: _rows_product_us(M, N, K, *f), default=None)
+
+
+@functools.lru_cache(maxsize=1024)
+def rows_product_stored(M: int, N: int, K: int) -> int:
+    """Row tiles a block of the product of many rows that is stored in bfloat16, or 0 for the library's: a short K, whose few turns
+    the wide results' blocks walk while the library's start (us, library / this: 4096 x 1024, 130 rows 8.8 / 10.1, 409 rows 10.3 / 10.8,
+    560 rows 13.2 / 10.6, 1356 rows 20.6 / 15.2, 1700 rows 19.9 / 18.2; 6144 x 1024, 409 rows 16.2 / 14.5, 1100 rows 21.3 / 19.1, 1356 rows,
+    beyond the line, 23.8 / 26; 4096 x 2048, 409 rows 17.0 / 23.5).  Below 409 rows the steps are bound by their launches, of which the
+    library's costs the host 12 us more."""
+    if M <= DECODE_ROWS_PLAIN or N % 16 or K % 128 or K > 1024 or N < 4096 or M * N > 7e6:
+        return 0
+    return min((t for t in range(4, 9) if 16 * t <= M), key=lambda t: _rows_product_us(M, N, K, t, 1))
 
 
 @functools.lru_cache(maxsize=1024)
@@ -571,7 +591,7 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor]
     N = w.shape[0]
     _check(tuple(tiled.shape) == (N, K) and w.shape[1] == K, "linear_parts: the matrix or its tiled copy does not fit rows of %d", K)
     parts = torch.empty((plan[1], M, N), dtype=torch.float32, device=x.device)
-    hip().call("spy_gemm_rows", _ptr(parts), _ptr(x), _ptr(tiled), M, N, K, plan[0], plan[1], 0, 0, _Hip.stream())
+    hip().call("spy_gemm_rows", _ptr(parts), _ptr(x), _ptr(tiled), M, N, K, plan[0], plan[1], ROWS_PARTS, 0, _Hip.stream())
     return ProductParts(parts)
 
 
@@ -627,7 +647,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, tiled: Optional[torc
         if tiles:
             _check(tiled.shape == w_gate_up.shape, "linear_swiglu: the tiled copy does not fit")
             out = torch.empty((M, I), dtype=x.dtype, device=x.device)
-            hip().call("spy_gemm_rows", _ptr(out), _ptr(x), _ptr(tiled), M, 2 * I, K, tiles, 1, 1, GATED_ACTIVATIONS[activation], _Hip.stream())
+            hip().call("spy_gemm_rows", _ptr(out), _ptr(x), _ptr(tiled), M, 2 * I, K, tiles, 1, ROWS_GATED, GATED_ACTIVATIONS[activation], _Hip.stream())
             return out
     return swiglu(linear(x, w_gate_up), activation)
 

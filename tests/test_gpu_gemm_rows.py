@@ -27,6 +27,17 @@ def test_parts(M, N, K, tiles, parts, monkeypatch):
         assert float((out.parts[p].cpu().double() - ref).abs().max()) < 1e-5
 
 
+@pytest.mark.parametrize("M,N,K,tiles", [(65, 272, 128, 4), (200, 1040, 384, 7), (131, 512, 640, 5), (193, 48, 1024, 6), (300, 256, 256, 8)])
+def test_stored(M, N, K, tiles, monkeypatch):
+    from spyinfer_amd.kernels import ops
+    monkeypatch.setattr(ops, "rows_product_stored", lambda *size: tiles)
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn((M, K), generator=g).bfloat16(), (torch.randn((N, K), generator=g) * K ** -0.5).bfloat16()
+    wd = w.to(dev)
+    close(ops.linear(x.to(dev), wd, tiled=ops.tile_weight(wd)), x.double() @ w.double().T, torch.bfloat16, what="product of many rows")
+
+
 @pytest.mark.parametrize("M,N,K,parts", [(17, 64, 32, 1), (65, 100, 132, 2), (64, 1000, 2048, 12), (130, 66, 1000, 5), (200, 384, 612, 3)])
 def test_float32_parts(M, N, K, parts, monkeypatch):
     from spyinfer_amd.kernels import ops

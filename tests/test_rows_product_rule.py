@@ -15,6 +15,8 @@ def test_launches_fit_the_kernel():
             assert N * K < 1 << 30 and M * K < 1 << 30
         tiles = ops.rows_product_gated.__wrapped__(M, 2 * N, K, True)
         assert tiles == 0 or (M > 64 and 4 <= tiles <= 8 and 16 * tiles <= M and 2 * N * K < 1 << 30 and M * K < 1 << 30)
+        tiles = ops.rows_product_stored.__wrapped__(M, N, K)
+        assert tiles == 0 or (M > 64 and 4 <= tiles <= 8 and 16 * tiles <= M)
         parts = ops.f32_product_parts.__wrapped__(M, N, K)
         assert parts is None or (M > 16 and 2 <= parts <= K // 128 and parts * M * N * 4 <= ops.PARTS_MAX_BYTES)
 
@@ -28,3 +30,4 @@ def test_sizes_on_both_sides_of_the_line():
     assert ops.rows_product_gated(2011, 24576, 4096, True) == 0 and ops.rows_product_gated(2011, 24576, 4096, False) > 0
     assert ops.rows_product_gated(200, 6144, 4096, True) == 0
     assert ops.f32_product_parts(611, 1024, 2048) == 3 and ops.f32_product_parts(16, 1024, 2048) is None and ops.f32_product_parts(1500, 2048, 2048) is None
+    assert ops.rows_product_stored(409, 4096, 1024) > 0 and ops.rows_product_stored(409, 4096, 2048) == 0 and ops.rows_product_stored(1356, 6144, 1024) == 0
