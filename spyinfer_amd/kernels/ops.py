@@ -523,9 +523,10 @@ def rows_product_stored(M: int, N: int, K: int) -> int:
     """Row tiles a block of the product of many rows that is stored in bfloat16, or 0 for the library's: a short K, whose few turns
     the wide results' blocks walk while the library's start (us, library / this: 4096 x 1024, 130 rows 8.8 / 10.1, 409 rows 10.3 / 10.8,
     560 rows 13.2 / 10.6, 1356 rows 20.6 / 15.2, 1700 rows 19.9 / 18.2; 6144 x 1024, 409 rows 16.2 / 14.5, 1100 rows 21.3 / 19.1, 1356 rows,
-    beyond the line, 23.8 / 26; 4096 x 2048, 409 rows 17.0 / 23.5).  Below 409 rows the steps are bound by their launches, of which the
+    beyond the line, 23.8 / 26; 4096 x 2048, 409 rows, beyond, 17.0 / 23.5, 560 rows 24.3 / 23.6, 1356 rows 31.0 / 28.4; 6144 x 2048, 1100 rows
+    33.0 / 30.1).  Below 409 rows the steps are bound by their launches, of which the
     library's costs the host 12 us more."""
-    if M <= DECODE_ROWS_PLAIN or N % 16 or K % 128 or K > 1024 or N < 4096 or M * N > 7e6:
+    if M <= DECODE_ROWS_PLAIN or N % 16 or K % 128 or K > 2048 or (K > 1024 and M < 560) or N < 4096 or M * N > 7e6:
         return 0
     return min((t for t in range(4, 9) if 16 * t <= M), key=lambda t: _rows_product_us(M, N, K, t, 1))
 
@@ -576,14 +577,17 @@ class ProductParts:
 def linear_parts(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor] = None):
     """``linear_few``, or, where a product of many rows is better cut along K, its ``ProductParts``."""
     M, K = x.shape
-    if x.dtype == torch.float32 and x.is_cuda and isinstance(w, torch.Tensor) and w.dtype == torch.float32 and x.is_contiguous() and w.is_contiguous() \
-            and (x.data_ptr() | w.data_ptr()) % 16 == 0 and w.shape[1] == K:
+    if M <= 16:                        # (short steps are bound by their launches: nothing more is asked of them)
+        return linear_few(x, w, tiled)
+    if x.dtype == torch.float32:
         parts = f32_product_parts(M, w.shape[0], K)
-        if parts is not None:
+        if parts is not None and x.is_cuda and isinstance(w, torch.Tensor) and w.dtype == torch.float32 and x.is_contiguous() and w.is_contiguous() \
+                and (x.data_ptr() | w.data_ptr()) % 16 == 0 and w.shape[1] == K:
             _dev(x, w)
             out = torch.empty((parts, M, w.shape[0]), dtype=torch.float32, device=x.device)
             hip().call("spy_gemm_f32_parts", _ptr(out), _ptr(x), _ptr(w), M, w.shape[0], K, parts, _Hip.stream())
             return ProductParts(out)
+        return linear_few(x, w, tiled)
     plan = rows_product_parts(M, w.shape[0], K) if tiled is not None and x.dtype == torch.bfloat16 and x.is_contiguous() else None
     if plan is None:
         return linear_few(x, w, tiled)
@@ -637,7 +641,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, tiled: Optional[torc
         hip().call("spy_gemm_skinny_swiglu", _ptr(x), _ptr(w_gate_up), _ptr(out), _code(out, "out"), ctypes.c_int(M),
                    ctypes.c_int(I), ctypes.c_int(K), ctypes.c_int(GATED_ACTIVATIONS[activation]), _Hip.stream())
         return out
-    if x.dtype == torch.float32 and x.is_cuda and isinstance(w_gate_up, torch.Tensor) and w_gate_up.dtype == torch.float32 and 0 < M <= 4 and K % 4 == 0 \
+    if 0 < M <= 4 and x.dtype == torch.float32 and x.is_cuda and isinstance(w_gate_up, torch.Tensor) and w_gate_up.dtype == torch.float32 and K % 4 == 0 \
             and x.is_contiguous() and w_gate_up.is_contiguous() and (x.data_ptr() | w_gate_up.data_ptr()) % 16 == 0:
         out = torch.empty((M, I), dtype=x.dtype, device=x.device)
         hip().call("spy_gemm_f32_gated", _ptr(out), _ptr(x), _ptr(w_gate_up), M, I, K, GATED_ACTIVATIONS[activation], _Hip.stream())

@@ -396,7 +396,7 @@ class PagedAttention(Mixer):
 
     def forward_parts(self, x, batch, cache, store=True):
         """``forward`` for a block whose next norm takes the result in parts (``ops.ProductParts``)."""
-        if type(self).forward is not PagedAttention.forward or (batch.T <= ops.DECODE_ROWS_PLAIN and batch.act_dtype != torch.float32):
+        if batch.T <= 16 or type(self).forward is not PagedAttention.forward or (batch.T <= ops.DECODE_ROWS_PLAIN and batch.act_dtype != torch.float32):
             return self.forward(x, batch, cache, store)
         return ops.linear_parts(self._attend(x, batch, cache, store), self.w_o, self.w_o_tiled)
 

@@ -30,4 +30,4 @@ def test_sizes_on_both_sides_of_the_line():
     assert ops.rows_product_gated(2011, 24576, 4096, True) == 0 and ops.rows_product_gated(2011, 24576, 4096, False) > 0
     assert ops.rows_product_gated(200, 6144, 4096, True) == 0
     assert ops.f32_product_parts(611, 1024, 2048) == 3 and ops.f32_product_parts(16, 1024, 2048) is None and ops.f32_product_parts(1500, 2048, 2048) is None
-    assert ops.rows_product_stored(409, 4096, 1024) > 0 and ops.rows_product_stored(409, 4096, 2048) == 0 and ops.rows_product_stored(1356, 6144, 1024) == 0
+    assert ops.rows_product_stored(409, 4096, 1024) > 0 and ops.rows_product_stored(409, 4096, 2048) == 0 and ops.rows_product_stored(1356, 4096, 2048) > 0 and ops.rows_product_stored(1356, 6144, 1024) == 0
