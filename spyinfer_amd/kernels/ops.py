@@ -450,7 +450,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         return decode_linear(x, tiled, out_dtype, out)
     if all_bf16 and tiled is not None and out_dtype == torch.bfloat16 and x.is_contiguous():
         tiles = rows_product_stored(M, N, K)
-        if tiles:
+        if tiles and (x.data_ptr() | out.data_ptr()) % 16 == 0:
             _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
             hip().call("spy_gemm_rows", _ptr(out), _ptr(x), _ptr(tiled), M, N, K, tiles, 1, ROWS_STORE, 0, _Hip.stream())
             return out
@@ -573,6 +573,11 @@ class ProductParts:
     def resolve(self):
         return self.parts.sum(dim=0)
 
+    def to(self, dtype):
+        return self.resolve().to(dtype)
+
+    float = resolve                    # (for a block of another arrangement, which adds what is pending itself)
+
 
 def linear_parts(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor] = None):
     """``linear_few``, or, where a product of many rows is better cut along K, its ``ProductParts``."""
@@ -589,7 +594,7 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor]
             return ProductParts(out)
         return linear_few(x, w, tiled)
     plan = rows_product_parts(M, w.shape[0], K) if tiled is not None and x.dtype == torch.bfloat16 and x.is_contiguous() else None
-    if plan is None:
+    if plan is None or x.data_ptr() % 16:
         return linear_few(x, w, tiled)
     _dev(x, tiled)
     N = w.shape[0]
@@ -648,7 +653,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, tiled: Optional[torc
         return out
     if x.dtype == torch.bfloat16 and tiled is not None and x.is_contiguous():
         tiles = rows_product_gated(M, 2 * I, K, not isinstance(w_gate_up, TiledOnly))
-        if tiles:
+        if tiles and x.data_ptr() % 16 == 0:
             _check(tiled.shape == w_gate_up.shape, "linear_swiglu: the tiled copy does not fit")
             out = torch.empty((M, I), dtype=x.dtype, device=x.device)
             hip().call("spy_gemm_rows", _ptr(out), _ptr(x), _ptr(tiled), M, 2 * I, K, tiles, 1, ROWS_GATED, GATED_ACTIVATIONS[activation], _Hip.stream())
@@ -2320,6 +2325,8 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
     _check(gated or not weight_input, "moe_experts: experts without a gate take their weights at the output")
     if x.dtype != torch.bfloat16:              # (the kernels for float32 rows read the matrices' rows)
         w_gate_up, w_down = (w.rows() if isinstance(w, TiledExperts) else w for w in (w_gate_up, w_down))
+    elif x.data_ptr() % 16 and isinstance(w_gate_up, TiledExperts):
+        x = x.clone()
     up_tiled, down_tiled = isinstance(w_gate_up, TiledExperts), isinstance(w_down, TiledExperts)
     up, down = w_gate_up.data if up_tiled else w_gate_up, w_down.data if down_tiled else w_down
     _dev(x, ids, weights, up, down)
