@@ -1603,8 +1603,14 @@ def latent_key_parts(num_tiles: int, max_keys: int) -> int:
 
 def latent_few_key_parts(num_tiles: int, max_keys: int) -> int:
     """The same for ``latent_few_tiles``: chunks of 32 keys one after the other cost 2.6 us each, a second block on a compute unit as much
-    (32 tiles, 500 keys: 17.7 us in 8 parts, 22.4 in 16; one tile: 19.1 / 13.2 / 11.0 in 4 / 8 / 16)."""
-    return max(1, min(256 // max(1, num_tiles), 32, -(-max_keys // 32)))
+    (32 tiles, 500 keys: 17.7 us in 8 parts, 22.4 in 16; one tile: 19.1 / 13.2 / 11.0 in 4 / 8 / 16).  The number is part of a captured
+    step's shape, so it takes few values while a request grows, 7 at most (one for every chunk made 32, and a step run kernel by kernel
+    and a capture every 32 tokens); the parts beyond the chunks have nothing to do.  Launches alone, one part a chunk / this, us: one
+    tile, 300 keys 10.7 / 10.2, 700 keys 12.3 / 10.8; 5 tiles, 540 keys 11.6 / 12.1; 12 tiles, 300 keys 12.5 / 13.0, 540 keys 13.9 / 15.3;
+    100, 500 and 1500 keys have the same parts either way."""
+    chunks = -(-max_keys // 32)
+    steps = next((n for n in (1, 2, 4, 8, 16, 24) if n >= chunks), 32)
+    return max(1, min(256 // max(1, num_tiles), steps))
 
 
 def latent_attention(qa: torch.Tensor, cache: torch.Tensor, page_size: int, meta: "AttentionMeta", sink: Optional[torch.Tensor],
