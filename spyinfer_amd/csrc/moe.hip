@@ -252,10 +252,13 @@ extern "C" int spy_moe_tile_rows() { return MOE_TM; }
 extern "C" int spy_moe_group_ints(int max_tiles, int E, int P) { return 1 + 2 * moe_max_groups(max_tiles, E, P); }
 
 // A tile of MOE_TM sorted rows x 64 columns per block; 256 threads, thread (ty, tx) has row ty and columns 4 tx .. + 3.
-// gather > 0: row r reads A[sorted_pair[r] / gather] (the token of the pair); 0: A[r].
+// gather > 0: row r reads A[sorted_pair[r] / gather] (the token of the pair); 0: A[r].  TILED: the experts' matrices lie in operand
+// order (gemm_decode.h), where four neighbours in K are neighbours too: float32 rows of matrices that are kept so for bfloat16 ones.
+// Measured, both products of 32 experts of 2 x 1536 x 2048, four a token, us, matrices in row order / in operand order with a copy in row
+// order made in every call / as they lie: 4 tokens 483 / 1038 / 392, 200 tokens 1108 / 1615 / 731.
 #define MG_TN 64
 #define MG_K 16
-template <typename TA, typename TW, typename TC, bool GATED>
+template <typename TA, typename TW, typename TC, bool GATED, bool TILED>
 __global__ __launch_bounds__(256) void moe_gemm_kernel(TC* __restrict__ C, const TA* __restrict__ A, const TW* __restrict__ W,
                                                        const int* __restrict__ tile_expert, const int* __restrict__ sorted_pair,
                                                        int gather, int N, int K, long long w_stride, MoeAct act) {
@@ -277,6 +280,11 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(TC* __restrict__ C, const
     // staging: A 16 x 16 values, one per thread; W 64 x 16 values, four per thread
     const int ar = threadIdx.x >> 4, ak = threadIdx.x & 15;
     const int wr = threadIdx.x >> 2, wk = (threadIdx.x & 3) * 4;
+    const int w_tiles = (GATED ? 2 : 1) * N / 16;
+    auto w_at = [&](int n, int k) {
+        if (!TILED) return (size_t)n * K + k;
+        return ((size_t)(k >> 7) * w_tiles + (n >> 4)) * 2048 + ((k >> 5) & 3) * 512 + ((k >> 3) & 3) * 128 + (n & 15) * 8 + (k & 7);
+    };
     for (int k0 = 0; k0 < K; k0 += MG_K) {
         {
             const int sr = src[ar], k = k0 + ak;
@@ -285,8 +293,8 @@ __global__ __launch_bounds__(256) void moe_gemm_kernel(TC* __restrict__ C, const
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int k = k0 + wk + i, n = n0 + wr;
-            Ws[0][wk + i][wr] = (n < N && k < K) ? to_f32<TW>(We[(size_t)n * K + k]) : 0.f;
-            if (GATED) Ws[GATED ? 1 : 0][wk + i][wr] = (n < N && k < K) ? to_f32<TW>(We[(size_t)(N + n) * K + k]) : 0.f;
+            Ws[0][wk + i][wr] = (n < N && k < K) ? to_f32<TW>(We[w_at(n, k)]) : 0.f;
+            if (GATED) Ws[GATED ? 1 : 0][wk + i][wr] = (n < N && k < K) ? to_f32<TW>(We[w_at(N + n, k)]) : 0.f;
         }
         __syncthreads();
 #pragma unroll
@@ -885,8 +893,8 @@ extern "C" int spy_moe_gemm(void* C, int c_dtype, const void* A, int a_dtype, co
     SPY_REQUIRE((act_kind == 0 && !pair_w) || (act_kind == 1 && gated && limit > 0.f) || (act_kind == 2 && !gated && !pair_w), "spy_moe_gemm: activation %d with limit %g", act_kind, (double)limit);
     const MoeAct act = {act_kind, limit, pair_w};
     // bfloat16 operands in 16-byte pieces: the matrix cores; tiles_per_block: 0 = the plain float32 kernel
-    SPY_REQUIRE(!w_tiled || (tiles_per_block > 0 && a_dtype == SPY_BF16 && w_dtype == SPY_BF16 && K % 128 == 0 && N % 16 == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0),
-                "spy_moe_gemm: matrices in operand order are for bfloat16 rows, %d x %d", N, K);
+    SPY_REQUIRE(!w_tiled || (w_dtype == SPY_BF16 && K % 128 == 0 && N % 16 == 0 && ((uintptr_t)W % 16) == 0),
+                "spy_moe_gemm: matrices of %d x %d (dtype %d) do not lie in operand order", N, K, w_dtype);
     if (tiles_per_block >= 8 && group && a_dtype == SPY_BF16 && w_dtype == SPY_BF16 && K % 64 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C) % 16) == 0 && (!w_tiled || moe_rows_fit(gather, P, max_tiles, gated, N, K))) {
         const bool wide = w_tiled != 0;
         const int cols = wide ? (gated ? 128 : 256) : (gated ? 64 : 128), gy = (N + cols - 1) / cols;
@@ -921,13 +929,14 @@ extern "C" int spy_moe_gemm(void* C, int c_dtype, const void* A, int a_dtype, co
     SPY_REQUIRE(max_tiles <= 65535, "spy_moe_gemm: %d tiles are too many for the plain kernel", max_tiles);
     const dim3 grid((N + MG_TN - 1) / MG_TN, max_tiles);
     const long long ws = (long long)(gated ? 2 : 1) * N * K;
-    if (gated) {
-        SPY_DISPATCH(a_dtype, TA, SPY_DISPATCH(w_dtype, TW, SPY_DISPATCH(c_dtype, TC, (moe_gemm_kernel<TA, TW, TC, true><<<grid, 256, 0, st>>>(
-            (TC*)C, (const TA*)A, (const TW*)W, tile_expert, sorted_pair, gather, N, K, ws, act)))));
-    } else {
-        SPY_DISPATCH(a_dtype, TA, SPY_DISPATCH(w_dtype, TW, SPY_DISPATCH(c_dtype, TC, (moe_gemm_kernel<TA, TW, TC, false><<<grid, 256, 0, st>>>(
-            (TC*)C, (const TA*)A, (const TW*)W, tile_expert, sorted_pair, gather, N, K, ws, act)))));
-    }
+#define MOE_PLAIN_LAUNCH(TW, G, TILED)                                                                                                   \
+    SPY_DISPATCH(a_dtype, TA, SPY_DISPATCH(c_dtype, TC, (moe_gemm_kernel<TA, TW, TC, G, TILED><<<grid, 256, 0, st>>>(                     \
+        (TC*)C, (const TA*)A, (const TW*)W, tile_expert, sorted_pair, gather, N, K, ws, act))))
+    if (gated && w_tiled) { MOE_PLAIN_LAUNCH(bf16_t, true, true); }
+    else if (w_tiled) { MOE_PLAIN_LAUNCH(bf16_t, false, true); }
+    else if (gated) { SPY_DISPATCH(w_dtype, TW, MOE_PLAIN_LAUNCH(TW, true, false)); }
+    else { SPY_DISPATCH(w_dtype, TW, MOE_PLAIN_LAUNCH(TW, false, false)); }
+#undef MOE_PLAIN_LAUNCH
     SPY_CHECK_LAUNCH("spy_moe_gemm");
     return 0;
 }

@@ -2329,10 +2329,8 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
     act_kind = {"silu": 0, "clamped": 1, "gelu": ACT_GELU}[activation]
     gated = activation != "gelu"
     _check(gated or not weight_input, "moe_experts: experts without a gate take their weights at the output")
-    if x.dtype != torch.bfloat16:              # (the kernels for float32 rows read the matrices' rows)
-        w_gate_up, w_down = (w.rows() if isinstance(w, TiledExperts) else w for w in (w_gate_up, w_down))
-    elif x.data_ptr() % 16 and isinstance(w_gate_up, TiledExperts):
-        x = x.clone()
+    if x.dtype == torch.bfloat16 and x.data_ptr() % 16 and isinstance(w_gate_up, TiledExperts):
+        x = x.clone()                          # (the matrix cores' kernels take rows in 16-byte pieces)
     up_tiled, down_tiled = isinstance(w_gate_up, TiledExperts), isinstance(w_down, TiledExperts)
     up, down = w_gate_up.data if up_tiled else w_gate_up, w_down.data if down_tiled else w_down
     _dev(x, ids, weights, up, down)

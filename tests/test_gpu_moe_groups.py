@@ -98,3 +98,22 @@ def test_experts_in_operand_order(kind, E, top, K, F, form, by_groups, monkeypat
     close(out, ref, torch.bfloat16, scale=2.0, what="experts in operand order")
     if kind == "even":
         close(ops.moe_experts(x.float(), ids.to(dev), w, *tiled, **kw), ref, torch.float32, what="float32 rows of the same matrices")
+
+
+@pytest.mark.parametrize("dtype,form", [("float32", "silu"), ("float32", "gelu")])
+def test_plain_kernel_reads_operand_order(dtype, form, monkeypatch):
+    """The plain kernel (float32 rows) reads matrices in operand order as they lie, and sums the same values in the same order as from rows; no
+    copy of the matrices is made."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(11)
+    E, top, K, F, T, gated = 5, 2, 256, 384, 37, form != "gelu"
+    bf = lambda *s, std=1.0: (torch.randn(s, generator=g) * std).bfloat16().to(dev)
+    x, wgu, wd = bf(T, K).to(getattr(torch, dtype)), bf(E, (2 if gated else 1) * F, K, std=K ** -0.5), bf(E, K, F, std=F ** -0.5)
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).int().to(dev)
+    w = torch.rand((T, top), generator=g).to(dev)
+    tiled = [ops.expert_forms([[m] for m in mats]) for mats in (wgu, wd)]
+    assert all(isinstance(m, ops.TiledExperts) for m in tiled)
+    ref = ops.moe_experts(x, ids, w, wgu, wd, activation=form)
+    monkeypatch.setattr(ops.TiledExperts, "rows", lambda self: pytest.fail("the matrices were copied"))
+    assert torch.equal(ops.moe_experts(x, ids, w, *tiled, activation=form), ref)
