@@ -1577,7 +1577,7 @@ LATENT_TILE_ROWS_MANY = 128  # the same for steps with rows for every compute un
 
 def latent_tile_rows(total_rows: int) -> int:
     return LATENT_TILE_ROWS_MANY if total_rows >= LATENT_TILE_ROWS_MANY * 512 else LATENT_TILE_ROWS
-LATENT_MFMA = True          # False forces the plain kernel for bfloat16 too (tests flip it; nothing else does)
+LATENT_MFMA = True          # False forces the plain kernel for bfloat16 too, whatever the matrices' order (tests flip it; nothing else does)
 
 
 def latent_attention_mfma_ok(dtype, R: int, D: int) -> bool:
@@ -2162,7 +2162,7 @@ def moe_route(z: torch.Tensor, correction: Optional[torch.Tensor], top: int, gro
     return ids, w
 
 
-MOE_MFMA = True            # False forces the plain float32 kernel for bfloat16 too (tests flip it; nothing else does)
+MOE_MFMA = True            # False forces the plain float32 kernel for bfloat16 too, whatever the matrices' order (tests flip it; nothing else does)
 
 
 class MoEAlignment:
@@ -2365,7 +2365,7 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
         sorted_pairs, tile_experts, group_list = _ptr(sorted_pair), _ptr(tile_expert), _ptr(groups)
     # bfloat16: the matrix cores, a block taking one row tile of an expert (decoding: blocks for the whole device) or up to eight
     many = experts_by_groups(P, E, K, F, gated, up_tiled and down_tiled)
-    per_block = 0 if not (MOE_MFMA or up_tiled or down_tiled) or x.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16 else (8 if many else 1)
+    per_block = 0 if not MOE_MFMA or x.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16 else (8 if many else 1)
     act = torch.empty((max_tiles * tm, F), dtype=x.dtype, device=dev)
     hip().call("spy_moe_gemm", _ptr(act), _code(act, "act"), _ptr(x), _code(x, "x"), _ptr(up), _code(up, "expert matrices"), ctypes.c_int(up_tiled),
                tile_experts, sorted_pairs, group_list, ctypes.c_int(P), ctypes.c_int(top), ctypes.c_int(1 if gated else 0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(F),

@@ -100,11 +100,12 @@ def test_experts_in_operand_order(kind, E, top, K, F, form, by_groups, monkeypat
         close(ops.moe_experts(x.float(), ids.to(dev), w, *tiled, **kw), ref, torch.float32, what="float32 rows of the same matrices")
 
 
-@pytest.mark.parametrize("dtype,form", [("float32", "silu"), ("float32", "gelu")])
+@pytest.mark.parametrize("dtype,form", [("float32", "silu"), ("float32", "gelu"), ("bfloat16", "silu"), ("bfloat16", "gelu")])
 def test_plain_kernel_reads_operand_order(dtype, form, monkeypatch):
-    """The plain kernel (float32 rows) reads matrices in operand order as they lie, and sums the same values in the same order as from rows; no
-    copy of the matrices is made."""
+    """The plain kernel (float32 rows; bfloat16 ones with MOE_MFMA off) reads matrices in operand order as they lie, and sums the same values
+    in the same order as from rows; no copy of the matrices is made."""
     from spyinfer_amd.kernels import ops
+    monkeypatch.setattr(ops, "MOE_MFMA", False)
     dev = require_gpu()
     g = torch.Generator().manual_seed(11)
     E, top, K, F, T, gated = 5, 2, 256, 384, 37, form != "gelu"
