@@ -2366,6 +2366,13 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
     # bfloat16: the matrix cores, a block taking one row tile of an expert (decoding: blocks for the whole device) or up to eight
     many = experts_by_groups(P, E, K, F, gated, up_tiled and down_tiled)
     per_block = 0 if not MOE_MFMA or x.dtype != torch.bfloat16 or w_gate_up.dtype != torch.bfloat16 else (8 if many else 1)
+    if many and per_block:
+        # Byte offsets are 31 bits in the kernel for groups and matrices in operand order.  Beyond, a copy in row order, whose kernel has no
+        # such bound: a tile at a time would read an expert's matrix for every 16 rows, and takes 2^20 sorted rows at most
+        if up_tiled and 2 * max(T * K, F2 * K) >= 1 << 31:
+            up, up_tiled = w_gate_up.rows(), False
+        if down_tiled and 2 * max(rows * F, K * F) >= 1 << 31:
+            down, down_tiled = w_down.rows(), False
     act = torch.empty((max_tiles * tm, F), dtype=x.dtype, device=dev)
     hip().call("spy_moe_gemm", _ptr(act), _code(act, "act"), _ptr(x), _code(x, "x"), _ptr(up), _code(up, "expert matrices"), ctypes.c_int(up_tiled),
                tile_experts, sorted_pairs, group_list, ctypes.c_int(P), ctypes.c_int(top), ctypes.c_int(1 if gated else 0), ctypes.c_int(max_tiles), ctypes.c_int(E), ctypes.c_int(F),

@@ -118,3 +118,22 @@ def test_plain_kernel_reads_operand_order(dtype, form, monkeypatch):
     ref = ops.moe_experts(x, ids, w, wgu, wd, activation=form)
     monkeypatch.setattr(ops.TiledExperts, "rows", lambda self: pytest.fail("the matrices were copied"))
     assert torch.equal(ops.moe_experts(x, ids, w, *tiled, activation=form), ref)
+
+
+def test_more_rows_than_offsets_of_31_bits_reach():
+    """Experts in operand order where the activations pass 2^31 bytes and the sorted rows 2^20."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(12)
+    E, K, F, T = 8, 128, 1024, 131200
+    bf = lambda *s, std=1.0: (torch.randn(s, generator=g) * std).bfloat16()
+    x, wgu, wd, w = bf(T, K), bf(E, 2 * F, K, std=K ** -0.5), bf(E, K, F, std=F ** -0.5), torch.rand((T, E), generator=g)
+    ids = torch.arange(E, dtype=torch.int32).expand(T, E).contiguous()
+    assert 2 * T * E * F >= 1 << 31 and T * E > 1 << 20 and ops.experts_by_groups(T * E, E, K, F, True, True)
+    mats = [ops.expert_forms([[m] for m in mats.to(dev)]) for mats in (wgu, wd)]
+    assert all(isinstance(m, ops.TiledExperts) for m in mats)
+    out = ops.moe_experts(x.to(dev), ids.to(dev), w.to(dev), *mats)
+    at = torch.tensor([0, 1, 16, 77777, T // 2, T - 17, T - 1])
+    h = torch.einsum("tk,enk->ten", x[at].double(), wgu.double())
+    ref = torch.einsum("tef,ekf,te->tk", torch.nn.functional.silu(h[..., :F]) * h[..., F:], wd.double(), w[at].double())
+    close(out[at.to(dev)], ref, torch.bfloat16, scale=2.0, what="experts of many rows")
