@@ -13,8 +13,10 @@ from .base import Norm
 class RMSNorm(Norm):
     @property
     def takes_product_parts(self) -> bool:
-        """Whether ``add_norm`` sums a product's parts (``ops.ProductParts``) in its own pass."""
-        return type(self).add_norm is RMSNorm.add_norm
+        """Whether ``add_norm`` sums a product's parts (``ops.ProductParts``) in its own pass: one root mean square over the
+        whole row, and rows and a weight that the kernel takes."""
+        return type(self).add_norm is RMSNorm.add_norm and self.groups == 1 and self.size % 4 == 0 and self.size <= 8192 \
+            and self.weight is not None and self.weight.data_ptr() % 16 == 0
 
     def __init__(self, size: int, eps: float, suffix: str = ".weight", offset: float = 0.0, groups: int = 1, scalar: bool = False):
         """``groups``: the vector is cut into that many equal consecutive parts, each over its own root mean square (the
@@ -53,8 +55,7 @@ class RMSNorm(Norm):
         ``ops.EntryAddends`` (any of these plus an earlier state of the stream and a vector for every row).  ``second``:
         another norm of this kind that reads the same sum: the result is the pair of both outputs, from one pass."""
         if isinstance(delta, ops.ProductParts):
-            if second is None and self.groups == 1 and self.size % 4 == 0 and self.size <= (8192 if self.size >= 2048 else 2048) \
-                    and (self.weight.data_ptr() | resid.data_ptr()) % 16 == 0:
+            if second is None and self.takes_product_parts and resid.data_ptr() % 16 == 0:
                 return ops.add_parts_rms_norm(resid, delta, self.weight, self.eps, out_dtype, rows)
             delta = delta.resolve().to(out_dtype)
         if isinstance(delta, ops.NormedAddend):
