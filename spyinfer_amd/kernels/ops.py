@@ -564,11 +564,26 @@ def rows_product_gated(M: int, N: int, K: int, library: bool) -> int:
 
 class ProductParts:
     """A product's result while it still lies in parts [parts, T, N] float32 (K cut over blocks); the norm that reads the result
-    sums them in its pass (``add_parts_rms_norm``)."""
+    sums them in its pass (``add_parts_rms_norm``).  To a block that adds what is pending itself it is an addend [T, N] like another:
+    in torch's functions and operators, and those of the stream's tensor, it stands for its sum."""
     __slots__ = ("parts",)
 
     def __init__(self, parts):
         self.parts = parts
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        whole = lambda a: a.resolve() if isinstance(a, ProductParts) else a
+        return func(*(whole(a) for a in args), **{k: whole(a) for k, a in (kwargs or {}).items()})
+
+    def __add__(self, other):
+        return self.resolve() + other
+
+    __radd__ = __add__
+
+    shape = property(lambda self: self.parts.shape[1:])
+    dtype = property(lambda self: self.parts.dtype)
+    device = property(lambda self: self.parts.device)
 
     def resolve(self):
         return self.parts.sum(dim=0)
@@ -576,7 +591,8 @@ class ProductParts:
     def to(self, dtype):
         return self.resolve().to(dtype)
 
-    float = resolve                    # (for a block of another arrangement, which adds what is pending itself)
+    def float(self):
+        return self.resolve()
 
 
 def linear_parts(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor] = None):

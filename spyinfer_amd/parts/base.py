@@ -135,7 +135,8 @@ class Block(Part):
         """(residual stream, pending) -> (residual stream, pending).  ``pending`` is None, an addend [T, H] that
         the next norm sums into the stream (or a pair of addends, from a block whose two sublayers read one norm), or a ``ScaledInput``: then the stream is complete and the input of
         the norm named in it is prepared (a block that cannot use it ignores it).  ``next_norm``: the norm that
-        reads the stream after this block, if the caller knows it; only then may a ``ScaledInput`` be returned."""
+        reads the stream after this block, if the caller knows it; only then may a ``ScaledInput`` be returned, and, if
+        that norm ``takes_product_parts``, an addend in parts (``ops.ProductParts``, which is added like a tensor)."""
         raise NotImplementedError
 
     def entry_norm(self) -> Optional[Norm]:

@@ -22,3 +22,18 @@ def test_a_norm_with_a_sum_of_its_own_gets_none():
     norm = Own(128, 1e-6)
     norm.weight = torch.ones(128)
     assert not norm.takes_product_parts and not getattr(LayerNorm(128, 1e-6), "takes_product_parts", False)
+
+
+def test_parts_are_added_like_a_tensor():
+    """What a block of another arrangement may do with an addend that is pending."""
+    from spyinfer_amd.kernels import ops
+    y = torch.randn((3, 5, 8), generator=torch.Generator().manual_seed(2))
+    parts, stream, total = ops.ProductParts(y), torch.randn((5, 8)), y.sum(0)
+    assert tuple(parts.shape) == (5, 8) and parts.dtype == torch.float32 and parts.device == y.device
+    for out in (stream + parts, parts + stream, torch.add(stream, parts), stream.clone().add_(parts), stream.clone().add_(parts.float()),
+                stream + parts.to(torch.float32)):
+        assert torch.equal(out, stream + total)
+    held = stream.clone()
+    held += parts
+    assert torch.equal(held, stream + total)
+    assert torch.equal(torch.cat([parts.to(torch.float64), total.double()]), torch.cat([total.double(), total.double()]))
