@@ -16,6 +16,7 @@ import torch
 from ..cache.manager import CacheManager
 from ..cache.storage import CacheStorage
 from ..config.registry import load_model_config
+from ..kernels import ops
 from ..models.base import DecoderModel
 from ..weights.loader import load_weights
 from .batch import StepBatch, StepEntry
@@ -35,7 +36,6 @@ def resolve_dtype(name) -> torch.dtype:
 
 def bind_weights(model: DecoderModel, weights, device, weight_copies: str = "both") -> None:
     """``model.bind`` with the engine's choice of the forms in which matrices are kept (EngineConfig.weight_copies)."""
-    from ..kernels import ops
     before = ops.ROW_MAJOR_WEIGHTS
     ops.ROW_MAJOR_WEIGHTS = weight_copies != "tiled"
     try:
@@ -218,7 +218,10 @@ class ModelRunner:
             self._upload(batch, None)
             if token_source is not None:
                 batch.token_ids.copy_(token_source)
-            return self.model.forward(batch, self.storage)
+            if len(self._graphs) >= self.max_graphs:
+                return self.model.forward(batch, self.storage)
+            with ops.replayed_step():            # (the products that the capture will record)
+                return self.model.forward(batch, self.storage)
         _layout, total = batch.layout()
         dev_buf = torch.empty(total, dtype=torch.int32, device=self.device)
         self._upload(batch, dev_buf)
@@ -238,7 +241,7 @@ class ModelRunner:
         collecting = gc.isenabled()
         gc.disable()
         try:
-            with torch.cuda.graph(graph, pool=self._graph_pool):
+            with ops.replayed_step(), torch.cuda.graph(graph, pool=self._graph_pool):
                 logits = self.model.forward(batch, self.storage, out)
         finally:
             if collecting:

@@ -12,8 +12,10 @@ the activations (a tensor stored in 32-bit stays so).
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import functools
+import threading
 from typing import Optional
 
 import torch
@@ -449,7 +451,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
         return decode_linear(x, tiled, out_dtype, out)
     if all_bf16 and tiled is not None and out_dtype == torch.bfloat16 and x.is_contiguous():
-        tiles = rows_product_stored(M, N, K)
+        tiles = rows_product_stored(M, N, K, _step.replayed and not isinstance(w, TiledOnly))      # (whose library product copies the rows first)
         if tiles and (x.data_ptr() | out.data_ptr()) % 16 == 0:
             _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
             hip().call("spy_gemm_rows", _ptr(out), _ptr(x), _ptr(tiled), M, N, K, tiles, 1, ROWS_STORE, 0, _Hip.stream())
@@ -502,6 +504,24 @@ def _rows_product_us(M: int, N: int, K: int, tiles: int, parts: int) -> float:
     return 5.0 + -(-blocks // 256) * -(-K // 128 // parts) * (0.7 + 0.05 * tiles) + parts * M * N * 4 / 2.25e6
 
 
+class _Step(threading.local):
+    replayed = False
+
+
+_step = _Step()
+
+
+@contextlib.contextmanager
+def replayed_step():
+    """What runs inside (on this thread) is a step that is recorded in a graph, or the run of its kernels before the recording, which
+    has to be the same: the host's time for a launch is paid once, and ``rows_product_stored`` leaves it out."""
+    before, _step.replayed = _step.replayed, True
+    try:
+        yield
+    finally:
+        _step.replayed = before
+
+
 @functools.lru_cache(maxsize=1024)
 def rows_product_parts(M: int, N: int, K: int):
     """(row tiles, parts of K) for a product of M rows whose result the next norm sums from its parts (``linear_parts``), or None
@@ -510,7 +530,9 @@ def rows_product_parts(M: int, N: int, K: int):
     the line): 106 / 104; 1356 rows, 4096 x 12288: 137 / 138; 800 rows, 2560 x 4096: 29 / 35, 1100 rows (beyond): 33 / 31; 1356 rows,
     2048 x 6144: 46 / 45; 560 rows, 1024 x 3072: 12.0 / 13.8; K = 2048: 288 rows, 2048 columns: 10.4 / 10.6, 409 rows
     (beyond): 13 / 11; 200 rows, 1024 columns: 7.9 / 8.3 (and a launch costs the host 8 us, the library's product 20: a step of 200
-    tokens, 1024 wide, whose launches bound it: 4.19 -> 3.43 ms)."""
+    tokens, 1024 wide, whose launches bound it: 4.19 -> 3.43 ms).  The line holds without the host too: steps of 129 to 330 decoding
+    requests, replayed from a graph, 12 layers, all products of o and down the library's / K = 2048 and less the library's / by this rule:
+    1024 wide, 140 requests 1164 / 1177 / 1159 us, 2048 wide 1552 / 1482 / 1459, 250 requests 1747 / 1704 / 1679, 4096 wide 2872 / 2652 / 2662."""
     if M <= DECODE_ROWS_PLAIN or N % 16 or K % 128 or K < 2048 or M * N * 4096 > 2.3e6 * K or (K < 3072 and M * N > 6e5) or N * K >= 1 << 30 or M * K >= 1 << 30:
         return None
     fits = [(t, p) for t in range(4, 9) if 16 * t <= M for p in range(1, min(12, K // 256) + 1)
@@ -519,14 +541,16 @@ def rows_product_parts(M: int, N: int, K: int):
 
 
 @functools.lru_cache(maxsize=1024)
-def rows_product_stored(M: int, N: int, K: int) -> int:
+def rows_product_stored(M: int, N: int, K: int, replayed: bool = False) -> int:
     """Row tiles a block of the product of many rows that is stored in bfloat16, or 0 for the library's: a short K, whose few turns
     the wide results' blocks walk while the library's start (us, library / this: 4096 x 1024, 130 rows 8.8 / 10.1, 409 rows 10.3 / 10.8,
     560 rows 13.2 / 10.6, 1356 rows 20.6 / 15.2, 1700 rows 19.9 / 18.2; 6144 x 1024, 409 rows 16.2 / 14.5, 1100 rows 21.3 / 19.1, 1356 rows,
     beyond the line, 23.8 / 26; 4096 x 2048, 409 rows, beyond, 17.0 / 23.5, 560 rows 24.3 / 23.6, 1356 rows 31.0 / 28.4; 6144 x 2048, 1100 rows
-    33.0 / 30.1).  Below 409 rows the steps are bound by their launches, of which the
-    library's costs the host 12 us more."""
-    if M <= DECODE_ROWS_PLAIN or N % 16 or K % 128 or K > 2048 or (K > 1024 and M < 560) or N < 4096 or M * N > 7e6:
+    33.0 / 30.1).  Below 409 rows the steps are bound by their launches, of which the library's costs the host 12 us more (28 layers 1024
+    wide, 130 to 500 tokens: 3.6 ms with the library's qkv, 3.0 with this one).  ``replayed``: a step that is replayed from a graph, where
+    that time is nobody's, takes the library's: 12 layers 1024 wide, 129 / 200 / 330 requests decoding, 1150 / 1320 / 1573 us, with this
+    kernel's qkv 1182 / 1345 / 1588; 4096 x 2048, 640 rows, in a graph 22.3 / 23.9."""
+    if replayed or M <= DECODE_ROWS_PLAIN or N % 16 or K % 128 or K > 2048 or (K > 1024 and M < 560) or N < 4096 or M * N > 7e6:
         return 0
     return min((t for t in range(4, 9) if 16 * t <= M), key=lambda t: _rows_product_us(M, N, K, t, 1))
 

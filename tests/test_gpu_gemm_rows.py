@@ -86,3 +86,52 @@ def test_norm_of_a_sum_of_parts(T, H, parts, dtype):
     close(some, ref[rows.long()], dtype, what="picked rows")
     close(ops.add_parts_rms_norm(stream, ops.ProductParts(y.to(dev)), w.to(dev), 1e-6, dtype), ref, dtype, what="normed sum")
     close(stream, total, torch.float32, what="the stream")
+
+
+def test_rules_of_steps_that_are_replayed(tmp_path, monkeypatch):
+    """140 requests decoding: the step before the capture and the capture ask the rule alike, for a step whose launches the host pays once;
+    a prompt and steps that no graph will hold ask for steps launched one by one."""
+    from spyinfer_amd.engine.batch import StepEntry
+    from spyinfer_amd.engine.runner import ModelRunner, load_model
+    from spyinfer_amd.kernels import ops
+    from spyinfer_amd.weights import write_random_model
+    from tests.configs import INIT, TINY_E
+    dev = require_gpu()
+    asked = []
+    monkeypatch.setattr(ops, "rows_product_stored", lambda M, N, K, replayed: asked.append(replayed) or 0)
+    folder = write_random_model(str(tmp_path / "model"), TINY_E, seed=3, dtype=torch.bfloat16, **INIT)
+    runner = ModelRunner(load_model(folder, "bfloat16", dev), "bfloat16", dev, 16, 200, 140, enforce_eager=False, max_model_len=32)
+    live = [runner.manager.admit("r%d" % i) for i in range(140)]
+
+    def step(tokens):
+        asked.clear()
+        for rc, t in zip(live, tokens):
+            runner.manager.reserve(rc, len(t))
+        return runner.step([StepEntry(rc, t, (len(t) - 1,)) for rc, t in zip(live, tokens)]).clone()
+
+    step([[i % 500, 7] for i in range(140)])
+    assert asked and not any(asked)
+    first = step([[i % 400] for i in range(140)])
+    assert asked and all(asked)
+    outs = []
+    for _ in range(3):
+        for rc in live:
+            assert runner.manager.rewind(rc, 2)
+        outs.append(step([[i % 400] for i in range(140)]))
+        assert all(asked)
+    assert runner.graph_replays == 3 and all(torch.equal(o, first) for o in outs)
+    runner.max_graphs = 1
+    live = live[:139]
+    step([[5]] * 139)
+    assert asked and not any(asked)
+
+
+def test_library_products_of_replayed_steps(monkeypatch):
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    x, w = torch.randn((130, 1024), device=dev).bfloat16(), torch.randn((4096, 1024), device=dev).bfloat16()
+    tiled = ops.tile_weight(w)
+    with ops.replayed_step():
+        assert torch.equal(ops.linear(x, w, tiled=tiled), x @ w.t())
+        monkeypatch.setattr(ops.TiledOnly, "rows", lambda self: pytest.fail("rows copied for the library's product"))
+        close(ops.linear(x, ops.TiledOnly(tiled)), x.double() @ w.double().t(), torch.bfloat16, what="product of a matrix kept in tiles only")

@@ -1,5 +1,6 @@
 """The sizes that go to the products of many rows, and what they are launched with: within what the kernel takes, for every size."""
 import random
+import threading
 
 from spyinfer_amd.kernels import ops
 
@@ -31,3 +32,25 @@ def test_sizes_on_both_sides_of_the_line():
     assert ops.rows_product_gated(200, 6144, 4096, True) == 0
     assert ops.f32_product_parts(611, 1024, 2048) == 3 and ops.f32_product_parts(16, 1024, 2048) is None and ops.f32_product_parts(1500, 2048, 2048) is None
     assert ops.rows_product_stored(409, 4096, 1024) > 0 and ops.rows_product_stored(409, 4096, 2048) == 0 and ops.rows_product_stored(1356, 4096, 2048) > 0 and ops.rows_product_stored(1356, 6144, 1024) == 0
+
+
+def test_replayed_steps_leave_the_host_s_time_out():
+    for size in ((130, 4096, 1024), (409, 6144, 512), (640, 4096, 2048)):
+        assert ops.rows_product_stored(*size) > 0 and ops.rows_product_stored(*size, True) == 0
+
+
+def test_a_replayed_step_is_one_thread_s():
+    seen = []
+    with ops.replayed_step():
+        with ops.replayed_step():
+            pass
+        other = threading.Thread(target=lambda: seen.append(ops._step.replayed))
+        other.start()
+        other.join()
+        seen.append(ops._step.replayed)
+    try:
+        with ops.replayed_step():
+            raise KeyError
+    except KeyError:
+        seen.append(ops._step.replayed)
+    assert seen == [False, True, False]
