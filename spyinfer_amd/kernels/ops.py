@@ -575,15 +575,27 @@ def f32_product_parts(M: int, N: int, K: int):
 @functools.lru_cache(maxsize=1024)
 def rows_product_gated(M: int, N: int, K: int, library: bool) -> int:
     """Row tiles a block of the gated product of many rows (N = 2 I rows of the matrix), or 0 where the library's product and a pass
-    for the activation are the better ones (``library`` false: that way is not at hand at its own price).  It loses where its blocks
-    leave half of the chip idle, but for a short K (us, with the library's activation pass: 409 rows, 6144 x 4096: 44 against 38, 560
-    rows: 44 / 46, 409 rows, 6144 x 1024: 14 / 21), and to the library's larger tiles for the largest products (1700 rows, 24576 x
-    4096: 291 / 284, 1356 rows: 237 / 259; 2011 rows, 19456 x 2560: 171 / 221)."""
+    for the activation are the better ones (``library`` false: that way is not at hand at its own price).  Both ways in steps replayed
+    from a graph, six layers, us a layer that this kernel takes more (+) or less (-) than the library:
+    it loses where blocks of 64 rows x 256 columns leave part of the chip idle, but for a short K, whose walk is soon over: 9728 x 2560, 180
+    rows (114 blocks) + 2.8, 240 rows (152) - 2.5, 6144 x 2560, 409 rows (168) + 2.4, 500 rows (192) - 2.4; with a longer K up to more
+    blocks: 409 rows, 6144 x 4096 (168) + 8.8, 760 rows, 4096 x 4096 (192) + 8.8, 180 rows, 16384 x 3072 (192) - 0.4, 129 rows, 17408 x 5120
+    (204) - 7.3, 561 rows, 6144 x 5120 (216) - 1.8;
+    where compute units have a second block and its rows are few, while the library takes the matrix in one round of larger tiles: 288 rows,
+    24576 x 4096 (480 blocks of four row tiles) + 6.0, 450 rows, 17408 x 5120 (408 of five) + 12.9, 369 rows, 27648 x 5120 (432 of six) +
+    8.9, 409 rows (432 of seven) - 18, 640 rows, 17408 x 5120 (476 of six) - 26 (eager: 18 layers 4096 wide, 320 tokens 4186 us, with the
+    library's 4081);
+    and for the largest products (1700 rows, 24576 x 4096: 291 us, the library's 284, 1356 rows: 237 / 259; 2011 rows, 19456 x 2560: 171 / 221)."""
     if M <= DECODE_ROWS_PLAIN or N % 32 or K % 128 or N * K >= 1 << 30 or M * K >= 1 << 30:
         return 0
-    if library and ((-(-M // 64) * -(-N // 256) < 128 and K > 1024) or (M > 1500 and N * K > 90e6)):
+    few = 0 if K <= 1024 else 128 if K <= 2560 else 200
+    if library and (-(-M // 64) * -(-N // 256) < few or (M > 1500 and N * K > 90e6)):
         return 0
-    return min((t for t in range(4, 9) if 16 * t <= M), key=lambda t: _rows_product_us(M, N, K, t, 1))
+    tiles = min((t for t in range(4, 9) if 16 * t <= M), key=lambda t: _rows_product_us(M, N, K, t, 1))
+    blocks = -(-M // (16 * tiles)) * -(-N // 256)
+    if library and K > 2560 and 256 < blocks <= 512 and blocks * tiles < 2600:
+        return 0
+    return tiles
 
 
 class ProductParts:

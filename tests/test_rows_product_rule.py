@@ -54,3 +54,13 @@ def test_a_replayed_step_is_one_thread_s():
     except KeyError:
         seen.append(ops._step.replayed)
     assert seen == [False, True, False]
+
+
+def test_gated_products_go_to_the_side_that_was_measured_faster():
+    slower = [(180, 9728, 2560), (409, 6144, 4096), (760, 4096, 4096), (240, 8192, 3072), (450, 6144, 5120), (288, 24576, 4096), (320, 24576, 4096),
+              (450, 17408, 5120), (369, 27648, 5120), (561, 16384, 3072)]
+    faster = [(409, 6144, 1024), (240, 9728, 2560), (500, 6144, 2560), (409, 19456, 2560), (1356, 12288, 2048), (561, 6144, 5120), (129, 17408, 5120),
+              (450, 8192, 3072), (240, 24576, 4096), (561, 24576, 4096), (409, 27648, 5120), (640, 17408, 5120), (760, 6144, 4096)]
+    assert [ops.rows_product_gated(*size, True) > 0 for size in slower] == [False] * len(slower)
+    assert [ops.rows_product_gated(*size, True) > 0 for size in faster] == [True] * len(faster)
+    assert all(ops.rows_product_gated(*size, False) > 0 for size in slower + faster)
