@@ -135,3 +135,60 @@ def test_library_products_of_replayed_steps(monkeypatch):
         assert torch.equal(ops.linear(x, w, tiled=tiled), x @ w.t())
         monkeypatch.setattr(ops.TiledOnly, "rows", lambda self: pytest.fail("rows copied for the library's product"))
         close(ops.linear(x, ops.TiledOnly(tiled)), x.double() @ w.double().t(), torch.bfloat16, what="product of a matrix kept in tiles only")
+
+
+@pytest.mark.parametrize("form", ["parts", "stored", "gated"])
+def test_infinities_and_nan_stay_in_their_rows(form, monkeypatch):
+    """A row with NaN and one with infinities, in the rows that the last tile shares with the one before; and a row of the matrix."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    M, N, K = 200, 1056, 384
+    monkeypatch.setattr(ops, "rows_product_parts", lambda *size: (7, 3))
+    monkeypatch.setattr(ops, "rows_product_stored", lambda *size: 7)
+    monkeypatch.setattr(ops, "rows_product_gated", lambda *size: 7)
+    g = torch.Generator().manual_seed(6)
+    x, w = torch.randn((M, K), generator=g).bfloat16(), torch.randn((N, K), generator=g).bfloat16()
+    x[100, 3], x[M - 1, 70], w[N - 1, 200] = float("nan"), float("inf"), float("nan")
+    x, w = x.to(dev), w.to(dev)
+    ref = x.float() @ w.float().t()
+    if form == "parts":
+        got = ops.linear_parts(x, w, ops.tile_weight(w)).resolve()
+    elif form == "stored":
+        got = ops.linear(x, w, tiled=ops.tile_weight(w))
+    else:
+        got = ops.linear_swiglu(x, w, ops.tile_weight(w))
+        ref = ops.swiglu(ref)                                        # (its activation as it is for infinite values)
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+    some = torch.arange(M, device=dev)[~ref[:, 0].isnan() & ~ref[:, 0].isinf()]
+    assert len(some) == M - 2
+    close(got[some, :-1], ref[some, :-1], torch.bfloat16, scale=2.0, what="the other rows")
+
+
+def test_operands_off_16_bytes():
+    """Views that begin between two 16-byte pieces: the kernels that take no such operand are passed by."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+
+    def off(t, n):
+        buf = torch.empty((t.numel() + 8,), dtype=t.dtype, device=dev)[n:n + t.numel()].view(t.shape)
+        return buf.copy_(t)
+
+    g = torch.Generator().manual_seed(8)
+    x, w, small = torch.randn((600, 1024), generator=g), torch.randn((4096, 1024), generator=g) / 32, torch.randn((1024, 2048), generator=g) / 45
+    xb, wb = off(x.bfloat16(), 4), w.bfloat16().to(dev)
+    tiled, ref = ops.tile_weight(wb), x.bfloat16().double() @ w.bfloat16().double().t()
+    assert xb.data_ptr() % 16 and ops.rows_product_stored(600, 4096, 1024) and ops.rows_product_gated(600, 4096, 1024, True)
+    close(ops.linear(xb, wb, tiled=tiled), ref, torch.bfloat16, what="rows off 16 bytes")
+    out = off(torch.zeros((600, 4096)).bfloat16(), 4)
+    assert ops.linear(xb.clone(), wb, tiled=tiled, out=out) is out
+    close(out, ref, torch.bfloat16, what="a result off 16 bytes")
+    close(ops.linear_swiglu(xb, wb, tiled), torch.nn.functional.silu(ref[:, :2048]) * ref[:, 2048:], torch.bfloat16, what="gated, rows off 16 bytes")
+    sb, xs = small.bfloat16().to(dev), torch.randn((200, 2048), generator=g)
+    assert ops.rows_product_parts(200, 1024, 2048)
+    y = ops.linear_parts(off(xs.bfloat16(), 4), sb, ops.tile_weight(sb))
+    close(y, xs.bfloat16().double() @ small.bfloat16().double().t(), torch.bfloat16, what="parts, rows off 16 bytes")
+    assert ops.f32_product_parts(200, 1024, 2048)
+    for x32, w32 in ((off(xs, 1), small.to(dev)), (xs.to(dev), off(small, 1))):
+        close(ops.linear_parts(x32, w32), xs.double() @ small.double().t(), torch.float32, what="float32 off 16 bytes")
+    h = xs[:3].double() @ small.double().t()
+    close(ops.linear_swiglu(off(xs[:3], 1), small.to(dev)), torch.nn.functional.silu(h[:, :512]) * h[:, 512:], torch.float32, what="gated float32 off 16 bytes")

@@ -137,3 +137,22 @@ def test_more_rows_than_offsets_of_31_bits_reach():
     h = torch.einsum("tk,enk->ten", x[at].double(), wgu.double())
     ref = torch.einsum("tef,ekf,te->tk", torch.nn.functional.silu(h[..., :F]) * h[..., F:], wd.double(), w[at].double())
     close(out[at.to(dev)], ref, torch.bfloat16, scale=2.0, what="experts of many rows")
+
+
+@pytest.mark.parametrize("by_groups", [True, False])
+def test_nan_stays_with_its_token(by_groups, monkeypatch):
+    """Rows that do not exist are read as row 0: what it holds stays with its own token."""
+    from spyinfer_amd.kernels import ops
+    monkeypatch.setattr(ops, "experts_by_groups", lambda *sizes: by_groups)
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(13)
+    E, top, K, F = 6, 2, 256, 384
+    ids = rows_for("even", E, top, g).to(dev)
+    T = ids.shape[0]
+    bf = lambda *s, std=1.0: (torch.randn(s, generator=g) * std).bfloat16().to(dev)
+    x, w = bf(T, K), torch.rand((T, top), generator=g).to(dev)
+    mats = [ops.expert_forms([[m] for m in t]) for t in (bf(E, 2 * F, K, std=K ** -0.5), bf(E, K, F, std=F ** -0.5))]
+    ref = ops.moe_experts(x, ids, w, *mats)
+    x[0, 5], x[T - 1, 7] = float("nan"), float("inf")
+    out = ops.moe_experts(x, ids, w, *mats)
+    assert not ref.isnan().any() and out[0].isnan().all() and torch.equal(out[1:-1], ref[1:-1])
