@@ -1,12 +1,14 @@
 // C[M, N] = A[M, K] . W[N, K]^T in float32: products and sums of 32-bit numbers, no reduced-precision mode (the matrix cores'
-// float32 instructions multiply and add as fmaf does).  Three kernels by the number of rows:
+// float32 instructions multiply and add as fmaf does; gemm_f32_split.hip, which has most products of more than 32 rows, cuts the
+// numbers without loss).  Three kernels by the number of rows:
 //
 //   few    (up to 4 or 8 rows)   bound by streaming W from memory.  A wave owns NR rows of W and walks K with 64 lanes side by side, so
 //                           that every load of W is 1 KiB in one piece; A comes from the caches; the lanes' sums meet at the end.
 //   narrow (tens of rows)   bound by W from memory as well, but A's rows would be read once per row of W by the kernel above.
 //                           A block owns 16 rows of W and MT tiles of 16 rows of A; its eight waves take the chunks of 64 of K in
 //                           turn, operands straight from memory into v_mfma_f32_16x16x4_f32 registers, and add through LDS.
-//   tile   (many rows)      bound by the matrix cores (256 flops a cycle and compute unit).  Tiles of A and W through LDS.
+//   tile   (many rows that gemm_f32_split.hip does not take)      bound by the matrix cores (256 flops a cycle and compute unit).  Tiles of
+//                           A and W through LDS.
 //
 // Which kernel, how many row tiles a block and how many parts of K follow the number of rows, and with them the order of a row's sums: a
 // row in a step of other sizes is the same within rounding, not bit for bit (as it is from gemm_generic.hip).
@@ -364,6 +366,7 @@ int gemm_f32(const float* A, const float* W, float* C, int M, int N, int K, hipS
 #define GF_NARROW(MT) gemm_f32_narrow_kernel<MT><<<dim3(tiles16, (M + 16 * MT - 1) / (16 * MT)), GF_WAVES * 64, 0, st>>>(A, W, C, M, N, K)
 #define GF_TILE(KS) gemm_f32_tile_kernel<KS><<<((tm * tn + 7) / 8) * 8, 256 * KS, 0, st>>>(A, W, C, M, N, K, tm, tn, 1)
     const int tiles16 = (N + 15) / 16, tm = (M + 63) / 64, tn = (N + 63) / 64;
+    if (gemm_f32_split_takes(M, N, K, 1)) return gemm_f32_split(A, W, C, M, N, K, 1, st);
     if (M <= 4 || (M <= 8 && N <= 1024)) {
         // Rows of W per wave: each more reads A once less, but takes waves away.  One up to 2048 rows of W (four rows of A, 2048 x
         // 2048: 7.3 us against 7.4 with two, 9.8 with four), four from 12288 on (29.9 / 25.1 / 23.8 us for 12288 x 2048); with one
@@ -394,11 +397,13 @@ int gemm_f32(const float* A, const float* W, float* C, int M, int N, int K, hipS
     return 0;
 }
 
-// act(A . Wgate^T) * (A . Wup^T) for up to four rows, W = [gate rows | up rows] of N each, without the [M][2 N] result in between.
+// act(A . Wgate^T) * (A . Wup^T) for up to four rows and for those that gemm_f32_split.hip takes, W = [gate rows | up rows] of N each, without the [M][2 N] result in between.
 extern "C" int spy_gemm_f32_gated(float* C, const float* A, const float* W, int M, int N, int K, int act_code, hipStream_t st) {
     GateAct act;
-    SPY_REQUIRE(M > 0 && M <= 4 && N > 0 && K > 0 && gate_act_of(act_code, &act), "spy_gemm_f32_gated: %d rows, activation %d", M, act_code);
+    SPY_REQUIRE(M > 0 && N > 0 && K > 0 && gate_act_of(act_code, &act), "spy_gemm_f32_gated: %d rows, activation %d", M, act_code);
     SPY_REQUIRE(gemm_f32_takes(A, W, C, M, N, K), "spy_gemm_f32_gated: operands of %d x %d x %d are not taken", M, N, K);
+    SPY_REQUIRE(M <= 4 || (N < (1 << 30) && gemm_f32_split_takes(M, 2 * N, K, 1)), "spy_gemm_f32_gated: %d rows of %d x %d are not taken", M, N, K);
+    if (M > 4) return gemm_f32_split_gated(A, W, C, M, 2 * N, K, act, st);
 #define GF_GATED(MR, U) gemm_f32_few_kernel<MR, 2, U, true><<<(N + 3) / 4, 256, 0, st>>>(A, W, C, M, N, K, act)
     if (M == 1) GF_GATED(1, 4); else if (M == 2) GF_GATED(2, 2); else GF_GATED(4, 2);
 #undef GF_GATED
@@ -409,11 +414,12 @@ extern "C" int spy_gemm_f32_gated(float* C, const float* A, const float* W, int 
 // A [M, K] . W [N, K]^T in parts of K: C [parts][M][N], a block a tile of one part, which the reader sums (spy_add_parts_rmsnorm).  For
 // results whose tiles fill no whole number of rounds of the chip (or of which there are too few even for that: the narrow kernel above
 // reads half lines of W).  Parts beat groups of a block's waves, which leave the other compute units idle.  Measured, us, the
-// kernels above / this one and what the sum adds to the norm's pass: 611 rows, 1024 x 2048 43.4 / 33.8 + 2; 1024 x 3072 62.6 / 44.6 + 5; 2048
-// x 6144 223 / 145 + 5; 65 rows, 2048 x 6144 62 / 35 + 2; 17 rows, 2560 x 4096 29 / 18.5 + 1.
+// kernels above / this one and what the sum adds to the norm's pass: 17 rows, 2560 x 4096 29 / 18.5 + 1; with gemm_f32_split.hip's blocks: 611
+// rows, 1024 x 2048 43 / 21.4 + 2, 1024 x 3072 63 / 28 + 5; 90 rows, 2048 x 2048 22 / 12.6 + 1.
 extern "C" int spy_gemm_f32_parts(float* C, const float* A, const float* W, int M, int N, int K, int parts, hipStream_t st) {
     SPY_REQUIRE(M > 0 && N > 0 && K > 0 && parts >= 1 && parts <= (K + GF_BK - 1) / GF_BK, "spy_gemm_f32_parts: %d parts of %d x %d x %d", parts, M, N, K);
     SPY_REQUIRE(gemm_f32_takes(A, W, C, M, N, K), "spy_gemm_f32_parts: operands of %d x %d x %d are not taken", M, N, K);
+    if (parts <= K / GF_BK && gemm_f32_split_takes(M, N, K, parts)) return gemm_f32_split(A, W, C, M, N, K, parts, st);
     const int tm = (M + 63) / 64, tn = (N + 63) / 64;
     const int64_t blocks = (int64_t)tm * tn * parts;
     SPY_REQUIRE(blocks < (1 << 28), "spy_gemm_f32_parts: too many blocks");

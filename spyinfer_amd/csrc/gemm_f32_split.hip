@@ -1,0 +1,274 @@
+// Products of many float32 rows, C[M, N] = A[M, K] . W[N, K]^T, on the matrix cores' bfloat16 instructions, which multiply sixteen times
+// as much in a cycle as their float32 ones do.  Every value is cut into three bfloat16 parts, x = high + middle + low, exactly (8 + 8 + 8
+// bits, each part the rounded rest of those before it), a product of two parts is exact in float32, and of the nine products of parts
+// the six from 2^-18 of the result on are formed: high high apart, high middle, middle high, middle middle, high low and low high
+// in a second sum; what is left out is below 2^-26 of |a||w|, a quarter of one rounding in float32.  Relative errors against 64 bits (2-norm, normal
+// values): K = 1024 1.9e-7, K = 2048 2.7e-7, in parts less; the float32 instructions' 2.9e-7 (gemm_f32.hip, whose chain ends every 256 of K).
+// GATED: W = [gate rows | up rows], C[M][N / 2] = act(gate) * up.
+//
+// A block splits its rows of A and W as it stages them: from memory into registers four steps of 32 of K ahead, from there as three planes
+// in operand order into the other of two LDS stages, while this step's products run.  128 x 128 values of C and eight waves
+// (two a SIMD, one block a compute unit) where the tiles fill the chip, else 64 x 64 and four waves, two blocks a compute unit.
+// What bounds it: a step of the large tile is 1536 cycles of products a SIMD and about 700 of the split (5.5 instructions a value), of which
+// the matrix cores' work hides less than half; it takes 1.0 us.  The split by v_dot2_f32_bf16 (3.5 instructions a value) was slower beside
+// MFMAs, and loads two steps ahead cost a third of the time (1.25 us).
+// Measured, us, gemm_f32.hip's float32 instructions / this: 611 rows, 4096 x 1024 67 / 44, 6144 x 1024 87 / 49 (157 TFLOP/s), 1024 x 3072 in
+// parts 44 / 28; 200 rows, 12288 x 2048 124 / 78, 2048 x 6144 in parts 61 / 38; 90 rows, 12288 x 2048 81 / 57.
+#include "gemm_f32.h"
+
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float gs_f32x4_t;
+typedef __attribute__((__vector_size__(16 * sizeof(float)))) float gs_f32x16_t;
+typedef __bf16 gs_bf16x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 gs_bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t gs_u32x4_t;
+
+#define GS_BK 32
+#define GS_PIECE 576          // bytes of 32 rows of 8 values of K in one plane, 64 of them unused
+#define GS_GROUP (4 * GS_PIECE)
+
+// x = high + middle + low, each a bfloat16, exactly; two values at a time
+__device__ __forceinline__ void gs_split(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = pack_bf16x2(x0, x1);
+    x0 -= __uint_as_float(h << 16);
+    x1 -= __uint_as_float(h & 0xffff0000u);
+    m = pack_bf16x2(x0, x1);
+    x0 -= __uint_as_float(m << 16);
+    x1 -= __uint_as_float(m & 0xffff0000u);
+    l = pack_bf16x2(x0, x1);
+}
+
+template <int BM, int BN, int WM, int WN, bool GATED>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
+                                                                      int M, int N, int K, int tiles_m, int tiles_n, int parts, GateAct act) {
+    constexpr int T = 64 * WM * WN, MT = BM / WM / 32, NT = BN / WN / 32, ROWS = T / 4, P = (BM + BN) / ROWS;
+    constexpr int PLANE = (BM + BN) / 32 * GS_GROUP, STAGE = 3 * PLANE;
+    static_assert(BM % ROWS == 0 && BN % ROWS == 0, "a thread's piece is of A or of W for the whole block");
+    __shared__ __align__(16) char lds[2 * STAGE];
+    const int tiles = tiles_m * tiles_n, total = tiles * parts, per = (total + 7) >> 3;
+    const int at = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || at >= total) return;
+    const int tile = at % tiles, k_part = at / tiles;
+    C += (size_t)k_part * M * N;                       // (parts are of the product alone, not of a gated one)
+    const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int i = lane & 31, h = lane >> 5;
+    const int wm = wave % WM, wn = wave / WM;
+    // W's row in place `at` of the block's BN (one that does not exist reads the last; nothing is stored).  GATED: of 32 places 16 are gate
+    // rows and 16 the up rows of the same columns, so that a lane has both values of a column
+    auto w_row = [&](int at) {
+        if (!GATED) return min(n0 + at, N - 1);
+        return min(n0 / 2 + (at >> 5) * 16 + (at & 15), N / 2 - 1) + ((at & 16) ? N / 2 : 0);
+    };
+    // staging: thread t has eight values of rows t / 4, t / 4 + ROWS, ...; four threads read 128 bytes of one row
+    const int sr = tid >> 2, kp = tid & 3;
+    const auto ares = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, M * K * 4, 0x00020000);
+    const auto wres = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, N * K * 4, 0x00020000);
+    int src[P], dst[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int row = sr + p * ROWS;
+        src[p] = ((p * ROWS < BM ? min(m0 + row, M - 1) : w_row(row - BM)) * K + kp * 8) * 4;
+        dst[p] = (row >> 5) * GS_GROUP + kp * GS_PIECE + (row & 31) * 16;
+    }
+    const int all_steps = K / GS_BK, step0 = (int)((long long)all_steps * k_part / parts);
+    const int steps = (int)((long long)all_steps * (k_part + 1) / parts) - step0;
+    struct Pieces { gs_f32x4_t v[P][2]; };
+    auto fetch = [&](Pieces& f, int s) {
+        const int k = (step0 + min(s, steps - 1)) * GS_BK * 4;
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                f.v[p][e] = __builtin_bit_cast(gs_f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(p * ROWS < BM ? ares : wres, src[p] + 16 * e, k, 0));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto stage = [&](Pieces& f, int s) {
+        char* to = lds + (s & 1) * STAGE;
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            gs_u32x4_t hi, mid, lo;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                uint32_t a, b, c;
+                gs_split(f.v[p][e >> 1][(e & 1) * 2], f.v[p][e >> 1][(e & 1) * 2 + 1], a, b, c);
+                hi[e] = a; mid[e] = b; lo[e] = c;
+            }
+            *reinterpret_cast<gs_u32x4_t*>(to + dst[p]) = hi;
+            *reinterpret_cast<gs_u32x4_t*>(to + dst[p] + PLANE) = mid;
+            *reinterpret_cast<gs_u32x4_t*>(to + dst[p] + 2 * PLANE) = lo;
+        }
+    };
+    constexpr bool FOLD = NT * MT == 1;
+    gs_f32x16_t big[NT][MT], small[NT][MT], sum;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sum[e] = 0.f;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) big[n][m][e] = small[n][m][e] = 0.f;
+    auto products = [&](int s) {
+        const char* from = lds + (s & 1) * STAGE + h * GS_PIECE + i * 16;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            gs_bf16x8_t a[MT][3], w[NT][3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m) a[m][q] = *reinterpret_cast<const gs_bf16x8_t*>(from + (wm * MT + m) * GS_GROUP + ks * 2 * GS_PIECE + q * PLANE);
+#pragma unroll
+                for (int n = 0; n < NT; ++n) w[n][q] = *reinterpret_cast<const gs_bf16x8_t*>(from + (BM / 32 + wn * NT + n) * GS_GROUP + ks * 2 * GS_PIECE + q * PLANE);
+            }
+#define GS_MFMA(SUM, WQ, AQ)                                                                                                     \
+    _Pragma("unroll") for (int n = 0; n < NT; ++n) _Pragma("unroll") for (int m = 0; m < MT; ++m)                                \
+        SUM[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[n][WQ], a[m][AQ], SUM[n][m], 0, 0, 0);
+            GS_MFMA(big, 0, 0)
+            GS_MFMA(small, 0, 1)
+            GS_MFMA(small, 1, 0)
+            GS_MFMA(small, 1, 1)
+            GS_MFMA(small, 0, 2)
+            GS_MFMA(small, 2, 0)
+        }
+    };
+    Pieces f0, f1, f2, f3;
+    fetch(f0, 0);
+    fetch(f1, 1);
+    fetch(f2, 2);
+    fetch(f3, 3);
+    stage(f0, 0);
+    __syncthreads();
+    // step s runs from LDS stage s & 1; behind it the pieces of step s + 1 are split into the other one
+    int s = 0;
+#define GS_STEP(FREE, NEXT, S)        \
+    fetch(FREE, (S) + 4);             \
+    products(S);                      \
+    stage(NEXT, (S) + 1);             \
+    __builtin_amdgcn_sched_barrier(0);\
+    __syncthreads();
+    for (; s + 4 < steps; s += 4) {
+        GS_STEP(f0, f1, s)
+        GS_STEP(f1, f2, s + 1)
+        GS_STEP(f2, f3, s + 2)
+        GS_STEP(f3, f0, s + 3)
+        if (FOLD && (s & 28) == 28) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                sum[e] += big[0][0][e];
+                big[0][0][e] = 0.f;
+            }
+        }
+    }
+    products(s);
+    if (s + 1 < steps) {
+        stage(f1, s + 1);
+        __syncthreads();
+        products(s + 1);
+    }
+    if (s + 2 < steps) {
+        stage(f2, s + 2);
+        __syncthreads();
+        products(s + 2);
+    }
+    if (s + 3 < steps) {
+        stage(f3, s + 3);
+        __syncthreads();
+        products(s + 3);
+    }
+    // A value beyond bfloat16's range, an infinity or a NaN does not split (its rest is a NaN): every sum that it is in is a NaN then
+    bool bad = false;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                big[n][m][e] += FOLD ? small[n][m][e] + sum[e] : small[n][m][e];
+                bad |= !(fabsf(big[n][m][e]) < INFINITY);
+            }
+    if (__any(bad)) {
+        // the wave's values once more by float32 instructions
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const float* a_at = A + (size_t)min(m0 + (wm * MT + m) * 32 + i, M - 1) * K;
+                const float* w_at = W + (size_t)w_row((wn * NT + n) * 32 + i) * K;
+                gs_f32x16_t acc;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+                for (int k = step0 * GS_BK; k < (step0 + steps) * GS_BK; k += 8) {
+                    const gs_f32x4_t va = *reinterpret_cast<const gs_f32x4_t*>(a_at + k + 4 * h), vw = *reinterpret_cast<const gs_f32x4_t*>(w_at + k + 4 * h);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(vw[j], va[j], acc, 0, 0, 0);
+                }
+                big[n][m] = acc;
+            }
+    }
+    // lane (i, h) has C[row i][columns 8 q + 4 h .. + 3], q < 4; GATED: gate values at q < 2, the same columns' up values at q + 2
+    const int width = GATED ? N / 2 : N;
+    const bool whole = (width & 3) == 0;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int row = m0 + (wm * MT + m) * 32 + i;
+        if (row >= M) continue;
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int q = 0; q < (GATED ? 2 : 4); ++q) {
+                const int col = (GATED ? n0 / 2 + (wn * NT + n) * 16 : n0 + (wn * NT + n) * 32) + 8 * q + 4 * h;
+                float* to = C + (size_t)row * width + col;
+                gs_f32x4_t y;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[e] = GATED ? gated_value(act, big[n][m][4 * q + e], big[n][m][4 * (q + 2) % 16 + e]) : big[n][m][4 * q + e];
+                if (whole) {
+                    if (col < width) *reinterpret_cast<gs_f32x4_t*>(to) = y;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (col + e < width) to[e] = y[e];
+                }
+            }
+    }
+}
+
+// ---- dispatch --------------------------------------------------------------------------------------------------------------
+// Estimated time of both tiles, fitted to 120 launches of 40 to 611 rows, K of 1024 to 6144 and 1 to 12 parts: a compute unit takes 0.9 us for a
+// step of a large block (1.03 with the chip full), 0.5 us for one small block, 0.83 for two, 1.0 with the chip full.  (611 rows: 4096 x
+// 1024, 160 large or 640 small blocks 44 / 49 us, 1024 x 2048, 40 or 160 blocks 68 / 36; 400 rows, 4096 x 2048, 128 or 448: 69 / 58.)  A chain of
+// products of the large tile is the part's whole K, which to 2048 rounds no more than the float32 instructions do; the small tile's
+// sums change every 1024.
+static bool gs_large_tile(int M, int N, int K, int parts) {
+    const int64_t large = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * parts, small = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * parts;
+    const double steps = (double)K / GS_BK / parts, rest = small % 512 == 0 ? 0.0 : (small % 512 <= 256 ? 0.5 : 0.83);
+    return K / parts <= 2048
+        && 8.0 + steps * (double)((large + 255) / 256) * (0.9 + 0.13 * (large < 256 ? large / 256.0 : 1.0)) <= 5.0 + steps * ((double)(small / 512) + rest);
+}
+
+// More than 32 rows (below, the products are bound by W's way from memory: 24 rows, 4096 x 1024 8.7 us / 18.7), and without parts tiles
+// for half of the compute units (2048 x 2048, 90 rows: 64 tiles 22 / 33; 4096 x 2048: 128 tiles 40 / 35).
+bool gemm_f32_split_takes(int M, int N, int K, int parts) {
+    return M > 32 && K % GS_BK == 0 && (int64_t)M * K < (1 << 29) && (int64_t)N * K < (1 << 29)
+        && (parts > 1 || (int64_t)((M + 63) / 64) * ((N + 63) / 64) >= 128);
+}
+
+template <int BM, int BN, int WM, int WN, bool GATED>
+static int gs_launch(const float* A, const float* W, float* C, int M, int N, int K, int parts, GateAct act, hipStream_t st) {
+    const int tm = (M + BM - 1) / BM, tn = (N + BN - 1) / BN;
+    const int64_t blocks = (int64_t)tm * tn * parts;
+    SPY_REQUIRE(parts >= 1 && parts <= K / GS_BK && blocks < (1 << 28), "spy_gemm (float32): %d parts of %d x %d x %d", parts, M, N, K);
+    gemm_f32_split_kernel<BM, BN, WM, WN, GATED><<<(unsigned)((blocks + 7) / 8 * 8), 64 * WM * WN, 0, st>>>(A, W, C, M, N, K, tm, tn, parts, act);
+    SPY_CHECK_LAUNCH("spy_gemm (float32)");
+    return 0;
+}
+
+int gemm_f32_split(const float* A, const float* W, float* C, int M, int N, int K, int parts, hipStream_t st) {
+    const GateAct none = {1.f, 0.f};
+    return gs_large_tile(M, N, K, parts) ? gs_launch<128, 128, 2, 4, false>(A, W, C, M, N, K, parts, none, st)
+                                         : gs_launch<64, 64, 2, 2, false>(A, W, C, M, N, K, parts, none, st);
+}
+
+int gemm_f32_split_gated(const float* A, const float* W, float* C, int M, int N, int K, GateAct act, hipStream_t st) {
+    return gs_large_tile(M, N, K, 1) ? gs_launch<128, 128, 2, 4, true>(A, W, C, M, N, K, 1, act, st)
+                                     : gs_launch<64, 64, 2, 2, true>(A, W, C, M, N, K, 1, act, st);
+}

@@ -555,20 +555,38 @@ def rows_product_stored(M: int, N: int, K: int, replayed: bool = False) -> int:
     return min((t for t in range(4, 9) if 16 * t <= M), key=lambda t: _rows_product_us(M, N, K, t, 1))
 
 
+def f32_rows_split(M: int, N: int, K: int, parts: int = 1) -> bool:
+    """Whether a float32 product goes through the kernel that cuts its values into bfloat16 parts (csrc/gemm_f32_split.hip, whose own
+    rule this is)."""
+    return M > 32 and K % 32 == 0 and M * K < 1 << 29 and N * K < 1 << 29 and (parts > 1 or -(-M // 64) * -(-N // 64) >= 128)
+
+
 @functools.lru_cache(maxsize=1024)
 def f32_product_parts(M: int, N: int, K: int):
     """Parts of K for a float32 product whose result the next norm sums from them, or None where one pass is the better one.  A part of a
-    tile of 64 x 64 is a block; the numbers are fitted to 380 launches of 17 to 2048 rows (the choice is 0.13 % behind the best on average,
-    6 % at most, the parts' sum counted), and up to 16 rows the streaming kernel stands."""
+    tile is a block: of 64 x 64 by the float32 instructions, its numbers fitted to 380 launches of 17 to 2048 rows (the choice is 0.13 % behind
+    the best on average, 6 % at most, the parts' sum counted; up to 16 rows the streaming kernel stands); of 128 x 128 (to 2048 of K) or 64 x
+    64 by the kernel that splits values, with the estimate that it chooses its tile by.  Of its numbers of parts the smallest within 6 % of the
+    best, which the estimate does not tell apart (611 rows, 1024 x 2048, with the sum: three parts 25.7 us, six 25.0)."""
     if M <= 16 or K % 4 or -(-M // 64) * -(-N // 64) >= 1 << 20:
         return None
-    tiles = -(-M // 64) * -(-N // 64)
+    tiles, large = -(-M // 64) * -(-N // 64), -(-M // 128) * -(-N // 128)
 
     def us(p):
         total = p * M * N * 4
-        return -(-tiles * p // 256) * (K / p) * 0.0178 + (K / p) * 0.0066 + total / 8e6 + (total / 4.5e6 + 0.3 if p > 1 else 0.0)
+        if f32_rows_split(M, N, K, p):
+            rest = tiles * p % 512
+            time = 5.0 + K / 32 / p * (tiles * p // 512 + (0.0 if rest == 0 else 0.5 if rest <= 256 else 0.83))
+            if K // p <= 2048:
+                time = min(time, 8.0 + K / 32 / p * -(-large * p // 256) * (0.9 + 0.13 * min(1.0, large * p / 256)))
+        else:
+            time = -(-tiles * p // 256) * (K / p) * 0.0178 + (K / p) * 0.0066
+        return time + total / 8e6 + (total / 4.5e6 + 0.3 if p > 1 else 0.0)
 
-    best = min((p for p in (1, 2, 3, 4, 5, 6, 8, 12) if p == 1 or (K // 32 // p >= 4 and tiles * p <= 1400 and p * M * N * 4 <= PARTS_MAX_BYTES)), key=us)
+    fits = [p for p in (1, 2, 3, 4, 5, 6, 8, 12) if p == 1 or (K // 32 // p >= 4 and tiles * p <= 1400 and p * M * N * 4 <= PARTS_MAX_BYTES)]
+    best = min(fits, key=us)
+    if f32_rows_split(M, N, K, 2):
+        best = next(p for p in fits if us(p) <= 1.06 * us(best))
     return best if best > 1 else None
 
 
@@ -698,8 +716,8 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, tiled: Optional[torc
         hip().call("spy_gemm_skinny_swiglu", _ptr(x), _ptr(w_gate_up), _ptr(out), _code(out, "out"), ctypes.c_int(M),
                    ctypes.c_int(I), ctypes.c_int(K), ctypes.c_int(GATED_ACTIVATIONS[activation]), _Hip.stream())
         return out
-    if 0 < M <= 4 and x.dtype == torch.float32 and x.is_cuda and isinstance(w_gate_up, torch.Tensor) and w_gate_up.dtype == torch.float32 and K % 4 == 0 \
-            and x.is_contiguous() and w_gate_up.is_contiguous() and (x.data_ptr() | w_gate_up.data_ptr()) % 16 == 0:
+    if x.dtype == torch.float32 and (0 < M <= 4 or f32_rows_split(M, 2 * I, K)) and x.is_cuda and isinstance(w_gate_up, torch.Tensor) \
+            and w_gate_up.dtype == torch.float32 and K % 4 == 0 and x.is_contiguous() and w_gate_up.is_contiguous() and (x.data_ptr() | w_gate_up.data_ptr()) % 16 == 0:
         out = torch.empty((M, I), dtype=x.dtype, device=x.device)
         hip().call("spy_gemm_f32_gated", _ptr(out), _ptr(x), _ptr(w_gate_up), M, I, K, GATED_ACTIVATIONS[activation], _Hip.stream())
         return out

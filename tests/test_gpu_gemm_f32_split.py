@@ -1,0 +1,87 @@
+"""Float32 products whose values are cut into bfloat16 parts (csrc/gemm_f32_split.hip) against 64 bits: both tiles at their edges, one step
+of 32 of K to more than the loads run ahead, parts of uneven length, the gated product, values that cannot be cut."""
+import pytest
+import torch
+
+from tests.gpu_util import require_gpu
+
+pytestmark = pytest.mark.gpu
+
+# (M, N, K): the small tile, the large one, columns that are multiples of nothing
+SHAPES = [(33, 8192, 32), (64, 8130, 64), (65, 4097, 96), (129, 5441, 128), (130, 8190, 160), (257, 2052, 192), (611, 1030, 224), (385, 1283, 1024),
+          (640, 5377, 288), (1030, 4100, 256), (300, 1700, 4160)]
+
+
+def operands(M, N, K, dev):
+    g = torch.Generator().manual_seed(M + 3 * N + 7 * K)
+    # (values of many sizes: each by a power of two of its own)
+    x, w = (torch.randn((n, K), generator=g) * torch.exp2(torch.randint(-8, 8, (n, K), generator=g).float()) for n in (M, N))
+    return x.to(dev), w.to(dev)
+
+
+def bound(x, w):
+    # what is left out of a product of two values is below 2^-26 of it; a chain rounds once or twice for sixteen of K, and there are at most
+    # 2048 / 16 of them before the sums' sums
+    return (2.0 ** -26 + (2 * 128 + 16) * 2.0 ** -24) * (x.double().abs() @ w.double().abs().t())
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_product(M, N, K):
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    assert ops.f32_rows_split(M, N, K)
+    x, w = operands(M, N, K, dev)
+    held = torch.full((M * N + 4096,), float("nan"), device=dev)          # what lies behind the result stays as it is
+    out = ops.linear(x, w, out=held[:M * N].view(M, N))
+    assert bool(((out.double() - x.double() @ w.double().t()).abs() <= bound(x, w)).all())
+    assert bool(held[M * N:].isnan().all())
+
+
+@pytest.mark.parametrize("M,N,K,parts", [(33, 70, 64, 2), (129, 130, 416, 3), (200, 2048, 1056, 12), (611, 1030, 1120, 5), (300, 3000, 2048, 2)])
+def test_parts(M, N, K, parts, monkeypatch):
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    monkeypatch.setattr(ops, "f32_product_parts", lambda *size: parts)
+    x, w = operands(M, N, K, dev)
+    out = ops.linear_parts(x, w).parts
+    for p in range(parts):
+        a, b = K // 32 * p // parts * 32, K // 32 * (p + 1) // parts * 32
+        assert bool(((out[p].double() - x[:, a:b].double() @ w[:, a:b].double().t()).abs() <= bound(x[:, a:b], w[:, a:b])).all())
+
+
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("M,I,K", [(33, 4096, 32), (65, 2050, 160), (200, 6111, 96), (611, 3072, 1024)])
+def test_gated(M, I, K, activation):
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    x, w = operands(M, 2 * I, K, dev)
+    x, w = x / 16, w / (16 * K ** 0.5)
+    h, err = x.double() @ w.double().t(), bound(x, w)
+    act = torch.nn.functional.silu if activation == "silu" else lambda z: torch.nn.functional.gelu(z, approximate="tanh")
+    out = ops.linear_swiglu(x, w, activation=activation)
+    a, up = act(h[:, :I]), h[:, I:]
+    # (both activations' slopes are below 1.13; the activation itself is a handful of roundings)
+    limit = 1.13 * err[:, :I] * (up.abs() + err[:, I:]) + a.abs() * err[:, I:] + 16 * 2.0 ** -24 * (h[:, :I] * up).abs() + 1e-30
+    assert bool(((out.double() - a * up).abs() <= limit).all())
+
+
+@pytest.mark.parametrize("M,N", [(65, 5000), (600, 5000)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_values_that_cannot_be_cut(M, N, gated):
+    """Infinities, NaN and values that bfloat16 rounds to infinity: the rows and columns they stand in are what float32 arithmetic makes of
+    them, all others as ever."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    x, w = torch.ones((M, 96), device=dev), torch.ones((N, 96), device=dev)
+    x[M - 1, 3], x[M - 2, 70], x[5, 1] = float("inf"), float("nan"), 3.4e38
+    w[N - 1, 7], w[0, 95], w[64] = float("nan"), float("-inf"), 1e-38
+    x[5, 2], w[9, 1] = -3.4e38, -1.0
+    want = (x.double() @ w.double().t()).float()
+    if gated:
+        out, want = ops.linear_swiglu(x, w), ops.swiglu(want)          # (the activation of infinities is the activation pass's)
+    else:
+        out = ops.linear(x, w)
+    finite = want.isfinite()
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out[want.isinf()], want[want.isinf()])
+    # (96 values of up to 3.4e38 that cancel but for a rounding of the largest)
+    assert bool(((out - want).abs() <= 96 * 2.0 ** -24 * (x.abs().double() @ w.abs().double().t()).float()[:, :want.shape[1]].clamp(min=1.0))[finite].all())

@@ -64,3 +64,14 @@ def test_gated_products_go_to_the_side_that_was_measured_faster():
     assert [ops.rows_product_gated(*size, True) > 0 for size in slower] == [False] * len(slower)
     assert [ops.rows_product_gated(*size, True) > 0 for size in faster] == [True] * len(faster)
     assert all(ops.rows_product_gated(*size, False) > 0 for size in slower + faster)
+
+
+def test_float32_products_in_parts_that_split_values():
+    rng = random.Random(5)
+    for _ in range(2000):
+        M, N, K = int(2 ** rng.uniform(0, 12)), 4 * rng.randint(1, 4000), 32 * rng.randint(1, 400)
+        parts = ops.f32_product_parts.__wrapped__(M, N, K)
+        assert parts is None or (2 <= parts <= K // 128 and parts * M * N * 4 <= ops.PARTS_MAX_BYTES)
+    assert ops.f32_rows_split(33, 8192, 1024) and not ops.f32_rows_split(32, 8192, 1024) and not ops.f32_rows_split(90, 4032, 1024)
+    assert ops.f32_rows_split(90, 1024, 1024, 2) and not ops.f32_rows_split(600, 8192, 1000)
+    assert ops.f32_product_parts(611, 1024, 3072) == 6 and ops.f32_product_parts(90, 2048, 2048) == 4
