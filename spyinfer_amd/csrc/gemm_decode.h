@@ -44,13 +44,13 @@ __device__ __forceinline__ void gd_ss_share(const float* __restrict__ ss_in, int
 // The residual epilogue for one lane's four columns n .. n + 3 of row m: h = h_old + v goes back to the stream (float32),
 // bf16(h * w_next) to the next product's input (row-major, or in operand order for MT row tiles), and the four lanes of
 // a row add their shares of sum(h^2); lane group 0 writes the row's part to ss_part_row[m].  Rows beyond M write nothing
-// to the stream and the part 0.  wn: the next norm's weight for the four columns, two bfloat16 per word.
+// to the stream and the part 0, as do lanes that have no columns (mine false).  wn: the next norm's weight for the four columns, two bfloat16 per word.
 template <bool OT>
 __device__ __forceinline__ void gd_residual_epilogue(const f32x4_t& v, const f32x4_t& h_old, uint2 wn, float* __restrict__ resid_out,
                                                      bf16_t* __restrict__ xw_out, float* __restrict__ ss_part_row, int m, int n, int g,
-                                                     int M, int N, int MT) {
+                                                     int M, int N, int MT, bool mine = true) {
     float s = 0.f;
-    if (m < M) {
+    if (m < M && mine) {
         f32x4_t h = h_old;
 #pragma unroll
         for (int i = 0; i < 4; ++i) { h[i] += v[i]; s += h[i] * h[i]; }
@@ -70,6 +70,7 @@ struct GdArgs {
     int n_parts; float eps; int M, N, K; bool xt, ot; hipStream_t st;
     GateAct act;                           // the gated epilogue's activation
     void* ws; long long ws_bytes;          // the device's workspace of the products that split K over blocks (or none)
+    bool half_parts = false;               // the residual product by blocks of half a column tile, N / 8 parts of the sums of squares
 };
 
 // Compute units of the current device (asked for once per device).

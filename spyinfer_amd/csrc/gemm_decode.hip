@@ -35,14 +35,19 @@ constexpr int GD_WAVES_GATED = 4;     // waves of a block of the gated product w
 // block half of the units stream two tiles and the others one.  A half tile is the lanes r < 8 (or r >= 8) of every
 // fragment of W, 128 bytes in one piece each, and the columns 4 g + i of the lane groups g < 2 (g >= 2) of the result.
 // The stored product only.
-// HT: 0, or the number of half tiles of a block, 3 or 5 (two and a half tiles per unit: qkv of 10240 columns).
-template <int EPI, bool SCALED, typename TC, int GD_WAVES, bool XT, bool OT, int HT = 0>
+// HT: 0, or the number of half tiles of a block, 3 or 5 (two and a half tiles per unit: qkv of 10240 columns), or one: a matrix with column
+// tiles for at most half of the compute units (o, down of a narrow model) then has blocks for twice as many, each with half of the
+// bytes to pull (the residual product too, whose parts of sum(h^2) are N / 8).  Measured, us, whole tiles / halves: residual product of
+// 2048 x 6144, 4 rows 8.8 / 8.1, 16 rows 10.1 / 9.3; 1024 x 3072 5.4 / 4.95, 6.2 / 5.4; 1024 x 2048, 16 rows 4.7 / 4.45 (1 row 4.0 / 4.1).
+// RC: a wave's chunks of K per round of loads, where they make one round (K = 3072 three, the third costs a round trip of its own otherwise:
+// 5.4 / 4.9 us of these); more than four gain nothing (2048 x 6144 in one round of six 8.4, in three of two 8.1).
+template <int EPI, bool SCALED, typename TC, int GD_WAVES, bool XT, bool OT, int HT = 0, int RC = 2>
 __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_kernel(
     const bf16_t* __restrict__ X, const bf16_t* __restrict__ Wt, TC* __restrict__ C, float* __restrict__ resid_out,
     bf16_t* __restrict__ xw_out, const bf16_t* __restrict__ w_next, float* __restrict__ ss_out, const float* __restrict__ ss_in,
     int n_parts, float eps, int M, int N, int K, GateAct gact) {
     constexpr bool H3 = HT != 0;
-    static_assert(!H3 || (EPI == EPI_STORE && (HT == 3 || HT == 5)), "three or five halves of column tiles, the stored product only");
+    static_assert(!H3 || (EPI == EPI_STORE && (HT == 3 || HT == 5)) || (EPI != EPI_GATED && HT == 1), "one half of a column tile, or three or five for the stored product");
     constexpr int NT = H3 ? (HT + 1) / 2 : (EPI == EPI_GATED ? 2 : 1);
     __shared__ float red[(GD_WAVES - 1) * NT * 64 * 4];
     __shared__ float ss_red[GD_WAVES * 4 * 16];
@@ -75,7 +80,8 @@ __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_kernel(
     }
     f32x4_t h_old = {0.f, 0.f, 0.f, 0.f};
     uint2 wn = {0u, 0u};
-    if (EPI == EPI_RESID && wave == 0 && x_ok) {
+    const bool mine_g = HT != 1 || (g < 2) == lower;           // (HT 1: the lane groups that have the block's columns)
+    if (EPI == EPI_RESID && wave == 0 && x_ok && mine_g) {
         h_old = *reinterpret_cast<const f32x4_t*>(resid_out + (size_t)r * N + n_base + 4 * g);
         wn = *reinterpret_cast<const uint2*>(w_next + n_base + 4 * g);
     }
@@ -92,7 +98,7 @@ __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_kernel(
     // tile's lower half only)
     bool w_on[NT];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) w_on[nt] = !H3 || (nt == 0 ? (lower || r >= 8) : (nt == NT - 1 ? (!lower || r < 8) : true));
+    for (int nt = 0; nt < NT; ++nt) w_on[nt] = !H3 || (HT == 1 ? (r < 8) == lower : nt == 0 ? (lower || r >= 8) : (nt == NT - 1 ? (!lower || r < 8) : true));
     const char* xbase = reinterpret_cast<const char*>(X);
     const unsigned xoff = XT ? 16u * lane : (unsigned)min(r, M - 1) * (unsigned)K * 2u + 16u * g;
 
@@ -122,6 +128,18 @@ __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_kernel(
     // gate/up 33.2 against 32.5, down 20.3 against 17.5, the output head 216 against 191; the memory serves the bursts of
     // 24 loads a wave better than the same loads twelve at a time between products.)
     int c = wave;
+    if constexpr (RC > 2) {
+        bf16x8_t a[RC][NT][4], b[RC][4];
+        for (; c + (RC - 1) * GD_WAVES < nfull; c += RC * GD_WAVES) {
+#pragma unroll
+            for (int q = 0; q < RC; ++q) GD_LOAD(a[q], b[q], c + q * GD_WAVES)
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = 0; q < RC; ++q) {
+                if (q & 1) { GD_MFMA(a[q], b[q], acc2) } else { GD_MFMA(a[q], b[q], acc) }
+            }
+        }
+    }
     for (; c + GD_WAVES < nfull; c += 2 * GD_WAVES) {
         GD_LOAD(a0, b0, c)
         GD_LOAD(a1, b1, c + GD_WAVES)
@@ -170,7 +188,7 @@ __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_kernel(
     // lane (m = r, g) holds C[m][n_base + 4 g + i]
     const int m = r, n = n_base + 4 * g;
     if (EPI == EPI_RESID) {
-        gd_residual_epilogue<OT>(acc[0], h_old, wn, resid_out, xw_out, ss_out + blockIdx.x * 16, m, n, g, M, N, 1);
+        gd_residual_epilogue<OT>(acc[0], h_old, wn, resid_out, xw_out, ss_out + blockIdx.x * 16, m, n, g, M, N, 1, mine_g);
         return;
     }
     if (m >= M) return;
@@ -179,7 +197,7 @@ __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_kernel(
         // tile0: all columns (lower) or those of its upper half; the next tile: its lower half, or all
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            const bool mine = nt == 0 ? (lower || g >= 2) : (nt == NT - 1 ? (!lower || g < 2) : true);
+            const bool mine = HT == 1 ? mine_g : nt == 0 ? (lower || g >= 2) : (nt == NT - 1 ? (!lower || g < 2) : true);
             if (!mine) continue;
             TC* out = C + (size_t)m * N + n + 16 * nt;
 #pragma unroll
@@ -425,6 +443,21 @@ static bool gd_launch2(const GdArgs& a) {
     if (a.M <= 16) {
         // one and a half column tiles per compute unit: three halves of tiles per block
         bool halves = false;
+        const int each = (a.K / GD_CHUNK + W - 1) / W;
+#define GD_HALF_N(RC) gemm_decode_kernel<EPI, SCALED, TC, W, XT, OT, 1, RC><<<a.N / 8, W * 64, 0, a.st>>>(GD_ARGS)
+#define GD_HALF if (each == 3) GD_HALF_N(3); else GD_HALF_N(2);
+        if constexpr (EPI == EPI_STORE && sizeof(TC) == 2) {
+            if (a.N / 8 <= gd_compute_units()) {
+                GD_HALF
+                halves = true;
+            }
+        }
+        if constexpr (EPI == EPI_RESID) {
+            if (a.half_parts) {
+                GD_HALF
+                halves = true;
+            }
+        }
         if constexpr (EPI == EPI_STORE && SCALED && XT && !OT && sizeof(TC) == 2) {
             const int cus = gd_compute_units();
             const bool uneven = (a.N / 16) % cus != 0;
@@ -487,11 +520,12 @@ extern "C" int64_t spy_gemm_decode_workspace() { return gd_splitk_workspace_byte
 // or 128 beyond).  scaled != 0: x = bf16(h * w_norm) and ss_in
 // [n_parts, MP] holds the parts of sum(h^2); the result is multiplied by rsqrt(sum / K + eps).
 // epi 0: C [M, N] (c_dtype), with w_next = two bfloat16 numbers (p, q): xIELU of the result, with act SPY_ACT_GELU: its gelu;  epi 1: W = [gate | up], C [M, N] = act(gate) * up (act: SPY_ACT_*);  epi 2: resid [M, N] += result,
-// xw_out [M, N] = bf16(resid * w_next), ss_out [N / 16, MP] = every block's part of the rows' sums of squares.
+// xw_out [M, N] = bf16(resid * w_next), ss_out [out_parts, MP] = every block's part of the rows' sums of squares (out_parts N / 16, or N / 8
+// for up to 16 rows: blocks of half a column tile).
 // x_tiled / out_tiled: X / the bfloat16 output for the next product (xw_out of epi 2, C of epi 1) are in operand order.
 extern "C" int spy_gemm_decode(const void* X, int scaled, const float* ss_in, int n_parts, float eps, const void* Wt, int epi,
                                void* C, int c_dtype, float* resid, void* xw_out, const void* w_next, float* ss_out, int M, int N,
-                               int K, int x_tiled, int out_tiled, int act, void* ws, int64_t ws_bytes, hipStream_t st) {
+                               int K, int x_tiled, int out_tiled, int act, void* ws, int64_t ws_bytes, int out_parts, hipStream_t st) {
     SPY_REQUIRE(M > 0 && M <= 128, "spy_gemm_decode: M = %d rows (1..128 allowed)", M);
     SPY_REQUIRE(N > 0 && N % 16 == 0 && K > 0 && K % 128 == 0, "spy_gemm_decode: N = %d must be a multiple of 16 and K = %d of 128", N, K);
     SPY_REQUIRE(epi >= 0 && epi <= 2, "spy_gemm_decode: unknown epilogue %d", epi);
@@ -510,10 +544,12 @@ extern "C" int spy_gemm_decode(const void* X, int scaled, const float* ss_in, in
     else SPY_REQUIRE(gate_act_of(act, &gact), "spy_gemm_decode: unknown activation %d of the gated epilogue", act);
     GdArgs a = {(const bf16_t*)X, (const bf16_t*)Wt, C, resid, (bf16_t*)xw_out, (const bf16_t*)w_next, ss_out, ss_in, n_parts, eps, M, N, K,
                 x_tiled != 0, out_tiled != 0, st, gact, ws, (long long)ws_bytes};
+    SPY_REQUIRE(epi != EPI_RESID || out_parts == N / 16 || (out_parts == N / 8 && M <= 16), "spy_gemm_decode: %d parts of the sums of squares of %d columns", out_parts, N);
+    a.half_parts = epi == EPI_RESID && out_parts == N / 8;
     const bool f32 = c_dtype == SPY_F32;
     // (a stored product with an activation is built in this file's kernels only)
     const bool store_act = epi == EPI_STORE && (w_next != nullptr || act == SPY_ACT_GELU);
-    if (!store_act && (gd_splitk_try(a, epi, scaled != 0, f32) || gd_wide_try(a, epi, scaled != 0, f32))) {
+    if (!store_act && !a.half_parts && (gd_splitk_try(a, epi, scaled != 0, f32) || gd_wide_try(a, epi, scaled != 0, f32))) {
         SPY_CHECK_LAUNCH("spy_gemm_decode");
         return 0;
     }

@@ -92,7 +92,7 @@ class _Hip:
         # the entry point that a step calls most: with its argument types declared, plain numbers go in as they are (no
         # ctypes object per argument: 3 us of the host's 14 per call)
         P, I = ctypes.c_void_p, ctypes.c_int
-        self.lib.spy_gemm_decode.argtypes = [P, I, P, I, ctypes.c_float, P, I, P, I, P, P, P, P, I, I, I, I, I, I, P, ctypes.c_int64, P]
+        self.lib.spy_gemm_decode.argtypes = [P, I, P, I, ctypes.c_float, P, I, P, I, P, P, P, P, I, I, I, I, I, I, P, ctypes.c_int64, I, P]
 
     def call(self, name, *args):
         rc = getattr(self.lib, name)(*args)
@@ -903,7 +903,7 @@ def _gemm_decode(x, tiled: torch.Tensor, epi: int, n_out: int, out, resid, xw_ou
     out_tiled = isinstance(out, OperandRows) or isinstance(xw_out, OperandRows)
     mp = 16 * row_tiles(M)
     _check(ss is None or ss.shape[1] == mp, "decode product: the parts of the sums of squares must have %d columns", mp)
-    _check(ss_out is None or tuple(ss_out.shape) == (n_out // 16, mp), "decode product: the new parts must be [N / 16, %d]", mp)
+    _check(ss_out is None or tuple(ss_out.shape) in ((n_out // 16, mp), (n_out // 8, mp)), "decode product: the new parts must be [N / 16 or N / 8, %d]", mp)
     for o in (out, xw_out):
         if isinstance(o, OperandRows):
             _check(o.rows == M and o.width == n_out and tuple(o.data.shape) == (n_out // 32, o.tiles, 64, 8),
@@ -916,7 +916,8 @@ def _gemm_decode(x, tiled: torch.Tensor, epi: int, n_out: int, out, resid, xw_ou
     at = lambda t: None if t is None else t.data_ptr()              # (argument types are declared: see _Hip)
     hip().call("spy_gemm_decode", at(xs), 0 if ss is None else 1, at(ss), 0 if ss is None else ss.shape[0], eps, at(tiled), epi,
                at(out_t), 0 if out_t is None else _code(out_t, "out"), at(resid), at(xw_t), at(w_next), at(ss_out), M, n_out, K,
-               1 if x_tiled else 0, 1 if out_tiled else 0, act, at(ws), 0 if ws is None else ws.numel(), _Hip.stream())
+               1 if x_tiled else 0, 1 if out_tiled else 0, act, at(ws), 0 if ws is None else ws.numel(), 0 if ss_out is None else ss_out.shape[0],
+               _Hip.stream())
 
 
 def _rows_of(x) -> int:
@@ -955,6 +956,12 @@ def decode_linear_swiglu(x, tiled_gate_up: torch.Tensor, for_product: bool = Fal
     return out
 
 
+def residual_parts(rows: int, columns: int) -> int:
+    """Parts of the rows' sums of squares that the residual product writes, one a block: for up to 16 rows of at most 2048 columns, whose
+    tiles of 16 are blocks for half of the compute units at most, a block has half a tile (csrc/gemm_decode.hip)."""
+    return columns // 8 if rows <= 16 and columns <= 2048 else columns // 16
+
+
 def decode_linear_residual(x, tiled: torch.Tensor, resid: torch.Tensor, next_norm_weight: torch.Tensor,
                            eps: float, norm=None) -> ScaledInput:
     """resid += x . w^T (float32, in place) for at most 128 rows (beyond 64: x in operand order only) -> the ScaledInput of the norm that reads the
@@ -965,7 +972,7 @@ def decode_linear_residual(x, tiled: torch.Tensor, resid: torch.Tensor, next_nor
            "decode_linear_residual: the stream must be float32 [M, %d]", N)
     _check(next_norm_weight.dtype == torch.bfloat16 and next_norm_weight.shape == (N,),
            "decode_linear_residual: the next norm's weight must be bfloat16 [%d]", N)
-    ss = torch.empty((N // 16, 16 * row_tiles(M)), dtype=torch.float32, device=resid.device)
+    ss = torch.empty((residual_parts(M, N), 16 * row_tiles(M)), dtype=torch.float32, device=resid.device)
     if _operand_order_ok(N):
         xw = OperandRows.empty(M, N, resid.device)
     else:
