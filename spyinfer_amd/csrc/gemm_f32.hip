@@ -2,8 +2,7 @@
 // float32 instructions multiply and add as fmaf does; gemm_f32_split.hip, which has most products of more than 32 rows, cuts the
 // numbers without loss).  Three kernels by the number of rows:
 //
-//   few    (up to 4 or 8 rows)   bound by streaming W from memory.  A wave owns NR rows of W and walks K with 64 lanes side by side, so
-//                           that every load of W is 1 KiB in one piece; A comes from the caches; the lanes' sums meet at the end.
+//   few    (up to 8 rows)   bound by streaming W from memory: a block's waves share K, 64 lanes side by side along it.
 //   narrow (tens of rows)   bound by W from memory as well, but A's rows would be read once per row of W by the kernel above.
 //                           A block owns 16 rows of W and MT tiles of 16 rows of A; its eight waves take the chunks of 64 of K in
 //                           turn, operands straight from memory into v_mfma_f32_16x16x4_f32 registers, and add through LDS.
@@ -24,38 +23,49 @@ __device__ __forceinline__ gf_f32x4_t gf_load(const float* p) { return *reinterp
 __device__ __forceinline__ gf_f32x4_t gf_stream(const float* p) { return __builtin_nontemporal_load(reinterpret_cast<const gf_f32x4_t*>(p)); }
 
 // ---- few rows ------------------------------------------------------------------------------------------------------------
-// V sums over a wave's lanes at once: every step hands half of a lane's values to its partner and adds the other half's, so V - 1 exchanges
-// and 6 - log2 V more do what 6 V do for one value after the other, in the same order of sums.  Lane l ends with value gf_value<V>(l).
-template <int V>
-__device__ __forceinline__ float gf_wave_sums(float (&v)[V], int lane) {
-    int mask = 32;
+// V sums over each 16 lanes of a wave at once, without LDS: partners are lanes l ^ 15, l ^ 7, l ^ 3, l ^ 1 (moves within a row of lanes), of
+// which one keeps the lower half of the values and the other the upper.  Lane l ends with V / 16 sums, of the values from l % 16 V / 16 on
+// (V < 16: with one, of value l % 16 / (16 / V)).
+template <int CTRL> __device__ __forceinline__ float gf_moved(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL, int BIT, int N, int V>
+__device__ __forceinline__ void gf_row_step(float (&v)[V], int lane) {
+    if constexpr (N >= 2) {
+        const bool upper = (lane & BIT) != 0;
 #pragma unroll
-    for (int n = V / 2; n >= 1; n /= 2, mask /= 2) {
-        const bool upper = (lane & mask) != 0;
-#pragma unroll
-        for (int i = 0; i < n; ++i) {
-            const float keep = upper ? v[i + n] : v[i], give = upper ? v[i] : v[i + n];
-            v[i] = keep + __shfl_xor(give, mask, 64);
+        for (int i = 0; i < N / 2; ++i) {
+            const float keep = upper ? v[i + N / 2] : v[i], give = upper ? v[i] : v[i + N / 2];
+            v[i] = keep + gf_moved<CTRL>(give);
         }
+    } else {
+        v[0] += gf_moved<CTRL>(v[0]);
     }
-#pragma unroll
-    for (; mask >= 1; mask /= 2) v[0] += __shfl_xor(v[0], mask, 64);
-    return v[0];
 }
 template <int V>
-__device__ __forceinline__ int gf_value(int lane) { return lane / (64 / V); }
+__device__ __forceinline__ void gf_row_sums(float (&v)[V], int lane) {
+    gf_row_step<0x140, 8, V>(v, lane);                                    // row_mirror
+    gf_row_step<0x141, 4, (V >= 2 ? V / 2 : 1)>(v, lane);                 // row_half_mirror
+    gf_row_step<0x1b, 2, (V >= 4 ? V / 4 : 1)>(v, lane);                  // quad_perm 3 2 1 0
+    gf_row_step<0xb1, 1, (V >= 8 ? V / 8 : 1)>(v, lane);                  // quad_perm 1 0 3 2
+}
 
-// GATED: W = [gate rows | up rows] of N columns each; a wave owns NR / 2 columns, their gate rows and their up rows, and stores
-// act(gate) * up.  Measured, us, the product with the activation's launch / this: 12288 x 2048,
-// 4 rows 23.8 / 21.3, 1 row 18.2 / 16.7; 6144 x 1024, 4 rows 9.8 / 7.6.  (The lanes' sums one after the other cost 0.3 to 0.8 us a launch;
-// A through LDS, or asked for a group ahead, gave nothing.)
-template <int MR, int NR, int U, bool GATED>
-__global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
-                                                           int M, int N, int K, GateAct act) {
-    constexpr int NC = GATED ? NR / 2 : NR, V = NR * MR;              // columns of a wave, its sums
+// A block owns NR rows of W; its WV waves take the chunks of 256 of K in turn, U of them and A's pieces asked for at once, and the next
+// ones before these are multiplied; the sums of 16 lanes meet in registers, those of a block's rows of lanes in LDS.  Every load of W is 1
+// KiB in one piece, and A's rows come out of the caches once per NR rows of W: with a row or two of W a wave, as this kernel had it, A was
+// twice to four times W's bytes on a compute unit's way from L2.  Sums over a wave by lane exchanges through LDS took 2.5 us of a launch.
+// GATED: W = [gate rows | up rows] of N columns each; a block owns NR / 2 columns, their gate rows and their up rows, and stores act(gate)
+// * up.  Measured, us, with one to four rows of W a wave and its own K / this, 4 rows of A: 2048 x 2048 6.9 / 5.6, 2048 x 6144 15.6 / 10.6 (4.7
+// TB/s), 4096 x 2048 9.7 / 8.2, 12288 x 2048 gated 22.3 / 18.3 (5.5 TB/s), 151936 x 2048 192 / 186; 1 row: 2048 x 6144 10.3 / 9.9, 1024 x 3072
+// 4.3 / 4.5; 8 rows, the narrow kernel / this: 2048 x 6144 23.4 / 13.8, 12288 x 2048 with its activation 45 / 22, 151936 x 2048 356 / 225.
+template <int MR, int NR, int U, int WV, bool GATED>
+__global__ __launch_bounds__(WV * 64) void gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
+                                                              int M, int N, int K, GateAct act) {
+    constexpr int NC = GATED ? NR / 2 : NR, V = NR * MR;              // columns of the block, its sums
+    constexpr int LEFT = V >= 16 ? V / 16 : 1, SHARE = V >= 16 ? 1 : 16 / V;      // sums a lane ends with; lanes with the same one
+    __shared__ float red[WV * 4][V];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int n0 = (blockIdx.x * 4 + wave) * NC;
-    if (n0 >= N) return;
+    const int n0 = blockIdx.x * NC;
     const float* wrow[NR];
     const float* arow[MR];
 #pragma unroll
@@ -63,18 +73,17 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
 #pragma unroll
     for (int m = 0; m < MR; ++m) arow[m] = A + (size_t)min(m, M - 1) * K + 4 * lane;
     float acc[NR][MR] = {};
-    auto fetch = [&](gf_f32x4_t (&w)[U][NR], int c) {
+    struct Round { gf_f32x4_t w[U][NR], a[U][MR]; };
+    auto fetch = [&](Round& f, int c) {                                // chunks c, c + WV, ...
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u) {
 #pragma unroll
-            for (int n = 0; n < NR; ++n) w[u][n] = gf_stream(wrow[n] + (c + u) * 256);
+            for (int n = 0; n < NR; ++n) f.w[u][n] = gf_stream(wrow[n] + (c + WV * u) * 256);
+#pragma unroll
+            for (int m = 0; m < MR; ++m) f.a[u][m] = gf_load(arow[m] + (c + WV * u) * 256);
+        }
     };
-    auto products = [&](const gf_f32x4_t (&w)[U][NR], int c) {
-        gf_f32x4_t a[U][MR];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int m = 0; m < MR; ++m) a[u][m] = gf_load(arow[m] + (c + u) * 256);
+    auto products = [&](const Round& f) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -82,7 +91,7 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
 #pragma unroll
                 for (int n = 0; n < NR; ++n)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[n][m] = fmaf(a[u][m][j], w[u][n][j], acc[n][m]);
+                    for (int j = 0; j < 4; ++j) acc[n][m] = fmaf(f.a[u][m][j], f.w[u][n][j], acc[n][m]);
     };
     auto single = [&](int k) {
         gf_f32x4_t w[NR];
@@ -97,39 +106,49 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
                 for (int j = 0; j < 4; ++j) acc[n][m] = fmaf(a[j], w[n][j], acc[n][m]);
         }
     };
-    // groups of U chunks of 256 of K; the next group's rows of W are asked for before this one's products (no load under a
-    // condition: the compiler would wait for all of them)
-    const int groups = (K >> 8) / U;
-    gf_f32x4_t w0[U][NR], w1[U][NR];
-    if (groups > 0) {
-        fetch(w0, 0);
+    const int chunks = K >> 8, rounds = chunks / (WV * U);
+    Round f0, f1;
+    if (rounds > 0) {
+        fetch(f0, wave);
         int i = 0;
-        for (; i + 2 < groups; i += 2) {
-            fetch(w1, (i + 1) * U);
-            products(w0, i * U);
-            fetch(w0, (i + 2) * U);
-            products(w1, (i + 1) * U);
+        for (; i + 2 < rounds; i += 2) {
+            fetch(f1, wave + (i + 1) * WV * U);
+            products(f0);
+            fetch(f0, wave + (i + 2) * WV * U);
+            products(f1);
         }
-        if (i + 1 < groups) {
-            fetch(w1, (i + 1) * U);
-            products(w0, i * U);
-            products(w1, (i + 1) * U);
+        if (i + 1 < rounds) {
+            fetch(f1, wave + (i + 1) * WV * U);
+            products(f0);
+            products(f1);
         } else {
-            products(w0, i * U);
+            products(f0);
         }
     }
-    int k = groups * U * 256;
-    for (; k + 256 <= K; k += 256) single(k);
-    if (k + 4 * lane < K) single(k);                              // the rest of K, a multiple of 4
+    int c = wave + rounds * WV * U;
+    for (; c < chunks; c += WV) single(c * 256);
+    if (c == chunks && chunks * 256 + 4 * lane < K) single(c * 256);      // the rest of K, a multiple of 4: the wave whose turn it is
     float sums[V];
 #pragma unroll
     for (int n = 0; n < NR; ++n)
 #pragma unroll
         for (int m = 0; m < MR; ++m) sums[n * MR + m] = acc[n][m];
-    float y = gf_wave_sums<V>(sums, lane);
-    const int at = gf_value<V>(lane), n = n0 + at / MR, m = at % MR;
-    if (GATED) y = gated_value(act, y, __shfl_xor(y, 32, 64));       // (the upper half of the values is the upper half of the lanes)
-    if (lane % (64 / V) == 0 && at / MR < NC && m < M && n < N) C[(size_t)m * N + n] = y;
+    gf_row_sums<V>(sums, lane);
+    if (lane % SHARE == 0) {
+#pragma unroll
+        for (int i = 0; i < LEFT; ++i) red[wave * 4 + (lane >> 4)][(lane & 15) / SHARE * LEFT + i] = sums[i];
+    }
+    __syncthreads();
+    const int t = threadIdx.x, n = t / MR, m = t % MR;
+    if (t >= NC * MR) return;
+    float y = 0.f, up = 0.f;
+#pragma unroll
+    for (int p = 0; p < WV * 4; ++p) {
+        y += red[p][t];
+        if (GATED) up += red[p][t + V / 2];
+    }
+    if (GATED) y = gated_value(act, y, up);
+    if (m < M && n0 + n < N) C[(size_t)m * N + n0 + n] = y;
 }
 
 // ---- a few tiles of rows ----------------------------------------------------------------------------------------------------
@@ -361,22 +380,30 @@ bool gemm_f32_takes(const void* A, const void* W, const void* C, int M, int N, i
     return K % 4 == 0 && at % 16 == 0 && (int64_t)((N + 63) / 64) * ((M + 63) / 64) < (1 << 28);
 }
 
+// Up to 8 rows; from 5 on not 4096 rows of W and more with a K up to 1024, whose blocks have little to stream (8 rows, 4096 x 1024: 7.3 us,
+// the narrow kernel 6.9; 4096 x 2048 10.1 / 11.0).
+static bool gf_few_takes(int M, int N, int K) { return M <= 4 || (M <= 8 && (N < 4096 || K > 1024)); }
+
+// Rows of W a block, and waves: eight rows where there are plenty (4 rows of A: 12288 x 2048 gated 18.3 us, with four 19.5; 2048 x 6144 11.5 / 10.6;
+// 8 rows of A: 4096 x 2048 10.1 / 10.9), and up to 1024 rows of W eight waves a block to have enough of them (4 rows of A, 1024 x 3072 5.0
+// us, four waves 5.7) or, for one or two rows of A, two rows of W (1024 x 2048 3.7 / 3.8, 1024 x 3072 4.5 / 4.4).
+template <bool GATED>
+static void gf_few(const float* A, const float* W, float* C, int M, int N, int w_rows, int K, GateAct act, hipStream_t st) {
+#define GF_FEW(MR, NR, U, WV) gemm_f32_few_kernel<MR, NR, U, WV, GATED><<<(N + NR / (GATED ? 2 : 1) - 1) / (NR / (GATED ? 2 : 1)), WV * 64, 0, st>>>(A, W, C, M, N, K, act)
+    if (M == 1) { if (w_rows <= 1024) GF_FEW(1, 2, 2, 4); else GF_FEW(1, 4, 2, 4); }
+    else if (M == 2) { if (w_rows <= 1024) GF_FEW(2, 2, 2, 4); else GF_FEW(2, 4, 2, 4); }
+    else if (M <= 4) { if (w_rows <= 1024) GF_FEW(4, 4, 1, 8); else if (w_rows < 8192) GF_FEW(4, 4, 1, 4); else GF_FEW(4, 8, 1, 4); }
+    else { if (w_rows <= 1024) GF_FEW(8, 4, 1, 8); else if (w_rows < 4096) GF_FEW(8, 4, 1, 4); else GF_FEW(8, 8, 1, 4); }
+#undef GF_FEW
+}
+
 int gemm_f32(const float* A, const float* W, float* C, int M, int N, int K, hipStream_t st) {
-#define GF_FEW(MR, NR, U) gemm_f32_few_kernel<MR, NR, U, false><<<(N + 4 * NR - 1) / (4 * NR), 256, 0, st>>>(A, W, C, M, N, K, GateAct{1.f, 0.f})
 #define GF_NARROW(MT) gemm_f32_narrow_kernel<MT><<<dim3(tiles16, (M + 16 * MT - 1) / (16 * MT)), GF_WAVES * 64, 0, st>>>(A, W, C, M, N, K)
 #define GF_TILE(KS) gemm_f32_tile_kernel<KS><<<((tm * tn + 7) / 8) * 8, 256 * KS, 0, st>>>(A, W, C, M, N, K, tm, tn, 1)
     const int tiles16 = (N + 15) / 16, tm = (M + 63) / 64, tn = (N + 63) / 64;
     if (gemm_f32_split_takes(M, N, K, 1)) return gemm_f32_split(A, W, C, M, N, K, 1, st);
-    if (M <= 4 || (M <= 8 && N <= 1024)) {
-        // Rows of W per wave: each more reads A once less, but takes waves away.  One up to 2048 rows of W (four rows of A, 2048 x
-        // 2048: 7.3 us against 7.4 with two, 9.8 with four), four from 12288 on (29.9 / 25.1 / 23.8 us for 12288 x 2048); with one
-        // or two rows of A, where A costs little, one up to 12288 (20.4 / 21.8 / 21.1) and for the output heads (1 row of A, 151936 x
-        // 1024: 100 / 106 / 115) or two (116 / 108 / 125).  5 to 8 rows take this kernel only where the next has blocks for a
-        // quarter of the compute units (1024 x 3072: 8.9 against 12.7 us; 2048 x 2048 10.3 against 9.3).
-        if (M == 1) GF_FEW(1, 1, 4);
-        else if (M == 2) { if (N > 12288) GF_FEW(2, 2, 2); else GF_FEW(2, 1, 4); }
-        else if (M <= 4) { if (N >= 12288) GF_FEW(4, 4, 2); else if (N > 2048) GF_FEW(4, 2, 2); else GF_FEW(4, 1, 4); }
-        else GF_FEW(8, 1, 2);
+    if (gf_few_takes(M, N, K)) {
+        gf_few<false>(A, W, C, M, N, N, K, GateAct{1.f, 0.f}, st);
     } else if (tm * tn < 160) {
         // Row tiles per block: as many as leave a block for every compute unit, W being read once per group of them (24 rows, 2048 x
         // 2048: 10.4 us with one, 13.1 with two; 4096 x 2048: 19.4 with one, 14.5 with two; 64 rows, 4096 x 1024: 20 / 15.3 / 13.9
@@ -397,16 +424,14 @@ int gemm_f32(const float* A, const float* W, float* C, int M, int N, int K, hipS
     return 0;
 }
 
-// act(A . Wgate^T) * (A . Wup^T) for up to four rows and for those that gemm_f32_split.hip takes, W = [gate rows | up rows] of N each, without the [M][2 N] result in between.
+// act(A . Wgate^T) * (A . Wup^T) for up to eight rows and for those that gemm_f32_split.hip takes, W = [gate rows | up rows] of N each, without the [M][2 N] result in between.
 extern "C" int spy_gemm_f32_gated(float* C, const float* A, const float* W, int M, int N, int K, int act_code, hipStream_t st) {
     GateAct act;
     SPY_REQUIRE(M > 0 && N > 0 && K > 0 && gate_act_of(act_code, &act), "spy_gemm_f32_gated: %d rows, activation %d", M, act_code);
     SPY_REQUIRE(gemm_f32_takes(A, W, C, M, N, K), "spy_gemm_f32_gated: operands of %d x %d x %d are not taken", M, N, K);
-    SPY_REQUIRE(M <= 4 || (N < (1 << 30) && gemm_f32_split_takes(M, 2 * N, K, 1)), "spy_gemm_f32_gated: %d rows of %d x %d are not taken", M, N, K);
-    if (M > 4) return gemm_f32_split_gated(A, W, C, M, 2 * N, K, act, st);
-#define GF_GATED(MR, U) gemm_f32_few_kernel<MR, 2, U, true><<<(N + 3) / 4, 256, 0, st>>>(A, W, C, M, N, K, act)
-    if (M == 1) GF_GATED(1, 4); else if (M == 2) GF_GATED(2, 2); else GF_GATED(4, 2);
-#undef GF_GATED
+    SPY_REQUIRE(M <= 8 || (N < (1 << 30) && gemm_f32_split_takes(M, 2 * N, K, 1)), "spy_gemm_f32_gated: %d rows of %d x %d are not taken", M, N, K);
+    if (M > 8) return gemm_f32_split_gated(A, W, C, M, 2 * N, K, act, st);
+    gf_few<true>(A, W, C, M, N, 2 * N, K, act, st);
     SPY_CHECK_LAUNCH("spy_gemm_f32_gated");
     return 0;
 }

@@ -716,7 +716,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, tiled: Optional[torc
         hip().call("spy_gemm_skinny_swiglu", _ptr(x), _ptr(w_gate_up), _ptr(out), _code(out, "out"), ctypes.c_int(M),
                    ctypes.c_int(I), ctypes.c_int(K), ctypes.c_int(GATED_ACTIVATIONS[activation]), _Hip.stream())
         return out
-    if x.dtype == torch.float32 and (0 < M <= 4 or f32_rows_split(M, 2 * I, K)) and x.is_cuda and isinstance(w_gate_up, torch.Tensor) \
+    if x.dtype == torch.float32 and (0 < M <= 8 or f32_rows_split(M, 2 * I, K)) and x.is_cuda and isinstance(w_gate_up, torch.Tensor) \
             and w_gate_up.dtype == torch.float32 and K % 4 == 0 and x.is_contiguous() and w_gate_up.is_contiguous() and (x.data_ptr() | w_gate_up.data_ptr()) % 16 == 0:
         out = torch.empty((M, I), dtype=x.dtype, device=x.device)
         hip().call("spy_gemm_f32_gated", _ptr(out), _ptr(x), _ptr(w_gate_up), M, I, K, GATED_ACTIVATIONS[activation], _Hip.stream())
