@@ -659,43 +659,60 @@ __global__ __launch_bounds__(QK_WAVES * 64) void qknorm_rope_store_kernel(
     }
 }
 
-// The same for many tokens of bfloat16 with the whole head rotated (rot == d) and d in {16, 32, 64, 128, 256}:
-// d / 16 lanes per (token, q or k head), each with 8 + 8 values that pair up in the rotation, so all loads and
-// stores are 16 bytes; and the values of 16 tokens of a kv head go through LDS, so that 8 tokens that follow each
-// other in a page are stored as one 16-byte piece of each row of the transposed page (single stores otherwise).
-// Blocks [0, qk_blocks) do q and k, the rest one (16 tokens, kv head) tile of v each.
-typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t qk_u32x4;
-template <typename TW, int LPH>
+// The same for many tokens with the whole head rotated (rot == d) and d in {16, 32, 64, 128, 256}: d / 16 lanes per (token, q or k
+// head), each with 8 + 8 values that pair up in the rotation, so all loads and stores are 16 bytes; and the values of 16 tokens of a kv
+// head go through LDS, so that 8 tokens that follow each other in a page are stored in 16-byte pieces of each row of the transposed page
+// (single stores otherwise).  Blocks [0, qk_blocks) do q and k, the rest one (16 tokens, kv head) tile of v each.  Quotients are of
+// unsigned 32-bit numbers, and a token's rotation is asked for beside its values.  Measured, us: 2048 tokens, 32 + 8 + 8 heads of 128, bfloat16
+// 11.3 (4.5 TB/s; 12.1 with 64-bit quotients); float32, 16 + 8 + 8 heads, 611 tokens 7.1, 200 tokens 3.6 (a wave a head, 4 bytes a lane: 12.4 and 5.8).
+template <typename TA> struct Eight;
+template <> struct Eight<bf16_t> {
+    static __device__ __forceinline__ void load(const bf16_t* p, float (&v)[8]) {
+        const uint4 r = *reinterpret_cast<const uint4*>(p);
+        const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { v[2 * i] = __uint_as_float(w[i] << 16); v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u); }
+    }
+    static __device__ __forceinline__ void store(bf16_t* p, const float (&v)[8]) {
+        *reinterpret_cast<uint4*>(p) = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+    }
+};
+template <> struct Eight<float> {
+    static __device__ __forceinline__ void load(const float* p, float (&v)[8]) { Vec4<float>::load(p, v); Vec4<float>::load(p + 4, v + 4); }
+    static __device__ __forceinline__ void store(float* p, const float (&v)[8]) { Vec4<float>::store(p, v); Vec4<float>::store(p + 4, v + 4); }
+};
+
+template <typename TA, typename TW, int LPH>
 __global__ __launch_bounds__(256) void qknorm_rope_store_vec_kernel(
-    const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out, int T, int n_q, int n_kv, const TW* __restrict__ qw,
+    const TA* __restrict__ qkv, TA* __restrict__ q_out, int T, int n_q, int n_kv, const TW* __restrict__ qw,
     const TW* __restrict__ kw, float eps, const float* __restrict__ cos_t, const float* __restrict__ sin_t, int max_pos,
-    const int* __restrict__ positions, bf16_t* __restrict__ kc, bf16_t* __restrict__ vc, int P, int num_pages,
+    const int* __restrict__ positions, TA* __restrict__ kc, TA* __restrict__ vc, int P, int num_pages,
     const int* __restrict__ slots, int qk_blocks) {
-    constexpr int d = LPH * 16, half = LPH * 8;
-    __shared__ __align__(16) bf16_t tile[16 * (d + 8)];
+    constexpr int d = LPH * 16, half = LPH * 8, LD = d + 16 / sizeof(TA);
+    __shared__ __align__(16) TA tile[16 * LD];
     const int heads = n_q + 2 * n_kv, qk_heads = n_q + n_kv;
     if ((int)blockIdx.x < qk_blocks) {
-        const long long u = (long long)blockIdx.x * (256 / LPH) + threadIdx.x / LPH;
+        const unsigned u = blockIdx.x * (256 / LPH) + threadIdx.x / LPH;
         const int sub = threadIdx.x % LPH;
-        if (u >= (long long)T * qk_heads) return;
-        const int t = (int)(u / qk_heads), h = (int)(u % qk_heads);
+        if (u >= (unsigned)T * (unsigned)qk_heads) return;
+        const int t = (int)(u / (unsigned)qk_heads), h = (int)(u % (unsigned)qk_heads);
         const bool is_q = h < n_q;
+        const TA* x = qkv + (size_t)t * heads * d + (size_t)h * d + 8 * sub;
+        float a[8], b[8], ss = 0.f;
+        Eight<TA>::load(x, a);
+        Eight<TA>::load(x + half, b);
+        int p = positions[t];
         int page = 0, off = 0;
         if (!is_q) {
-            if (!slots) return;
             const int slot = slots[t];
             if (slot < 0 || slot >= num_pages * P) return;      // (all LPH lanes of a head take the same way)
-            page = slot / P;
+            page = (int)((unsigned)slot / (unsigned)P);
             off = slot - page * P;
         }
-        const bf16_t* x = qkv + (size_t)t * heads * d + (size_t)h * d + 8 * sub;
-        const qk_u32x4 ra = *reinterpret_cast<const qk_u32x4*>(x), rb = *reinterpret_cast<const qk_u32x4*>(x + half);
-        float a[8], b[8], ss = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            a[2 * i] = __uint_as_float(ra[i] << 16); a[2 * i + 1] = __uint_as_float(ra[i] & 0xffff0000u);
-            b[2 * i] = __uint_as_float(rb[i] << 16); b[2 * i + 1] = __uint_as_float(rb[i] & 0xffff0000u);
-        }
+        p = p < 0 ? 0 : (p >= max_pos ? max_pos - 1 : p);
+        float cp[8], sp[8];
+        Eight<float>::load(cos_t + (size_t)p * half + 8 * sub, cp);
+        Eight<float>::load(sin_t + (size_t)p * half + 8 * sub, sp);
 #pragma unroll
         for (int i = 0; i < 8; ++i) ss += a[i] * a[i] + b[i] * b[i];
         const TW* w = is_q ? qw : kw;
@@ -709,32 +726,25 @@ __global__ __launch_bounds__(256) void qknorm_rope_store_vec_kernel(
                 b[i] = (scale * b[i]) * to_f32<TW>(w[half + 8 * sub + i]);
             }
         }
-        int p = positions[t];
-        p = p < 0 ? 0 : (p >= max_pos ? max_pos - 1 : p);
-        const float* cp = cos_t + (size_t)p * half + 8 * sub;
-        const float* sp = sin_t + (size_t)p * half + 8 * sub;
         float ya[8], yb[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const float c = cp[i], sn = sp[i];
-            ya[i] = a[i] * c - b[i] * sn;
-            yb[i] = a[i] * sn + b[i] * c;
+            ya[i] = a[i] * cp[i] - b[i] * sp[i];
+            yb[i] = a[i] * sp[i] + b[i] * cp[i];
         }
-        bf16_t* dst = (is_q ? q_out + ((size_t)t * n_q + h) * d : kc + (((size_t)page * n_kv + (h - n_q)) * P + off) * d) + 8 * sub;
-        const qk_u32x4 oa = {pack_bf16x2(ya[0], ya[1]), pack_bf16x2(ya[2], ya[3]), pack_bf16x2(ya[4], ya[5]), pack_bf16x2(ya[6], ya[7])};
-        const qk_u32x4 ob = {pack_bf16x2(yb[0], yb[1]), pack_bf16x2(yb[2], yb[3]), pack_bf16x2(yb[4], yb[5]), pack_bf16x2(yb[6], yb[7])};
-        *reinterpret_cast<qk_u32x4*>(dst) = oa;
-        *reinterpret_cast<qk_u32x4*>(dst + half) = ob;
+        TA* dst = (is_q ? q_out + ((size_t)t * n_q + h) * d : kc + (((size_t)page * n_kv + (h - n_q)) * P + off) * d) + 8 * sub;
+        Eight<TA>::store(dst, ya);
+        Eight<TA>::store(dst + half, yb);
         return;
     }
     // ---- values: 16 tokens of one kv head ---------------------------------------------------------------------
-    const int vb = blockIdx.x - qk_blocks;
-    const int t0 = (vb / n_kv) * 16, hv = vb % n_kv;
+    const unsigned vb = blockIdx.x - qk_blocks;
+    const int t0 = (int)(vb / (unsigned)n_kv) * 16, hv = (int)(vb % (unsigned)n_kv);
     for (int i = threadIdx.x; i < 16 * (d / 8); i += 256) {
         const int tt = i / (d / 8), c8 = i % (d / 8);
-        qk_u32x4 v = {0u, 0u, 0u, 0u};
-        if (t0 + tt < T) v = *reinterpret_cast<const qk_u32x4*>(qkv + (size_t)(t0 + tt) * heads * d + (size_t)(qk_heads + hv) * d + 8 * c8);
-        *reinterpret_cast<qk_u32x4*>(tile + tt * (d + 8) + 8 * c8) = v;
+        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (t0 + tt < T) Eight<TA>::load(qkv + (size_t)(t0 + tt) * heads * d + (size_t)(qk_heads + hv) * d + 8 * c8, v);
+        Eight<TA>::store(tile + tt * LD + 8 * c8, v);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 2 * d; i += 256) {
@@ -748,18 +758,17 @@ __global__ __launch_bounds__(256) void qknorm_rope_store_vec_kernel(
             for (int e = 1; e < 8; ++e) run = run && slots[tb + e] == s0 + e;
         }
         if (run) {                                            // P is a multiple of 8: the 8 slots lie in one page
-            uint32_t pk[4];
+            float v[8];
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                pk[e] = (uint32_t)tile[(8 * tg + 2 * e) * (d + 8) + j] | ((uint32_t)tile[(8 * tg + 2 * e + 1) * (d + 8) + j] << 16);
-            const int page = s0 / P, off = s0 - page * P;
-            *reinterpret_cast<qk_u32x4*>(vc + (((size_t)page * n_kv + hv) * d + j) * P + off) = qk_u32x4{pk[0], pk[1], pk[2], pk[3]};
+            for (int e = 0; e < 8; ++e) v[e] = to_f32<TA>(tile[(8 * tg + e) * LD + j]);
+            const int page = (int)((unsigned)s0 / (unsigned)P), off = s0 - page * P;
+            Eight<TA>::store(vc + (((size_t)page * n_kv + hv) * d + j) * P + off, v);
         } else {
             for (int e = 0; e < 8 && tb + e < T; ++e) {
                 const int slot = slots[tb + e];
                 if (slot < 0 || slot >= num_pages * P) continue;
                 const int page = slot / P, off = slot - page * P;
-                vc[(((size_t)page * n_kv + hv) * d + j) * P + off] = tile[(8 * tg + e) * (d + 8) + j];
+                vc[(((size_t)page * n_kv + hv) * d + j) * P + off] = tile[(8 * tg + e) * LD + j];
             }
         }
     }
@@ -776,19 +785,19 @@ extern "C" int spy_qknorm_rope_store(const void* qkv, int dtype, void* q_out, in
     SPY_REQUIRE(!slots || (kc && vc && P > 0 && num_pages > 0), "spy_qknorm_rope_store: slots without a cache");
     SPY_REQUIRE(n_q + 2 * n_kv <= 65535 * QK_WAVES, "spy_qknorm_rope_store: too many heads");
     const int wd = w_dtype < 0 ? SPY_F32 : w_dtype;
-    // many bfloat16 tokens, whole head rotated, a head size that is 16 times a power of two: the kernel with wide accesses
-    if (dtype == SPY_BF16 && T >= 64 && rot == d && (d == 16 || d == 32 || d == 64 || d == 128 || d == 256) && slots && P % 8 == 0 &&
-        ((uintptr_t)qkv % 16) == 0 && ((uintptr_t)q_out % 16) == 0 && ((uintptr_t)kc % 16) == 0 && ((uintptr_t)vc % 16) == 0 &&
-        (!qw) == (!kw)) {
+    // many tokens, whole head rotated, a head size that is 16 times a power of two: the kernel with wide accesses
+    if (T >= 64 && rot == d && (d == 16 || d == 32 || d == 64 || d == 128 || d == 256) && slots && P % 8 == 0 &&
+        (((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)kc | (uintptr_t)vc | (uintptr_t)cos_t | (uintptr_t)sin_t) % 16) == 0 && (!qw) == (!kw) &&
+        (long long)T * (n_q + n_kv) < (1ll << 31) - 256) {
         const int lph = d / 16;
         const long long units = (long long)T * (n_q + n_kv);
         const long long qk_blocks = (units + 256 / lph - 1) / (256 / lph);
         const long long v_blocks = (long long)((T + 15) / 16) * n_kv;
         SPY_REQUIRE(qk_blocks + v_blocks < (1ll << 31), "spy_qknorm_rope_store: too many tokens");
 #define QKV_CASE(L)                                                                                                             \
-    SPY_DISPATCH(wd, TW, (qknorm_rope_store_vec_kernel<TW, L><<<(unsigned)(qk_blocks + v_blocks), 256, 0, st>>>(               \
-        (const bf16_t*)qkv, (bf16_t*)q_out, T, n_q, n_kv, (const TW*)qw, (const TW*)kw, eps, cos_t, sin_t, max_pos, positions,  \
-        (bf16_t*)kc, (bf16_t*)vc, P, num_pages, slots, (int)qk_blocks)))
+    SPY_DISPATCH(dtype, TA, SPY_DISPATCH(wd, TW, (qknorm_rope_store_vec_kernel<TA, TW, L><<<(unsigned)(qk_blocks + v_blocks), 256, 0, st>>>( \
+        (const TA*)qkv, (TA*)q_out, T, n_q, n_kv, (const TW*)qw, (const TW*)kw, eps, cos_t, sin_t, max_pos, positions,          \
+        (TA*)kc, (TA*)vc, P, num_pages, slots, (int)qk_blocks))))
         switch (lph) {
             case 1: QKV_CASE(1); break;
             case 2: QKV_CASE(2); break;
