@@ -125,6 +125,11 @@ inline bool gate_act_of(int code, GateAct* a) {
 __device__ __forceinline__ float gated_value(const GateAct& a, float z, float up) {
     return (z / (1.0f + expf(-(z * fmaf(a.c3 * z, z, a.c1))))) * up;
 }
+// The same where the result is rounded to bfloat16: the hardware's exponential and reciprocal (a unit or two in the last of 24 bits each, where
+// the result keeps 8) instead of the library's expf and a division, a dozen instructions for three dozen
+__device__ __forceinline__ float gated_value_short(const GateAct& a, float z, float up) {
+    return z * __builtin_amdgcn_rcpf(1.0f + __expf(-(z * fmaf(a.c3 * z, z, a.c1)))) * up;
+}
 
 // Dispatch on a dtype code: binds `T` in `body`.
 #define SPY_DISPATCH(code, T, ...)                  \

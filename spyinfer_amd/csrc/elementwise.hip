@@ -481,7 +481,8 @@ __global__ void swiglu_vec_kernel(const TA* __restrict__ in, TA* __restrict__ ou
 }
 
 // bfloat16, 8 values per thread and step: 16-byte loads that do not stay in the caches (the product's output passes
-// once), one 16-byte store (the next product reads it)
+// once), one 16-byte store (the next product reads it).  Bound by its instructions with the library's expf and a division: 2048 x 2 x
+// 12288 31.5 us, by gated_value_short 26.7 (5.7 TB/s).
 __global__ void swiglu_bf16x8_kernel(const bf16_t* __restrict__ in, bf16_t* __restrict__ out, int T, int I8, GateAct act) {
     typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
     const size_t n = (size_t)T * I8, I = (size_t)I8 * 8;
@@ -494,7 +495,7 @@ __global__ void swiglu_bf16x8_kernel(const bf16_t* __restrict__ in, bf16_t* __re
         for (int e = 0; e < 4; ++e) {
             const float g0 = __uint_as_float(g[e] << 16), g1 = __uint_as_float(g[e] & 0xffff0000u);
             const float u0 = __uint_as_float(u[e] << 16), u1 = __uint_as_float(u[e] & 0xffff0000u);
-            y[e] = pack_bf16x2(gated_value(act, g0, u0), gated_value(act, g1, u1));
+            y[e] = pack_bf16x2(gated_value_short(act, g0, u0), gated_value_short(act, g1, u1));
         }
         *reinterpret_cast<u32x4_t*>(out + t * I + i) = y;
     }
