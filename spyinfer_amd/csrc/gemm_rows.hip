@@ -34,20 +34,12 @@ typedef float gr_f32x4_t __attribute__((ext_vector_type(4)));
 // X and W are not declared free of aliases: the waits below count the loads issued before them, and with that promise the compiler may
 // move loads of W across a wait.
 template <int MT, int EPI>
-__global__ __launch_bounds__(256, 2) void gemm_rows_kernel(void* C, const bf16_t* X, const bf16_t* W, int M, int N, int K, int n_rows,
-                                                           int n_cols, int parts, int blocks, GateAct act) {
-    __shared__ __align__(1024) bf16_t stage0[MT * 16 * 128];
-    __shared__ __align__(1024) bf16_t stage1[MT * 16 * 128];
-    // Blocks go to the dies in turn: a die takes a run of the blocks in (part, columns, rows) order, so that the blocks that read the
-    // same rows of W run beside each other and the matrix comes into one L2 once
-    const int per = (blocks + ROWS_DIES - 1) / ROWS_DIES, idx = blockIdx.x / ROWS_DIES;
-    const int v = (blockIdx.x % ROWS_DIES) * per + idx;
-    if (idx >= per || v >= blocks) return;
-    const int cp = v / n_rows, col_t = cp % n_cols, part = cp / n_cols;
+__device__ __forceinline__ void gemm_rows_block(void* C, const bf16_t* X, const bf16_t* W, int M, int N, int K, int col_t, int part, int parts, int tile0,
+                                                GateAct act, bf16_t* stage0, bf16_t* stage1) {
     const int chunks = K / 128, c0 = (int)((long long)chunks * part / parts);
     const int n = (int)((long long)chunks * (part + 1) / parts) - c0;                  // (at least one: the launcher's check)
     // The last rows' tile ends with row M - 1 (M >= 16 MT): what it shares with the tile before, both blocks form alike
-    const int row0 = min((v % n_rows) * MT * 16, M - MT * 16);
+    const int row0 = min(tile0 * 16, M - MT * 16);
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int NT = N / 16;
     // byte offsets below 2^31 (the launcher's check)
@@ -156,17 +148,52 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(void* C, const bf16_t
     }
 }
 
+// A column of tiles (256 columns, one part) has n_rows blocks, `tall` of them with MT row tiles and the others with one less, as many in
+// all as the rows need.  Which ones are tall moves on by `tall` from one column to the next, so that those that follow each other on a
+// compute unit are of both kinds.
+template <int MT, int EPI>
+__global__ __launch_bounds__(256, 2) void gemm_rows_kernel(void* C, const bf16_t* X, const bf16_t* W, int M, int N, int K, int n_rows, int tall,
+                                                           int n_cols, int parts, int blocks, GateAct act) {
+    __shared__ __align__(1024) bf16_t stage0[MT * 16 * 128];
+    __shared__ __align__(1024) bf16_t stage1[MT * 16 * 128];
+    // Blocks go to the dies in turn: a die takes a run of the blocks in (part, columns, rows) order, so that the blocks that read the
+    // same rows of W run beside each other and the matrix comes into one L2 once
+    const int per = (blocks + ROWS_DIES - 1) / ROWS_DIES, idx = blockIdx.x / ROWS_DIES;
+    const int v = (blockIdx.x % ROWS_DIES) * per + idx;
+    if (idx >= per || v >= blocks) return;
+    const int cp = v / n_rows, i = v % n_rows, col_t = cp % n_cols, part = cp / n_cols;
+    const int shift = (int)((unsigned)cp * (unsigned)tall % (unsigned)n_rows), at = i + shift;
+    const int before = (at >= n_rows ? tall + min(at - n_rows, tall) : min(at, tall)) - min(shift, tall);      // tall blocks before this one
+    const int tile0 = i * (MT - 1) + before;
+    if ((at >= n_rows ? at - n_rows : at) < tall) gemm_rows_block<MT, EPI>(C, X, W, M, N, K, col_t, part, parts, tile0, act, stage0, stage1);
+    else gemm_rows_block<MT - 1, EPI>(C, X, W, M, N, K, col_t, part, parts, tile0, act, stage0, stage1);
+}
+
 template <int MT>
-static int rows_launch(void* C, const void* X, const void* W, int M, int N, int K, int parts, int epi, GateAct act, hipStream_t st) {
-    const int n_rows = (M + MT * 16 - 1) / (MT * 16), n_cols = (N + 255) / 256;
+static int rows_launch(void* C, const void* X, const void* W, int M, int N, int K, int n_rows, int parts, int epi, GateAct act, hipStream_t st) {
+    // (blocks of four tiles overlap where there are not four for each)
+    const int n_cols = (N + 255) / 256, left = (M + 15) / 16 - n_rows * (MT - 1), tall = MT == 4 && left < 1 ? n_rows : left;
     const int64_t blocks = (int64_t)n_rows * n_cols * parts;
-    SPY_REQUIRE(M >= MT * 16 && blocks < (1 << 30), "spy_gemm_rows: %d rows in tiles of %d, %lld blocks", M, MT * 16, (long long)blocks);
+    SPY_REQUIRE(M >= MT * 16 && tall >= 1 && tall <= n_rows && blocks < (1 << 30), "spy_gemm_rows: %d rows in %d tiles of %d, %lld blocks", M, n_rows, MT, (long long)blocks);
     const unsigned grid = (unsigned)((blocks + ROWS_DIES - 1) / ROWS_DIES * ROWS_DIES);
-    if (epi == ROWS_STORE) gemm_rows_kernel<MT, ROWS_STORE><<<grid, 256, 0, st>>>(C, (const bf16_t*)X, (const bf16_t*)W, M, N, K, n_rows, n_cols, 1, (int)blocks, act);
-    else if (epi == ROWS_GATED) gemm_rows_kernel<MT, ROWS_GATED><<<grid, 256, 0, st>>>(C, (const bf16_t*)X, (const bf16_t*)W, M, N, K, n_rows, n_cols, 1, (int)blocks, act);
-    else gemm_rows_kernel<MT, ROWS_PARTS><<<grid, 256, 0, st>>>(C, (const bf16_t*)X, (const bf16_t*)W, M, N, K, n_rows, n_cols, parts, (int)blocks, act);
+#define ROWS(EPI, PARTS) gemm_rows_kernel<MT, EPI><<<grid, 256, 0, st>>>(C, (const bf16_t*)X, (const bf16_t*)W, M, N, K, n_rows, tall, n_cols, PARTS, (int)blocks, act)
+    if (epi == ROWS_STORE) ROWS(ROWS_STORE, 1);
+    else if (epi == ROWS_GATED) ROWS(ROWS_GATED, 1);
+    else ROWS(ROWS_PARTS, parts);
+#undef ROWS
     SPY_CHECK_LAUNCH("spy_gemm_rows");
     return 0;
+}
+
+// Blocks that share a column's rows, of at most `most` row tiles each.  A compute unit's time is the row tiles of its blocks together, whether
+// they run beside or behind each other (1356 rows, 12288 x 2048: 720 blocks of six, three a unit, 65 us; 816 of five, four a unit, 72; 624 of
+// seven, three a unit, 70), so where it has two or more, as many blocks as leave its number of them what it is, and the rows dealt
+// evenly to them (409 rows, 19456 x 2560, six blocks of five and four 50.3 us, of five 51.4; 640 rows, six of seven and six 58.1 / 59.5).  With one a
+// unit the largest counts, and the fewest blocks stand.
+static int rows_blocks(int tiles, int most, int columns) {
+    const int fewest = (tiles + most - 1) / most, each = (int)(((int64_t)fewest * columns + 255) / 256);
+    if (each < 2) return fewest;
+    return max(fewest, (int)min((int64_t)256 * each / columns, (int64_t)tiles / 4));
 }
 
 // epi: what is formed (see the top): C bfloat16 [M, N], float32 [parts, M, N] or bfloat16 [M, N / 2].  X: bfloat16 rows [M, K]; W: the tiled copy of [N, K].  row_tiles: MT.
@@ -178,12 +205,14 @@ extern "C" int spy_gemm_rows(void* C, const void* X, const void* W, int M, int N
     SPY_REQUIRE(parts >= 1 && parts <= K / 128 && (parts == 1 || epi == ROWS_PARTS) && epi >= ROWS_STORE && epi <= ROWS_GATED, "spy_gemm_rows: %d parts of K = %d", parts, K);
     SPY_REQUIRE((((uintptr_t)C | (uintptr_t)X | (uintptr_t)W) % 16) == 0, "spy_gemm_rows: operands must be 16-byte aligned");
     SPY_REQUIRE(epi != ROWS_GATED || gate_act_of(act_code, &act), "spy_gemm_rows: unknown activation %d", act_code);
-    switch (row_tiles) {
-        case 4: return rows_launch<4>(C, X, W, M, N, K, parts, epi, act, st);
-        case 5: return rows_launch<5>(C, X, W, M, N, K, parts, epi, act, st);
-        case 6: return rows_launch<6>(C, X, W, M, N, K, parts, epi, act, st);
-        case 7: return rows_launch<7>(C, X, W, M, N, K, parts, epi, act, st);
-        case 8: return rows_launch<8>(C, X, W, M, N, K, parts, epi, act, st);
+    SPY_REQUIRE(row_tiles >= 4 && row_tiles <= 8, "spy_gemm_rows: %d row tiles", row_tiles);
+    const int tiles = (M + 15) / 16, n_rows = rows_blocks(tiles, row_tiles, (N + 255) / 256 * parts);
+    switch (max(4, (tiles + n_rows - 1) / n_rows)) {
+        case 4: return rows_launch<4>(C, X, W, M, N, K, n_rows, parts, epi, act, st);
+        case 5: return rows_launch<5>(C, X, W, M, N, K, n_rows, parts, epi, act, st);
+        case 6: return rows_launch<6>(C, X, W, M, N, K, n_rows, parts, epi, act, st);
+        case 7: return rows_launch<7>(C, X, W, M, N, K, n_rows, parts, epi, act, st);
+        case 8: return rows_launch<8>(C, X, W, M, N, K, n_rows, parts, epi, act, st);
     }
     return spy_fail("spy_gemm_rows: %d row tiles", row_tiles);
 }
