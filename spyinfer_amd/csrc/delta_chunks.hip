@@ -10,18 +10,20 @@
 //   delta_chunk_prepare   a block per (chunk, head): A, B, M and from them MV = M V, MW = M W, Q_t = G_t q_t, K_s = G_15 / G_s k_s (stored
 //                         [channel][token]), G_15, into a workspace.  The quotients of decays are never formed as quotients, which
 //                         underflow: they are powers of two of differences of sums of logarithms, sums in 64 bits.
-//   delta_chunk_walk      a block of four waves per (entry, head, 16 value channels); a wave has a quarter of the key channels' rows of
-//                         S in registers.  Per chunk, on v_mfma_f32_16x16x4_f32: its part of MW S0 and of Q S0, the parts of u met in
+//   delta_chunk_walk      a block per (entry, head, 16 value channels), a wave per 16 key channels, whose rows of S it has in
+//                         registers.  Per chunk, on v_mfma_f32_16x16x4_f32: its part of MW S0 and of Q S0, the parts of u met in
 //                         LDS, S = G_15 S + K^T u, and B u for the read-out, whose parts meet one chunk later.
 // The result's layout (lane (column r, g): rows 4 g + i) is the second operand's layout of the next product, so S and u go from product to
 // product without a move.  All of it is float32 (the sums of logarithms float64), as the token walk is.
-// What bounds it: the walk's chain of about 1000 cycles a chunk (8 products, LDS, 8 products), 94 times for 1500 tokens; the preparation's
-// 136 x d powers of two a chunk.  Chunks of 16 because a chunk's tokens are then one matrix tile; the preparation grows with the square.
-// Measured: 1500 tokens, 16 heads of 128 x 128: 51 us of preparation and 104 us of walk a layer against 1712 us token by token.
+// What bounds it: the walk's chain of about 2000 cycles a chunk (4 products, LDS, 4 products, the read-out's way through LDS), 94 times for
+// 1500 tokens, not its operands' way (95 us, 92 with every chunk's from one place); the preparation's 136 x d powers of two a chunk.  Chunks
+// of 16 because a chunk's tokens are then one matrix tile; the preparation grows with the square.
+// Measured: 1500 tokens, 16 heads of 128 x 128: 51 us of preparation and 95 us of walk a layer (104 by four waves with 32 key channels each)
+// against 1712 us token by token.
 // The mLSTM, S = a S + b k v^T with numbers a and b a token, is the same with nothing taken back: u = v, B_ts = b_s G_t / G_s (q_t . k_s), K_s =
 // b_s G_15 / G_s k_s, and its vector n = a n + b k goes along in the lanes' registers (a lane has the rows of n that it has of Q as an
-// operand, so n . q costs eight products a lane).  8 heads of 128 x 256, 1500 tokens: 190 us
-// a layer, scalars and preparation among it, against 765 for pieces of 64 tokens walked twice and folded.
+// operand, so n . q costs eight products a lane).  8 heads of 128 x 256, 1500 tokens: a walk
+// of 94 us (118 by four waves that asked for the read-out's two numbers a token where they needed them), 165 us a layer with scalars and preparation, against 765 for pieces of 64 tokens walked twice and folded.
 #include "delta_chunks.h"
 #include <math.h>
 
@@ -250,10 +252,11 @@ struct ChunkWalk {
 };
 
 template <int D, bool DELTA>
-__global__ __launch_bounds__(256) void chunk_walk_kernel(ChunkWalk a, int number0, int number1) {
-    constexpr int TI = D / 64;                              // tiles of 16 key channels that a wave has
-    __shared__ __align__(16) float pu[DELTA ? 2 : 1][4][64][4], po[2][4][64][4];
-    __shared__ float pn[2][4][16];
+__global__ __launch_bounds__(D * 4) void chunk_walk_kernel(ChunkWalk a, int number0, int number1) {
+    constexpr int W = D / 16;                               // waves, each with 16 key channels
+    constexpr int READ = W > 4 ? 4 : 0;                     // four waves multiply B by u (from 0 on), four read out (from here on)
+    __shared__ __align__(16) float pu[DELTA ? 2 : 1][W][64][4], po[2][W][64][4];
+    __shared__ float pn[2][W][16];
     const int e = blockIdx.x, h = blockIdx.y, col0 = blockIdx.z * 16;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int slot = a.slot_ids[e];
@@ -261,118 +264,121 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(ChunkWalk a, int number
     const int q0 = a.cu_q[e], q1 = a.cu_q[e + 1], first = dc_first(a.cu_q, e), chunks = (q1 - q0 + DC_TOKENS - 1) / DC_TOKENS;
     const int c0 = max(0, number0 - first), c1 = min(chunks, number1 - first);
     if (c0 >= c1) return;
-    const int row0 = wave * (D / 4) + 4 * g;                // lane (column r, g) has rows row0 + 16 i + e
+    const int row0 = wave * 16 + 4 * g;                     // lane (column r, g) has rows row0 .. row0 + 3
     float* head = a.state + (size_t)slot * a.slot_stride + (size_t)h * a.head_stride;
     float* st = head + col0 + r;
     float* nm = head + (size_t)D * a.dv + (size_t)blockIdx.z * (D + 1);          // (mLSTM)
-    dc_f32x4_t S[TI], N[TI];
+    dc_f32x4_t S, N;
 #pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-            S[i][x] = st[(size_t)(row0 + 16 * i + x) * a.dv];
-            N[i][x] = DELTA ? 0.f : nm[row0 + 16 * i + x];
-        }
+    for (int x = 0; x < 4; ++x) {
+        S[x] = st[(size_t)(row0 + x) * a.dv];
+        N[x] = DELTA ? 0.f : nm[row0 + x];
+    }
     const int rec = dc_record(D, a.dv);
     auto record = [&](int c) { return a.ws + ((size_t)(first + min(c, c1 - 1) - number0) * a.H + h) * rec; };
-    // this lane's operands of a chunk (mw: the mLSTM's sums of K)
-    struct Ops { dc_f32x4_t mw[TI], q[TI], k[TI], gl[TI], b, mv; };
+    // this lane's operands of a chunk (mw: the mLSTM's sums of K; nb, em: its row's sum of B and e^-m).  Their places in a record are
+    // 32-bit numbers that are worked out once, beside an address that the whole block has in common.
+    const int o_row = 4 * g + (wave & 3);                   // the row that the lane reads out
+    const unsigned at_mw = 4u * ((DELTA ? r * D : 0) + row0), at_q = 4u * (16 * D + r * D + row0), at_k = 4u * (32 * D + (wave * 16 + r) * 16 + 4 * g);
+    const unsigned at_b = 4u * (48 * D + 16 * a.dv + r * 16 + 4 * g), at_g = 4u * (48 * D + 16 * a.dv + 256 + row0), at_n = 4u * (D + o_row);
+    unsigned at_v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) at_v[i] = 4u * (48 * D + (4 * g + i) * a.dv + col0 + r);
+    struct Ops { dc_f32x4_t mw, q, k, gl, b, mv; float nb, em; };
     auto load = [&](Ops& x, int c) {
-        const float* p = record(c);
-        const float* mv = p + 48 * D + 4 * g * a.dv + col0 + r;
+        const char* p = reinterpret_cast<const char*>(record(c));
+        x.mw = *reinterpret_cast<const dc_f32x4_t*>(p + at_mw);
+        x.q = *reinterpret_cast<const dc_f32x4_t*>(p + at_q);
+        x.k = *reinterpret_cast<const dc_f32x4_t*>(p + at_k);
+        x.gl = *reinterpret_cast<const dc_f32x4_t*>(p + at_g);
+        x.b = *reinterpret_cast<const dc_f32x4_t*>(p + at_b);
 #pragma unroll
-        for (int i = 0; i < TI; ++i) {
-            x.mw[i] = *reinterpret_cast<const dc_f32x4_t*>(p + (DELTA ? r * D : 0) + row0 + 16 * i);
-            x.q[i] = *reinterpret_cast<const dc_f32x4_t*>(p + 16 * D + r * D + row0 + 16 * i);
-            x.k[i] = *reinterpret_cast<const dc_f32x4_t*>(p + 32 * D + (row0 - 4 * g + 16 * i + r) * 16 + 4 * g);
-            x.gl[i] = *reinterpret_cast<const dc_f32x4_t*>(p + 48 * D + 16 * a.dv + 256 + row0 + 16 * i);
-        }
-        x.b = *reinterpret_cast<const dc_f32x4_t*>(p + 48 * D + 16 * a.dv + r * 16 + 4 * g);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x.mv[i] = mv[(size_t)i * a.dv];
+        for (int i = 0; i < 4; ++i) x.mv[i] = *reinterpret_cast<const float*>(p + at_v[i]);
+        x.nb = DELTA ? 0.f : *reinterpret_cast<const float*>(p + at_n);
+        x.em = DELTA ? 0.f : *reinterpret_cast<const float*>(p + at_n + 64);
     };
-    // read-out of chunk c: the waves' parts, row 4 g + wave of lane (column r, g)
-    auto read_out = [&](int c) {
-        const int row = 4 * g + wave, t = q0 + c * DC_TOKENS + row;
+    // read-out of chunk c: the waves' parts, row o_row of column r
+    float* const o_at = a.o + (size_t)h * a.dv + col0 + r;
+    auto read_out = [&](int c, float nb, float em) {
+        const int t = q0 + c * DC_TOKENS + o_row;
         float y = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) y += po[c & 1][w][lane][wave];
+        for (int w = 0; w < W; ++w) y += po[c & 1][w][lane][wave & 3];
         if (!DELTA) {
-            const float* p = record(c) + D;
-            float nq = p[row];
+            float nq = nb;
 #pragma unroll
-            for (int w = 0; w < 4; ++w) nq += pn[c & 1][w][row];
-            y /= fmaxf(fabsf(nq), p[16 + row]) + 1e-6f;
+            for (int w = 0; w < W; ++w) nq += pn[c & 1][w][o_row];
+            y /= fmaxf(fabsf(nq), em) + 1e-6f;
         }
-        if (t < q1) a.o[((size_t)t * a.H + h) * a.dv + col0 + r] = y;
+        if (t < q1) o_at[(size_t)t * a.H * a.dv] = y;
     };
+    float nb = 0.f, em = 0.f;                               // of the chunk before
     auto chunk = [&](const Ops& x, int c) {
         dc_f32x4_t o0 = {0.f, 0.f, 0.f, 0.f}, o1 = {0.f, 0.f, 0.f, 0.f};
         if (DELTA) {
             dc_f32x4_t u0 = {0.f, 0.f, 0.f, 0.f}, u1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < TI; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; j += 2) {
-                    u0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[i][j], S[i][j], u0, 0, 0, 0);
-                    u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[i][j + 1], S[i][j + 1], u1, 0, 0, 0);
-                }
+            for (int j = 0; j < 4; j += 2) {
+                u0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[j], S[j], u0, 0, 0, 0);
+                u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[j + 1], S[j + 1], u1, 0, 0, 0);
+            }
             *reinterpret_cast<dc_f32x4_t*>(pu[DELTA ? c & 1 : 0][wave][lane]) = u0 + u1;
         }
-#pragma unroll
-        for (int i = 0; i < TI; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; j += 2) {
-                o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][j], S[i][j], o0, 0, 0, 0);
-                o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][j + 1], S[i][j + 1], o1, 0, 0, 0);
-            }
         float nq = 0.f;
         if (!DELTA) {
 #pragma unroll
-            for (int i = 0; i < TI; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) nq = fmaf(x.q[i][j], N[i][j], nq);        // lane (token r, g): its rows' share of n . q
+            for (int j = 0; j < 4; ++j) nq = fmaf(x.q[j], N[j], nq);        // lane (token r, g): its rows' share of n . q
             nq += __shfl_xor(nq, 16, 64);
             nq += __shfl_xor(nq, 32, 64);
 #pragma unroll
-            for (int i = 0; i < TI; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) N[i][j] = fmaf(x.gl[i][j], N[i][j], x.mw[i][j]);
+            for (int j = 0; j < 4; ++j) N[j] = fmaf(x.gl[j], N[j], x.mw[j]);
         }
         __syncthreads();                                    // parts of u of this chunk, and of the read-out of the chunk before
+        dc_f32x4_t parts[DELTA ? W : 1];
+        if (DELTA) {
+#pragma unroll
+            for (int w = 0; w < W; ++w) parts[w] = *reinterpret_cast<const dc_f32x4_t*>(pu[DELTA ? c & 1 : 0][w][lane]);
+        }
+        // (Q S0 runs while the parts of u come out of LDS)
+#pragma unroll
+        for (int j = 0; j < 4; j += 2) {
+            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[j], S[j], o0, 0, 0, 0);
+            o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[j + 1], S[j + 1], o1, 0, 0, 0);
+        }
         dc_f32x4_t u = x.mv;
         if (DELTA) {
 #pragma unroll
-            for (int w = 0; w < 4; ++w) u -= *reinterpret_cast<const dc_f32x4_t*>(pu[DELTA ? c & 1 : 0][w][lane]);
+            for (int w = 0; w < W; ++w) u -= parts[w];
         }
+        S *= x.gl;
 #pragma unroll
-        for (int i = 0; i < TI; ++i) S[i] *= x.gl[i];
+        for (int j = 0; j < 4; ++j) S = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[j], u[j], S, 0, 0, 0);
+        if (wave < 4) {
+            // of B u, this wave's share: tokens s = 4 g + wave
+            float bw = x.b[0], uw = u[0];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+            for (int j = 1; j < 4; ++j)
+                if (wave == j) { bw = x.b[j]; uw = u[j]; }
+            // (B is zero where a token does not read: infinities and NaN, which zero does not take away, go to the rows that do read them)
+            const bool odd = !(fabsf(uw) < INFINITY);
+            if (__any(odd)) {
+                const dc_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+                const dc_f32x4_t f = __builtin_amdgcn_mfma_f32_16x16x4f32(4 * g + wave <= r ? 1.f : 0.f, odd ? 1.f : 0.f, zero, 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < TI; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i][j], u[j], S[i], 0, 0, 0);
-        // of B u, this wave's share: tokens s = 4 g + wave
-        float bw = x.b[0], uw = u[0];
-#pragma unroll
-        for (int j = 1; j < 4; ++j)
-            if (wave == j) { bw = x.b[j]; uw = u[j]; }
-        // (B is zero where a token does not read: infinities and NaN, which zero does not take away, go to the rows that do read them)
-        const bool odd = !(fabsf(uw) < INFINITY);
-        if (__any(odd)) {
-            const dc_f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-            const dc_f32x4_t f = __builtin_amdgcn_mfma_f32_16x16x4f32(4 * g + wave <= r ? 1.f : 0.f, odd ? 1.f : 0.f, zero, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (f[i] > 0.f) o0[i] = __builtin_nanf("");
-            if (odd) uw = 0.f;
+                for (int i = 0; i < 4; ++i)
+                    if (f[i] > 0.f) o0[i] = __builtin_nanf("");
+                if (odd) uw = 0.f;
+            }
+            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(bw, uw, o0, 0, 0, 0);
         }
-        o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(bw, uw, o0, 0, 0, 0);
-        if (c > c0) read_out(c - 1);
+        if (wave >= READ && c > c0) read_out(c - 1, nb, em);
+        nb = x.nb;
+        em = x.em;
         // (the place was read for chunk c - 2 behind the barrier of chunk c - 1, which every wave has passed)
         *reinterpret_cast<dc_f32x4_t*>(po[c & 1][wave][lane]) = o0 + o1;
         if (!DELTA && g == 0) pn[c & 1][wave][r] = nq;
     };
-    Ops x0, x1;                                             // (three chunks' operands under way instead of one: no faster)
+    Ops x0, x1;                                             // (three chunks' operands under way instead of one: 97 to 105 us)
     load(x0, c0);
     int c = c0;
     for (; c + 2 <= c1; c += 2) {
@@ -383,14 +389,12 @@ __global__ __launch_bounds__(256) void chunk_walk_kernel(ChunkWalk a, int number
     }
     if (c < c1) chunk(x0, c);
     __syncthreads();
-    read_out(c1 - 1);
+    if (wave >= READ) read_out(c1 - 1, nb, em);
 #pragma unroll
-    for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int y = 0; y < 4; ++y) {
-            st[(size_t)(row0 + 16 * i + y) * a.dv] = S[i][y];
-            if (!DELTA && r == 0) nm[row0 + 16 * i + y] = N[i][y];
-        }
+    for (int y = 0; y < 4; ++y) {
+        st[(size_t)(row0 + y) * a.dv] = S[y];
+        if (!DELTA && r == 0) nm[row0 + y] = N[y];
+    }
     if (!DELTA && threadIdx.x == 0) nm[D] = a.mfin[(size_t)e * a.H + h];
 }
 
@@ -414,7 +418,7 @@ int delta_chunks(const DeltaChunks& a, int dtype, hipStream_t st) {
             chunk_walk_kernel<64, true><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
         } else {
             SPY_DISPATCH(dtype, TA, (delta_chunk_prepare_kernel<TA, 128><<<pgrid, 256, 0, st>>>(a, (int)n0)));
-            chunk_walk_kernel<128, true><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
+            chunk_walk_kernel<128, true><<<wgrid, 512, 0, st>>>(w, (int)n0, n1);
         }
         SPY_CHECK_LAUNCH("spy_delta_rule (chunks)");
     }
@@ -435,7 +439,7 @@ int memory_chunks(const MemoryChunks& a, int dtype, hipStream_t st) {
             chunk_walk_kernel<64, false><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
         } else {
             SPY_DISPATCH(dtype, TA, (memory_chunk_prepare_kernel<TA, 128><<<pgrid, 256, 0, st>>>(a, (int)n0)));
-            chunk_walk_kernel<128, false><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
+            chunk_walk_kernel<128, false><<<wgrid, 512, 0, st>>>(w, (int)n0, n1);
         }
         SPY_CHECK_LAUNCH("spy_mlstm (chunks)");
     }
