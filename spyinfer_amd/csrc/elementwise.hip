@@ -166,11 +166,15 @@ extern "C" int spy_embedding_sumsq(float* out, void* xw, float* ss, const void* 
 // ---------------------------------------------------------------------------------------------
 // x = resid[t] (+ delta[t] (+ delta2[t]));  rows == null: resid[t] = x.  out[r] = (x / sqrt(mean(x^2) + eps)) * w
 // (two addends: the results of two sublayers that read the same norm, summed in float32 before they meet the stream)
-// One block per row.  The row is read once and kept in registers (4 values per thread and pass,
-// up to NORM_PASSES passes); longer rows are read again for the second pass.
+// One block per row.  The row is read once and kept in registers (4 values per thread and pass, up to NP passes); longer rows (NP 0) are
+// read again for the second pass.  Few rows: as many threads as make one pass where they can, whose loads go
+// out together (a thread with several passes has one's under way at a time); rows that fill the chip by themselves do better in blocks
+// of 256.  Measured, us, several passes / one: 1 row of 1024 3.4 / 2.7, 4 of 2048 in float32 3.6 / 2.8, 409 of 2560 5.7 / 4.7, 611 of 1024 in float32
+// 4.3 / 3.8; 1356 of 2048 8.6 / 9.0, 2048 of 4096 17.0 / 19.5 (5.9 / 5.2 TB/s).  The line is two million values.
 #define NORM_PASSES 8
-template <typename TA, typename TW, bool VEC>
-__global__ void add_rmsnorm_kernel(float* __restrict__ resid, const TA* __restrict__ delta, const TA* __restrict__ delta2,
+inline int norm_threads(int H) { return min(1024, (H / 4 + 63) / 64 * 64); }       // (rows in pieces of four values)
+template <typename TA, typename TW, int NP>
+__global__ __launch_bounds__(1024) void add_rmsnorm_kernel(float* __restrict__ resid, const TA* __restrict__ delta, const TA* __restrict__ delta2,
                                    const TW* __restrict__ w, float eps, TA* __restrict__ out, const int* __restrict__ rows, int T,
                                    int H, int ld, const TA* __restrict__ gate, const TW* __restrict__ gbias, float mult,
                                    const float* __restrict__ base, const float* __restrict__ vec, const TW* __restrict__ w2,
@@ -205,12 +209,12 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ resid, const TA* __restri
     w += g0;
     if (w2) w2 += g0;
     const bool write_back = (dl || bs || vc) && !rows;
-    if (VEC) {
+    if constexpr (NP > 0) {
         // H % 4 == 0 and 16-byte aligned rows (checked by the launcher); the row fits the register passes
-        float v[NORM_PASSES][4];
+        float v[NP][4];
         float ss = 0.f;
 #pragma unroll
-        for (int p = 0; p < NORM_PASSES; ++p) {
+        for (int p = 0; p < NP; ++p) {
             const int i = (p * blockDim.x + threadIdx.x) * 4;
             if (i < H) {
                 Vec4<float>::load(x + i, v[p]);
@@ -253,7 +257,7 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ resid, const TA* __restri
         ss = block_sum(ss, red);
         const float scale = 1.0f / sqrtf(ss / (float)H + eps);
 #pragma unroll
-        for (int p = 0; p < NORM_PASSES; ++p) {
+        for (int p = 0; p < NP; ++p) {
             const int i = (p * blockDim.x + threadIdx.x) * 4;
             if (i < H) {
                 float w4[4], y[4];
@@ -312,28 +316,29 @@ extern "C" int spy_add_rmsnorm(float* resid, const void* delta, const void* delt
     SPY_REQUIRE(delta || !delta2, "spy_add_rmsnorm: a second addend without a first");
     const int H = ld / groups;
     const dim3 grid(n_out, groups);
-    const int threads = H >= 2048 ? 256 : (H >= 512 ? 128 : 64);
+    const int threads = (int64_t)n_out * ld > (2 << 20) ? (H >= 2048 ? 256 : (H >= 512 ? 128 : 64)) : norm_threads(H);
     const bool aligned = H % 4 == 0 && ((uintptr_t)resid % 16) == 0 && ((uintptr_t)delta % 16) == 0 && ((uintptr_t)delta2 % 16) == 0 && ((uintptr_t)w % 16) == 0 &&
                          ((uintptr_t)out % 16) == 0 && ((uintptr_t)gate % 16) == 0 && ((uintptr_t)gbias % 16) == 0 &&
                          ((uintptr_t)base % 16) == 0 && ((uintptr_t)vec % 16) == 0 && ((uintptr_t)w2 % 16) == 0 && ((uintptr_t)out2 % 16) == 0;
     const bool by_pieces = aligned && H <= threads * 4 * NORM_PASSES;
-    if (by_pieces) {
-        SPY_DISPATCH(out_dtype, TA, SPY_DISPATCH(w_dtype, TW, (add_rmsnorm_kernel<TA, TW, true><<<grid, threads, 0, st>>>(
-            resid, (const TA*)delta, (const TA*)delta2, (const TW*)w, eps, (TA*)out, rows, T, H, ld, (const TA*)gate, (const TW*)gbias, mult,
-            base, vec, (const TW*)w2, (TA*)out2))));
-    } else {
-        SPY_DISPATCH(out_dtype, TA, SPY_DISPATCH(w_dtype, TW, (add_rmsnorm_kernel<TA, TW, false><<<grid, 512, 0, st>>>(
-            resid, (const TA*)delta, (const TA*)delta2, (const TW*)w, eps, (TA*)out, rows, T, H, ld, (const TA*)gate, (const TW*)gbias, mult,
-            base, vec, (const TW*)w2, (TA*)out2))));
-    }
+#define NORM_LAUNCH(NP, THREADS)                                                                                            \
+    SPY_DISPATCH(out_dtype, TA, SPY_DISPATCH(w_dtype, TW, (add_rmsnorm_kernel<TA, TW, NP><<<grid, THREADS, 0, st>>>(         \
+        resid, (const TA*)delta, (const TA*)delta2, (const TW*)w, eps, (TA*)out, rows, T, H, ld, (const TA*)gate, (const TW*)gbias, mult, \
+        base, vec, (const TW*)w2, (TA*)out2))))
+    if (!by_pieces) { NORM_LAUNCH(0, 512); }
+    else if (H <= threads * 4) { NORM_LAUNCH(1, threads); }
+    else { NORM_LAUNCH(NORM_PASSES, threads); }
+#undef NORM_LAUNCH
     SPY_CHECK_LAUNCH("spy_add_rmsnorm");
     return 0;
 }
 
 // The same norm where the addend is still a product's parts [n_parts, T, H] (float32, gemm_rows.hip): resid += their sum, which is
-// not rounded before it meets the stream.  Bound by the parts' way through the caches; a thread asks for all pieces of two parts at once.
-template <typename TA, typename TW>
-__global__ void add_parts_rmsnorm_kernel(float* __restrict__ resid, const float* __restrict__ parts, int n_parts, const TW* __restrict__ w,
+// not rounded before it meets the stream.  Bound by the parts' way through the caches; a thread has one piece of a row of up
+// to 4096 values and asks for those of AHEAD parts at once.  Measured, us, several pieces of two parts / this: 409 rows of 2560 in six parts 10.6 /
+// 7.9, 1356 of 2048 in two 11.7 / 10.2, 2048 of 4096 in two 27.4 / 26.6, 611 of 1024 in float32 in six 8.0 / 5.7 (an eighth to a third of it the launch).
+template <typename TA, typename TW, int NP, int AHEAD>
+__global__ __launch_bounds__(1024) void add_parts_rmsnorm_kernel(float* __restrict__ resid, const float* __restrict__ parts, int n_parts, const TW* __restrict__ w,
                                          float eps, TA* __restrict__ out, const int* __restrict__ rows, int T, int H) {
     __shared__ float red[16];
     const int r = blockIdx.x;
@@ -348,31 +353,34 @@ __global__ void add_parts_rmsnorm_kernel(float* __restrict__ resid, const float*
     float* x = resid + (size_t)t * H;
     const float* pr = parts + (size_t)t * H;
     const size_t step = (size_t)T * H;
-    float v[NORM_PASSES][4], s[NORM_PASSES][4];
+    float v[NP][4], s[NP][4];
 #pragma unroll
-    for (int p = 0; p < NORM_PASSES; ++p) {
+    for (int p = 0; p < NP; ++p) {
         const int i = (p * blockDim.x + threadIdx.x) * 4;
         if (i < H) {
             Vec4<float>::load(x + i, v[p]);
             Vec4<float>::load(pr + i, s[p]);
         }
     }
-#pragma unroll 2
-    for (int k = 1; k < n_parts; ++k) {
+    for (int k0 = 1; k0 < n_parts; k0 += AHEAD) {
+        float a[AHEAD][NP][4];
 #pragma unroll
-        for (int p = 0; p < NORM_PASSES; ++p) {
-            const int i = (p * blockDim.x + threadIdx.x) * 4;
-            if (i < H) {
-                float a[4];
-                Vec4<float>::load(pr + k * step + i, a);
+        for (int k = 0; k < AHEAD; ++k)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) s[p][e] += a[e];
+            for (int p = 0; p < NP; ++p) {
+                const int i = (p * blockDim.x + threadIdx.x) * 4;
+                if (i < H) Vec4<float>::load(pr + min(k0 + k, n_parts - 1) * step + i, a[k][p]);
             }
-        }
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k)
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[p][e] += k0 + k < n_parts ? a[k][p][e] : 0.f;      // (in the order of the parts)
     }
     float ss = 0.f;
 #pragma unroll
-    for (int p = 0; p < NORM_PASSES; ++p) {
+    for (int p = 0; p < NP; ++p) {
         const int i = (p * blockDim.x + threadIdx.x) * 4;
         if (i < H) {
 #pragma unroll
@@ -386,7 +394,7 @@ __global__ void add_parts_rmsnorm_kernel(float* __restrict__ resid, const float*
     ss = block_sum(ss, red);
     const float scale = 1.0f / sqrtf(ss / (float)H + eps);
 #pragma unroll
-    for (int p = 0; p < NORM_PASSES; ++p) {
+    for (int p = 0; p < NP; ++p) {
         const int i = (p * blockDim.x + threadIdx.x) * 4;
         if (i < H) {
             float w4[4], y[4];
@@ -402,11 +410,16 @@ __global__ void add_parts_rmsnorm_kernel(float* __restrict__ resid, const float*
 extern "C" int spy_add_parts_rmsnorm(float* resid, const float* parts, int n_parts, const void* w, int w_dtype, float eps, void* out, int out_dtype,
                                      const int* rows, int n_out, int T, int H, hipStream_t st) {
     SPY_REQUIRE(n_out > 0 && T > 0 && H > 0 && n_parts > 0, "spy_add_parts_rmsnorm: empty operand");
-    const int threads = H >= 2048 ? 256 : (H >= 512 ? 128 : 64);
+    const int threads = norm_threads(H);
     SPY_REQUIRE(H % 4 == 0 && H <= threads * 4 * NORM_PASSES, "spy_add_parts_rmsnorm: rows of %d", H);
     SPY_REQUIRE((((uintptr_t)resid | (uintptr_t)parts | (uintptr_t)w | (uintptr_t)out) % 16) == 0, "spy_add_parts_rmsnorm: operands must be 16-byte aligned");
-    SPY_DISPATCH(out_dtype, TA, SPY_DISPATCH(w_dtype, TW, (add_parts_rmsnorm_kernel<TA, TW><<<n_out, threads, 0, st>>>(
-        resid, parts, n_parts, (const TW*)w, eps, (TA*)out, rows, T, H))));
+#define PARTS_LAUNCH(NP, AHEAD)                                                                                             \
+    SPY_DISPATCH(out_dtype, TA, SPY_DISPATCH(w_dtype, TW, (add_parts_rmsnorm_kernel<TA, TW, NP, AHEAD><<<n_out, threads, 0, st>>>( \
+        resid, parts, n_parts, (const TW*)w, eps, (TA*)out, rows, T, H))))
+    if (H > threads * 4) { PARTS_LAUNCH(NORM_PASSES, 1); }
+    else if (n_parts <= 3) { PARTS_LAUNCH(1, 2); }
+    else { PARTS_LAUNCH(1, 5); }
+#undef PARTS_LAUNCH
     SPY_CHECK_LAUNCH("spy_add_parts_rmsnorm");
     return 0;
 }
