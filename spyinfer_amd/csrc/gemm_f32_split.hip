@@ -6,6 +6,12 @@
 // values): K = 1024 1.9e-7, K = 2048 2.7e-7, in parts less; the float32 instructions' 2.9e-7 (gemm_f32.hip, whose chain ends every 256 of K).
 // GATED: W = [gate rows | up rows], C[M][N / 2] = act(gate) * up.
 //
+// Three of the six are of W's middle and low parts, which are zero where a matrix is a bfloat16 checkpoint's, widened: a block begins
+// without them, keeps the low halves' bits of all that it stages of W, and if any is set behind its first step or its last it forms the tile anew
+// with all six.  The sums are the same bit for bit; nothing about a matrix is kept from one block or call to the next.  Measured, us, a
+// matrix of float32 values (with all six from the start) / a widened one: 611 rows, 4096 x 1024 46.9 (44.3) / 31.2, 6144 x 1024 gated 51.5 (48.5) / 33.9,
+// 1024 x 3072 in parts 30.8 (27.8) / 21.8; 400 rows, 12288 x 2048 171 (151) / 108.
+//
 // A block splits its rows of A and W as it stages them: from memory into registers four steps of 32 of K ahead, from there as three planes
 // in operand order into the other of two LDS stages, while this step's products run.  128 x 128 values of C and eight waves
 // (two a SIMD, one block a compute unit) where the tiles fill the chip, else 64 x 64 and four waves, two blocks a compute unit.
@@ -15,6 +21,7 @@
 // Measured, us, gemm_f32.hip's float32 instructions / this: 611 rows, 4096 x 1024 67 / 44, 6144 x 1024 87 / 49 (157 TFLOP/s), 1024 x 3072 in
 // parts 44 / 28; 200 rows, 12288 x 2048 124 / 78, 2048 x 6144 in parts 61 / 38; 90 rows, 12288 x 2048 81 / 57.
 #include "gemm_f32.h"
+#include <type_traits>
 
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float gs_f32x4_t;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float gs_f32x16_t;
@@ -82,11 +89,24 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
                 f.v[p][e] = __builtin_bit_cast(gs_f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(p * ROWS < BM ? ares : wres, src[p] + 16 * e, k, 0));
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto stage = [&](Pieces& f, int s) {
+    // (WHOLE: W's values are taken to be bfloat16 numbers, whose middle and low parts are zero; `rest` keeps the bits that say otherwise)
+    uint32_t rest = 0;
+    auto stage = [&](Pieces& f, int s, auto whole) {
+        constexpr bool WHOLE = decltype(whole)::value;
         char* to = lds + (s & 1) * STAGE;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             gs_u32x4_t hi, mid, lo;
+            if (WHOLE && p * ROWS >= BM) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t x0 = __float_as_uint(f.v[p][e >> 1][(e & 1) * 2]), x1 = __float_as_uint(f.v[p][e >> 1][(e & 1) * 2 + 1]);
+                    hi[e] = __builtin_amdgcn_perm(x1, x0, 0x07060302);
+                    rest |= x0 | x1;
+                }
+                *reinterpret_cast<gs_u32x4_t*>(to + dst[p]) = hi;
+                continue;
+            }
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 uint32_t a, b, c;
@@ -100,15 +120,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
     };
     constexpr bool FOLD = NT * MT == 1;
     gs_f32x16_t big[NT][MT], small[NT][MT], sum;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) sum[e] = 0.f;
-#pragma unroll
-    for (int n = 0; n < NT; ++n)
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) big[n][m][e] = small[n][m][e] = 0.f;
-    auto products = [&](int s) {
+    auto products = [&](int s, auto whole) {
+        constexpr bool WHOLE = decltype(whole)::value;
         const char* from = lds + (s & 1) * STAGE + h * GS_PIECE + i * 16;
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
@@ -118,63 +131,85 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
 #pragma unroll
                 for (int m = 0; m < MT; ++m) a[m][q] = *reinterpret_cast<const gs_bf16x8_t*>(from + (wm * MT + m) * GS_GROUP + ks * 2 * GS_PIECE + q * PLANE);
 #pragma unroll
-                for (int n = 0; n < NT; ++n) w[n][q] = *reinterpret_cast<const gs_bf16x8_t*>(from + (BM / 32 + wn * NT + n) * GS_GROUP + ks * 2 * GS_PIECE + q * PLANE);
+                for (int n = 0; n < NT && (q == 0 || !WHOLE); ++n) w[n][q] = *reinterpret_cast<const gs_bf16x8_t*>(from + (BM / 32 + wn * NT + n) * GS_GROUP + ks * 2 * GS_PIECE + q * PLANE);
             }
 #define GS_MFMA(SUM, WQ, AQ)                                                                                                     \
     _Pragma("unroll") for (int n = 0; n < NT; ++n) _Pragma("unroll") for (int m = 0; m < MT; ++m)                                \
         SUM[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[n][WQ], a[m][AQ], SUM[n][m], 0, 0, 0);
             GS_MFMA(big, 0, 0)
             GS_MFMA(small, 0, 1)
-            GS_MFMA(small, 1, 0)
-            GS_MFMA(small, 1, 1)
+            if constexpr (!WHOLE) {
+                GS_MFMA(small, 1, 0)
+                GS_MFMA(small, 1, 1)
+            }
             GS_MFMA(small, 0, 2)
-            GS_MFMA(small, 2, 0)
-        }
-    };
-    Pieces f0, f1, f2, f3;
-    fetch(f0, 0);
-    fetch(f1, 1);
-    fetch(f2, 2);
-    fetch(f3, 3);
-    stage(f0, 0);
-    __syncthreads();
-    // step s runs from LDS stage s & 1; behind it the pieces of step s + 1 are split into the other one
-    int s = 0;
-#define GS_STEP(FREE, NEXT, S)        \
-    fetch(FREE, (S) + 4);             \
-    products(S);                      \
-    stage(NEXT, (S) + 1);             \
-    __builtin_amdgcn_sched_barrier(0);\
-    __syncthreads();
-    for (; s + 4 < steps; s += 4) {
-        GS_STEP(f0, f1, s)
-        GS_STEP(f1, f2, s + 1)
-        GS_STEP(f2, f3, s + 2)
-        GS_STEP(f3, f0, s + 3)
-        if (FOLD && (s & 28) == 28) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                sum[e] += big[0][0][e];
-                big[0][0][e] = 0.f;
+            if constexpr (!WHOLE) {
+                GS_MFMA(small, 2, 0)
             }
         }
-    }
-    products(s);
-    if (s + 1 < steps) {
-        stage(f1, s + 1);
+    };
+    // The tile's sums; false: `rest` says that W's values are no bfloat16 numbers, and the sums are of no use.  Step s runs from LDS stage s & 1;
+    // behind it the pieces of step s + 1 are split into the other one.
+    auto run = [&](auto whole) {
+        constexpr bool WHOLE = decltype(whole)::value;
+        // (block-wide, behind two barriers: the stages are free for the other way then)
+        auto others = [&]() { return WHOLE && __syncthreads_or((rest & 0xffffu) != 0); };
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sum[e] = 0.f;
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) big[n][m][e] = small[n][m][e] = 0.f;
+        Pieces f0, f1, f2, f3;
+        fetch(f0, 0);
+        fetch(f1, 1);
+        fetch(f2, 2);
+        fetch(f3, 3);
+        stage(f0, 0, whole);
+        if (others()) return false;
         __syncthreads();
-        products(s + 1);
-    }
-    if (s + 2 < steps) {
-        stage(f2, s + 2);
-        __syncthreads();
-        products(s + 2);
-    }
-    if (s + 3 < steps) {
-        stage(f3, s + 3);
-        __syncthreads();
-        products(s + 3);
-    }
+        int s = 0;
+#define GS_STEP(FREE, NEXT, S)        \
+    fetch(FREE, (S) + 4);             \
+    products(S, whole);               \
+    stage(NEXT, (S) + 1, whole);      \
+    __builtin_amdgcn_sched_barrier(0);\
+    __syncthreads();
+        for (; s + 4 < steps; s += 4) {
+            GS_STEP(f0, f1, s)
+            GS_STEP(f1, f2, s + 1)
+            GS_STEP(f2, f3, s + 2)
+            GS_STEP(f3, f0, s + 3)
+            if (FOLD && (s & 28) == 28) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    sum[e] += big[0][0][e];
+                    big[0][0][e] = 0.f;
+                }
+            }
+        }
+#undef GS_STEP
+        products(s, whole);
+        if (s + 1 < steps) {
+            stage(f1, s + 1, whole);
+            __syncthreads();
+            products(s + 1, whole);
+        }
+        if (s + 2 < steps) {
+            stage(f2, s + 2, whole);
+            __syncthreads();
+            products(s + 2, whole);
+        }
+        if (s + 3 < steps) {
+            stage(f3, s + 3, whole);
+            __syncthreads();
+            products(s + 3, whole);
+        }
+        return !others();
+    };
+    if (!run(std::true_type{})) run(std::false_type{});
     // A value beyond bfloat16's range, an infinity or a NaN does not split (its rest is a NaN): every sum that it is in is a NaN then
     bool bad = false;
 #pragma unroll

@@ -85,3 +85,25 @@ def test_values_that_cannot_be_cut(M, N, gated):
     assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out[want.isinf()], want[want.isinf()])
     # (96 values of up to 3.4e38 that cancel but for a rounding of the largest)
     assert bool(((out - want).abs() <= 96 * 2.0 ** -24 * (x.abs().double() @ w.abs().double().t()).float()[:, :want.shape[1]].clamp(min=1.0))[finite].all())
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 4100, 32), (130, 5441, 160), (611, 4096, 1024), (300, 1700, 4160)])
+@pytest.mark.parametrize("where", ["nowhere", "first", "inside", "last"])
+def test_matrices_of_bfloat16_values(M, N, K, where):
+    """A matrix whose values are bfloat16 numbers, but for one of a row: the other rows' results are those of the matrix without it, bit for
+    bit, whichever way their tiles went."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    x, w = operands(M, N, K, dev)
+    w = w.bfloat16().float()
+    whole = ops.linear(x, w)
+    assert bool(((whole.double() - x.double() @ w.double().t()).abs() <= bound(x, w)).all())
+    if where != "nowhere":
+        w[N - 1, {"first": 0, "inside": K // 2, "last": K - 1}[where]] = 1.0 + 2.0 ** -20
+    out = ops.linear(x, w)
+    assert torch.equal(out[:, :N - 1], whole[:, :N - 1])
+    assert bool(((out.double() - x.double() @ w.double().t()).abs() <= bound(x, w)).all())
+    parts = ops.linear_swiglu(x, w[:N // 2 * 2].contiguous())
+    g = x.double() @ w.double().t()
+    a, up = torch.nn.functional.silu(g[:, :N // 2]), g[:, N // 2:N // 2 * 2]
+    assert float((parts.double() - a * up).norm() / (a * up).norm()) < 1e-5
