@@ -1,11 +1,13 @@
 // C[M, N] = A[M, K] . W[N, K]^T in float32: products and sums of 32-bit numbers, no reduced-precision mode (the matrix cores'
 // float32 instructions multiply and add as fmaf does; gemm_f32_split.hip, which has most products of more than 32 rows, cuts the
-// numbers without loss).  Three kernels by the number of rows:
+// numbers without loss).  Four kernels by the number of rows:
 //
 //   few    (up to 8 rows)   bound by streaming W from memory: a block's waves share K, 64 lanes side by side along it.
 //   narrow (tens of rows)   bound by W from memory as well, but A's rows would be read once per row of W by the kernel above.
 //                           A block owns 16 rows of W and MT tiles of 16 rows of A; its eight waves take the chunks of 64 of K in
 //                           turn, operands straight from memory into v_mfma_f32_16x16x4_f32 registers, and add through LDS.
+//   held   (up to 32 rows of which K is a multiple of 512, up to 2048 or in parts of that)      the same for more tiles of W than compute
+//                           units, or for parts of K beside each other: a block stays, its waves keep A in registers.
 //   tile   (many rows that gemm_f32_split.hip does not take)      bound by the matrix cores (256 flops a cycle and compute unit).  Tiles of
 //                           A and W through LDS.
 //
@@ -235,6 +237,92 @@ __global__ __launch_bounds__(GF_WAVES * 64) void gemm_f32_narrow_kernel(const fl
         if (n0 + 4 * g + i < N) C[(size_t)m * N + n0 + 4 * g + i] = sum[i];
 }
 
+// ---- up to 32 rows, plenty of rows of W ------------------------------------------------------------------------------------------
+// Bound by W from memory, as few rows are, but with the matrix cores' arithmetic, and without the narrow kernel's reading of A once per 16
+// rows of W (as many bytes as W from 16 rows on: there 16 rows cost more than 9 at the same products).  A block of eight waves stays on its
+// compute unit: each wave keeps its eighth of K of all of A in registers (16 CH a row tile; CH chunks of 64 of K) and goes through every
+// so many-th tile of 16 rows of W, a chunk's registers filled for the next tile as soon as its products are done.  Waves add through LDS,
+// one barrier a tile.  `parts` parts of K go to blocks of their own, for results too narrow to give every compute unit a tile: C
+// [parts][M][N].  GATED: a tile is 8 rows of the gate and the same 8 of the other half.  us, the kernels it stands for / this, at 16 and at 32 rows:
+// 12288 x 2048 43 / 24.5 and 43 / 31, with its activation 45 / 23.5 and 45 / 29; 32768 x 2048 84 / 55 and 84 / 66; 151936 x 1024 196 / 144 and 196 /
+// 157 (8 rows 187 / 132); 6144 x 1024 11.6 / 9.9 and 15.2 / 13.6; in parts of 512 of K 1024 x 2048 10.1 / 4.9 and 7.7 / 6.0, 2048 x 6144 27.8 /
+// 14.1 and 21.9 / 18.9, 2560 x 4096 18.6 / 11.5 and 18.7 / 15.3.
+#define GF_HELD_WAVES 8
+template <int MT, int CH, bool GATED>
+__global__ __launch_bounds__(GF_HELD_WAVES * 64) void gemm_f32_held_kernel(const float* __restrict__ A, const float* __restrict__ W,
+                                                                           float* __restrict__ C, int M, int N, int K, int parts, GateAct act) {
+    constexpr int NC = GATED ? 8 : 16;                                            // columns of a tile
+    __shared__ float red[2][GF_HELD_WAVES][MT][64][4];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int r = lane & 15, g = lane >> 4;
+    const int part = blockIdx.x % parts, step = gridDim.x / parts, tiles = (N + NC - 1) / NC;
+    const int k0 = (part * GF_HELD_WAVES + wave) * 64 * CH + 4 * g;
+    C += (size_t)part * M * N;
+    int t = blockIdx.x / parts, turn = 0;
+    gf_f32x4_t w[CH][4], a[MT][CH][4], acc[MT];
+    auto row_of = [&](int t) {                                                    // rows beyond N or M: the last row's, not stored
+        const int n = min(t * NC + r % NC, N - 1);
+        return W + (size_t)(GATED && r >= NC ? N + n : n) * K + k0;
+    };
+    const float* wrow = row_of(t);
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) w[c][s] = gf_stream(wrow + c * 64 + 16 * s);
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) a[mt][c][s] = gf_load(A + (size_t)min(mt * 16 + r, M - 1) * K + k0 + c * 64 + 16 * s);
+    auto tile = [&](auto more) {
+        if (more) wrow = row_of(t + step);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[mt] = gf_f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) acc[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[c][s][j], a[mt][c][s][j], acc[mt], 0, 0, 0);
+            if (more) {                                                           // the next tile's, as soon as this chunk's registers are free
+#pragma unroll
+                for (int s = 0; s < 4; ++s) w[c][s] = gf_stream(wrow + c * 64 + 16 * s);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        // the waves' sums meet in one of two places; a wave that writes one again has passed the barrier behind its last reader
+        float (&to)[GF_HELD_WAVES][MT][64][4] = red[turn & 1];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) *reinterpret_cast<gf_f32x4_t*>(to[wave][mt][lane]) = acc[mt];
+        __syncthreads();
+        const int mt = (wave - turn * MT) & (GF_HELD_WAVES - 1);                   // (the waves take turns to add)
+        if (mt < MT) {
+            // lane (r, g) has C[row r][columns 4 g ..]; gated: columns 4 g .. of the gate for g < 2, lane + 32 the same of the other
+            gf_f32x4_t sum = *reinterpret_cast<const gf_f32x4_t*>(to[0][mt][lane]);
+#pragma unroll
+            for (int v = 1; v < GF_HELD_WAVES; ++v) sum += *reinterpret_cast<const gf_f32x4_t*>(to[v][mt][lane]);
+            if constexpr (GATED) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float up = __shfl_xor(sum[i], 32, 64);
+                    sum[i] = gated_value(act, sum[i], up);
+                }
+            }
+            const int m = mt * 16 + r;
+            if (m < M && 4 * g < NC) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (t * NC + 4 * g + i < N) C[(size_t)m * N + t * NC + 4 * g + i] = sum[i];
+            }
+        }
+    };
+    for (; t + step < tiles; t += step, ++turn) tile(std::true_type{});
+    tile(std::false_type{});
+}
+
 // ---- many rows ----------------------------------------------------------------------------------------------------------------
 // A tile of 64 x 64 of C per 256 threads, a wave a quarter of it (v_mfma_f32_32x32x2_f32, 64 cycles each).  Steps of 32 of K: two
 // steps' pieces of A and W are on their way to registers while this one's products run from LDS, two LDS stages, one barrier a
@@ -397,6 +485,19 @@ static void gf_few(const float* A, const float* W, float* C, int M, int N, int w
 #undef GF_FEW
 }
 
+static bool gf_held_takes(int M, int N, int K, int parts) { return M <= 32 && N < (1 << 30) && K % (512 * parts) == 0 && K / parts <= 2048; }
+
+// a block for each compute unit: another one brings A's values again and takes no part of the memory's time (12288 x 2048, 16 rows 24.5 us, two
+// blocks 28.9; 32 rows 31 / 40)
+template <bool GATED>
+static void gf_held(const float* A, const float* W, float* C, int M, int N, int K, int parts, GateAct act, hipStream_t st) {
+    const int tiles = (N + (GATED ? 7 : 15)) / (GATED ? 8 : 16), grid = parts * min(tiles, max(1, 256 / parts)), ch = K / parts / 512;
+#define GF_HELD(MT, CH) gemm_f32_held_kernel<MT, CH, GATED><<<grid, GF_HELD_WAVES * 64, 0, st>>>(A, W, C, M, N, K, parts, act)
+    if (M <= 16) { if (ch == 1) GF_HELD(1, 1); else if (ch == 2) GF_HELD(1, 2); else if (ch == 3) GF_HELD(1, 3); else GF_HELD(1, 4); }
+    else { if (ch == 1) GF_HELD(2, 1); else if (ch == 2) GF_HELD(2, 2); else if (ch == 3) GF_HELD(2, 3); else GF_HELD(2, 4); }
+#undef GF_HELD
+}
+
 int gemm_f32(const float* A, const float* W, float* C, int M, int N, int K, hipStream_t st) {
 #define GF_NARROW(MT) gemm_f32_narrow_kernel<MT><<<dim3(tiles16, (M + 16 * MT - 1) / (16 * MT)), GF_WAVES * 64, 0, st>>>(A, W, C, M, N, K)
 #define GF_TILE(KS) gemm_f32_tile_kernel<KS><<<((tm * tn + 7) / 8) * 8, 256 * KS, 0, st>>>(A, W, C, M, N, K, tm, tn, 1)
@@ -404,6 +505,10 @@ int gemm_f32(const float* A, const float* W, float* C, int M, int N, int K, hipS
     if (gemm_f32_split_takes(M, N, K, 1)) return gemm_f32_split(A, W, C, M, N, K, 1, st);
     if (gf_few_takes(M, N, K)) {
         gf_few<false>(A, W, C, M, N, N, K, GateAct{1.f, 0.f}, st);
+    } else if (gf_held_takes(M, N, K, 1) && N > 4096) {
+        // (from the first size on that gives a compute unit two tiles: 4112 x 1024, 16 rows, the narrow kernel 10.7 us, this 9.3, 32 rows 14.1 / 12.2,
+        // 4112 x 2048 17.9 / 16.0 and 25.0 / 21.4; with one tile a unit 4096 x 1024 7.4 / 7.6 and 9.1 / 11.0)
+        gf_held<false>(A, W, C, M, N, K, 1, GateAct{1.f, 0.f}, st);
     } else if (tm * tn < 160) {
         // Row tiles per block: as many as leave a block for every compute unit, W being read once per group of them (24 rows, 2048 x
         // 2048: 10.4 us with one, 13.1 with two; 4096 x 2048: 19.4 with one, 14.5 with two; 64 rows, 4096 x 1024: 20 / 15.3 / 13.9
@@ -424,14 +529,16 @@ int gemm_f32(const float* A, const float* W, float* C, int M, int N, int K, hipS
     return 0;
 }
 
-// act(A . Wgate^T) * (A . Wup^T) for up to eight rows and for those that gemm_f32_split.hip takes, W = [gate rows | up rows] of N each, without the [M][2 N] result in between.
+// act(A . Wgate^T) * (A . Wup^T) for up to eight rows, up to 32 where A is held, and for those that gemm_f32_split.hip takes, W = [gate rows | up rows] of N each, without the [M][2 N] result in between.
 extern "C" int spy_gemm_f32_gated(float* C, const float* A, const float* W, int M, int N, int K, int act_code, hipStream_t st) {
     GateAct act;
     SPY_REQUIRE(M > 0 && N > 0 && K > 0 && gate_act_of(act_code, &act), "spy_gemm_f32_gated: %d rows, activation %d", M, act_code);
     SPY_REQUIRE(gemm_f32_takes(A, W, C, M, N, K), "spy_gemm_f32_gated: operands of %d x %d x %d are not taken", M, N, K);
-    SPY_REQUIRE(M <= 8 || (N < (1 << 30) && gemm_f32_split_takes(M, 2 * N, K, 1)), "spy_gemm_f32_gated: %d rows of %d x %d are not taken", M, N, K);
-    if (M > 8) return gemm_f32_split_gated(A, W, C, M, 2 * N, K, act, st);
-    gf_few<true>(A, W, C, M, N, 2 * N, K, act, st);
+    const bool held = M > 8 && gf_held_takes(M, N, K, 1);
+    SPY_REQUIRE(M <= 8 || held || (N < (1 << 30) && gemm_f32_split_takes(M, 2 * N, K, 1)), "spy_gemm_f32_gated: %d rows of %d x %d are not taken", M, N, K);
+    if (held) gf_held<true>(A, W, C, M, N, K, 1, act, st);
+    else if (M > 8) return gemm_f32_split_gated(A, W, C, M, 2 * N, K, act, st);
+    else gf_few<true>(A, W, C, M, N, 2 * N, K, act, st);
     SPY_CHECK_LAUNCH("spy_gemm_f32_gated");
     return 0;
 }
@@ -445,6 +552,11 @@ extern "C" int spy_gemm_f32_parts(float* C, const float* A, const float* W, int 
     SPY_REQUIRE(M > 0 && N > 0 && K > 0 && parts >= 1 && parts <= (K + GF_BK - 1) / GF_BK, "spy_gemm_f32_parts: %d parts of %d x %d x %d", parts, M, N, K);
     SPY_REQUIRE(gemm_f32_takes(A, W, C, M, N, K), "spy_gemm_f32_parts: operands of %d x %d x %d are not taken", M, N, K);
     if (parts <= K / GF_BK && gemm_f32_split_takes(M, N, K, parts)) return gemm_f32_split(A, W, C, M, N, K, parts, st);
+    if (gf_held_takes(M, N, K, parts)) {
+        gf_held<false>(A, W, C, M, N, K, parts, GateAct{1.f, 0.f}, st);
+        SPY_CHECK_LAUNCH("spy_gemm_f32_parts");
+        return 0;
+    }
     const int tm = (M + 63) / 64, tn = (N + 63) / 64;
     const int64_t blocks = (int64_t)tm * tn * parts;
     SPY_REQUIRE(blocks < (1 << 28), "spy_gemm_f32_parts: too many blocks");

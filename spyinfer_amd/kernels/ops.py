@@ -561,11 +561,27 @@ def f32_rows_split(M: int, N: int, K: int, parts: int = 1) -> bool:
     return M > 32 and K % 32 == 0 and M * K < 1 << 29 and N * K < 1 << 29 and (parts > 1 or -(-M // 64) * -(-N // 64) >= 128)
 
 
+def f32_rows_held(M: int, K: int, parts: int = 1) -> bool:
+    """Whether the float32 kernel that keeps the rows in registers takes a product of more than eight (csrc/gemm_f32.hip, whose own rule this is)."""
+    return 8 < M <= 32 and K % (512 * parts) == 0 and K // parts <= 2048
+
+
+@functools.lru_cache(maxsize=1024)
+def f32_held_parts(M: int, N: int, K: int):
+    """Parts of K for that kernel where the next norm sums them, or None.  A part's blocks share the compute units; a block takes as many times
+    as it has tiles, and once more for its first, a part's length (16 rows, us, parts 1 / 2 / 4: 4096 x 2048 12.4 / 10.5 / 9.4; 2048 x 6144 with 3 /
+    4 / 6 / 12: 17.7 / 14.3 / 15.9 / 14.1; 1024 x 3072 with 2 / 3 / 6: 9.6 / 7.3 / 6.3).  Up to 4096 columns; wider ones give every unit several tiles."""
+    if N > 4096:
+        return None
+    fits = [p for p in range(2, 13) if f32_rows_held(M, K, p) and p * M * N * 4 <= PARTS_MAX_BYTES]
+    return min(fits, key=lambda p: K // 512 / p * (1 + -(-(-(-N // 16)) // (256 // p))) + 0.1 * p, default=None)
+
+
 @functools.lru_cache(maxsize=1024)
 def f32_product_parts(M: int, N: int, K: int):
     """Parts of K for a float32 product whose result the next norm sums from them, or None where one pass is the better one.  A part of a
     tile is a block: of 64 x 64 by the float32 instructions, its numbers fitted to 380 launches of 17 to 2048 rows (the choice is 0.13 % behind
-    the best on average, 6 % at most, the parts' sum counted; up to 16 rows the streaming kernel stands); of 128 x 128 (to 2048 of K) or 64 x
+    the best on average, 6 % at most, the parts' sum counted; up to 32 rows ``f32_held_parts`` comes first); of 128 x 128 (to 2048 of K) or 64 x
     64 by the kernel that splits values, with the estimate that it chooses its tile by.  Of its numbers of parts the smallest within 6 % of the
     best, which the estimate does not tell apart (611 rows, 1024 x 2048, with the sum: three parts 25.7 us, six 25.0)."""
     if M <= 16 or K % 4 or -(-M // 64) * -(-N // 64) >= 1 << 20:
@@ -652,10 +668,10 @@ class ProductParts:
 def linear_parts(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor] = None):
     """``linear_few``, or, where a product of many rows is better cut along K, its ``ProductParts``."""
     M, K = x.shape
-    if M <= 16:                        # (short steps are bound by their launches: nothing more is asked of them)
+    if M <= (8 if x.dtype == torch.float32 else 16):      # (short steps are bound by their launches: nothing more is asked of them)
         return linear_few(x, w, tiled)
     if x.dtype == torch.float32:
-        parts = f32_product_parts(M, w.shape[0], K)
+        parts = f32_held_parts(M, w.shape[0], K) or f32_product_parts(M, w.shape[0], K)
         if parts is not None and x.is_cuda and isinstance(w, torch.Tensor) and w.dtype == torch.float32 and x.is_contiguous() and w.is_contiguous() \
                 and (x.data_ptr() | w.data_ptr()) % 16 == 0 and w.shape[1] == K:
             _dev(x, w)
@@ -716,7 +732,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, tiled: Optional[torc
         hip().call("spy_gemm_skinny_swiglu", _ptr(x), _ptr(w_gate_up), _ptr(out), _code(out, "out"), ctypes.c_int(M),
                    ctypes.c_int(I), ctypes.c_int(K), ctypes.c_int(GATED_ACTIVATIONS[activation]), _Hip.stream())
         return out
-    if x.dtype == torch.float32 and (0 < M <= 8 or f32_rows_split(M, 2 * I, K)) and x.is_cuda and isinstance(w_gate_up, torch.Tensor) \
+    if x.dtype == torch.float32 and (0 < M <= 8 or (I > 2048 and f32_rows_held(M, K)) or f32_rows_split(M, 2 * I, K)) and x.is_cuda and isinstance(w_gate_up, torch.Tensor) \
             and w_gate_up.dtype == torch.float32 and K % 4 == 0 and x.is_contiguous() and w_gate_up.is_contiguous() and (x.data_ptr() | w_gate_up.data_ptr()) % 16 == 0:
         out = torch.empty((M, I), dtype=x.dtype, device=x.device)
         hip().call("spy_gemm_f32_gated", _ptr(out), _ptr(x), _ptr(w_gate_up), M, I, K, GATED_ACTIVATIONS[activation], _Hip.stream())

@@ -75,3 +75,12 @@ def test_float32_products_in_parts_that_split_values():
     assert ops.f32_rows_split(33, 8192, 1024) and not ops.f32_rows_split(32, 8192, 1024) and not ops.f32_rows_split(90, 4032, 1024)
     assert ops.f32_rows_split(90, 1024, 1024, 2) and not ops.f32_rows_split(600, 8192, 1000)
     assert ops.f32_product_parts(611, 1024, 3072) == 6 and ops.f32_product_parts(90, 2048, 2048) == 4
+
+
+def test_float32_products_in_parts_of_rows_that_are_held():
+    rng = random.Random(6)
+    for _ in range(2000):
+        M, N, K = rng.randint(1, 40), rng.randint(1, 5000), rng.choice((1, 8, 64)) * 64 * rng.randint(1, 40)
+        parts = ops.f32_held_parts.__wrapped__(M, N, K)
+        assert parts is None or (8 < M <= 32 and N <= 4096 and 2 <= parts <= 12 and K % (512 * parts) == 0 and K // parts <= 2048)
+    assert ops.f32_held_parts(16, 1024, 3072) == 6 and ops.f32_held_parts(16, 1024, 3000) is None and ops.f32_held_parts(33, 1024, 3072) is None
