@@ -125,10 +125,19 @@ inline bool gate_act_of(int code, GateAct* a) {
 __device__ __forceinline__ float gated_value(const GateAct& a, float z, float up) {
     return (z / (1.0f + expf(-(z * fmaf(a.c3 * z, z, a.c1))))) * up;
 }
-// The same where the result is rounded to bfloat16: the hardware's exponential and reciprocal (a unit or two in the last of 24 bits each, where
-// the result keeps 8) instead of the library's expf and a division, a dozen instructions for three dozen
+// The same by the hardware's exponential and reciprocal, each with what it leaves out added back: the rest of s log2 e, which a rounded
+// product loses (|s| / 2 units of 2^-24 of the exponential), and the quotient's remainder.  18 instructions for expf and a division's 29.  Against 64 bits,
+// in units of 2^-24 of the result, largest / root of the mean square, above / this: silu, |z| up to 1 3.26 0.803 / 3.26 0.804, up to 8 8.1 1.63 /
+// 4.0 0.88, up to 30 24.5 5.5 / 4.5 0.84, z of -87 to -60 47 26 / 4.6 0.99; gelu_tanh, whose s is rounded before, up to 1 4.7 0.88 / 4.7 0.88, up to 8
+// 135 11.9 / 95 10.1.  Quarters of both sides keep the reciprocal of what is beyond 2^126 above the smallest normal number; infinities, NaN
+// and exponentials that overflow come out as above.
 __device__ __forceinline__ float gated_value_short(const GateAct& a, float z, float up) {
-    return z * __builtin_amdgcn_rcpf(1.0f + __expf(-(z * fmaf(a.c3 * z, z, a.c1)))) * up;
+    // (beyond 126 the exponential is an infinity or nothing beside one; a NaN stays one)
+    const float s = __builtin_elementwise_maximum(__builtin_elementwise_minimum(-(z * fmaf(a.c3 * z, z, a.c1)), 126.0f), -126.0f);
+    const float h = s * 1.44269504f, rest = fmaf(s, 1.925963033e-8f, fmaf(s, 1.44269504f, -h));
+    const float d = fmaf(__builtin_amdgcn_exp2f(h), fmaf(rest, 0.693147181f, 1.0f), 1.0f);
+    const float d4 = 0.25f * d, z4 = 0.25f * z, r = __builtin_amdgcn_rcpf(d4), q = z4 * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d4, q, z4), r, q), d, z) * up;
 }
 
 // Dispatch on a dtype code: binds `T` in `body`.

@@ -495,7 +495,7 @@ __global__ void swiglu_vec_kernel(const TA* __restrict__ in, TA* __restrict__ ou
 
 // bfloat16, 8 values per thread and step: 16-byte loads that do not stay in the caches (the product's output passes
 // once), one 16-byte store (the next product reads it).  Bound by its instructions with the library's expf and a division: 2048 x 2 x
-// 12288 31.5 us, by gated_value_short 26.7 (5.7 TB/s).
+// 12288 30.4 us, by gated_value_short 27.6 (5.5 TB/s).
 __global__ void swiglu_bf16x8_kernel(const bf16_t* __restrict__ in, bf16_t* __restrict__ out, int T, int I8, GateAct act) {
     typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
     const size_t n = (size_t)T * I8, I = (size_t)I8 * 8;

@@ -209,6 +209,7 @@ __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         float v = acc[0][i];
+        // (gated_value_short: 1 row, 6144 x 1024 5.43 -> 5.32 us; from 17 rows on its gain is below half a per cent, and the library stands)
         if (EPI == EPI_GATED) v = sizeof(TC) == 2 ? gated_value_short(gact, v, acc[NT - 1][i]) : gated_value(gact, v, acc[NT - 1][i]);
         if (act) v = xielu_f(v, act_p, act_q);
         if (gelu) v = gelu_f(v);
@@ -395,7 +396,7 @@ __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_rows_kernel(
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 float v = acc[ct][mt][i];
-                if (EPI == EPI_GATED) v = sizeof(TC) == 2 ? gated_value_short(gact, v, acc[CT + ct][mt][i]) : gated_value(gact, v, acc[CT + ct][mt][i]);
+                if (EPI == EPI_GATED) v = gated_value(gact, v, acc[CT + ct][mt][i]);
                 if (act) v = xielu_f(v, act_p, act_q);
                 if (gelu) v = gelu_f(v);
                 out[i] = from_f32<TC>(v);

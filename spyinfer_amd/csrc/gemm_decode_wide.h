@@ -195,7 +195,7 @@ __global__ __launch_bounds__(GW * 64, 1) void gemm_decode_wide_kernel(
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         float y = v[i] * scale;
-                        if (EPI == EPI_GATED) y = sizeof(TC) == 2 ? gated_value_short(gact, y, up[i] * scale) : gated_value(gact, y, up[i] * scale);
+                        if (EPI == EPI_GATED) y = gated_value(gact, y, up[i] * scale);
                         out[i] = from_f32<TC>(y);
                     }
                 }

@@ -18,7 +18,7 @@
 // 2560 x 4096: 23.8, 17.2 + 4; 200 rows, 4096 x 12288: 50.7, 31.2 + 6; 800 rows, 2048 x 6144: 39.0, 28.4 + 4.  Gated, with the
 // library's activation pass: 409 rows, 19456 x 2560: 53.2 + 8, 57.7; 1356 rows, 12288 x 2048: 85.6 + 13, 70.7 (965 TFLOP/s); 130 rows,
 // 19456 x 2560: 40.8 + 5, 33.2.
-// (Each with expf and a division in the epilogue; with gated_value_short 409 rows 55.5 -> 53.9, 1356 rows 69.8 -> 65.0, 2048 rows, 24576 x 4096 332 -> 314.)
+// (Each with expf and a division in the epilogue; with gated_value_short 409 rows 46.1 -> 45.1, 1356 rows 65.4 -> 63.5, 2048 rows, 24576 x 4096 333 -> 323.)
 // What bounds it: a turn takes 0.7 + 0.05 MT us, its 16 MT products per SIMD 0.11 MT us of that at four waves a compute unit; the rest
 // is the loads' way, from memory where few tiles share W, and the turn's barrier.
 #include "common.h"

@@ -159,7 +159,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const bf16_t* _
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float gt = acc[0][mt][i], up = acc[NT - 1][mt][i];
-                if (n + i < N) out[i] = from_f32<TC>(sizeof(TC) == 2 ? gated_value_short(gact, gt, up) : gated_value(gact, gt, up));
+                if (n + i < N) out[i] = from_f32<TC>(gated_value(gact, gt, up));
             }
         }
         return;
