@@ -210,34 +210,45 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
         return !others();
     };
     if (!run(std::true_type{})) run(std::false_type{});
-    // A value beyond bfloat16's range, an infinity or a NaN does not split (its rest is a NaN): every sum that it is in is a NaN then
-    bool bad = false;
+    // A value beyond bfloat16's range, an infinity or a NaN does not split (its rest is a NaN): every sum that it is in is a NaN then, and is
+    // formed once more by float32 instructions; the wave's other values stay
+    uint32_t again[NT][MT];
+    bool any = false;
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
+        for (int m = 0; m < MT; ++m) {
+            again[n][m] = 0;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 big[n][m][e] += FOLD ? small[n][m][e] + sum[e] : small[n][m][e];
-                bad |= !(fabsf(big[n][m][e]) < INFINITY);
+                again[n][m] |= fabsf(big[n][m][e]) < INFINITY ? 0u : 1u << e;
             }
-    if (__any(bad)) {
-        // the wave's values once more by float32 instructions
+            any |= again[n][m] != 0;
+        }
+    if (__any(any)) {
 #pragma unroll
         for (int n = 0; n < NT; ++n)
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
-                const float* a_at = A + (size_t)min(m0 + (wm * MT + m) * 32 + i, M - 1) * K;
-                const float* w_at = W + (size_t)w_row((wn * NT + n) * 32 + i) * K;
-                gs_f32x16_t acc;
+                const float* a_at = A + (size_t)min(m0 + (wm * MT + m) * 32 + i, M - 1) * K + 4 * h;
+                const float* w_at = W + (size_t)w_row((wn * NT + n) * 32 + i) * K + 4 * h;
+                gs_f32x16_t total, acc;
 #pragma unroll
-                for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-                for (int k = step0 * GS_BK; k < (step0 + steps) * GS_BK; k += 8) {
-                    const gs_f32x4_t va = *reinterpret_cast<const gs_f32x4_t*>(a_at + k + 4 * h), vw = *reinterpret_cast<const gs_f32x4_t*>(w_at + k + 4 * h);
+                for (int e = 0; e < 16; ++e) total[e] = acc[e] = 0.f;
+                const int end = (step0 + steps) * GS_BK;
+                for (int k0 = step0 * GS_BK; k0 < end; k0 += 256) {                // a chain ends every 256 of K, as in gemm_f32.hip
+#pragma unroll 4
+                    for (int k = k0; k < min(k0 + 256, end); k += 8) {
+                        const gs_f32x4_t va = *reinterpret_cast<const gs_f32x4_t*>(a_at + k), vw = *reinterpret_cast<const gs_f32x4_t*>(w_at + k);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(vw[j], va[j], acc, 0, 0, 0);
+                        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(vw[j], va[j], acc, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) { total[e] += acc[e]; acc[e] = 0.f; }
                 }
-                big[n][m] = acc;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) big[n][m][e] = again[n][m] >> e & 1 ? total[e] : big[n][m][e];
             }
     }
     // lane (i, h) has C[row i][columns 8 q + 4 h .. + 3], q < 4; GATED: gate values at q < 2, the same columns' up values at q + 2

@@ -107,3 +107,29 @@ def test_matrices_of_bfloat16_values(M, N, K, where):
     g = x.double() @ w.double().t()
     a, up = torch.nn.functional.silu(g[:, :N // 2]), g[:, N // 2:N // 2 * 2]
     assert float((parts.double() - a * up).norm() / (a * up).norm()) < 1e-5
+
+
+@pytest.mark.parametrize("M,N", [(65, 5000), (611, 5000)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_neighbours_of_values_that_cannot_be_cut(M, N, gated):
+    """Rows and columns beside an infinity, a NaN or a value beyond bfloat16's range are bit for bit what they are without it; and the results
+    of a row with such a value that a zero of the matrix takes away are as exact as others."""
+    from spyinfer_amd.kernels import ops
+    dev, K = require_gpu(), 2080
+    g = torch.Generator().manual_seed(M + N)
+    x, w = torch.randn((M, K), generator=g).to(dev), (torch.randn((N, K), generator=g) * K ** -0.5).to(dev)
+    w[:, 1030] = 0.0
+    product = ops.linear_swiglu if gated else ops.linear
+    before = product(x, w)
+    y, v = x.clone(), w.clone()
+    y[3, 77], y[M - 1, 2079], y[40, 1030] = float("inf"), float("nan"), 3.4e38
+    v[N // 2 + 9, 5], v[20, 1000] = float("-inf"), float("nan")
+    out = product(y, v)
+    rows, columns = torch.ones(M, dtype=torch.bool), torch.ones(out.shape[1], dtype=torch.bool)
+    rows[[3, 40, M - 1]], columns[[9 if gated else N // 2 + 9, 20]] = False, False
+    assert torch.equal(out[rows][:, columns], before[rows][:, columns])
+    if not gated:
+        want = x[40].double() @ w.double().t()
+        columns = columns.to(dev)
+        # (the chains of float32 instructions end every 256 of K: 2.9e-7 as gemm_f32.hip has it; one chain over all of K has 8e-7)
+        assert float((out[40].double() - want)[columns].norm() / want[columns].norm()) < 4e-7
