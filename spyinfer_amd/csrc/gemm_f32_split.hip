@@ -33,8 +33,9 @@ typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t gs_u32x4
 #define GS_PIECE 576          // bytes of 32 rows of 8 values of K in one plane, 64 of them unused
 #define GS_GROUP (4 * GS_PIECE)
 
-// x = high + middle + low, each a bfloat16, exactly; two values at a time
-__device__ __forceinline__ void gs_split(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+// x = high + middle + low, each a bfloat16, two values at a time.  What the low part is rounded from has eight bits at most and the same
+// smallest exponent as a bfloat16, so nothing is lost unless its 24 - 8 last bits are beyond that exponent: those bits go to `lost`.
+__device__ __forceinline__ void gs_split(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l, uint32_t& lost) {
     h = pack_bf16x2(x0, x1);
     x0 -= __uint_as_float(h << 16);
     x1 -= __uint_as_float(h & 0xffff0000u);
@@ -42,6 +43,7 @@ __device__ __forceinline__ void gs_split(float x0, float x1, uint32_t& h, uint32
     x0 -= __uint_as_float(m << 16);
     x1 -= __uint_as_float(m & 0xffff0000u);
     l = pack_bf16x2(x0, x1);
+    lost |= __float_as_uint(x0) | __float_as_uint(x1);
 }
 
 template <int BM, int BN, int WM, int WN, bool GATED>
@@ -90,7 +92,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
         __builtin_amdgcn_sched_barrier(0);
     };
     // (WHOLE: W's values are taken to be bfloat16 numbers, whose middle and low parts are zero; `rest` keeps the bits that say otherwise)
-    uint32_t rest = 0;
+    uint32_t rest = 0, lost[P] = {};
     auto stage = [&](Pieces& f, int s, auto whole) {
         constexpr bool WHOLE = decltype(whole)::value;
         char* to = lds + (s & 1) * STAGE;
@@ -110,7 +112,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 uint32_t a, b, c;
-                gs_split(f.v[p][e >> 1][(e & 1) * 2], f.v[p][e >> 1][(e & 1) * 2 + 1], a, b, c);
+                gs_split(f.v[p][e >> 1][(e & 1) * 2], f.v[p][e >> 1][(e & 1) * 2 + 1], a, b, c, lost[p]);
                 hi[e] = a; mid[e] = b; lo[e] = c;
             }
             *reinterpret_cast<gs_u32x4_t*>(to + dst[p]) = hi;
@@ -210,10 +212,22 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
         return !others();
     };
     if (!run(std::true_type{})) run(std::false_type{});
-    // A value beyond bfloat16's range, an infinity or a NaN does not split (its rest is a NaN): every sum that it is in is a NaN then, and is
-    // formed once more by float32 instructions; the wave's other values stay
+    // Two kinds of values do not split, and the sums that they are in are formed once more by float32 instructions, the wave's other values
+    // stay: those beyond bfloat16's range, infinities and NaN, whose rest is a NaN as every sum with it then, and those below 2^-110 or so, of
+    // which bits are lost: their rows of A and W
     uint32_t again[NT][MT];
     bool any = false;
+    uint32_t short_of = 0;
+#pragma unroll
+    for (int p = 0; p < P; ++p) short_of |= lost[p];
+    const bool shorts = __syncthreads_or((short_of & 0xffffu) != 0);                // (and the stages are free)
+    uint32_t* row_lost = reinterpret_cast<uint32_t*>(lds);                          // [BM + BN][4]
+    if (shorts) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) row_lost[(sr + p * ROWS) * 4 + kp] = lost[p] & 0xffffu;
+        __syncthreads();
+    }
+    auto lost_in = [&](int row) { const gs_u32x4_t f = *reinterpret_cast<const gs_u32x4_t*>(row_lost + row * 4); return (f[0] | f[1] | f[2] | f[3]) != 0; };
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
@@ -223,6 +237,11 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
             for (int e = 0; e < 16; ++e) {
                 big[n][m][e] += FOLD ? small[n][m][e] + sum[e] : small[n][m][e];
                 again[n][m] |= fabsf(big[n][m][e]) < INFINITY ? 0u : 1u << e;
+            }
+            if (shorts) {
+                if (lost_in((wm * MT + m) * 32 + i)) again[n][m] = 0xffffu;
+                for (int e = 0; e < 16; ++e)
+                    if (lost_in(BM + (wn * NT + n) * 32 + 8 * (e >> 2) + 4 * h + (e & 3))) again[n][m] |= 1u << e;
             }
             any |= again[n][m] != 0;
         }
