@@ -1,16 +1,21 @@
 // Products of many float32 rows, C[M, N] = A[M, K] . W[N, K]^T, on the matrix cores' bfloat16 instructions, which multiply sixteen times
-// as much in a cycle as their float32 ones do.  Every value is cut into three bfloat16 parts, x = high + middle + low, exactly (8 + 8 + 8
+// as much in a cycle as their float32 ones do.  Every value is cut into three bfloat16 parts, x = high + middle + low (8 + 8 + 8
 // bits, each part the rounded rest of those before it), a product of two parts is exact in float32, and of the nine products of parts
 // the six from 2^-18 of the result on are formed: high high apart, high middle, middle high, middle middle, high low and low high
-// in a second sum; what is left out is below 2^-26 of |a||w|, a quarter of one rounding in float32.  Relative errors against 64 bits (2-norm, normal
+// in a second sum.  What is left out is at most 2^-24 of |a||w|, one rounding in float32 (middle parts are up to 2^-8 of a value, low ones
+// 2^-17), and 2^-27.4 in the root of the mean square.  Relative errors against 64 bits (2-norm, normal
 // values): K = 1024 1.9e-7, K = 2048 2.7e-7, in parts less; the float32 instructions' 2.9e-7 (gemm_f32.hip, whose chain ends every 256 of K).
+// The cut loses nothing down to about 2^-110, where low parts meet bfloat16's smallest number; sums with smaller values, infinities, NaN or what
+// bfloat16 rounds to infinity are formed by float32 instructions (at the end).
 // GATED: W = [gate rows | up rows], C[M][N / 2] = act(gate) * up.
 //
 // Three of the six are of W's middle and low parts, which are zero where a matrix is a bfloat16 checkpoint's, widened: a block begins
-// without them, keeps the low halves' bits of all that it stages of W, and if any is set behind its first step or its last it forms the tile anew
-// with all six.  The sums are the same bit for bit; nothing about a matrix is kept from one block or call to the next.  Measured, us, a
-// matrix of float32 values (with all six from the start) / a widened one: 611 rows, 4096 x 1024 46.9 (44.3) / 31.2, 6144 x 1024 gated 51.5 (48.5) / 33.9,
-// 1024 x 3072 in parts 30.8 (27.8) / 21.8; 400 rows, 12288 x 2048 171 (151) / 108.
+// without them, keeps the low halves' bits of all that it stages of W, and looks at them behind its first step, every eighth and its last.  If
+// any is set, what the steps since the last look left out is added and the others are formed with all six.  Rows of W without such bits have the
+// same sums bit for bit either way; nothing about a matrix is kept from one block or call to the next.  Measured, us, a widened matrix / one of
+// float32 values / widened but for its last 32 of K / for its second half: 611 rows, 4096 x 1024 30.0 / 41 / 38 / 44, 6144 x 1024 gated 34 / 50 / 42.5 /
+// 51; 400 rows, 4096 x 2048 43.5 / 61 / 48.5 / 56, 12288 x 2048 gated 106 / 162 / 125 / 149; 90 rows, 4096 x 2048 30.5 / 38.4 / 34.8 / 39.1 (tiles anew from the
+// start cost 61.6, 72, 91, 240 and 64 for the last two).  A look behind each step, and on from there, took 2 to 3 us of a widened 4096 x 1024.
 //
 // A block splits its rows of A and W as it stages them: from memory into registers four steps of 32 of K ahead, from there as three planes
 // in operand order into the other of two LDS stages, while this step's products run.  128 x 128 values of C and eight waves
@@ -33,17 +38,19 @@ typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t gs_u32x4
 #define GS_PIECE 576          // bytes of 32 rows of 8 values of K in one plane, 64 of them unused
 #define GS_GROUP (4 * GS_PIECE)
 
-// x = high + middle + low, each a bfloat16, two values at a time.  What the low part is rounded from has eight bits at most and the same
-// smallest exponent as a bfloat16, so nothing is lost unless its 24 - 8 last bits are beyond that exponent: those bits go to `lost`.
-__device__ __forceinline__ void gs_split(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l, uint32_t& lost) {
-    h = pack_bf16x2(x0, x1);
-    x0 -= __uint_as_float(h << 16);
-    x1 -= __uint_as_float(h & 0xffff0000u);
+// Middle and low parts of what is left of two values behind their high ones.  What the low part is rounded from has eight bits at most and the
+// same smallest exponent as a bfloat16, so nothing is lost unless its 24 - 8 last bits are beyond that exponent: those bits go to `lost`.
+__device__ __forceinline__ void gs_split_rest(float x0, float x1, uint32_t& m, uint32_t& l, uint32_t& lost) {
     m = pack_bf16x2(x0, x1);
     x0 -= __uint_as_float(m << 16);
     x1 -= __uint_as_float(m & 0xffff0000u);
     l = pack_bf16x2(x0, x1);
     lost |= __float_as_uint(x0) | __float_as_uint(x1);
+}
+// x = high + middle + low, each a bfloat16, two values at a time
+__device__ __forceinline__ void gs_split(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l, uint32_t& lost) {
+    h = pack_bf16x2(x0, x1);
+    gs_split_rest(x0 - __uint_as_float(h << 16), x1 - __uint_as_float(h & 0xffff0000u), m, l, lost);
 }
 
 template <int BM, int BN, int WM, int WN, bool GATED>
@@ -53,6 +60,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
     constexpr int PLANE = (BM + BN) / 32 * GS_GROUP, STAGE = 3 * PLANE;
     static_assert(BM % ROWS == 0 && BN % ROWS == 0, "a thread's piece is of A or of W for the whole block");
     __shared__ __align__(16) char lds[2 * STAGE];
+    __shared__ uint32_t no_bf16;                       // whether a value of W is no bfloat16 number
     const int tiles = tiles_m * tiles_n, total = tiles * parts, per = (total + 7) >> 3;
     const int at = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per || at >= total) return;
@@ -79,10 +87,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
         src[p] = ((p * ROWS < BM ? min(m0 + row, M - 1) : w_row(row - BM)) * K + kp * 8) * 4;
         dst[p] = (row >> 5) * GS_GROUP + kp * GS_PIECE + (row & 31) * 16;
     }
-    const int all_steps = K / GS_BK, step0 = (int)((long long)all_steps * k_part / parts);
-    const int steps = (int)((long long)all_steps * (k_part + 1) / parts) - step0;
+    const int all_steps = K / GS_BK, part0 = (int)((long long)all_steps * k_part / parts), part1 = (int)((long long)all_steps * (k_part + 1) / parts);
+    int step0 = part0, steps = part1 - part0;          // what is still to do of the part
     struct Pieces { gs_f32x4_t v[P][2]; };
-    auto fetch = [&](Pieces& f, int s) {
+    auto fetch = [&](Pieces& f, int s) __attribute__((always_inline)) {
         const int k = (step0 + min(s, steps - 1)) * GS_BK * 4;
 #pragma unroll
         for (int p = 0; p < P; ++p)
@@ -91,39 +99,44 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
                 f.v[p][e] = __builtin_bit_cast(gs_f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(p * ROWS < BM ? ares : wres, src[p] + 16 * e, k, 0));
         __builtin_amdgcn_sched_barrier(0);
     };
-    // (WHOLE: W's values are taken to be bfloat16 numbers, whose middle and low parts are zero; `rest` keeps the bits that say otherwise)
+    // Ways to form a step.  WHOLE: W's values are taken to be bfloat16 numbers, whose middle and low parts are zero; `rest` keeps the bits that
+    // say otherwise.  FULL: all six products.  REST: what WHOLE left out of a step where it does say otherwise: its high part is the value cut off
+    // behind 16 bits, so that the middle part here is up to 2^-7 of the value, and its product with A's low part comes along.
+    enum Way { WHOLE, FULL, REST };
     uint32_t rest = 0, lost[P] = {};
-    auto stage = [&](Pieces& f, int s, auto whole) {
-        constexpr bool WHOLE = decltype(whole)::value;
+    auto stage = [&](Pieces& f, int s, auto way) __attribute__((always_inline)) {
+        constexpr int WAY = decltype(way)::value;
         char* to = lds + (s & 1) * STAGE;
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             gs_u32x4_t hi, mid, lo;
-            if (WHOLE && p * ROWS >= BM) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t x0 = __float_as_uint(f.v[p][e >> 1][(e & 1) * 2]), x1 = __float_as_uint(f.v[p][e >> 1][(e & 1) * 2 + 1]);
-                    hi[e] = __builtin_amdgcn_perm(x1, x0, 0x07060302);
-                    rest |= x0 | x1;
-                }
-                *reinterpret_cast<gs_u32x4_t*>(to + dst[p]) = hi;
-                continue;
-            }
+            const bool cut = WAY != FULL && p * ROWS >= BM;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
+                float x0 = f.v[p][e >> 1][(e & 1) * 2], x1 = f.v[p][e >> 1][(e & 1) * 2 + 1];
                 uint32_t a, b, c;
-                gs_split(f.v[p][e >> 1][(e & 1) * 2], f.v[p][e >> 1][(e & 1) * 2 + 1], a, b, c, lost[p]);
-                hi[e] = a; mid[e] = b; lo[e] = c;
+                if (cut) {
+                    const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
+                    a = __builtin_amdgcn_perm(u1, u0, 0x07060302);
+                    rest |= u0 | u1;
+                    if (WAY == REST) gs_split_rest(x0 - __uint_as_float(u0 & 0xffff0000u), x1 - __uint_as_float(u1 & 0xffff0000u), b, c, lost[p]);
+                } else {
+                    gs_split(x0, x1, a, b, c, lost[p]);
+                }
+                hi[e] = a;
+                if (!cut || WAY == REST) { mid[e] = b; lo[e] = c; }
             }
             *reinterpret_cast<gs_u32x4_t*>(to + dst[p]) = hi;
-            *reinterpret_cast<gs_u32x4_t*>(to + dst[p] + PLANE) = mid;
-            *reinterpret_cast<gs_u32x4_t*>(to + dst[p] + 2 * PLANE) = lo;
+            if (!cut || WAY == REST) {
+                *reinterpret_cast<gs_u32x4_t*>(to + dst[p] + PLANE) = mid;
+                *reinterpret_cast<gs_u32x4_t*>(to + dst[p] + 2 * PLANE) = lo;
+            }
         }
     };
     constexpr bool FOLD = NT * MT == 1;
     gs_f32x16_t big[NT][MT], small[NT][MT], sum;
-    auto products = [&](int s, auto whole) {
-        constexpr bool WHOLE = decltype(whole)::value;
+    auto products = [&](int s, auto way) __attribute__((always_inline)) {
+        constexpr int WAY = decltype(way)::value;
         const char* from = lds + (s & 1) * STAGE + h * GS_PIECE + i * 16;
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
@@ -133,85 +146,120 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
 #pragma unroll
                 for (int m = 0; m < MT; ++m) a[m][q] = *reinterpret_cast<const gs_bf16x8_t*>(from + (wm * MT + m) * GS_GROUP + ks * 2 * GS_PIECE + q * PLANE);
 #pragma unroll
-                for (int n = 0; n < NT && (q == 0 || !WHOLE); ++n) w[n][q] = *reinterpret_cast<const gs_bf16x8_t*>(from + (BM / 32 + wn * NT + n) * GS_GROUP + ks * 2 * GS_PIECE + q * PLANE);
+                for (int n = 0; n < NT && (q == 0 ? WAY != REST : WAY != WHOLE); ++n) w[n][q] = *reinterpret_cast<const gs_bf16x8_t*>(from + (BM / 32 + wn * NT + n) * GS_GROUP + ks * 2 * GS_PIECE + q * PLANE);
             }
 #define GS_MFMA(SUM, WQ, AQ)                                                                                                     \
     _Pragma("unroll") for (int n = 0; n < NT; ++n) _Pragma("unroll") for (int m = 0; m < MT; ++m)                                \
         SUM[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[n][WQ], a[m][AQ], SUM[n][m], 0, 0, 0);
-            GS_MFMA(big, 0, 0)
-            GS_MFMA(small, 0, 1)
-            if constexpr (!WHOLE) {
+            if constexpr (WAY != REST) {
+                GS_MFMA(big, 0, 0)
+                GS_MFMA(small, 0, 1)
+            }
+            if constexpr (WAY != WHOLE) {
                 GS_MFMA(small, 1, 0)
                 GS_MFMA(small, 1, 1)
             }
-            GS_MFMA(small, 0, 2)
-            if constexpr (!WHOLE) {
+            if constexpr (WAY != REST) {
+                GS_MFMA(small, 0, 2)
+            } else {
+                GS_MFMA(small, 1, 2)
+            }
+            if constexpr (WAY != WHOLE) {
                 GS_MFMA(small, 2, 0)
             }
         }
     };
-    // The tile's sums; false: `rest` says that W's values are no bfloat16 numbers, and the sums are of no use.  Step s runs from LDS stage s & 1;
-    // behind it the pieces of step s + 1 are split into the other one.
-    auto run = [&](auto whole) {
-        constexpr bool WHOLE = decltype(whole)::value;
-        // (block-wide, behind two barriers: the stages are free for the other way then)
-        auto others = [&]() { return WHOLE && __syncthreads_or((rest & 0xffffu) != 0); };
-#pragma unroll
-        for (int e = 0; e < 16; ++e) sum[e] = 0.f;
-#pragma unroll
-        for (int n = 0; n < NT; ++n)
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) big[n][m][e] = small[n][m][e] = 0.f;
-        Pieces f0, f1, f2, f3;
-        fetch(f0, 0);
-        fetch(f1, 1);
-        fetch(f2, 2);
-        fetch(f3, 3);
-        stage(f0, 0, whole);
-        if (others()) return false;
+    // The sums of steps 0 .. steps - 1 from step0 on, the first four of which are in f0 .. f3.  Step s runs from LDS stage s & 1; behind it the pieces
+    // of step s + 1 are split into the other one.  Returns the steps done: WHOLE looks at `rest` behind its first stage, behind every eighth
+    // and behind its last, and ends where any of it is set.  (no_bf16 is set by the barrier that it is read behind, and is never taken back.)
+    Pieces f0, f1, f2, f3;
+    int done = 0;
+    auto note = [&]() __attribute__((always_inline)) { if (__any((rest & 0xffffu) != 0)) no_bf16 = 1; };
+    auto noted = [&]() { return __builtin_amdgcn_readfirstlane(no_bf16) != 0; };
+    auto run = [&](auto way) __attribute__((always_inline)) {
+        constexpr bool LOOK = decltype(way)::value == WHOLE;
+        stage(f0, 0, way);
+        if (LOOK) note();
         __syncthreads();
+        if (LOOK && noted()) return 0;
         int s = 0;
-#define GS_STEP(FREE, NEXT, S)        \
-    fetch(FREE, (S) + 4);             \
-    products(S, whole);               \
-    stage(NEXT, (S) + 1, whole);      \
-    __builtin_amdgcn_sched_barrier(0);\
+#define GS_STEP(FREE, NEXT, S, LOOKS)     \
+    fetch(FREE, (S) + 4);                 \
+    products(S, way);                     \
+    stage(NEXT, (S) + 1, way);            \
+    __builtin_amdgcn_sched_barrier(0);    \
+    if (LOOKS) note();                    \
     __syncthreads();
         for (; s + 4 < steps; s += 4) {
-            GS_STEP(f0, f1, s)
-            GS_STEP(f1, f2, s + 1)
-            GS_STEP(f2, f3, s + 2)
-            GS_STEP(f3, f0, s + 3)
-            if (FOLD && (s & 28) == 28) {
+            const bool looks = LOOK && (s & 4);
+            GS_STEP(f0, f1, s, false)
+            GS_STEP(f1, f2, s + 1, false)
+            GS_STEP(f2, f3, s + 2, false)
+            GS_STEP(f3, f0, s + 3, looks)
+            if (FOLD && ((s + done) & 28) == 28) {                 // (`done` is a multiple of eight)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     sum[e] += big[0][0][e];
                     big[0][0][e] = 0.f;
                 }
             }
+            if (looks && noted()) return s + 4;
         }
 #undef GS_STEP
-        products(s, whole);
-        if (s + 1 < steps) {
-            stage(f1, s + 1, whole);
+        products(s, way);
+#define GS_LAST(NEXT, S)        \
+    if ((S) < steps) {          \
+        stage(NEXT, S, way);    \
+        __syncthreads();        \
+        products(S, way);       \
+    }
+        GS_LAST(f1, s + 1)
+        GS_LAST(f2, s + 2)
+        GS_LAST(f3, s + 3)
+#undef GS_LAST
+        if (LOOK) {
+            note();
             __syncthreads();
-            products(s + 1, whole);
         }
-        if (s + 2 < steps) {
-            stage(f2, s + 2, whole);
-            __syncthreads();
-            products(s + 2, whole);
-        }
-        if (s + 3 < steps) {
-            stage(f3, s + 3, whole);
-            __syncthreads();
-            products(s + 3, whole);
-        }
-        return !others();
+        return steps;
     };
-    if (!run(std::true_type{})) run(std::false_type{});
+    auto fetch_first = [&]() __attribute__((always_inline)) {
+        fetch(f0, 0);
+        fetch(f1, 1);
+        fetch(f2, 2);
+        fetch(f3, 3);
+    };
+    fetch_first();
+    if (tid == 0) no_bf16 = 0;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sum[e] = 0.f;
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) big[n][m][e] = small[n][m][e] = 0.f;
+    __syncthreads();
+    const int whole_steps = run(std::integral_constant<int, WHOLE>{});
+    if (noted()) {
+        // what the steps since the last look left out, and the others in full
+        const int all = steps;
+        if (whole_steps > 0) {
+            done = max(0, (whole_steps - 1) & ~7);
+            step0 = part0 + done;
+            steps = whole_steps - done;
+            fetch_first();
+            run(std::integral_constant<int, REST>{});
+            __syncthreads();
+        }
+        done = whole_steps;
+        step0 = part0 + done;
+        steps = all - done;
+        if (steps > 0) {
+            if (done > 0) fetch_first();
+            run(std::integral_constant<int, FULL>{});
+        }
+    }
     // Two kinds of values do not split, and the sums that they are in are formed once more by float32 instructions, the wave's other values
     // stay: those beyond bfloat16's range, infinities and NaN, whose rest is a NaN as every sum with it then, and those below 2^-110 or so, of
     // which bits are lost: their rows of A and W
@@ -255,8 +303,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
                 gs_f32x16_t total, acc;
 #pragma unroll
                 for (int e = 0; e < 16; ++e) total[e] = acc[e] = 0.f;
-                const int end = (step0 + steps) * GS_BK;
-                for (int k0 = step0 * GS_BK; k0 < end; k0 += 256) {                // a chain ends every 256 of K, as in gemm_f32.hip
+                const int end = part1 * GS_BK;
+                for (int k0 = part0 * GS_BK; k0 < end; k0 += 256) {                // a chain ends every 256 of K, as in gemm_f32.hip
 #pragma unroll 4
                     for (int k = k0; k < min(k0 + 256, end); k += 8) {
                         const gs_f32x4_t va = *reinterpret_cast<const gs_f32x4_t*>(a_at + k), vw = *reinterpret_cast<const gs_f32x4_t*>(w_at + k);
@@ -311,7 +359,8 @@ static bool gs_large_tile(int M, int N, int K, int parts) {
 }
 
 // More than 32 rows (below, the products are bound by W's way from memory: 24 rows, 4096 x 1024 8.7 us / 18.7), and without parts tiles
-// for half of the compute units (2048 x 2048, 90 rows: 64 tiles 22 / 33; 4096 x 2048: 128 tiles 40 / 35).
+// for half of the compute units (2048 x 2048, 90 rows: 64 tiles 22 / 33; 4096 x 2048: 128 tiles 38.5 / 30.5 with a widened matrix, 38.3 with one of
+// float32 values; the smallest of that many, 4096 x 1024, 22.8 / 18.0 and 22.5).
 bool gemm_f32_split_takes(int M, int N, int K, int parts) {
     return M > 32 && K % GS_BK == 0 && (int64_t)M * K < (1 << 29) && (int64_t)N * K < (1 << 29)
         && (parts > 1 || (int64_t)((M + 63) / 64) * ((N + 63) / 64) >= 128);

@@ -182,6 +182,27 @@ def test_matrices_of_bfloat16_values(M, N, K, where):
     assert float((parts.double() - a * up).norm() / (a * up).norm()) < 1e-5
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 4100, 1184), (611, 4096, 1120)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_the_step_of_the_first_value_that_is_no_bfloat16_number(M, N, K, gated):
+    """A block goes on from the step in which it meets such a value: the other rows of the matrix have the bits that they have without it,
+    whichever of the steps it is, and its own row has the product in full."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    x, w = operands(M, N, K, dev)
+    w = w.bfloat16().float()
+    product = ops.linear_swiglu if gated else ops.linear
+    whole, row = product(x, w), N // 2 - 3
+    others = torch.arange(N // 2 if gated else N, device=dev) != row
+    for k in range(31, K, 32):
+        kept, w[row, k] = float(w[row, k]), 0.7 + 2.0 ** -20
+        out = product(x, w)
+        assert torch.equal(out[:, others], whole[:, others]), k
+        if not gated:
+            assert bool(((out[:, row].double() - x.double() @ w[row].double()).abs() <= bound(x, w[row:row + 1])[:, 0]).all()), k
+        w[row, k] = kept
+
+
 @pytest.mark.parametrize("M,N", [(65, 5000), (611, 5000)])
 @pytest.mark.parametrize("gated", [False, True])
 def test_neighbours_of_values_that_cannot_be_cut(M, N, gated):
