@@ -37,10 +37,9 @@ constexpr int GD_WAVES_GATED = 4;     // waves of a block of the gated product w
 // The stored product only.
 // HT: 0, or the number of half tiles of a block, 3 or 5 (two and a half tiles per unit: qkv of 10240 columns), or one: a matrix with column
 // tiles for at most half of the compute units (o, down of a narrow model) then has blocks for twice as many, each with half of the
-// bytes to pull (the residual product too, whose parts of sum(h^2) are N / 8).  Measured, us, whole tiles / halves: residual product of
-// 2048 x 6144, 4 rows 8.8 / 8.1, 16 rows 10.1 / 9.3; 1024 x 3072 5.4 / 4.95, 6.2 / 5.4; 1024 x 2048, 16 rows 4.7 / 4.45 (1 row 4.0 / 4.1).
+// bytes to pull (the residual product too, whose parts of sum(h^2) are N / 8), where gd_half_tiles says so.
 // RC: a wave's chunks of K per round of loads, where they make one round (K = 3072 three, the third costs a round trip of its own otherwise:
-// 5.4 / 4.9 us of these); more than four gain nothing (2048 x 6144 in one round of six 8.4, in three of two 8.1).
+// 1024 x 3072 5.4 / 4.9 us); more than four gain nothing (2048 x 6144 in one round of six 8.4, in three of two 8.1).
 template <int EPI, bool SCALED, typename TC, int GD_WAVES, bool XT, bool OT, int HT = 0, int RC = 2>
 __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_kernel(
     const bf16_t* __restrict__ X, const bf16_t* __restrict__ Wt, TC* __restrict__ C, float* __restrict__ resid_out,
@@ -419,6 +418,18 @@ int gd_compute_units() {
 }
 
 // false: this combination is not built for the call's number of rows (beyond 64 rows only what a decode step has is built)
+// Whether blocks of half a column tile pay for up to 16 rows of x in operand order (the residual product too, ops.residual_parts) or of
+// ordinary rows.  Measured with 256 to 2048 columns, us, whole / half, at 2048 columns.  Operand order, residual, 8 and 16 rows: K = 1024 3.5 /
+// 3.8 and 3.7 / 3.9, 1536 4.15 / 3.92 and 4.43 / 4.07, 2048, where every wave has one full round of two chunks, 4.25 / 4.33 and 4.8 / 4.6 (1024 columns 4.0
+// / 4.05 and 4.6 / 4.3), 3072 5.6 / 5.2 and 6.4 / 5.6, 4096 6.1 / 6.0 and 7.3 / 6.5, 6144 8.1 / 7.6 and 9.9 / 8.5; fewer rows as 8.  Ordinary rows, whose loads
+// grow with them, 1, 4 and 16: K = 1024 3.3 / 3.55, 3.4 / 3.75 and 3.75 / 4.07, 2048 3.9 / 4.15, 4.1 / 4.3 and 5.2 / 5.2, 2560 4.65 / 4.5, 4.9 / 4.6 and 6.2 /
+// 5.9, 3072 5.2 / 5.0, 5.5 / 5.1 and 7.0 / 6.5, 4096 5.45 / 5.75, 6.0 / 6.05 and 8.4 / 8.1 (512 columns 4.85 / 4.95, 5.5 / 5.25, 7.75 / 7.5), 6144 7.2 / 7.45, 8.2 / 7.7
+// and 11.2 / 10.6.
+static bool gd_half_tiles(int M, int N, int K, bool operand_order) {
+    if (N > 2048) return false;
+    return operand_order ? K > 1024 && (K != 2048 || M > 8) : K > 2048 && (K <= 3072 || M >= 4);
+}
+
 template <int EPI, bool SCALED, typename TC, bool XT, bool OT>
 static bool gd_launch2(const GdArgs& a) {
     constexpr int W = EPI == EPI_GATED ? GD_WAVES_GATED : 8;
@@ -448,7 +459,7 @@ static bool gd_launch2(const GdArgs& a) {
 #define GD_HALF_N(RC) gemm_decode_kernel<EPI, SCALED, TC, W, XT, OT, 1, RC><<<a.N / 8, W * 64, 0, a.st>>>(GD_ARGS)
 #define GD_HALF if (each == 3) GD_HALF_N(3); else GD_HALF_N(2);
         if constexpr (EPI == EPI_STORE && sizeof(TC) == 2) {
-            if (a.N / 8 <= gd_compute_units()) {
+            if (gd_half_tiles(a.M, a.N, a.K, XT)) {
                 GD_HALF
                 halves = true;
             }

@@ -972,10 +972,13 @@ def decode_linear_swiglu(x, tiled_gate_up: torch.Tensor, for_product: bool = Fal
     return out
 
 
-def residual_parts(rows: int, columns: int) -> int:
+def residual_parts(rows: int, columns: int, inner: Optional[int] = None) -> int:
     """Parts of the rows' sums of squares that the residual product writes, one a block: for up to 16 rows of at most 2048 columns, whose
-    tiles of 16 are blocks for half of the compute units at most, a block has half a tile (csrc/gemm_decode.hip)."""
-    return columns // 8 if rows <= 16 and columns <= 2048 else columns // 16
+    tiles of 16 are blocks for half of the compute units at most, a block has half a tile, unless ``inner`` (K; None: a long one) makes
+    no more than one full round of loads (csrc/gemm_decode.hip, gd_half_tiles, with what was measured)."""
+    if rows > 16 or columns > 2048 or (inner is not None and (inner <= 1024 or (inner == 2048 and rows <= 8))):
+        return columns // 16
+    return columns // 8
 
 
 def decode_linear_residual(x, tiled: torch.Tensor, resid: torch.Tensor, next_norm_weight: torch.Tensor,
@@ -988,7 +991,7 @@ def decode_linear_residual(x, tiled: torch.Tensor, resid: torch.Tensor, next_nor
            "decode_linear_residual: the stream must be float32 [M, %d]", N)
     _check(next_norm_weight.dtype == torch.bfloat16 and next_norm_weight.shape == (N,),
            "decode_linear_residual: the next norm's weight must be bfloat16 [%d]", N)
-    ss = torch.empty((residual_parts(M, N), 16 * row_tiles(M)), dtype=torch.float32, device=resid.device)
+    ss = torch.empty((residual_parts(M, N, tiled.shape[1]), 16 * row_tiles(M)), dtype=torch.float32, device=resid.device)
     if _operand_order_ok(N):
         xw = OperandRows.empty(M, N, resid.device)
     else:
