@@ -59,7 +59,7 @@ __device__ __forceinline__ void gf_row_sums(float (&v)[V], int lane) {
 // GATED: W = [gate rows | up rows] of N columns each; a block owns NR / 2 columns, their gate rows and their up rows, and stores act(gate)
 // * up.  Measured, us, with one to four rows of W a wave and its own K / this, 4 rows of A: 2048 x 2048 6.9 / 5.6, 2048 x 6144 15.6 / 10.6 (4.7
 // TB/s), 4096 x 2048 9.7 / 8.2, 12288 x 2048 gated 22.3 / 18.3 (5.5 TB/s), 151936 x 2048 192 / 186; 1 row: 2048 x 6144 10.3 / 9.9, 1024 x 3072
-// 4.3 / 4.5; 8 rows, the narrow kernel / this: 2048 x 6144 23.4 / 13.8, 12288 x 2048 with its activation 45 / 22, 151936 x 2048 356 / 225.
+// 4.1 / 3.95; 8 rows, the narrow kernel / this: 2048 x 6144 23.4 / 13.8, 12288 x 2048 with its activation 45 / 22, 151936 x 2048 356 / 225.
 template <int MR, int NR, int U, int WV, bool GATED>
 __global__ __launch_bounds__(WV * 64) void gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
                                                               int M, int N, int K, GateAct act) {
@@ -474,10 +474,20 @@ static bool gf_few_takes(int M, int N, int K) { return M <= 4 || (M <= 8 && (N <
 
 // Rows of W a block, and waves: eight rows where there are plenty (4 rows of A: 12288 x 2048 gated 18.3 us, with four 19.5; 2048 x 6144 11.5 / 10.6;
 // 8 rows of A: 4096 x 2048 10.1 / 10.9), and up to 1024 rows of W eight waves a block to have enough of them (4 rows of A, 1024 x 3072 5.0
-// us, four waves 5.7) or, for one or two rows of A, two rows of W (1024 x 2048 3.7 / 3.8, 1024 x 3072 4.5 / 4.4).
+// us, four waves 5.7) or, for two rows of A, two rows of W (1024 x 2048 3.7 / 3.6, 1024 x 3072 4.6 / 4.4).  One row of A costs little to bring
+// again, and up to 4 million numbers of W blocks of one row are the fastest, a chunk a wave and round (what stood before / two rows, or four beyond
+// 1024 of W / one): 1024 x 1024 2.76 / 2.79 / 2.74, 1024 x 2048 3.50 / 3.44 / 3.38, 1024 x 3072 4.05 / 4.23 / 3.94, 1024 x 4096 5.15 / 4.81 / 4.64, 2048 x 2048
+// 4.65 / 4.72 / 4.57, 4096 x 1024 4.93 / 4.75 / 4.70; beyond, 2048 x 3072 four 5.78, one 6.16, 4096 x 2048 7.35 / 7.12 / 7.40.  Below 1024 rows of W two
+// chunks a round, where that leaves no rest: 512 x 2048 2.68, one 2.96 (two rows of W 2.78); 256 x 2048 2.34, 2.69 (2.50); 512 x 3072 3.26, 3.14 (3.40).
 template <bool GATED>
 static void gf_few(const float* A, const float* W, float* C, int M, int N, int w_rows, int K, GateAct act, hipStream_t st) {
 #define GF_FEW(MR, NR, U, WV) gemm_f32_few_kernel<MR, NR, U, WV, GATED><<<(N + NR / (GATED ? 2 : 1) - 1) / (NR / (GATED ? 2 : 1)), WV * 64, 0, st>>>(A, W, C, M, N, K, act)
+    if constexpr (!GATED) {
+        if (M == 1 && (int64_t)w_rows * K <= (4 << 20)) {
+            if (w_rows < 1024 && K % 2048 == 0) GF_FEW(1, 1, 2, 4); else GF_FEW(1, 1, 1, 4);
+            return;
+        }
+    }
     if (M == 1) { if (w_rows <= 1024) GF_FEW(1, 2, 2, 4); else GF_FEW(1, 4, 2, 4); }
     else if (M == 2) { if (w_rows <= 1024) GF_FEW(2, 2, 2, 4); else GF_FEW(2, 4, 2, 4); }
     else if (M <= 4) { if (w_rows <= 1024) GF_FEW(4, 4, 1, 8); else if (w_rows < 8192) GF_FEW(4, 4, 1, 4); else GF_FEW(4, 8, 1, 4); }

@@ -30,6 +30,18 @@ def test_product(M, N, K):
     assert bool(((out.double() - x.double() @ w.double().t()).abs() <= limit).all()) and bool(held[M * N:].isnan().all())
 
 
+@pytest.mark.parametrize("N,K", [(1023, 2048), (1023, 4096), (1024, 4096), (1025, 4096), (300, 6144), (2048, 2052)])
+def test_one_row(N, K):
+    """Blocks of one row of W, one and two chunks a round, up to 4 million numbers of W, and one size beyond."""
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    g = torch.Generator().manual_seed(N + K)
+    x, w = torch.randn((1, K), generator=g).to(dev), torch.randn((N, K), generator=g).to(dev)
+    held = torch.full((N + 64,), float("nan"), device=dev)
+    out = ops.linear(x, w, out=held[:N].view(1, N))
+    assert bool(((out.double() - x.double() @ w.double().t()).abs() <= bound(x, w)).all()) and bool(held[N:].isnan().all())
+
+
 @pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
 @pytest.mark.parametrize("M", [1, 2, 4, 5, 7, 8])
 @pytest.mark.parametrize("I,K", [(1, 4), (511, 1028), (2045, 512), (3072, 1024), (4101, 2048)])
