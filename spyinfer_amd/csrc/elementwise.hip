@@ -690,10 +690,33 @@ template <> struct Eight<bf16_t> {
     static __device__ __forceinline__ void store(bf16_t* p, const float (&v)[8]) {
         *reinterpret_cast<uint4*>(p) = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
     }
+    // values that are only moved keep their bits (a conversion would change those of a NaN): from one place, or every `step`
+    static __device__ __forceinline__ void move(bf16_t* to, const bf16_t* from, bool there) {
+        uint4 r = {0u, 0u, 0u, 0u};
+        if (there) r = *reinterpret_cast<const uint4*>(from);
+        *reinterpret_cast<uint4*>(to) = r;
+    }
+    static __device__ __forceinline__ void gather(bf16_t* to, const bf16_t* from, int step) {
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = (uint32_t)from[2 * i * step] | ((uint32_t)from[(2 * i + 1) * step] << 16);
+        *reinterpret_cast<uint4*>(to) = make_uint4(w[0], w[1], w[2], w[3]);
+    }
 };
 template <> struct Eight<float> {
     static __device__ __forceinline__ void load(const float* p, float (&v)[8]) { Vec4<float>::load(p, v); Vec4<float>::load(p + 4, v + 4); }
     static __device__ __forceinline__ void store(float* p, const float (&v)[8]) { Vec4<float>::store(p, v); Vec4<float>::store(p + 4, v + 4); }
+    static __device__ __forceinline__ void move(float* to, const float* from, bool there) {
+        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (there) load(from, v);
+        store(to, v);
+    }
+    static __device__ __forceinline__ void gather(float* to, const float* from, int step) {
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = from[e * step];
+        store(to, v);
+    }
 };
 
 template <typename TA, typename TW, int LPH>
@@ -756,9 +779,7 @@ __global__ __launch_bounds__(256) void qknorm_rope_store_vec_kernel(
     const int t0 = (int)(vb / (unsigned)n_kv) * 16, hv = (int)(vb % (unsigned)n_kv);
     for (int i = threadIdx.x; i < 16 * (d / 8); i += 256) {
         const int tt = i / (d / 8), c8 = i % (d / 8);
-        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (t0 + tt < T) Eight<TA>::load(qkv + (size_t)(t0 + tt) * heads * d + (size_t)(qk_heads + hv) * d + 8 * c8, v);
-        Eight<TA>::store(tile + tt * LD + 8 * c8, v);
+        Eight<TA>::move(tile + tt * LD + 8 * c8, qkv + (size_t)(t0 + tt) * heads * d + (size_t)(qk_heads + hv) * d + 8 * c8, t0 + tt < T);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 2 * d; i += 256) {
@@ -772,11 +793,8 @@ __global__ __launch_bounds__(256) void qknorm_rope_store_vec_kernel(
             for (int e = 1; e < 8; ++e) run = run && slots[tb + e] == s0 + e;
         }
         if (run) {                                            // P is a multiple of 8: the 8 slots lie in one page
-            float v[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = to_f32<TA>(tile[(8 * tg + e) * LD + j]);
             const int page = (int)((unsigned)s0 / (unsigned)P), off = s0 - page * P;
-            Eight<TA>::store(vc + (((size_t)page * n_kv + hv) * d + j) * P + off, v);
+            Eight<TA>::gather(vc + (((size_t)page * n_kv + hv) * d + j) * P + off, tile + 8 * tg * LD + j, LD);
         } else {
             for (int e = 0; e < 8 && tb + e < T; ++e) {
                 const int slot = slots[tb + e];

@@ -38,3 +38,22 @@ def test_many_tokens(d, n_q, n_kv, T, normed, order, dtype):
         tol = 2.0 ** -18 if dtype == torch.float32 else 2.0 ** -7
         assert bool(((a.float() - b.float()).abs() <= tol * (b.float().abs() + float(b.float().pow(2).mean().sqrt()))).all())
     assert torch.equal(many[2], few[2])                                            # values are only moved
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("order", ["straight", "mixed"])
+def test_values_keep_their_bits(dtype, order):
+    """Every number of bfloat16, NaN with all their bits among them, and as many of float32."""
+    from spyinfer_amd.kernels import ops
+    dev, T, d, P = require_gpu(), 512, 128, 16
+    bits = torch.arange(65536, dtype=torch.int32)
+    values = (bits << 16 | bits).view(torch.float32) if dtype == torch.float32 else bits.to(torch.int16).view(torch.bfloat16)
+    x = torch.zeros((T, 3 * d), dtype=dtype)
+    raw = torch.int32 if dtype == torch.float32 else torch.int16
+    x.view(raw)[:, 2 * d:] = values.view(raw).view(T, d)
+    slots = (torch.arange(T) if order == "straight" else torch.randperm(T, generator=torch.Generator().manual_seed(1))).int()
+    k, v = torch.zeros((T // P, 1, P, d), device=dev, dtype=dtype), torch.zeros((T // P, 1, d, P), device=dev, dtype=dtype)
+    table = torch.ones((T, d // 2), device=dev)
+    ops.qk_norm_rope_store(x.to(dev), 1, 1, d, None, None, 1e-6, table, table, d, torch.arange(T, device=dev).int(), k, v, P, slots.to(dev))
+    kept = v.view(raw).cpu().permute(0, 3, 1, 2).reshape(T, d)[slots.long()]
+    assert torch.equal(kept, x.view(raw)[:, 2 * d:])
