@@ -170,11 +170,15 @@ extern "C" int spy_embedding_sumsq(float* out, void* xw, float* ss, const void* 
 // read again for the second pass.  Few rows: as many threads as make one pass where they can, whose loads go
 // out together (a thread with several passes has one's under way at a time); rows that fill the chip by themselves do better in blocks
 // of 256.  Measured, us, several passes / one: 1 row of 1024 3.4 / 2.7, 4 of 2048 in float32 3.6 / 2.8, 409 of 2560 5.7 / 4.7, 611 of 1024 in float32
-// 4.3 / 3.8; 1356 of 2048 8.6 / 9.0, 2048 of 4096 17.0 / 19.5 (5.9 / 5.2 TB/s).  The line is two million values.
+// 4.3 / 3.8; 1356 of 2048 8.6 / 9.0, 2048 of 4096 17.0 / 19.5 (5.9 / 5.2 TB/s).  The line is two million values (beyond 4096 of a row blocks of
+// 512: 300 of 8192 11.2 / 8.9).
+// A row's sum of squares is added in one order on both sides of it, so that a row is normed to the same bits in steps of every size: each
+// 256 values by a wave, these in order.  A wave sums its passes together, half of a lane's handed over at each step (seven exchanges for four
+// passes; one pass after the other cost 0.3 us of 1000 rows of 2560); as many passes' registers as the row needs, so that eight waves a SIMD fit.
 #define NORM_PASSES 8
 inline int norm_threads(int H) { return min(1024, (H / 4 + 63) / 64 * 64); }       // (rows in pieces of four values)
 template <typename TA, typename TW, int NP>
-__global__ __launch_bounds__(1024) void add_rmsnorm_kernel(float* __restrict__ resid, const TA* __restrict__ delta, const TA* __restrict__ delta2,
+__global__ __launch_bounds__(1024, NP > 4 ? 4 : 8) void add_rmsnorm_kernel(float* __restrict__ resid, const TA* __restrict__ delta, const TA* __restrict__ delta2,
                                    const TW* __restrict__ w, float eps, TA* __restrict__ out, const int* __restrict__ rows, int T,
                                    int H, int ld, const TA* __restrict__ gate, const TW* __restrict__ gbias, float mult,
                                    const float* __restrict__ base, const float* __restrict__ vec, const TW* __restrict__ w2,
@@ -186,7 +190,7 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_kernel(float* __restrict__ r
     // gate), formed here in float32 from the sublayer's result and the gate's product.
     // H: values that are normed together: the whole row (ld == H), or one of the row's ld / H consecutive groups, which
     // blockIdx.y counts
-    __shared__ float red[16];
+    __shared__ __align__(16) float red[NP > 0 ? 16 * NP : 16];
     const int r = blockIdx.x;
     const size_t g0 = (size_t)blockIdx.y * H;
     int t = r;
@@ -211,11 +215,11 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_kernel(float* __restrict__ r
     const bool write_back = (dl || bs || vc) && !rows;
     if constexpr (NP > 0) {
         // H % 4 == 0 and 16-byte aligned rows (checked by the launcher); the row fits the register passes
-        float v[NP][4];
-        float ss = 0.f;
+        float v[NP][4], squares[NP];
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
             const int i = (p * blockDim.x + threadIdx.x) * 4;
+            squares[p] = 0.f;
             if (i < H) {
                 Vec4<float>::load(x + i, v[p]);
                 if (dl) {
@@ -251,10 +255,29 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_kernel(float* __restrict__ r
                 }
                 if (write_back) Vec4<float>::store(x + i, v[p]);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) ss += v[p][e] * v[p][e];
+                for (int e = 0; e < 4; ++e) squares[p] += v[p][e] * v[p][e];
             }
         }
-        ss = block_sum(ss, red);
+        // a lane's sums meet those of the other lanes, half of them handed over at each step while there are several: lane l ends with pass l NP / 64's
+        const int lane = threadIdx.x & 63, pieces = blockDim.x >> 6, all = (H + 255) / 256;
+        int mask = 32;
+#pragma unroll
+        for (int n = NP / 2; n >= 1; n /= 2, mask /= 2) {
+            const bool upper = (lane & mask) != 0;
+#pragma unroll
+            for (int p = 0; p < n; ++p) squares[p] = (upper ? squares[p + n] : squares[p]) + __shfl_xor(upper ? squares[p] : squares[p + n], mask, 64);
+        }
+#pragma unroll
+        for (; mask >= 1; mask /= 2) squares[0] += __shfl_xor(squares[0], mask, 64);
+        if (lane % (64 / NP) == 0) red[lane * NP / 64 * pieces + (threadIdx.x >> 6)] = squares[0];
+        __syncthreads();
+        float ss = 0.f;
+        int i = 0;
+        for (; i + 4 <= all; i += 4) {
+            const float4 q = *reinterpret_cast<const float4*>(red + i);
+            ss = ((ss + q.x) + q.y) + q.z + q.w;
+        }
+        for (; i < all; ++i) ss += red[i];
         const float scale = 1.0f / sqrtf(ss / (float)H + eps);
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
@@ -316,7 +339,7 @@ extern "C" int spy_add_rmsnorm(float* resid, const void* delta, const void* delt
     SPY_REQUIRE(delta || !delta2, "spy_add_rmsnorm: a second addend without a first");
     const int H = ld / groups;
     const dim3 grid(n_out, groups);
-    const int threads = (int64_t)n_out * ld > (2 << 20) ? (H >= 2048 ? 256 : (H >= 512 ? 128 : 64)) : norm_threads(H);
+    const int threads = (int64_t)n_out * ld > (2 << 20) && H <= 8192 ? (H > 4096 ? 512 : H >= 2048 ? 256 : (H >= 512 ? 128 : 64)) : norm_threads(H);
     const bool aligned = H % 4 == 0 && ((uintptr_t)resid % 16) == 0 && ((uintptr_t)delta % 16) == 0 && ((uintptr_t)delta2 % 16) == 0 && ((uintptr_t)w % 16) == 0 &&
                          ((uintptr_t)out % 16) == 0 && ((uintptr_t)gate % 16) == 0 && ((uintptr_t)gbias % 16) == 0 &&
                          ((uintptr_t)base % 16) == 0 && ((uintptr_t)vec % 16) == 0 && ((uintptr_t)w2 % 16) == 0 && ((uintptr_t)out2 % 16) == 0;
@@ -327,6 +350,8 @@ extern "C" int spy_add_rmsnorm(float* resid, const void* delta, const void* delt
         base, vec, (const TW*)w2, (TA*)out2))))
     if (!by_pieces) { NORM_LAUNCH(0, 512); }
     else if (H <= threads * 4) { NORM_LAUNCH(1, threads); }
+    else if (H <= threads * 8) { NORM_LAUNCH(2, threads); }
+    else if (H <= threads * 16) { NORM_LAUNCH(4, threads); }
     else { NORM_LAUNCH(NORM_PASSES, threads); }
 #undef NORM_LAUNCH
     SPY_CHECK_LAUNCH("spy_add_rmsnorm");

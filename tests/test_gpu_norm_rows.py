@@ -14,7 +14,7 @@ def limit(want, dtype, H):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("T,H", [(1, 4), (3, 252), (5, 1028), (2, 4096), (3, 4100), (2, 8192), (2, 8196), (600, 4096), (1030, 2048)])
+@pytest.mark.parametrize("T,H", [(1, 4), (3, 252), (5, 1028), (2, 4096), (3, 4100), (2, 8192), (2, 8196), (2, 16388), (600, 4096), (1030, 2048)])
 def test_add_rms_norm(T, H, dtype):
     from spyinfer_amd.kernels import ops
     dev = require_gpu()
@@ -44,3 +44,19 @@ def test_parts(T, H, parts):
     assert torch.equal(resid.cpu(), s)
     want = s.double() * torch.rsqrt(s.double().pow(2).mean(1, keepdim=True) + 1e-5) * w.double()
     assert bool(((out.cpu().double() - want).abs() <= limit(want, torch.float32, H)).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H", [252, 512, 700, 1028, 2048, 2560, 4096, 4100, 5120, 8192, 8196, 16388])
+def test_a_row_is_the_same_bits_in_steps_of_every_size(H, dtype):
+    from spyinfer_amd.kernels import ops
+    dev = require_gpu()
+    T, few = (2 << 20) // H + 1, 3
+    g = torch.Generator().manual_seed(H)
+    x, y, w = (torch.randn(s, generator=g) for s in ((T, H), (T, H), (H,)))
+    x, y, w = x.to(dev), y.to(dtype).to(dev), w.to(dtype).to(dev)
+    streams, outs = [], []
+    for t in (T, few):
+        streams.append(x[:t].clone())
+        outs.append(ops.add_rms_norm(streams[-1], y[:t].clone(), w, 1e-5, dtype))
+    assert torch.equal(streams[0][:few], streams[1]) and torch.equal(outs[0][:few], outs[1])
