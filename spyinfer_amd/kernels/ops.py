@@ -582,8 +582,10 @@ def f32_product_parts(M: int, N: int, K: int):
     """Parts of K for a float32 product whose result the next norm sums from them, or None where one pass is the better one.  A part of a
     tile is a block: of 64 x 64 by the float32 instructions, its numbers fitted to 380 launches of 17 to 2048 rows (the choice is 0.13 % behind
     the best on average, 6 % at most, the parts' sum counted; up to 32 rows ``f32_held_parts`` comes first); of 128 x 128 (to 2048 of K) or 64 x
-    64 by the kernel that splits values, with the estimate that it chooses its tile by.  Of its numbers of parts the smallest within 6 % of the
-    best, which the estimate does not tell apart (611 rows, 1024 x 2048, with the sum: three parts 25.7 us, six 25.0)."""
+    64 by the kernel that splits values, with the estimate that it chooses its tile by, as many as pay (802 rows, 2560 x 4096, with the sum and
+    norm: two parts 108 us, three 95; 1354 rows, 2048 x 6144: one 200, four 156).  Of its numbers of parts the smallest within 6 % of the best,
+    which the estimate does not tell apart (611 rows, 1024 x 2048, with the sum: three parts 25.7 us, six 25.0).  The estimate is of float32 values'
+    six products; widened bfloat16 matrices take two thirds of the time in the same order (47 sizes of 38 to 1354 rows: 2 % behind the best either way)."""
     if M <= 16 or K % 4 or -(-M // 64) * -(-N // 64) >= 1 << 20:
         return None
     tiles, large = -(-M // 64) * -(-N // 64), -(-M // 128) * -(-N // 128)
@@ -599,7 +601,8 @@ def f32_product_parts(M: int, N: int, K: int):
             time = -(-tiles * p // 256) * (K / p) * 0.0178 + (K / p) * 0.0066
         return time + total / 8e6 + (total / 4.5e6 + 0.3 if p > 1 else 0.0)
 
-    fits = [p for p in (1, 2, 3, 4, 5, 6, 8, 12) if p == 1 or (K // 32 // p >= 4 and tiles * p <= 1400 and p * M * N * 4 <= PARTS_MAX_BYTES)]
+    fits = [p for p in (1, 2, 3, 4, 5, 6, 8, 12)
+            if p == 1 or (K // 32 // p >= 4 and (tiles * p <= 1400 or f32_rows_split(M, N, K, p)) and p * M * N * 4 <= PARTS_MAX_BYTES)]
     best = min(fits, key=us)
     if f32_rows_split(M, N, K, 2):
         best = next(p for p in fits if us(p) <= 1.06 * us(best))

@@ -75,6 +75,8 @@ def test_float32_products_in_parts_that_split_values():
     assert ops.f32_rows_split(33, 8192, 1024) and not ops.f32_rows_split(32, 8192, 1024) and not ops.f32_rows_split(90, 4032, 1024)
     assert ops.f32_rows_split(90, 1024, 1024, 2) and not ops.f32_rows_split(600, 8192, 1000)
     assert ops.f32_product_parts(611, 1024, 3072) == 6 and ops.f32_product_parts(90, 2048, 2048) == 4
+    # (long prompts too: more parts than small tiles would need)
+    assert all(-(-M // 64) * (N // 64) * ops.f32_product_parts(M, N, K) > 1400 for M, N, K in ((1354, 2048, 6144), (802, 2560, 4096), (4096, 1024, 3072)))
 
 
 def test_float32_products_in_parts_of_rows_that_are_held():
