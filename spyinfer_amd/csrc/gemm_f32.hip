@@ -1,6 +1,6 @@
 // C[M, N] = A[M, K] . W[N, K]^T in float32: products and sums of 32-bit numbers, no reduced-precision mode (the matrix cores'
 // float32 instructions multiply and add as fmaf does; gemm_f32_split.hip, which has most products of more than 32 rows, cuts the
-// numbers without loss).  Four kernels by the number of rows:
+// numbers into parts that keep their 24 bits, and leaves those that cannot be cut so to float32 instructions).  Four kernels by the number of rows:
 //
 //   few    (up to 8 rows)   bound by streaming W from memory: a block's waves share K, 64 lanes side by side along it.
 //   narrow (tens of rows)   bound by W from memory as well, but A's rows would be read once per row of W by the kernel above.
@@ -495,6 +495,9 @@ static void gf_few(const float* A, const float* W, float* C, int M, int N, int w
 #undef GF_FEW
 }
 
+// K (or a part of it) ends at 2048 because a wave's registers do: a chunk of 64 takes 16 of them for W and 16 for each row tile, and with two row
+// tiles four chunks leave room in 256, five do not.  (One row tile would fit K = 3072; it is not built: in parts o and down of a wider model are
+// taken, its gate/up and head stay with the narrow kernel.)
 static bool gf_held_takes(int M, int N, int K, int parts) { return M <= 32 && N < (1 << 30) && K % (512 * parts) == 0 && K / parts <= 2048; }
 
 // a block for each compute unit: another one brings A's values again and takes no part of the memory's time (12288 x 2048, 16 rows 24.5 us, two

@@ -346,11 +346,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_f32_split_kernel(const floa
 }
 
 // ---- dispatch --------------------------------------------------------------------------------------------------------------
-// Estimated time of both tiles, fitted to 120 launches of 40 to 611 rows, K of 1024 to 6144 and 1 to 12 parts: a compute unit takes 0.9 us for a
-// step of a large block (1.03 with the chip full), 0.5 us for one small block, 0.83 for two, 1.0 with the chip full.  (611 rows: 4096 x
-// 1024, 160 large or 640 small blocks 44 / 49 us, 1024 x 2048, 40 or 160 blocks 68 / 36; 400 rows, 4096 x 2048, 128 or 448: 69 / 58.)  A chain of
-// products of the large tile is the part's whole K, which to 2048 rounds no more than the float32 instructions do; the small tile's
-// sums change every 1024.
+// Estimated time of both tiles for a matrix of float32 values, fitted to 120 launches of 40 to 611 rows, K of 1024 to 6144 and 1 to 12 parts:
+// a compute unit takes 0.9 us for a step of a large block (1.03 with the chip full), 0.5 us for one small block, 0.83 for two, 1.0 with the
+// chip full.  A widened matrix takes two thirds of it with either tile, so that the choice is the same: over 344 launches of 38 to 1435 rows it is 0.5 %
+// behind the better tile for float32 values, 0.4 % for widened ones (17 and 13 % at most, in 12 parts).  Large / small tile, us, float32 values and
+// widened: 611 rows, 4096 x 1024 (160 or 640 blocks) 40.5 / 49.1 and 29.8 / 35.9, 1024 x 2048 in three parts 28.7 / 25.5 and 21.7 / 18.2, 400
+// rows, 4096 x 2048 71.4 / 63.4 and 51.5 / 44.9, 12288 x 2048 160 / 178 and 110 / 122.  A chain of products of the large tile is the part's whole
+// K, which to 2048 rounds no more than the float32 instructions do; the small tile's sums change every 1024.
 static bool gs_large_tile(int M, int N, int K, int parts) {
     const int64_t large = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * parts, small = (int64_t)((M + 63) / 64) * ((N + 63) / 64) * parts;
     const double steps = (double)K / GS_BK / parts, rest = small % 512 == 0 ? 0.0 : (small % 512 <= 256 ? 0.5 : 0.83);
