@@ -10,7 +10,7 @@
 //   delta_chunk_prepare   a block per (chunk, head): A, B, M and from them MV = M V, MW = M W, Q_t = G_t q_t, K_s = G_15 / G_s k_s (stored
 //                         [channel][token]), G_15, into a workspace.  The quotients of decays are never formed as quotients, which
 //                         underflow: they are powers of two of differences of sums of logarithms, sums in 64 bits.
-//   delta_chunk_walk      a block per (entry, head, 16 value channels), a wave per 16 key channels, whose rows of S it has in
+//   delta_chunk_walk      a block per (entry, head, 16 value channels), a wave per 16 key channels (or 32), whose rows of S it has in
 //                         registers.  Per chunk, on v_mfma_f32_16x16x4_f32: its part of MW S0 and of Q S0, the parts of u met in
 //                         LDS, S = G_15 S + K^T u, and B u for the read-out, whose parts meet one chunk later.
 // The result's layout (lane (column r, g): rows 4 g + i) is the second operand's layout of the next product, so S and u go from product to
@@ -19,7 +19,10 @@
 // 1500 tokens, not its operands' way (95 us, 92 with every chunk's from one place); the preparation's 136 x d powers of two a chunk.  Chunks
 // of 16 because a chunk's tokens are then one matrix tile; the preparation grows with the square.
 // Measured: 1500 tokens, 16 heads of 128 x 128: 51 us of preparation and 95 us of walk a layer (104 by four waves with 32 key channels each)
-// against 1712 us token by token.
+// against 1712 us token by token.  Four waves with two tiles of channels each where the delta rule's blocks outnumber the compute units: every
+// wave reads all waves' parts of u out of LDS, four times as much by eight waves.  16 heads of 128 x 128, preparation and walk, four / eight: entries of 300,
+// 20 and 411 tokens (384 blocks) 98 / 109, eight of 64 72 / 76, two of 300 (256 blocks) 82 / 81.5; 4 heads of 128 x 256, 32 of 40 73 / 81.5.  (The
+// mLSTM, which has no such parts, is faster by eight at any number: 12 entries of 150, 8 heads of 128 x 256, 109 / 104.)
 // The mLSTM, S = a S + b k v^T with numbers a and b a token, is the same with nothing taken back: u = v, B_ts = b_s G_t / G_s (q_t . k_s), K_s =
 // b_s G_15 / G_s k_s, and its vector n = a n + b k goes along in the lanes' registers (a lane has the rows of n that it has of Q as an
 // operand, so n . q costs eight products a lane).  8 heads of 128 x 256, 1500 tokens: a walk
@@ -251,9 +254,9 @@ struct ChunkWalk {
     const float* ws;
 };
 
-template <int D, bool DELTA>
-__global__ __launch_bounds__(D * 4) void chunk_walk_kernel(ChunkWalk a, int number0, int number1) {
-    constexpr int W = D / 16;                               // waves, each with 16 key channels
+template <int D, bool DELTA, int TI>
+__global__ __launch_bounds__(D * 4 / TI) void chunk_walk_kernel(ChunkWalk a, int number0, int number1) {
+    constexpr int W = D / (16 * TI);                        // waves, each with TI tiles of 16 key channels
     constexpr int READ = W > 4 ? 4 : 0;                     // four waves multiply B by u (from 0 on), four read out (from here on)
     __shared__ __align__(16) float pu[DELTA ? 2 : 1][W][64][4], po[2][W][64][4];
     __shared__ float pn[2][W][16];
@@ -264,33 +267,38 @@ __global__ __launch_bounds__(D * 4) void chunk_walk_kernel(ChunkWalk a, int numb
     const int q0 = a.cu_q[e], q1 = a.cu_q[e + 1], first = dc_first(a.cu_q, e), chunks = (q1 - q0 + DC_TOKENS - 1) / DC_TOKENS;
     const int c0 = max(0, number0 - first), c1 = min(chunks, number1 - first);
     if (c0 >= c1) return;
-    const int row0 = wave * 16 + 4 * g;                     // lane (column r, g) has rows row0 .. row0 + 3
+    const int row0 = wave * 16 * TI + 4 * g;                // lane (column r, g) has rows row0 + 16 i .. + 3
     float* head = a.state + (size_t)slot * a.slot_stride + (size_t)h * a.head_stride;
     float* st = head + col0 + r;
     float* nm = head + (size_t)D * a.dv + (size_t)blockIdx.z * (D + 1);          // (mLSTM)
-    dc_f32x4_t S, N;
+    dc_f32x4_t S[TI], N[TI];
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-        S[x] = st[(size_t)(row0 + x) * a.dv];
-        N[x] = DELTA ? 0.f : nm[row0 + x];
-    }
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            S[i][x] = st[(size_t)(row0 + 16 * i + x) * a.dv];
+            N[i][x] = DELTA ? 0.f : nm[row0 + 16 * i + x];
+        }
     const int rec = dc_record(D, a.dv);
     auto record = [&](int c) { return a.ws + ((size_t)(first + min(c, c1 - 1) - number0) * a.H + h) * rec; };
     // this lane's operands of a chunk (mw: the mLSTM's sums of K; nb, em: its row's sum of B and e^-m).  Their places in a record are
     // 32-bit numbers that are worked out once, beside an address that the whole block has in common.
     const int o_row = 4 * g + (wave & 3);                   // the row that the lane reads out
-    const unsigned at_mw = 4u * ((DELTA ? r * D : 0) + row0), at_q = 4u * (16 * D + r * D + row0), at_k = 4u * (32 * D + (wave * 16 + r) * 16 + 4 * g);
+    const unsigned at_mw = 4u * ((DELTA ? r * D : 0) + row0), at_q = 4u * (16 * D + r * D + row0), at_k = 4u * (32 * D + (wave * 16 * TI + r) * 16 + 4 * g);
     const unsigned at_b = 4u * (48 * D + 16 * a.dv + r * 16 + 4 * g), at_g = 4u * (48 * D + 16 * a.dv + 256 + row0), at_n = 4u * (D + o_row);
     unsigned at_v[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) at_v[i] = 4u * (48 * D + (4 * g + i) * a.dv + col0 + r);
-    struct Ops { dc_f32x4_t mw, q, k, gl, b, mv; float nb, em; };
+    struct Ops { dc_f32x4_t mw[TI], q[TI], k[TI], gl[TI], b, mv; float nb, em; };
     auto load = [&](Ops& x, int c) {
         const char* p = reinterpret_cast<const char*>(record(c));
-        x.mw = *reinterpret_cast<const dc_f32x4_t*>(p + at_mw);
-        x.q = *reinterpret_cast<const dc_f32x4_t*>(p + at_q);
-        x.k = *reinterpret_cast<const dc_f32x4_t*>(p + at_k);
-        x.gl = *reinterpret_cast<const dc_f32x4_t*>(p + at_g);
+#pragma unroll
+        for (int i = 0; i < TI; ++i) {                      // (a tile's numbers lie 16 of a row, or 16 rows of 16, behind the one before)
+            x.mw[i] = *reinterpret_cast<const dc_f32x4_t*>(p + at_mw + 64 * i);
+            x.q[i] = *reinterpret_cast<const dc_f32x4_t*>(p + at_q + 64 * i);
+            x.k[i] = *reinterpret_cast<const dc_f32x4_t*>(p + at_k + 1024 * i);
+            x.gl[i] = *reinterpret_cast<const dc_f32x4_t*>(p + at_g + 64 * i);
+        }
         x.b = *reinterpret_cast<const dc_f32x4_t*>(p + at_b);
 #pragma unroll
         for (int i = 0; i < 4; ++i) x.mv[i] = *reinterpret_cast<const float*>(p + at_v[i]);
@@ -318,20 +326,26 @@ __global__ __launch_bounds__(D * 4) void chunk_walk_kernel(ChunkWalk a, int numb
         if (DELTA) {
             dc_f32x4_t u0 = {0.f, 0.f, 0.f, 0.f}, u1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < 4; j += 2) {
-                u0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[j], S[j], u0, 0, 0, 0);
-                u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[j + 1], S[j + 1], u1, 0, 0, 0);
-            }
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; j += 2) {
+                    u0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[i][j], S[i][j], u0, 0, 0, 0);
+                    u1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.mw[i][j + 1], S[i][j + 1], u1, 0, 0, 0);
+                }
             *reinterpret_cast<dc_f32x4_t*>(pu[DELTA ? c & 1 : 0][wave][lane]) = u0 + u1;
         }
         float nq = 0.f;
         if (!DELTA) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) nq = fmaf(x.q[j], N[j], nq);        // lane (token r, g): its rows' share of n . q
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) nq = fmaf(x.q[i][j], N[i][j], nq);        // lane (token r, g): its rows' share of n . q
             nq += __shfl_xor(nq, 16, 64);
             nq += __shfl_xor(nq, 32, 64);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) N[j] = fmaf(x.gl[j], N[j], x.mw[j]);
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) N[i][j] = fmaf(x.gl[i][j], N[i][j], x.mw[i][j]);
         }
         __syncthreads();                                    // parts of u of this chunk, and of the read-out of the chunk before
         dc_f32x4_t parts[DELTA ? W : 1];
@@ -341,18 +355,23 @@ __global__ __launch_bounds__(D * 4) void chunk_walk_kernel(ChunkWalk a, int numb
         }
         // (Q S0 runs while the parts of u come out of LDS)
 #pragma unroll
-        for (int j = 0; j < 4; j += 2) {
-            o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[j], S[j], o0, 0, 0, 0);
-            o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[j + 1], S[j + 1], o1, 0, 0, 0);
-        }
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; j += 2) {
+                o0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][j], S[i][j], o0, 0, 0, 0);
+                o1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[i][j + 1], S[i][j + 1], o1, 0, 0, 0);
+            }
         dc_f32x4_t u = x.mv;
         if (DELTA) {
 #pragma unroll
             for (int w = 0; w < W; ++w) u -= parts[w];
         }
-        S *= x.gl;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) S = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[j], u[j], S, 0, 0, 0);
+        for (int i = 0; i < TI; ++i) S[i] *= x.gl[i];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < TI; ++i) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[i][j], u[j], S[i], 0, 0, 0);
         if (wave < 4) {
             // of B u, this wave's share: tokens s = 4 g + wave
             float bw = x.b[0], uw = u[0];
@@ -391,10 +410,12 @@ __global__ __launch_bounds__(D * 4) void chunk_walk_kernel(ChunkWalk a, int numb
     __syncthreads();
     if (wave >= READ) read_out(c1 - 1, nb, em);
 #pragma unroll
-    for (int y = 0; y < 4; ++y) {
-        st[(size_t)(row0 + y) * a.dv] = S[y];
-        if (!DELTA && r == 0) nm[row0 + y] = N[y];
-    }
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) {
+            st[(size_t)(row0 + 16 * i + y) * a.dv] = S[i][y];
+            if (!DELTA && r == 0) nm[row0 + 16 * i + y] = N[i][y];
+        }
     if (!DELTA && threadIdx.x == 0) nm[D] = a.mfin[(size_t)e * a.H + h];
 }
 
@@ -415,10 +436,12 @@ int delta_chunks(const DeltaChunks& a, int dtype, hipStream_t st) {
         const dim3 pgrid((unsigned)(n1 - n0), a.H), wgrid(a.S, a.H, a.dv / 16);
         if (a.d == 64) {
             SPY_DISPATCH(dtype, TA, (delta_chunk_prepare_kernel<TA, 64><<<pgrid, 256, 0, st>>>(a, (int)n0)));
-            chunk_walk_kernel<64, true><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
+            chunk_walk_kernel<64, true, 1><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
         } else {
             SPY_DISPATCH(dtype, TA, (delta_chunk_prepare_kernel<TA, 128><<<pgrid, 256, 0, st>>>(a, (int)n0)));
-            chunk_walk_kernel<128, true><<<wgrid, 512, 0, st>>>(w, (int)n0, n1);
+            // (more blocks than compute units: fewer waves, see the top)
+            if ((int64_t)a.S * a.H * (a.dv / 16) > 256) chunk_walk_kernel<128, true, 2><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
+            else chunk_walk_kernel<128, true, 1><<<wgrid, 512, 0, st>>>(w, (int)n0, n1);
         }
         SPY_CHECK_LAUNCH("spy_delta_rule (chunks)");
     }
@@ -436,10 +459,10 @@ int memory_chunks(const MemoryChunks& a, int dtype, hipStream_t st) {
         const dim3 pgrid((unsigned)(n1 - n0), a.H), wgrid(a.S, a.H, a.dv / 16);
         if (a.d == 64) {
             SPY_DISPATCH(dtype, TA, (memory_chunk_prepare_kernel<TA, 64><<<pgrid, 256, 0, st>>>(a, (int)n0)));
-            chunk_walk_kernel<64, false><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
+            chunk_walk_kernel<64, false, 1><<<wgrid, 256, 0, st>>>(w, (int)n0, n1);
         } else {
             SPY_DISPATCH(dtype, TA, (memory_chunk_prepare_kernel<TA, 128><<<pgrid, 256, 0, st>>>(a, (int)n0)));
-            chunk_walk_kernel<128, false><<<wgrid, 512, 0, st>>>(w, (int)n0, n1);
+            chunk_walk_kernel<128, false, 1><<<wgrid, 512, 0, st>>>(w, (int)n0, n1);
         }
         SPY_CHECK_LAUNCH("spy_mlstm (chunks)");
     }

@@ -28,7 +28,9 @@ def unit(x):
 
 # heads, kv heads, key size, value size, decays per head (0: one per channel), lengths of the steps' entries
 CASES = [(2, 1, 128, 128, 0, [(1, 17), (16, 31)]), (4, 2, 64, 48, 0, [(15, 1, 40), (2, 33, 1)]), (3, 3, 128, 16, 1, [(50, 5), (1, 1), (64, 2)]),
-         (1, 1, 64, 32, 0, [(2300,), (7,)]), (2, 2, 128, 32, 1, [(1, 1, 1, 1, 2)])]
+         (1, 1, 64, 32, 0, [(2300,), (7,)]), (2, 2, 128, 32, 1, [(1, 1, 1, 1, 2)]),
+         # more blocks than compute units
+         (11, 11, 128, 48, 0, [(17, 2, 16, 1, 33, 5, 1, 20), (1,) * 7 + (35,)])]
 
 
 @pytest.mark.parametrize("how", ["slow", "fast", "mixed"])
