@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("d,n_q,n_kv,T,normed", [(16, 3, 1, 64, True), (32, 4, 2, 77, False), (64, 6, 2, 130, True), (128, 5, 5, 211, True), (256, 2, 1, 65, False)])
+@pytest.mark.parametrize("d,n_q,n_kv,T,normed", [(16, 3, 1, 64, True), (32, 4, 2, 77, False), (64, 6, 2, 130, True), (128, 5, 5, 211, True), (256, 2, 1, 65, False), (256, 2, 1, 260, True)])
 @pytest.mark.parametrize("order", ["straight", "shifted", "mixed"])
 def test_many_tokens(d, n_q, n_kv, T, normed, order, dtype):
     from spyinfer_amd.kernels import ops
