@@ -362,7 +362,8 @@ static bool gs_large_tile(int M, int N, int K, int parts) {
 
 // More than 32 rows (below, the products are bound by W's way from memory: 24 rows, 4096 x 1024 8.7 us / 18.7), and without parts tiles
 // for half of the compute units (2048 x 2048, 90 rows: 64 tiles 22 / 33; 4096 x 2048: 128 tiles 38.5 / 30.5 with a widened matrix, 38.3 with one of
-// float32 values; the smallest of that many, 4096 x 1024, 22.8 / 18.0 and 22.5).
+// float32 values; the smallest of that many, 4096 x 1024, 22.8 / 18.0 and 22.5; 65 rows, the fewest of two tiles, 36.1 / 30.3 and 38.2, 20.9 / 17.8 and
+// 21.9: what float32 values lose there is less than widened ones, which a call cannot tell from them beforehand, gain).
 bool gemm_f32_split_takes(int M, int N, int K, int parts) {
     return M > 32 && K % GS_BK == 0 && (int64_t)M * K < (1 << 29) && (int64_t)N * K < (1 << 29)
         && (parts > 1 || (int64_t)((M + 63) / 64) * ((N + 63) / 64) >= 128);
