@@ -907,13 +907,14 @@ def _gemm_decode(x, tiled: torch.Tensor, epi: int, n_out: int, out, resid, xw_ou
     K = tiled.shape[1]
     if isinstance(x, ScaledInput):
         xs, ss, eps = x.xw, x.ss_parts, x.eps
-        _check(ss.dtype == torch.float32 and ss.dim() == 2 and ss.shape[0] > 0,
+        _check(ss.dtype == torch.float32 and ss.dim() == 2,
                "decode product: the parts of the sums of squares must be float32 [n, rows rounded up to 16]")
+        parts_in, columns_in = ss.shape
     else:
-        xs, ss, eps = x, None, 0.0
+        xs, ss, eps, parts_in, columns_in = x, None, 0.0, 0, 0
     x_tiled = isinstance(xs, OperandRows)
     if x_tiled:
-        _check(xs.width == K and tuple(xs.data.shape) == (K // 32, xs.tiles, 64, 8) and xs.data.dtype == torch.bfloat16,
+        _check(xs.width == K and xs.data.shape == (K // 32, xs.tiles, 64, 8) and xs.data.dtype == torch.bfloat16,
                "decode product: x in operand order must be bfloat16 [%d / 32, row tiles, 64, 8]", K)
         M, xs = xs.rows, xs.data
     else:
@@ -921,11 +922,15 @@ def _gemm_decode(x, tiled: torch.Tensor, epi: int, n_out: int, out, resid, xw_ou
         M = xs.shape[0]
     out_tiled = isinstance(out, OperandRows) or isinstance(xw_out, OperandRows)
     mp = 16 * row_tiles(M)
-    _check(ss is None or ss.shape[1] == mp, "decode product: the parts of the sums of squares must have %d columns", mp)
-    _check(ss_out is None or tuple(ss_out.shape) in ((n_out // 16, mp), (n_out // 8, mp)), "decode product: the new parts must be [N / 16 or N / 8, %d]", mp)
+    _check(ss is None or (parts_in > 0 and columns_in == mp), "decode product: the parts of the sums of squares must be at least one, of %d columns", mp)
+    parts_out = 0
+    if ss_out is not None:
+        _check(ss_out.dim() == 2, "decode product: the new parts must be [N / 16 or N / 8, %d]", mp)
+        parts_out, columns_out = ss_out.shape
+        _check(columns_out == mp and (parts_out == n_out // 16 or parts_out == n_out // 8), "decode product: the new parts must be [N / 16 or N / 8, %d]", mp)
     for o in (out, xw_out):
         if isinstance(o, OperandRows):
-            _check(o.rows == M and o.width == n_out and tuple(o.data.shape) == (n_out // 32, o.tiles, 64, 8),
+            _check(o.rows == M and o.width == n_out and o.data.shape == (n_out // 32, o.tiles, 64, 8),
                    "decode product: the output in operand order does not fit")
     out_t = out.data if isinstance(out, OperandRows) else out
     xw_t = xw_out.data if isinstance(xw_out, OperandRows) else xw_out
@@ -933,10 +938,9 @@ def _gemm_decode(x, tiled: torch.Tensor, epi: int, n_out: int, out, resid, xw_ou
     _check(0 < M <= FUSED_DECODE_MAX_ROWS, "decode product: %d rows (1..%d allowed)", M, FUSED_DECODE_MAX_ROWS)
     ws = decode_workspace(xs.device)
     at = lambda t: None if t is None else t.data_ptr()              # (argument types are declared: see _Hip)
-    hip().call("spy_gemm_decode", at(xs), 0 if ss is None else 1, at(ss), 0 if ss is None else ss.shape[0], eps, at(tiled), epi,
+    hip().call("spy_gemm_decode", at(xs), 0 if ss is None else 1, at(ss), parts_in, eps, at(tiled), epi,
                at(out_t), 0 if out_t is None else _code(out_t, "out"), at(resid), at(xw_t), at(w_next), at(ss_out), M, n_out, K,
-               1 if x_tiled else 0, 1 if out_tiled else 0, act, at(ws), 0 if ws is None else ws.numel(), 0 if ss_out is None else ss_out.shape[0],
-               _Hip.stream())
+               1 if x_tiled else 0, 1 if out_tiled else 0, act, at(ws), 0 if ws is None else ws.numel(), parts_out, _Hip.stream())
 
 
 def _rows_of(x) -> int:
@@ -987,14 +991,14 @@ def residual_parts(rows: int, columns: int, inner: Optional[int] = None) -> int:
 def decode_linear_residual(x, tiled: torch.Tensor, resid: torch.Tensor, next_norm_weight: torch.Tensor,
                            eps: float, norm=None) -> ScaledInput:
     """resid += x . w^T (float32, in place) for at most 128 rows (beyond 64: x in operand order only) -> the ScaledInput of the norm that reads the
-    stream next: bfloat16(resid * next_norm_weight) and the parts [N / 16, 16] of the new rows' sums of squares."""
-    N = tiled.shape[0]
+    stream next: bfloat16(resid * next_norm_weight) and the parts [``residual_parts``, 16 a row tile] of the new rows' sums of squares."""
+    N, K = tiled.shape
     M = _rows_of(x)
-    _check(resid.dtype == torch.float32 and resid.dim() == 2 and resid.shape == (M, N),
+    _check(resid.dtype == torch.float32 and resid.shape == (M, N),
            "decode_linear_residual: the stream must be float32 [M, %d]", N)
     _check(next_norm_weight.dtype == torch.bfloat16 and next_norm_weight.shape == (N,),
            "decode_linear_residual: the next norm's weight must be bfloat16 [%d]", N)
-    ss = torch.empty((residual_parts(M, N, tiled.shape[1]), 16 * row_tiles(M)), dtype=torch.float32, device=resid.device)
+    ss = torch.empty((residual_parts(M, N, K), 16 * row_tiles(M)), dtype=torch.float32, device=resid.device)
     if _operand_order_ok(N):
         xw = OperandRows.empty(M, N, resid.device)
     else:
