@@ -11,7 +11,7 @@
 // 128, all there is.  A turn is 128 of K: X's next 128 go from memory into the other of two LDS stages while this one's 16 MT
 // products run, and a step's W registers are asked for again, for the next turn, as soon as their last product is issued.  Piece p of
 // an LDS row lies at place p ^ (row % 16), which the lanes' source addresses see to, so that the operands' reads meet in no bank.
-// Two blocks fit a compute unit.  Turns of 256 (twice the bytes under way) and loads spread over the products one by one were not faster.
+// Two blocks fit a compute unit.  (Blocks of 9 to 16 row tiles, one a unit: gemm_rows_tall.hip, for all but small shares of work.)  Turns of 256 (twice the bytes under way) and loads spread over the products one by one were not faster.
 //
 // Why parts: a prompt of a few hundred rows has fewer tiles than compute units, and each would walk all of K alone.  Measured (us;
 // library, this kernel, and what the sum of its parts adds to the norm's pass):  409 rows, 2560 x 9728: 53.7, 27.8 + 5 (six parts);
@@ -21,15 +21,7 @@
 // (Each with expf and a division in the epilogue; with gated_value_short 409 rows 46.1 -> 45.1, 1356 rows 65.4 -> 63.5, 2048 rows, 24576 x 4096 333 -> 323.)
 // What bounds it: a turn takes 0.7 + 0.05 MT us, its 16 MT products per SIMD 0.11 MT us of that at four waves a compute unit; the rest
 // is the loads' way, from memory where few tiles share W, and the turn's barrier.
-#include "common.h"
-
-#define ROWS_STORE 0
-#define ROWS_PARTS 1
-#define ROWS_GATED 2
-#define ROWS_DIES 8
-
-typedef __bf16 gr_bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float gr_f32x4_t __attribute__((ext_vector_type(4)));
+#include "gemm_rows.h"
 
 // X and W are not declared free of aliases: the waits below count the loads issued before them, and with that promise the compiler may
 // move loads of W across a wait.
@@ -204,7 +196,7 @@ static int rows_blocks(int tiles, int most, int columns) {
     return max(fewest, (int)min((int64_t)256 * each / columns, (int64_t)tiles / 4));
 }
 
-// epi: what is formed (see the top): C bfloat16 [M, N], float32 [parts, M, N] or bfloat16 [M, N / 2].  X: bfloat16 rows [M, K]; W: the tiled copy of [N, K].  row_tiles: MT.
+// epi: what is formed (see the top): C bfloat16 [M, N], float32 [parts, M, N] or bfloat16 [M, N / 2].  X: bfloat16 rows [M, K]; W: the tiled copy of [N, K].  row_tiles: most of a block, 4 to 16.
 extern "C" int spy_gemm_rows(void* C, const void* X, const void* W, int M, int N, int K, int row_tiles, int parts, int epi, int act_code,
                              hipStream_t st) {
     GateAct act = {1.f, 0.f};
@@ -213,8 +205,14 @@ extern "C" int spy_gemm_rows(void* C, const void* X, const void* W, int M, int N
     SPY_REQUIRE(parts >= 1 && parts <= K / 128 && (parts == 1 || epi == ROWS_PARTS) && epi >= ROWS_STORE && epi <= ROWS_GATED, "spy_gemm_rows: %d parts of K = %d", parts, K);
     SPY_REQUIRE((((uintptr_t)C | (uintptr_t)X | (uintptr_t)W) % 16) == 0, "spy_gemm_rows: operands must be 16-byte aligned");
     SPY_REQUIRE(epi != ROWS_GATED || gate_act_of(act_code, &act), "spy_gemm_rows: unknown activation %d", act_code);
-    SPY_REQUIRE(row_tiles >= 4 && row_tiles <= 8, "spy_gemm_rows: %d row tiles", row_tiles);
-    const int tiles = (M + 15) / 16, n_rows = rows_blocks(tiles, row_tiles, (N + 255) / 256 * parts);
+    SPY_REQUIRE(row_tiles >= 4 && row_tiles <= 16, "spy_gemm_rows: %d row tiles", row_tiles);
+    const int tiles = (M + 15) / 16;
+    if (row_tiles > 8) {
+        const int shared = (tiles + row_tiles - 1) / row_tiles, MT = (tiles + shared - 1) / shared;
+        SPY_REQUIRE(MT > 8, "spy_gemm_rows: %d rows make no blocks of %d row tiles", M, row_tiles);
+        return gr_tall_launch(C, X, W, M, N, K, MT, shared, parts, epi, act, st);
+    }
+    const int n_rows = rows_blocks(tiles, row_tiles, (N + 255) / 256 * parts);
     switch (max(4, (tiles + n_rows - 1) / n_rows)) {
         case 4: return rows_launch<4>(C, X, W, M, N, K, n_rows, parts, epi, act, st);
         case 5: return rows_launch<5>(C, X, W, M, N, K, n_rows, parts, epi, act, st);

@@ -451,7 +451,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
         return decode_linear(x, tiled, out_dtype, out)
     if all_bf16 and tiled is not None and out_dtype == torch.bfloat16 and x.is_contiguous():
-        tiles = rows_product_stored(M, N, K, _step.replayed and not isinstance(w, TiledOnly))      # (whose library product copies the rows first)
+        tall = rows_product_tall(M, N, K, ROWS_STORE)
+        tiles = tall[0] if tall else rows_product_stored(M, N, K, _step.replayed and not isinstance(w, TiledOnly))      # (whose library product copies the rows first)
         if tiles and (x.data_ptr() | out.data_ptr()) % 16 == 0:
             _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
             hip().call("spy_gemm_rows", _ptr(out), _ptr(x), _ptr(tiled), M, N, K, tiles, 1, ROWS_STORE, 0, _Hip.stream())
@@ -635,6 +636,61 @@ def rows_product_gated(M: int, N: int, K: int, library: bool) -> int:
     return tiles
 
 
+#: what the estimate of a product by tall blocks is made of, microseconds, per kind of result: the launch; a turn of 128 of K, and each row
+#: tile of it; a round's way in and out, and each row tile of that; a turn's row tile in the rounds where every unit has a block (the clock falls)
+_TALL_US = {ROWS_STORE: (4.8, 0.32, 0.110, -2.8, 0.33, 0.039), ROWS_PARTS: (7.5, 0.33, 0.119, 0.6, -0.06, 0.023), ROWS_GATED: (1.3, 0.52, 0.113, -0.95, 0.59, 0.013)}
+
+
+def _rows_tall_us(M: int, N: int, K: int, tiles: int, parts: int, kind: int) -> float:
+    """Estimated time of ``spy_gemm_rows`` with ``tiles`` row tiles a block, more than eight (one block a compute unit), the norm's pass that sums the
+    parts counted.  Fitted to 2600 launches of 144 to 2048 rows, 1024 to 24576 columns and K of 1024 to 12288: 5 % rms (8 % stored)."""
+    launch, turn, turn_tile, way, way_tile, full = _TALL_US[kind]
+    blocks, turns = -(-M // (16 * tiles)) * -(-N // 256) * parts, -(-(K // 128) // parts)
+    time = launch + -(-blocks // 256) * (turns * (turn + turn_tile * tiles) + way + way_tile * tiles) + full * (blocks // 256) * turns * tiles
+    return time + ((1.34 * parts + 1.09) * M * N / 1e6 if kind == ROWS_PARTS else 0.0)
+
+
+@functools.lru_cache(maxsize=1024)
+def rows_product_tall(M: int, N: int, K: int, kind: int, other: int = 0):
+    """(row tiles, parts of K) of blocks of more than eight row tiles, one a compute unit (csrc/gemm_rows_tall.hip), for a product of many rows,
+    or None where blocks of up to eight (``other``: those that the product would get) or the library's product are the better ones.  ``kind``:
+    ROWS_STORE, ROWS_PARTS (the next norm sums them) or ROWS_GATED.
+
+    What decides is a unit's share of the work, row tiles times blocks of 256 columns over 256 units: a tall block wants six and more,
+    fewer are spread better by small blocks.  Measured, us, what stood there / this:
+    stored: 4096 x 1024, 1500 rows (5.9 a unit) 16.9 / 16.7, 1700 (6.7) 19.0 / 17.3; 6144 x 2048, 1024 rows (6.0) 28.9 / 28.8, 1200 (7.0) 33.4 / 28.6,
+    2048 45.8 / 41.3; 6144 x 2560, 1356 rows 54.6 / 37.8; 6144 x 4096, 900 rows (5.3) 49.1 / 49.6, 2048 83.6 / 75.6; 15 or 16 row tiles
+    on nearly every unit are the library's own tile: 8192 x 2048, 2048 rows 52.0 / 53.1.
+    gated: 12288 x 2048, 640 rows (7.5) 32.6 / 34.2, 760 (9.0) 43.8 / 36.9, 1356 70.3 / 65.9; 19456 x 2560, 360 rows (6.8) 38.9 / 44.5, 409 (7.7)
+    53.5 / 41.6, 2048 165 / 160; two rounds of nine for 13 a unit: 24576 x 4096, 550 rows 99 / 112, which the estimates tell; against the
+    library and its activation's pass: 24576 x 4096, 300 rows 75.4 / 62.4, 2048 302 / 291; 17408 x 5120, 409 rows 89.2 / 70.0.  K = 1024: 2 % either way.
+    parts, with the norm that sums them, which multiply a unit's share: 2560 x 9728, 640 rows (1.6) 43.4 / 44.4, 900 (2.2) 58.6 / 54.0, 2048 109 /
+    98; 2048 x 6144, 900 rows (1.8) 34.4 / 35.1, 1024 (2.0) 40.8 / 39.0, 2048 66.5 / 61.2; 4096 x 12288, 1356 rows 154 / 121, 2048 193 / 169; 2560 x
+    4096, 1200 rows 44.7 / 41.5, 2048 (5.0) 58.2 / 56.8; 4096 x 4096, 640 rows 44.8 / 37.3, 1500 rows (5.9) 64.6 / 64.5; 2048 x 2048, 1356 rows 31.3 / 28.7,
+    1700 32.2 / 31.7."""
+    if M < 144 or N % (32 if kind == ROWS_GATED else 16) or K % 128 or N * K >= 1 << 30 or M * K >= 1 << 30:
+        return None
+    rows, columns, chunks = -(-M // 16), -(-N // 256), K // 128
+    share = rows * columns / 256
+    if kind == ROWS_PARTS:
+        if N < 2048 or K < 2048 or share < (2.3 if K < 4096 else 2.0) or (share > 5.4 and K < 8192) or (K < 4096 and M * N > 3e6):
+            return None
+    elif K < (2048 if kind == ROWS_GATED else 1024) or share < (7.6 if kind == ROWS_GATED and other else 6.2):
+        return None
+    fits = [(t, p) for t in range(9, 17) if 16 * t <= M and -(-rows // -(-rows // t)) == t
+            for p in ((1,) if kind != ROWS_PARTS else range(1, min(6, chunks // 4) + 1))
+            if kind != ROWS_PARTS or (p * M * N * 4 <= PARTS_MAX_BYTES and -(-M // (16 * t)) * columns * p <= 512 and chunks // p <= 64)]
+    best = min(fits, key=lambda f: _rows_tall_us(M, N, K, f[0], f[1], kind), default=None)
+    if best is None or kind == ROWS_PARTS:
+        return best
+    blocks = -(-M // (16 * best[0])) * columns
+    if kind == ROWS_GATED and other:
+        return best if _rows_tall_us(M, N, K, best[0], 1, kind) < 0.96 * _rows_product_us(M, N, K, other, 1) else None
+    if share < 0.62 * -(-blocks // 256) * best[0] or (kind == ROWS_STORE and best[0] >= 15 and (blocks - 1) % 256 >= 200):
+        return None
+    return best
+
+
 class ProductParts:
     """A product's result while it still lies in parts [parts, T, N] float32 (K cut over blocks); the norm that reads the result
     sums them in its pass (``add_parts_rms_norm``).  To a block that adds what is pending itself it is an addend [T, N] like another:
@@ -682,7 +738,9 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor]
             hip().call("spy_gemm_f32_parts", _ptr(out), _ptr(x), _ptr(w), M, w.shape[0], K, parts, _Hip.stream())
             return ProductParts(out)
         return linear_few(x, w, tiled)
-    plan = rows_product_parts(M, w.shape[0], K) if tiled is not None and x.dtype == torch.bfloat16 and x.is_contiguous() else None
+    plan = None
+    if tiled is not None and x.dtype == torch.bfloat16 and x.is_contiguous():
+        plan = rows_product_tall(M, w.shape[0], K, ROWS_PARTS) or rows_product_parts(M, w.shape[0], K)
     if plan is None or x.data_ptr() % 16:
         return linear_few(x, w, tiled)
     _dev(x, tiled)
@@ -742,6 +800,8 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, tiled: Optional[torc
         return out
     if x.dtype == torch.bfloat16 and tiled is not None and x.is_contiguous():
         tiles = rows_product_gated(M, 2 * I, K, not isinstance(w_gate_up, TiledOnly))
+        tall = rows_product_tall(M, 2 * I, K, ROWS_GATED, tiles)
+        tiles = tall[0] if tall else tiles
         if tiles and x.data_ptr() % 16 == 0:
             _check(tiled.shape == w_gate_up.shape, "linear_swiglu: the tiled copy does not fit")
             out = torch.empty((M, I), dtype=x.dtype, device=x.device)
