@@ -10,7 +10,8 @@
 //     bursts of 4 and of MT at a turn's ends held the products up: a turn of nine row tiles took 3400 clocks, spread 2850, its
 //     products alone 2304; of thirteen 3780 of 3328;
 //   - results leave through LDS, so that a store's lanes write whole lines of a row (6144 x 4096, 2048 rows: 81 -> 73 us; straight from the
-//     sums a store is sixteen pieces of 32 bytes, and thirteen row tiles' took 14 250 clocks).
+//     sums a store is sixteen pieces of 32 bytes, and thirteen row tiles' took 14 250 clocks), formed by a short loop on their way
+//     (24576 x 4096 gated, 2048 rows: 292 -> 287 us).
 // A turn's X and W are 64 KB + 4 KB a row tile, so a product of thirteen row tiles moves 45 KB for what one of five moves 84 KB: the first-level
 // caches and L2s, which the small blocks keep busy, have half the work.  Measured, us, the small blocks or the library (with its activation's
 // pass, with the norm that sums parts) / this: gated, 19456 x 2560, 409 rows 53.5 / 41.6 (0.98 PFLOP/s), 24576 x 4096, 300 rows 75.4 / 62.4,
@@ -29,45 +30,20 @@ __device__ __forceinline__ void gr_mfma2(gr_f32x4_t& a, gr_f32x4_t& b, gr_bf16x8
 }
 __device__ __forceinline__ void gr_sums_settle() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 
-template <int MT, int EPI>
-__global__ __launch_bounds__(256, 1) void gemm_rows_tall_kernel(void* C, const bf16_t* X, const bf16_t* W, int M, int N, int K, int n_rows, int n_cols,
-                                                                int parts, int blocks, GateAct act) {
-    __shared__ __align__(1024) bf16_t stage0[MT * 16 * 128];
-    __shared__ __align__(1024) bf16_t stage1[MT * 16 * 128];
-    // (a die takes a run of the blocks in (part, columns, rows) order: see gemm_rows_kernel)
-    const int per = (blocks + ROWS_DIES - 1) / ROWS_DIES, idx = blockIdx.x / ROWS_DIES;
-    const int v = (blockIdx.x % ROWS_DIES) * per + idx;
-    if (idx >= per || v >= blocks) return;
-    const int cp = v / n_rows, col_t = cp % n_cols, part = cp / n_cols;
-    const int chunks = K / 128, c0 = (int)((long long)chunks * part / parts);
-    const int n = (int)((long long)chunks * (part + 1) / parts) - c0;                  // (at least one: the launcher's check)
-    const int row0 = min((v % n_rows) * MT * 16, M - MT * 16);                         // the last rows' tile ends with row M - 1
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int NT = N / 16;
-    const auto wres = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, N * K * 2, 0x00020000);
-    const auto xres = __builtin_amdgcn_make_buffer_rsrc((void*)X, 0, M * K * 2, 0x00020000);
-    const int w_lane = lane * 16, w_turn = N * 256;
-    int w_at[4];                                       // this wave's column tiles; one that does not exist reads the last (nothing is stored)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        int tile;
-        if (EPI == ROWS_GATED) tile = (j >> 1) * (NT / 2) + min(col_t * 8 + wave * 2 + (j & 1), NT / 2 - 1);
-        else tile = min(col_t * 16 + wave * 4 + j, NT - 1);
-        w_at[j] = __builtin_amdgcn_readfirstlane(c0 * w_turn + tile * 4096);
-    }
-    // X: a wave's load brings 4 rows of 256 bytes; lane l has the piece that belongs to place l % 16 of row l / 16
-    const int s_row = wave * 4 + (lane >> 4);
-    const int x_lane = (s_row * K + ((lane & 15) ^ s_row) * 8) * 2, x_at = (row0 * K + c0 * 128) * 2;
-    gr_f32x4_t acc[4][MT];
+// All turns of a block: n of them, of 128 of K.  wres, w_lane, w_at, w_turn: W's buffer, this lane's bytes in a load, each column tile's place and a
+// turn's bytes.  load_x(stage, i, c): asks for row tile i of turn c, straight into LDS (a wave 4 of its 16 rows).  Ends with nothing under way,
+// the stages free and the sums fit to be read.  MT: 8 to 16.
+template <int MT, typename RES, typename X>
+__device__ __forceinline__ void gr_tall_turns(gr_f32x4_t (&acc)[4][MT], RES wres, int w_lane, const int (&w_at)[4], int w_turn, int n, bf16_t* stage0, bf16_t* stage1,
+                                              int lane, X load_x) {
+    // (two arrays of their own: reads of a stage that the compiler cannot tell from the one that loads go to wait for these)
+    static_assert(MT >= 8 && MT <= 16, "eight loads of W go between the row tiles of a step");
+    const int r = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int i = 0; i < MT; ++i) acc[j][i] = gr_f32x4_t{0.f, 0.f, 0.f, 0.f};
     gr_bf16x8_t w[2][4][4];
-    auto load_x = [&](bf16_t* stage, int i, int c) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (__attribute__((address_space(3))) void*)(stage + (i * 4 + wave) * 512), 16, x_lane,
-                                                 x_at + i * 32 * K + c * 256, 0, 0);
-    };
     auto load_w = [&](int d, int s, int j, int c) {
         w[d][s][j] = __builtin_bit_cast(gr_bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(wres, w_lane, w_at[j] + c * w_turn + s * 1024, 0));
     };
@@ -126,55 +102,93 @@ __global__ __launch_bounds__(256, 1) void gemm_rows_tall_kernel(void* C, const b
     }
     if (c < n) products(0, stage0, stage1, n - 1, n - 1);
     gr_sums_settle();
-    // The results, a row tile at a time, through a corner of the stages that the wave has to itself: no load into them is under way, and
-    // the other waves have read them.  (A wave's LDS accesses stay in order.)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    // (a row tile's sums are read where they are written out, not all at once: registers)
-    auto sums = [&](int i) { asm volatile("" : "+a"(acc[0][i]), "+a"(acc[1][i]), "+a"(acc[2][i]), "+a"(acc[3][i])); };
+}
+
+// The results through a stage, up to three row tiles at a time, in a part that the wave has to itself (a wave's LDS accesses stay in order): the
+// sums go there as they are, and a loop of few instructions reads whole pieces of rows, forms the values and stores them.  Formed
+// where the sums lie, the values of sixteen row tiles are 20 to 40 KB of instructions that every block runs through once, and waits for.
+// PAIRED: the wave's columns 32 on are the up values of the first 32.  form(v, u): a piece's values in v (their up values in u) become
+// results; out, width: the block's first output row and the rows' length; at: this wave's first column.
+template <int MT, bool PAIRED, typename T, typename F>
+__device__ __forceinline__ void gr_tall_results(gr_f32x4_t (&acc)[4][MT], bf16_t* stage, T* out, int width, int at, int lane, int wave, F form) {
+    constexpr int LD = 68, CT = MT * 16 * 128 * 2 / (4 * 16 * LD * 4);       // (16 bytes more than a row: rows begin in other banks)
+    constexpr int VEC = 16 / sizeof(T), PIECES = (PAIRED ? 32 : 64) / VEC, ROWS = 64 / PIECES;
+    static_assert(CT >= 1, "four waves' row tiles fit the stage");
+    float* mine = reinterpret_cast<float*>(stage) + wave * CT * 16 * LD;
+    const int r = lane & 15, g = lane >> 4, col = (lane % PIECES) * VEC;
+#pragma unroll
+    for (int i0 = 0; i0 < MT; i0 += CT) {
+#pragma unroll
+        for (int i = i0; i < i0 + CT && i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) *reinterpret_cast<gr_f32x4_t*>(mine + ((i - i0) * 16 + r) * LD + j * 16 + 4 * g) = acc[j][i];
+        __builtin_amdgcn_sched_barrier(0);
+        const int rows = 16 * min(CT, MT - i0);
+#pragma unroll 1
+        for (int row = lane / PIECES; row < rows; row += ROWS) {
+            const float* from = mine + row * LD + col;
+            float v[VEC], u[VEC];
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) v[e] = from[e];
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) u[e] = PAIRED ? from[32 + e] : 0.f;
+            form(v, u);
+            if (at + col < width) {
+                T* o = out + (size_t)(i0 * 16 + row) * width + at + col;
+                if constexpr (sizeof(T) == 2) *reinterpret_cast<uint4*>(o) = uint4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
+                else *reinterpret_cast<gr_f32x4_t*>(o) = gr_f32x4_t{v[0], v[1], v[2], v[3]};
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+template <int MT, int EPI>
+__global__ __launch_bounds__(256, 1) void gemm_rows_tall_kernel(void* C, const bf16_t* X, const bf16_t* W, int M, int N, int K, int n_rows, int n_cols,
+                                                                int parts, int blocks, GateAct act) {
+    __shared__ __align__(1024) bf16_t stage0[MT * 16 * 128];
+    __shared__ __align__(1024) bf16_t stage1[MT * 16 * 128];
+    // (a die takes a run of the blocks in (part, columns, rows) order: see gemm_rows_kernel)
+    const int per = (blocks + ROWS_DIES - 1) / ROWS_DIES, idx = blockIdx.x / ROWS_DIES;
+    const int v = (blockIdx.x % ROWS_DIES) * per + idx;
+    if (idx >= per || v >= blocks) return;
+    const int cp = v / n_rows, col_t = cp % n_cols, part = cp / n_cols;
+    const int chunks = K / 128, c0 = (int)((long long)chunks * part / parts);
+    const int n = (int)((long long)chunks * (part + 1) / parts) - c0;                  // (at least one: the launcher's check)
+    const int row0 = min((v % n_rows) * MT * 16, M - MT * 16);                         // the last rows' tile ends with row M - 1
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int NT = N / 16;
+    const auto wres = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, N * K * 2, 0x00020000);
+    const auto xres = __builtin_amdgcn_make_buffer_rsrc((void*)X, 0, M * K * 2, 0x00020000);
+    const int w_lane = lane * 16, w_turn = N * 256;
+    int w_at[4];                                       // this wave's column tiles; one that does not exist reads the last (nothing is stored)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        int tile;
+        if (EPI == ROWS_GATED) tile = (j >> 1) * (NT / 2) + min(col_t * 8 + wave * 2 + (j & 1), NT / 2 - 1);
+        else tile = min(col_t * 16 + wave * 4 + j, NT - 1);
+        w_at[j] = __builtin_amdgcn_readfirstlane(c0 * w_turn + tile * 4096);
+    }
+    // X: a wave's load brings 4 rows of 256 bytes; lane l has the piece that belongs to place l % 16 of row l / 16
+    const int s_row = wave * 4 + (lane >> 4);
+    const int x_lane = (s_row * K + ((lane & 15) ^ s_row) * 8) * 2, x_at = (row0 * K + c0 * 128) * 2;
+    gr_f32x4_t acc[4][MT];
+    gr_tall_turns<MT>(acc, wres, w_lane, w_at, w_turn, n, stage0, stage1, lane, [&](bf16_t* stage, int i, int c) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (__attribute__((address_space(3))) void*)(stage + (i * 4 + wave) * 512), 16, x_lane,
+                                                 x_at + i * 32 * K + c * 256, 0, 0);
+    });
     if constexpr (EPI == ROWS_PARTS) {
-        constexpr int LD = 68;                         // floats a row: 64 columns and 16 bytes, so that rows begin in other banks
-        float* mine = (float*)stage0 + wave * 16 * LD;
-        const int col = (lane & 15) * 4, at = col_t * 256 + wave * 64 + col;
-#pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            sums(i);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) *reinterpret_cast<gr_f32x4_t*>(mine + r * LD + j * 16 + 4 * g) = acc[j][i];
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int h = 0; h < 4; ++h) {
-                const int row = h * 4 + (lane >> 4);
-                const gr_f32x4_t o = *reinterpret_cast<const gr_f32x4_t*>(mine + row * LD + col);
-                if (at < N) *reinterpret_cast<gr_f32x4_t*>((float*)C + ((size_t)part * M + row0 + i * 16 + row) * N + at) = o;
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        gr_tall_results<MT, false>(acc, stage0, (float*)C + ((size_t)part * M + row0) * N, N, col_t * 256 + wave * 64, lane, wave, [](float (&)[4], float (&)[4]) {});
+    } else if constexpr (EPI == ROWS_STORE) {
+        gr_tall_results<MT, false>(acc, stage0, (bf16_t*)C + (size_t)row0 * N, N, col_t * 256 + wave * 64, lane, wave, [](float (&)[8], float (&)[8]) {});
     } else {
-        constexpr int COLS = EPI == ROWS_GATED ? 32 : 64, LD = COLS + 8, PIECES = COLS / 8;      // columns of a wave, 16-byte pieces of its rows
-        bf16_t* mine = stage0 + wave * 16 * LD;
-        const int width = EPI == ROWS_GATED ? N / 2 : N;
-        const int col = (lane % PIECES) * 8, at = col_t * 4 * COLS + wave * COLS + col;
+        gr_tall_results<MT, true>(acc, stage0, (bf16_t*)C + (size_t)row0 * (N / 2), N / 2, col_t * 128 + wave * 32, lane, wave, [&](float (&v)[8], float (&u)[8]) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            sums(i);
-#pragma unroll
-            for (int j = 0; j < COLS / 16; ++j) {
-                float y[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) y[e] = EPI == ROWS_GATED ? gated_value_short(act, acc[j][i][e], acc[(j + 2) % 4][i][e]) : acc[j][i][e];
-                *reinterpret_cast<uint2*>(mine + r * LD + j * 16 + 4 * g) = uint2{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int h = 0; h < COLS / 32; ++h) {
-                const int row = h * (64 / PIECES) + lane / PIECES;
-                const uint4 o = *reinterpret_cast<const uint4*>(mine + row * LD + col);
-                if (at < width) *reinterpret_cast<uint4*>((bf16_t*)C + (size_t)(row0 + i * 16 + row) * width + at) = o;
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
+            for (int e = 0; e < 8; ++e) v[e] = gated_value_short(act, v[e], u[e]);
+        });
     }
 }
 

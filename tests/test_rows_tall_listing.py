@@ -1,31 +1,38 @@
-"""The matrix instructions that the blocks of many row tiles write out themselves (csrc/gemm_rows_tall.hip): the compiler does not see them as
+"""The matrix instructions that the tall blocks' products write out themselves (csrc/gemm_rows_tall.hip): the compiler does not see them as
 such, so its wait states are not there.  In the listing of every variant: no ordinary vector instruction in the two places before a
 product, and the sums read only behind the two long waits."""
 import re
 import subprocess
 
+import pytest
+
 from spyinfer_amd.kernels import build
 
 
-def test_no_vector_instruction_beside_a_product(tmp_path):
+@pytest.mark.parametrize("source,variants", [("gemm_rows_tall", 24)])
+def test_no_vector_instruction_beside_a_product(source, variants, tmp_path):
     out = str(tmp_path / "tall.s")
-    cmd = [build._hipcc()] + build.HIPCC_FLAGS + ["-I", build.CSRC, "-S", "--cuda-device-only", build.CSRC + "/gemm_rows_tall.hip", "-o", out]
+    cmd = [build._hipcc()] + build.HIPCC_FLAGS + ["-I", build.CSRC, "-S", "--cuda-device-only", build.CSRC + "/" + source + ".hip", "-o", out]
     done = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
     assert done.returncode == 0, done.stdout.decode(errors="replace")
     with open(out) as f:
-        kernels = re.findall(r"^(_Z\d+gemm_rows_tall_kernel\S*):(.*?)s_endpgm", f.read(), re.S | re.M)
-    assert len(kernels) == 24
+        kernels = re.findall(r"^(_Z\d+%s_kernel\S*):(.*?)^\.Lfunc_end" % source, f.read(), re.S | re.M)
+    assert len(kernels) == variants
     for name, body in kernels:
         lines = [x.split(";")[0].strip() for x in body.split("\n")]
-        lines = [x for x in lines if x and not x.startswith((".", ";"))]                  # (labels begin with a dot)
-        products = [i for i, x in enumerate(lines) if x.startswith("v_mfma")]
-        assert len(products) > 0
-        for i in products:
-            waits = 0
-            for x in reversed(lines[max(0, i - 2):i]):
-                if x.startswith("s_nop"):
-                    waits += int(x.split()[1], 0) + 1
-                assert waits >= 2 or x.startswith("v_mfma") or not x.startswith("v_"), (name, lines[i - 2:i + 1])
-        first = [i for i, x in enumerate(lines) if x.startswith("v_accvgpr_read") or (re.match(r"(ds_write|global_store|buffer_store|scratch_store)", x) and re.search(r"\ba(\d|\[)", x))]
-        assert first and min(first) > max(products), name
-        assert [x for x in lines[max(products):min(first)] if x.startswith("s_nop")][:2] == ["s_nop 15", "s_nop 15"], name
+        lines = [x for x in lines if x and not x.startswith(".")]                         # (labels begin with a dot)
+        products = read = 0
+        settled = True                                      # no product since the last two long waits
+        for i, x in enumerate(lines):
+            if x.startswith("v_mfma"):
+                products, settled, waits = products + 1, False, 0
+                for before in reversed(lines[max(0, i - 2):i]):
+                    if before.startswith("s_nop"):
+                        waits += int(before.split()[1], 0) + 1
+                    assert waits >= 2 or before.startswith("v_mfma") or not before.startswith("v_"), (name, lines[i - 2:i + 1])
+            elif (x == "s_nop 15" and lines[i - 1] == "s_nop 15") or x.startswith(("s_branch", "s_endpgm")):
+                settled = True                              # (what follows a branch that is always taken does not follow a product)
+            elif x.startswith("v_accvgpr_read") or (re.match(r"(ds_write|ds_store|global_store|buffer_store|scratch_store|v_)", x) and re.search(r"\ba(\d|\[)", x.split(",", 1)[-1])):
+                read += 1
+                assert settled, (name, lines[i - 2:i + 1])
+        assert products > 0 and read > 0, name
