@@ -15,6 +15,22 @@ __global__ __launch_bounds__(AW * 64, (FUSED && DMAX <= 128) ? 2 : 1) void atten
                                            sink, chunk, og, blockIdx.x, blockIdx.y, blockIdx.z, lds);
 }
 
+// The fused variant by blocks of eight waves (heads of 128), one a compute unit: for steps that have no more blocks than units.  A block's
+// waves then have half the turns, and the unit as many loads under way as with two blocks of four.  Two blocks of keys a wave under way, in two sets of registers,
+// were 0.8 us slower a launch (25 KB of code for 16).  Where the line lies: piece_waves in kernels/key_pieces.py.
+template <int FULL>
+__global__ __launch_bounds__(2 * AW * 64, 1) void attention_mfma_wide_kernel(
+    bf16_t* __restrict__ out, bf16_t* kc, bf16_t* vc,
+    int P, int num_pages, const int* __restrict__ cu_q, const int* __restrict__ pos0, const int* __restrict__ kv_len,
+    const int* __restrict__ block_table, int max_blocks, const int* __restrict__ tile_entry, const int* __restrict__ tile_row0,
+    int n_q, int n_kv, float scale, int window, float* __restrict__ ws, FusedQKV fz, int out_tiles, unsigned* counters, int log2p,
+    const int* __restrict__ pieces) {
+    __shared__ float lds[2 * AW * (128 / 4 + 2) * 64];
+    attention_mfma_body<128, true, FULL, 2 * AW>(out, nullptr, kc, vc, P, num_pages, cu_q, pos0, kv_len, block_table, max_blocks, tile_entry, tile_row0,
+                                                 n_q, n_kv, 128, scale, window, 0.f, 1, ws, fz, out_tiles, counters, log2p, pieces, nullptr,
+                                                 nullptr, 0, OutGate{}, blockIdx.x, blockIdx.y, blockIdx.z, lds);
+}
+
 static int dmax_of(int d) { return d <= 64 ? 64 : (d <= 128 ? 128 : 256); }
 
 // Floats of one part's sums in the workspace (keys cut by the host: one part per record).
@@ -29,14 +45,14 @@ extern "C" int64_t spy_attention_mfma_workspace(int num_tiles, int n_kv, int d, 
 // decode product that reads it next.
 // qkv != null: the fused variant (see the top of the file).  Then q is not read, every entry must be a single token
 // (T == S), head_dim 64, 128 or 256 with the whole head rotated (or no rotation: cos_t == null), and the new keys and
-// values are written to kc and vc by this call (store != 0).
+// values are written to kc and vc by this call (store != 0).  waves: of a block, 4, or 8 for keys cut by the host and heads of 128.
 extern "C" int spy_attention_mfma(void* out, const void* q, void* kc, void* vc, int P, int num_pages, const int* cu_q,
                                   const int* pos0, const int* kv_len, const int* block_table, int max_blocks, const int* tile_entry,
                                   const int* tile_row0, int num_tiles, int S, int T, int n_q, int n_kv, int d, float scale,
                                   int window, float softcap, int splits, float* ws, const void* qkv, const void* qw, const void* kw, int w_dtype,
                                   float eps, const float* cos_t, const float* sin_t, int max_pos, int store, int out_tiles,
                                   unsigned* counters, int n_counters, const int* pieces, int num_pieces, const float* dist, const float* sink,
-                                  int chunk, const void* gate, long long gate_ld, hipStream_t st) {
+                                  int chunk, const void* gate, long long gate_ld, int waves, hipStream_t st) {
     SPY_REQUIRE(!qkv || (!dist && !sink && !gate && !chunk), "spy_attention_mfma: the fused variant takes neither a penalty on the distance nor a sink, chunks or a gate");
     SPY_REQUIRE(chunk >= 0 && !(chunk > 0 && window > 0), "spy_attention_mfma: a window or chunks, not both");
     SPY_REQUIRE(!gate || (gate_ld >= (long long)n_q * d && gate_ld % 4 == 0 && ((uintptr_t)gate % 8) == 0),
@@ -75,6 +91,16 @@ extern "C" int spy_attention_mfma(void* out, const void* q, void* kc, void* vc, 
     if ((P & (P - 1)) == 0) { log2p = 0; while ((1 << log2p) < P) ++log2p; }
     const dim3 grid = pieces ? dim3(num_pieces, 1, 1) : dim3(num_tiles, n_kv, splits);
     const dim3 mgrid(num_tiles, n_kv);
+    SPY_REQUIRE(waves == AW || (waves == 2 * AW && pieces && d == 128), "spy_attention_mfma: blocks of %d waves", waves);
+    if (waves == 2 * AW) {
+#define ATT_WIDE(FL)                                                                                                          \
+        attention_mfma_wide_kernel<FL><<<grid, 2 * AW * 64, 0, st>>>((bf16_t*)out, (bf16_t*)kc, (bf16_t*)vc, P, num_pages, cu_q, pos0, kv_len, block_table, max_blocks, \
+                                                                     tile_entry, tile_row0, n_q, n_kv, scale, window, ws, fz, out_tiles, counters, log2p, pieces)
+        if (P <= 32) ATT_WIDE(FULL_STREAMED); else ATT_WIDE(FULL_KEPT);
+#undef ATT_WIDE
+        SPY_CHECK_LAUNCH("spy_attention_mfma");
+        return 0;
+    }
     // The parts merged by each (tile, kv head)'s last block instead of a second kernel: with counters (zeroed once by the
     // caller, one per tile and head, left at zero by every call; calls that overlap on one device race on them), up to
     // 16 parts (the grid's; the host's records may name up to 32 of an entry) and head sizes up to 128.

@@ -24,8 +24,10 @@
 // the raw q, k, v of the step's product itself.  A query row's values lie in one lane and the three lanes beside it the
 // way the rotation pairs them (dims j and j + d/2 are 32-wide chunks kk and kk + KK/2 of the same lane), so the
 // per-head RMS norm costs two lane exchanges and the rotation none.  The entry's new key is prepared the same way
-// by every lane for its own 8-value pieces, put in the place of the cache's row in the one block and round that reach
-// its position, and stored to the cache from there; so is the new value.  No other block reads that position.
+// by the last wave of the one block that reaches its position, while that wave's first keys are on their way: its score is
+// where the wave's running maximum starts, with a sum of one and the new value as the result so far.  The wave stores
+// both to the cache; nobody reads that position there.  (Put in the place of the cache's row in the keys' last block instead, by
+// every wave that might have it, it made the blocks with the new key end 1.7 us after the others.)
 // (The merge by the last block uses no fence: with device-scope fences on both sides, each of which writes back and
 // invalidates the whole L2, it took 26 us against 17 us at 8 requests.  What orders it instead is said at the site.)
 #pragma once
@@ -131,13 +133,14 @@ __device__ __forceinline__ void norm_rotate(bf16x8_t (&x)[KK], bool normed, cons
 // FULL_STREAMED / FULL_KEPT: whether the values are read with the hint that they will not be read again (pages of up to 32
 // keys) or without it (larger pages).
 constexpr int FULL_STREAMED = 1, FULL_KEPT = 2;
-// WAVES: AW, or 2 AW for blocks of eight waves (the merge then folds the upper four waves' sums into the lower four's first).
+// WAVES: AW, or 2 AW for blocks of eight waves.  These merge all at once in the fused variant, which has LDS for it; else the upper four waves'
+// sums are folded into the lower four's first.
 // Which (tile, kv head, part of the keys) the block has comes from the caller: its place in the grid, or (FUSED, `pieces`
 // given) from a record of 8 ints that the host made for this block: { entry, kv head, first and end block of 32 keys, number
 // of this part, parts of the (entry, kv head), first workspace slot of its parts, the entry's keys }.  The host cuts every
 // entry's keys by what the whole step has to read, so that blocks have even shares whatever the entries' lengths
 // are; a record with entry -1 is a block without work.
-// lds: the waves' O, m, l: AW (head sizes up to 128) or AW - 1 times (DMAX / 16 * 4 + 2) * 64 floats.
+// lds: the waves' O, m, l: AW (head sizes up to 128; the fused variant WAVES) or AW - 1 times (DMAX / 16 * 4 + 2) * 64 floats.
 template <int DMAX, bool FUSED, int FULL, int WAVES = AW>
 __device__ __forceinline__ void attention_mfma_body(
     bf16_t* __restrict__ out, const bf16_t* __restrict__ q, bf16_t* kc, bf16_t* vc,
@@ -200,12 +203,16 @@ __device__ __forceinline__ void attention_mfma_body(
     }
     // keys this tile can see: from the first row's window start to the last row's position
     const int last_row = min(nrows, row0 + 16) - 1;
-    const int hi = min(p0 + last_row / G, kvl - 1);
+    // (the fused variant's new key, at p0, is not read from the cache)
+    const int kvl_read = FUSED && fz.store ? min(kvl, p0) : kvl;
+    const int hi = min(p0 + last_row / G, kvl_read - 1);
     int lo = attention_first_key(p0 + row0 / G, window, chunk);
     lo &= ~31;
     const int nblk = hi >= lo ? (hi - lo) / 32 + 1 : 0;
     const int per = (nblk + splits - 1) / splits;
     const int b_begin = cut_by_host ? pc_begin : sp * per, b_end = min(nblk, cut_by_host ? pc_end : b_begin + per);
+    // the part whose keys reach p0 (the last one that has any, as the cut counts p0 among them; without the cut's records the last of all)
+    const bool has_new = FUSED && fz.store && wave == WAVES - 1 && sp == splits - 1;
 
     f32x4_t acc[DT];
 #pragma unroll
@@ -214,42 +221,40 @@ __device__ __forceinline__ void attention_mfma_body(
     if (sink && sp == 0 && wave == 0 && row_ok) { m = sink[head]; l = g == 0 ? 1.f : 0.f; }
     const float d1 = dist ? dist[head] : 0.f, d2 = dist ? dist[n_q + head] : 0.f;
 
-    // FUSED: the entry's one new token lies at position p0 = kvl - 1; its query rows have that position too.  The block
-    // whose keys reach it prepares the new key (every lane its pieces for its g, as for q) and takes the new value's
-    // elements of its rows dd.
     // The kernel's start is a chain of memory round trips (about a microsecond each when the step's weights have swept
     // the caches), so loads are issued in the order of what they depend on, each group together and ahead of any wait:
     // what depends on the block alone (raw k and v, the norm weights; the raw query row is on its way already), then
-    // what needs the entry's position (rotation table, pages), then the first keys (they need the pages); the norm and
-    // the rotation are worked out while the keys are on their way.
+    // what needs the entry's position (rotation table, pages), then the first keys and values (they need the pages); the norm and
+    // the rotation are worked out while these are on their way.
     const int newpos = p0;
-    bool has_new = false;
     bf16x8_t knew[KK];
-    bf16_t vnew[DT];
+    uint2 vnew[DT];                                        // the new value's dims 16 dt + 4 g on, as the results lie
+    bf16_t vstore[DMAX / 64];                              // and its dims lane, lane + 64, for the cache
     int new_page = -1;
     constexpr int HKF = FUSED ? KK / 2 : 1;
     float cs[HKF][8], sn[HKF][8];
     bf16x8_t wq_raw[FUSED ? KK : 1], wk_raw[FUSED ? KK : 1];
     const bool normed = FUSED && fz.qw != nullptr, rotated = FUSED && fz.cos_t != nullptr;
     if constexpr (FUSED) {
-        if (fz.store) {
+        if (has_new) {
             const bf16_t* base = fz.qkv + (size_t)q0 * (n_q + 2 * n_kv) * d;
             const bf16_t* kp_raw = base + (size_t)(n_q + hk) * d;
             const bf16_t* vp_raw = base + (size_t)(n_q + n_kv + hk) * d;
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) knew[kk] = *reinterpret_cast<const bf16x8_t*>(kp_raw + kk * 32 + 8 * g);
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) vnew[dt] = vp_raw[dt * 16 + r16];
+            for (int dt = 0; dt < DT; ++dt) vnew[dt] = *reinterpret_cast<const uint2*>(vp_raw + dt * 16 + 4 * g);
+#pragma unroll
+            for (int i = 0; i < DMAX / 64; ++i) vstore[i] = vp_raw[i * 64 + lane];
             if (normed) load_weight_pieces<KK>(wk_raw, fz.kw, fz.w_dtype, g);
         }
         if (normed) load_weight_pieces<KK>(wq_raw, fz.qw, fz.w_dtype, g);
         __builtin_amdgcn_sched_barrier(0);
-        has_new = fz.store && n == 1 && newpos >= lo + 32 * b_begin && newpos < lo + 32 * b_end;
     }
     // A wave's loop is a chain of memory round trips, so they are overlapped: pages are looked up two blocks ahead (both
     // lookups together); the keys of the next block are asked for as soon as this block's S^T products have read the
-    // key registers, and arrive while the softmax and the second product run; the values are asked for at the top of
-    // their block and arrive behind the first product.
+    // key registers, and arrive while the softmax and the second product run; a block's values are asked for behind the
+    // second product of the one before (the first's with its keys) and arrive behind the first product.
     int kpage = -1, vpage = -1, kpage_n = -1, vpage_n = -1;
 #define AM_LOOKUP(B, KP, VP)                                                                                  \
     {                                                                                                         \
@@ -258,8 +263,8 @@ __device__ __forceinline__ void attention_mfma_body(
         if ((B) < b_end) {                                                                                    \
             const int c0_ = lo + 32 * (B);                                                                    \
             const int ka_ = c0_ + 8 * (r16 >> 2) + (r16 & 3), kv_ = c0_ + 8 * g;                              \
-            if (ka_ < kvl) KP = bt[page_of(ka_)];                                                                \
-            if (kv_ < kvl) VP = bt[page_of(kv_)];                                                                \
+            if (ka_ < kvl_read) KP = bt[page_of(ka_)];                                                                \
+            if (kv_ < kvl_read) VP = bt[page_of(kv_)];                                                                \
         }                                                                                                     \
     }
     bf16x8_t ka[KK], kb[KK];
@@ -279,51 +284,16 @@ __device__ __forceinline__ void attention_mfma_body(
                 kb[kk] = zero8();                                                                             \
                 if (ok_ && dofs < d) {                                                                        \
                     ka[kk] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(kp_ + dofs));                                  \
-                    if (key_ + 4 < kvl) kb[kk] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(kp_ + 4 * d + dofs));      \
+                    if (key_ + 4 < kvl_read) kb[kk] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(kp_ + 4 * d + dofs));      \
                 }                                                                                             \
             }                                                                                                 \
         }                                                                                                     \
     }
-    AM_LOOKUP(b_begin + wave, kpage, vpage)
-    AM_LOOKUP(b_begin + wave + WAVES, kpage_n, vpage_n)
-    if constexpr (FUSED) {
-        if (has_new) new_page = bt[page_of(newpos)];
-        if (rotated) {
-            const size_t trow = (size_t)min(newpos, fz.max_pos - 1) * (d / 2);
-#pragma unroll
-            for (int kk = 0; kk < HKF; ++kk) {
-                const f32x4_t c0 = *reinterpret_cast<const f32x4_t*>(fz.cos_t + trow + kk * 32 + 8 * g);
-                const f32x4_t c1 = *reinterpret_cast<const f32x4_t*>(fz.cos_t + trow + kk * 32 + 8 * g + 4);
-                const f32x4_t s0 = *reinterpret_cast<const f32x4_t*>(fz.sin_t + trow + kk * 32 + 8 * g);
-                const f32x4_t s1 = *reinterpret_cast<const f32x4_t*>(fz.sin_t + trow + kk * 32 + 8 * g + 4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { cs[kk][e] = c0[e]; cs[kk][e + 4] = c1[e]; sn[kk][e] = s0[e]; sn[kk][e + 4] = s1[e]; }
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    if (b_begin + wave < b_end) AM_LOAD_K(b_begin + wave, kpage)
-    if constexpr (FUSED) {
-        __builtin_amdgcn_sched_barrier(0);
-        float wv[KK][8];
-        if (normed) widen_weight_pieces<KK>(wv, wq_raw, fz.qw, fz.w_dtype, g);
-        norm_rotate<KK>(bq, normed, wv, fz.eps, rotated, cs, sn, d);
-        if (has_new) {
-            if (normed) widen_weight_pieces<KK>(wv, wk_raw, fz.kw, fz.w_dtype, g);
-            norm_rotate<KK>(knew, normed, wv, fz.eps, rotated, cs, sn, d);
-            if (new_page < 0 || new_page >= num_pages) has_new = false;   // no page: nothing to store or to use
-        }
-    }
-    // One block of 32 keys.  LAST: the wave's last block, which alone can hold keys beyond the request's and the step's
-    // new key, and after which no keys are asked for; the blocks before it have no condition around their loads.
-    auto block = [&](const int b, auto last_block) {
-        constexpr bool LAST = decltype(last_block)::value;
-        const int c0 = lo + 32 * b;
-        const int key_a = c0 + 8 * (r16 >> 2) + (r16 & 3);      // tile a; tile b is key_a + 4
-        const int key_v = c0 + 8 * g;                             // this lane's 8 keys of V
-        const bool v_ok = vpage >= 0 && vpage < num_pages;
-        const bf16_t* vp = vc + (((size_t)(v_ok ? vpage : 0) * n_kv + hk) * d) * P + in_page(key_v);
-        bf16x8_t vt[DT];
+    bf16x8_t vt[DT];
+    auto load_v = [&](const int b, const int page) {
+        const int key_v = lo + 32 * b + 8 * g;                    // this lane's 8 keys of V
+        const bool v_ok = page >= 0 && page < num_pages;
+        const bf16_t* vp = vc + (((size_t)(v_ok ? page : 0) * n_kv + hk) * d) * P + in_page(key_v);
         if constexpr (FULL == FULL_STREAMED) {
             // (a block's 32 keys of a dim are whole lines of pages of up to 32 keys: read once, not to be kept)
 #pragma unroll
@@ -349,34 +319,70 @@ __device__ __forceinline__ void attention_mfma_body(
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) vt[dt] = zero8();
         }
-        int kpage_nn, vpage_nn;
-        AM_LOOKUP(b + 2 * WAVES, kpage_nn, vpage_nn)
-        if (FUSED && LAST && has_new && newpos >= c0 && newpos < c0 + 32) {
-            // the new key: the four lanes of its row take the prepared pieces; the lanes with r16 % 16 == its row store it
-            const bool mine_a = key_a == newpos, mine_b = key_a + 4 == newpos;
+    };
+    AM_LOOKUP(b_begin + wave, kpage, vpage)
+    AM_LOOKUP(b_begin + wave + WAVES, kpage_n, vpage_n)
+    if constexpr (FUSED) {
+        if (has_new) new_page = bt[page_of(newpos)];
+        if (rotated) {
+            const size_t trow = (size_t)min(newpos, fz.max_pos - 1) * (d / 2);
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                if (mine_a) ka[kk] = knew[kk];
-                if (mine_b) kb[kk] = knew[kk];
-            }
-            if (mine_a || mine_b) {
-                bf16_t* dst = kc + (((size_t)new_page * n_kv + hk) * P + in_page(newpos)) * d + 8 * g;
+            for (int kk = 0; kk < HKF; ++kk) {
+                const f32x4_t c0 = *reinterpret_cast<const f32x4_t*>(fz.cos_t + trow + kk * 32 + 8 * g);
+                const f32x4_t c1 = *reinterpret_cast<const f32x4_t*>(fz.cos_t + trow + kk * 32 + 8 * g + 4);
+                const f32x4_t s0 = *reinterpret_cast<const f32x4_t*>(fz.sin_t + trow + kk * 32 + 8 * g);
+                const f32x4_t s1 = *reinterpret_cast<const f32x4_t*>(fz.sin_t + trow + kk * 32 + 8 * g + 4);
 #pragma unroll
-                for (int kk = 0; kk < KK; ++kk) *reinterpret_cast<bf16x8_t*>(dst + kk * 32) = knew[kk];
-            }
-            // the new value: element newpos - key_v of the lanes whose 8 keys hold it
-            const int jn = newpos - key_v;
-            if (jn >= 0 && jn < 8) {
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) {
-#pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        if (j == jn) vt[dt][j] = (short)vnew[dt];
-                    vc[(((size_t)new_page * n_kv + hk) * d + dt * 16 + r16) * P + in_page(newpos)] = vnew[dt];
-                }
+                for (int e = 0; e < 4; ++e) { cs[kk][e] = c0[e]; cs[kk][e + 4] = c1[e]; sn[kk][e] = s0[e]; sn[kk][e + 4] = s1[e]; }
             }
         }
-        const int v_valid = min(8, kvl - key_v);                  // keys of the group that exist (slots beyond hold anything)
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (b_begin + wave < b_end) {
+        AM_LOAD_K(b_begin + wave, kpage)
+        load_v(b_begin + wave, vpage);
+    }
+    if constexpr (FUSED) {
+        __builtin_amdgcn_sched_barrier(0);
+        float wv[KK][8];
+        if (normed) widen_weight_pieces<KK>(wv, wq_raw, fz.qw, fz.w_dtype, g);
+        norm_rotate<KK>(bq, normed, wv, fz.eps, rotated, cs, sn, d);
+        if (has_new) {
+            if (normed) widen_weight_pieces<KK>(wv, wk_raw, fz.kw, fz.w_dtype, g);
+            norm_rotate<KK>(knew, normed, wv, fz.eps, rotated, cs, sn, d);
+            // every row of the first operand is the new key: all of a lane's four results are its query row's score
+            f32x4_t sn4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) sn4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(knew[kk], bq[kk], sn4, 0, 0, 0);
+            if (row_ok) {
+                m = sn4[0] * scale;
+                l = g == 0 ? 1.f : 0.f;                    // (the four lanes of a row hold partial sums)
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+                    acc[dt] = f32x4_t{__uint_as_float(vnew[dt].x << 16), __uint_as_float(vnew[dt].x & 0xffff0000u),
+                                      __uint_as_float(vnew[dt].y << 16), __uint_as_float(vnew[dt].y & 0xffff0000u)};
+            }
+            if (new_page >= 0 && new_page < num_pages) {   // (no page: nothing to store)
+                if (r16 == 0) {
+                    bf16_t* dst = kc + (((size_t)new_page * n_kv + hk) * P + in_page(newpos)) * d + 8 * g;
+#pragma unroll
+                    for (int kk = 0; kk < KK; ++kk) *reinterpret_cast<bf16x8_t*>(dst + kk * 32) = knew[kk];
+                }
+#pragma unroll
+                for (int i = 0; i < DMAX / 64; ++i) vc[(((size_t)new_page * n_kv + hk) * d + i * 64 + lane) * P + in_page(newpos)] = vstore[i];
+            }
+        }
+    }
+    // One block of 32 keys.  LAST: the wave's last block, which alone can hold keys beyond the request's, and after which
+    // nothing is asked for; the blocks before it have no condition around their loads.
+    auto block = [&](const int b, auto last_block) {
+        constexpr bool LAST = decltype(last_block)::value;
+        const int c0 = lo + 32 * b;
+        const int key_v = c0 + 8 * g;                             // this lane's 8 keys of V
+        const bool v_ok = vpage >= 0 && vpage < num_pages;
+        int kpage_nn, vpage_nn;
+        AM_LOOKUP(b + 2 * WAVES, kpage_nn, vpage_nn)
+        const int v_valid = min(8, kvl_read - key_v);                  // keys of the group that exist (slots beyond hold anything)
         // ---- S^T = K . Q^T ------------------------------------------------------------------
         f32x4_t sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -388,10 +394,6 @@ __device__ __forceinline__ void attention_mfma_body(
         }
         // the key registers are free: the next block's keys
         if (!LAST) AM_LOAD_K(b + WAVES, kpage_n)
-        kpage = kpage_n;
-        vpage = vpage_n;
-        kpage_n = kpage_nn;
-        vpage_n = vpage_nn;
         if ((LAST || !FULL) && (FULL || v_ok) && v_valid < 8) {
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)
@@ -408,7 +410,7 @@ __device__ __forceinline__ void attention_mfma_body(
             float v = (j < 4 ? sa[j] : sb[j - 4]) * scale;
             if (softcap > 0.f) v = softcap * capped_tanh(v * inv_cap);          // scores capped: cap tanh(score / cap)
             if (dist) v -= d1 * __logf(fmaf(d2, (float)max(pos - key, 0), 1.0f));
-            const bool ok = row_ok && key <= pos && key >= lo_row && key < kvl;
+            const bool ok = row_ok && key <= pos && key >= lo_row && key < kvl_read;
             sc[j] = ok ? v : -INFINITY;
             bmax = fmaxf(bmax, sc[j]);
         }
@@ -437,6 +439,11 @@ __device__ __forceinline__ void attention_mfma_body(
                 acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[dt], pb, acc[dt], 0, 0, 0);
             }
         }
+        if (!LAST) load_v(b + WAVES, vpage_n);
+        kpage = kpage_n;
+        vpage = vpage_n;
+        kpage_n = kpage_nn;
+        vpage_n = vpage_nn;
     };
     {
         int b = b_begin + wave;
@@ -454,10 +461,11 @@ __device__ __forceinline__ void attention_mfma_body(
     // beyond 128 the four waves' sums do not fit the LDS that a block may ask for: there wave 0 merges them all.)
     constexpr int PER = DT * 4 + 2;
     constexpr bool SPREAD = DMAX <= 128;
-    constexpr int MINE = SPREAD ? DT / AW : DT;       // tiles of the head dim that this wave merges
-    static_assert(!SPREAD || DT % AW == 0, "the head dim's tiles are dealt evenly to the waves");
+    constexpr int MW = FUSED ? WAVES : AW;            // waves that merge
+    constexpr int MINE = SPREAD ? DT / MW : DT;       // tiles of the head dim that this wave merges
+    static_assert(!SPREAD || DT % MW == 0, "the head dim's tiles are dealt evenly to the waves");
     const int dt0 = SPREAD ? wave * MINE : 0;
-    if constexpr (WAVES == 2 * AW) {
+    if constexpr (WAVES > MW) {
         // the upper waves' sums into the lower waves', wave AW + w into wave w; then the lower waves merge as below
         static_assert(SPREAD, "blocks of eight waves: head sizes up to 128");
         if (wave >= AW) {
@@ -481,7 +489,7 @@ __device__ __forceinline__ void attention_mfma_body(
     }
     f32x4_t mo[MINE];
     if (SPREAD) {
-        if (WAVES == AW || wave < AW) {
+        if (WAVES == MW || wave < MW) {
             float* mine = lds + (size_t)wave * PER * 64;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4_t*>(mine + (dt * 64 + lane) * 4) = acc[dt];
@@ -489,11 +497,11 @@ __device__ __forceinline__ void attention_mfma_body(
             mine[(DT * 4 + 1) * 64 + lane] = l;
         }
         __syncthreads();
-        if (WAVES > AW && wave >= AW) return;
-        float mw[AW], lw[AW];
+        if (WAVES > MW && wave >= MW) return;
+        float mw[MW], lw[MW];
         float mn = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < AW; ++w) {
+        for (int w = 0; w < MW; ++w) {
             mw[w] = lds[((size_t)w * PER + DT * 4) * 64 + lane];
             lw[w] = lds[((size_t)w * PER + DT * 4 + 1) * 64 + lane];
             mn = fmaxf(mn, mw[w]);
@@ -502,7 +510,7 @@ __device__ __forceinline__ void attention_mfma_body(
 #pragma unroll
         for (int i = 0; i < MINE; ++i) mo[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < AW; ++w) {                 // in the order of the waves, whichever wave adds
+        for (int w = 0; w < MW; ++w) {                 // in the order of the waves, whichever wave adds
             const float a = (mw[w] == -INFINITY) ? 0.f : __expf(mw[w] - mn);
             l += lw[w] * a;
 #pragma unroll
@@ -582,12 +590,14 @@ __device__ __forceinline__ void attention_mfma_body(
         // system scope miss L1 and L2 (sc0 sc1) and so read what memory holds, and they are issued after the barrier
         // that follows the increment's return.  Do not weaken any of the three (ordinary stores, no wait, ordinary
         // loads), and do not "strengthen" the atomics to release/acquire without measuring: it is correct and slow.
-        // A part lies lane for lane: O[(dt 4 + i)][64 lanes], then m[16], l[16].
+        // A part lies lane for lane: O[(dt 2 + i)][64 lanes] in pairs of numbers, then m[16], l[16].
         __shared__ unsigned am_last;
 #pragma unroll
         for (int i = 0; i < MINE; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) __hip_atomic_store(w + ((dt0 + i) * 4 + j) * 64 + lane, mo[i][j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            for (int j = 0; j < 2; ++j)
+                __hip_atomic_store(reinterpret_cast<unsigned long long*>(w) + ((dt0 + i) * 2 + j) * 64 + lane,
+                                   (unsigned long long)__float_as_uint(mo[i][2 * j + 1]) << 32 | __float_as_uint(mo[i][2 * j]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         if (g == 0 && wave == 0) {
             __hip_atomic_store(w + 16 * DMAX + r16, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             __hip_atomic_store(w + 16 * DMAX + 16 + r16, l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -602,52 +612,69 @@ __device__ __forceinline__ void attention_mfma_body(
         }
         __syncthreads();
         if (!am_last) return;
-        // All that is read of the parts is asked for before any of it is used, eight parts at a time: one memory round
-        // trip for up to eight parts (a loop that adds as it loads has one per part; sixteen at a time cost the step of
-        // 8 requests, which has four parts, 1.2 us for the code's length).
+        // All that is read of eight parts is asked for before any of it is used: one memory round trip (a loop that adds as it loads
+        // has one per part).  A lane has the maximum and the sum of its row for every fourth part; the results come in pairs of
+        // numbers.  A loop of eight parts a turn, not all 32 written out: a block runs through this once, and code that the
+        // instruction cache has yet to get costs more than it does (steps of 8 requests 0.5 us a layer).
         constexpr int MAXS = 32, BATCH = 8;                // (the caller keeps to 32 parts: 16 from the grid, 32 in the host's records)
         constexpr int PART = 16 * (DMAX + 2);
         const float* base = ws + slot0 * PART;
-        float pm[MAXS], pl[MAXS];
+        float pm[MAXS / 4], pl[MAXS / 4];
 #pragma unroll
-        for (int i = 0; i < MAXS; ++i) {
-            pm[i] = -INFINITY;
-            pl[i] = 0.f;
-            if (i < splits) {
-                pm[i] = __hip_atomic_load(base + (size_t)i * PART + 16 * DMAX + r16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                pl[i] = __hip_atomic_load(base + (size_t)i * PART + 16 * DMAX + 16 + r16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        for (int i = 0; i < MAXS / 4; ++i) { pm[i] = -INFINITY; pl[i] = 0.f; }
+        auto load_sums = [&](int i) {
+            const int part = 4 * i + g;
+            if (part < splits) {
+                pm[i] = __hip_atomic_load(base + (size_t)part * PART + 16 * DMAX + r16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                pl[i] = __hip_atomic_load(base + (size_t)part * PART + 16 * DMAX + 16 + r16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             }
+        };
+        load_sums(0);
+        load_sums(1);
+        if (splits > BATCH) {
+#pragma unroll
+            for (int i = 2; i < MAXS / 4; ++i) load_sums(i);
         }
         f32x4_t o[MINE];
 #pragma unroll
         for (int i = 0; i < MINE; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         float mn = -INFINITY, L = 0.f;
-#pragma unroll
-        for (int i0 = 0; i0 < MAXS; i0 += BATCH) {
-            if (i0 >= splits) break;
-            float ov[BATCH][MINE][4];
+#pragma unroll 1
+        for (int i0 = 0; i0 < splits; i0 += BATCH) {
+            unsigned long long ov[BATCH][MINE][2];
 #pragma unroll
             for (int i = 0; i < BATCH; ++i)
 #pragma unroll
                 for (int k = 0; k < MINE; ++k)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        ov[i][k][j] = i0 + i < splits ? __hip_atomic_load(base + (size_t)(i0 + i) * PART + ((dt0 + k) * 4 + j) * 64 + lane,
-                                                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) : 0.f;
+                    for (int j = 0; j < 2; ++j)
+                        ov[i][k][j] = i0 + i < splits ? __hip_atomic_load(reinterpret_cast<const unsigned long long*>(base + (size_t)(i0 + i) * PART) + ((dt0 + k) * 2 + j) * 64 + lane,
+                                                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) : 0ull;
             if (i0 == 0) {
 #pragma unroll
-                for (int i = 0; i < MAXS; ++i) mn = fmaxf(mn, pm[i]);
+                for (int i = 0; i < MAXS / 4; ++i) mn = fmaxf(mn, pm[i]);
+                mn = fmaxf(mn, __shfl_xor(mn, 16, 64));
+                mn = fmaxf(mn, __shfl_xor(mn, 32, 64));
             }
+            // (this turn's parts' weights: of part 4 i + g in lane group g; the later turns' move up)
+            const float a0 = pm[0] == -INFINITY ? 0.f : __expf(pm[0] - mn), a1 = pm[1] == -INFINITY ? 0.f : __expf(pm[1] - mn);
+            L += pl[0] * a0 + pl[1] * a1;
 #pragma unroll
             for (int i = 0; i < BATCH; ++i) {              // in the order of the parts
-                const float a = (pm[i0 + i] == -INFINITY) ? 0.f : __expf(pm[i0 + i] - mn);
-                L += pl[i0 + i] * a;
+                const float a = __shfl(i < 4 ? a0 : a1, (i & 3) * 16 + r16, 64);
 #pragma unroll
                 for (int k = 0; k < MINE; ++k)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) o[k][j] += a * ov[i][k][j];
+                    for (int j = 0; j < 2; ++j) {
+                        o[k][2 * j] += a * __uint_as_float((uint32_t)ov[i][k][j]);
+                        o[k][2 * j + 1] += a * __uint_as_float((uint32_t)(ov[i][k][j] >> 32));
+                    }
             }
+#pragma unroll
+            for (int i = 0; i + 2 < MAXS / 4; ++i) { pm[i] = pm[i + 2]; pl[i] = pl[i + 2]; }
         }
+        L += __shfl_xor(L, 16, 64);
+        L += __shfl_xor(L, 32, 64);
         if (!row_ok) return;
         const float inv = L > 0.f ? 1.0f / L : 0.f;
         bf16_t* op = out + ((size_t)(q0 + tq) * n_q + head) * d;

@@ -31,8 +31,17 @@ PIECE_SHARED_US = 0.56      # what all units reading at once add to it (the two 
 PIECE_FEW = 4               # most requests whose lengths are taken as they are (a choice in 8 to 32 steps)
 PIECE_WAVES = 4             # waves of a block, which take its blocks of keys in turn
 PIECE_TURN_US = 1.75        # a turn (heads of 128: 1 to 4 requests of 130 to 1300 keys)
+PIECE_WIDE_US = 0.37        # a block of 32 keys in a block of eight waves that has its unit to itself
 PIECE_PARTS_US = 2.35       # the merge of an entry's parts, and
 PIECE_PART_US = 0.17        # each part of it, up to the eight that the merging block asks for at a time
+
+
+def piece_waves(entries: int, n_kv: int, d: int) -> int:
+    """Waves of a block of the fused attention kernel for keys that are cut here (a launch shape: it follows the entries' number alone): eight where
+    every (entry, kv head) has a compute unit of its own, and as many again are left for five eighths of them to be cut (8 kv heads of 128, four
+    waves / eight, each with its cut, us a layer less: 1 request of 500 keys 1.5, 8 of 1152 1.9, 16 of 1300 2.2, 18 of 100 to 900 1.5; beyond
+    the line 24 and 32 of one length 0.6 to 2.4 less, 32 of 100 to 500 1.3 less, but 24 of 100 to 1300, too few units for their parts, 3.0 more)."""
+    return 8 if d == 128 and 8 * entries * n_kv <= 5 * PIECE_UNITS else PIECE_WAVES
 
 
 def decode_pieces_capacity(entries: int, n_kv: int) -> int:
@@ -156,6 +165,21 @@ def _few_width(nblk, n_kv):
     return None if whole <= best[2] else (best[1], True, PIECE_WAVES)
 
 
+def _wide_width(nblk, n_kv):
+    """The width for entries whose pieces, in blocks of eight waves, all find a compute unit of their own: None (whole) or (W, even).  A block's time goes
+    by its blocks of keys, 0.37 us each, an entry in parts takes 1.1 us more, and 0.55 for each eight parts beyond eight (18 steps of 1 to 16 requests of
+    130 to 1500 keys, every number of parts: 0.3 us rms, the choice within 0.3 us of the best)."""
+    longest = int(nblk.max(initial=1))
+    parts = np.arange(1, (MAX_PARTS if longest > 64 else 8) + 1)       # (up to eight are asked for at once)
+    width = np.unique(np.maximum(np.maximum(1, PIECE_MIN_BLOCKS // 2), -(-longest // parts)))
+    each = -(-nblk[None, :] // width[:, None])                     # parts of every entry at every width
+    most = each.max(axis=1)
+    time = PIECE_WIDE_US * (-(-longest // most)) + np.where(most > 1, PIECE_MERGE_US * 0.37, 0.0) + PIECE_MERGE_MORE_US * 0.22 * (-(-most // 8) - 1)
+    time = np.where(each.sum(axis=1) * n_kv <= PIECE_UNITS, time, np.inf)
+    best = int(time.argmin())
+    return None if most[best] <= 1 or not np.isfinite(time[best]) else (int(width[best]), True, PIECE_WAVES)
+
+
 _piece_choices = {}
 
 
@@ -165,8 +189,8 @@ def _piece_choice(nblk, n_kv, d=128):
     longest entry 16 parts, or 32), an entry's parts of one size or W and a rest, or ("fill", True) (``_fill_widths``):
     whichever has the shortest estimated time.
     Decided from the lengths rounded up to 8 blocks, so that a step is always cut the same way and the choice is looked
-    up in most steps (a request's rounded length changes once in 256 steps); the last choices are kept.  Few requests: by their
-    lengths as they are where ``_few_width`` stands."""
+    up in most steps (a request's rounded length changes once in 256 steps); the last choices are kept.  Few requests, and those in
+    blocks of eight waves: by their lengths as they are where ``_few_width`` and ``_wide_width`` stand."""
     if nblk.shape[0] <= PIECE_FEW and d == 128:
         key = (nblk.tobytes(), n_kv, PIECE_UNITS, PIECE_MIN_BLOCKS)
         few = _piece_choices.get(key, 0)
@@ -177,6 +201,13 @@ def _piece_choice(nblk, n_kv, d=128):
             _piece_choices[key] = few
         if few is not False:
             return few
+    if piece_waves(nblk.shape[0], n_kv, d) > PIECE_WAVES:
+        key = (nblk.tobytes(), n_kv, PIECE_UNITS, PIECE_MIN_BLOCKS, PIECE_MERGE_US, PIECE_MERGE_MORE_US)
+        if key not in _piece_choices:
+            if len(_piece_choices) >= 64:
+                _piece_choices.pop(next(iter(_piece_choices)))
+            _piece_choices[key] = _wide_width(nblk, n_kv)
+        return _piece_choices[key]
     coarse = nblk >> 3
     key = (coarse.tobytes(), n_kv, d, MAX_PARTS, PIECE_UNITS, PIECE_MIN_BLOCKS, PIECE_START_US, PIECE_MERGE_US, PIECE_ROUND_US)
     if key in _piece_choices:
