@@ -24,8 +24,8 @@
 #include "gemm_rows.h"
 
 // X and W are not declared free of aliases: the waits below count the loads issued before them, and with that promise the compiler may
-// move loads of W across a wait.
-template <int MT, int EPI>
+// move loads of W across a wait.  STAGE: row tiles that an LDS stage has room for.
+template <int MT, int STAGE, int EPI>
 __device__ __forceinline__ void gemm_rows_block(void* C, const bf16_t* X, const bf16_t* W, int M, int N, int K, int col_t, int part, int parts, int tile0,
                                                 GateAct act, bf16_t* stage0, bf16_t* stage1) {
     const int chunks = K / 128, c0 = (int)((long long)chunks * part / parts);
@@ -107,26 +107,12 @@ __device__ __forceinline__ void gemm_rows_block(void* C, const bf16_t* X, const 
         turn();
     }
     if (c < n) products(stage0, 0, false);
+    if (EPI == ROWS_GATED) {
+        // (formed where the sums lie: behind LDS, as the other results, 500 rows, 6144 x 1024 take 11.2 us for 10.6, 640 rows, 12288 x 2048 32.4 for 31.7)
+        const int NG = NT / 2;
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-        const int row = row0 + i * 16 + r;
-        if (EPI == ROWS_PARTS) {
-            float* c_row = (float*)C + ((size_t)part * M + row) * N + 4 * g;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int tile = col_t * 16 + wave * 4 + j;
-                if (tile < NT) *reinterpret_cast<gr_f32x4_t*>(c_row + tile * 16) = acc[j][i];
-            }
-        } else if (EPI == ROWS_STORE) {
-            bf16_t* c_row = (bf16_t*)C + (size_t)row * N + 4 * g;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int tile = col_t * 16 + wave * 4 + j;
-                const uint2 o = {pack_bf16x2(acc[j][i][0], acc[j][i][1]), pack_bf16x2(acc[j][i][2], acc[j][i][3])};
-                if (tile < NT) *reinterpret_cast<uint2*>(c_row + tile * 16) = o;
-            }
-        } else {
-            bf16_t* c_row = (bf16_t*)C + (size_t)row * (N / 2) + 4 * g;
+        for (int i = 0; i < MT; ++i) {
+            bf16_t* c_row = (bf16_t*)C + (size_t)(row0 + i * 16 + r) * (N / 2) + 4 * g;
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int tile = col_t * 8 + wave * 2 + j;
@@ -134,10 +120,17 @@ __device__ __forceinline__ void gemm_rows_block(void* C, const bf16_t* X, const 
 #pragma unroll
                 for (int e = 0; e < 4; ++e) y[e] = gated_value_short(act, acc[j][i][e], acc[j + 2][i][e]);
                 const uint2 o = {pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
-                if (tile < NT / 2) *reinterpret_cast<uint2*>(c_row + tile * 16) = o;
+                if (tile < NG) *reinterpret_cast<uint2*>(c_row + tile * 16) = o;
             }
         }
+        return;
     }
+    // (nothing under way into the stages, and nobody reads them)
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (EPI != ROWS_GATED) gr_block_out<MT, STAGE, EPI>(acc, stage0, C, M, N, row0, col_t, part, act, lane, wave);
 }
 
 // A column of tiles (256 columns, one part) has n_rows blocks, `tall` of them with MT row tiles and the others with one less, as many in
@@ -157,14 +150,14 @@ __global__ __launch_bounds__(256, 2) void gemm_rows_kernel(void* C, const bf16_t
     if (idx >= per || v >= blocks) return;
     const int cp = v / n_rows, i = v % n_rows, col_t = cp % n_cols, part = cp / n_cols;
     if (!DEALT || tall == n_rows) {
-        gemm_rows_block<MT, EPI>(C, X, W, M, N, K, col_t, part, parts, i * MT, act, stage0, stage1);
+        gemm_rows_block<MT, MT, EPI>(C, X, W, M, N, K, col_t, part, parts, i * MT, act, stage0, stage1);
         return;
     }
     const int shift = (int)((unsigned)cp * (unsigned)tall % (unsigned)n_rows), at = i + shift;
     const int before = (at >= n_rows ? tall + min(at - n_rows, tall) : min(at, tall)) - min(shift, tall);      // tall blocks before this one
     const int tile0 = i * (MT - 1) + before;
-    if ((at >= n_rows ? at - n_rows : at) < tall) gemm_rows_block<MT, EPI>(C, X, W, M, N, K, col_t, part, parts, tile0, act, stage0, stage1);
-    else gemm_rows_block<MT - 1, EPI>(C, X, W, M, N, K, col_t, part, parts, tile0, act, stage0, stage1);
+    if ((at >= n_rows ? at - n_rows : at) < tall) gemm_rows_block<MT, MT, EPI>(C, X, W, M, N, K, col_t, part, parts, tile0, act, stage0, stage1);
+    else gemm_rows_block<MT - 1, MT, EPI>(C, X, W, M, N, K, col_t, part, parts, tile0, act, stage0, stage1);
 }
 
 template <int MT>

@@ -107,45 +107,6 @@ __device__ __forceinline__ void gr_tall_turns(gr_f32x4_t (&acc)[4][MT], RES wres
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// The results through a stage, up to three row tiles at a time, in a part that the wave has to itself (a wave's LDS accesses stay in order): the
-// sums go there as they are, and a loop of few instructions reads whole pieces of rows, forms the values and stores them.  Formed
-// where the sums lie, the values of sixteen row tiles are 20 to 40 KB of instructions that every block runs through once, and waits for.
-// PAIRED: the wave's columns 32 on are the up values of the first 32.  form(v, u): a piece's values in v (their up values in u) become
-// results; out, width: the block's first output row and the rows' length; at: this wave's first column.
-template <int MT, bool PAIRED, typename T, typename F>
-__device__ __forceinline__ void gr_tall_results(gr_f32x4_t (&acc)[4][MT], bf16_t* stage, T* out, int width, int at, int lane, int wave, F form) {
-    constexpr int LD = 68, CT = MT * 16 * 128 * 2 / (4 * 16 * LD * 4);       // (16 bytes more than a row: rows begin in other banks)
-    constexpr int VEC = 16 / sizeof(T), PIECES = (PAIRED ? 32 : 64) / VEC, ROWS = 64 / PIECES;
-    static_assert(CT >= 1, "four waves' row tiles fit the stage");
-    float* mine = reinterpret_cast<float*>(stage) + wave * CT * 16 * LD;
-    const int r = lane & 15, g = lane >> 4, col = (lane % PIECES) * VEC;
-#pragma unroll
-    for (int i0 = 0; i0 < MT; i0 += CT) {
-#pragma unroll
-        for (int i = i0; i < i0 + CT && i < MT; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) *reinterpret_cast<gr_f32x4_t*>(mine + ((i - i0) * 16 + r) * LD + j * 16 + 4 * g) = acc[j][i];
-        __builtin_amdgcn_sched_barrier(0);
-        const int rows = 16 * min(CT, MT - i0);
-#pragma unroll 1
-        for (int row = lane / PIECES; row < rows; row += ROWS) {
-            const float* from = mine + row * LD + col;
-            float v[VEC], u[VEC];
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) v[e] = from[e];
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) u[e] = PAIRED ? from[32 + e] : 0.f;
-            form(v, u);
-            if (at + col < width) {
-                T* o = out + (size_t)(i0 * 16 + row) * width + at + col;
-                if constexpr (sizeof(T) == 2) *reinterpret_cast<uint4*>(o) = uint4{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
-                else *reinterpret_cast<gr_f32x4_t*>(o) = gr_f32x4_t{v[0], v[1], v[2], v[3]};
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
 template <int MT, int EPI>
 __global__ __launch_bounds__(256, 1) void gemm_rows_tall_kernel(void* C, const bf16_t* X, const bf16_t* W, int M, int N, int K, int n_rows, int n_cols,
                                                                 int parts, int blocks, GateAct act) {
@@ -180,16 +141,7 @@ __global__ __launch_bounds__(256, 1) void gemm_rows_tall_kernel(void* C, const b
         __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (__attribute__((address_space(3))) void*)(stage + (i * 4 + wave) * 512), 16, x_lane,
                                                  x_at + i * 32 * K + c * 256, 0, 0);
     });
-    if constexpr (EPI == ROWS_PARTS) {
-        gr_tall_results<MT, false>(acc, stage0, (float*)C + ((size_t)part * M + row0) * N, N, col_t * 256 + wave * 64, lane, wave, [](float (&)[4], float (&)[4]) {});
-    } else if constexpr (EPI == ROWS_STORE) {
-        gr_tall_results<MT, false>(acc, stage0, (bf16_t*)C + (size_t)row0 * N, N, col_t * 256 + wave * 64, lane, wave, [](float (&)[8], float (&)[8]) {});
-    } else {
-        gr_tall_results<MT, true>(acc, stage0, (bf16_t*)C + (size_t)row0 * (N / 2), N / 2, col_t * 128 + wave * 32, lane, wave, [&](float (&v)[8], float (&u)[8]) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = gated_value_short(act, v[e], u[e]);
-        });
-    }
+    gr_block_out<MT, MT, EPI>(acc, stage0, C, M, N, row0, col_t, part, act, lane, wave);
 }
 
 template <int MT>

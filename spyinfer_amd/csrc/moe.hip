@@ -13,7 +13,7 @@
 //            Experts without a gate: W = [up rows], C = gelu(up).
 //            Where tables name the experts by token id, the align step of all mixtures is one launch ahead of the layers.
 //   combine: out[t] = scale * sum_k weight[t, k] * Y[row of pair (t, k)].
-#include "common.h"
+#include "gemm_rows.h"
 #include <math.h>
 #include <type_traits>
 
@@ -729,8 +729,8 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_group_kernel(TC* __restrict__
 // the same rows of W loaded from row order, 64 bytes of 16 rows a load, 322 for 268 of the first ones' 251 rows.
 #define MOE_HALVES 128
 template <int MT, bool GATED, typename TC>
-__device__ __forceinline__ void moe_rows_block(TC* C, const bf16_t* A, unsigned a_bytes, const bf16_t* We, const int* src_row, bf16_t* stage0,
-                                               bf16_t* stage1, int N, int K, int by, int t, const int* sorted_pair, const MoeAct& act) {
+__device__ __forceinline__ void moe_rows_block(TC* C, const bf16_t* A, unsigned a_bytes, const bf16_t* We, const int* src_row, const float* row_w,
+                                               bf16_t* stage0, bf16_t* stage1, int N, int K, int by, int t, const MoeAct& act) {
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int NT = N / 16;
     const auto wres = __builtin_amdgcn_make_buffer_rsrc((void*)We, 0, (GATED ? 2 : 1) * N * K * 2, 0x00020000);
@@ -800,20 +800,34 @@ __device__ __forceinline__ void moe_rows_block(TC* C, const bf16_t* A, unsigned 
         turn();
     }
     if (c < n) products(stage0, 0, false);
+    const int64_t row0 = (int64_t)t * MOE_TM;
+    if constexpr (GATED) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-        if (src_row[i * 16 + r] < 0) continue;
-        const size_t row = (size_t)t * MOE_TM + i * 16 + r;
-        const float rw = (GATED && act.pair_w) ? act.pair_w[sorted_pair[row]] : 1.f;
+        for (int i = 0; i < MT; ++i) {
+            if (src_row[i * 16 + r] < 0) continue;
+            const float rw = row_w[i * 16 + r];
 #pragma unroll
-        for (int j = 0; j < (GATED ? 2 : 4); ++j) {
-            const int tile = GATED ? by * 8 + wave * 2 + j : by * 16 + wave * 4 + j;
-            if (tile >= NT) continue;
-            float y[4];
+            for (int j = 0; j < 2; ++j) {
+                const int tile = by * 8 + wave * 2 + j;
+                if (tile >= NT) continue;
+                float y[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) y[e] = GATED ? moe_gated(acc[j][i][e], acc[GATED ? j + 2 : j][i][e], act, rw) : moe_ungated(acc[j][i][e], act);
-            Vec4<TC>::store(C + row * N + tile * 16 + 4 * g, y);
+                for (int e = 0; e < 4; ++e) y[e] = moe_gated(acc[j][i][e], acc[j + 2][i][e], act, rw);
+                Vec4<TC>::store(C + (row0 + i * 16 + r) * N + tile * 16 + 4 * g, y);
+            }
         }
+    } else {
+        // (nothing under way into the stages, and nobody reads them)
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr int VEC = 16 / sizeof(TC);
+        gr_results<MT, 8, false>(acc, stage0, C, N, N, by * 256 + wave * 64, lane, wave, [&](int, float (&v)[VEC], float (&)[VEC]) {
+            if (act.kind != 2) return;
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) v[e] = gelu_f(v[e]);
+        }, [&](int row) { return src_row[row] < 0 ? (int64_t)-1 : row0 + row; });
     }
 }
 
@@ -824,6 +838,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_rows_kernel(TC* C, const bf16
     __shared__ __align__(1024) bf16_t stage0[128 * 128];
     __shared__ __align__(1024) bf16_t stage1[128 * 128];
     __shared__ int src_row[128];
+    __shared__ float row_w[128];
     // (blocks to the dies in runs of the (band, columns, group of the band) order, as above)
     // Up to MOE_HALVES blocks, which leave half of the compute units idle, become two with half of their group's rows (2 experts of 2 x
     // 1536 x 2048 with 128 rows each: 38 us for both products, 64 without; 8 of 2 x 4096 x 2048: 138, 151; with a line at 256 blocks 8
@@ -838,17 +853,20 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_rows_kernel(TC* C, const bf16
     const bf16_t* We = W + (size_t)tile_expert[t] * w_stride;
     if (threadIdx.x < 128) {
         int src = -1;
+        float weight = 1.f;
         if ((int)threadIdx.x < tiles * MOE_TM) {
             const int p = sorted_pair[t * MOE_TM + threadIdx.x];
             src = p < 0 ? -1 : (gather > 0 ? p / gather : t * MOE_TM + (int)threadIdx.x);
+            if (GATED && act.pair_w && p >= 0) weight = act.pair_w[p];
         }
         src_row[threadIdx.x] = src;
+        row_w[threadIdx.x] = weight;
     }
     __syncthreads();
-    if (tiles > 6) moe_rows_block<8, GATED>(C, A, a_bytes, We, src_row, stage0, stage1, N, K, by, t, sorted_pair, act);
-    else if (tiles > 4) moe_rows_block<6, GATED>(C, A, a_bytes, We, src_row, stage0, stage1, N, K, by, t, sorted_pair, act);
-    else if (tiles > 2) moe_rows_block<4, GATED>(C, A, a_bytes, We, src_row, stage0, stage1, N, K, by, t, sorted_pair, act);
-    else moe_rows_block<2, GATED>(C, A, a_bytes, We, src_row, stage0, stage1, N, K, by, t, sorted_pair, act);
+    if (tiles > 6) moe_rows_block<8, GATED>(C, A, a_bytes, We, src_row, row_w, stage0, stage1, N, K, by, t, act);
+    else if (tiles > 4) moe_rows_block<6, GATED>(C, A, a_bytes, We, src_row, row_w, stage0, stage1, N, K, by, t, act);
+    else if (tiles > 2) moe_rows_block<4, GATED>(C, A, a_bytes, We, src_row, row_w, stage0, stage1, N, K, by, t, act);
+    else moe_rows_block<2, GATED>(C, A, a_bytes, We, src_row, row_w, stage0, stage1, N, K, by, t, act);
 }
 
 static int moe_gemm_mfma_launch(void* C, int c_dtype, const void* A, const void* W, const int* tile_expert, const int* sorted_pair,
