@@ -170,7 +170,7 @@ def _wide_width(nblk, n_kv):
     by its blocks of keys, 0.37 us each, an entry in parts takes 1.1 us more, and 0.55 for each eight parts beyond eight (18 steps of 1 to 16 requests of
     130 to 1500 keys, every number of parts: 0.3 us rms, the choice within 0.3 us of the best)."""
     longest = int(nblk.max(initial=1))
-    parts = np.arange(1, (MAX_PARTS if longest > 64 else 8) + 1)       # (up to eight are asked for at once)
+    parts = np.arange(1, (MAX_PARTS if longest > 8 * PIECE_MIN_BLOCKS else 8) + 1)       # (up to eight are asked for at once)
     width = np.unique(np.maximum(np.maximum(1, PIECE_MIN_BLOCKS // 2), -(-longest // parts)))
     each = -(-nblk[None, :] // width[:, None])                     # parts of every entry at every width
     most = each.max(axis=1)
