@@ -27,6 +27,19 @@
 
 typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
 
+// The activations of the stored product, one call for a lane's values: most products have none, and code that is written out at every value
+// is stepped over at every value.
+template <int N>
+__device__ __forceinline__ void gd_activate(f32x4_t (&v)[N], bool xielu, uint32_t raw, bool gelu) {
+    if (__builtin_expect(xielu || gelu, 0)) {
+        const float p = xielu ? softplus_f(__uint_as_float(raw << 16)) : 0.f, q = xielu ? 0.5f + softplus_f(__uint_as_float(raw & 0xffff0000u)) : 0.f;
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[n][i] = xielu ? xielu_f(v[n][i], p, q) : gelu_f(v[n][i]);
+    }
+}
+
 constexpr int GD_WAVES_GATED = 4;     // waves of a block of the gated product with a pair of column tiles per block
 
 // H3: a block has three halves of column tiles (24 columns) instead of one tile: tile t whole and the lower half of
@@ -191,7 +204,7 @@ __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_kernel(
         return;
     }
     if (m >= M) return;
-    const float act_p = act ? softplus_f(__uint_as_float(act_raw << 16)) : 0.f, act_q = act ? 0.5f + softplus_f(__uint_as_float(act_raw & 0xffff0000u)) : 0.f;
+    if constexpr (EPI == EPI_STORE) gd_activate(acc, act, act_raw, gelu);
     if constexpr (H3) {
         // tile0: all columns (lower) or those of its upper half; the next tile: its lower half, or all
 #pragma unroll
@@ -200,7 +213,7 @@ __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_kernel(
             if (!mine) continue;
             TC* out = C + (size_t)m * N + n + 16 * nt;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) out[i] = from_f32<TC>(act ? xielu_f(acc[nt][i], act_p, act_q) : (gelu ? gelu_f(acc[nt][i]) : acc[nt][i]));
+            for (int i = 0; i < 4; ++i) out[i] = from_f32<TC>(acc[nt][i]);
         }
         return;
     }
@@ -210,8 +223,6 @@ __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_kernel(
         float v = acc[0][i];
         // (gated_value_short: 1 row, 6144 x 1024 5.43 -> 5.32 us; from 17 rows on its gain is below half a per cent, and the library stands)
         if (EPI == EPI_GATED) v = sizeof(TC) == 2 ? gated_value_short(gact, v, acc[NT - 1][i]) : gated_value(gact, v, acc[NT - 1][i]);
-        if (act) v = xielu_f(v, act_p, act_q);
-        if (gelu) v = gelu_f(v);
         out[i] = from_f32<TC>(v);
     }
 }
@@ -390,14 +401,16 @@ __global__ __launch_bounds__(GD_WAVES * 64) void gemm_decode_rows_kernel(
                 continue;
             }
             if (m >= M) continue;
-            const float act_p = act ? softplus_f(__uint_as_float(act_raw << 16)) : 0.f, act_q = act ? 0.5f + softplus_f(__uint_as_float(act_raw & 0xffff0000u)) : 0.f;
+            if constexpr (EPI == EPI_STORE) {
+                f32x4_t mine[1] = {acc[ct][mt]};
+                gd_activate(mine, act, act_raw, gelu);
+                acc[ct][mt] = mine[0];
+            }
             TC* out = C + (OT ? operand_order(m, n, MT) : (size_t)m * N + n);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 float v = acc[ct][mt][i];
                 if (EPI == EPI_GATED) v = gated_value(gact, v, acc[CT + ct][mt][i]);
-                if (act) v = xielu_f(v, act_p, act_q);
-                if (gelu) v = gelu_f(v);
                 out[i] = from_f32<TC>(v);
             }
         }
