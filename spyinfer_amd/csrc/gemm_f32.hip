@@ -60,14 +60,48 @@ __device__ __forceinline__ void gf_row_sums(float (&v)[V], int lane) {
 // * up.  Measured, us, with one to four rows of W a wave and its own K / this, 4 rows of A: 2048 x 2048 6.9 / 5.6, 2048 x 6144 15.6 / 10.6 (4.7
 // TB/s), 4096 x 2048 9.7 / 8.2, 12288 x 2048 gated 22.3 / 18.3 (5.5 TB/s), 151936 x 2048 192 / 186; 1 row: 2048 x 6144 10.3 / 9.9, 1024 x 3072
 // 4.1 / 3.95; 8 rows, the narrow kernel / this: 2048 x 6144 23.4 / 13.8, 12288 x 2048 with its activation 45 / 22, 151936 x 2048 356 / 225.
-template <int MR, int NR, int U, int WV, bool GATED>
+//
+// INTO and SCALED fold the norm between two products into them, as gemm_decode.hip does for bfloat16 rows (a norm kernel is 3.7 us between two
+// products of 5 to 20; a step of 4 requests, 28 layers 2048 wide, 2064 / 1952 us, the products each as long as before).  INTO: C is the residual stream, which the result is added to; the block also stores the new values times the next
+// norm's weight and, for every row, the sum of their squares over its columns (fold.squares [blocks][MR]).  SCALED: A is such a product's
+// rows, and the results are scaled by 1 / sqrt(sum / K + eps).  A block reads all of the squares, 8 KB of them beside 4 KB a row of A for a
+// stream of 2048 (A's rows squared and multiplied by the weight as they come by, without all that, cost the registers of a block or two a compute unit:
+// gate/up of 12288 x 2048, 4 rows, 21.2 us for 19.5).
+struct GfFold {
+    const float* squares_in;
+    int n_squares;             // of squares_in: parts times MR
+    float eps;
+    float* rows_out;
+    const float* weight;
+    float* squares_out;
+};
+template <int CTRL> __device__ __forceinline__ float gf_rotated_sum(float v) { return v + gf_moved<CTRL>(v); }
+
+template <int MR, int NR, int U, int WV, bool GATED, bool SCALED, bool INTO>
 __global__ __launch_bounds__(WV * 64) void gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
-                                                              int M, int N, int K, GateAct act) {
+                                                              int M, int N, int K, GateAct act, GfFold fold) {
     constexpr int NC = GATED ? NR / 2 : NR, V = NR * MR;              // columns of the block, its sums
     constexpr int LEFT = V >= 16 ? V / 16 : 1, SHARE = V >= 16 ? 1 : 16 / V;      // sums a lane ends with; lanes with the same one
     __shared__ float red[WV * 4][V];
+    __shared__ float squares[SCALED ? WV * 4 : 1][MR];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int n0 = blockIdx.x * NC;
+    // what the end needs beside the sums is asked for now: the result that this thread forms is (n, m); its share of the squares (of row t % MR)
+    static_assert(!INTO || NC * MR <= 64, "one wave forms the results");
+    const int t = threadIdx.x, n = t / MR, m = t % MR;
+    const bool stores = t < NC * MR && m < M && n0 + n < N;
+    const size_t at = (size_t)m * N + n0 + n;
+    float before = 0.f, next = 0.f;
+    if (INTO && stores) {
+        before = C[at];
+        next = fold.weight[n0 + n];
+    }
+    constexpr int SQ = 8, T = WV * 64;
+    float sq[SCALED ? SQ : 1];
+    if (SCALED) {
+#pragma unroll
+        for (int i = 0; i < SQ; ++i) sq[i] = t + T * i < fold.n_squares ? fold.squares_in[t + T * i] : 0.f;
+    }
     const float* wrow[NR];
     const float* arow[MR];
 #pragma unroll
@@ -140,17 +174,49 @@ __global__ __launch_bounds__(WV * 64) void gemm_f32_few_kernel(const float* __re
 #pragma unroll
         for (int i = 0; i < LEFT; ++i) red[wave * 4 + (lane >> 4)][(lane & 15) / SHARE * LEFT + i] = sums[i];
     }
-    __syncthreads();
-    const int t = threadIdx.x, n = t / MR, m = t % MR;
-    if (t >= NC * MR) return;
-    float y = 0.f, up = 0.f;
+    if (SCALED) {
+        float s = 0.f;
 #pragma unroll
-    for (int p = 0; p < WV * 4; ++p) {
-        y += red[p][t];
-        if (GATED) up += red[p][t + V / 2];
+        for (int i = 0; i < SQ; ++i) s += sq[i];
+        for (int i = t + T * SQ; i < fold.n_squares; i += T) s += fold.squares_in[i];
+        s = gf_rotated_sum<0x128>(s);                          // lanes l and l + 8 of 16 (row_ror), ...
+        if (MR <= 4) s = gf_rotated_sum<0x124>(s);
+        if (MR <= 2) s = gf_rotated_sum<0x122>(s);
+        if (MR <= 1) s = gf_rotated_sum<0x121>(s);
+        if ((lane & 15) < MR) squares[wave * 4 + (lane >> 4)][lane & 15] = s;
+    }
+    __syncthreads();
+    if (INTO ? wave > 0 : !stores) return;
+    float y = 0.f, up = 0.f;
+    if (!INTO || stores) {
+#pragma unroll
+        for (int p = 0; p < WV * 4; ++p) {
+            y += red[p][t];
+            if (GATED) up += red[p][t + V / 2];
+        }
+    }
+    if (SCALED) {
+        float s = 0.f;
+#pragma unroll
+        for (int p = 0; p < WV * 4; ++p) s += squares[p][m];
+        const float scale = 1.0f / sqrtf(s / (float)K + fold.eps);
+        y *= scale;
+        up *= scale;
     }
     if (GATED) y = gated_value(act, y, up);
-    if (m < M && n0 + n < N) C[(size_t)m * N + n0 + n] = y;
+    if (!INTO) {
+        C[at] = y;
+        return;
+    }
+    y += before;                                               // (lanes that store nothing: zero)
+    if (stores) {
+        C[at] = y;
+        fold.rows_out[at] = y * next;
+    }
+    float s = y * y;
+#pragma unroll
+    for (int o = MR; o < NC * MR; o <<= 1) s += __shfl_xor(s, o, 64);
+    if (t < MR) fold.squares_out[(size_t)blockIdx.x * MR + t] = s;
 }
 
 // ---- a few tiles of rows ----------------------------------------------------------------------------------------------------
@@ -479,19 +545,25 @@ static bool gf_few_takes(int M, int N, int K) { return M <= 4 || (M <= 8 && (N <
 // 1024 of W / one): 1024 x 1024 2.76 / 2.79 / 2.74, 1024 x 2048 3.50 / 3.44 / 3.38, 1024 x 3072 4.05 / 4.23 / 3.94, 1024 x 4096 5.15 / 4.81 / 4.64, 2048 x 2048
 // 4.65 / 4.72 / 4.57, 4096 x 1024 4.93 / 4.75 / 4.70; beyond, 2048 x 3072 four 5.78, one 6.16, 4096 x 2048 7.35 / 7.12 / 7.40.  Below 1024 rows of W two
 // chunks a round, where that leaves no rest: 512 x 2048 2.68, one 2.96 (two rows of W 2.78); 256 x 2048 2.34, 2.69 (2.50); 512 x 3072 3.26, 3.14 (3.40).
-template <bool GATED>
-static void gf_few(const float* A, const float* W, float* C, int M, int N, int w_rows, int K, GateAct act, hipStream_t st) {
-#define GF_FEW(MR, NR, U, WV) gemm_f32_few_kernel<MR, NR, U, WV, GATED><<<(N + NR / (GATED ? 2 : 1) - 1) / (NR / (GATED ? 2 : 1)), WV * 64, 0, st>>>(A, W, C, M, N, K, act)
+// With `blocks` given nothing runs, and it becomes the number of blocks.
+template <bool GATED, bool SCALED = false, bool INTO = false>
+static void gf_few(const float* A, const float* W, float* C, int M, int N, int w_rows, int K, GateAct act, hipStream_t st, const GfFold& fold = GfFold{}, int* blocks = nullptr) {
+#define GF_FEW(MR, NR, U, WV)                                                                                                      \
+    {                                                                                                                              \
+        const int grid = (N + NR / (GATED ? 2 : 1) - 1) / (NR / (GATED ? 2 : 1));                                                  \
+        if (blocks) *blocks = grid;                                                                                                \
+        else gemm_f32_few_kernel<MR, NR, U, WV, GATED, SCALED, INTO><<<grid, WV * 64, 0, st>>>(A, W, C, M, N, K, act, fold);       \
+    }
     if constexpr (!GATED) {
         if (M == 1 && (int64_t)w_rows * K <= (4 << 20)) {
-            if (w_rows < 1024 && K % 2048 == 0) GF_FEW(1, 1, 2, 4); else GF_FEW(1, 1, 1, 4);
+            if (w_rows < 1024 && K % 2048 == 0) GF_FEW(1, 1, 2, 4) else GF_FEW(1, 1, 1, 4)
             return;
         }
     }
-    if (M == 1) { if (w_rows <= 1024) GF_FEW(1, 2, 2, 4); else GF_FEW(1, 4, 2, 4); }
-    else if (M == 2) { if (w_rows <= 1024) GF_FEW(2, 2, 2, 4); else GF_FEW(2, 4, 2, 4); }
-    else if (M <= 4) { if (w_rows <= 1024) GF_FEW(4, 4, 1, 8); else if (w_rows < 8192) GF_FEW(4, 4, 1, 4); else GF_FEW(4, 8, 1, 4); }
-    else { if (w_rows <= 1024) GF_FEW(8, 4, 1, 8); else if (w_rows < 4096) GF_FEW(8, 4, 1, 4); else GF_FEW(8, 8, 1, 4); }
+    if (M == 1) { if (w_rows <= 1024) GF_FEW(1, 2, 2, 4) else GF_FEW(1, 4, 2, 4) }
+    else if (M == 2) { if (w_rows <= 1024) GF_FEW(2, 2, 2, 4) else GF_FEW(2, 4, 2, 4) }
+    else if (M <= 4) { if (w_rows <= 1024) GF_FEW(4, 4, 1, 8) else if (w_rows < 8192) GF_FEW(4, 4, 1, 4) else GF_FEW(4, 8, 1, 4) }
+    else { if (w_rows <= 1024) GF_FEW(8, 4, 1, 8) else if (w_rows < 4096) GF_FEW(8, 4, 1, 4) else GF_FEW(8, 8, 1, 4) }
 #undef GF_FEW
 }
 
@@ -575,5 +647,37 @@ extern "C" int spy_gemm_f32_parts(float* C, const float* A, const float* W, int 
     SPY_REQUIRE(blocks < (1 << 28), "spy_gemm_f32_parts: too many blocks");
     gemm_f32_tile_kernel<1><<<(unsigned)((blocks + 7) / 8 * 8), 256, 0, st>>>(A, W, C, M, N, K, tm, tn, parts);
     SPY_CHECK_LAUNCH("spy_gemm_f32_parts");
+    return 0;
+}
+
+// Parts of a row's squares that the product into the stream writes: one a block, [parts][rows rounded up to a power of two]
+extern "C" int spy_gemm_f32_into_parts(int M, int N, int K) {
+    int blocks = 0;
+    if (M > 0 && M <= 8 && N > 0 && K > 0) gf_few<false, false, true>(nullptr, nullptr, nullptr, M, N, N, K, GateAct{1.f, 0.f}, nullptr, GfFold{}, &blocks);
+    return blocks;
+}
+
+// C (the stream, [M, N]) += A . W^T for up to eight rows; rows_out = C weight; squares: see gemm_f32_few_kernel, `parts` of them.
+extern "C" int spy_gemm_f32_into(float* C, const float* A, const float* W, float* rows_out, const float* weight, float* squares, int parts, int M, int N, int K,
+                                 hipStream_t st) {
+    SPY_REQUIRE(M > 0 && M <= 8 && N > 0 && K > 0 && parts == spy_gemm_f32_into_parts(M, N, K), "spy_gemm_f32_into: %d rows, %d parts", M, parts);
+    SPY_REQUIRE(gemm_f32_takes(A, W, C, M, N, K), "spy_gemm_f32_into: operands of %d x %d x %d are not taken", M, N, K);
+    gf_few<false, false, true>(A, W, C, M, N, N, K, GateAct{1.f, 0.f}, st, GfFold{nullptr, 0, 0.f, rows_out, weight, squares});
+    SPY_CHECK_LAUNCH("spy_gemm_f32_into");
+    return 0;
+}
+
+// The products of such rows [M, K], up to eight: C [M, N] = A . W^T scaled by row, or, gated, act(gate) * up of that, W = [gate rows | up rows] of N each.
+extern "C" int spy_gemm_f32_scaled(float* C, const float* A, const float* W, const float* squares, int parts, float eps, int M, int N, int K, int gated, int act_code,
+                                   hipStream_t st) {
+    GateAct act = {1.f, 0.f};
+    SPY_REQUIRE(M > 0 && M <= 8 && N > 0 && K > 0 && parts > 0 && parts <= (1 << 24), "spy_gemm_f32_scaled: %d rows, %d parts", M, parts);
+    SPY_REQUIRE(!gated || gate_act_of(act_code, &act), "spy_gemm_f32_scaled: activation %d", act_code);
+    SPY_REQUIRE(gemm_f32_takes(A, W, C, M, N, K), "spy_gemm_f32_scaled: operands of %d x %d x %d are not taken", M, N, K);
+    const int MR = M <= 2 ? M : M <= 4 ? 4 : 8;
+    const GfFold fold = {squares, parts * MR, eps, nullptr, nullptr, nullptr};
+    if (gated) gf_few<true, true>(A, W, C, M, N, 2 * N, K, act, st, fold);
+    else gf_few<false, true>(A, W, C, M, N, N, K, act, st, fold);
+    SPY_CHECK_LAUNCH("spy_gemm_f32_scaled");
     return 0;
 }

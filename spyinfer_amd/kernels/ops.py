@@ -84,7 +84,8 @@ class _Hip:
                      "spy_moe_align", "spy_moe_gemm", "spy_moe_combine", "spy_moe_tile_rows", "spy_moe_group_ints", "spy_token_shift", "spy_tanh", "spy_time_mix",
                      "spy_norm_pair_mean", "spy_scale_cap", "spy_result_norm", "spy_moe_align_tables", "spy_layer_norm", "spy_layer_norm_residual",
                      "spy_gelu", "spy_norm_rope_store", "spy_map_difference", "spy_rotation_angles", "spy_decay_memory", "spy_group_norm", "spy_gemm_rows",
-                     "spy_add_parts_rmsnorm", "spy_gemm_f32_parts", "spy_gemm_f32_gated"):
+                     "spy_add_parts_rmsnorm", "spy_gemm_f32_parts", "spy_gemm_f32_gated", "spy_gemm_f32_into", "spy_gemm_f32_into_parts",
+                     "spy_gemm_f32_scaled"):
             if not hasattr(self.lib, name):
                 raise KernelError("the kernel library %s lacks %s: it is older than its sources; build it again "
                                   "(spyinfer_amd.kernels.build.build())" % (self.lib._name, name))
@@ -894,7 +895,7 @@ class EntryAddends:
 
 
 class ScaledInput:
-    """The input of a product as 'the RMS norm of the residual stream' with the scale still to come:
+    """The input of a product as 'the RMS norm of the residual stream' with the scale still to come (``ScaledF32``: the same for a few float32 rows):
     ``xw`` = bfloat16(h * w_norm), as [M, K] or as OperandRows, and the parts ``ss_parts [n, MP]`` of every row's sum
     of squares (row r of the stream in column r; their sum over n is sum(h[r]^2); MP = M rounded up to 16).  ``decode_linear`` and
     ``decode_linear_swiglu`` multiply their result by rsqrt(sum / K + eps), which equals the product with the
@@ -903,6 +904,11 @@ class ScaledInput:
 
     def __init__(self, xw, ss_parts: torch.Tensor, eps: float, norm=None):
         self.xw, self.ss_parts, self.eps, self.norm = xw, ss_parts, float(eps), norm
+
+
+class ScaledF32(ScaledInput):
+    """Up to FOLDED_F32_ROWS float32 rows: ``xw`` = h * w_norm [M, K], ``ss_parts [n, M rounded up to a power of two]``."""
+    __slots__ = ()
 
 
 # Two switches that the tests flip, to hold the folded decode steps against the same steps with norm kernels of their own,
@@ -927,6 +933,59 @@ def fused_decode_ok(rows: int, act_dtype, *tiled_weights, max_rows: Optional[int
         return False                 # beyond 64 rows the products are built for hand-over in operand order only
     return all(t is not None and t.dtype == torch.bfloat16 and t.shape[0] % 16 == 0 and t.shape[1] % 128 == 0
                for t in tiled_weights)
+
+
+#: most float32 rows of a step whose norms and sums are folded into its products (csrc/gemm_f32.hip, the kernel of few rows)
+FOLDED_F32_ROWS = 8
+
+
+def folded_f32_ok(rows: int, act_dtype, *weights) -> bool:
+    """True if products of ``rows`` float32 rows with these matrices can run with the norm's scale and the residual sum folded in."""
+    return FUSED_DECODE and act_dtype == torch.float32 and 0 < rows <= FOLDED_F32_ROWS and all(
+        isinstance(w, torch.Tensor) and w.is_cuda and w.dtype == torch.float32 and w.dim() == 2 and w.shape[1] % 4 == 0 and w.is_contiguous()
+        and w.data_ptr() % 16 == 0 for w in weights)
+
+
+@functools.lru_cache(maxsize=256)
+def _f32_into_parts(M: int, N: int, K: int) -> int:
+    return hip().lib.spy_gemm_f32_into_parts(M, N, K)
+
+
+def _scaled_f32(x: ScaledF32, w: torch.Tensor, out: torch.Tensor, gated: bool, act: int) -> None:
+    (M, K), N, rows = x.xw.shape, out.shape[1], x.ss_parts.shape[1]
+    _dev(x.xw, x.ss_parts, w, out)
+    _check(x.xw.dtype == w.dtype == out.dtype == x.ss_parts.dtype == torch.float32 and 0 < M <= FOLDED_F32_ROWS and rows == 1 << (M - 1).bit_length()
+           and out.shape[0] == M and tuple(w.shape) == ((2 if gated else 1) * N, K) and x.xw.is_contiguous() and w.is_contiguous() and out.is_contiguous(),
+           "scaled float32 product: 1..%d rows, their squares and a matrix that fit each other expected", FOLDED_F32_ROWS)
+    hip().call("spy_gemm_f32_scaled", _ptr(out), _ptr(x.xw), _ptr(w), _ptr(x.ss_parts), x.ss_parts.shape[0], ctypes.c_float(x.eps), M, N, K,
+               1 if gated else 0, act, _Hip.stream())
+
+
+def scaled_f32_linear(x: ScaledF32, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """norm(stream) . w^T in float32 -> [M, N], in ``out`` if one is brought."""
+    out = _result(out, x.xw.shape[0], w.shape[0], torch.float32, w.device)
+    _scaled_f32(x, w, out, False, 0)
+    return out
+
+
+def scaled_f32_swiglu(x: ScaledF32, w_gate_up: torch.Tensor, activation: str = "silu") -> torch.Tensor:
+    """act(n . Wgate^T) * (n . Wup^T) in float32, n = norm(stream), ``w_gate_up [2 I, K]`` = [Wgate | Wup] -> [M, I]."""
+    out = torch.empty((x.xw.shape[0], w_gate_up.shape[0] // 2), dtype=torch.float32, device=w_gate_up.device)
+    _scaled_f32(x, w_gate_up, out, True, GATED_ACTIVATIONS[activation])
+    return out
+
+
+def f32_linear_residual(x: torch.Tensor, w: torch.Tensor, resid: torch.Tensor, next_norm_weight: torch.Tensor, eps: float, norm=None) -> ScaledF32:
+    """resid += x . w^T (float32, in place) for at most FOLDED_F32_ROWS rows -> the ScaledF32 of the norm that reads the stream next."""
+    (M, K), N = x.shape, w.shape[0]
+    _dev(x, w, resid, next_norm_weight)
+    _check(x.dtype == w.dtype == resid.dtype == next_norm_weight.dtype == torch.float32 and 0 < M <= FOLDED_F32_ROWS and resid.shape == (M, N)
+           and w.shape[1] == K and next_norm_weight.shape == (N,) and x.is_contiguous() and w.is_contiguous() and resid.is_contiguous()
+           and next_norm_weight.is_contiguous(), "f32_linear_residual: 1..%d float32 rows, a matrix, a stream and a norm weight that fit each other expected", FOLDED_F32_ROWS)
+    ss = torch.empty((_f32_into_parts(M, N, K), 1 << (M - 1).bit_length()), dtype=torch.float32, device=resid.device)
+    xw = torch.empty((M, N), dtype=torch.float32, device=resid.device)
+    hip().call("spy_gemm_f32_into", _ptr(resid), _ptr(x), _ptr(w), _ptr(xw), _ptr(next_norm_weight), _ptr(ss), ss.shape[0], M, N, K, _Hip.stream())
+    return ScaledF32(xw, ss, eps, norm)
 
 
 def folded_products_take(prepared, rows: int) -> bool:

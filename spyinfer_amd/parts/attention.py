@@ -326,13 +326,17 @@ class PagedAttention(Mixer):
         # (beyond 64 rows the products take their inputs in operand order only: the attention must hand its result over so)
         if not self._plain_projections():
             return False
+        if batch.act_dtype == torch.float32:
+            return ops.folded_f32_ok(batch.T, batch.act_dtype, self.w_qkv, self.w_o)
         if batch.T > 64 and not ops.attention_hands_over_operand_rows(batch.act_dtype, self.num_heads, self.head_dim, batch.page_size):
             return False
         return ops.fused_decode_ok(batch.T, batch.act_dtype, self.w_qkv_tiled, self.w_o_tiled, max_rows=self.fold_rows)
 
     def _attend(self, x, batch, cache, store, for_product=False):
         nq, nkv, d = self.num_heads, self.num_kv_heads, self.head_dim
-        if isinstance(x, ops.ScaledInput):
+        if isinstance(x, ops.ScaledF32):
+            qkv = ops.scaled_f32_linear(x, self.w_qkv)
+        elif isinstance(x, ops.ScaledInput):
             qkv = ops.decode_linear(x, self.w_qkv_tiled)
         elif not self._plain_projections():
             qkv = ops.linear_few(x, self.w_qkv, self.w_qkv_tiled)       # (no folded path here: the decode products up to 64 rows)
@@ -402,5 +406,7 @@ class PagedAttention(Mixer):
 
     def forward_into(self, x, batch, cache, store, resid, next_norm):
         weight, eps = next_norm.foldable(batch.act_dtype)
+        if batch.act_dtype == torch.float32:
+            return ops.f32_linear_residual(self._attend(x, batch, cache, store), self.w_o, resid, weight, eps, next_norm)
         return ops.decode_linear_residual(self._attend(x, batch, cache, store, for_product=True), self.w_o_tiled, resid, weight, eps,
                                           next_norm)

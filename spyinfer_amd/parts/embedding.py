@@ -79,6 +79,9 @@ class LMHead(Part):
     def can_fold(self, batch):
         # without the matrix's rows the library's product would have them restored first (more bytes than the product
         # itself reads): the folded product stands as far as it is built
+        if batch.act_dtype == torch.float32:
+            # (5 to 8 rows with a K up to 1024 are the held kernel's, behind a norm kernel)
+            return ops.folded_f32_ok(batch.T, batch.act_dtype, self.weight) and (batch.T <= 4 or self.hidden_size > 1024)
         rows = ops.FUSED_DECODE_MAX_ROWS if isinstance(self.weight, ops.TiledOnly) else self.fold_rows
         return ops.fused_decode_ok(batch.T, batch.act_dtype, self.weight_tiled, max_rows=rows)
 
@@ -99,6 +102,8 @@ class LMHead(Part):
         return logits
 
     def _product(self, normed, out=None):
+        if isinstance(normed, ops.ScaledF32):
+            return ops.scaled_f32_linear(normed, self.weight, out)
         if isinstance(normed, ops.ScaledInput):
             return ops.decode_linear(normed, self.weight_tiled, torch.float32, out)
         if normed.shape[0] <= self.fold_rows:

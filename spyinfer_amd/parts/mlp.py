@@ -51,9 +51,13 @@ class GatedMLP(FeedForward):
         return True
 
     def can_fold(self, batch):
+        if batch.act_dtype == torch.float32:
+            return ops.folded_f32_ok(batch.T, batch.act_dtype, self.w_gate_up, self.w_down)
         return ops.fused_decode_ok(batch.T, batch.act_dtype, self.w_gate_up_tiled, self.w_down_tiled, max_rows=self.fold_rows)
 
     def forward(self, x, batch):
+        if isinstance(x, ops.ScaledF32):
+            return ops.linear(ops.scaled_f32_swiglu(x, self.w_gate_up, self.activation), self.w_down)
         if isinstance(x, ops.ScaledInput):
             return ops.linear(ops.decode_linear_swiglu(x, self.w_gate_up_tiled, activation=self.activation), self.w_down, tiled=self.w_down_tiled)
         return ops.linear_few(ops.linear_swiglu(x, self.w_gate_up, self.w_gate_up_tiled, few_rows=ops.DECODE_ROWS_PLAIN, activation=self.activation),
@@ -68,6 +72,8 @@ class GatedMLP(FeedForward):
 
     def forward_into(self, x, batch, resid, next_norm):
         weight, eps = next_norm.foldable(batch.act_dtype)
+        if isinstance(x, ops.ScaledF32):
+            return ops.f32_linear_residual(ops.scaled_f32_swiglu(x, self.w_gate_up, self.activation), self.w_down, resid, weight, eps, next_norm)
         act = ops.decode_linear_swiglu(x, self.w_gate_up_tiled, for_product=True, activation=self.activation)
         return ops.decode_linear_residual(act, self.w_down_tiled, resid, weight, eps, next_norm)
 

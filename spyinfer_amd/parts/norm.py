@@ -104,7 +104,9 @@ class RMSNorm(Norm):
         return ops.norm_residual(base, y, self.weight, self.eps, out, copy_dtype, mix)
 
     def foldable(self, out_dtype):
-        if self.groups == 1 and not self.scalar and out_dtype == torch.bfloat16 and self.weight is not None and self.weight.dtype == torch.bfloat16:
+        if self.groups != 1 or self.scalar or self.weight is None or self.weight.dtype != out_dtype:
+            return None
+        if out_dtype == torch.bfloat16 or (out_dtype == torch.float32 and self.weight.is_cuda and self.weight.is_contiguous()):
             return self.weight, self.eps
         return None
 

@@ -1,0 +1,124 @@
+"""The float32 products of a few rows with the norm before them, or the sum into the stream behind them, folded in (csrc/gemm_f32.hip)."""
+import pytest
+import torch
+
+from spyinfer_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+EPS = 1e-6
+
+# (rows, columns, K): every number of rows a block is built for and between them; columns beside and at the sizes of a block and at the lines of
+# the rule for blocks; K below a lane's piece of a wave, a rest behind whole chunks of 256, a rest of rounds, and whole rounds
+SIZES = [(1, 1, 4), (1, 1000, 1024), (1, 4097, 2052), (2, 7, 260), (2, 1025, 1024), (3, 1023, 516), (4, 1024, 3072), (4, 2050, 2048), (4, 8193, 256),
+         (5, 30, 1024), (6, 4095, 768), (8, 4096, 1024), (8, 1024, 2048), (8, 9, 5124)]
+
+
+def _bound(terms, K):
+    # every sum has at most K / 256 pieces of 4 in a lane, 8 additions over lanes and 32 over waves, and 8 roundings for norm, scale and sum
+    return (K / 64 + 48) * 2.0 ** -23 * terms
+
+
+def _case(M, N, K, seed, factor=1):
+    gen = torch.Generator().manual_seed(seed)
+    x = torch.randn((M, K), generator=gen) * torch.logspace(-3, 3, M)[:, None]
+    w = torch.randn((factor * N, K), generator=gen) * K ** -0.5
+    g = 1.0 + 0.2 * torch.randn((K,), generator=gen)
+    return x, w, g
+
+
+def _normed(x, g):
+    x = x.double()
+    return x / torch.sqrt((x * x).mean(dim=1, keepdim=True) + EPS) * g.double()
+
+
+def _scaled(x, g, parts):
+    """The input as a product into the stream leaves it, its squares in ``parts`` parts."""
+    rows = 1 << (x.shape[0] - 1).bit_length()
+    ss = torch.zeros((parts, rows))
+    squares = torch.nn.functional.pad(x * x, (0, -x.shape[1] % parts)).reshape(x.shape[0], -1, parts).sum(dim=1)
+    ss[:, :x.shape[0]] = squares.t()
+    return ops.ScaledF32((x * g).to(DEV), ss.to(DEV), EPS)
+
+
+# (one part of the squares, fewer than a block has threads, and more than its threads ask for ahead)
+@pytest.mark.parametrize("parts", [1, 37, 2500])
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_products_of_the_normed_stream(M, N, K, parts):
+    x, w, g = _case(M, N, K, M + N + K)
+    got = ops.scaled_f32_linear(_scaled(x, g, parts), w.to(DEV)).cpu().double()
+    n = _normed(x, g)
+    assert bool(((got - n @ w.double().t()).abs() <= _bound(n.abs() @ w.double().abs().t(), K)).all())
+
+
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_gated_products_of_the_normed_stream(M, N, K, activation):
+    x, w, g = _case(M, N, K, M + N + K + 1, 2)
+    got = ops.scaled_f32_swiglu(_scaled(x, g, 64), w.to(DEV), activation).cpu().double()
+    n = _normed(x, g)
+    z, u = n @ w.double()[:N].t(), n @ w.double()[N:].t()
+    act = torch.nn.functional.silu if activation == "silu" else (lambda t: torch.nn.functional.gelu(t, approximate="tanh"))
+    bz, bu = _bound(n.abs() @ w.double()[:N].abs().t(), K), _bound(n.abs() @ w.double()[N:].abs().t(), K)
+    # (the activations' slope is at most 1.13, their value at most |z|; their own functions are right to a few parts in 2^23)
+    assert bool(((got - act(z) * u).abs() <= 1.13 * bz * (u.abs() + bu) + z.abs() * bu + 16 * 2.0 ** -23 * ((z * u).abs() + u.abs())).all())
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_sums_into_the_stream(M, N, K):
+    x, w, g = _case(M, N, K, M + N + K + 2)
+    h = torch.randn((M, N), generator=torch.Generator().manual_seed(5))
+    stream, after_w = h.to(DEV), 1.0 + 0.3 * torch.randn((N,), generator=torch.Generator().manual_seed(6))
+    after = ops.f32_linear_residual(x.to(DEV), w.to(DEV), stream, after_w.to(DEV), EPS)
+    want = h.double() + x.double() @ w.double().t()
+    assert bool(((stream.cpu().double() - want).abs() <= _bound(x.double().abs() @ w.double().abs().t(), K) + 2.0 ** -23 * want.abs()).all())
+    assert torch.equal(after.xw, stream * after_w.to(DEV))
+    squares = after.ss_parts.cpu().double().sum(dim=0)
+    want = (stream.cpu().double() ** 2).sum(dim=1)
+    assert bool(((squares[:M] - want).abs() <= 8 * 2.0 ** -23 * want).all()) and bool((squares[M:] == 0).all())       # (a part: up to 8 columns)
+
+
+def test_what_is_refused():
+    x, w, g = _case(9, 8, 256, 1)
+    with pytest.raises(ops.KernelError):
+        ops.scaled_f32_linear(_scaled(x, g, 2), w.to(DEV))
+    with pytest.raises(ops.KernelError):
+        ops.scaled_f32_linear(_scaled(x[:4, :128], g[:128], 2), w.to(DEV))
+    with pytest.raises(ops.KernelError):
+        ops.f32_linear_residual(x.to(DEV), w.to(DEV), torch.zeros((9, 8), device=DEV), torch.ones(8, device=DEV), EPS)
+
+
+@pytest.mark.parametrize("requests", [1, 4, 8])
+def test_steps_with_and_without_folded_norms(requests, tmp_path):
+    """Decoding with the norms folded in and by kernels of their own, eagerly and from graphs: the same logits within what float32 sums of
+    another order differ by (2e-5 of a logit's size of a few; 12 roundings a layer of 1e-7 each and their growth over the layers)."""
+    from spyinfer_amd.engine.batch import StepEntry
+    from spyinfer_amd.engine.runner import ModelRunner, load_model
+    from spyinfer_amd.weights import write_random_model
+    from tests.configs import INIT, TINY_D
+    model = load_model(write_random_model(str(tmp_path / "m"), TINY_D, 63, torch.bfloat16, **INIT), "float32", DEV)
+    gen = torch.Generator().manual_seed(3)
+    prompts = [torch.randint(0, 400, (5 + 9 * i,), generator=gen).tolist() for i in range(requests)]
+    real, runs, calls = ops.f32_linear_residual, [], []
+    for folded, eager in ((True, True), (True, False), (False, True)):
+        ops.FUSED_DECODE, n = folded, [0]
+        ops.f32_linear_residual = lambda *a, **k: (n.__setitem__(0, n[0] + 1), real(*a, **k))[1]
+        try:
+            runner = ModelRunner(model, "float32", DEV, 16, 96, requests, enforce_eager=eager, max_model_len=320)
+            caches = [runner.manager.admit(i) for i in range(requests)]
+            for c, p in zip(caches, prompts):
+                runner.manager.reserve(c, len(p))
+            runner.step([StepEntry(c, p, []) for c, p in zip(caches, prompts)])
+            tokens, outs = torch.Generator().manual_seed(4), []
+            for _ in range(6):
+                step = torch.randint(0, 400, (requests,), generator=tokens).tolist()
+                for c in caches:
+                    runner.manager.reserve(c, 1)
+                outs.append(runner.step([StepEntry(c, [t], [0]) for c, t in zip(caches, step)]).cpu().clone())
+            runs.append(outs)
+            calls.append(n[0])
+        finally:
+            ops.FUSED_DECODE, ops.f32_linear_residual = True, real
+    assert calls[0] > 0 and calls[2] == 0
+    for a, b, c in zip(*runs):
+        assert torch.equal(a, b) and torch.allclose(a, c, rtol=2e-5, atol=2e-5), (a - c).abs().max()
