@@ -10,6 +10,13 @@
 //   softmax           running maximum and sum per row; only the maximum is combined over a row's four lanes
 //   O^T += V^T . P^T  lane (dim r, g) loads the values of keys 4 g .. of its dim (values lie [d][key] in a page): product j takes the
 //                     j-th of them and the j-th of its own four weights, so nothing moves between lanes.
+//
+// RAW: steps of single tokens take the step's product [q | k | v] as it is (no kernel of its own for norms, rotation and store: a step of 4 requests, 28 layers of
+// 8 kv heads of 128, 1952 / 1884 us): a lane has
+// of its query row the values 16 i + 4 g .., the rotation's pairs i and i + D / 32 side by side, so the norm costs two lane exchanges and the
+// rotation none.  The entry's new key and value are prepared by the last wave of its last part while that wave's first keys are on their
+// way: the key's score is where the wave's maximum starts, the value its result so far; the wave stores both.  Nobody reads that place.
+//
 // What bounds it: decoding, the round trips of one block after another (pages are looked up two blocks ahead, the next block's keys
 // asked for ahead of this one's softmax, its values ahead of its scores); prompts, L2, from which a tile of 16 rows reads 1 KB a
 // key of 128 dims: 8 kv heads are dealt to the 8 dies, a die's blocks reading one head's keys.
@@ -46,6 +53,48 @@ struct AfArgs {
     long long gate_ld;
 };
 
+// The step's raw product, rows [q | k | v]; null: q comes normed and rotated.  qw, kw: the heads' norm weights (null: no norm); cos_t, sin_t: [max_pos][d / 2]
+// (null: no rotation); store: this call's keys and values go to the cache (else they are there).
+struct AfRaw {
+    const float* qkv;
+    const float* qw;
+    const float* kw;
+    float eps;
+    const float* cos_t;
+    const float* sin_t;
+    int max_pos, store;
+};
+
+// One row's norm and rotation, of which lane (row, g) has the values 16 i + 4 g .. + 3
+template <int DT>
+__device__ __forceinline__ void af_prepare(af_f32x4_t (&x)[DT], bool normed, const af_f32x4_t (&w)[DT], float eps, bool rotated, const af_f32x4_t (&cs)[DT / 2],
+                                           const af_f32x4_t (&sn)[DT / 2]) {
+    if (normed) {
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < DT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ss = fmaf(x[i][e], x[i][e], ss);
+        ss += __shfl_xor(ss, 16, 64);
+        ss += __shfl_xor(ss, 32, 64);
+        const float scale = 1.0f / sqrtf(ss / (float)(16 * DT) + eps);
+#pragma unroll
+        for (int i = 0; i < DT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[i][e] = (scale * x[i][e]) * w[i][e];
+    }
+    if (rotated) {
+#pragma unroll
+        for (int i = 0; i < DT / 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float a = x[i][e], b = x[i + DT / 2][e];
+                x[i][e] = a * cs[i][e] - b * sn[i][e];
+                x[i + DT / 2][e] = a * sn[i][e] + b * cs[i][e];
+            }
+    }
+}
+
 // the result of one row's four neighbouring dims, gated and stored
 __device__ __forceinline__ void af_store(const AfArgs& a, int t, int col, int width, af_f32x4_t o, float l) {
     float4 y;
@@ -59,17 +108,19 @@ __device__ __forceinline__ void af_store(const AfArgs& a, int t, int col, int wi
 }
 
 // (two blocks a compute unit: left to itself the compiler takes 260 registers for heads of 128 and leaves room for one)
-template <int D>
-__global__ __launch_bounds__(AF * 64, 2) void attention_f32_kernel(AfArgs a, int tiles) {
+template <int D, bool RAW>
+__global__ __launch_bounds__(AF * 64, 2) void attention_f32_kernel(AfArgs a, int tiles, AfRaw z) {
     constexpr int DT = D / 16;
     __shared__ float lo_[AF][DT][64][4];
     __shared__ float lm_[AF][16], ll_[AF][16];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r = lane & 15, g = lane >> 4;
     const int hk = blockIdx.x, tile = tiles - 1 - (int)blockIdx.y, sp = blockIdx.z;      // an entry's last tile, which reads most keys, first
-    const int s = a.tile_entry[tile], row0 = a.tile_row0[tile];
+    // (RAW: every entry is one token and has one tile, which the caller has checked: tile t is entry t with token t)
+    const int s = RAW ? tile : a.tile_entry[tile], row0 = RAW ? 0 : a.tile_row0[tile];
     const int G = a.n_q / a.n_kv;
-    const int q0 = a.cu_q[s], nrows = (a.cu_q[s + 1] - q0) * G, p0 = a.pos0[s], kvl = a.kv_len[s];
+    const int q0 = RAW ? s : a.cu_q[s], nrows = (RAW ? 1 : a.cu_q[s + 1] - q0) * G, p0 = a.pos0[s];
+    const int kvl = RAW && z.store ? min(a.kv_len[s], p0) : a.kv_len[s];                  // (the new key, at p0, is not read from the cache)
     const int* bt = a.block_table + (size_t)s * a.max_blocks;
     const int row = row0 + r;
     const bool row_ok = row < nrows;
@@ -78,7 +129,7 @@ __global__ __launch_bounds__(AF * 64, 2) void attention_f32_kernel(AfArgs a, int
     const int first = row_ok ? attention_first_key(p0 + tq, a.window, a.chunk) : 0;
     af_f32x4_t q[DT];
     {
-        const float* qp = a.q + ((size_t)(q0 + tq) * a.n_q + head) * D + 4 * g;
+        const float* qp = (RAW ? z.qkv + ((size_t)(q0 + tq) * (a.n_q + 2 * a.n_kv) + head) * D : a.q + ((size_t)(q0 + tq) * a.n_q + head) * D) + 4 * g;
 #pragma unroll
         for (int i = 0; i < DT; ++i) q[i] = *reinterpret_cast<const af_f32x4_t*>(qp + 16 * i);
     }
@@ -94,6 +145,39 @@ __global__ __launch_bounds__(AF * 64, 2) void attention_f32_kernel(AfArgs a, int
     float m = -INFINITY, l = 0.f;
     if (a.sink && sp == 0 && wave == 0 && row_ok) { m = a.sink[head]; l = g == 0 ? 1.f : 0.f; }
     const float d1 = a.dist ? a.dist[head] : 0.f, d2 = a.dist ? a.dist[a.n_q + head] : 0.f;
+    // RAW: what the preparation needs is asked for ahead of the keys, which need the pages first
+    const bool has_new = RAW && z.store && wave == AF - 1 && sp == a.splits - 1;
+    constexpr int RT = RAW ? DT : 2;
+    af_f32x4_t knew[RT], wq[RT], wk[RT], cs[RT / 2], sn[RT / 2];
+    float vnew[RAW ? D / 64 : 1];                           // the new value's dims lane, lane + 64, for the cache
+    int new_page = -1;
+    if constexpr (RAW) {
+        if (has_new) {
+            const float* kp = z.qkv + ((size_t)q0 * (a.n_q + 2 * a.n_kv) + a.n_q + hk) * D;
+            const float* vp = kp + (size_t)a.n_kv * D;
+            new_page = bt[p0 / a.P];
+#pragma unroll
+            for (int i = 0; i < DT; ++i) {
+                knew[i] = *reinterpret_cast<const af_f32x4_t*>(kp + 16 * i + 4 * g);
+                acc[i] = *reinterpret_cast<const af_f32x4_t*>(vp + 16 * i + 4 * g);
+                if (z.kw) wk[i] = *reinterpret_cast<const af_f32x4_t*>(z.kw + 16 * i + 4 * g);
+            }
+#pragma unroll
+            for (int i = 0; i < D / 64; ++i) vnew[i] = vp[64 * i + lane];
+        }
+        if (z.qw) {
+#pragma unroll
+            for (int i = 0; i < DT; ++i) wq[i] = *reinterpret_cast<const af_f32x4_t*>(z.qw + 16 * i + 4 * g);
+        }
+        if (z.cos_t) {
+            const size_t at = (size_t)max(0, min(p0, z.max_pos - 1)) * (D / 2) + 4 * g;
+#pragma unroll
+            for (int i = 0; i < DT / 2; ++i) {
+                cs[i] = *reinterpret_cast<const af_f32x4_t*>(z.cos_t + at + 16 * i);
+                sn[i] = *reinterpret_cast<const af_f32x4_t*>(z.sin_t + at + 16 * i);
+            }
+        }
+    }
 
     // the page of block b of 16 keys (a page holds whole blocks); beyond the part's end the last block's
     auto page_of = [&](int b) { return bt[(lo + 16 * min(b, b_end - 1)) / a.P]; };
@@ -103,15 +187,44 @@ __global__ __launch_bounds__(AF * 64, 2) void attention_f32_kernel(AfArgs a, int
         return base + (((size_t)pg * a.n_kv + hk) * a.P * D + (size_t)(c0 % a.P) * per_key) + lane_off;
     };
     int b = sp * per + wave;
-    if (b < b_end) {
-        af_f32x4_t k[DT], v[DT];
-        int page = page_of(b), page_n = page_of(b + AF);
+    af_f32x4_t k[DT], v[DT];
+    int page = 0, page_n = 0;
+    {
         auto load_k = [&](int bb, int pg) {
             const float* kp = place(bb, pg, a.kc, D, r * D + 4 * g);
 #pragma unroll
             for (int i = 0; i < DT; ++i) k[i] = *reinterpret_cast<const af_f32x4_t*>(kp + 16 * i);
         };
-        load_k(b, page);
+        if (b < b_end) {
+            page = page_of(b);
+            page_n = page_of(b + AF);
+            load_k(b, page);
+        }
+        if constexpr (RAW) {
+            af_prepare<DT>(q, z.qw != nullptr, wq, z.eps, z.cos_t != nullptr, cs, sn);
+            if (has_new) {
+                af_prepare<DT>(knew, z.kw != nullptr, wk, z.eps, z.cos_t != nullptr, cs, sn);
+                float x = 0.f;
+#pragma unroll
+                for (int i = 0; i < DT; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x = fmaf(q[i][e], knew[i][e], x);
+                x += __shfl_xor(x, 16, 64);
+                x += __shfl_xor(x, 32, 64);
+                m = x * a.scale;
+                l = g == 0 ? 1.f : 0.f;                    // (the four lanes of a row hold partial sums)
+                if (new_page >= 0 && new_page < a.num_pages) {
+                    const int off = p0 % a.P;
+                    if (r == 0) {
+                        float* to = const_cast<float*>(a.kc) + (((size_t)new_page * a.n_kv + hk) * a.P + off) * D + 4 * g;
+#pragma unroll
+                        for (int i = 0; i < DT; ++i) *reinterpret_cast<af_f32x4_t*>(to + 16 * i) = knew[i];
+                    }
+#pragma unroll
+                    for (int i = 0; i < D / 64; ++i) const_cast<float*>(a.vc)[(((size_t)new_page * a.n_kv + hk) * D + 64 * i + lane) * a.P + off] = vnew[i];
+                }
+            }
+        }
         for (; b < b_end; b += AF) {
             const int c0 = lo + 16 * b + 4 * g;                                            // this lane's four keys
             const float* vp = place(b, page, a.vc, 1, r * a.P + 4 * g);
@@ -255,8 +368,9 @@ extern "C" int64_t spy_attention_f32_workspace(int tiles, int n_kv, int d, int s
 extern "C" int spy_attention_f32(float* out, const float* q, const float* kc, const float* vc, int P, int num_pages, const int* cu_q,
                                  const int* pos0, const int* kv_len, const int* block_table, int max_blocks, const int* tile_entry,
                                  const int* tile_row0, int tiles, int S, int T, int n_q, int n_kv, int d, float scale, int window,
-                                 float softcap, int splits, float* ws, const float* dist, const float* sink, int chunk, const float* gate,
-                                 long long gate_ld, hipStream_t st) {
+                                 float softcap, int splits, float* ws, const float* raw_qkv, const float* qw, const float* kw, float eps,
+                                 const float* cos_t, const float* sin_t, int max_pos, int store, const float* dist, const float* sink, int chunk,
+                                 const float* gate, long long gate_ld, hipStream_t st) {
     SPY_REQUIRE(T > 0 && S > 0 && n_q > 0 && n_kv > 0 && P > 0 && num_pages > 0 && max_blocks > 0 && tiles > 0, "spy_attention_f32: empty operand");
     SPY_REQUIRE((d == 64 || d == 128) && P % 16 == 0, "spy_attention_f32: head_dim %d and pages of %d are not for this kernel", d, P);
     SPY_REQUIRE(n_q % n_kv == 0 && tiles <= 65535 && splits >= 1 && splits <= 64, "spy_attention_f32: %d tiles of %d / %d heads in %d parts", tiles, n_q, n_kv, splits);
@@ -268,8 +382,18 @@ extern "C" int spy_attention_f32(float* out, const float* q, const float* kc, co
     const AfArgs a = {out, q, kc, vc, P, num_pages, cu_q, pos0, kv_len, block_table, max_blocks, tile_entry, tile_row0, n_q, n_kv,
                       scale, window, softcap, splits, ws, dist, sink, chunk, gate, gate_ld};
     const dim3 grid(n_kv, tiles, splits);
-    if (d == 64) attention_f32_kernel<64><<<grid, AF * 64, 0, st>>>(a, tiles);
-    else attention_f32_kernel<128><<<grid, AF * 64, 0, st>>>(a, tiles);
+    if (raw_qkv) {
+        const uintptr_t raw = (uintptr_t)raw_qkv | (uintptr_t)qw | (uintptr_t)kw | (uintptr_t)cos_t | (uintptr_t)sin_t;
+        SPY_REQUIRE(raw % 16 == 0 && (qw == nullptr) == (kw == nullptr) && (cos_t == nullptr) == (sin_t == nullptr) && (!cos_t || max_pos > 0),
+                    "spy_attention_f32: operands of the raw product");
+        SPY_REQUIRE(tiles == S && T == S && n_q / n_kv <= 16 && !gate && !dist && !sink && !chunk && softcap == 0.f, "spy_attention_f32: the raw product is for single tokens");
+        const AfRaw z = {raw_qkv, qw, kw, eps, cos_t, sin_t, max_pos, store};
+        if (d == 64) attention_f32_kernel<64, true><<<grid, AF * 64, 0, st>>>(a, tiles, z);
+        else attention_f32_kernel<128, true><<<grid, AF * 64, 0, st>>>(a, tiles, z);
+    } else {
+        if (d == 64) attention_f32_kernel<64, false><<<grid, AF * 64, 0, st>>>(a, tiles, AfRaw{});
+        else attention_f32_kernel<128, false><<<grid, AF * 64, 0, st>>>(a, tiles, AfRaw{});
+    }
     SPY_CHECK_LAUNCH("spy_attention_f32");
     if (splits > 1) {
         if (d == 64) attention_f32_merge_kernel<64><<<dim3(n_kv, tiles), 256, 0, st>>>(a);

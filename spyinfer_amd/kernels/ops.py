@@ -1353,9 +1353,14 @@ class RawQKV:
 
 
 def fused_attention_ok(dtype, meta: AttentionMeta, n_q: int, n_kv: int, d: int, page_size: int, rotary_dim: int, q_norm_w, k_norm_w) -> bool:
-    """True if this step's attention may take the raw product (``RawQKV``): every entry a single token, bfloat16,
-    head_dim 64, 128 or 256 rotated whole or not at all, 16-row tiles built for this group size."""
-    if not mfma_attention_ok(dtype, d, page_size):
+    """True if this step's attention may take the raw product (``RawQKV``): every entry a single token, bfloat16 with
+    head_dim 64, 128 or 256 or float32 with 64 or 128 (and float32 norm weights), rotated whole or not at all, 16-row tiles built for this group size."""
+    if dtype == torch.float32:
+        if not FUSED_DECODE or not f32_attention_ok(dtype, d, page_size) or meta.S > 65535:
+            return False
+        if any(w is not None and (w.dtype != torch.float32 or w.data_ptr() % 16) for w in (q_norm_w, k_norm_w)):
+            return False
+    elif not mfma_attention_ok(dtype, d, page_size):
         return False
     if meta.T != meta.S or meta.max_q_len != 1 or meta.tiles is None or meta.tiles_group != n_q // n_kv or n_q // n_kv > 16:
         return False
@@ -1383,7 +1388,7 @@ def paged_attention(q: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: t
     T, S = meta.T, meta.S
     if raw is not None:
         _dev(raw.qkv, raw.q_norm_w, raw.k_norm_w, raw.cos, raw.sin)
-        _check(raw.qkv.dtype == torch.bfloat16 and raw.qkv.shape == (T, (n_q + 2 * n_kv) * d), "paged_attention: raw qkv must be bfloat16 [T, (n_q + 2 n_kv) d]")
+        _check(raw.qkv.dtype in _CODES and raw.qkv.shape == (T, (n_q + 2 * n_kv) * d), "paged_attention: raw qkv must be [T, (n_q + 2 n_kv) d]")
         rot = 0 if raw.cos is None else d
         _check(fused_attention_ok(raw.qkv.dtype, meta, n_q, n_kv, d, page_size, rot, raw.q_norm_w, raw.k_norm_w),
                "paged_attention: this step cannot take the raw product (ops.fused_attention_ok)")
@@ -1524,13 +1529,18 @@ def paged_attention(q: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: t
         splits = 1
         if reach > 128 or (most > 128 and meta.max_q_len == 1):
             splits = max(1, min(DECODE_SPLIT_TARGET // max(1, n_tiles * n_kv), 2 * key_parts_for(reach)))
+        fused = (_ptr(None), _ptr(None), _ptr(None), ctypes.c_float(0.0), _ptr(None), _ptr(None), ctypes.c_int(0), ctypes.c_int(0))
+        if raw is not None:
+            fused = (_ptr(raw.qkv), _ptr(raw.q_norm_w), _ptr(raw.k_norm_w), ctypes.c_float(raw.eps), _ptr(raw.cos), _ptr(raw.sin),
+                     ctypes.c_int(0 if raw.cos is None else raw.cos.shape[0]), ctypes.c_int(1 if raw.store else 0))
         ws = torch.empty((max(1, hip().lib.spy_attention_f32_workspace(ctypes.c_int(n_tiles), ctypes.c_int(n_kv), ctypes.c_int(d), ctypes.c_int(splits))),),
                          dtype=torch.float32, device=q.device)
         hip().call("spy_attention_f32", _ptr(out), _ptr(q), _ptr(k_cache), _ptr(v_cache), ctypes.c_int(page_size), ctypes.c_int(num_pages),
                    _ptr(meta.cu_q), _ptr(meta.pos0), _ptr(meta.kv_len), _ptr(meta.block_table), ctypes.c_int(meta.max_blocks), _ptr(tile_entry),
                    _ptr(tile_row0), ctypes.c_int(n_tiles), ctypes.c_int(S), ctypes.c_int(T), ctypes.c_int(n_q), ctypes.c_int(n_kv), ctypes.c_int(d),
-                   ctypes.c_float(scale), ctypes.c_int(win), ctypes.c_float(softcap), ctypes.c_int(splits), _ptr(ws), *extras, _Hip.stream())
+                   ctypes.c_float(scale), ctypes.c_int(win), ctypes.c_float(softcap), ctypes.c_int(splits), _ptr(ws), *fused, *extras, _Hip.stream())
         return out
+    _check(raw is None, "paged_attention: the raw product needs caches at 16-byte addresses")
     hip().call("spy_attention_generic", _ptr(out), _ptr(q), _code(q, "q"), _ptr(k_cache), _ptr(v_cache),
                ctypes.c_int(page_size), ctypes.c_int(num_pages), _ptr(meta.kv_len), _ptr(meta.block_table),
                ctypes.c_int(meta.max_blocks), _ptr(meta.token_entry), _ptr(meta.positions), ctypes.c_int(S), ctypes.c_int(T),

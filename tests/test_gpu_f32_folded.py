@@ -122,3 +122,51 @@ def test_steps_with_and_without_folded_norms(requests, tmp_path):
     assert calls[0] > 0 and calls[2] == 0
     for a, b, c in zip(*runs):
         assert torch.equal(a, b) and torch.allclose(a, c, rtol=2e-5, atol=2e-5), (a - c).abs().max()
+
+
+# (query heads, kv heads, head size, page, keys before the step's token by request, window, head norms, rotation): no key before, the edges of blocks of
+# 16 keys and of pages, one part of the keys and many, more parts than blocks, a window that ends with the new key alone
+RAW_CASES = [(16, 8, 128, 16, [0, 1, 15, 16, 17, 500], None, True, True), (8, 1, 128, 32, [31, 32, 33, 1300], None, True, True), (4, 4, 64, 16, [700], None, False, True),
+             (32, 2, 64, 64, [63, 64, 200, 5, 129], None, True, False), (16, 8, 128, 16, [40, 300, 16, 2], 1, True, True), (6, 2, 128, 48, [47, 48, 95, 333], 50, True, True)]
+
+
+@pytest.mark.parametrize("case", range(len(RAW_CASES)))
+def test_attention_taking_the_raw_product(case):
+    """Single tokens: the attention norms, rotates and stores by itself.  The new tokens' places hold NaN before the call; the rest of the cache stays as
+    it was.  Reference: the plain attention in float64 over the normed and rotated rows."""
+    from spyinfer_amd.parts.rotary import RotaryEmbedding
+    from tests.test_gpu_kernels import make_attention_case, plain_paged_attention, plain_qk
+    n_q, n_kv, d, P, cached, window, norm, rotate = RAW_CASES[case]
+    f32, T = torch.float32, len(cached)
+    _q, kc, vc, bt, te, ps, meta = make_attention_case(f32, DEV, n_q, n_kv, d, P, [(a, 1) for a in cached], seed=70 + case, window=window)
+    gen = torch.Generator().manual_seed(case)
+    qkv = torch.randn((T, (n_q + 2 * n_kv) * d), generator=gen)
+    qw, kw = ((1 + 0.2 * torch.randn((d,), generator=gen)) if norm else None for _ in range(2))
+    rope = RotaryEmbedding(d, 23456.0, d)
+    rope.prepare(DEV, 2100)
+    rq, rk, rv = plain_qk(qkv, n_q, n_kv, d, qw, kw, 1e-6, 23456.0, d if rotate else 0, torch.tensor(cached, dtype=torch.int32))
+    kc_ref, vc_ref, new = kc.clone(), vc.clone(), torch.zeros(kc.shape[:3], dtype=torch.bool)
+    kc_dev, vc_dev = kc.clone(), vc.clone()
+    for s, a in enumerate(cached):
+        page = bt[s][a // P]
+        kc_ref[page, :, a % P, :], vc_ref[page, :, :, a % P] = rk[s].to(f32), rv[s].to(f32)
+        kc_dev[page, :, a % P, :] = vc_dev[page, :, :, a % P] = float("nan")
+        new[page, :, a % P] = True
+    scale = d ** -0.5
+    ref = plain_paged_attention(rq.reshape(T, n_q * d).to(f32), kc_ref, vc_ref, P, bt, te, ps, n_q, n_kv, d, scale, window).double()
+    on = lambda t: None if t is None else t.to(DEV)
+    assert ops.fused_attention_ok(f32, meta, n_q, n_kv, d, P, d if rotate else 0, on(qw), on(kw))
+    raw = ops.RawQKV(on(qkv), on(qw), on(kw), 1e-6, rope.cos if rotate else None, rope.sin if rotate else None, True)
+    # A score has d products of sizes up to 10 times 10 over sqrt(d), each rounded, and the rotation's table 2^-24 of an angle of up to 1300: 1e-4 of a
+    # score, and as much of a weight; values are of size one
+    near = lambda a, b: torch.allclose(a.cpu().double(), b.double(), rtol=1e-4, atol=1e-4)
+    k1, v1 = on(kc_dev), on(vc_dev)
+    out = ops.paged_attention(None, k1, v1, P, meta, n_q, n_kv, d, scale, window, raw)
+    assert near(out, ref), (out.cpu().double() - ref).abs().max()
+    same = lambda a, b: torch.equal(torch.nan_to_num(a.cpu(), nan=-77.0), torch.nan_to_num(b, nan=-77.0))
+    assert same(v1, vc_ref) and same(k1.cpu()[~new], kc_ref[~new]) and near(k1.cpu()[new], kc_ref[new])
+    # nothing stored, the new place read from the cache
+    k2, v2 = on(kc_ref), on(vc_ref)
+    raw.store = False
+    out = ops.paged_attention(None, k2, v2, P, meta, n_q, n_kv, d, scale, window, raw)
+    assert near(out, ref) and same(k2, kc_ref) and same(v2, vc_ref)
