@@ -250,8 +250,10 @@ static bool gd_launch_wide_with(const GdArgs& a, int ct, int blocks) {
 
 template <int EPI, bool SCALED, typename TC, int MT, bool XT, bool OT>
 static bool gd_launch_wide(const GdArgs& a) {
-    // (only the combination that a decode step has, a normed input in operand order, to keep the library's build short)
-    if constexpr (EPI == EPI_RESID || !SCALED || !XT) return false;
+    // (only the combinations that steps have, a normed input in operand order, and plain rows for the output head, to keep the library's build short)
+    constexpr bool PLAIN = EPI == EPI_STORE && !SCALED && !XT && sizeof(TC) == 4;
+    constexpr int MIN_CT = PLAIN ? 3 : 1;
+    if constexpr (EPI == EPI_RESID || !(PLAIN || (SCALED && XT))) return false;
     else {
         constexpr int GATES = EPI == EPI_GATED ? 2 : 1;
         // beyond four row tiles (the stored product: beyond two): four waves with a SIMD's registers each
@@ -266,7 +268,7 @@ static bool gd_launch_wide(const GdArgs& a) {
         if constexpr (FOUR) {
             int ct = wide_ct(per, MT, GATES, wide_max_ct<GATES, MT, 4>());
             if (only && ct < 2) ct = 2;
-            return gd_launch_wide_with<EPI, SCALED, TC, MT, XT, OT, 4>(a, ct, blocks);
+            return gd_launch_wide_with<EPI, SCALED, TC, MT, XT, OT, 4, MIN_CT>(a, ct, blocks);
         } else {
             const int ct = wide_ct(per, MT, GATES, wide_max_ct<GATES, MT, 8>());
             // The gated product at three and four row tiles: four waves where their larger groups take a block's run in
@@ -278,7 +280,7 @@ static bool gd_launch_wide(const GdArgs& a) {
                 if (ct4 >= 4 && (per + ct4 - 1) / ct4 < (per + ct - 1) / ct)
                     return gd_launch_wide_with<EPI, SCALED, TC, MT, XT, OT, 4, 4>(a, ct4, blocks);
             }
-            return gd_launch_wide_with<EPI, SCALED, TC, MT, XT, OT, 8>(a, ct, blocks);
+            return gd_launch_wide_with<EPI, SCALED, TC, MT, XT, OT, 8, MIN_CT>(a, ct, blocks);
         }
     }
 }

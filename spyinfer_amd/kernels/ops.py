@@ -448,6 +448,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
     if isinstance(w, TiledOnly):
         _check(x.dtype == torch.bfloat16, "linear: a matrix kept in tiles only takes bfloat16 rows")
         tiled = w.tiled
+    if all_bf16 and tiled is not None and out_dtype == torch.float32 and x.is_contiguous() and (x.data_ptr() | out.data_ptr()) % 16 == 0:
+        tiles = rows_product_logits(M, N, K)
+        if tiles:
+            _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
+            hip().call("spy_gemm_rows", _ptr(out), _ptr(x), _ptr(tiled), M, N, K, tiles, 1, ROWS_PARTS, 0, _Hip.stream())
+            return out
     if all_bf16 and tiled is not None and M <= (TILED_ONLY_DIRECT_ROWS if isinstance(w, TiledOnly) else SKINNY_MAX_ROWS):
         _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
         return decode_linear(x, tiled, out_dtype, out)
@@ -486,7 +492,8 @@ def linear_few(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor] =
     """``linear`` for parts that do not fold norms into their products: up to DECODE_ROWS_PLAIN bfloat16 rows go to the
     decode products (which stream the tiled matrix once and beat the library there: 18.7 against 20.3 us for 6144 x 4096 at
     32 rows, 10.5 against 20.6 for 4096 x 4096), everything else to ``linear``."""
-    if tiled is not None and x.dtype == torch.bfloat16 and x.dim() == 2 and 0 < x.shape[0] <= DECODE_ROWS_PLAIN and x.is_contiguous():
+    if tiled is not None and x.dtype == torch.bfloat16 and x.dim() == 2 and 0 < x.shape[0] <= DECODE_ROWS_PLAIN and x.is_contiguous() \
+            and not (out_dtype == torch.float32 and rows_product_logits(x.shape[0], w.shape[0], w.shape[1])):
         return decode_linear(x, tiled, out_dtype or torch.bfloat16, out)
     return linear(x, w, out_dtype, tiled=tiled, out=out)
 
@@ -495,6 +502,17 @@ def linear_few(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor] =
 ROWS_STORE, ROWS_PARTS, ROWS_GATED = 0, 1, 2
 #: most bytes of a product's parts
 PARTS_MAX_BYTES = 64 << 20
+
+
+def rows_product_logits(M: int, N: int, K: int) -> int:
+    """Row tiles a block of ``spy_gemm_rows`` for logits (float32 results, one part of K) of 64 to 208 rows, or 0 where the decode products or the library's
+    stand.  Bound by the matrix from memory, which a block reads once for up to eight row tiles.  Measured, us, what stood there (the library's; 64 rows:
+    the decode product that walks column tiles, its norm folded in) / this: 151936 x 2560, 64 rows 179 / 157 and 4 for the norm, 80 rows 173 / 159, 128
+    rows 204 / 173, 200 rows 257 / 207; x 4096, 64 rows 267 / 241, 96 rows 276 / 247, 129 rows 301 / 286; x 1024, 200 rows 152 / 102; 65536 x 2048, 128
+    rows 78 / 56; 32768 x 2048, 80 rows 40 / 33, 200 rows 42 / 39, but 64 rows 29 / 32.  Rows beyond 208 and fewer columns were not measured."""
+    if not 64 <= M <= 208 or N < (65536 if M == 64 else 32768) or N % 16 or K % 128 or N * K >= 1 << 30:
+        return 0
+    return min(8, M // 16)
 
 
 def _rows_product_us(M: int, N: int, K: int, tiles: int, parts: int) -> float:

@@ -50,10 +50,9 @@ class TokenEmbedding(Part):
 class LMHead(Part):
     def __init__(self, vocab_size: int, hidden_size: int, tied_to: TokenEmbedding = None, fold_rows: int = 64, suffix: str = ".weight",
                  scale: float = 1.0, softcap: float = 0.0):
-        """``fold_rows``: most rows for which the head runs as a decode product with the final norm folded in.  Above,
-        the library's product after a norm kernel is faster for a large matrix (measured with 151936 x 4096: 235 / 246 /
-        253 / 267 us at 24 / 32 / 48 / 64 rows against the library's 263 / 270 / 258 / 268 and a norm kernel of 6, but
-        281 / 288 / 367 against 274 / 280 / 293 at 80 / 96 / 128).  ``scale``, ``softcap``: the logits are multiplied by
+        """``fold_rows``: most rows for which the head runs as a decode product with the final norm folded in.  Above, and at 64
+        rows of a large matrix, the products of many rows or the library's after a norm kernel are faster (``ops.rows_product_logits``;
+        151936 x 4096 folded 235 / 246 / 253 / 267 us at 24 / 32 / 48 / 64 rows, 281 / 288 / 367 at 80 / 96 / 128).  ``scale``, ``softcap``: the logits are multiplied by
         ``scale`` and then, with a cap > 0, become cap tanh(logit / cap), in float32 and in place."""
         self.scale, self.softcap = float(scale), float(softcap)
         self.vocab_size, self.hidden_size, self.tied_to = vocab_size, hidden_size, tied_to
@@ -82,6 +81,8 @@ class LMHead(Part):
         if batch.act_dtype == torch.float32:
             # (5 to 8 rows with a K up to 1024 are the held kernel's, behind a norm kernel)
             return ops.folded_f32_ok(batch.T, batch.act_dtype, self.weight) and (batch.T <= 4 or self.hidden_size > 1024)
+        if self.weight_tiled is not None and ops.rows_product_logits(batch.T, *self.weight_tiled.shape):
+            return False
         rows = ops.FUSED_DECODE_MAX_ROWS if isinstance(self.weight, ops.TiledOnly) else self.fold_rows
         return ops.fused_decode_ok(batch.T, batch.act_dtype, self.weight_tiled, max_rows=rows)
 
