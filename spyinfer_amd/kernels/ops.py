@@ -458,7 +458,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
         return decode_linear(x, tiled, out_dtype, out)
     if all_bf16 and tiled is not None and out_dtype == torch.bfloat16 and x.is_contiguous():
-        tall = rows_product_tall(M, N, K, ROWS_STORE)
+        tall = rows_product_tall(M, N, K, ROWS_STORE, rows_product_stored(M, N, K))
         tiles = tall[0] if tall else rows_product_stored(M, N, K, _step.replayed and not isinstance(w, TiledOnly))      # (whose library product copies the rows first)
         if tiles and (x.data_ptr() | out.data_ptr()) % 16 == 0:
             _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
@@ -655,18 +655,34 @@ def rows_product_gated(M: int, N: int, K: int, library: bool) -> int:
     return tiles
 
 
-#: what the estimate of a product by tall blocks is made of, microseconds, per kind of result: the launch; a turn of 128 of K, and each row
-#: tile of it; a round's way in and out, and each row tile of that; a turn's row tile in the rounds where every unit has a block (the clock falls)
-_TALL_US = {ROWS_STORE: (4.8, 0.32, 0.110, -2.8, 0.33, 0.039), ROWS_PARTS: (7.5, 0.33, 0.119, 0.6, -0.06, 0.023), ROWS_GATED: (1.3, 0.52, 0.113, -0.95, 0.59, 0.013)}
+#: what the estimate of a product by tall blocks is made of, microseconds, per kind of result: the launch; a round's turn of 128 of K, and each row
+#: tile of it; a round's way in and out, and each row tile of that; a turn's row tile of a unit's even share of all blocks (units that work
+#: together take memory and clock from each other, whether their last round is full or nearly so)
+_TALL_US = {ROWS_STORE: (2.0, 0.397, 0.0757, 0.54, 0.426, 0.0697), ROWS_PARTS: (6.6, 0.168, 0.0868, 4.65, 0.169, 0.0978), ROWS_GATED: (2.9, 0.334, 0.0888, 3.0, 0.339, 0.0626)}
 
 
 def _rows_tall_us(M: int, N: int, K: int, tiles: int, parts: int, kind: int) -> float:
     """Estimated time of ``spy_gemm_rows`` with ``tiles`` row tiles a block, more than eight (one block a compute unit), the norm's pass that sums the
-    parts counted.  Fitted to 2600 launches of 144 to 2048 rows, 1024 to 24576 columns and K of 1024 to 12288: 5 % rms (8 % stored)."""
-    launch, turn, turn_tile, way, way_tile, full = _TALL_US[kind]
+    parts counted.  Fitted to 2000 launches of 150 to 4000 rows, 2048 to 27648 columns and K of 1024 to 12288, each with another matrix, from memory:
+    3 % rms per kind; of the row tiles that fit it takes the fastest within 1 % (parts: 8 % at most where they are taken)."""
+    launch, turn, turn_tile, way, way_tile, even = _TALL_US[kind]
     blocks, turns = -(-M // (16 * tiles)) * -(-N // 256) * parts, -(-(K // 128) // parts)
-    time = launch + -(-blocks // 256) * (turns * (turn + turn_tile * tiles) + way + way_tile * tiles) + full * (blocks // 256) * turns * tiles
-    return time + ((1.34 * parts + 1.09) * M * N / 1e6 if kind == ROWS_PARTS else 0.0)
+    time = launch + -(-blocks // 256) * (turns * (turn + turn_tile * tiles) + way + way_tile * tiles) + even * blocks / 256 * turns * tiles
+    return time + ((0.645 * parts + 0.936) * M * N / 1e6 if kind == ROWS_PARTS else 0.0)
+
+
+def _rows_gated_us(M: int, N: int, K: int, tiles: int):
+    """Estimated time of the gated product by blocks of up to eight row tiles where a compute unit has two and more of them, else None.  A unit's blocks go
+    in pairs, whose turns take 1.2 us and 0.11 for each row tile; the rows are dealt to the blocks as csrc/gemm_rows.hip does.  Fitted to 143
+    launches of 256 to 16384 rows, 6144 to 27648 columns and K of 2048 to 5120, with the numbers of row tiles that ``rows_product_gated`` names: 2.5 % rms."""
+    rows, columns, turns = -(-M // 16), -(-N // 256), K // 128
+    few = -(-rows // tiles)
+    each = -(-few * columns // 256)
+    if each < 2:
+        return None
+    dealt = max(few, min(256 * each // columns, rows // 4))
+    each = -(-dealt * columns // 256)
+    return 4.35 + turns * (1.22 * -(-each // 2) - 0.576 * (each % 2) + 0.113 * each * rows / dealt) + 2.71 * each
 
 
 @functools.lru_cache(maxsize=1024)
@@ -675,18 +691,23 @@ def rows_product_tall(M: int, N: int, K: int, kind: int, other: int = 0):
     or None where blocks of up to eight (``other``: those that the product would get) or the library's product are the better ones.  ``kind``:
     ROWS_STORE, ROWS_PARTS (the next norm sums them) or ROWS_GATED.
 
-    What decides is a unit's share of the work, row tiles times blocks of 256 columns over 256 units: a tall block wants six and more,
-    fewer are spread better by small blocks.  Measured, us, what stood there / this:
-    stored: 4096 x 1024, 1500 rows (5.9 a unit) 16.9 / 16.7, 1700 (6.7) 19.0 / 17.3; 6144 x 2048, 1024 rows (6.0) 28.9 / 28.8, 1200 (7.0) 33.4 / 28.6,
-    2048 45.8 / 41.3; 6144 x 2560, 1356 rows 54.6 / 37.8; 6144 x 4096, 900 rows (5.3) 49.1 / 49.6, 2048 83.6 / 75.6; 15 or 16 row tiles
-    on nearly every unit are the library's own tile: 8192 x 2048, 2048 rows 52.0 / 53.1.
-    gated: 12288 x 2048, 640 rows (7.5) 32.6 / 34.2, 760 (9.0) 43.8 / 36.9, 1356 70.3 / 65.9; 19456 x 2560, 360 rows (6.8) 38.9 / 44.5, 409 (7.7)
-    53.5 / 41.6, 2048 165 / 160; two rounds of nine for 13 a unit: 24576 x 4096, 550 rows 99 / 112, which the estimates tell; against the
-    library and its activation's pass: 24576 x 4096, 300 rows 75.4 / 62.4, 2048 302 / 291; 17408 x 5120, 409 rows 89.2 / 70.0.  K = 1024: 2 % either way.
-    parts, with the norm that sums them, which multiply a unit's share: 2560 x 9728, 640 rows (1.6) 43.4 / 44.4, 900 (2.2) 58.6 / 54.0, 2048 109 /
-    98; 2048 x 6144, 900 rows (1.8) 34.4 / 35.1, 1024 (2.0) 40.8 / 39.0, 2048 66.5 / 61.2; 4096 x 12288, 1356 rows 154 / 121, 2048 193 / 169; 2560 x
-    4096, 1200 rows 44.7 / 41.5, 2048 (5.0) 58.2 / 56.8; 4096 x 4096, 640 rows 44.8 / 37.3, 1500 rows (5.9) 64.6 / 64.5; 2048 x 2048, 1356 rows 31.3 / 28.7,
-    1700 32.2 / 31.7."""
+    Measured, us, what stood there / this, matrices from memory:
+    gated, against small blocks: not where a unit has one of these (12288 x 2048, 640 rows 32.2 / 35.3); with two it is the better one, the more so the
+    fewer their row tiles (19456 x 2560, 385 rows 55.0 / 42.8, 760 rows 69.6 / 66.4; 12288 x 2048, 760 rows 45.0 / 37.3, 1200 rows 54.9 / 50.4);
+    with more it goes by what its rounds leave idle (in a whole step: 12288 x 2048, 1356 rows 69.9 / 67.0, 1500 rows 72.2 / 71.5, 1790 rows 78.4 / 82.4, 2011 rows
+    84.8 / 89.9; 19456 x 2560, 1356 rows 115.5 / 116.3; 24576 x 4096, 700 rows 131 / 118, 1000 rows 153.9 / 154.2, 1356 rows 216 / 205).  The two estimates tell: of
+    143 sizes they leave 3 that gain more than 4 % to the small blocks, and take 2 that lose, by 1 and 1.4 %.
+    gated, against the library and its activation's pass, and stored: a unit's share of the work, row tiles times blocks of 256 columns over 256 units,
+    has to be six and more.  24576 x 4096, 290 rows (7.1) 76.7 / 65.9, 2048 302 / 293; 17408 x 5120, 409 rows 93 / 75; stored: 4096 x 1024, 1900 rows (7.4) 21.0 /
+    20.2; 6144 x 2048, 1356 rows 43.9 / 32.5, 6144 x 4096, 900 rows (5.3) 51.7 / 55.2, 1100 (6.5) 56.5 / 55.3, 2048 81.0 / 76.5; 8192 x 4096, 1356 rows 78.5 / 69.1.
+    Stored small blocks, one a unit, stand (4096 x 2048, 1600 rows 29.2 / 30.7; 8192 x 2048, 800 rows 29.3 / 31.1), and so does the library below 3072
+    columns, where rows make the share (2048 x 2048, 3600 rows 31.2 / 33.8; 2048 x 6144, 4200 rows 94.8 / 99.7; 3072 x 2048, 3000 rows 36.5 / 33.5).
+    15 or 16 row tiles on nearly every unit are the library's own tile (8192 x 2048, 2048 rows 51.9 / 52.7; gated, 16 from four rounds on: 24576 x 4096, 8192 rows
+    1191 / 1237), with K = 1024 14 (4096 x 1024, 3400 rows 28.0 / 29.0).  Stored, a second round pays with a long K and up to a share of 20
+    (6144 x 4096, 3400 rows (20.0) 142 / 134, 4600 rows (27) 168 / 173; 4096 x 4096, 4200 rows 139 / 126; but 4096 x 2048, 4600 rows 71 / 79).
+    parts, with the norm that sums them, which multiply a unit's share: 2560 x 9728, 640 rows (1.6) 44.9 / 45.5, 900 (2.2) 58.4 / 56.3, 2048 117 /
+    106; 2048 x 6144, 900 rows (1.8) 39.8 / 40.0, 1356 52.8 / 47.4, 2048 69.9 / 64.9; 4096 x 12288, 1356 rows 160 / 128, 2048 201 / 187; 2560 x
+    4096, 1200 rows 48.1 / 43.2, 2048 (5.0) 62.2 / 60.2; 4096 x 4096, 640 rows 45.2 / 39.1, 1500 rows (5.9) 65.5 / 65.4."""
     if M < 144 or N % (32 if kind == ROWS_GATED else 16) or K % 128 or N * K >= 1 << 30 or M * K >= 1 << 30:
         return None
     rows, columns, chunks = -(-M // 16), -(-N // 256), K // 128
@@ -694,18 +715,25 @@ def rows_product_tall(M: int, N: int, K: int, kind: int, other: int = 0):
     if kind == ROWS_PARTS:
         if N < 2048 or K < 2048 or share < (2.3 if K < 4096 else 2.0) or (share > 5.4 and K < 8192) or (K < 4096 and M * N > 3e6):
             return None
-    elif K < (2048 if kind == ROWS_GATED else 1024) or share < (7.6 if kind == ROWS_GATED and other else 6.2):
+    elif (kind == ROWS_STORE and (other or N < 3072)) or K < (2048 if kind == ROWS_GATED else 1024) or (not other and share < 6.2):
         return None
     fits = [(t, p) for t in range(9, 17) if 16 * t <= M and -(-rows // -(-rows // t)) == t
-            for p in ((1,) if kind != ROWS_PARTS else range(1, min(6, chunks // 4) + 1))
+            for p in ((1,) if kind != ROWS_PARTS else range(1, min(6, max(2, chunks // 10)) + 1))
             if kind != ROWS_PARTS or (p * M * N * 4 <= PARTS_MAX_BYTES and -(-M // (16 * t)) * columns * p <= 512 and chunks // p <= 64)]
     best = min(fits, key=lambda f: _rows_tall_us(M, N, K, f[0], f[1], kind), default=None)
     if best is None or kind == ROWS_PARTS:
         return best
     blocks = -(-M // (16 * best[0])) * columns
-    if kind == ROWS_GATED and other:
-        return best if _rows_tall_us(M, N, K, best[0], 1, kind) < 0.96 * _rows_product_us(M, N, K, other, 1) else None
-    if share < 0.62 * -(-blocks // 256) * best[0] or (kind == ROWS_STORE and best[0] >= 15 and (blocks - 1) % 256 >= 200):
+    if other:
+        small = _rows_gated_us(M, N, K, other)
+        return best if small is not None and _rows_tall_us(M, N, K, best[0], 1, kind) < 0.965 * small else None
+    rounds, full = -(-blocks // 256), (blocks - 1) % 256 >= 200
+    if share < 0.62 * rounds * best[0]:
+        return None
+    if kind == ROWS_STORE:
+        if (rounds > 1 and (K <= 2048 or share > 20.5)) or (full and best[0] >= (14 if K <= 1024 else 15)):
+            return None
+    elif full and best[0] == 16 and rounds >= 4:
         return None
     return best
 
