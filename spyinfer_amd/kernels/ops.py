@@ -458,8 +458,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
         return decode_linear(x, tiled, out_dtype, out)
     if all_bf16 and tiled is not None and out_dtype == torch.bfloat16 and x.is_contiguous():
-        tall = rows_product_tall(M, N, K, ROWS_STORE, rows_product_stored(M, N, K))
-        tiles = tall[0] if tall else rows_product_stored(M, N, K, _step.replayed and not isinstance(w, TiledOnly))      # (whose library product copies the rows first)
+        tiles = rows_product_stored(M, N, K, _step.replayed and not isinstance(w, TiledOnly))      # (whose library product copies the rows first)
+        tall = None if tiles else rows_product_tall(M, N, K, ROWS_STORE)
+        tiles = tall[0] if tall else tiles
         if tiles and (x.data_ptr() | out.data_ptr()) % 16 == 0:
             _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
             hip().call("spy_gemm_rows", _ptr(out), _ptr(x), _ptr(tiled), M, N, K, tiles, 1, ROWS_STORE, 0, _Hip.stream())
