@@ -32,16 +32,26 @@ PIECE_FEW = 4               # most requests whose lengths are taken as they are 
 PIECE_WAVES = 4             # waves of a block, which take its blocks of keys in turn
 PIECE_TURN_US = 1.75        # a turn (heads of 128: 1 to 4 requests of 130 to 1300 keys)
 PIECE_WIDE_US = 0.37        # a block of 32 keys in a block of eight waves that has its unit to itself
+PIECE_WIDE_KEYS = 1024      # most keys of an entry in blocks of eight waves where more than half of the units have a whole entry's block
 PIECE_PARTS_US = 2.35       # the merge of an entry's parts, and
 PIECE_PART_US = 0.17        # each part of it, up to the eight that the merging block asks for at a time
 
 
-def piece_waves(entries: int, n_kv: int, d: int) -> int:
-    """Waves of a block of the fused attention kernel for keys that are cut here (a launch shape: it follows the entries' number alone): eight where
-    every (entry, kv head) has a compute unit of its own, and as many again are left for five eighths of them to be cut (8 kv heads of 128, four
-    waves / eight, each with its cut, us a layer less: 1 request of 500 keys 1.5, 8 of 1152 1.9, 16 of 1300 2.2, 18 of 100 to 900 1.5; beyond
-    the line 24 and 32 of one length 0.6 to 2.4 less, 32 of 100 to 500 1.3 less, but 24 of 100 to 1300, too few units for their parts, 3.0 more)."""
-    return 8 if d == 128 and 8 * entries * n_kv <= 5 * PIECE_UNITS else PIECE_WAVES
+def keys_read(longest: int, window: int) -> int:
+    """Most keys that a single token reads in a step whose longest request has ``longest``, whole blocks of 32 counted under a window."""
+    return min(longest, window + 31) if window > 0 else longest
+
+
+def piece_waves(entries: int, n_kv: int, d: int, keys: int = 0) -> int:
+    """Waves of a block of the fused attention kernel for keys that are cut here (a launch shape: it follows the entries' number and whether the longest,
+    of ``keys``, has more than PIECE_WIDE_KEYS): eight where every (entry, kv head) has a compute unit of its own, and as many again are left for
+    entries to be cut: up to half of the units, and up to five eighths where keys are few.  8 kv heads of 128, four waves / eight, each with its cut,
+    us: 1 request of 500 keys 12.6 / 10.4, 8 of 1152 16.3 / 14.7, 16 of 1300 24.7 / 22.7, 16 of 130 to 1300 20.1 / 19.7; 20 of 700 21.6 / 19.9, 20 of 70 to 700 19.0 /
+    17.0, but 18 of 1300 27.4 / 30.0, 20 of 2500 44.8 / 51.5, 20 of 250 to 2500 30.4 / 43.9: an entry that
+    gets no second unit is read by one.  20 of 850 and of 1000: 22.8 / 22.1, 23.8 / 25.1; of 100 to 1000, three draws, 19.9 / 19.6."""
+    pairs = entries * n_kv
+    wide = 2 * pairs <= PIECE_UNITS or (8 * pairs <= 5 * PIECE_UNITS and keys <= PIECE_WIDE_KEYS)
+    return 8 if d == 128 and wide else PIECE_WAVES
 
 
 def decode_pieces_capacity(entries: int, n_kv: int) -> int:
@@ -183,7 +193,7 @@ def _wide_width(nblk, n_kv):
 _piece_choices = {}
 
 
-def _piece_choice(nblk, n_kv, d=128):
+def _piece_choice(nblk, n_kv, d=128, waves=None):
     """How a step whose entries have ``nblk`` blocks of keys is cut: None (not at all), (W, even): parts of at most W
     blocks, W being the whole step's blocks over the compute units or over twice as many (and no less than gives the
     longest entry 16 parts, or 32), an entry's parts of one size or W and a rest, or ("fill", True) (``_fill_widths``):
@@ -201,7 +211,7 @@ def _piece_choice(nblk, n_kv, d=128):
             _piece_choices[key] = few
         if few is not False:
             return few
-    if piece_waves(nblk.shape[0], n_kv, d) > PIECE_WAVES:
+    if (waves or piece_waves(nblk.shape[0], n_kv, d)) > PIECE_WAVES:
         key = (nblk.tobytes(), n_kv, PIECE_UNITS, PIECE_MIN_BLOCKS, PIECE_MERGE_US, PIECE_MERGE_MORE_US)
         if key not in _piece_choices:
             if len(_piece_choices) >= 64:
@@ -245,9 +255,9 @@ def _piece_choice(nblk, n_kv, d=128):
     return best[1]
 
 
-def _piece_plan(nblk, n_kv, d=128):
+def _piece_plan(nblk, n_kv, d=128, waves=None):
     """(sizes [S, 16], parts [S]) for entries of ``nblk`` blocks (``_piece_choice``, ``_piece_sizes``)."""
-    choice = _piece_choice(nblk, n_kv, d)
+    choice = _piece_choice(nblk, n_kv, d, waves)
     if choice is not None and choice[0] == "fill":
         widths = _fill_widths(nblk, n_kv)
         choice = None if widths is None else (widths, True)
@@ -256,13 +266,14 @@ def _piece_plan(nblk, n_kv, d=128):
     return _piece_sizes(nblk, *choice)
 
 
-def decode_pieces(kv_len, n_kv: int, window: int = 0, capacity: Optional[int] = None, head_dim: int = 128):
+def decode_pieces(kv_len, n_kv: int, window: int = 0, capacity: Optional[int] = None, head_dim: int = 128, waves: Optional[int] = None):
     """Cuts the keys of a step of single tokens into pieces for the fused attention kernel, one block each, so that the
     compute units have even shares whatever the requests' lengths are (with one number of parts for all entries, a step
     takes as long as its longest request's part).  ``kv_len`` [S]: keys of every entry after this step.  Returns int32
     [capacity, 8] records { entry, kv head, first and end block of 32 keys (counted from the first block the entry's
     window sees), number of the part, parts of the (entry, kv head), workspace slot of its first part, kv_len }, the
-    largest pieces first (see below for the order), entry -1 in the unused ones.
+    largest pieces first (see below for the order), entry -1 in the unused ones.  ``waves``: of the blocks that the kernel is launched with (None:
+    ``piece_waves`` of few keys); any cut is right for either.
 
     Entries are cut into parts of at most W blocks, W being the whole step's blocks over the 256 compute units or over
     twice as many, the parts of an entry even or W and a rest, or the longest entries whole and the others fine
@@ -273,7 +284,7 @@ def decode_pieces(kv_len, n_kv: int, window: int = 0, capacity: Optional[int] = 
     p0 = kv_len - 1
     lo = (np.maximum(0, p0 - window + 1) if window > 0 else np.zeros_like(p0)) & ~31
     nblk = np.maximum(0, (p0 - lo) // 32 + 1)
-    sizes, parts = _piece_plan(nblk, n_kv, head_dim)
+    sizes, parts = _piece_plan(nblk, n_kv, head_dim, waves)
     begin = np.cumsum(sizes, axis=1) - sizes
     ent, part = np.nonzero(sizes > 0)
     count = int(ent.shape[0])

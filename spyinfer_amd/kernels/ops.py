@@ -1559,7 +1559,8 @@ def paged_attention(q: Optional[torch.Tensor], k_cache: torch.Tensor, v_cache: t
                        ctypes.c_int(operand.tiles if operand is not None else 0), _ptr(counters),
                        ctypes.c_int(0 if counters is None else ATTENTION_COUNTERS), _ptr(pieces),
                        ctypes.c_int(0 if pieces is None else pieces.shape[0]), *extras,
-                       ctypes.c_int(key_pieces.piece_waves(S, n_kv, d) if pieces is not None else key_pieces.PIECE_WAVES), _Hip.stream())
+                       ctypes.c_int(key_pieces.piece_waves(S, n_kv, d, key_pieces.keys_read(meta.max_kv_len, win)) if pieces is not None else key_pieces.PIECE_WAVES),
+                       _Hip.stream())
         return operand if operand is not None else out
     if f32_attention_ok(q.dtype, d, page_size) and meta.tiles is not None and meta.tiles_group == group and meta.tiles["big"][2] == 0 \
             and meta.tiles["small"][2] <= 65535 and (q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()) % 16 == 0:

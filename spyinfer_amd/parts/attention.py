@@ -96,10 +96,12 @@ def plan_attention_tiles(batch, group_size: int, big_rows: int = 0, key_parts: b
 def plan_decode_pieces(batch, n_kv: int, window: int, head_dim: int) -> None:
     """Adds to the arrays of a step of single tokens its keys cut into pieces of even size (``key_pieces.decode_pieces``), for
     layers of ``n_kv`` kv heads of ``head_dim`` and this window.  The array's length follows the numbers of entries and
-    heads alone."""
+    heads alone; the waves of a block, a launch shape too, the longest request as well."""
     note = ("decode_pieces", n_kv, window, head_dim)
     if note not in batch.shared:
-        batch.add_array("decode_pieces_%d_%d_%d" % note[1:], key_pieces.decode_pieces(batch.host_array("kv_len"), n_kv, window, head_dim=head_dim))
+        waves = key_pieces.piece_waves(batch.S, n_kv, head_dim, key_pieces.keys_read(batch.max_kv_len, window))
+        batch.add_graph_key("decode_pieces_waves_%d_%d_%d" % note[1:], waves)
+        batch.add_array("decode_pieces_%d_%d_%d" % note[1:], key_pieces.decode_pieces(batch.host_array("kv_len"), n_kv, window, head_dim=head_dim, waves=waves))
         batch.shared[note] = True
 
 

@@ -32,3 +32,35 @@ def test_the_last_part_has_the_new_key():
     live = rec[rec[:, 0] >= 0]
     last = live[live[:, 4] == live[:, 5] - 1]
     assert len(last) == 5 * 8 and (last[:, 3] == (last[:, 7] - 1) // 32 + 1).all()
+
+
+def test_more_entries_than_half_of_the_units_have_such_blocks_for_few_keys_only():
+    """17 to 20 entries of 8 kv heads leave 96 to 120 units of 256 for the parts of 136 to 160 whole entries: with many keys the longest stay whole, and the
+    step waits for them."""
+    waves = key_pieces.piece_waves
+    assert [waves(n, 8, 128, 1024) for n in (16, 17, 20, 21)] == [8, 8, 8, 4] and [waves(n, 8, 128, 1025) for n in (1, 16, 17, 20)] == [8, 8, 4, 4]
+    assert waves(64, 2, 128, 5000) == 8 and waves(65, 2, 128, 5000) == 4
+    assert key_pieces.keys_read(5000, 0) == 5000 and key_pieces.keys_read(5000, 512) == 543 and key_pieces.keys_read(100, 512) == 100
+
+
+@pytest.mark.parametrize("lens,window,waves", [([2500] * 20, 0, 4), ([250 + 118 * i for i in range(20)], 0, 4), ([700] * 20, 0, 8), ([2500] * 20, 512, 8), ([2500] * 16, 0, 8)])
+def test_the_plan_of_a_step_says_which_blocks_it_is_cut_for(lens, window, waves):
+    from spyinfer_amd.parts import attention
+
+    class Batch:
+        S, lens_, max_kv_len, shared, arrays, keys = len(lens), lens, max(lens), {}, {}, {}
+        host_array = staticmethod(lambda name: np.array(lens))
+        add_array = staticmethod(lambda name, values: Batch.arrays.__setitem__(name, values))
+        add_graph_key = staticmethod(lambda name, value: Batch.keys.__setitem__(name, value))
+
+    attention.plan_decode_pieces(Batch, 8, window, 128)
+    assert list(Batch.keys.values()) == [waves]                      # (a launch shape: steps with other blocks are other graphs)
+    rec = next(iter(Batch.arrays.values()))
+    live = rec[rec[:, 0] >= 0]
+    assert (len(live) <= key_pieces.PIECE_UNITS) == (waves == 8)
+    # the unit with most blocks of keys, of all that it has in two rounds, against an even share
+    sizes = live[:, 3] - live[:, 2]
+    load = np.zeros(key_pieces.PIECE_UNITS)
+    load[:min(len(sizes), 256)] += sizes[:256]
+    load[:max(0, len(sizes) - 256)] += sizes[256:]
+    assert waves == 8 or load.max() <= 1.35 * sizes.sum() / key_pieces.PIECE_UNITS
