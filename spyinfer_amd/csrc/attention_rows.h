@@ -338,9 +338,13 @@ __device__ __forceinline__ void attention_mfma_body(
         }
         __builtin_amdgcn_sched_barrier(0);
     }
+    // (Heads of 64: the first block's values behind the preparation of the query and the new key.  Ahead of it they make 132 registers of 118, three waves a
+    // SIMD for four: us, ahead / behind, 8 kv heads, 8 requests of 1152 keys 12.9 / 12.3, 32 of 1000 21.6 / 19.9, 64 of 100 to 1300 27.5 / 25.3, 1 of
+    // 500 9.7 / 9.8.  Larger heads have two waves or one either way.)
+    constexpr bool VALUES_FIRST = !FUSED || DMAX > 64;
     if (b_begin + wave < b_end) {
         AM_LOAD_K(b_begin + wave, kpage)
-        load_v(b_begin + wave, vpage);
+        if (VALUES_FIRST) load_v(b_begin + wave, vpage);
     }
     if constexpr (FUSED) {
         __builtin_amdgcn_sched_barrier(0);
@@ -373,6 +377,7 @@ __device__ __forceinline__ void attention_mfma_body(
             }
         }
     }
+    if (!VALUES_FIRST && b_begin + wave < b_end) load_v(b_begin + wave, vpage);
     // One block of 32 keys.  LAST: the wave's last block, which alone can hold keys beyond the request's, and after which
     // nothing is asked for; the blocks before it have no condition around their loads.
     auto block = [&](const int b, auto last_block) {
