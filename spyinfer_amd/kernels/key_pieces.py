@@ -8,6 +8,7 @@ of records whatever the lengths are.  Plain numpy: nothing here touches the devi
 """
 from __future__ import annotations
 
+import functools
 from typing import Optional
 
 import numpy as np
@@ -26,15 +27,16 @@ PIECE_MERGE_MORE_US = 2.5   # each eight parts beyond sixteen of the entry with 
 PIECE_ROUND_US = 4.0        # each further round of blocks on the units beyond the two that are there from the start
 PIECE_BLOCK_US = 0.45       # a unit's time for a block of 32 keys (16 KB) while it reads alone
 PIECE_SHARED_US = 0.56      # what all units reading at once add to it (the two add as squares)
-# Few requests, whose pieces all have a unit of their own: there a piece's time goes by the turns of its block's waves, four blocks
-# of keys costing what one does, and the last part of an entry, which prepares the new key and stores it, takes a turn more.
+# Few requests in blocks of four waves, whose pieces all have a unit of their own (more kv heads than blocks of eight waves are for): a piece's
+# time goes by the turns of its block's waves, four blocks of keys costing what one does, with a turn more for the entry's last part.
 PIECE_FEW = 4               # most requests whose lengths are taken as they are (a choice in 8 to 32 steps)
 PIECE_WAVES = 4             # waves of a block, which take its blocks of keys in turn
 PIECE_TURN_US = 1.75        # a turn (heads of 128: 1 to 4 requests of 130 to 1300 keys)
-PIECE_WIDE_US = 0.37        # a block of 32 keys in a block of eight waves that has its unit to itself
-PIECE_WIDE_KEYS = 1024      # most keys of an entry in blocks of eight waves where more than half of the units have a whole entry's block
 PIECE_PARTS_US = 2.35       # the merge of an entry's parts, and
 PIECE_PART_US = 0.17        # each part of it, up to the eight that the merging block asks for at a time
+# Blocks of eight waves that have their unit to themselves
+PIECE_WIDE_US = 0.37        # a block of 32 keys
+PIECE_WIDE_KEYS = 1024      # most keys of an entry where more than half of the units have a whole entry's block
 
 
 def keys_read(longest: int, window: int) -> int:
@@ -139,14 +141,12 @@ def _fill_widths(nblk, n_kv):
 
 
 def _few_width(nblk, n_kv):
-    """The width for up to PIECE_FEW requests of heads of 128 whose pieces all find a unit of their own: None (whole), parts of at
+    """The width for up to PIECE_FEW requests of heads of 128 whose pieces, in blocks of four waves, all find a unit of their own: None (whole), parts of at
     most W blocks (W, even, of PIECE_WAVES blocks at least), or False where the entries are too long for that (more than eight parts or
     256 pieces at 8 blocks a part).  Parts of four blocks where every part is one turn then; else the width of 5 to 8 with the fewest
-    turns, and of these the fewest parts.  One request of 8 kv heads, microseconds whole / in parts of 4 / of 8, and of what is
-    taken: 8 blocks 10.8 / 11.7 / -, whole; 13 blocks 13.8 / 13.7 / 13.6, 5: 12.3; 16 blocks 13.9 / 12.2 / 13.5, 4; 22 blocks 18.3 / 12.6 /
-    14.2, 5: 12.5; 25 blocks 19.9 / 14.3 / 12.7, 7 (parts of 4, 5 or 6 leave a block over, so that the last part has three turns); 37
-    blocks 25.4 / 15.8 (nine parts) / 14.4, 7: 12.9; four requests of 37 blocks 26.4 / 16.8 / 15.0, 7: 13.8.  (A rule that took parts of
-    four blocks for any number of requests was up to an eighth slower than parts of eight: 8 requests of 700 keys 16.2 / 15.5.)"""
+    turns, and of these the fewest parts.  (8 kv heads, for which eight waves stand now, microseconds whole / in parts of 4 / of 8, and of what is
+    taken: 8 blocks 10.8 / 11.7 / -, whole; 16 blocks 13.9 / 12.2 / 13.5, 4; 22 blocks 18.3 / 12.6 / 14.2, 5: 12.5; 37 blocks 25.4 / 15.8 (nine
+    parts) / 14.4, 7: 12.9.)"""
     lens = nblk.tolist()
     longest = max(lens)
     if longest > 64:
@@ -175,19 +175,29 @@ def _few_width(nblk, n_kv):
     return None if whole <= best[2] else (best[1], True, PIECE_WAVES)
 
 
+@functools.lru_cache(maxsize=512)
+def _wide_order(longest, least, merge, more, few):
+    """(width, parts) for an entry of ``longest`` blocks in parts of ``least`` blocks and more, by estimated time.  A block's time goes by its blocks of
+    keys, 0.37 us each; an entry in parts takes 1.4 us more (1.1 beside more requests than PIECE_FEW), 0.1 for each of them and 0.55 for each
+    eight beyond eight (1, 2 and 4 requests of 2, 4 and 8 kv heads of 3 to 90 blocks, every number of parts up to 16: the choice 0.2 us behind the
+    best on average; 12 requests of 25 to 250 keys 10.8 in parts, 11.2 whole, one request 9.5, 9.4)."""
+    most = range(1, (MAX_PARTS if longest > 16 * least else 8) + 1)                     # (up to eight are asked for at once)
+    widths = {max(least, -(-longest // p)) for p in most}
+    parts = {w: -(-longest // w) for w in widths}
+    time = lambda w: PIECE_WIDE_US * -(-longest // parts[w]) + (merge * (0.47 if few else 0.37) + more * 0.04 * parts[w] if parts[w] > 1 else 0.0) + more * 0.22 * (-(-parts[w] // 8) - 1)
+    return [(w, parts[w]) for w in sorted(widths, key=lambda w: (time(w), -w))]
+
+
 def _wide_width(nblk, n_kv):
-    """The width for entries whose pieces, in blocks of eight waves, all find a compute unit of their own: None (whole) or (W, even).  A block's time goes
-    by its blocks of keys, 0.37 us each, an entry in parts takes 1.1 us more, and 0.55 for each eight parts beyond eight (18 steps of 1 to 16 requests of
-    130 to 1500 keys, every number of parts: 0.3 us rms, the choice within 0.3 us of the best)."""
-    longest = int(nblk.max(initial=1))
-    parts = np.arange(1, (MAX_PARTS if longest > 8 * PIECE_MIN_BLOCKS else 8) + 1)       # (up to eight are asked for at once)
-    width = np.unique(np.maximum(np.maximum(1, PIECE_MIN_BLOCKS // 2), -(-longest // parts)))
-    each = -(-nblk[None, :] // width[:, None])                     # parts of every entry at every width
-    most = each.max(axis=1)
-    time = PIECE_WIDE_US * (-(-longest // most)) + np.where(most > 1, PIECE_MERGE_US * 0.37, 0.0) + PIECE_MERGE_MORE_US * 0.22 * (-(-most // 8) - 1)
-    time = np.where(each.sum(axis=1) * n_kv <= PIECE_UNITS, time, np.inf)
-    best = int(time.argmin())
-    return None if most[best] <= 1 or not np.isfinite(time[best]) else (int(width[best]), True, PIECE_WAVES)
+    """The width for entries whose pieces, in blocks of eight waves, all find a compute unit of their own: None (whole) or (W, even).  By the longest
+    entry (``_wide_order``), the first width that leaves no unit two pieces."""
+    for width, parts in _wide_order(int(nblk.max(initial=1)), max(1, PIECE_MIN_BLOCKS // 2), PIECE_MERGE_US, PIECE_MERGE_MORE_US,
+                                     nblk.shape[0] <= PIECE_FEW):
+        if parts <= 1:
+            return None
+        if int((-(-nblk // width)).sum()) * n_kv <= PIECE_UNITS:
+            return (width, True, 1)                        # (a rest is a part: the key block that it spares the part before it takes longer than its merge)
+    return None
 
 
 _piece_choices = {}
@@ -199,8 +209,10 @@ def _piece_choice(nblk, n_kv, d=128, waves=None):
     longest entry 16 parts, or 32), an entry's parts of one size or W and a rest, or ("fill", True) (``_fill_widths``):
     whichever has the shortest estimated time.
     Decided from the lengths rounded up to 8 blocks, so that a step is always cut the same way and the choice is looked
-    up in most steps (a request's rounded length changes once in 256 steps); the last choices are kept.  Few requests, and those in
-    blocks of eight waves: by their lengths as they are where ``_few_width`` and ``_wide_width`` stand."""
+    up in most steps (a request's rounded length changes once in 256 steps); the last choices are kept.  Steps in blocks of eight waves go by their
+    lengths as they are (``_wide_width``, a few comparisons), and so do few requests where ``_few_width`` stands."""
+    if (waves or piece_waves(nblk.shape[0], n_kv, d)) > PIECE_WAVES:
+        return _wide_width(nblk, n_kv)
     if nblk.shape[0] <= PIECE_FEW and d == 128:
         key = (nblk.tobytes(), n_kv, PIECE_UNITS, PIECE_MIN_BLOCKS)
         few = _piece_choices.get(key, 0)
@@ -211,13 +223,6 @@ def _piece_choice(nblk, n_kv, d=128, waves=None):
             _piece_choices[key] = few
         if few is not False:
             return few
-    if (waves or piece_waves(nblk.shape[0], n_kv, d)) > PIECE_WAVES:
-        key = (nblk.tobytes(), n_kv, PIECE_UNITS, PIECE_MIN_BLOCKS, PIECE_MERGE_US, PIECE_MERGE_MORE_US)
-        if key not in _piece_choices:
-            if len(_piece_choices) >= 64:
-                _piece_choices.pop(next(iter(_piece_choices)))
-            _piece_choices[key] = _wide_width(nblk, n_kv)
-        return _piece_choices[key]
     coarse = nblk >> 3
     key = (coarse.tobytes(), n_kv, d, MAX_PARTS, PIECE_UNITS, PIECE_MIN_BLOCKS, PIECE_START_US, PIECE_MERGE_US, PIECE_ROUND_US)
     if key in _piece_choices:

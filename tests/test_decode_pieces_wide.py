@@ -64,3 +64,31 @@ def test_the_plan_of_a_step_says_which_blocks_it_is_cut_for(lens, window, waves)
     load[:min(len(sizes), 256)] += sizes[:256]
     load[:max(0, len(sizes) - 256)] += sizes[256:]
     assert waves == 8 or load.max() <= 1.35 * sizes.sum() / key_pieces.PIECE_UNITS
+
+
+@pytest.mark.parametrize("requests", [1, 2, 4])
+@pytest.mark.parametrize("blocks", [29, 37, 45, 55])
+def test_few_requests_are_cut_for_the_blocks_that_they_get(requests, blocks):
+    """Blocks of eight waves, whose time goes by their blocks of keys: eight parts, not as many as blocks of four waves have turns (29 blocks, microseconds:
+    six parts 10.0, eight 9.6; 37: 11.3, 11.0; 45: 11.6, 11.4)."""
+    rec = key_pieces.decode_pieces(np.full(requests, 32 * blocks), 8)
+    live = rec[rec[:, 0] >= 0]
+    assert (live[:, 5] == 8).all()
+
+
+def test_the_cut_of_a_step_follows_its_lengths_without_being_kept():
+    """Nothing is kept by all of a step's lengths: with uneven ones these are new in almost every step."""
+    rng = np.random.default_rng(4)
+    lens = rng.integers(50, 1300, 16)
+    key_pieces._piece_choices.clear()
+    for step in range(64):
+        key_pieces.decode_pieces(lens + step, 8)
+    assert not key_pieces._piece_choices
+    # the first width, by the longest entry's estimated time, that gives every piece a unit: as looking at every width finds it
+    for _ in range(200):
+        n_kv = int(rng.integers(1, 9))
+        nblk = rng.integers(1, 200, int(rng.integers(1, 160 // n_kv + 1)))
+        choice = key_pieces._wide_width(nblk, n_kv)
+        order = key_pieces._wide_order(int(nblk.max()), 4, key_pieces.PIECE_MERGE_US, key_pieces.PIECE_MERGE_MORE_US, nblk.shape[0] <= key_pieces.PIECE_FEW)
+        fits = [w for w, _ in order if int((-(-nblk // w)).sum()) * n_kv <= key_pieces.PIECE_UNITS]
+        assert (fits[0] if -(-int(nblk.max()) // fits[0]) > 1 else None) == (choice and choice[0])
