@@ -64,9 +64,11 @@ __device__ __forceinline__ void gf_row_sums(float (&v)[V], int lane) {
 // INTO and SCALED fold the norm between two products into them, as gemm_decode.hip does for bfloat16 rows (a norm kernel is 3.7 us between two
 // products of 5 to 20; a step of 4 requests, 28 layers 2048 wide, 2064 / 1952 us, the products each as long as before).  INTO: C is the residual stream, which the result is added to; the block also stores the new values times the next
 // norm's weight and, for every row, the sum of their squares over its columns (fold.squares [blocks][MR]).  SCALED: A is such a product's
-// rows, and the results are scaled by 1 / sqrt(sum / K + eps).  A block reads all of the squares, 8 KB of them beside 4 KB a row of A for a
-// stream of 2048 (A's rows squared and multiplied by the weight as they come by, without all that, cost the registers of a block or two a compute unit:
-// gate/up of 12288 x 2048, 4 rows, 21.2 us for 19.5).
+// rows, and the results are scaled by 1 / sqrt(sum / K + eps).  A block reads all of the squares, one for each row (rounded up to 1, 2,
+// 4 or 8) of every block of the product that wrote them: for a stream of 2048, 8 KB behind a product of 2048 x 2048 with one row of A, else 2 KB a row, beside
+// the 8 KB of a row of A.  What its threads ask for at their start, 2048 squares, is there by the end; beyond, the block waits: the line of
+// folded_f32_pays in kernels/ops.py.  (A's rows squared and multiplied by the weight as they come by, without all that, cost the registers of a block or two a
+// compute unit: gate/up of 12288 x 2048, 4 rows, 21.2 us for 19.5.)
 struct GfFold {
     const float* squares_in;
     int n_squares;             // of squares_in: parts times MR

@@ -986,6 +986,10 @@ def fused_decode_ok(rows: int, act_dtype, *tiled_weights, max_rows: Optional[int
 FOLDED_F32_ROWS = 8
 
 
+#: most squares (parts of a row's sum, times the rows) that a block of the scaled float32 products reads: as many as its threads ask for at their start
+FOLDED_F32_SQUARES = 2048
+
+
 def folded_f32_ok(rows: int, act_dtype, *weights) -> bool:
     """True if products of ``rows`` float32 rows with these matrices can run with the norm's scale and the residual sum folded in."""
     return FUSED_DECODE and act_dtype == torch.float32 and 0 < rows <= FOLDED_F32_ROWS and all(
@@ -996,6 +1000,16 @@ def folded_f32_ok(rows: int, act_dtype, *weights) -> bool:
 @functools.lru_cache(maxsize=256)
 def _f32_into_parts(M: int, N: int, K: int) -> int:
     return hip().lib.spy_gemm_f32_into_parts(M, N, K)
+
+
+def folded_f32_pays(rows: int, w_in: torch.Tensor, w_out: torch.Tensor) -> bool:
+    """Whether a sublayer of ``rows`` float32 rows is faster with its norm folded into its first product and its sum into the stream into its last.
+    Every block of a scaled product reads all squares of the stream's rows, which the last product writes in one part for each of its blocks: beyond
+    FOLDED_F32_SQUARES it waits for a second way to them at its end.  Measured, us a layer's four products and two norms (2.6 to 3.3 each), norms in
+    kernels of their own / folded: 512 wide, 1 row (512 squares) 17.2 / 13.9, 8 rows (1024) 21.3 / 18.2; 1024 wide, 1 row 24.5 / 22.5, 2 rows 25.6 / 22.3, 8 rows
+    (2048) 33.0 / 29.2; 2048 wide, 4 rows (2048) 50.1 / 46.3, 5 rows (4096) 58.0 / 57.4, 8 rows 59.3 / 59.9; 2560 wide, 2 rows (1280) 80.8 / 78.8, 4 rows (2560) 86.3 /
+    86.4, 5 rows 104.5 / 110.5; 4096 wide, 2 rows (2048) 133.6 / 129.5, 3 rows (4096) 141.5 / 144.4, 8 rows 155.7 / 166.1."""
+    return folded_f32_ok(rows, torch.float32, w_in, w_out) and _f32_into_parts(rows, *w_out.shape) << (rows - 1).bit_length() <= FOLDED_F32_SQUARES
 
 
 def _scaled_f32(x: ScaledF32, w: torch.Tensor, out: torch.Tensor, gated: bool, act: int) -> None:

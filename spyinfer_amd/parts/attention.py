@@ -329,7 +329,7 @@ class PagedAttention(Mixer):
         if not self._plain_projections():
             return False
         if batch.act_dtype == torch.float32:
-            return ops.folded_f32_ok(batch.T, batch.act_dtype, self.w_qkv, self.w_o)
+            return ops.folded_f32_pays(batch.T, self.w_qkv, self.w_o)
         if batch.T > 64 and not ops.attention_hands_over_operand_rows(batch.act_dtype, self.num_heads, self.head_dim, batch.page_size):
             return False
         return ops.fused_decode_ok(batch.T, batch.act_dtype, self.w_qkv_tiled, self.w_o_tiled, max_rows=self.fold_rows)

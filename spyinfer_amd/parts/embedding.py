@@ -79,8 +79,11 @@ class LMHead(Part):
         # without the matrix's rows the library's product would have them restored first (more bytes than the product
         # itself reads): the folded product stands as far as it is built
         if batch.act_dtype == torch.float32:
-            # (5 to 8 rows with a K up to 1024 are the held kernel's, behind a norm kernel)
-            return ops.folded_f32_ok(batch.T, batch.act_dtype, self.weight) and (batch.T <= 4 or self.hidden_size > 1024)
+            # A block of the head has little of the matrix beside the squares that all blocks read (``ops.folded_f32_pays``), and one norm is all that is
+            # saved, 3 us.  151936 x 1024, without that norm / folded: 1 row 91 / 128, 4 rows 94 / 109, 8 rows 123 / 167; x 2048: 1 row 182 / 183, 2
+            # rows 185 / 192 (a step 656 / 660), 4 rows 188 / 189 (682 / 678), 5 rows 213 / 275; x 2560: 1 row 227 / 225, 2 rows 231 / 239, 4 rows 229 / 242
+            few = batch.T in (1, 3, 4) and self.hidden_size << (batch.T - 1).bit_length() <= 4 * ops.FOLDED_F32_SQUARES
+            return few and self.hidden_size >= 2048 and ops.folded_f32_ok(batch.T, batch.act_dtype, self.weight)
         if self.weight_tiled is not None and ops.rows_product_logits(batch.T, *self.weight_tiled.shape):
             return False
         rows = ops.FUSED_DECODE_MAX_ROWS if isinstance(self.weight, ops.TiledOnly) else self.fold_rows

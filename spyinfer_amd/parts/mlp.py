@@ -52,7 +52,7 @@ class GatedMLP(FeedForward):
 
     def can_fold(self, batch):
         if batch.act_dtype == torch.float32:
-            return ops.folded_f32_ok(batch.T, batch.act_dtype, self.w_gate_up, self.w_down)
+            return ops.folded_f32_pays(batch.T, self.w_gate_up, self.w_down)
         return ops.fused_decode_ok(batch.T, batch.act_dtype, self.w_gate_up_tiled, self.w_down_tiled, max_rows=self.fold_rows)
 
     def forward(self, x, batch):

@@ -170,3 +170,22 @@ def test_attention_taking_the_raw_product(case):
     raw.store = False
     out = ops.paged_attention(None, k2, v2, P, meta, n_q, n_kv, d, scale, window, raw)
     assert near(out, ref) and same(k2, kc_ref) and same(v2, vc_ref)
+
+
+@pytest.mark.parametrize("hidden,inner,rows", [(512, 1536, [1, 2, 3, 4, 5, 8]), (1024, 3072, [1, 2, 3, 4, 5, 8]), (2048, 6144, [1, 2, 3, 4]), (2560, 9728, [1, 2]), (4096, 12288, [1, 2])])
+def test_which_sublayers_fold(hidden, inner, rows):
+    """As many squares as a block's threads ask for at their start, and the head's blocks, which have little else, only with a wide matrix and few rows."""
+    from spyinfer_amd.parts.embedding import LMHead
+    w_in, w_out = torch.zeros((2 * inner, hidden), device=DEV), torch.zeros((hidden, inner), device=DEV)
+    assert [m for m in range(1, 10) if m != 6 and m != 7 and ops.folded_f32_pays(m, w_in, w_out)] == rows
+    head = LMHead(4096, hidden)
+    head.weight, head.weight_tiled = w_in, None
+
+    class Batch:
+        act_dtype = torch.float32
+
+    fold = []
+    for Batch.T in range(1, 10):
+        if head.can_fold(Batch):
+            fold.append(Batch.T)
+    assert fold == {512: [], 1024: [], 2048: [1, 3, 4], 2560: [1], 4096: [1]}[hidden]
