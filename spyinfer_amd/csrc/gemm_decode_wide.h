@@ -289,7 +289,8 @@ static bool gd_launch_wide(const GdArgs& a) {
 // 17 rows on for matrices with two column tiles per compute unit and more, beyond 64 rows the gated product of any
 // width; and the stored product (the output head) from 9 rows on: with a column tile per block its blocks pull as many
 // bytes of X through L2 as of W at 16 rows (251 us; walking six tiles at a time 222; up to 8 rows the kernel with a tile
-// per block stays, 187-194 against 206-211 us).
+// per block stays, 187-194 against 206-211 us).  Plain rows with float32 results (the output head behind a norm kernel) walk too, from 9 to 64 of them and
+// where a group has three column tiles or more (gd_wide_try, with what was measured).
 template <int EPI, typename TC, bool OT>
 static bool wide_rows(const GdArgs& a) {
     if (EPI == EPI_STORE && a.M >= GD_WIDE_MIN_ROWS && a.M <= 16) return gd_launch_wide<EPI, true, TC, 1, true, OT>(a);
