@@ -822,6 +822,9 @@ __device__ __forceinline__ void moe_rows_block(TC* C, const bf16_t* A, unsigned 
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
+        // (bfloat16 results of experts without a gate, eight values of the exact gelu a turn: 28 bytes of scratch, on the way out only.  Four a turn have none and
+        // take as long or 2 % longer: both products of 32 experts of 768 x 1024, 50 rows each 51.4 / 52.7 us, 1536 x 2048, 250 rows 195 / 196, 3072 x
+        // 4096, 125 rows 451 / 444; formed where the sums lie, without LDS 54.5, 203 and 450.)
         constexpr int VEC = 16 / sizeof(TC);
         gr_results<MT, 8, false>(acc, stage0, C, N, N, by * 256 + wave * 64, lane, wave, [&](int, float (&v)[VEC], float (&)[VEC]) {
             if (act.kind != 2) return;
