@@ -1413,10 +1413,13 @@ class RawQKV:
 
 
 
-def fused_attention_ok(dtype, meta: AttentionMeta, n_q: int, n_kv: int, d: int, page_size: int, rotary_dim: int, q_norm_w, k_norm_w) -> bool:
+def fused_attention_ok(dtype, meta: AttentionMeta, n_q: int, n_kv: int, d: int, page_size: int, rotary_dim: int, q_norm_w, k_norm_w, operands=()) -> bool:
     """True if this step's attention may take the raw product (``RawQKV``): every entry a single token, bfloat16 with
-    head_dim 64, 128 or 256 or float32 with 64 or 128 (and float32 norm weights), rotated whole or not at all, 16-row tiles built for this group size."""
+    head_dim 64, 128 or 256 or float32 with 64 or 128 (and float32 norm weights), rotated whole or not at all, 16-row tiles built for this group size.
+    ``operands``: what else the kernel would read (caches, rotation table); float32 ones that do not lie at 16 bytes go by kernels that take any."""
     if dtype == torch.float32:
+        if any(t is not None and t.data_ptr() % 16 for t in operands):
+            return False
         if not FUSED_DECODE or not f32_attention_ok(dtype, d, page_size) or meta.S > 65535:
             return False
         if any(w is not None and (w.dtype != torch.float32 or w.data_ptr() % 16) for w in (q_norm_w, k_norm_w)):

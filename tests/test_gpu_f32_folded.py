@@ -189,3 +189,34 @@ def test_which_sublayers_fold(hidden, inner, rows):
         if head.can_fold(Batch):
             fold.append(Batch.T)
     assert fold == {512: [], 1024: [], 2048: [1, 3, 4], 2560: [1], 4096: [1]}[hidden]
+
+
+def test_caches_off_16_bytes_take_the_plain_kernels(tmp_path):
+    """Decoding over caches that lie at 4 bytes: the same logits as over aligned ones, within rounding of float32 sums in another order."""
+    from spyinfer_amd.engine.batch import StepEntry
+    from spyinfer_amd.engine.runner import ModelRunner, load_model
+    from spyinfer_amd.weights import write_random_model
+    from tests.configs import INIT, TINY_D
+    model = load_model(write_random_model(str(tmp_path / "m"), TINY_D, 64, torch.bfloat16, **INIT), "float32", DEV)
+    prompts = [[5, 9, 200, 31], list(range(40, 77))]
+    outs = []
+    for shifted in (False, True):
+        runner = ModelRunner(model, "float32", DEV, 16, 32, 2, enforce_eager=True, max_model_len=320)
+        if shifted:
+            for layer in runner.storage.layers.values():
+                for name in ("k", "v"):
+                    t = getattr(layer, name)
+                    moved = torch.zeros(t.numel() + 1, device=DEV)[1:].view(t.shape)
+                    assert moved.data_ptr() % 16 == 4
+                    setattr(layer, name, moved)
+        caches = [runner.manager.admit(i) for i in range(2)]
+        for c, p in zip(caches, prompts):
+            runner.manager.reserve(c, len(p))
+        runner.step([StepEntry(c, p, []) for c, p in zip(caches, prompts)])
+        got = []
+        for t in (3, 250, 17):
+            for c in caches:
+                runner.manager.reserve(c, 1)
+            got.append(runner.step([StepEntry(c, [t + i], [0]) for i, c in enumerate(caches)]).cpu().clone())
+        outs.append(torch.stack(got))
+    assert torch.allclose(outs[0], outs[1], rtol=2e-5, atol=2e-5), (outs[0] - outs[1]).abs().max()
