@@ -510,10 +510,17 @@ def rows_product_logits(M: int, N: int, K: int) -> int:
     stand.  Bound by the matrix from memory, which a block reads once for up to eight row tiles.  Measured, us, what stood there (the library's; 64 rows:
     the decode product that walks column tiles, its norm folded in) / this: 151936 x 2560, 64 rows 179 / 157 and 4 for the norm, 80 rows 173 / 159, 128
     rows 204 / 173, 200 rows 257 / 207; x 4096, 64 rows 267 / 241, 96 rows 276 / 247, 129 rows 301 / 286; x 1024, 200 rows 152 / 102; 65536 x 2048, 128
-    rows 78 / 56; 32768 x 2048, 80 rows 40 / 33, 200 rows 42 / 39, but 64 rows 29 / 32.  Rows beyond 208 and fewer columns were not measured."""
+    rows 78 / 56; 32768 x 2048, 80 rows 40 / 33, 200 rows 44 / 36, but 64 rows 29 / 32.  Up to 128 columns of blocks a column's rows go in two (32768 x
+    1024, the library / in one block / in two: 96 rows 18.5 / 20.6 / 18.9, 128 rows 19.6 / 22.5 / 19.5; x 4096, 128 rows 70.5 / 66.8 / 58.0).  More than 128
+    rows, two blocks a column, not where the last of several rounds is nearly empty (100352 x 2048, 784 blocks, 176 rows 118 / 126).  Rows beyond 208 and
+    fewer columns were not measured."""
     if not 64 <= M <= 208 or N < (65536 if M == 64 else 32768) or N % 16 or K % 128 or N * K >= 1 << 30:
         return 0
-    return min(8, M // 16)
+    columns = -(-N // 256)
+    if M > 128 and columns > 256 and 2 * columns % 256 in range(1, 64):
+        return 0
+    # a column's rows in one block up to 128 of them; in two where both find a unit of their own
+    return min(8, M // 16) if 2 * columns > 256 else min(M // 16, max(4, -(-M // 32)))
 
 
 def _rows_product_us(M: int, N: int, K: int, tiles: int, parts: int) -> float:
