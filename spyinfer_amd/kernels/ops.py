@@ -459,7 +459,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         return decode_linear(x, tiled, out_dtype, out)
     if all_bf16 and tiled is not None and out_dtype == torch.bfloat16 and x.is_contiguous():
         tiles = rows_product_stored(M, N, K, _step.replayed and not isinstance(w, TiledOnly))      # (whose library product copies the rows first)
-        tall = None if tiles else rows_product_tall(M, N, K, ROWS_STORE)
+        tall = None if tiles or M < ROWS_TALL_MIN else rows_product_tall(M, N, K, ROWS_STORE)
         tiles = tall[0] if tall else tiles
         if tiles and (x.data_ptr() | out.data_ptr()) % 16 == 0:
             _check(tiled.shape == w.shape, "linear: the tiled copy does not fit the matrix")
@@ -663,6 +663,8 @@ def rows_product_gated(M: int, N: int, K: int, library: bool) -> int:
     return tiles
 
 
+#: fewest rows of a tall block (callers ask first: short prompts are bound by the host, whose every question is 0.3 us)
+ROWS_TALL_MIN = 144
 #: what the estimate of a product by tall blocks is made of, microseconds, per kind of result: the launch; a round's turn of 128 of K, and each row
 #: tile of it; a round's way in and out, and each row tile of that; a turn's row tile of a unit's even share of all blocks (units that work
 #: together take memory and clock from each other, whether their last round is full or nearly so)
@@ -716,7 +718,7 @@ def rows_product_tall(M: int, N: int, K: int, kind: int, other: int = 0):
     parts, with the norm that sums them, which multiply a unit's share: 2560 x 9728, 640 rows (1.6) 44.9 / 45.5, 900 (2.2) 58.4 / 56.3, 2048 117 /
     106; 2048 x 6144, 900 rows (1.8) 39.8 / 40.0, 1356 52.8 / 47.4, 2048 69.9 / 64.9; 4096 x 12288, 1356 rows 160 / 128, 2048 201 / 187; 2560 x
     4096, 1200 rows 48.1 / 43.2, 2048 (5.0) 62.2 / 60.2; 4096 x 4096, 640 rows 45.2 / 39.1, 1500 rows (5.9) 65.5 / 65.4."""
-    if M < 144 or N % (32 if kind == ROWS_GATED else 16) or K % 128 or N * K >= 1 << 30 or M * K >= 1 << 30:
+    if M < ROWS_TALL_MIN or N % (32 if kind == ROWS_GATED else 16) or K % 128 or N * K >= 1 << 30 or M * K >= 1 << 30:
         return None
     rows, columns, chunks = -(-M // 16), -(-N // 256), K // 128
     share = rows * columns / 256
@@ -795,7 +797,7 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor, tiled: Optional[torch.Tensor]
         return linear_few(x, w, tiled)
     plan = None
     if tiled is not None and x.dtype == torch.bfloat16 and x.is_contiguous():
-        plan = rows_product_tall(M, w.shape[0], K, ROWS_PARTS) or rows_product_parts(M, w.shape[0], K)
+        plan = (rows_product_tall(M, w.shape[0], K, ROWS_PARTS) if M >= ROWS_TALL_MIN else None) or rows_product_parts(M, w.shape[0], K)
     if plan is None or x.data_ptr() % 16:
         return linear_few(x, w, tiled)
     _dev(x, tiled)
@@ -855,7 +857,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, tiled: Optional[torc
         return out
     if x.dtype == torch.bfloat16 and tiled is not None and x.is_contiguous():
         tiles = rows_product_gated(M, 2 * I, K, not isinstance(w_gate_up, TiledOnly))
-        tall = rows_product_tall(M, 2 * I, K, ROWS_GATED, tiles)
+        tall = rows_product_tall(M, 2 * I, K, ROWS_GATED, tiles) if M >= ROWS_TALL_MIN else None
         tiles = tall[0] if tall else tiles
         if tiles and x.data_ptr() % 16 == 0:
             _check(tiled.shape == w_gate_up.shape, "linear_swiglu: the tiled copy does not fit")
@@ -1424,18 +1426,19 @@ def fused_attention_ok(dtype, meta: AttentionMeta, n_q: int, n_kv: int, d: int, 
     """True if this step's attention may take the raw product (``RawQKV``): every entry a single token, bfloat16 with
     head_dim 64, 128 or 256 or float32 with 64 or 128 (and float32 norm weights), rotated whole or not at all, 16-row tiles built for this group size.
     ``operands``: what else the kernel would read (caches, rotation table); float32 ones that do not lie at 16 bytes go by kernels that take any."""
+    # (what a step with several tokens of a request fails by comes first: it is asked in every layer of a prompt, whose launches the host bounds)
+    if meta.T != meta.S or meta.max_q_len != 1 or meta.tiles is None or meta.tiles_group != n_q // n_kv or n_q // n_kv > 16:
+        return False
+    if meta.tiles["small"][2] != meta.S or meta.tiles["big"][2] != 0:
+        return False
     if dtype == torch.float32:
-        if any(t is not None and t.data_ptr() % 16 for t in operands):
-            return False
         if not FUSED_DECODE or not f32_attention_ok(dtype, d, page_size) or meta.S > 65535:
+            return False
+        if any(t is not None and t.data_ptr() % 16 for t in operands):
             return False
         if any(w is not None and (w.dtype != torch.float32 or w.data_ptr() % 16) for w in (q_norm_w, k_norm_w)):
             return False
     elif not mfma_attention_ok(dtype, d, page_size):
-        return False
-    if meta.T != meta.S or meta.max_q_len != 1 or meta.tiles is None or meta.tiles_group != n_q // n_kv or n_q // n_kv > 16:
-        return False
-    if meta.tiles["small"][2] != meta.S or meta.tiles["big"][2] != 0:
         return False
     if d not in (64, 128, 256) or rotary_dim not in (0, d) or (q_norm_w is None) != (k_norm_w is None):
         return False

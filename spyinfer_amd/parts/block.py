@@ -100,7 +100,7 @@ class PreNormBlock(Block):
         ready = isinstance(pending, ops.ScaledInput)
         mine = ready and pending.norm is self.norm1
         plain = self.ffn is not None and self.gate1 is None and self.gate2 is None
-        fold = plain and self.norm2.foldable(act) is not None and self.mixer.can_fold(batch) and self.ffn.can_fold(batch)
+        fold = plain and self.mixer.can_fold(batch) and self.ffn.can_fold(batch) and self.norm2.foldable(act) is not None
         if fold and not ops.folded_products_take(pending if mine else None, batch.T):
             # beyond 64 rows the folded products take an input in operand order only, which only the part before this
             # block can have prepared (another kind of block, a position encoding on the embeddings, parts that fold up
