@@ -18,7 +18,7 @@ MAX_PARTS = 32              # most parts of an (entry, kv head): what the kernel
 PIECE_UNITS = 256           # compute units that the pieces are dealt to; each runs two blocks at a time
 PIECE_MIN_BLOCKS = 8        # a part wants this many blocks of 32 keys at least (measured at 1100 keys, 1 to 4 requests: 4-8 parts best)
 PIECE_RECORD = 8            # ints per record
-# What the estimate of a cut's time is made of, in microseconds (measured with 8 kv heads of 128, 8 to 96 requests of
+# What the estimate of a cut's time is made of, in microseconds (measured with 8 kv heads of 128 in blocks of four waves, 8 to 96 requests of
 # even and uneven lengths; the estimates are within 8 % rms of the kernel's times, and the cut they choose was the
 # fastest of those measured, to within the timings' noise, in every case):
 PIECE_START_US = 7.0        # from the kernel's start to a block's first keys, and its end
