@@ -11,7 +11,7 @@
 // 128, all there is.  A turn is 128 of K: X's next 128 go from memory into the other of two LDS stages while this one's 16 MT
 // products run, and a step's W registers are asked for again, for the next turn, as soon as their last product is issued.  Piece p of
 // an LDS row lies at place p ^ (row % 16), which the lanes' source addresses see to, so that the operands' reads meet in no bank.
-// Two blocks fit a compute unit.  (Blocks of 9 to 16 row tiles, one a unit: gemm_rows_tall.hip, for all but small shares of work.)  Turns of 256 (twice the bytes under way) and loads spread over the products one by one were not faster.
+// Two blocks fit a compute unit.  (Blocks of 9 to 16 row tiles, one a unit: gemm_rows_tall.hip; which of the two: rows_product_tall in kernels/ops.py.)  Turns of 256 (twice the bytes under way) and loads spread over the products one by one were not faster.
 //
 // Why parts: a prompt of a few hundred rows has fewer tiles than compute units, and each would walk all of K alone.  Measured (us;
 // library, this kernel, and what the sum of its parts adds to the norm's pass):  409 rows, 2560 x 9728: 53.7, 27.8 + 5 (six parts);
