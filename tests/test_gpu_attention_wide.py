@@ -49,3 +49,34 @@ def test_few_single_tokens(cached, P, window):
     assert torch.equal(again, out)
     raw.store = False                                                   # (the new key read from the cache, where another call put it)
     close(ops.paged_attention(None, kd, vd, P, meta, n_q, n_kv, d, d ** -0.5, window, raw), ref, dtype, scale=3.0, what="without store")
+
+
+def test_steps_whose_longest_request_passes_the_line(tmp_path):
+    """18 requests of 8 kv heads, the longest passing 1024 keys while they decode under graphs: blocks of eight waves, then of four, which are two graphs; the
+    same logits as eager steps, and the graphs go by the longest request."""
+    from spyinfer_amd.engine.batch import StepEntry
+    from spyinfer_amd.engine.runner import ModelRunner, load_model
+    from spyinfer_amd.weights import write_random_model
+    from tests.configs import INIT, TINY_E
+    require_gpu()
+    config = dict(TINY_E, num_hidden_layers=1, num_key_value_heads=8, max_position_embeddings=1100)
+    model = load_model(write_random_model(str(tmp_path / "m"), config, 5, torch.bfloat16, **INIT), "bfloat16", "cuda:0")
+    gen = torch.Generator().manual_seed(9)
+    prompts = [torch.randint(0, 300, (1020 if i == 3 else 30 + 7 * i,), generator=gen).tolist() for i in range(18)]
+    runs = []
+    for eager in (True, False):
+        runner = ModelRunner(model, "bfloat16", "cuda:0", 16, 300, 18, enforce_eager=eager, max_model_len=1100)
+        caches = [runner.manager.admit(i) for i in range(18)]
+        for c, p in zip(caches, prompts):
+            runner.manager.reserve(c, len(p))
+        runner.step([StepEntry(c, p, []) for c, p in zip(caches, prompts)])
+        outs, tokens = [], torch.Generator().manual_seed(10)
+        for _ in range(9):
+            step = torch.randint(0, 300, (18,), generator=tokens).tolist()
+            for c in caches:
+                runner.manager.reserve(c, 1)
+            outs.append(runner.step([StepEntry(c, [t], [0]) for c, t in zip(caches, step)]).cpu().clone())
+        runs.append(outs)
+    assert sorted(dict(key[2])["decode_pieces_waves_8_0_128"] for key in runner._graphs) == [4, 8]
+    assert runner.graph_replays == 7                                    # (of 4 steps and 5, the first of each shape runs kernel by kernel)
+    assert all(torch.equal(a, b) for a, b in zip(*runs)) and all(torch.isfinite(a).all() for a in runs[0])
